@@ -18,7 +18,10 @@ AUX_PAD = 64          # floats between the per-(b,d,l) part of the auxiliary buf
 MAX_STATE = 64
 VAR_UNITARY, VAR_COMPLEX, VAR_REAL = 0, 1, 2   # variant codes of the C ABI
 
+HOST_PATH = os.path.join(_HERE, "lib", "_aussm_host.so")
+
 _lib = None
+_host = None
 
 _P = c_void_p
 _I = c_int
@@ -49,6 +52,7 @@ _SIGNATURES = {
     "aussm_swap_last2_act": [_P] * 4 + [_I] * 3 + [_LL] * 4 + [_I] * 2 + [_P],
     "aussm_gate_fwd": [_P] * 3 + [ctypes.c_size_t, _P],
     "aussm_gate_bwd": [_P] * 5 + [ctypes.c_size_t, _P],
+    "aussm_zero_f32": [_P, ctypes.c_size_t, _P],
     "aussm_hbm_probe": [_P] * 5 + [_I] * 4 + [_P],
     "aussm_ssm_adaptive_unitary_fwd": [_P] * 16 + [_I] * 4 + [_P],
     "aussm_ssm_adaptive_unitary_bwd": [_P] * 30 + [_I] * 4 + [_P],
@@ -93,6 +97,23 @@ def load() -> ctypes.CDLL:
     lib.aussm_error_string.restype = c_char_p
     _lib = lib
     return lib
+
+
+def host():
+    """The native host path (csrc/host): argument checks, allocation, launches and autograd nodes of the package's
+    calls in C++.  Loaded once; raises AussmError if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise AussmError(f"{HOST_PATH} not found: build it with `python -m aussm_amd.build`")
+        import importlib.machinery
+        import importlib.util
+        loader = importlib.machinery.ExtensionFileLoader("_aussm_host", HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_aussm_host", loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def check(code: int, what: str) -> None:

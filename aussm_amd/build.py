@@ -1,7 +1,8 @@
-"""Builds libaussm_hip.so (hand-written HIP for gfx950) in-tree with hipcc.
+"""Builds libaussm_hip.so (hand-written HIP for gfx950) and the host module _aussm_host.so in-tree.
 
     python -m aussm_amd.build                 # compile every translation unit and link
     python -m aussm_amd.build --only k_px     # recompile one unit (the others' objects must exist) and relink
+    python -m aussm_amd.build --only host     # recompile the host module only
     python -m aussm_amd.build --asm DIR       # also keep the compiler's gfx950 assembly in DIR
     python -m aussm_amd.build --check         # compile k_px.hip to assembly and check its listings (below)
 
@@ -25,7 +26,7 @@ LIBNAME = "libaussm_hip.so"
 
 # One translation unit per kernel family: they compile side by side, and a change in one family
 # does not recompile the others' objects by hand (`--only k_px` rebuilds one unit and relinks).
-SOURCES = ["scan_api.hip", "k_generic.hip", "k_xdl.hip", "k_px.hip", "k_dropin.hip"]
+SOURCES = ["scan_api.hip", "k_fwd.hip", "k_ubwd.hip", "k_rbwd.hip", "k_generic.hip", "k_xdl.hip", "k_px.hip", "k_dropin.hip"]
 
 # Packed-FP32 instructions are switched off on purpose (see the flag): the kernels are written
 # with scalar float arithmetic only.
@@ -44,6 +45,12 @@ HIPCC_FLAGS = [
 VALIDATED_HIPCC = "HIP version: 7.2.26015-fc0010cf6a"
 # units whose kernels issue loads as hand-written instructions: their listings are checked by every build
 HAND_TRACKED = ("k_px.hip", "k_xdl.hip")
+
+
+# The native host path: a Python extension module over torch's C++ API, linked to the library beside it.
+HOST_DIR = os.path.join(CSRC, "host")
+HOST_SOURCES = ["module.cpp", "scans.cpp"]
+HOST_NAME = "_aussm_host.so"
 
 
 def hipcc_version(hipcc: str) -> str:
@@ -73,6 +80,32 @@ def _compile(hipcc: str, src: str, verbose: bool, asm_dir: str | None, extra) ->
     subprocess.run(cmd, check=True, cwd=cwd)
 
 
+def _host_flags():
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension as ext
+    inc = [p for p in ext.include_paths("cuda") if not p.endswith("THH")] + [sysconfig.get_paths()["include"]]
+    cflags = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DTORCH_EXTENSION_NAME=_aussm_host"]
+    cflags += [f for p in inc for f in ("-isystem", p)]
+    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    ldflags = [f"-L{tlib}", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lc10", "-lc10_hip", f"-L{LIBDIR}",
+               f"-l:{LIBNAME}", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{tlib}"]
+    return cflags, ldflags
+
+
+def _host_obj(src: str) -> str:
+    return os.path.join(LIBDIR, "host_" + os.path.splitext(src)[0] + ".o")
+
+
+def _compile_host(src: str, cflags, verbose: bool) -> None:
+    cmd = ["g++", *cflags, "-c", os.path.join(HOST_DIR, src), "-o", _host_obj(src)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True, cwd=LIBDIR)
+
+
 def build(verbose: bool = True, asm_dir: str | None = None, only=None, extra=()) -> str:
     """Compile every translation unit (all of them, every time, unless `only` names a subset whose
     siblings' objects already exist) and link libaussm_hip.so."""
@@ -98,8 +131,12 @@ def build(verbose: bool = True, asm_dir: str | None = None, only=None, extra=())
     todo = [s for s in SOURCES if not only or os.path.splitext(s)[0] in only or not os.path.exists(_obj(s))]
     # the listings of the hand-tracked units among them are checked alongside (same compiler, same flags);
     # a finding fails the build before the library is put in place
+    cflags, ldflags = _host_flags()
+    host_todo = [h for h in HOST_SOURCES if not only or "host" in only or "host_" + os.path.splitext(h)[0] in only
+                 or not os.path.exists(_host_obj(h))]
     with ThreadPoolExecutor(max_workers=8) as ex:
         jobs = [ex.submit(_compile, hipcc, s, verbose, asm_dir, extra) for s in todo]
+        jobs += [ex.submit(_compile_host, h, cflags, verbose) for h in host_todo]
         jobs += [ex.submit(check_unit_listing, u, verbose) for u in HAND_TRACKED if u in todo]
         for f in jobs:
             f.result()
@@ -110,6 +147,12 @@ def build(verbose: bool = True, asm_dir: str | None = None, only=None, extra=())
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True, cwd=LIBDIR)
     os.replace(tmp, out)
+    host = os.path.join(LIBDIR, HOST_NAME)
+    cmd = ["g++", "-shared", "-o", host + ".tmp"] + [_host_obj(h) for h in HOST_SOURCES] + ldflags
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True, cwd=LIBDIR)
+    os.replace(host + ".tmp", host)
     return out
 
 

@@ -1,0 +1,110 @@
+// Shared pieces of the native host path: the Python extension module _aussm_host (torch C++ API over the C ABI of
+// libaussm_hip.so).  It holds what a call of the package does between Python and the kernel launches - argument
+// checks, output and workspace allocation, the autograd graph node - so that a small call costs a few microseconds
+// of host time.  (Python autograd functions over ctypes took 60-100 us per forward + backward.)
+#pragma once
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
+#include <optional>
+#include <sstream>
+#include <stdexcept>
+#include <string>
+
+#include "../../../include/aussm_hip.h"
+
+namespace aussm_host {
+
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+typedef std::optional<Tensor> OptTensor;
+
+// raised in Python as aussm_amd._lib.AussmError
+struct AussmError : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+// raised in Python as RuntimeError / ValueError, without the C++ call stack that TORCH_CHECK appends
+struct ArgError : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+struct ValueArgError : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
+template <typename... T>
+std::string cat(const T&... v) {
+  std::ostringstream s;
+  (s << ... << v);
+  return s.str();
+}
+template <typename... T>
+[[noreturn]] void fail(const T&... v) { throw ArgError(cat(v...)); }
+
+inline std::string shape_str(at::IntArrayRef v) {
+  std::ostringstream s;
+  s << '(';
+  for (size_t i = 0; i < v.size(); ++i) s << (i ? ", " : "") << v[i];
+  if (v.size() == 1) s << ',';
+  s << ')';
+  return s.str();
+}
+
+inline void check(int code, const char* what) {
+  if (code != 0) throw AussmError(cat(what, " failed with code ", code, ": ", aussm_error_string(code)));
+}
+
+template <typename T = float>
+T* ptr(const Tensor& t) { return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr; }
+
+inline void* cur_stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
+
+inline Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+
+// a tensor whose data pointer can be handed to a kernel: dense, no lazy conjugation or negation.
+// (Called with gradient recording off: the graph node keeps the edges of the tensor it was given.)
+inline Tensor dense(const Tensor& t) {
+  if (!t.defined()) return t;
+  Tensor r = t;
+  if (r.is_conj()) r = r.resolve_conj();
+  if (r.is_neg()) r = r.resolve_neg();
+  return r.contiguous();
+}
+
+inline bool wants_grad(const Tensor& t) { return t.defined() && t.requires_grad(); }
+
+inline Tensor empty_f32(at::IntArrayRef shape, const Tensor& like) {
+  return at::empty(shape, at::TensorOptions().dtype(at::kFloat).device(like.device()));
+}
+
+// float32 (optional) tensor of a given shape
+inline Tensor f32(const Tensor& t, const char* name, at::IntArrayRef shape) {
+  if (!t.defined()) return t;
+  if (t.scalar_type() != at::kFloat) fail("expected ", name, " to be float32, got torch.", t.scalar_type());
+  if (t.sizes() != shape) fail("expected ", name, " of shape ", shape_str(shape), ", got ", shape_str(t.sizes()));
+  return dense(t);
+}
+
+// A graph node over saved tensors: `saved` are released together, and unpacking them after that raises torch's
+// usual error about a second backward pass.
+struct SavingNode : Node {
+  std::vector<SavedVariable> saved;
+  void save(std::initializer_list<Tensor> ts) {
+    saved.reserve(ts.size());
+    for (const Tensor& t : ts) saved.emplace_back(t, false);
+  }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (auto& s : saved) s.reset_data();
+  }
+};
+
+template <typename N>
+std::shared_ptr<N> make_node() { return std::shared_ptr<N>(new N(), torch::autograd::deleteNode); }
+
+}  // namespace aussm_host

@@ -1,0 +1,410 @@
+// The core scans of aussm_amd/scan.py: unitary_scan, complex_scan, selective_scan_fn.
+// Argument meaning, shapes and error texts are documented there.
+#include "common.h"
+#include "host.h"
+
+namespace aussm_host {
+
+namespace {
+
+constexpr int TILE = AUSSM_TILE;
+constexpr int REC_CK = AUSSM_TILE / 2;          // checkpoint interval of the recomputing backward kernels
+constexpr int VAR_COMPLEX = 1, VAR_REAL = 2;
+constexpr int AUX_PAD = 64;
+
+int in_dtype(const Tensor& t) {
+  if (t.scalar_type() == at::kFloat) return AUSSM_F32;
+  if (t.scalar_type() == at::kBFloat16) return AUSSM_BF16;
+  fail("expected float32 or bfloat16 scan input, got torch.", t.scalar_type());
+}
+
+void check_bdl(const Tensor& u, const Tensor& delta) {
+  if (u.dim() != 3) fail("expected u of shape (b, d, l), got ", shape_str(u.sizes()));
+  if (!u.is_cuda()) fail("scan inputs must be on the GPU (no CPU implementation is shipped)");
+  if (delta.sizes() != u.sizes() || delta.scalar_type() != u.scalar_type()) fail("delta must match u in shape and dtype");
+}
+
+// (b, n, l) complex64 or (b, n, l, 2) of dtype: dense
+Tensor complex_rows(const Tensor& t, const char* name, int64_t b, int64_t l, at::ScalarType dtype) {
+  at::ScalarType st = t.scalar_type();
+  const bool cplx = at::isComplexType(st);
+  if (cplx) {
+    if (st != at::kComplexFloat) fail("expected ", name, " to be complex64, got torch.", st);
+    st = at::kFloat;
+  }
+  const bool ok = cplx ? t.dim() == 3 && t.size(0) == b && t.size(2) == l
+                       : t.dim() == 4 && t.size(0) == b && t.size(2) == l && t.size(3) == 2;
+  if (!ok) fail("expected ", name, " of shape (b, n, l) complex or (b, n, l, 2), got ", shape_str(t.sizes()));
+  if (st != dtype) fail(name, " must have the dtype of u (torch.", dtype, "), got torch.", st);
+  return dense(t);
+}
+
+Tensor check_h0(const Tensor& h0, int64_t b, int64_t d, int64_t n) {
+  if (!h0.defined()) return h0;
+  if (h0.scalar_type() != at::kComplexFloat || h0.sizes() != at::IntArrayRef({b, d, n}))
+    fail("expected h0 complex64 of shape ", shape_str({b, d, n}));
+  return dense(h0);
+}
+
+// gradient of a (b, n, l[, 2]) float buffer in the type and shape of the tensor it belongs to
+Tensor as_like(const Tensor& g, bool complex, at::ScalarType dtype) {
+  if (complex) return at::view_as_complex(g);
+  return dtype == at::kFloat ? g : g.to(dtype);
+}
+
+Tensor workspace(int variant, const Tensor& u, int b, int d, int n, int l, int ck, int dt) {
+  const size_t f = aussm_scan_workspace_floats(variant, b, d, n, l, ck, dt);
+  return f ? empty_f32({(int64_t)f}, u) : Tensor();
+}
+
+// ---- buffers that the backward kernels accumulate into: one allocation and one clearing launch
+struct Acc {
+  Tensor all;
+  std::vector<int64_t> at_;
+  int64_t total = 0;
+  int add(int64_t n) {
+    at_.push_back(total);
+    total += (n + 3) / 4 * 4;                   // every part starts on 16 bytes
+    return (int)at_.size() - 1;
+  }
+  void make(const Tensor& like) {
+    all = empty_f32({total}, like);
+    check(aussm_zero_f32(ptr(all), (size_t)total, cur_stream()), "aussm_zero_f32");
+  }
+  Tensor part(int i, at::IntArrayRef shape) const {
+    std::vector<int64_t> strides(shape.size());
+    int64_t s = 1;
+    for (size_t k = shape.size(); k-- > 0;) { strides[k] = s; s *= shape[k]; }
+    return all.as_strided(shape, strides, at_[i]);
+  }
+};
+
+// ============================================================================ unitary
+
+struct UnitaryNode : SavingNode {
+  int b, d, n, l, ck, dt;
+  bool bc_complex;
+  std::string name() const override { return "AussmUnitaryScanBackward"; }
+  variable_list apply(variable_list&& g) override;
+};
+
+enum { U_U, U_DELTA, U_THETA, U_B, U_C, U_D, U_Z, U_H0, U_INPUTS };
+
+variable_list UnitaryNode::apply(variable_list&& g) {
+  std::lock_guard<std::mutex> lock(mutex_);
+  at::NoGradGuard no_grad;
+  variable_list out(U_INPUTS);
+  if (!g[0].defined() && !(g.size() > 1 && g[1].defined())) return out;
+  const Tensor u = saved[0].unpack(), delta = saved[1].unpack(), theta = saved[2].unpack(), B = saved[3].unpack(),
+               C = saved[4].unpack(), D = saved[5].unpack(), z = saved[6].unpack(), hck = saved[7].unpack(),
+               aux = saved[8].unpack(), ypre = saved[9].unpack();
+  const c10::DeviceGuard guard(u.device());
+  Tensor dy = g[0].defined() ? dense(g[0]) : at::zeros({b, d, l}, theta.options());
+  const Tensor dhL = g.size() > 1 ? dense(g[1]) : Tensor();
+  if (z.defined()) {
+    // the kernels take the gradient of the ungated output
+    Tensor dpre = empty_f32({b, d, l}, u), dz = empty_f32({b, d, l}, u);
+    check(aussm_gate_bwd(ptr(dy), ptr(ypre), ptr(z), ptr(dpre), ptr(dz), (size_t)b * d * l, cur_stream()), "aussm_gate_bwd");
+    dy = dpre;
+    out[U_Z] = dz;
+  }
+  Tensor du = empty_f32({b, d, l}, u), ddelta = empty_f32({b, d, l}, u), dtheta = empty_f32({b, d, l}, u);
+  const bool want_dD = D.defined() && task_should_compute_output(U_D);
+  const bool want_dh0 = task_should_compute_output(U_H0);
+  Acc acc;
+  const int iB = acc.add((int64_t)b * n * l * 2), iC = acc.add((int64_t)b * n * l * 2), iD = want_dD ? acc.add(d) : 0;
+  acc.make(u);
+  Tensor dB = acc.part(iB, {b, n, l, 2}), dC = acc.part(iC, {b, n, l, 2}), dD = want_dD ? acc.part(iD, {d}) : Tensor();
+  Tensor dh0 = want_dh0 ? empty_f32({b, d, n, 2}, u) : Tensor();
+  check(aussm_unitary_bwd_aux(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(hck), ptr(aux),
+                              ptr(du), ptr(ddelta), ptr(dtheta), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), b, d, n, l, ck, dt,
+                              b / (int)u.size(0), cur_stream()),
+        "aussm_unitary_bwd_aux");
+  if (u.size(0) != b) {                          // u, delta shared by consecutive batch elements
+    du = du.view({u.size(0), -1, d, l}).sum(1);
+    ddelta = ddelta.view({u.size(0), -1, d, l}).sum(1);
+  }
+  out[U_U] = as_like(du, false, u.scalar_type());
+  out[U_DELTA] = as_like(ddelta, false, u.scalar_type());
+  out[U_THETA] = dtheta;
+  out[U_B] = as_like(dB, bc_complex, u.scalar_type());
+  out[U_C] = as_like(dC, bc_complex, u.scalar_type());
+  if (want_dD) out[U_D] = dD;
+  if (want_dh0) out[U_H0] = at::view_as_complex(dh0);
+  return out;
+}
+
+}  // namespace
+
+// Checkpoint interval of the unitary scan for a shape: 256, or half of it where that lets a launch with few (batch,
+// channel) pairs be split into more segments along L (a segment is a whole number of checkpoint blocks); calls
+// that are not split at all checkpoint every 4096 steps (one checkpoint, at the end, for shorter sequences).
+int unitary_ck(int b, int d, int n, int l) {
+  constexpr int CK = 256, CK_LONG = 4096;
+  const int s_half = aussm_unitary_split_segments(b, d, n, l, CK / 2), s_full = aussm_unitary_split_segments(b, d, n, l, CK);
+  if (s_half > s_full) return CK / 2;
+  if (s_full <= 1) return std::min(CK_LONG, (l + TILE - 1) / TILE * TILE);
+  return CK;
+}
+
+std::pair<Tensor, Tensor> unitary_scan(const Tensor& u_, const Tensor& delta_, const Tensor& theta_, const Tensor& Bc, const Tensor& Cc,
+                                       const OptTensor& D_, const OptTensor& z_, const OptTensor& h0_, bool want_state) {
+  check_bdl(u_, delta_);
+  const c10::DeviceGuard guard(u_.device());
+  const Tensor Dv = opt(D_), zv = opt(z_), hv = opt(h0_);
+  const bool needs_grad = at::GradMode::is_enabled() && (wants_grad(u_) || wants_grad(delta_) || wants_grad(theta_) || wants_grad(Bc) ||
+                                                         wants_grad(Cc) || wants_grad(Dv) || wants_grad(zv) || wants_grad(hv));
+  Tensor y, hL;
+  std::shared_ptr<UnitaryNode> node;
+  {
+    at::NoGradGuard no_grad;
+    const Tensor u = dense(u_), delta = dense(delta_);
+    const int64_t bu = u.size(0), d = u.size(1), l = u.size(2);
+    const int64_t b = theta_.dim() == 3 ? theta_.size(0) : bu;
+    if (b % bu != 0) fail("batch size of theta (", b, ") must be a multiple of that of u (", bu, ")");
+    const Tensor theta = f32(theta_, "theta", {b, d, l});
+    const Tensor B = complex_rows(Bc, "B", b, l, u.scalar_type()), C = complex_rows(Cc, "C", b, l, u.scalar_type());
+    const int64_t n = B.size(1);
+    if (C.size(1) != n) fail("B and C must have the same state size");
+    const Tensor D = f32(Dv, "D", {d}), z = f32(zv, "z", {b, d, l}), h0 = check_h0(hv, b, d, n);
+    const int dt = in_dtype(u), urep = (int)(b / bu), ck = unitary_ck(b, d, n, l);
+    y = empty_f32({b, d, l}, u);
+    if (want_state) hL = empty_f32({b, d, n, 2}, u);
+    const size_t aux_floats = aussm_unitary_aux_floats(b, d, n, l, ck);
+    Tensor aux;
+    if (needs_grad) {
+      // not where neither direction would touch the buffer: the vector-ALU kernels use it only for the segment
+      // states of a call that is split along the sequence
+      if (aussm_unitary_kernel_mode(0, b, d, n, l, ck, dt, urep, 1) || aussm_unitary_kernel_mode(1, b, d, n, l, ck, dt, urep, 1) ||
+          aussm_unitary_split_segments(b, d, n, l, ck) > 1)
+        aux = empty_f32({(int64_t)aux_floats}, u);
+      const Tensor hck = empty_f32({b, (l + ck - 1) / ck, n, 2, d}, u);
+      check(aussm_unitary_fwd_aux(ptr(u), ptr(delta), ptr(theta), ptr(B), ptr(C), ptr(D), nullptr, ptr(h0), ptr(y), ptr(hL), ptr(hck),
+                                  ptr(aux), b, d, n, l, ck, dt, urep, cur_stream()),
+            "aussm_unitary_fwd_aux");
+      Tensor ypre;
+      if (z.defined()) {
+        ypre = y;
+        y = empty_f32({b, d, l}, u);
+        check(aussm_gate_fwd(ptr(ypre), ptr(z), ptr(y), (size_t)b * d * l, cur_stream()), "aussm_gate_fwd");
+      }
+      node = make_node<UnitaryNode>();
+      node->set_next_edges(torch::autograd::collect_next_edges(u_, delta_, theta_, Bc, Cc, Dv, zv, hv));
+      node->save({u, delta, theta, B, C, D, z, hck, aux, ypre});
+      node->b = b; node->d = d; node->n = n; node->l = l; node->ck = ck; node->dt = dt;
+      node->bc_complex = Bc.is_complex();
+    } else {
+      // no backward pass: the buffer serves as workspace only (prepared operands of the matrix-core kernels, segment
+      // states of a launch that is split along L) and no checkpoints are kept.  (The buffer of a shape that the
+      // matrix-core kernels serve starts with b d l floats that only a backward call would read.)
+      const size_t body = aux_floats - AUX_PAD;
+      if (body != 0 && body != (size_t)b * d * l && urep == 1) aux = empty_f32({(int64_t)aux_floats}, u);
+      check(aussm_unitary_fwd_aux(ptr(u), ptr(delta), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(z), ptr(h0), ptr(y), ptr(hL), nullptr,
+                                  ptr(aux), b, d, n, l, aux.defined() ? ck : TILE, dt, urep, cur_stream()),
+            "aussm_unitary_fwd_aux");
+    }
+    if (want_state) hL = at::view_as_complex(hL);
+  }
+  if (node) {
+    torch::autograd::set_history(y, node);
+    if (want_state) torch::autograd::set_history(hL, node);
+  }
+  return {y, hL};
+}
+
+// ============================================================================ complex
+
+namespace {
+
+struct ComplexNode : SavingNode {
+  int b, d, n, l, dt;
+  bool bc_complex;
+  std::string name() const override { return "AussmComplexScanBackward"; }
+  variable_list apply(variable_list&& g) override;
+};
+
+enum { X_U, X_DELTA, X_RHO, X_THETA, X_B, X_C, X_D, X_H0, X_Z, X_INPUTS };
+
+variable_list ComplexNode::apply(variable_list&& g) {
+  std::lock_guard<std::mutex> lock(mutex_);
+  at::NoGradGuard no_grad;
+  variable_list out(X_INPUTS);
+  if (!g[0].defined() && !(g.size() > 1 && g[1].defined())) return out;
+  const Tensor u = saved[0].unpack(), delta = saved[1].unpack(), rho = saved[2].unpack(), theta = saved[3].unpack(),
+               B = saved[4].unpack(), C = saved[5].unpack(), D = saved[6].unpack(), h0 = saved[7].unpack(),
+               z = saved[8].unpack(), hck = saved[9].unpack();
+  const c10::DeviceGuard guard(u.device());
+  const Tensor dy = g[0].defined() ? dense(g[0]) : at::zeros({b, d, l}, theta.options());
+  const Tensor dhL = g.size() > 1 ? dense(g[1]) : Tensor();
+  Tensor du = empty_f32({b, d, l}, u), ddelta = empty_f32({b, d, l}, u), drho = empty_f32({b, d, l}, u),
+         dtheta = empty_f32({b, d, l}, u), dz = z.defined() ? empty_f32({b, d, l}, u) : Tensor();
+  const bool want_dD = D.defined() && task_should_compute_output(X_D);
+  const bool want_dh0 = h0.defined() && task_should_compute_output(X_H0);
+  Acc acc;
+  const int iB = acc.add((int64_t)b * n * l * 2), iC = acc.add((int64_t)b * n * l * 2), iD = want_dD ? acc.add(d) : 0;
+  acc.make(u);
+  Tensor dB = acc.part(iB, {b, n, l, 2}), dC = acc.part(iC, {b, n, l, 2}), dD = want_dD ? acc.part(iD, {d}) : Tensor();
+  Tensor dh0 = want_dh0 ? empty_f32({b, d, n, 2}, u) : Tensor();
+  const Tensor ws = workspace(VAR_COMPLEX, u, b, d, n, l, REC_CK, dt);
+  check(aussm_complex_bwd(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(rho), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(h0), ptr(hck),
+                          ptr(du), ptr(ddelta), ptr(drho), ptr(dtheta), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), ptr(z), ptr(dz), ptr(ws),
+                          b, d, n, l, REC_CK, dt, cur_stream()),
+        "aussm_complex_bwd");
+  out[X_U] = as_like(du, false, u.scalar_type());
+  out[X_DELTA] = as_like(ddelta, false, u.scalar_type());
+  out[X_RHO] = drho;
+  out[X_THETA] = dtheta;
+  out[X_B] = as_like(dB, bc_complex, u.scalar_type());
+  out[X_C] = as_like(dC, bc_complex, u.scalar_type());
+  if (want_dD) out[X_D] = dD;
+  if (want_dh0) out[X_H0] = at::view_as_complex(dh0);
+  if (z.defined()) out[X_Z] = dz;
+  return out;
+}
+
+}  // namespace
+
+std::pair<Tensor, Tensor> complex_scan(const Tensor& u_, const Tensor& delta_, const Tensor& rho_, const Tensor& theta_, const Tensor& Bc,
+                                       const Tensor& Cc, const OptTensor& D_, const OptTensor& z_, const OptTensor& h0_, bool want_state) {
+  check_bdl(u_, delta_);
+  const c10::DeviceGuard guard(u_.device());
+  const Tensor Dv = opt(D_), zv = opt(z_), hv = opt(h0_);
+  const bool needs_grad = at::GradMode::is_enabled() &&
+                          (wants_grad(u_) || wants_grad(delta_) || wants_grad(rho_) || wants_grad(theta_) || wants_grad(Bc) ||
+                           wants_grad(Cc) || wants_grad(Dv) || wants_grad(zv) || wants_grad(hv));
+  Tensor y, hL;
+  std::shared_ptr<ComplexNode> node;
+  {
+    at::NoGradGuard no_grad;
+    const Tensor u = dense(u_), delta = dense(delta_);
+    const int64_t b = u.size(0), d = u.size(1), l = u.size(2);
+    const Tensor rho = f32(rho_, "rho", {b, d, l}), theta = f32(theta_, "theta", {b, d, l});
+    const Tensor B = complex_rows(Bc, "B", b, l, u.scalar_type()), C = complex_rows(Cc, "C", b, l, u.scalar_type());
+    const int64_t n = B.size(1);
+    if (C.size(1) != n) fail("B and C must have the same state size");
+    const Tensor D = f32(Dv, "D", {d}), z = f32(zv, "z", {b, d, l}), h0 = check_h0(hv, b, d, n);
+    if (needs_grad && n > AUSSM_MAX_STATE)
+      fail("the complex backward pass supports at most ", AUSSM_MAX_STATE, " states per channel");
+    const int dt = in_dtype(u), ck = needs_grad ? REC_CK : TILE;
+    y = empty_f32({b, d, l}, u);
+    if (want_state) hL = empty_f32({b, d, n, 2}, u);
+    const Tensor hck = needs_grad ? empty_f32({b, (l + ck - 1) / ck, n, 2, d}, u) : Tensor();
+    const Tensor ws = workspace(VAR_COMPLEX, u, b, d, n, l, ck, dt);
+    check(aussm_complex_fwd(ptr(u), ptr(delta), ptr(rho), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(z), ptr(h0), ptr(y), ptr(hL), ptr(hck),
+                            ptr(ws), b, d, n, l, ck, dt, cur_stream()),
+          "aussm_complex_fwd");
+    if (needs_grad) {
+      node = make_node<ComplexNode>();
+      node->set_next_edges(torch::autograd::collect_next_edges(u_, delta_, rho_, theta_, Bc, Cc, Dv, hv, zv));
+      node->save({u, delta, rho, theta, B, C, D, h0, z, hck});
+      node->b = b; node->d = d; node->n = n; node->l = l; node->dt = dt;
+      node->bc_complex = Bc.is_complex();
+    }
+    if (want_state) hL = at::view_as_complex(hL);
+  }
+  if (node) {
+    torch::autograd::set_history(y, node);
+    if (want_state) torch::autograd::set_history(hL, node);
+  }
+  return {y, hL};
+}
+
+// ============================================================================ real (S6)
+
+namespace {
+
+struct RealNode : SavingNode {
+  int b, d, n, l, dt, softplus;
+  std::string name() const override { return "AussmSelectiveScanBackward"; }
+  variable_list apply(variable_list&& g) override;
+};
+
+enum { R_U, R_DELTA, R_A, R_B, R_C, R_D, R_BIAS, R_H0, R_Z, R_INPUTS };
+
+variable_list RealNode::apply(variable_list&& g) {
+  std::lock_guard<std::mutex> lock(mutex_);
+  at::NoGradGuard no_grad;
+  variable_list out(R_INPUTS);
+  if (!g[0].defined() && !(g.size() > 1 && g[1].defined())) return out;
+  const Tensor u = saved[0].unpack(), delta = saved[1].unpack(), A = saved[2].unpack(), B = saved[3].unpack(), C = saved[4].unpack(),
+               D = saved[5].unpack(), bias = saved[6].unpack(), h0 = saved[7].unpack(), z = saved[8].unpack(), hck = saved[9].unpack();
+  const c10::DeviceGuard guard(u.device());
+  const Tensor dy = g[0].defined() ? dense(g[0]) : at::zeros({b, d, l}, A.options());
+  const Tensor dhL = g.size() > 1 ? dense(g[1]) : Tensor();
+  Tensor du = empty_f32({b, d, l}, u), ddelta = empty_f32({b, d, l}, u), dz = z.defined() ? empty_f32({b, d, l}, u) : Tensor();
+  const bool want_dD = D.defined() && task_should_compute_output(R_D);
+  const bool want_dh0 = h0.defined() && task_should_compute_output(R_H0);
+  Acc acc;
+  const int iA = acc.add((int64_t)d * n), iB = acc.add((int64_t)b * n * l), iC = acc.add((int64_t)b * n * l), iD = want_dD ? acc.add(d) : 0;
+  acc.make(u);
+  Tensor dA = acc.part(iA, {d, n}), dB = acc.part(iB, {b, n, l}), dC = acc.part(iC, {b, n, l}), dD = want_dD ? acc.part(iD, {d}) : Tensor();
+  Tensor dh0 = want_dh0 ? empty_f32({b, d, n}, u) : Tensor();
+  const Tensor ws = workspace(VAR_REAL, u, b, d, n, l, REC_CK, dt);
+  check(aussm_real_bwd(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(A), ptr(B), ptr(C), ptr(D), ptr(bias), softplus, ptr(h0), ptr(hck),
+                       ptr(du), ptr(ddelta), ptr(dA), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), ptr(z), ptr(dz), ptr(ws), b, d, n, l, REC_CK, dt,
+                       cur_stream()),
+        "aussm_real_bwd");
+  if (bias.defined() && task_should_compute_output(R_BIAS)) out[R_BIAS] = ddelta.sum(at::IntArrayRef({0, 2}));
+  out[R_U] = as_like(du, false, u.scalar_type());
+  out[R_DELTA] = as_like(ddelta, false, u.scalar_type());
+  out[R_A] = dA;
+  out[R_B] = as_like(dB, false, u.scalar_type());
+  out[R_C] = as_like(dC, false, u.scalar_type());
+  if (want_dD) out[R_D] = dD;
+  if (want_dh0) out[R_H0] = dh0;
+  if (z.defined()) out[R_Z] = dz;
+  return out;
+}
+
+}  // namespace
+
+std::pair<Tensor, Tensor> selective_scan(const Tensor& u_, const Tensor& delta_, const Tensor& A_, const Tensor& B_, const Tensor& C_,
+                                         const OptTensor& D_, const OptTensor& z_, const OptTensor& bias_, bool softplus, bool want_state,
+                                         const OptTensor& h0_) {
+  check_bdl(u_, delta_);
+  const c10::DeviceGuard guard(u_.device());
+  const Tensor Dv = opt(D_), zv = opt(z_), bv = opt(bias_), hv = opt(h0_);
+  const bool needs_grad = at::GradMode::is_enabled() &&
+                          (wants_grad(u_) || wants_grad(delta_) || wants_grad(A_) || wants_grad(B_) || wants_grad(C_) ||
+                           wants_grad(Dv) || wants_grad(zv) || wants_grad(bv) || wants_grad(hv));
+  Tensor y, hL;
+  std::shared_ptr<RealNode> node;
+  {
+    at::NoGradGuard no_grad;
+    const Tensor u = dense(u_), delta = dense(delta_);
+    const int64_t b = u.size(0), d = u.size(1), l = u.size(2);
+    if (A_.scalar_type() != at::kFloat) fail("expected A to be float32, got torch.", A_.scalar_type());
+    if (A_.dim() != 2 || A_.size(0) != d) fail("expected A of shape (d, n) with d = ", d, ", got ", shape_str(A_.sizes()));
+    const Tensor A = dense(A_);
+    const int64_t n = A.size(1);
+    auto rows = [&](const Tensor& t, const char* name) {
+      if (t.sizes() != at::IntArrayRef({b, n, l})) fail("expected ", name, " of shape ", shape_str({b, n, l}), ", got ", shape_str(t.sizes()));
+      if (t.scalar_type() != u.scalar_type()) fail(name, " must have the dtype of u (torch.", u.scalar_type(), "), got torch.", t.scalar_type());
+      return dense(t);
+    };
+    const Tensor B = rows(B_, "B"), C = rows(C_, "C");
+    const Tensor D = f32(Dv, "D", {d}), z = f32(zv, "z", {b, d, l}), bias = f32(bv, "delta_bias", {d}), h0 = f32(hv, "h0", {b, d, n});
+    if (needs_grad && n > AUSSM_MAX_STATE) fail("the S6 backward pass supports at most ", AUSSM_MAX_STATE, " states per channel");
+    const int dt = in_dtype(u), ck = needs_grad ? REC_CK : TILE;
+    y = empty_f32({b, d, l}, u);
+    if (want_state) hL = empty_f32({b, d, n}, u);
+    const Tensor hck = needs_grad ? empty_f32({b, (l + ck - 1) / ck, n, 1, d}, u) : Tensor();
+    const Tensor ws = workspace(VAR_REAL, u, b, d, n, l, ck, dt);
+    check(aussm_real_fwd(ptr(u), ptr(delta), ptr(A), ptr(B), ptr(C), ptr(D), ptr(z), ptr(bias), softplus, ptr(h0), ptr(y), ptr(hL), ptr(hck),
+                         ptr(ws), b, d, n, l, ck, dt, cur_stream()),
+          "aussm_real_fwd");
+    if (needs_grad) {
+      node = make_node<RealNode>();
+      node->set_next_edges(torch::autograd::collect_next_edges(u_, delta_, A_, B_, C_, Dv, bv, hv, zv));
+      node->save({u, delta, A, B, C, D, bias, h0, z, hck});
+      node->b = b; node->d = d; node->n = n; node->l = l; node->dt = dt; node->softplus = softplus;
+    }
+  }
+  if (node) {
+    torch::autograd::set_history(y, node);
+    if (want_state) torch::autograd::set_history(hL, node);
+  }
+  return {y, hL};
+}
+
+}  // namespace aussm_host

@@ -1,116 +1,11 @@
-// Translation unit of the vector-ALU kernels: the three forward scans, the unitary reverse scan,
-// the recomputing reverse scans (complex, real), the causal convolution and the layout swap.
+// Translation unit of the kernels around the vector-ALU scans: their split along the sequence, the causal convolution,
+// the layout swap, the gate.
 #include "conv1d.h"
 #include "launch.h"
 #include "layout.h"
-#include "scan_bwd_recompute.h"
-#include "scan_bwd_unitary.h"
-#include "scan_fwd.h"
 #include "scan_seg_generic.h"
 
 namespace aussm {
-
-#define AUSSM_FWD_CASE(NW_, NT_)                                                                     \
-  if (c.nw == NW_ && c.nt == NT_) {                                                                  \
-    hipLaunchKernelGGL((core_fwd_kernel<VAR, NW_, NT_, Tin, Tbc>), grid, dim3(NT_), 0, s, a);        \
-    return launch_status();                                                                          \
-  }
-
-// in_dtype of the launch functions below: 0 float, 1 bf16, 2 (complex and real scans only, which take no
-// bf16 B_t / C_t) u and delta bf16 with B_t / C_t already converted to float
-constexpr int IN_BF16_BC32 = 2;
-
-template <int VAR, typename Tin, typename Tbc>
-static int core_fwd_t(const FwdArgs& a, Cfg c, hipStream_t s) {
-  const dim3 grid((unsigned)(a.B * a.ncg));
-  AUSSM_FWD_CASE(1, 256) AUSSM_FWD_CASE(2, 256) AUSSM_FWD_CASE(4, 256) AUSSM_FWD_CASE(8, 256)
-  AUSSM_FWD_CASE(16, 256) AUSSM_FWD_CASE(1, 512) AUSSM_FWD_CASE(2, 512) AUSSM_FWD_CASE(4, 512)
-  AUSSM_FWD_CASE(8, 512)
-  return -2;
-}
-
-template <int VAR>
-static int core_fwd_v(const FwdArgs& a, int in_dtype, Cfg c, hipStream_t s) {
-  if (in_dtype == 0) return core_fwd_t<VAR, float, float>(a, c, s);
-  if constexpr (VAR == VAR_UNITARY) {
-    if (in_dtype == 1) return core_fwd_t<VAR, bf16_t, bf16_t>(a, c, s);
-  } else {
-    if (in_dtype == IN_BF16_BC32) return core_fwd_t<VAR, bf16_t, float>(a, c, s);
-  }
-  return -2;
-}
-
-int run_core_fwd(int variant, const FwdArgs& a, int in_dtype, Cfg c, hipStream_t s) {
-  if (variant == VAR_UNITARY) return core_fwd_v<VAR_UNITARY>(a, in_dtype, c, s);
-  if (variant == VAR_COMPLEX) return core_fwd_v<VAR_COMPLEX>(a, in_dtype, c, s);
-  return core_fwd_v<VAR_REAL>(a, in_dtype, c, s);
-}
-
-// The backward workgroup keeps a (dw, dtheta) slab per wavefront in LDS: four wavefronts afford
-// 32-step tiles, eight wavefronts 16-step tiles.
-#define AUSSM_UBWD_CASE(NW_, NT_, TT_)                                                               \
-  if (c.nw == NW_ && c.nt == NT_) {                                                                  \
-    hipLaunchKernelGGL((unitary_bwd_kernel<NW_, NT_, TT_, Tin>), grid, dim3(NT_), 0, s, a);          \
-    return launch_status();                                                                          \
-  }
-
-template <typename Tin>
-static int unitary_bwd_t(const UniBwdArgs& a, Cfg c, hipStream_t s) {
-  const dim3 grid((unsigned)(a.B * a.ncg));
-  AUSSM_UBWD_CASE(1, 256, 32) AUSSM_UBWD_CASE(2, 256, 32) AUSSM_UBWD_CASE(4, 256, 32)
-  AUSSM_UBWD_CASE(8, 256, 32) AUSSM_UBWD_CASE(16, 256, 32)
-  AUSSM_UBWD_CASE(1, 512, 16) AUSSM_UBWD_CASE(2, 512, 16) AUSSM_UBWD_CASE(4, 512, 16)
-  AUSSM_UBWD_CASE(8, 512, 16)
-  return -2;
-}
-
-int run_unitary_bwd_generic(const UniBwdArgs& a, int in_dtype, Cfg c, hipStream_t s) {
-  return in_dtype == 1 ? unitary_bwd_t<bf16_t>(a, c, s) : unitary_bwd_t<float>(a, c, s);
-}
-
-#define AUSSM_RBWD_CASE(NW_)                                                                         \
-  if (nw == NW_) {                                                                                   \
-    hipLaunchKernelGGL((recompute_bwd_kernel<VAR, NW_, 256, Tin, float>), grid, dim3(256), 0, s, a); \
-    done = true;                                                                                     \
-  }
-
-template <int VAR, typename Tin>
-static int rec_bwd_t(const RecBwdArgs& args, hipStream_t s) {
-  const dim3 grid((unsigned)(args.B * args.ncg));
-  // one launch per block of 16 states (stream order makes the later blocks' additions safe)
-  for (int nbase = 0; nbase < args.N; nbase += 16) {
-    RecBwdArgs a = args;
-    a.nbase = nbase;
-    a.accum = nbase > 0;
-    const int left = args.N - nbase;
-    const int nw = left <= 4 ? 1 : (left <= 8 ? 2 : 4);
-    bool done = false;
-#ifndef AUSSM_REC_NARROW
-    // a full block of 16 states: eight wavefronts of two states, two wavefronts per SIMD (the complex scan with a
-    // gate gradient to return keeps a fourth partial sum per wavefront)
-    if (left > 8) {
-      if constexpr (VAR == VAR_COMPLEX) {
-        if (a.dz) hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, true>), grid, dim3(512), 0, s, a);
-        else hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, false>), grid, dim3(512), 0, s, a);
-      } else {
-        hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float>), grid, dim3(512), 0, s, a);
-      }
-      done = true;
-    }
-#endif
-    if (!done) { AUSSM_RBWD_CASE(1) AUSSM_RBWD_CASE(2) AUSSM_RBWD_CASE(4) }
-    if (!done) return -2;
-    if (int e = launch_status()) return e;
-  }
-  return 0;
-}
-
-int run_rec_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s) {
-  if (in_dtype != 0 && in_dtype != IN_BF16_BC32) return -2;      // B_t / C_t are float in every instance
-  if (variant == VAR_COMPLEX)
-    return in_dtype ? rec_bwd_t<VAR_COMPLEX, bf16_t>(a, s) : rec_bwd_t<VAR_COMPLEX, float>(a, s);
-  return in_dtype ? rec_bwd_t<VAR_REAL, bf16_t>(a, s) : rec_bwd_t<VAR_REAL, float>(a, s);
-}
 
 int run_adjoint_seg(int variant, const AdjSegArgs& a, int in_dtype, unsigned grid, hipStream_t s) {
   // (B_t / C_t are float in every instance of the complex and real scans; the complex kernel reads no u / delta
@@ -247,6 +142,13 @@ int run_conv_bwd(const ConvArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(causal_conv1d_bwd_data_kernel, dim3((unsigned)rows, (unsigned)((a.D + 255) / 256)), dim3(256), 0, s, a);
     hipLaunchKernelGGL(causal_conv1d_bwd_weight_kernel, wgrid, dim3(256), 0, s, a);
   }
+  return launch_status();
+}
+
+int run_zero(float* p, size_t n, hipStream_t s) {
+  const size_t blocks = (n + 1023) / 1024;
+  hipLaunchKernelGGL(zero_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, s, p, n,
+                     (reinterpret_cast<uintptr_t>(p) & 15) == 0);
   return launch_status();
 }
 

@@ -18,8 +18,10 @@ inline int launch_status() {
 // wavefront owns nw states.
 struct Cfg { int nw, nt; };
 
-// ---- k_generic.hip: vector-ALU scans, convolution, layout swap
-// in_dtype: 0 float, 1 bf16 (unitary only), 2 = u / delta bf16 and B_t / C_t float (complex and real only)
+// ---- k_fwd.hip, k_ubwd.hip, k_rbwd.hip: vector-ALU scans; k_generic.hip: their split along L, convolution, layout swap
+// in_dtype: 0 float, 1 bf16 (unitary only), 2 = u / delta bf16 and B_t / C_t float (complex and real only, whose
+// kernels take no bf16 B_t / C_t: converted to float once per call)
+constexpr int IN_BF16_BC32 = 2;
 int run_core_fwd(int variant, const FwdArgs& a, int in_dtype, Cfg c, hipStream_t s);
 int run_unitary_bwd_generic(const UniBwdArgs& a, int in_dtype, Cfg c, hipStream_t s);
 int run_rec_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s);
@@ -33,6 +35,7 @@ int run_hbm_probe(const float* a, const float* b, const float* c, float* o1, flo
                   int write, hipStream_t s);
 int run_conv_fwd(const ConvArgs& a, hipStream_t s);
 int run_conv_bwd(const ConvArgs& a, hipStream_t s);
+int run_zero(float* p, size_t n, hipStream_t s);
 int run_swap_last2(const SwapArgs& a, int B, hipStream_t s);
 // dz null: out = ypre silu(z); else out = dy silu(z), dz = dy ypre silu'(z)
 int run_gate(const float* dy, const float* ypre, const float* z, float* out, float* dz, size_t n, hipStream_t s);

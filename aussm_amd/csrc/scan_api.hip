@@ -673,6 +673,12 @@ int aussm_gate_bwd(const float* dy, const float* y_pre, const float* z, float* d
   return run_gate(dy, y_pre, z, dy_pre, dz, n, (hipStream_t)stream);
 }
 
+int aussm_zero_f32(float* p, size_t n, void* stream) {
+  if (!p) return AUSSM_E_NULL;
+  if (misaligned(p, 4)) return AUSSM_E_ALIGN;
+  return n ? run_zero(p, n, (hipStream_t)stream) : AUSSM_OK;
+}
+
 // ---- the reference's operator extension_cpp::ssm_adaptive_unitary as fused kernels (dropin.h)
 
 // blocks of 16 states per channel, one per wavefront: 1, 2 or 4 (they have to divide the wavefronts of a workgroup)

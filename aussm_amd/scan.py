@@ -1,4 +1,6 @@
-"""Core selective scans on MI355X: Python host over the C ABI of libaussm_hip.so.
+"""Core selective scans on MI355X, over the C ABI of libaussm_hip.so.  The three operators run through the native host
+path (csrc/host/scans.cpp: checks, allocation, launches, autograd nodes); the raw launches further down are the same
+entry points without autograd.
 
 Three operators, each differentiable through torch.autograd:
 
@@ -47,14 +49,9 @@ def unitary_ck(b: int, d: int, n: int, l: int) -> int:
     lets a launch with few (batch, channel) pairs be split into more segments along L (a segment
     is a whole number of checkpoint blocks); calls that are not split at all checkpoint every
     UNITARY_CK_LONG steps (one checkpoint, at the end, for shorter sequences)."""
-    lib = _lib.load()
-    half = UNITARY_CK // 2
-    s_half, s_full = (lib.aussm_unitary_split_segments(b, d, n, l, ck) for ck in (half, UNITARY_CK))
-    if s_half > s_full:
-        return half
-    if s_full <= 1:
-        return min(UNITARY_CK_LONG, -(-l // _lib.TILE) * _lib.TILE)
-    return UNITARY_CK
+    return _lib.host().unitary_ck(b, d, n, l)
+
+
 TILE_CK = _lib.TILE
 
 
@@ -68,39 +65,6 @@ def _in_dtype(t: Tensor) -> int:
     if t.dtype == torch.bfloat16:
         return _lib.BF16
     raise RuntimeError(f"expected float32 or bfloat16 scan input, got {t.dtype}")
-
-
-def _f32(t: Optional[Tensor], name: str, shape=None) -> Optional[Tensor]:
-    if t is None:
-        return None
-    if t.dtype != torch.float32:
-        raise RuntimeError(f"expected {name} to be float32, got {t.dtype}")
-    if shape is not None and tuple(t.shape) != tuple(shape):
-        raise RuntimeError(f"expected {name} of shape {tuple(shape)}, got {tuple(t.shape)}")
-    return t.contiguous()
-
-
-def _check_bdl(u: Tensor, delta: Tensor):
-    if u.dim() != 3:
-        raise RuntimeError(f"expected u of shape (b, d, l), got {tuple(u.shape)}")
-    if not u.is_cuda:
-        raise RuntimeError("scan inputs must be on the GPU (no CPU implementation is shipped)")
-    if delta.shape != u.shape or delta.dtype != u.dtype:
-        raise RuntimeError("delta must match u in shape and dtype")
-    return u.shape
-
-
-def _complex_as_real(t: Tensor, name: str, b: int, l: int, dtype: torch.dtype) -> Tensor:
-    """(b, n, l) complex64 or (b, n, l, 2) real -> contiguous real (b, n, l, 2) of `dtype`."""
-    if t.is_complex():
-        if t.dtype != torch.complex64:
-            raise RuntimeError(f"expected {name} to be complex64, got {t.dtype}")
-        t = torch.view_as_real(t)
-    if t.dim() != 4 or t.shape[0] != b or t.shape[2] != l or t.shape[3] != 2:
-        raise RuntimeError(f"expected {name} of shape (b, n, l) complex or (b, n, l, 2), got {tuple(t.shape)}")
-    if t.dtype != dtype:
-        raise RuntimeError(f"{name} must have the dtype of u ({dtype}), got {t.dtype}")
-    return t.contiguous()
 
 
 def num_checkpoints(L: int, ck: int) -> int:
@@ -177,64 +141,6 @@ def unitary_bwd_raw(dy, dhL, u, delta, theta, Bri, Cri, D, hck, ck, want_dD=True
     return du, ddelta, dtheta, dB, dC, dD, dh0
 
 
-# --------------------------------------------------------------------------------------------
-# autograd
-# --------------------------------------------------------------------------------------------
-
-class _UnitaryScanFn(torch.autograd.Function):
-    """y, hL = scan(u, delta, theta, B, C, D, h0) with all tensors real (complex ones as (..., 2))."""
-
-    @staticmethod
-    def forward(ctx, u, delta, theta, Bri, Cri, D, h0):
-        ck = unitary_ck(theta.shape[0], theta.shape[1], Bri.shape[1], theta.shape[2])
-        b, d, l = theta.shape
-        n = Bri.shape[1]
-        aux = unitary_aux(theta, n, ck) if unitary_aux_useful(b, d, n, l, ck, _in_dtype(u), b // u.shape[0]) else None
-        y, hL, hck = unitary_fwd_raw(u, delta, theta, Bri, Cri, D, None, h0, want_state=True, ck=ck, aux=aux)
-        ctx.save_for_backward(u, delta, theta, Bri, Cri, D, hck, aux)
-        ctx.ck = ck
-        ctx.has_h0 = h0 is not None
-        return y, hL
-
-    @staticmethod
-    def backward(ctx, dy, dhL):
-        u, delta, theta, Bri, Cri, D, hck, aux = ctx.saved_tensors
-        dy = dy.contiguous()
-        dhL = None if dhL is None else dhL.contiguous()
-        du, ddelta, dtheta, dB, dC, dD, dh0 = unitary_bwd_raw(
-            dy, dhL, u, delta, theta, Bri, Cri, D, hck, ctx.ck,
-            want_dD=D is not None and ctx.needs_input_grad[5], want_dh0=ctx.has_h0 and ctx.needs_input_grad[6],
-            aux=aux)
-        if u.shape[0] != theta.shape[0]:             # u, delta shared by consecutive batch elements
-            du = du.view(u.shape[0], -1, *u.shape[1:]).sum(dim=1)
-            ddelta = ddelta.view(u.shape[0], -1, *u.shape[1:]).sum(dim=1)
-        return (du.to(u.dtype), ddelta.to(delta.dtype), dtheta, dB.to(Bri.dtype), dC.to(Cri.dtype), dD, dh0)
-
-
-class _GateFn(torch.autograd.Function):
-    """y = y_pre silu(z) behind the unitary scan, whose backward kernels take the gradient of the ungated output:
-    one pass forward, one backward (dy_pre = dy silu(z), dz = dy y_pre silu'(z)); reference
-    extension-cpp/extension_cpp/ops.py:226."""
-
-    @staticmethod
-    def forward(ctx, y_pre, z):
-        lib = _lib.load()
-        y_pre = y_pre.contiguous()
-        y = torch.empty_like(y_pre)
-        check(lib.aussm_gate_fwd(ptr(y_pre), ptr(z), ptr(y), y_pre.numel(), _stream()), "aussm_gate_fwd")
-        ctx.save_for_backward(y_pre, z)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        lib = _lib.load()
-        y_pre, z = ctx.saved_tensors
-        dy = dy.contiguous()
-        dy_pre, dz = torch.empty_like(y_pre), torch.empty_like(z)
-        check(lib.aussm_gate_bwd(ptr(dy), ptr(y_pre), ptr(z), ptr(dy_pre), ptr(dz), dy.numel(), _stream()), "aussm_gate_bwd")
-        return dy_pre, dz
-
-
 def unitary_scan(u: Tensor, delta: Tensor, theta: Tensor, Bc: Tensor, Cc: Tensor, D: Optional[Tensor] = None,
                  z: Optional[Tensor] = None, h0: Optional[Tensor] = None, return_last_state: bool = False):
     """Adaptive-unitary scan.  u, delta, theta, z: (b, d, l); Bc, Cc: (b, n, l) complex64 (or
@@ -242,45 +148,7 @@ def unitary_scan(u: Tensor, delta: Tensor, theta: Tensor, Bc: Tensor, Cc: Tensor
     state (b, d, n) complex64 if return_last_state.  u and delta may be (b / r, d, l): batch element i
     of theirs then serves the r consecutive batch elements i r .. i r + r - 1 of everything else
     (one input, r phase sequences)."""
-    bu, d, l = _check_bdl(u, delta)
-    u = u.contiguous()
-    delta = delta.contiguous()
-    b = theta.shape[0] if theta.dim() == 3 else bu
-    if b % bu != 0:
-        raise RuntimeError(f"batch size of theta ({b}) must be a multiple of that of u ({bu})")
-    theta = _f32(theta, "theta", (b, d, l))
-    Bri = _complex_as_real(Bc, "B", b, l, u.dtype)
-    Cri = _complex_as_real(Cc, "C", b, l, u.dtype)
-    n = Bri.shape[1]
-    if Cri.shape[1] != n:
-        raise RuntimeError("B and C must have the same state size")
-    D = _f32(D, "D", (d,))
-    z = _f32(z, "z", (b, d, l))
-    h0r = None
-    if h0 is not None:
-        if h0.dtype != torch.complex64 or tuple(h0.shape) != (b, d, n):
-            raise RuntimeError(f"expected h0 complex64 of shape {(b, d, n)}")
-        h0r = torch.view_as_real(h0).contiguous()
-    needs_grad = torch.is_grad_enabled() and any(
-        t is not None and t.requires_grad for t in (u, delta, theta, Bri, Cri, D, z, h0r))
-    if needs_grad:
-        y, hL = _UnitaryScanFn.apply(u, delta, theta, Bri, Cri, D, h0r)
-        if z is not None:
-            y = _GateFn.apply(y, z)
-    else:
-        # no backward pass: the auxiliary buffer serves as workspace only (prepared operands of the
-        # matrix-core kernels, segment states of a launch that is split along L); no checkpoints are kept
-        lib = _lib.load()
-        ck = unitary_ck(b, d, n, l)
-        # (the buffer of a shape that the matrix-core kernels serve starts with b d l floats that only a backward
-        # call would read; anything beyond them - segment states, operand images - is workspace of this call)
-        work = lib.aussm_unitary_aux_floats(b, d, n, l, ck) - _lib.AUX_PAD not in (0, b * d * l)
-        aux = unitary_aux(theta, n, ck) if (work and u.shape[0] == b) else None
-        y, hL, _ = unitary_fwd_raw(u, delta, theta, Bri, Cri, D, z, h0r, want_state=return_last_state,
-                                   ck=0, aux=aux, ck_arg=ck if aux is not None else 0)
-    if return_last_state:
-        return y, torch.view_as_complex(hL)
-    return y
+    return _lib.host().unitary_scan(u, delta, theta, Bc, Cc, D, z, h0, return_last_state)
 
 
 # --------------------------------------------------------------------------------------------
@@ -333,57 +201,11 @@ def complex_bwd_raw(dy, dhL, u, delta, rho, theta, Bri, Cri, D, h0, hck, want_dD
     return du, ddelta, drho, dtheta, dB, dC, dD, dh0, dz
 
 
-class _ComplexScanFn(torch.autograd.Function):
-    """The gate z (optional) is applied by the forward kernel and differentiated by the backward kernel."""
-
-    @staticmethod
-    def forward(ctx, u, delta, rho, theta, Bri, Cri, D, h0, z):
-        y, hL, hck = complex_fwd_raw(u, delta, rho, theta, Bri, Cri, D, z, h0, want_state=True, ck=REC_CK)
-        ctx.save_for_backward(u, delta, rho, theta, Bri, Cri, D, h0, hck, z)
-        return y, hL
-
-    @staticmethod
-    def backward(ctx, dy, dhL):
-        u, delta, rho, theta, Bri, Cri, D, h0, hck, z = ctx.saved_tensors
-        dhL = None if dhL is None else dhL.contiguous()
-        du, ddelta, drho, dtheta, dB, dC, dD, dh0, dz = complex_bwd_raw(
-            dy.contiguous(), dhL, u, delta, rho, theta, Bri, Cri, D, h0, hck,
-            want_dD=D is not None and ctx.needs_input_grad[6], want_dh0=h0 is not None and ctx.needs_input_grad[7], z=z)
-        return (du.to(u.dtype), ddelta.to(delta.dtype), drho, dtheta, dB.to(Bri.dtype), dC.to(Cri.dtype), dD, dh0, dz)
-
-
 def complex_scan(u: Tensor, delta: Tensor, rho: Tensor, theta: Tensor, Bc: Tensor, Cc: Tensor,
                  D: Optional[Tensor] = None, z: Optional[Tensor] = None, h0: Optional[Tensor] = None,
                  return_last_state: bool = False):
     """Complex scan, a_l = exp(rho_l + i theta_l).  Shapes as unitary_scan plus rho (b, d, l)."""
-    b, d, l = _check_bdl(u, delta)
-    u = u.contiguous()
-    delta = delta.contiguous()
-    rho = _f32(rho, "rho", (b, d, l))
-    theta = _f32(theta, "theta", (b, d, l))
-    Bri = _complex_as_real(Bc, "B", b, l, u.dtype)
-    Cri = _complex_as_real(Cc, "C", b, l, u.dtype)
-    n = Bri.shape[1]
-    if Cri.shape[1] != n:
-        raise RuntimeError("B and C must have the same state size")
-    D = _f32(D, "D", (d,))
-    z = _f32(z, "z", (b, d, l))
-    h0r = None
-    if h0 is not None:
-        if h0.dtype != torch.complex64 or tuple(h0.shape) != (b, d, n):
-            raise RuntimeError(f"expected h0 complex64 of shape {(b, d, n)}")
-        h0r = torch.view_as_real(h0).contiguous()
-    needs_grad = torch.is_grad_enabled() and any(
-        t is not None and t.requires_grad for t in (u, delta, rho, theta, Bri, Cri, D, z, h0r))
-    if needs_grad:
-        if n > REC_MAX_STATE:
-            raise RuntimeError(f"the complex backward pass supports at most {REC_MAX_STATE} states per channel")
-        y, hL = _ComplexScanFn.apply(u, delta, rho, theta, Bri, Cri, D, h0r, z)
-    else:
-        y, hL, _ = complex_fwd_raw(u, delta, rho, theta, Bri, Cri, D, z, h0r, want_state=return_last_state)
-    if return_last_state:
-        return y, torch.view_as_complex(hL)
-    return y
+    return _lib.host().complex_scan(u, delta, rho, theta, Bc, Cc, D, z, h0, return_last_state)
 
 
 # --------------------------------------------------------------------------------------------
@@ -426,28 +248,6 @@ def real_bwd_raw(dy, dhL, u, delta, A, Bm, Cm, D, delta_bias, delta_softplus, h0
     return du, ddelta, dA, dB, dC, dD, dh0, dz
 
 
-class _RealScanFn(torch.autograd.Function):
-    """The gate z (optional) is applied by the forward kernel and differentiated by the backward kernel."""
-
-    @staticmethod
-    def forward(ctx, u, delta, A, Bm, Cm, D, delta_bias, h0, delta_softplus, z):
-        y, hL, hck = real_fwd_raw(u, delta, A, Bm, Cm, D, z, delta_bias, delta_softplus, h0,
-                                  want_state=True, ck=REC_CK)
-        ctx.save_for_backward(u, delta, A, Bm, Cm, D, delta_bias, h0, hck, z)
-        ctx.delta_softplus = delta_softplus
-        return y, hL
-
-    @staticmethod
-    def backward(ctx, dy, dhL):
-        u, delta, A, Bm, Cm, D, delta_bias, h0, hck, z = ctx.saved_tensors
-        dhL = None if dhL is None else dhL.contiguous()
-        du, ddelta, dA, dB, dC, dD, dh0, dz = real_bwd_raw(
-            dy.contiguous(), dhL, u, delta, A, Bm, Cm, D, delta_bias, ctx.delta_softplus, h0, hck,
-            want_dD=D is not None and ctx.needs_input_grad[5], want_dh0=h0 is not None and ctx.needs_input_grad[7], z=z)
-        dbias = ddelta.sum(dim=(0, 2)) if (delta_bias is not None and ctx.needs_input_grad[6]) else None
-        return (du.to(u.dtype), ddelta.to(delta.dtype), dA, dB.to(Bm.dtype), dC.to(Cm.dtype), dD, dbias, dh0, None, dz)
-
-
 def selective_scan_fn(u: Tensor, delta: Tensor, A: Tensor, B: Tensor, C: Tensor, D: Optional[Tensor] = None,
                       z: Optional[Tensor] = None, delta_bias: Optional[Tensor] = None,
                       delta_softplus: bool = False, return_last_state: bool = False,
@@ -461,32 +261,4 @@ def selective_scan_fn(u: Tensor, delta: Tensor, A: Tensor, B: Tensor, C: Tensor,
 
     Returns y (b, d, l) float32, plus the last state (b, d, n) if return_last_state.
     `h0` (b, d, n), a start state, is an extension over the reference's signature."""
-    b, d, l = _check_bdl(u, delta)
-    u = u.contiguous()
-    delta = delta.contiguous()
-    A = _f32(A, "A")
-    if A.dim() != 2 or A.shape[0] != d:
-        raise RuntimeError(f"expected A of shape (d, n) with d = {d}, got {tuple(A.shape)}")
-    n = A.shape[1]
-    for name, t in (("B", B), ("C", C)):
-        if tuple(t.shape) != (b, n, l):
-            raise RuntimeError(f"expected {name} of shape {(b, n, l)}, got {tuple(t.shape)}")
-        if t.dtype != u.dtype:
-            raise RuntimeError(f"{name} must have the dtype of u ({u.dtype}), got {t.dtype}")
-    Bm, Cm = B.contiguous(), C.contiguous()
-    D = _f32(D, "D", (d,))
-    z = _f32(z, "z", (b, d, l))
-    delta_bias = _f32(delta_bias, "delta_bias", (d,))
-    h0 = _f32(h0, "h0", (b, d, n))
-    needs_grad = torch.is_grad_enabled() and any(
-        t is not None and t.requires_grad for t in (u, delta, A, Bm, Cm, D, z, delta_bias, h0))
-    if needs_grad:
-        if n > REC_MAX_STATE:
-            raise RuntimeError(f"the S6 backward pass supports at most {REC_MAX_STATE} states per channel")
-        y, hL = _RealScanFn.apply(u, delta, A, Bm, Cm, D, delta_bias, h0, bool(delta_softplus), z)
-    else:
-        y, hL, _ = real_fwd_raw(u, delta, A, Bm, Cm, D, z, delta_bias, delta_softplus, h0,
-                                want_state=return_last_state)
-    if return_last_state:
-        return y, hL
-    return y
+    return _lib.host().selective_scan(u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus), return_last_state, h0)

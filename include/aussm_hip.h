@@ -322,6 +322,10 @@ int aussm_swap_last2_act(const float* x, const float* bias, const float* pre, fl
 int aussm_gate_fwd(const float* y_pre, const float* z, float* y, size_t n, void* stream);
 int aussm_gate_bwd(const float* dy, const float* y_pre, const float* z, float* dy_pre, float* dz, size_t n, void* stream);
 
+/* Sets n floats to zero with one launch (a kernel, not a memory-set node, so a call may be recorded in a graph):
+ * the buffers that the backward calls above accumulate into. */
+int aussm_zero_f32(float* p, size_t n, void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * The reference's custom operator itself, as two calls: what
  *   torch.ops.extension_cpp.ssm_adaptive_unitary           (12 tensors -> y, next_hid_real, next_hid_imag)
