@@ -52,6 +52,19 @@ _SIGNATURES = {
     "aussm_swap_last2_act": [_P] * 4 + [_I] * 3 + [_LL] * 4 + [_I] * 2 + [_P],
     "aussm_gate_fwd": [_P] * 3 + [ctypes.c_size_t, _P],
     "aussm_gate_bwd": [_P] * 5 + [ctypes.c_size_t, _P],
+    "aussm_operator_fwd": [_P] * 6,
+    "aussm_operator_bwd": [_P] * 9,
+    "aussm_gemm": [_P, _P],
+    "aussm_conv_rows_fwd": [_P] * 4 + [_I] * 4 + [_LL, _P],
+    "aussm_conv_rows_bwd": [_P] * 6 + [_I] * 4 + [_LL] * 2 + [_P],
+    "aussm_rms_norm_fwd": [_P] * 4 + [ctypes.c_size_t, _I, ctypes.c_float, _P],
+    "aussm_rms_norm_bwd": [_P] * 7 + [ctypes.c_size_t, _I, _P],
+    "aussm_col_sum": [_P] * 2 + [ctypes.c_size_t, _I, ctypes.c_float, _P],
+    "aussm_row_sum": [_P] * 2 + [ctypes.c_size_t, _I, _I, ctypes.c_float, _P],
+    "aussm_neg_exp": [_P] * 3 + [_I, _P],
+    "aussm_zero_many": [_P] * 2 + [_I, _P],
+    "aussm_real_fwd_rows": [_P] * 8 + [_I] + [_P] * 6 + [_I] * 6 + [_P],
+    "aussm_real_bwd_rows": [_P] * 9 + [_I] + [_P] * 13 + [_I] * 6 + [_P],
     "aussm_zero_f32": [_P, ctypes.c_size_t, _P],
     "aussm_hbm_probe": [_P] * 5 + [_I] * 4 + [_P],
     "aussm_ssm_adaptive_unitary_fwd": [_P] * 16 + [_I] * 4 + [_P],
@@ -63,6 +76,14 @@ EXPORTED = tuple(_SIGNATURES) + ("aussm_error_string", "aussm_unitary_aux_floats
 
 
 OPT_UNITARY_FWD, OPT_UNITARY_BWD, OPT_SPLIT_CAP, OPT_GENERIC_NW, OPT_GENERIC_NT, OPT_BLOCK_KFLOATS = range(6)
+
+
+class GemmArgs(ctypes.Structure):
+    """aussm_gemm_args of include/aussm_hip.h."""
+    _fields_ = ([(k, _P) for k in ("A", "B", "C", "bias", "add")] + [("alpha", ctypes.c_float), ("bias_scale", ctypes.c_float)]
+                + [(k, _I) for k in ("act", "reduce")]
+                + [(k, _LL) for k in ("sam", "sak", "saz", "sbk", "sbn", "sbb", "sbz", "scm", "scn", "scb")]
+                + [(k, _I) for k in ("M", "N", "K", "Z", "nper")])
 
 
 class AussmError(RuntimeError):

@@ -14,6 +14,11 @@ input length (:863).
 
 Every block takes an optional `scan_impl` callable.  The default is the HIP operator; tests
 pass a CPU implementation with the same signature to check the plumbing around the scan.
+
+On the GPU, in float32 and with the default scan, a block (with the norm and the residual around it)
+is ONE node of the autograd graph that runs entirely on the library's kernels (csrc/host/blocks.cpp);
+everything else - an injected scan, tensors on the CPU or of another type, autocast, a layer that was
+replaced or carries hooks - is composed from the separate layers, as the reference composes it.
 """
 from __future__ import annotations
 
@@ -25,7 +30,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import conv, ops, scan
+from . import _lib, conv, ops, scan
 
 
 def _causal_conv(conv1d: nn.Conv1d, x: torch.Tensor, l: int) -> torch.Tensor:
@@ -95,6 +100,34 @@ def _swap(x: torch.Tensor) -> torch.Tensor:
     if x.is_cuda and x.dtype == torch.float32:
         return conv.swap_last2(x)
     return x.transpose(1, 2).contiguous()
+
+
+# ---- the native route -------------------------------------------------------------------------
+
+def _plain(module: nn.Module, cls) -> bool:
+    """A layer whose forward is exactly its class's: what it computes may be done without calling it."""
+    d = module.__dict__
+    return type(module) is cls and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                                        or d["_backward_pre_hooks"]) and "forward" not in d
+
+
+def _native(x: torch.Tensor) -> bool:
+    """Tensors the native route takes at all (it checks the rest itself)."""
+    m = torch.nn.modules.module
+    return (x.is_cuda and x.dtype is torch.float32 and not torch.is_autocast_enabled()
+            and not (m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
+                     or m._global_backward_pre_hooks))
+
+
+def _norm_linear(layer: nn.Linear, x: torch.Tensor, norm: Optional[nn.Module] = None) -> torch.Tensor:
+    """`layer(norm(x))`."""
+    if _native(x) and _plain(layer, nn.Linear) and (norm is None or _plain(norm, RMSNorm)):
+        p = layer._parameters
+        y = _lib.host().norm_linear(x, None if norm is None else norm.weight, 0.0 if norm is None else norm.eps,
+                                    p["weight"], p["bias"])
+        if y is not None:
+            return y
+    return _linear(layer, x if norm is None else norm(x))
 
 
 @dataclass
@@ -168,7 +201,24 @@ class MambaBlock(nn.Module):
         self.A_log._no_weight_decay = True
         self.scan_impl = scan_impl or scan.selective_scan_fn
 
+    def native(self, x: torch.Tensor, norm: Optional[nn.Module] = None, residual: bool = False) -> Optional[torch.Tensor]:
+        """The block (behind `norm`, plus x with `residual`) on the native route, or None where that does not apply."""
+        if (self.scan_impl is not scan.selective_scan_fn or not _native(x) or (norm is not None and not _plain(norm, RMSNorm))):
+            return None
+        mods = self._modules
+        ip, cv, op, xp, dp = (mods[k] for k in ("in_proj", "conv1d", "out_proj", "x_proj", "dt_proj"))
+        if not (_plain(ip, nn.Linear) and _plain(op, nn.Linear) and _plain(xp, nn.Linear) and _plain(dp, nn.Linear)
+                and _plain(cv, nn.Conv1d)) or xp.bias is not None or dp.bias is None or cv.padding[0] != cv.kernel_size[0] - 1:
+            return None
+        i, c, o = ip._parameters, cv._parameters, op._parameters
+        return _lib.host().mamba_block(x, None if norm is None else norm.weight, 0.0 if norm is None else norm.eps, residual,
+                                       i["weight"], i["bias"], c["weight"], c["bias"], xp._parameters["weight"],
+                                       dp._parameters["weight"], dp._parameters["bias"], self.A_log, self.D, o["weight"], o["bias"])
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = self.native(x)
+        if y is not None:
+            return y
         (b, l, d) = x.shape
         x_and_z = _linear(self.in_proj, x)
         (x, z) = x_and_z.split(split_size=[self.args.d_inner, self.args.d_inner], dim=-1)
@@ -221,8 +271,43 @@ class SSMauBlock(nn.Module):
         else:
             # the reference's pure-PyTorch form (aussm.py:842-843): same name, same signature, HIP kernels
             self.optimized_SSMa_function = ops.reference_ssm_adaptive_unitary_optimized_polar
+        self._default_scan = self.optimized_SSMa_function if scan_impl is None else None
+
+    @property
+    def ssm_args(self):
+        """What the last forward pass handed to the scan operator."""
+        if self._ssm_args is None and self._last_input is not None:
+            x, norm = self._last_input
+            x_and_z = _linear(self.in_proj, x if norm is None else norm(x))
+            x, z = x_and_z.split(self.args.d_model, dim=-1)
+            self._ssm_args = self._scan_args(_causal_conv(self.conv1d, x, x.shape[1]), z)
+        return self._ssm_args
+
+    _ssm_args = _last_input = None
+
+    def native(self, x: torch.Tensor, norm: Optional[nn.Module] = None, residual: bool = False) -> Optional[torch.Tensor]:
+        """The block (behind `norm`, plus x with `residual`) on the native route, or None where that does not apply."""
+        if (self._default_scan is None or self.optimized_SSMa_function is not self._default_scan or not self.args.conv_1d
+                or not _native(x) or (norm is not None and not _plain(norm, RMSNorm))):
+            return None
+        mods = self._modules
+        ip, cv, op, xp, dp, xa = (mods[k] for k in ("in_proj", "conv1d", "out_proj", "x_proj", "dt_proj", "xA_proj"))
+        if not (_plain(ip, nn.Linear) and _plain(op, nn.Linear) and _plain(xp, nn.Linear) and _plain(dp, nn.Linear)
+                and _plain(xa, nn.Linear) and _plain(cv, nn.Conv1d)) or xp.bias is not None or dp.bias is None \
+                or xa.bias is None or cv.padding[0] != cv.kernel_size[0] - 1:
+            return None
+        i, c, o, a = ip._parameters, cv._parameters, op._parameters, xa._parameters
+        return _lib.host().aussm_block(x, None if norm is None else norm.weight, 0.0 if norm is None else norm.eps, residual,
+                                       i["weight"], i["bias"], c["weight"], c["bias"], xp._parameters["weight"],
+                                       dp._parameters["weight"], dp._parameters["bias"], a["weight"], a["bias"], self.B, self.C,
+                                       self.D, o["weight"], o["bias"], 1 / math.sqrt(self.args.d_model))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = self.native(x)
+        if y is not None:
+            # (the operator's arguments never exist as tensors of their own here: ssm_args forms them when asked)
+            self._ssm_args, self._last_input = None, (x, None)
+            return y
         (b, l, d) = x.shape
         x_and_z = _linear(self.in_proj, x)
         (x, z) = x_and_z.split(split_size=[self.args.d_model, self.args.d_model], dim=-1)
@@ -231,7 +316,7 @@ class SSMauBlock(nn.Module):
         y = self.ssm_au(x, z)
         return _linear(self.out_proj, y)
 
-    def ssm_au(self, x, z):
+    def _scan_args(self, x, z):
         b, l, d_in = x.shape
         n = self.args.d_state
         dt = _linear(self.dt_proj, _linear(self.x_proj, x))
@@ -239,7 +324,7 @@ class SSMauBlock(nn.Module):
         # "(n dstate1) dstate -> dstate1 n dstate"
         x_param = self.xA_proj.weight.view(n, d_in, d_in).permute(1, 0, 2)
         x_bias = self.xA_proj.bias.view(n, d_in).t()
-        self.ssm_args = {
+        return {
             "u": _swap(x),
             "dt": _swap_act(dt, "softplus", self.dt_proj.bias.float()),
             "x": x_param.contiguous() * (1 / math.sqrt(self.args.d_model)),
@@ -249,7 +334,10 @@ class SSMauBlock(nn.Module):
             "D": self.D.float().contiguous(),
             "z": _swap(z),
         }
-        y = self.optimized_SSMa_function(**self.ssm_args)
+
+    def ssm_au(self, x, z):
+        self._ssm_args, self._last_input = self._scan_args(x, z), None
+        y = self.optimized_SSMa_function(**self._ssm_args)
         return _swap(y)
 
 
@@ -263,6 +351,13 @@ class ResidualBlock(nn.Module):
         self.norm = RMSNorm(args.d_model)
 
     def forward(self, x):
+        # norm, block and residual as one: the block itself must not be hooked either
+        if type(self.mixer) in (SSMauBlock, MambaBlock) and _plain(self.mixer, type(self.mixer)):
+            y = self.mixer.native(x, self.norm, True)
+            if y is not None:
+                if type(self.mixer) is SSMauBlock:
+                    self.mixer._ssm_args, self.mixer._last_input = None, (x, self.norm)
+                return y
         return self.mixer(self.norm(x)) + x
 
 
@@ -323,7 +418,7 @@ class SSMTS(nn.Module):
                 {"params": self.output.parameters()}]
 
     def forward(self, input_ids, **kwargs):
-        x = _linear(self.embedding, input_ids)
+        x = _norm_linear(self.embedding, input_ids)
         for layer in self.layers:
             x = layer(x)
-        return _linear(self.output, self.norm_f(x))
+        return _norm_linear(self.output, x, self.norm_f)

@@ -41,6 +41,17 @@ __device__ __forceinline__ float sigm_fast(float v) { return __builtin_amdgcn_rc
 __device__ __forceinline__ float silu_fast(float v) { return v * sigm_fast(v); }
 __device__ __forceinline__ float dsilu_fast(float v) { const float sg = sigm_fast(v); return sg * (1.0f + v * (1.0f - sg)); }
 
+// polar parameters of the operator: radius (softplus of it when given raw) and phase of state j
+__device__ __forceinline__ float op_radius(const DropinArgs& p, const float* r, int j) {
+  const float v = r[(size_t)j * p.bcs];
+  return p.raw ? softplusf_(v) : v;
+}
+__device__ __forceinline__ float op_phase(const DropinArgs& p, const float* th, int j) { return th[(size_t)j * p.bcs]; }
+// derivative of the softplus behind dt, from dt itself: 1 - e^-dt (by its series where that would cancel)
+__device__ __forceinline__ float dsoftplus_of(float dt) {
+  return dt < 0.05f ? dt * fmaf(-dt, fmaf(-dt, fmaf(dt, -0.041666668f, 0.16666667f), 0.5f), 1.0f) : 1.0f - __expf(-dt);
+}
+
 // ---- prefix / suffix sums along a row of 16 lanes
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov0(float v) {   // lanes that have no source read 0
@@ -66,9 +77,10 @@ __device__ __forceinline__ float row_last(float v, int) { return dpp_perm<0x15F>
 __device__ __forceinline__ float row_first(float v, int) { return dpp_perm<0x150>(v); }   // row_newbcast:0
 
 
-// x (d, n, d) -> operand records.  Record (v = i nb + sb, ks, piece, lane = (row = lane % 16, g = lane / 16))
+// x (rows of d: (channel i, state j) at row i xsi + j xsj), times scale -> operand records.  Record (v = i nb + sb, ks, piece, lane = (row = lane % 16, g = lane / 16))
 // holds x[i, 16 sb + row, 32 ks + 8 g .. + 7] (zero past the ends).  One thread per (v, ks, lane).
-__global__ __launch_bounds__(256) void dropin_xprep_kernel(const float* __restrict__ x, u4* __restrict__ xp, int d, int n, int ks, int nb) {
+__global__ __launch_bounds__(256) void dropin_xprep_kernel(const float* __restrict__ x, u4* __restrict__ xp, int d, int n, int ks, int nb,
+                                                           int xsi, int xsj, float scale) {
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (size_t)d * nb * ks * 64) return;
   const int lane = (int)(idx & 63);
@@ -79,7 +91,7 @@ __global__ __launch_bounds__(256) void dropin_xprep_kernel(const float* __restri
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     const int r = 32 * k + 8 * g + q;
-    v[q] = (j < n && r < d) ? x[((size_t)i * n + j) * d + r] : 0.0f;
+    v[q] = (j < n && r < d) ? x[((size_t)i * xsi + (size_t)j * xsj) * d + r] * scale : 0.0f;
   }
   u4 pc[3];
   split8<3>(sk, v, pc);
@@ -149,7 +161,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
   const int ic = iok ? i : p.d - 1, vc = ic * nb + sb;
   const int l_ = lane & 15, g = lane >> 4;
   const int d = p.d, n = p.n, L = p.L;
-  const size_t row = ((size_t)b * d + ic) * L;
+  const size_t row = ((size_t)b * d + ic) * L, zrow = (size_t)b * p.zs + (size_t)ic * L;
   const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * (KS * 3 * 64);   // + tile * (KS 3 64)
 
   // this wavefront's rows of x, split, for the whole launch
@@ -166,16 +178,17 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
     const int j = j0 + 4 * g + a;
     const bool ok = j < n;
     const int jc = ok ? j : 0;
-    xb[a] = ok ? p.x_bias[(size_t)ic * n + jc] : 0.0f;
+    xb[a] = ok ? p.x_bias[(size_t)ic * p.xsi + (size_t)jc * p.xsj] : 0.0f;
     float s, c;
-    fast_sincosf(p.B_th[jc], &s, &c);
-    btr[a] = ok ? p.B_r[jc] * c : 0.0f;
-    bti[a] = ok ? p.B_r[jc] * s : 0.0f;
-    fast_sincosf(p.C_th[jc], &s, &c);
-    ctr[a] = ok ? p.C_r[jc] * c : 0.0f;
-    cti[a] = ok ? p.C_r[jc] * s : 0.0f;
-    hr[a] = ok ? p.h_re[((size_t)b * d + ic) * n + jc] : 0.0f;
-    hi[a] = ok ? p.h_im[((size_t)b * d + ic) * n + jc] : 0.0f;
+    const float br = op_radius(p, p.B_r, jc), cr = op_radius(p, p.C_r, jc);
+    fast_sincosf(op_phase(p, p.B_th, jc), &s, &c);
+    btr[a] = ok ? br * c : 0.0f;
+    bti[a] = ok ? br * s : 0.0f;
+    fast_sincosf(op_phase(p, p.C_th, jc), &s, &c);
+    ctr[a] = ok ? cr * c : 0.0f;
+    cti[a] = ok ? cr * s : 0.0f;
+    hr[a] = ok && p.h_re ? p.h_re[((size_t)b * d + ic) * n + jc] : 0.0f;
+    hi[a] = ok && p.h_im ? p.h_im[((size_t)b * d + ic) * n + jc] : 0.0f;
   }
   const float Di = p.Dp[ic];
   const int ntiles = p.t1;
@@ -187,7 +200,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
   __syncthreads();
   // the wavefront's own inputs, requested one tile ahead
   const int lf = p.t0 * DT + l_;
-  float un = lf < L ? p.u[row + lf] : 0.0f, dtn = lf < L ? p.dt[row + lf] : 0.0f, zn = lf < L ? p.z[row + lf] : 0.0f;
+  float un = lf < L ? p.u[row + lf] : 0.0f, dtn = lf < L ? p.dt[row + lf] : 0.0f, zn = lf < L ? p.z[zrow + lf] : 0.0f;
   for (int t = p.t0; t < ntiles; ++t) {
     const int l0 = t * DT, l = l0 + l_;
     const bool lok = l < L;
@@ -196,7 +209,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
       const bool nok = l + DT < L;
       un = nok ? p.u[row + l + DT] : 0.0f;
       dtn = nok ? p.dt[row + l + DT] : 0.0f;
-      zn = nok ? p.z[row + l + DT] : 0.0f;
+      zn = nok ? p.z[zrow + l + DT] : 0.0f;
     }
     if (t + 1 < ntiles) tile_load<NT, NREC, KS>(upb + (size_t)(t + 1) * (KS * 3 * 64), sv, tid);
     // ---- running phases of the tile, less the bias: lane (column l, rows j = 4 g + a)
@@ -272,7 +285,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
 //     grad_x[i,j,r] = sum_{b,l} hat theta[b,i,j,l] u[b,r,l],   grad_u[b,r,l] += sum_{i,j} x[i,j,r] hat theta[b,i,j,l].
 // The second one sums over every channel of a batch element, so hat theta has to leave the wavefront
 // that made it: it goes to a workspace that holds it for a CHUNK of the sequence only (tens of MB,
-// cache resident), and a matrix-core GEMM kernel consumes it before the next chunk overwrites it.
+// cache resident), and the matrix-core GEMM (gemm.h) consumes it before the next chunk overwrites it.
 // A launch therefore covers the tiles t0 .. t1 - 1 of every (batch, channel) pair; the state and its
 // adjoint pass from launch to launch through two small buffers.
 
@@ -296,7 +309,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
   const int ic = iok ? i : p.d - 1, vc = ic * nb + sb;
   const int l_ = lane & 15, g = lane >> 4;
   const int d = p.d, n = p.n, L = p.L;
-  const size_t row = ((size_t)b * d + ic) * L;
+  const size_t row = ((size_t)b * d + ic) * L, zrow = (size_t)b * p.zs + (size_t)ic * L;
   const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * (KS * 3 * 64);   // + tile * (KS 3 64)
 
   u4 xa[KS][3];
@@ -313,11 +326,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     const bool ok = tid < n;
     const int jc = ok ? tid : 0;
     float sb, cb, sc, cc;
-    fast_sincosf(p.B_th[jc], &sb, &cb);
-    fast_sincosf(p.C_th[jc], &sc, &cc);
-    s_par[tid] = ok ? f4{p.B_r[jc] * cb, p.B_r[jc] * sb, p.C_r[jc] * cc, p.C_r[jc] * sc} : f4{0, 0, 0, 0};
+    fast_sincosf(op_phase(p, p.B_th, jc), &sb, &cb);
+    fast_sincosf(op_phase(p, p.C_th, jc), &sc, &cc);
+    const float br = op_radius(p, p.B_r, jc), cr = op_radius(p, p.C_r, jc);
+    s_par[tid] = ok ? f4{br * cb, br * sb, cr * cc, cr * sc} : f4{0, 0, 0, 0};
   }
-  if (lane < 16) s_xb[wave][lane] = j0 + lane < n ? p.x_bias[(size_t)ic * n + j0 + lane] : 0.0f;
+  if (lane < 16) s_xb[wave][lane] = j0 + lane < n ? p.x_bias[(size_t)ic * p.xsi + (size_t)(j0 + lane) * p.xsj] : 0.0f;
   float hr[4], hi[4], ar[4], ai[4];
   float gBr[4], gBi[4], gCr[4], gCi[4], gxb[4];
 #pragma unroll
@@ -333,9 +347,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     gBr[a] = gBi[a] = gCr[a] = gCi[a] = gxb[a] = 0.0f;
   }
   const float Di = p.Dp[ic];
-  float gD = 0.0f;
+  float gD = 0.0f, gdtb = 0.0f;
   const int t_first = q.t0, t_last = q.t1 - 1;
-  float* __restrict__ dth = q.dth + ((size_t)zb * d + ic) * n * q.lc - (size_t)t_first * DT;
+  float* __restrict__ dth = q.dth + ((size_t)zb * d * n + (size_t)ic * p.xsi) * q.lc - (size_t)t_first * DT;   // + state j: j xsj rows
 
   constexpr int NT = NW * 64, NREC = (KS * 3 * 64 + NT - 1) / NT;
   u4 sv[NREC];
@@ -349,7 +363,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     const bool ok = l < L;
     un = ok ? p.u[row + l] : 0.0f;
     dtn = ok ? p.dt[row + l] : 0.0f;
-    zn = ok ? p.z[row + l] : 0.0f;
+    zn = ok ? p.z[zrow + l] : 0.0f;
     gyn = ok ? q.gy[row + l] : 0.0f;
   }
   for (int t = t_last; t >= t_first; --t) {
@@ -359,7 +373,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     if (t > t_first) {                 // l - DT < L holds
       un = p.u[row + l - DT];
       dtn = p.dt[row + l - DT];
-      zn = p.z[row + l - DT];
+      zn = p.z[zrow + l - DT];
       gyn = q.gy[row + l - DT];
     }
     if (t > t_first) tile_load<NT, NREC, KS>(upb + (size_t)(t - 1) * (KS * 3 * 64), sv, tid);
@@ -404,7 +418,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
       float Gh = -(hdr * hei - hdi * her) + (phr * pi - phi * pr);
       if (l_ == 15) Gh -= ar[a] * hi[a] - ai[a] * hr[a];                              // h at the last step is h_out
       const float thh = row_suffix(Gh);
-      if (lok && iok && j0 + 4 * g + a < n) dth[(size_t)(j0 + 4 * g + a) * q.lc + l] = thh;
+      if (lok && iok && j0 + 4 * g + a < n) dth[(size_t)(j0 + 4 * g + a) * p.xsj * q.lc + l] = thh;
       gxb[a] += lok ? thh : 0.0f;
       // hat Bt += E w hat p ; hat Ct += a conj(h)
       const float ewr = cs * w, ewi = sn * w;
@@ -432,8 +446,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     }
     if (iok && lok && g == 0 && sb == 0) {
       const float pre = ysum + Di * ut;
-      q.dz[row + l] = gyv * pre * dsilu_fast(zv);
-      q.ddt[row + l] = wsum * ut;
+      q.dz[zrow + l] = gyv * pre * dsilu_fast(zv);
+      const float ddtv = q.dt_act ? wsum * ut * dsoftplus_of(dtv) : wsum * ut;
+      q.ddt[row + l] = ddtv;
+      gdtb += ddtv;
       q.du[row + l] = (wsum * dtv + av * Di) * dsilu_fast(uv);
       gD += av * ut;
     }
@@ -454,6 +470,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     gCi[a] = row_sum(gCi[a]);
   }
   gD = row_sum(gD);
+  gdtb = row_sum(gdtb);
   if (iok && l_ == 0) {
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
@@ -464,11 +481,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
         q.dh_im[sidx] = ai[a];
         q.hc_re[sidx] = hr[a];
         q.hc_im[sidx] = hi[a];
-        atomicAdd(q.dxb + (size_t)i * n + j, gxb[a]);
+        atomicAdd(q.dxb + (size_t)i * p.xsi + (size_t)j * p.xsj, gxb[a]);
         // polar parameters: Bt = B_r e^{i B_theta}
         float ebr, ebi, ecr, eci;
-        fast_sincosf(p.B_th[j], &ebi, &ebr);
-        fast_sincosf(p.C_th[j], &eci, &ecr);
+        fast_sincosf(op_phase(p, p.B_th, j), &ebi, &ebr);
+        fast_sincosf(op_phase(p, p.C_th, j), &eci, &ecr);
         const f4 par = s_par[j];
         atomicAdd(&s_red[0][j], gBr[a] * ebr + gBi[a] * ebi);
         atomicAdd(&s_red[1][j], gBi[a] * par[0] - gBr[a] * par[1]);
@@ -476,13 +493,20 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
         atomicAdd(&s_red[3][j], gCi[a] * par[2] - gCr[a] * par[3]);
       }
     }
-    if (g == 0 && sb == 0) atomicAdd(q.dD + i, gD);
+    if (g == 0 && sb == 0) {
+      atomicAdd(q.dD + i, gD);
+      if (q.ddtb) atomicAdd(q.ddtb + i, q.ddtb_scale * gdtb);
+    }
   }
   __syncthreads();
   if (tid < 4 * D_MAXN && (tid & (D_MAXN - 1)) < n) {
     constexpr int SH = 6;                              // log2(D_MAXN)
     float* dst = (tid >> SH) == 0 ? q.dB_r : (tid >> SH) == 1 ? q.dB_th : (tid >> SH) == 2 ? q.dC_r : q.dC_th;
-    atomicAdd(dst + (tid & (D_MAXN - 1)), (&s_red[0][0])[tid]);
+    const int j = tid & (D_MAXN - 1);
+    float v = (&s_red[0][0])[tid];
+    // (raw radii: through the softplus)
+    if (p.raw && !((tid >> SH) & 1)) v *= sigmoidf_(((tid >> SH) == 0 ? p.B_r : p.C_r)[(size_t)j * p.bcs]);
+    atomicAdd(dst + (size_t)j * p.bcs, v);
   }
 }
 
@@ -492,195 +516,6 @@ __global__ __launch_bounds__(256) void fill_kernel(const FillArgs a) {
   const float* __restrict__ src = a.src[blockIdx.y];
   const size_t n = a.n[blockIdx.y];
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = src ? src[i] : 0.0f;
-}
-
-// ---- fp32-accurate GEMM on the bf16 matrix cores ------------------------------------------------
-//     C_z[m][n] (+)= sum_k A_z(m, k) B_z(k, n)           z = 0 .. Z-1
-//     C[m][n]    += sum_z sum_k A_z(m, k) B_z(k, n)      (reduce_z)
-// Workgroup tile 128 x (64 TNH), four wavefronts of 64 x (32 TNH) each, 32 of k per step, one workgroup per (tile,
-// slice of z, slice of k): zper consecutive z per workgroup (1 unless reduce_z) and ksplit slices of k.  With more
-// than one slice per element of C the results are summed into C with atomics (C holds the addend beforehand).
-// A - the operand with the 128-row side of the tile - arrives split into three bf16 pieces in the order the
-// kernel keeps it in LDS (a pre-pass, gemm_aprep_kernel: the callers' A is small and used by every workgroup of
-// a column of tiles), so a step copies 24 KiB of records; B is fp32 with arbitrary strides and is split while
-// it is staged.  The values of the next step are requested before the products of the current one.
-// (Measured on the backward call of the fused operator, b = 32, d = 256, n = 16, L = 720.  Launches of 6.2 GFLOP in
-// fp32 terms with 128 x 64 tiles: 54-58 us; without the stores of C - atomics, the launch is cut along k or z -
-// 40-46 us; without the matrix instructions 41-43 us; with neither 30 us: operand traffic, LDS and the two barriers
-// of a step set the floor, the rest adds up.  Launches twice that size: 99-102 us with 128 x 64 tiles, 84-97 us
-// with 128 x 128 (TNH = 2).  Splitting A inside the loop, as B is, cost 5 % more.)
-// K1: B is contiguous along k.  Then four neighbouring lanes fetch the 32 values of one row as 16-byte
-// vectors (VEC; rows need not be 16-byte aligned) - a wavefront request covers 16 cache lines.  Otherwise it is
-// contiguous along n and a 16-lane row of the wavefront fetches 16 neighbouring rows' values of one k.
-// Rows of the B tile that lie past N are fetched from the last valid row instead (column n of B only reaches
-// column n of C, which is not stored then), so only the last, partial step along k takes the bounds-checked loads.
-// TR: the two operands change places in the matrix instruction, so that the lanes of a result register run
-// along m: for a C that is contiguous along m (the stores and atomics of a wavefront then cover whole lines).
-
-// Record slot of (row r of a 16-row tile, k group g = 8 values): 16 g + (r + 4 g) % 16.  The rotation keeps the
-// 16-byte writes of the K1 mapping (four neighbouring lanes = the four g of one row) and the reads (16
-// neighbouring lanes = 16 rows of one g) both free of bank conflicts.
-__device__ __forceinline__ int gemm_slot(int r, int g) { return 16 * g + ((r + 4 * g) & 15); }
-
-// A (fp32, strides sam / sak / saz) -> image: one thread per (z, 16-row tile, step, record)
-__global__ __launch_bounds__(256) void gemm_aprep_kernel(const float* __restrict__ A, u4* __restrict__ img, long sam, long sak, long saz,
-                                                         int M, int K, int m16, int nk, long total) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
-  const int slot = (int)(idx & 63);
-  const long rest = idx >> 6;
-  const int it = (int)(rest % nk), mt = (int)((rest / nk) % m16);
-  const long z = rest / ((long)nk * m16);
-  const int g = slot >> 4, r = ((slot & 15) - 4 * g) & 15;
-  const int m = mt * 16 + r, k0 = it * 32 + 8 * g;
-  const SplitK sk = make_splitk();
-  float v[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) v[q] = (m < M && k0 + q < K) ? A[z * saz + (long)m * sam + (long)(k0 + q) * sak] : 0.0f;
-  u4 pc[3];
-  split8<3>(sk, v, pc);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) img[(rest * 3 + c) * 64 + slot] = pc[c];
-}
-
-template <bool K1, bool VEC, bool TR, int TNH>
-__global__ __launch_bounds__(256) void split_gemm_kernel(const GemmArgs p) {
-  constexpr int NP = 3;                // bf16 pieces per operand: fp32-accurate products
-  constexpr int AREC = 8 * NP * 64;    // records of the A tile of one step
-  constexpr int AQ = AREC / 256;       // ... per thread
-  constexpr int TN = 64 * TNH;         // columns of the workgroup tile
-  constexpr int EN = 2 * TNH;          // 16-wide column tiles per wavefront
-  __shared__ u4 s_a[AREC], s_b[4 * TNH * NP * 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
-  const int m0 = blockIdx.x * 128, n0 = blockIdx.y * TN;
-  const int zs = blockIdx.z / p.ksplit, ksl = blockIdx.z % p.ksplit;
-  const int z_lo = zs * p.zper, z_hi = z_lo + p.zper < p.Z ? z_lo + p.zper : p.Z;
-  const int wm = (wave >> 1) * 4, wn = (wave & 1) * EN;      // this wavefront's first 16-wide tiles
-  const SplitK sk = make_splitk();
-  f4 acc[4][EN];
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-#pragma unroll
-    for (int f = 0; f < EN; ++f) acc[e][f] = f4{0, 0, 0, 0};
-  // the record of B this thread stages: row rb of the tile, k slots kq ..
-  const int rb = K1 ? tid >> 2 : wave * 16 + (lane & 15);
-  const int kq = 8 * (K1 ? tid & 3 : lane >> 4);
-  const int slot = (rb >> 4) * (NP * 64) + gemm_slot(rb & 15, kq >> 3);
-  const int rslot = gemm_slot(lane & 15, lane >> 4);       // the record of (row lane % 16, g lane / 16)
-  // uniform bases, 32-bit per-thread offsets (a z-slice of B is below 2^31 elements)
-  const unsigned sbk = (unsigned)p.sbk;
-  unsigned ob[TNH];
-#pragma unroll
-  for (int h = 0; h < TNH; ++h) {
-    const int n = n0 + rb + 64 * h;
-    ob[h] = (unsigned)(n < p.N ? n : p.N - 1) * (unsigned)p.sbn + (unsigned)kq * sbk;
-  }
-  const int nk = (p.K + 31) / 32, per = (nk + p.ksplit - 1) / p.ksplit;
-  const int it0 = ksl * per, it1 = it0 + per < nk ? it0 + per : nk;
-  const int nit = it1 > it0 ? (it1 - it0) * (z_hi - z_lo) : 0;      // steps of this workgroup: (z, k step) pairs
-  // this thread's records of the A tile: record tid + 256 q of the tile = record (tid + 256 q) % 192 of row tile
-  // m0 / 16 + (tid + 256 q) / 192, whose steps lie nk * 192 records apart
-  unsigned oa[AQ];
-#pragma unroll
-  for (int q = 0; q < AQ; ++q) {
-    const int idx = tid + 256 * q, e = idx / (NP * 64);
-    oa[q] = (unsigned)(((m0 >> 4) + e) * nk) * (unsigned)(NP * 64) + (unsigned)(idx - e * (NP * 64));
-  }
-  u4 ia[AQ];
-  float vb[TNH][8];
-  int fz = z_lo, fit = it0;                   // (z, k step) of the next fetch: steps are fetched in order
-  auto fetch = [&]() {
-    const int z = fz, it = fit;
-    if (++fit == it1) { fit = it0; ++fz; }
-    const u4* __restrict__ Az = p.Aimg + z * p.simz + (size_t)it * (NP * 64);
-#pragma unroll
-    for (int q = 0; q < AQ; ++q) ia[q] = Az[oa[q]];
-    const float* __restrict__ Bz = p.Bm + z * p.sbz;
-    const unsigned kb = (unsigned)(it * 32) * sbk;
-    if (it * 32 + 32 <= p.K) {
-      if constexpr (K1 && VEC) {
-        // 16-byte loads that are only known to be 4-byte aligned (rows start anywhere when the row length is
-        // not a multiple of four): the memory pipeline takes them, the type tells the compiler so
-        typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-          for (int h = 0; h < TNH; ++h) {
-            const f4u x = *reinterpret_cast<const f4u*>(Bz + (ob[h] + kb + 4 * q));
-#pragma unroll
-            for (int c = 0; c < 4; ++c) vb[h][4 * q + c] = x[c];
-          }
-      } else {
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-          for (int h = 0; h < TNH; ++h) vb[h][c] = Bz[ob[h] + kb + (unsigned)c * sbk];
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
-#pragma unroll
-        for (int h = 0; h < TNH; ++h) vb[h][c] = (it * 32 + kq + c < p.K) ? Bz[ob[h] + kb + (unsigned)c * sbk] : 0.0f;
-    }
-  };
-  if (nit > 0) fetch();
-  for (int step = 0; step < nit; ++step) {
-    u4 pb[TNH][NP];
-#pragma unroll
-    for (int h = 0; h < TNH; ++h) split8<NP>(sk, vb[h], pb[h]);
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < AQ; ++q) s_a[tid + 256 * q] = ia[q];
-#pragma unroll
-    for (int c = 0; c < NP; ++c)
-#pragma unroll
-      for (int h = 0; h < TNH; ++h) s_b[slot + 4 * h * (NP * 64) + c * 64] = pb[h][c];
-    __syncthreads();
-    if (step + 1 < nit) fetch();              // in flight during the products
-    u4 rB[EN][NP];
-#pragma unroll
-    for (int f = 0; f < EN; ++f)
-#pragma unroll
-      for (int c = 0; c < NP; ++c) rB[f][c] = s_b[((wn + f) * NP + c) * 64 + rslot];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      u4 rA[NP];
-#pragma unroll
-      for (int c = 0; c < NP; ++c) rA[c] = s_a[((wm + e) * NP + c) * 64 + rslot];
-#pragma unroll
-      for (int f = 0; f < EN; ++f) acc[e][f] = TR ? xmm<NP>(rB[f], rA, acc[e][f]) : xmm<NP>(rA, rB[f], acc[e][f]);
-    }
-  }
-  // result tile (e, f), register a: row 16 e + 4 (lane / 16) + a, column 16 f + lane % 16 of the wavefront's block
-  // (TR: row 16 e + lane % 16, column 16 f + 4 (lane / 16) + a)
-  float* __restrict__ C = p.C + (p.reduce_z ? 0 : z_lo * p.scz);
-  const bool atomic = p.ksplit > 1 || (p.reduce_z && p.zper < p.Z);
-  // element offsets inside a z-slice of C fit 32 bits (checked by the caller)
-  const unsigned scm = (unsigned)p.scm, scn = (unsigned)p.scn;
-  const int mr = m0 + wm * 16 + (TR ? (lane & 15) : 4 * (lane >> 4)), nc = n0 + wn * 16 + (TR ? 4 * (lane >> 4) : (lane & 15));
-  const unsigned o0 = (unsigned)mr * scm + (unsigned)nc * scn;
-  const unsigned sa = TR ? scn : scm;           // stride between the four registers of a result
-  if (atomic && m0 + 128 <= p.M && n0 + TN <= p.N) {       // uniform: a whole tile, summed into C
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int f = 0; f < EN; ++f)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) atomicAdd(C + (o0 + (unsigned)(16 * e) * scm + (unsigned)(16 * f) * scn + (unsigned)a * sa), acc[e][f][a]);
-    return;
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-#pragma unroll
-    for (int f = 0; f < EN; ++f)
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        if (mr + 16 * e + (TR ? 0 : a) < p.M && nc + 16 * f + (TR ? a : 0) < p.N) {
-          float* c = C + (o0 + (unsigned)(16 * e) * scm + (unsigned)(16 * f) * scn + (unsigned)a * sa);
-          if (atomic) atomicAdd(c, acc[e][f][a]);
-          else *c = p.accumulate ? *c + acc[e][f][a] : acc[e][f][a];
-        }
-      }
 }
 
 }  // namespace aussm

@@ -12,13 +12,13 @@ struct DropinArgs {
   const float* u;        // [b, d, L]
   const float* dt;       // [b, d, L]
   const float* z;        // [b, d, L]
-  const float* x_bias;   // [d, n]
-  const float* B_r;      // [n]
+  const float* x_bias;   // [d, n]: element (i, j) at i xsi + j xsj
+  const float* B_r;      // [n], consecutive states bcs elements apart
   const float* B_th;
   const float* C_r;
   const float* C_th;
   const float* Dp;       // [d]
-  const float* h_re;     // [b, d, n] state before tile t0
+  const float* h_re;     // [b, d, n] state before tile t0, or null: zero
   const float* h_im;
   float* y;              // [b, d, L] or null (states only)
   float* nh_re;          // [b, d, n] or null: state after tile t1 - 1 (may be the same buffer as h_*)
@@ -30,6 +30,9 @@ struct DropinArgs {
   int nb;                // blocks of 16 states per channel: 1, 2 or 4 (>= ceil(n / 16))
   int b0;                // first batch element of this launch (tensors are indexed by b0 + ...)
   int t0, t1;            // tiles of 16 timesteps of this launch (forward kernel; the backward kernel has its own)
+  int xsi, xsj;          // row of (channel i, state j) in x, x_bias and the phase adjoints: i xsi + j xsj (n, 1 or 1, d)
+  int bcs, raw;          // stride of the four polar parameters; raw: the radii are given before their softplus
+  long zs;               // elements between the batch elements of z (d L for a tensor of its own)
 };
 
 struct DropinBwdArgs {
@@ -40,7 +43,7 @@ struct DropinBwdArgs {
   float* dth;              // workspace [bg][d n][lc]: phase adjoints of the launch
   float* du;               // [b, d, L] direct part (the product with x is added afterwards)
   float* ddt;
-  float* dz;
+  float* dz;               // (batch elements f.zs apart)
   float* dxb;              // [d, n]   accumulated with atomics (zeroed by the host)
   float* dB_r;             // [n] each, accumulated with atomics
   float* dB_th;
@@ -52,6 +55,9 @@ struct DropinBwdArgs {
   int b0, bg;              // batch elements b0 .. b0 + bg - 1 ...
   int t0, t1;              // ... and tiles of 16 timesteps t0 .. t1 - 1 (in reverse) are this launch's
   int lc;                  // row length of dth (>= 16 (t1 - t0))
+  int dt_act;              // dt = softplus(pre): ddt is the gradient of pre, and ddtb [d] (or null) sums it (atomics)
+  float* ddtb;
+  float ddtb_scale;
 };
 
 // Up to 12 buffers set in one launch: dst[i] = src ? src[i] : 0 for i < n.
@@ -60,20 +66,6 @@ struct FillArgs {
   const float* src[12];
   unsigned long long n[12];
   int count;
-};
-
-// A is a prepared image (gemm_aprep_kernel): [z][16-row tile][step of 32 along k][piece][64 records], the
-// row tiles padded to whole workgroup tiles of 128 rows, zeros past M and K.
-struct GemmArgs {
-  const u4* Aimg; const float* Bm; float* C;
-  long simz;              // records between the images of consecutive z (0: one image for all)
-  long sbk, sbn, sbz;     // element strides of B over k, n, z
-  long scm, scn, scz;
-  int M, N, K, Z;
-  int reduce_z, accumulate;
-  int tr;                 // results leave with the lanes along m (for C contiguous along m) instead of along n
-  int ksplit;             // slices of k per (tile, slice of z)
-  int zper;               // z per workgroup (summed inside it; 1 unless reduce_z)
 };
 
 }  // namespace aussm

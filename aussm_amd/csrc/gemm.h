@@ -1,0 +1,256 @@
+// fp32-accurate matrix products on the bf16 matrix cores: the linear layers of the blocks and the two products with
+// the phase adjoints of the fused operator.
+//
+// Both operands are fp32 in memory and split EXACTLY into three bf16 pieces while they are staged into LDS (scan_fwd_xdl.h:
+// split8, xmm<3>): what a product drops is below 2^-26 of it, the sums are fp32.  Workgroup tile 128 x (64 TNH), four
+// wavefronts of 64 x (32 TNH), 32 of k per step; the values of the next step are requested before the products of
+// the current one, and two workgroups per compute unit cover each other's barriers.
+//
+// Operands may be contiguous along k or along their other index (AK1 / BK1), so no transposed copy is ever made:
+//   along k: four neighbouring lanes fetch the 32 values of a row (one 128-byte line), 16 bytes at a time;
+//   else:    a wavefront fetches all rows' values of one k (up to 512 bytes), eight k in turn.
+// TR: the operands change places in the matrix instruction, so that the lanes of a result register run along m,
+// for a C that is contiguous along m: the stores and atomics of 16 lanes cover one 64-byte piece either way.
+#pragma once
+#include "gemm_args.h"
+#include "scan_fwd_xdl.h"
+
+namespace aussm {
+
+// Record slot of (row r of a 16-row tile, k group g = 8 values): 16 g + (r + 4 g) % 16.  The rotation keeps the
+// 16-byte writes of the along-k mapping (four neighbouring lanes = the four g of one row) and the reads (16
+// neighbouring lanes = 16 rows of one g) both free of bank conflicts.
+__device__ __forceinline__ int xg_slot(int r, int g) { return 16 * g + ((r + 4 * g) & 15); }
+
+// 16-byte loads that are only known to be 4-byte aligned (rows start anywhere when the row length is not a
+// multiple of four): the memory pipeline takes them, the type tells the compiler so
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+
+// One thread's share of an operand tile of 64 H rows x 32 k: H records of 8 k each.
+//   K1:  row tid / 4 (+ 64), k group tid % 4
+//   else rows H lane .. H lane + H - 1 (one load for two rows), k group = wavefront: the k index, its bound and the
+//        stride along k are scalars, and a load instruction is a scalar base plus the row's offset
+// Loads are unconditional (no branch may hide from the compiler how many are in flight): in the last, partial step
+// along k they repeat valid elements, and stage() clears what lies past K.  QUAD: K is a multiple of four.
+template <bool K1, bool QUAD, int H>
+struct XgOperand {
+  const float* row[H];       // K1: this thread's rows; else row[0]: its first row (the second one is next to it)
+  long sk;
+  int r0, kq;
+  struct Vals { float v[H][8]; };
+  __device__ __forceinline__ void place(int tid) {
+    r0 = K1 ? tid >> 2 : H * (tid & 63);
+    kq = 8 * (K1 ? tid & 3 : wave_index());
+  }
+  __device__ __forceinline__ int local_row(int h) const { return K1 ? r0 + 64 * h : r0 + h; }
+  __device__ __forceinline__ int slot(int h) const {
+    const int r = local_row(h);
+    return (r >> 4) * (3 * 64) + xg_slot(r & 15, kq >> 3);
+  }
+  // pair: (not K1, H == 2) the thread's two rows are neighbours in memory
+  __device__ __forceinline__ void fetch(Vals& x, long zoff, int k0, int K, bool pair) const {
+    const int k = k0 + kq;
+    if constexpr (K1 && QUAD) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int kk = min(k + 4 * q, K - 4);
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          const f4u t = *reinterpret_cast<const f4u*>(row[h] + (zoff + kk));
+#pragma unroll
+          for (int c = 0; c < 4; ++c) x.v[h][4 * q + c] = t[c];
+        }
+      }
+    } else if (!K1 && H == 2 && pair) {                 // uniform
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const f2u t = *reinterpret_cast<const f2u*>(row[0] + (zoff + (long)min(k + c, K - 1) * sk));
+        x.v[0][c] = t[0]; x.v[H - 1][c] = t[1];
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const long o = zoff + (long)min(k + c, K - 1) * (K1 ? 1 : sk);
+#pragma unroll
+        for (int h = 0; h < H; ++h) x.v[h][c] = row[h][o];
+      }
+    }
+  }
+  __device__ __forceinline__ void stage(const SplitK& sk_, Vals& x, int k0, int K, u4* __restrict__ lds) const {
+    if (k0 + 32 > K) {                                  // uniform
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+#pragma unroll
+        for (int h = 0; h < H; ++h) x.v[h][c] = k0 + kq + c < K ? x.v[h][c] : 0.0f;
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      u4 pc[3];
+      split8<3>(sk_, x.v[h], pc);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) lds[slot(h) + c * 64] = pc[c];
+    }
+  }
+};
+
+// The results go through LDS to the memory: 64 registers written with fixed offsets, then rolled loops over the rows
+// along the contiguous index of C - 16 bytes a lane for whole, aligned tiles, else one element a lane (bounds, batch
+// borders, atomics).  Unrolled stores straight from the registers, each with its own bounds and offset, made the
+// code several times the size of the main loop and covered 64 bytes at a time: 32 x 720 columns, 256 rows, K = 16
+// 19.5 us, now 13 us.
+template <bool AK1, bool BK1, bool TR, int TNH, bool QUAD>
+__global__ __launch_bounds__(256, 2) void xgemm_kernel(const XGemmArgs p) {
+  constexpr int NP = 3, TN = 64 * TNH, EN = 2 * TNH;        // EN: 16-wide column tiles per wavefront
+  constexpr int WN = 16 * EN;                               // columns of a wavefront's block
+  constexpr int LD = (TR ? 64 : WN) + 4;                    // row stride of its slice in LDS: 64 rows x WN columns, or transposed
+  constexpr int SLICE = (TR ? WN : 64) * LD;
+  constexpr int TILES = (8 + 4 * TNH) * NP * 64;            // records of both operand tiles
+  constexpr int LDS16 = TILES > SLICE ? TILES : SLICE;      // (four slices of SLICE floats = SLICE 16-byte records)
+  __shared__ u4 s_mem[LDS16];
+  u4* const s_a = s_mem;
+  u4* const s_b = s_mem + 8 * NP * 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
+  // consecutive logical workgroups share their columns (B is the large operand) and an XCD
+  const int tm = (p.M + XG_TM - 1) / XG_TM, tn = (p.N + TN - 1) / TN;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int m0 = (wg % tm) * XG_TM, n0 = (wg / tm % tn) * TN, sl = wg / (tm * tn);
+  const int wm = (wave >> 1) * 4, wn = (wave & 1) * EN;     // this wavefront's first 16-wide tiles
+  const SplitK sk = make_splitk();
+  f4 acc[4][EN];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int f = 0; f < EN; ++f) acc[e][f] = f4{0, 0, 0, 0};
+  // batch and position of the tile's first column; most tiles lie in one batch (no division per column)
+  const int nb0 = n0 / p.nper, np0 = n0 - nb0 * p.nper;
+  const bool one = np0 + TN <= p.nper || p.nper >= p.N;
+  // rows past M / N are fetched from the last valid one (they only reach results that are not stored)
+  XgOperand<AK1, QUAD, 2> oa;
+  XgOperand<BK1, QUAD, TNH> ob;
+  oa.place(tid); ob.place(tid);
+  oa.sk = p.sak; ob.sk = p.sbk;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) oa.row[h] = p.A + (long)min(m0 + oa.local_row(h), p.M - 1) * p.sam;
+#pragma unroll
+  for (int h = 0; h < TNH; ++h) {
+    const int dn = min(ob.local_row(h), p.N - 1 - n0) + np0, nb = one ? 0 : dn / p.nper;
+    ob.row[h] = p.B + ((long)(nb0 + nb) * p.sbb + (long)(dn - nb * p.nper) * p.sbn);
+  }
+  // two neighbouring rows in one load: every pair of the tile exists and lies in one batch (uniform)
+  const bool pa = m0 + XG_TM <= p.M, pb = one && n0 + TN <= p.N;
+  const int nk = (p.K + 31) / 32, steps = nk * p.Z, per = (steps + p.slices - 1) / p.slices;
+  const int s0 = sl * per, s1 = s0 + per < steps ? s0 + per : steps;
+  int fz = s0 / nk, fit = s0 - fz * nk;                     // (z, k step) of the next fetch
+  typename XgOperand<AK1, QUAD, 2>::Vals va;
+  typename XgOperand<BK1, QUAD, TNH>::Vals vb;
+  const int rslot = xg_slot(lane & 15, lane >> 4);          // the record of (row lane % 16, g lane / 16)
+  if (s0 < s1) {
+    oa.fetch(va, (long)fz * p.saz, fit * 32, p.K, pa);
+    ob.fetch(vb, (long)fz * p.sbz, fit * 32, p.K, pb);
+  }
+#pragma unroll 1
+  for (int s = s0; s < s1; ++s) {
+    const int k0 = fit * 32;
+    if (s > s0) __syncthreads();
+    oa.stage(sk, va, k0, p.K, s_a);
+    ob.stage(sk, vb, k0, p.K, s_b);
+    __syncthreads();
+    if (++fit == nk) { fit = 0; ++fz; }
+    if (s + 1 < s1) {                                       // in flight during the products
+      oa.fetch(va, (long)fz * p.saz, fit * 32, p.K, pa);
+      ob.fetch(vb, (long)fz * p.sbz, fit * 32, p.K, pb);
+    }
+    u4 rB[EN][NP];
+#pragma unroll
+    for (int f = 0; f < EN; ++f)
+#pragma unroll
+      for (int c = 0; c < NP; ++c) rB[f][c] = s_b[((wn + f) * NP + c) * 64 + rslot];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      u4 rA[NP];
+#pragma unroll
+      for (int c = 0; c < NP; ++c) rA[c] = s_a[((wm + e) * NP + c) * 64 + rslot];
+#pragma unroll
+      for (int f = 0; f < EN; ++f) acc[e][f] = xmm<NP>(rA, rB[f], acc[e][f]);
+    }
+  }
+  // result tile (e, f), register a: row 16 e + 4 (lane / 16) + a, column 16 f + lane % 16 of the wavefront's block
+  __syncthreads();                                          // (the operand tiles are read no more)
+  float* const sw = reinterpret_cast<float*>(s_mem) + wave * SLICE;
+  const int c = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int f = 0; f < EN; ++f) {
+      if constexpr (TR) *reinterpret_cast<f4*>(sw + (16 * f + c) * LD + 16 * e + 4 * g) = acc[e][f];
+      else {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) sw[(16 * e + 4 * g + a) * LD + 16 * f + c] = acc[e][f][a];
+      }
+    }
+  __builtin_amdgcn_wave_barrier();                          // (a slice belongs to one wavefront)
+  const float* const add = p.add ? p.add : p.reduce ? p.C : nullptr;
+  const int mw = m0 + 16 * wm, nw = n0 + 16 * wn;
+  constexpr int ROWS = TR ? WN : 64, COLS = TR ? 64 : WN;   // rows of the slice run along the contiguous index of C
+  if (p.slices > 1) {                                       // uniform: summed into C (TR: one batch, nper = N)
+    constexpr int RA = 64 / COLS;                           // lane = column (two rows at a time where 32 fill the row)
+    const int q = lane % COLS;
+    const bool cok = TR ? mw + q < p.M : nw + q < p.N;
+    const int dq = nw + q - n0 + np0, bq = (TR || one) ? 0 : dq / p.nper;
+    float* const dst = p.C + (TR ? (long)(mw + q) * p.scm : (long)(nb0 + bq) * p.scb + (long)(dq - bq * p.nper) * p.scn);
+#pragma unroll 4
+    for (int r = lane / COLS; r < ROWS; r += RA) {
+      const int o = (TR ? nw : mw) + r;
+      if (cok && o < (TR ? p.N : p.M)) atomicAdd(dst + (long)o * (TR ? p.scn : p.scm), p.alpha * sw[r * LD + q]);
+    }
+    return;
+  }
+  constexpr int PR = COLS / 4, RR = 64 / PR;                // lanes per row, rows per iteration
+  const int q = 4 * (lane % PR);
+  // the other index's bounds and strides; four elements that exist, in one batch and aligned, leave as 16 bytes
+  const int cnt = min(4, TR ? p.M - (mw + q) : p.N - (nw + q));
+  const int dnq = nw + q - n0 + np0, nbq = (TR || one) ? 0 : dnq / p.nper, npq = dnq - nbq * p.nper;
+  const bool ptr16 = ((reinterpret_cast<uintptr_t>(p.C) | (add ? reinterpret_cast<uintptr_t>(add) : 0)) & 15) == 0;
+  const bool quad = cnt == 4 && (TR || one || npq + 4 <= p.nper);
+#pragma unroll 2
+  for (int r = lane / PR; r < ROWS; r += RR) {
+    if (cnt <= 0 || (TR ? nw : mw) + r >= (TR ? p.N : p.M)) continue;
+    f4 v = *reinterpret_cast<const f4*>(sw + r * LD + q) * p.alpha;
+    long o;
+    if constexpr (TR) {
+      const int dn = nw + r - n0 + np0, nb = one ? 0 : dn / p.nper;
+      o = (long)(nb0 + nb) * p.scb + (long)(dn - nb * p.nper) * p.scn + (mw + q);
+    } else {
+      o = (long)(nb0 + nbq) * p.scb + npq + (long)(mw + r) * p.scm;
+    }
+    if (p.bias) {
+#pragma unroll
+      for (int a = 0; a < 4; ++a) v[a] = fmaf(p.bias_scale, p.bias[TR ? min(mw + q + a, p.M - 1) : mw + r], v[a]);
+    }
+    if (quad && ptr16 && (o & 3) == 0) {
+      if (add) v += *reinterpret_cast<const f4*>(add + o);
+      if (p.act == 1) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) v[a] = softplusf_(v[a]);
+      }
+      *reinterpret_cast<f4*>(p.C + o) = v;
+    } else {
+      const float x[4] = {v[0], v[1], v[2], v[3]};
+#pragma unroll 1
+      for (int a = 0; a < cnt; ++a) {
+        long oa_ = o + a;
+        if (!quad && !TR && !one) {                         // the four may lie in more than one batch
+          const int nb = (dnq + a) / p.nper;
+          oa_ = (long)(nb0 + nb) * p.scb + (dnq + a - nb * p.nper) + (long)(mw + r) * p.scm;
+        }
+        float t = a == 0 ? x[0] : a == 1 ? x[1] : a == 2 ? x[2] : x[3];
+        if (add) t += add[oa_];
+        p.C[oa_] = p.act == 1 ? softplusf_(t) : t;
+      }
+    }
+  }
+}
+
+}  // namespace aussm

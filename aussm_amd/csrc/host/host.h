@@ -13,4 +13,18 @@ std::pair<Tensor, Tensor> selective_scan(const Tensor& u, const Tensor& delta, c
                                          const OptTensor& D, const OptTensor& z, const OptTensor& delta_bias, bool delta_softplus,
                                          bool want_state, const OptTensor& h0);
 
+bool operator_supported(int64_t b, int64_t d, int64_t n, int64_t l);
+Tensor adaptive_operator(const Tensor& u, const Tensor& dt, const Tensor& x, const Tensor& x_bias, const Tensor& B, const Tensor& C,
+                         const Tensor& D, const Tensor& z);
+
+// The blocks and linear layers answer nothing where they do not take the tensors (another type or device, sizes
+// beyond the kernels): the caller then composes the layer from separate operators.
+OptTensor aussm_block(const Tensor& x, const OptTensor& norm_w, double eps, bool residual, const Tensor& W_in, const OptTensor& b_in,
+                      const Tensor& conv_w, const OptTensor& conv_b, const Tensor& W_xp, const Tensor& W_dt, const Tensor& b_dt, const Tensor& xA_w,
+                      const Tensor& xA_b, const Tensor& B, const Tensor& C, const Tensor& D, const Tensor& W_out, const OptTensor& b_out, double scale);
+OptTensor mamba_block(const Tensor& x, const OptTensor& norm_w, double eps, bool residual, const Tensor& W_in, const OptTensor& b_in,
+                      const Tensor& conv_w, const OptTensor& conv_b, const Tensor& W_xp, const Tensor& W_dt, const Tensor& b_dt, const Tensor& A_log,
+                      const Tensor& D, const Tensor& W_out, const OptTensor& b_out);
+OptTensor norm_linear(const Tensor& x, const OptTensor& norm_w, double eps, const Tensor& W, const OptTensor& b);
+
 }  // namespace aussm_host

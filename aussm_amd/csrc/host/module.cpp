@@ -47,4 +47,9 @@ PYBIND11_MODULE(_aussm_host, m) {
                              const OptTensor& z, const OptTensor& bias, bool softplus, bool want_state, const OptTensor& h0) {
     return result(selective_scan(u, delta, A, B, C, D, z, bias, softplus, want_state, h0), want_state);
   });
+  m.def("operator_supported", &operator_supported);
+  m.def("adaptive_operator", &adaptive_operator);
+  m.def("aussm_block", &aussm_block);
+  m.def("mamba_block", &mamba_block);
+  m.def("norm_linear", &norm_linear);
 }

@@ -5,7 +5,9 @@
 #include <hip/hip_runtime.h>
 
 #include "scan_args.h"
+#include "block_args.h"
 #include "dropin_args.h"
+#include "gemm_args.h"
 
 namespace aussm {
 
@@ -54,16 +56,24 @@ int run_px_fwd(const FwdArgs& a, const u4* img, const ImgNote& note, int in_dtyp
 int run_px_bwd(const UniBwdArgs& a, const u4* img, int in_dtype, hipStream_t s);
 
 // ---- k_dropin.hip: the reference's 12-input operator as fused kernels
-int run_dropin_xprep(const float* x, u4* xp, int d, int n, int ks, int nb, hipStream_t s);
+int run_dropin_xprep(const float* x, u4* xp, int d, int n, int ks, int nb, int xsi, int xsj, float scale, hipStream_t s);
 int dropin_channels_per_workgroup(int ks);
 int dropin_compiled_ks(int ks);
 int run_dropin_uprep(const float* u, u4* up, int d, int L, int ks, int b0, int bg, int t0, int nt, hipStream_t s);
 int run_dropin_fwd(const DropinArgs& a, hipStream_t s);
 int run_dropin_bwd(const DropinBwdArgs& a, hipStream_t s);
 int run_fill(const FillArgs& a, hipStream_t s);   // several buffers set (zero or a copy) in one launch
-constexpr int GEMM_TILE_M = 128, GEMM_TILE_N = 128;   // workgroup tile of run_split_gemm
-int run_split_gemm(const GemmArgs& a, hipStream_t s);
-size_t gemm_image_records(int M, int K);       // 16-byte records of the prepared image of an M x K operand
-int run_gemm_aprep(const float* A, u4* img, long sam, long sak, long saz, int M, int K, int Z, hipStream_t s);
+
+// ---- k_blocks.hip: what the blocks do around the scans, on channel rows (b, d, l)
+int run_conv_rows_fwd(const ConvRowsArgs& a, hipStream_t s);
+int run_conv_rows_bwd(const ConvRowsArgs& a, hipStream_t s);
+int run_norm_fwd(const NormArgs& a, hipStream_t s);
+int run_norm_bwd(const NormArgs& a, hipStream_t s);
+int run_col_sum(const float* x, float* out, size_t rows, int d, float scale, hipStream_t s);
+int run_row_sum(const float* x, float* out, size_t rows, int d, int L, float scale, hipStream_t s);
+int run_neg_exp(const float* a_log, const float* dA, float* out, int n, hipStream_t s);
+
+// ---- k_gemm.hip: fp32-accurate matrix products on the bf16 matrix cores
+int run_xgemm(XGemmArgs a, hipStream_t s);
 
 }  // namespace aussm

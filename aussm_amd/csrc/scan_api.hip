@@ -35,6 +35,13 @@ inline Cfg pick_cfg(int N, int max_waves) {
   return Cfg{16, 256};
 }
 
+// flags that the backward entry points take beside the input type
+inline int take_flag(int& in_dtype, int flag) {
+  const int f = in_dtype & flag;
+  in_dtype &= ~flag;
+  return f != 0;
+}
+
 inline int check_common(int B, int D, int N, int L, int ck, int in_dtype) {
   if (B < 1 || D < 1 || N < 1 || L < 1) return AUSSM_E_SHAPE;
   if (N > AUSSM_MAX_STATE) return AUSSM_E_SHAPE;
@@ -301,6 +308,7 @@ int launch_generic_bwd(int variant, RecBwdArgs a, int in_dtype, float* ws, hipSt
     g.dy = a.dy; g.z = a.z; g.delta = a.delta; g.theta = a.theta; g.rho = a.rho; g.A = a.A; g.Cm = a.Cm;
     g.delta_bias = a.delta_bias; g.out = seg; g.ptot = ptot;
     g.D = a.D; g.N = a.N; g.L = sp.ls; g.ld = a.L; g.ns = sp.ns; g.ncg = a.ncg; g.delta_softplus = a.delta_softplus;
+    g.zrows = a.zrows; g.bcrows = a.bcrows;
     if (int e = run_adjoint_seg(variant, g, in_dtype, (unsigned)(B * sp.ns * a.ncg), s)) return e;
     if (int e = variant == VAR_COMPLEX ? run_seg_carry_bwd(seg, ptot, a.dhL, a.dh0, B, a.D, a.N, sp.ns, s)
                                        : run_seg_carry_real(true, seg, ptot, a.A, a.dhL, a.dh0, B, a.D, a.N, sp.ns, s))
@@ -481,12 +489,29 @@ int aussm_real_fwd(const void* u, const void* delta, const float* A, const void*
                    const float* Dskip, const float* z, const float* delta_bias, int delta_softplus,
                    const float* h0, float* y, float* hL, float* hck, float* workspace,
                    int B, int D, int N, int L, int ck, int in_dtype, void* stream) {
+  return aussm_real_fwd_rows(u, delta, A, Bm, Cm, Dskip, z, delta_bias, delta_softplus, h0, y, hL, hck, workspace, nullptr, B, D, N, L, ck,
+                             in_dtype, stream);
+}
+
+// (rows of wider tensors: float inputs only, whose B_t / C_t are not copied on the way)
+static int real_rows_check(const aussm_real_rows* r, int D, int N, int in_dtype) {
+  if (!r) return AUSSM_OK;
+  if ((r->z_rows && r->z_rows < D) || (r->bc_rows && r->bc_rows < N)) return AUSSM_E_SHAPE;
+  return r->bc_rows && in_dtype != AUSSM_F32 ? AUSSM_E_DTYPE : AUSSM_OK;
+}
+
+int aussm_real_fwd_rows(const void* u, const void* delta, const float* A, const void* Bm, const void* Cm,
+                        const float* Dskip, const float* z, const float* delta_bias, int delta_softplus,
+                        const float* h0, float* y, float* hL, float* hck, float* workspace, const aussm_real_rows* rows,
+                        int B, int D, int N, int L, int ck, int in_dtype, void* stream) {
   if (int e = check_common(B, D, N, L, ck, in_dtype)) return e;
   if (!u || !delta || !A || !Bm || !Cm) return AUSSM_E_NULL;
   FwdArgs a{};
   a.u = u; a.delta = delta; a.A = A; a.Bm = Bm; a.Cm = Cm; a.Dskip = Dskip; a.z = z;
   a.delta_bias = delta_bias; a.delta_softplus = delta_softplus;
   a.h0 = h0; a.y = y; a.hL = hL; a.hck = hck;
+  if (int e = real_rows_check(rows, D, N, in_dtype)) return e;
+  if (rows) { a.zrows = rows->z_rows; a.bcrows = rows->bc_rows; a.u_act = rows->u_silu; }
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
   a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.urep = 1;
   return launch_generic_fwd(VAR_REAL, a, in_dtype, workspace, (hipStream_t)stream);
@@ -504,6 +529,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
                           const void* Bc, const void* Cc, const float* Dskip, const float* hck, float* aux,
                           float* du, float* ddelta, float* dtheta, float* dB, float* dC, float* dD, float* dh0,
                           int B, int D, int N, int L, int ck, int in_dtype, int urep, void* stream) {
+  const int g16 = take_flag(in_dtype, AUSSM_GRADS_IN_DTYPE), own_aux = take_flag(in_dtype, AUSSM_AUX_FILLED);
   if (int e = check_common(B, D, N, L, ck, in_dtype)) return e;
   if (urep < 1 || B % urep != 0) return AUSSM_E_SHAPE;
   if (misaligned(aux, 16)) return AUSSM_E_ALIGN;
@@ -518,6 +544,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
   a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.urep = 1;
   a.urep = urep;
+  a.g16 = g16 && in_dtype == AUSSM_BF16;
   a.auxtag = aux_tag(u, delta, theta, Bc, Cc, B, D, N, L, in_dtype);
   const AuxLayout ws = aux_layout(aux, B, D, N, L, ck);
   const int mode = bwd_mode_for(B, D, N, L, ck, urep, ws.img != nullptr);
@@ -541,6 +568,12 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
       // The prepared-operand kernel needs Im(P S) from the forward call in the auxiliary buffer; its
       // workgroups leave at once if the buffer's tag says it is not there, and the kernel that
       // recomputes it (launched behind, leaving at once in the opposite case) does the work.
+      // A caller that made the forward call itself on these tensors and this buffer says so (AUSSM_AUX_FILLED), and
+      // neither of the two launches that would find nothing to do takes place (5 us each).
+      if (own_aux && aux) {
+        a.tag_mode = 0;
+        return run_px_bwd(a, ws.img, in_dtype, s);
+      }
       // (the pre-pass leaves at once when the forward call of these tensors has left the images)
       PrepArgs pa{Bc, Cc, nullptr, ws.img, N, L, (L + XT - 1) / XT, ws.stamp, img_stamp(Bc, Cc, B, N, L, in_dtype, true)};
       if (int e = run_px_prep(pa, B, in_dtype, s)) return e;
@@ -572,6 +605,7 @@ int aussm_complex_bwd(const float* dy, const float* dhL, const void* u, const vo
                       float* du, float* ddelta, float* drho, float* dtheta, float* dB, float* dC,
                       float* dD, float* dh0, const float* z, float* dz, float* workspace,
                       int B, int D, int N, int L, int ck, int in_dtype, void* stream) {
+  const int g16 = take_flag(in_dtype, AUSSM_GRADS_IN_DTYPE);
   if (int e = check_common(B, D, N, L, ck, in_dtype)) return e;
   if (ck != REC_CK) return AUSSM_E_CK;
   if (!dy || !u || !delta || !rho || !theta || !Bc || !Cc || !hck || !du || !ddelta || !drho || !dtheta ||
@@ -586,6 +620,9 @@ int aussm_complex_bwd(const float* dy, const float* dhL, const void* u, const vo
   if ((z == nullptr) != (dz == nullptr)) return AUSSM_E_NULL;
   a.z = z; a.dz = dz;
   a.B = B; a.D = D; a.N = N; a.L = L; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
+  // (several blocks of states add up in du and ddelta: those stay float)
+  if (g16 && in_dtype == AUSSM_BF16 && N > 16) return AUSSM_E_DTYPE;
+  a.g16 = g16 && in_dtype == AUSSM_BF16;
   a.ld = L; a.ns = 1;
   return launch_generic_bwd(VAR_COMPLEX, a, in_dtype, workspace, (hipStream_t)stream);
 }
@@ -596,6 +633,17 @@ int aussm_real_bwd(const float* dy, const float* dhL, const void* u, const void*
                    float* du, float* ddelta, float* dA, float* dB, float* dC, float* dD, float* dh0,
                    const float* z, float* dz, float* workspace,
                    int B, int D, int N, int L, int ck, int in_dtype, void* stream) {
+  return aussm_real_bwd_rows(dy, dhL, u, delta, A, Bm, Cm, Dskip, delta_bias, delta_softplus, h0, hck, du, ddelta, dA, dB, dC, dD, dh0, z, dz,
+                             workspace, nullptr, B, D, N, L, ck, in_dtype, stream);
+}
+
+int aussm_real_bwd_rows(const float* dy, const float* dhL, const void* u, const void* delta, const float* A,
+                   const void* Bm, const void* Cm, const float* Dskip, const float* delta_bias,
+                   int delta_softplus, const float* h0, const float* hck,
+                   float* du, float* ddelta, float* dA, float* dB, float* dC, float* dD, float* dh0,
+                   const float* z, float* dz, float* workspace, const aussm_real_rows* rows,
+                   int B, int D, int N, int L, int ck, int in_dtype, void* stream) {
+  const int g16 = take_flag(in_dtype, AUSSM_GRADS_IN_DTYPE);
   if (int e = check_common(B, D, N, L, ck, in_dtype)) return e;
   if (ck != REC_CK) return AUSSM_E_CK;
   if (!dy || !u || !delta || !A || !Bm || !Cm || !hck || !du || !ddelta || !dB || !dC) return AUSSM_E_NULL;
@@ -604,8 +652,16 @@ int aussm_real_bwd(const float* dy, const float* dhL, const void* u, const void*
   a.delta_bias = delta_bias; a.delta_softplus = delta_softplus; a.h0 = h0; a.hck = hck;
   a.du = du; a.ddelta = ddelta; a.dA = dA; a.dB = dB; a.dC = dC; a.dD = dD; a.dh0 = dh0;
   if ((z == nullptr) != (dz == nullptr)) return AUSSM_E_NULL;
+  if (int e = real_rows_check(rows, D, N, in_dtype)) return e;
+  if (rows) {
+    a.zrows = rows->z_rows; a.bcrows = rows->bc_rows; a.u_act = rows->u_silu;
+    a.dbias = rows->ddelta_bias; a.dbias_scale = rows->ddelta_bias_scale;
+  }
   a.z = z; a.dz = dz;
   a.B = B; a.D = D; a.N = N; a.L = L; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
+  // (several blocks of states add up in du and ddelta: those stay float)
+  if (g16 && in_dtype == AUSSM_BF16 && N > 16) return AUSSM_E_DTYPE;
+  a.g16 = g16 && in_dtype == AUSSM_BF16;
   a.ld = L; a.ns = 1;
   return launch_generic_bwd(VAR_REAL, a, in_dtype, workspace, (hipStream_t)stream);
 }
@@ -673,6 +729,79 @@ int aussm_gate_bwd(const float* dy, const float* y_pre, const float* z, float* d
   return run_gate(dy, y_pre, z, dy_pre, dz, n, (hipStream_t)stream);
 }
 
+int aussm_gemm(const aussm_gemm_args* g, void* stream) {
+  if (!g || !g->A || !g->B || !g->C) return AUSSM_E_NULL;
+  if (g->M < 1 || g->N < 1 || g->K < 1 || g->Z < 1 || g->nper < 1) return AUSSM_E_SHAPE;
+  if ((g->sam != 1 && g->sak != 1) || (g->sbk != 1 && g->sbn != 1) || (g->scm != 1 && g->scn != 1)) return AUSSM_E_SHAPE;
+  if (g->act != 0 && g->act != 1) return AUSSM_E_SHAPE;
+  if (g->reduce && (g->bias || g->add || g->act)) return AUSSM_E_SHAPE;
+  XGemmArgs a{};
+  a.A = g->A; a.B = g->B; a.C = g->C; a.bias = g->bias; a.add = g->add; a.alpha = g->alpha; a.bias_scale = g->bias_scale;
+  a.act = g->act; a.sam = g->sam; a.sak = g->sak; a.saz = g->saz; a.sbk = g->sbk; a.sbn = g->sbn; a.sbb = g->sbb; a.sbz = g->sbz;
+  a.scm = g->scm; a.scn = g->scn; a.scb = g->scb; a.M = g->M; a.N = g->N; a.K = g->K; a.Z = g->Z; a.nper = g->nper;
+  a.reduce = g->reduce != 0;
+  return run_xgemm(a, (hipStream_t)stream);
+}
+
+int aussm_conv_rows_fwd(const float* x, const float* w, const float* bias, float* y, int B, int D, int L, int K, long long xs_b, void* stream) {
+  if (B < 1 || D < 1 || L < 1 || K < 1 || K > CONV_MAX_K || xs_b < (long long)D * L) return AUSSM_E_SHAPE;
+  if (!x || !w || !y) return AUSSM_E_NULL;
+  if (misaligned(y, 16)) return AUSSM_E_ALIGN;
+  ConvRowsArgs a{};
+  a.x = x; a.w = w; a.bias = bias; a.y = y; a.xs_b = (long)xs_b; a.B = B; a.D = D; a.L = L; a.K = K;
+  return run_conv_rows_fwd(a, (hipStream_t)stream);
+}
+int aussm_conv_rows_bwd(const float* dy, const float* x, const float* w, float* dx, float* dw, float* dbias, int B, int D, int L, int K,
+                        long long xs_b, long long dxs_b, void* stream) {
+  if (B < 1 || D < 1 || L < 1 || K < 1 || K > CONV_MAX_K || xs_b < (long long)D * L || dxs_b < (long long)D * L) return AUSSM_E_SHAPE;
+  if (!dy || !x || !w || !dx || !dw) return AUSSM_E_NULL;
+  ConvRowsArgs a{};
+  a.dy = dy; a.x = x; a.w = w; a.dx = dx; a.dw = dw; a.dbias = dbias; a.xs_b = (long)xs_b; a.dxs_b = (long)dxs_b;
+  a.B = B; a.D = D; a.L = L; a.K = K;
+  return run_conv_rows_bwd(a, (hipStream_t)stream);
+}
+int aussm_rms_norm_fwd(const float* x, const float* w, float* y, float* rstd, size_t rows, int d, float eps, void* stream) {
+  if (rows < 1 || d < 1 || d > NORM_MAX_D) return AUSSM_E_SHAPE;
+  if (!x || !w || !y) return AUSSM_E_NULL;
+  NormArgs a{};
+  a.x = x; a.w = w; a.y = y; a.rstd = rstd; a.rows = rows; a.d = d; a.eps = eps;
+  return run_norm_fwd(a, (hipStream_t)stream);
+}
+int aussm_rms_norm_bwd(const float* dy, const float* x, const float* w, const float* rstd, const float* res, float* dx, float* dw,
+                       size_t rows, int d, void* stream) {
+  if (rows < 1 || d < 1 || d > NORM_MAX_D) return AUSSM_E_SHAPE;
+  if (!dy || !x || !w || !rstd || !dx || !dw) return AUSSM_E_NULL;
+  NormArgs a{};
+  a.dy = dy; a.x = x; a.w = w; a.rstd = const_cast<float*>(rstd); a.res = res; a.dx = dx; a.dw = dw; a.rows = rows; a.d = d;
+  return run_norm_bwd(a, (hipStream_t)stream);
+}
+int aussm_col_sum(const float* x, float* out, size_t rows, int d, float scale, void* stream) {
+  if (rows < 1 || d < 1) return AUSSM_E_SHAPE;
+  if (!x || !out) return AUSSM_E_NULL;
+  return run_col_sum(x, out, rows, d, scale, (hipStream_t)stream);
+}
+int aussm_row_sum(const float* x, float* out, size_t rows, int d, int L, float scale, void* stream) {
+  if (rows < 1 || d < 1 || L < 1) return AUSSM_E_SHAPE;
+  if (!x || !out) return AUSSM_E_NULL;
+  return run_row_sum(x, out, rows, d, L, scale, (hipStream_t)stream);
+}
+int aussm_neg_exp(const float* a_log, const float* dA, float* out, int n, void* stream) {
+  if (n < 1) return AUSSM_E_SHAPE;
+  if (!a_log || !out) return AUSSM_E_NULL;
+  return run_neg_exp(a_log, dA, out, n, (hipStream_t)stream);
+}
+int aussm_zero_many(float* const* p, const size_t* n, int count, void* stream) {
+  if (!p || !n) return AUSSM_E_NULL;
+  if (count < 0 || count > 12) return AUSSM_E_SHAPE;
+  FillArgs f{};
+  for (int i = 0; i < count; ++i) {
+    if (!n[i]) continue;
+    if (!p[i]) return AUSSM_E_NULL;
+    f.dst[f.count] = p[i]; f.src[f.count] = nullptr; f.n[f.count] = n[i]; ++f.count;
+  }
+  return run_fill(f, (hipStream_t)stream);
+}
+
 int aussm_zero_f32(float* p, size_t n, void* stream) {
   if (!p) return AUSSM_E_NULL;
   if (misaligned(p, 4)) return AUSSM_E_ALIGN;
@@ -713,31 +842,6 @@ static DropinBlocks dropin_blocks(int b, int d, int n, int L, bool largest = fal
   const size_t nc = ((size_t)ntiles + tmax - 1) / tmax;
   return DropinBlocks{bg, (int)(((size_t)ntiles + nc - 1) / nc)};
 }
-// How a GEMM launch is cut: about three workgroups of 128 x 128 per two compute units.  Without reduce_z every z is a
-// slice of its own and k is cut (at least four steps per slice); with reduce_z the z are dealt to the
-// slices first and k is cut only when there are too few z.
-constexpr long GEMM_TARGET = 384;     // workgroups per launch aimed at (measured: 256 and 512 +9 % of the backward call)
-static void gemm_slices(GemmArgs& g) {
-  const long tiles = (long)((g.M + GEMM_TILE_M - 1) / GEMM_TILE_M) * ((g.N + GEMM_TILE_N - 1) / GEMM_TILE_N);
-  const long target = GEMM_TARGET;
-  const int nk = (g.K + 31) / 32;
-  long zs = 1;                                   // slices of z
-  g.zper = 1;
-  if (g.reduce_z) {
-    zs = (target + tiles - 1) / tiles;
-    if (zs > g.Z) zs = g.Z;
-    if (zs < 1) zs = 1;
-    g.zper = (int)((g.Z + zs - 1) / zs);
-    zs = (g.Z + g.zper - 1) / g.zper;
-  } else {
-    zs = g.Z;
-  }
-  long s = (target + tiles * zs - 1) / (tiles * zs);
-  if (s > nk / 4) s = nk / 4;
-  if (s < 1) s = 1;
-  while (s > 1 && zs * s > 65535) --s;
-  g.ksplit = (int)s;
-}
 static size_t round4(size_t v) { return (v + 3) & ~(size_t)3; }
 static int dropin_check(int b, int d, int n, int L) {
   if (b < 1 || d < 1 || n < 1 || L < 1) return AUSSM_E_SHAPE;
@@ -763,12 +867,61 @@ size_t aussm_ssm_adaptive_unitary_workspace_floats(int b, int d, int n, int L, i
   if (backward) {
     const DropinBlocks k = dropin_blocks(b, d, n, L, true);
     f += 2 * round4((size_t)b * d * n) + (size_t)k.bg * k.ct * DT * d * n + (size_t)k.bg * k.ct * dropin_tile_floats(d);
-    // prepared first operands of the two products with the phase adjoints: x transposed (once per call), u of a block
-    f += 4 * (gemm_image_records(d, d * n) + (size_t)k.bg * gemm_image_records(d, k.ct * DT));
   } else {
     f += (size_t)b * dropin_fwd_chunk_tiles(b, d, L, true) * dropin_tile_floats(d);
   }
   return f;
+}
+
+// The call as the reference's operator gives it: polar parameters as they are, x and x_bias [d, n, ..], z a tensor of its own
+static aussm_operator_args operator_args(const float* u, const float* dt, const float* x, const float* x_bias, const float* B_r,
+                                         const float* B_theta, const float* C_r, const float* C_theta, const float* D, const float* z,
+                                         const float* h_re, const float* h_im, int b, int d, int n, int L) {
+  aussm_operator_args p{};
+  p.u = u; p.dt = dt; p.x = x; p.x_bias = x_bias; p.B_r = B_r; p.B_theta = B_theta; p.C_r = C_r; p.C_theta = C_theta;
+  p.D = D; p.z = z; p.h_re = h_re; p.h_im = h_im;
+  p.b = b; p.d = d; p.n = n; p.L = L; p.polar_stride = 1; p.x_scale = 1.0f;
+  return p;
+}
+static int operator_check(const aussm_operator_args* p) {
+  if (!p) return AUSSM_E_NULL;
+  if (int e = dropin_check(p->b, p->d, p->n, p->L)) return e;
+  if (!p->u || !p->dt || !p->x || !p->x_bias || !p->B_r || !p->B_theta || !p->C_r || !p->C_theta || !p->D || !p->z) return AUSSM_E_NULL;
+  if ((p->h_re == nullptr) != (p->h_im == nullptr)) return AUSSM_E_NULL;
+  if (p->polar_stride < 1 || p->z_batch_stride < 0) return AUSSM_E_SHAPE;
+  return AUSSM_OK;
+}
+static DropinArgs dropin_args(const aussm_operator_args& p) {
+  DropinArgs a{};
+  a.u = p.u; a.dt = p.dt; a.z = p.z; a.x_bias = p.x_bias; a.B_r = p.B_r; a.B_th = p.B_theta; a.C_r = p.C_r; a.C_th = p.C_theta;
+  a.Dp = p.D; a.h_re = p.h_re; a.h_im = p.h_im; a.d = p.d; a.n = p.n; a.L = p.L; a.ks = (p.d + 31) / 32; a.nb = dropin_state_blocks(p.n);
+  a.xsi = p.x_state_major ? 1 : p.n; a.xsj = p.x_state_major ? p.d : 1;
+  a.bcs = p.polar_stride; a.raw = p.radius_raw; a.zs = p.z_batch_stride ? (long)p.z_batch_stride : (long)p.d * p.L;
+  return a;
+}
+
+int aussm_operator_fwd(const aussm_operator_args* op, float* y, float* nh_re, float* nh_im, float* workspace, void* stream) {
+  if (int e = operator_check(op)) return e;
+  if (!y || !nh_re || !nh_im || !workspace) return AUSSM_E_NULL;
+  if (misaligned(workspace, 16)) return AUSSM_E_ALIGN;
+  hipStream_t s = (hipStream_t)stream;
+  const int b = op->b, d = op->d, n = op->n, L = op->L, ntiles = (L + DT - 1) / DT;
+  const int ct = dropin_fwd_chunk_tiles(b, d, L);
+  DropinArgs a = dropin_args(*op);
+  u4* xp = (u4*)workspace;
+  u4* up = (u4*)(workspace + dropin_xp_floats(d, n));
+  if (int e = run_dropin_xprep(op->x, xp, d, n, a.ks, a.nb, a.xsi, a.xsj, op->x_scale, s)) return e;
+  a.y = y; a.nh_re = nh_re; a.nh_im = nh_im; a.xp = xp; a.up = up; a.b = b;
+  // the sequence in chunks of ct tiles (one chunk unless it is long): prepared tiles of u for the chunk, then the
+  // scan over it, the state handed from chunk to chunk in the output buffers
+  for (int t0 = 0; t0 < ntiles; t0 += ct) {
+    const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
+    if (int e = run_dropin_uprep(op->u, up, d, L, a.ks, 0, b, t0, t1 - t0, s)) return e;
+    if (t0) { a.h_re = nh_re; a.h_im = nh_im; }
+    a.up_t0 = t0; a.up_nt = t1 - t0; a.t0 = t0; a.t1 = t1;
+    if (int e = run_dropin_fwd(a, s)) return e;
+  }
+  return AUSSM_OK;
 }
 
 int aussm_ssm_adaptive_unitary_fwd(const float* u, const float* dt, const float* x, const float* x_bias,
@@ -777,27 +930,102 @@ int aussm_ssm_adaptive_unitary_fwd(const float* u, const float* dt, const float*
                                    float* y, float* nh_re, float* nh_im, float* workspace,
                                    int b, int d, int n, int L, void* stream) {
   if (int e = dropin_check(b, d, n, L)) return e;
-  if (!u || !dt || !x || !x_bias || !B_r || !B_theta || !C_r || !C_theta || !D || !z || !h_re || !h_im || !y ||
-      !nh_re || !nh_im || !workspace)
+  if (!h_re || !h_im) return AUSSM_E_NULL;
+  const aussm_operator_args p = operator_args(u, dt, x, x_bias, B_r, B_theta, C_r, C_theta, D, z, h_re, h_im, b, d, n, L);
+  return aussm_operator_fwd(&p, y, nh_re, nh_im, workspace, stream);
+}
+
+int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const float* grad_nh_re, const float* grad_nh_im,
+                       const float* nh_re, const float* nh_im, const aussm_operator_grads* g, float* workspace, void* stream) {
+  if (int e = operator_check(op)) return e;
+  if (!grad_y || !g || !g->u || !g->dt || !g->x || !g->x_bias || !g->B_r || !g->B_theta || !g->C_r || !g->C_theta || !g->D || !g->z ||
+      !g->h_re || !g->h_im || !workspace)
     return AUSSM_E_NULL;
   if (misaligned(workspace, 16)) return AUSSM_E_ALIGN;
   hipStream_t s = (hipStream_t)stream;
-  const int ks = (d + 31) / 32, nb = dropin_state_blocks(n), ntiles = (L + DT - 1) / DT;
-  const int ct = dropin_fwd_chunk_tiles(b, d, L);
+  const int b = op->b, d = op->d, n = op->n, L = op->L;
+  const DropinBlocks blk = dropin_blocks(b, d, n, L);
+  const int ct = blk.ct, lc = ct * DT, ntiles = (L + DT - 1) / DT;
+  const size_t nstate = (size_t)b * d * n;
   u4* xp = (u4*)workspace;
-  u4* up = (u4*)(workspace + dropin_xp_floats(d, n));
-  if (int e = run_dropin_xprep(x, xp, d, n, ks, nb, s)) return e;
-  // the sequence in chunks of ct tiles (one chunk unless it is long): prepared tiles of u for the chunk, then the
-  // scan over it, the state handed from chunk to chunk in the output buffers
-  for (int t0 = 0; t0 < ntiles; t0 += ct) {
-    const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
-    if (int e = run_dropin_uprep(u, up, d, L, ks, 0, b, t0, t1 - t0, s)) return e;
-    DropinArgs a{};
-    a.u = u; a.dt = dt; a.z = z; a.x_bias = x_bias; a.B_r = B_r; a.B_th = B_theta; a.C_r = C_r; a.C_th = C_theta;
-    a.Dp = D; a.h_re = t0 ? nh_re : h_re; a.h_im = t0 ? nh_im : h_im; a.y = y; a.nh_re = nh_re; a.nh_im = nh_im;
-    a.xp = xp; a.up = up; a.up_b0 = 0; a.up_t0 = t0; a.up_nt = t1 - t0;
-    a.b = b; a.d = d; a.n = n; a.L = L; a.ks = ks; a.nb = nb; a.b0 = 0; a.t0 = t0; a.t1 = t1;
-    if (int e = run_dropin_fwd(a, s)) return e;
+  float* hc_re = workspace + dropin_xp_floats(d, n);
+  float* hc_im = hc_re + round4(nstate);
+  float* dth = hc_im + round4(nstate);
+  u4* up = (u4*)(dth + (size_t)blk.bg * ct * DT * d * n);
+  DropinArgs f = dropin_args(*op);
+  f.xp = xp; f.up = up;
+  if (int e = run_dropin_xprep(op->x, xp, d, n, f.ks, f.nb, f.xsi, f.xsj, op->x_scale, s)) return e;
+  FillArgs fa{};
+  auto fill = [&](float* dst, const float* src, size_t cnt) {
+    fa.dst[fa.count] = dst; fa.src[fa.count] = src; fa.n[fa.count] = cnt; ++fa.count;
+  };
+  const bool have_end = nh_re && nh_im;
+  if (have_end) {
+    fill(hc_re, nh_re, nstate);
+    fill(hc_im, nh_im, nstate);
+  }
+  fill(g->h_re, grad_nh_re, nstate);                  // the adjoint of the state travels in the output buffers
+  fill(g->h_im, grad_nh_im, nstate);
+  // the accumulated gradients start from zero; the polar ones are interleaved where their stride says so
+  fill(g->x, nullptr, (size_t)d * n * d);
+  fill(g->x_bias, nullptr, (size_t)d * n);
+  if (op->polar_stride == 1) {
+    fill(g->B_r, nullptr, n);
+    fill(g->B_theta, nullptr, n);
+    fill(g->C_r, nullptr, n);
+    fill(g->C_theta, nullptr, n);
+  } else {
+    fill(g->B_r, nullptr, (size_t)(n - 1) * op->polar_stride + 2);
+    fill(g->C_r, nullptr, (size_t)(n - 1) * op->polar_stride + 2);
+  }
+  fill(g->D, nullptr, d);
+  if (g->dt_bias) fill(g->dt_bias, nullptr, d);
+  if (int e = run_fill(fa, s)) return e;
+  const long dn = (long)d * n;
+  for (int b0 = 0; b0 < b; b0 += blk.bg) {
+    const int bg = b - b0 < blk.bg ? b - b0 : blk.bg;
+    f.b = bg; f.b0 = b0; f.up_b0 = b0;
+    if (!have_end) {
+      // the state at the end of the sequence: a forward sweep without outputs over this group's chunks
+      for (int t0 = 0; t0 < ntiles; t0 += ct) {
+        const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
+        if (int e = run_dropin_uprep(op->u, up, d, L, f.ks, b0, bg, t0, t1 - t0, s)) return e;
+        DropinArgs a = f;
+        a.y = nullptr; a.nh_re = hc_re; a.nh_im = hc_im;
+        if (t0) { a.h_re = hc_re; a.h_im = hc_im; }
+        a.up_t0 = t0; a.up_nt = t1 - t0; a.t0 = t0; a.t1 = t1;
+        if (int e = run_dropin_fwd(a, s)) return e;
+      }
+    }
+    // the chunks in reverse: chunk c covers the tiles c ct .. (same cuts as the forward sweep above)
+    for (int t0 = ((ntiles - 1) / ct) * ct; t0 >= 0; t0 -= ct) {
+      const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
+      const int l0 = t0 * DT, len = (t1 * DT < L ? t1 * DT : L) - l0;
+      if (int e = run_dropin_uprep(op->u, up, d, L, f.ks, b0, bg, t0, t1 - t0, s)) return e;
+      DropinBwdArgs q{};
+      q.f = f;
+      q.f.up_t0 = t0; q.f.up_nt = t1 - t0;
+      q.gy = grad_y; q.hc_re = hc_re; q.hc_im = hc_im; q.dth = dth;
+      q.du = g->u; q.ddt = g->dt; q.dz = g->z; q.dxb = g->x_bias;
+      q.dB_r = g->B_r; q.dB_th = g->B_theta; q.dC_r = g->C_r; q.dC_th = g->C_theta; q.dD = g->D;
+      q.dh_re = g->h_re; q.dh_im = g->h_im; q.b0 = b0; q.bg = bg; q.t0 = t0; q.t1 = t1; q.lc = lc;
+      q.dt_act = op->dt_softplus; q.ddtb = g->dt_bias; q.ddtb_scale = op->dt_bias_scale;
+      if (int e = run_dropin_bwd(q, s)) return e;
+      // grad_u[b, r, l0 + l] += scale sum_(i j) x[(i j), r] hat theta[b, (i j), l]   (rows (i j) in the order of x)
+      XGemmArgs gu{};
+      gu.A = op->x; gu.sam = 1; gu.sak = d;
+      gu.B = dth; gu.sbk = lc; gu.sbn = 1; gu.sbb = dn * lc;
+      gu.C = g->u + (size_t)b0 * d * L + l0; gu.scm = L; gu.scn = 1; gu.scb = (long)d * L;
+      gu.M = d; gu.N = bg * len; gu.K = (int)dn; gu.Z = 1; gu.nper = len; gu.reduce = 1; gu.alpha = op->x_scale;
+      if (int e = run_xgemm(gu, s)) return e;
+      // grad_x[(i j), r] += scale sum_b sum_l hat theta[b, (i j), l] u[b, r, l0 + l]
+      XGemmArgs gx{};
+      gx.A = dth; gx.sam = lc; gx.sak = 1; gx.saz = dn * lc;
+      gx.B = op->u + (size_t)b0 * d * L + l0; gx.sbk = 1; gx.sbn = L; gx.sbz = (long)d * L;
+      gx.C = g->x; gx.scm = d; gx.scn = 1;
+      gx.M = (int)dn; gx.N = d; gx.K = len; gx.Z = bg; gx.nper = d; gx.reduce = 1; gx.alpha = op->x_scale;
+      if (int e = run_xgemm(gx, s)) return e;
+    }
   }
   return AUSSM_OK;
 }
@@ -811,95 +1039,12 @@ int aussm_ssm_adaptive_unitary_bwd(const float* grad_y, const float* grad_nh_re,
                                    float* dC_r, float* dC_theta, float* dD, float* dz, float* dh_re, float* dh_im,
                                    float* workspace, int b, int d, int n, int L, void* stream) {
   if (int e = dropin_check(b, d, n, L)) return e;
-  if (!grad_y || !u || !dt || !x || !x_bias || !B_r || !B_theta || !C_r || !C_theta || !D || !z || !h_re || !h_im ||
-      !du || !ddt || !dx || !dx_bias || !dB_r || !dB_theta || !dC_r || !dC_theta || !dD || !dz || !dh_re || !dh_im ||
-      !workspace)
-    return AUSSM_E_NULL;
-  if (misaligned(workspace, 16)) return AUSSM_E_ALIGN;
-  hipStream_t s = (hipStream_t)stream;
-  const DropinBlocks blk = dropin_blocks(b, d, n, L);
-  const int ks = (d + 31) / 32, nb = dropin_state_blocks(n), ct = blk.ct, lc = ct * DT;
-  const int ntiles = (L + DT - 1) / DT;
-  const size_t nstate = (size_t)b * d * n;
-  u4* xp = (u4*)workspace;
-  float* hc_re = workspace + dropin_xp_floats(d, n);
-  float* hc_im = hc_re + round4(nstate);
-  float* dth = hc_im + round4(nstate);
-  u4* up = (u4*)(dth + (size_t)blk.bg * ct * DT * d * n);
-  u4* xt = up + (size_t)blk.bg * ct * (dropin_tile_floats(d) / 4);     // image of A(r, (i j)) = x[(i j), r]
-  u4* ui = xt + gemm_image_records(d, d * n);                          // images of A_b(r, l) = u[b, r, l0 + l] of a block
-  if (int e = run_dropin_xprep(x, xp, d, n, ks, nb, s)) return e;
-  if (int e = run_gemm_aprep(x, xt, 1, d, 0, d, d * n, 1, s)) return e;
-  DropinArgs f{};
-  f.u = u; f.dt = dt; f.z = z; f.x_bias = x_bias; f.B_r = B_r; f.B_th = B_theta; f.C_r = C_r; f.C_th = C_theta;
-  f.Dp = D; f.xp = xp; f.up = up; f.d = d; f.n = n; f.L = L; f.ks = ks; f.nb = nb;
-  FillArgs fa{};
-  auto fill = [&](float* dst, const float* src, size_t cnt) {
-    fa.dst[fa.count] = dst; fa.src[fa.count] = src; fa.n[fa.count] = cnt; ++fa.count;
-  };
-  const bool have_end = nh_re && nh_im;
-  if (have_end) {
-    fill(hc_re, nh_re, nstate);
-    fill(hc_im, nh_im, nstate);
-  }
-  fill(dh_re, grad_nh_re, nstate);                  // the adjoint of the state travels in the output buffers
-  fill(dh_im, grad_nh_im, nstate);
-  fill(dx, nullptr, (size_t)d * n * d);
-  fill(dx_bias, nullptr, (size_t)d * n);
-  fill(dB_r, nullptr, n);
-  fill(dB_theta, nullptr, n);
-  fill(dC_r, nullptr, n);
-  fill(dC_theta, nullptr, n);
-  fill(dD, nullptr, d);
-  if (int e = run_fill(fa, s)) return e;
-  const long dn = (long)d * n;
-  for (int b0 = 0; b0 < b; b0 += blk.bg) {
-    const int bg = b - b0 < blk.bg ? b - b0 : blk.bg;
-    f.b = bg; f.b0 = b0; f.up_b0 = b0;
-    if (!have_end) {
-      // the state at the end of the sequence: a forward sweep without outputs over this group's chunks
-      for (int t0 = 0; t0 < ntiles; t0 += ct) {
-        const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
-        if (int e = run_dropin_uprep(u, up, d, L, ks, b0, bg, t0, t1 - t0, s)) return e;
-        DropinArgs a = f;
-        a.h_re = t0 ? hc_re : h_re; a.h_im = t0 ? hc_im : h_im; a.y = nullptr; a.nh_re = hc_re; a.nh_im = hc_im;
-        a.up_t0 = t0; a.up_nt = t1 - t0; a.t0 = t0; a.t1 = t1;
-        if (int e = run_dropin_fwd(a, s)) return e;
-      }
-    }
-    // the chunks in reverse: chunk c covers the tiles c ct .. (same cuts as the forward sweep above)
-    for (int t0 = ((ntiles - 1) / ct) * ct; t0 >= 0; t0 -= ct) {
-      const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
-      const int l0 = t0 * DT, len = (t1 * DT < L ? t1 * DT : L) - l0;
-      if (int e = run_dropin_uprep(u, up, d, L, ks, b0, bg, t0, t1 - t0, s)) return e;
-      DropinBwdArgs q{};
-      q.f = f;
-      q.f.up_t0 = t0; q.f.up_nt = t1 - t0;
-      q.gy = grad_y; q.hc_re = hc_re; q.hc_im = hc_im; q.dth = dth;
-      q.du = du; q.ddt = ddt; q.dz = dz; q.dxb = dx_bias;
-      q.dB_r = dB_r; q.dB_th = dB_theta; q.dC_r = dC_r; q.dC_th = dC_theta; q.dD = dD;
-      q.dh_re = dh_re; q.dh_im = dh_im; q.b0 = b0; q.bg = bg; q.t0 = t0; q.t1 = t1; q.lc = lc;
-      if (int e = run_dropin_bwd(q, s)) return e;
-      // grad_u[b, r, l0 + l] += sum_(i j) x[(i j), r] hat theta[b, (i j), l]
-      GemmArgs gu{};
-      gu.Aimg = xt; gu.simz = 0;
-      gu.Bm = dth; gu.sbk = lc; gu.sbn = 1; gu.sbz = dn * lc;
-      gu.C = du + (size_t)b0 * d * L + l0; gu.scm = L; gu.scn = 1; gu.scz = (long)d * L;
-      gu.M = d; gu.N = len; gu.K = (int)dn; gu.Z = bg; gu.reduce_z = 0; gu.accumulate = 1; gu.tr = 0;
-      gemm_slices(gu);
-      if (int e = run_split_gemm(gu, s)) return e;
-      // grad_x[(i j), r] += sum_b sum_l u[b, r, l0 + l] hat theta[b, (i j), l]: rows r, columns (i j), C contiguous along r
-      if (int e = run_gemm_aprep(u + (size_t)b0 * d * L + l0, ui, L, 1, (long)d * L, d, len, bg, s)) return e;
-      GemmArgs gx{};
-      gx.Aimg = ui; gx.simz = (long)gemm_image_records(d, len);
-      gx.Bm = dth; gx.sbk = 1; gx.sbn = lc; gx.sbz = dn * lc;
-      gx.C = dx; gx.scm = 1; gx.scn = d; gx.scz = 0;
-      gx.M = d; gx.N = (int)dn; gx.K = len; gx.Z = bg; gx.reduce_z = 1; gx.accumulate = 1; gx.tr = 1;
-      gemm_slices(gx);
-      if (int e = run_split_gemm(gx, s)) return e;
-    }
-  }
-  return AUSSM_OK;
+  if (!h_re || !h_im) return AUSSM_E_NULL;
+  const aussm_operator_args p = operator_args(u, dt, x, x_bias, B_r, B_theta, C_r, C_theta, D, z, h_re, h_im, b, d, n, L);
+  aussm_operator_grads g{};
+  g.u = du; g.dt = ddt; g.x = dx; g.x_bias = dx_bias; g.B_r = dB_r; g.B_theta = dB_theta; g.C_r = dC_r; g.C_theta = dC_theta;
+  g.D = dD; g.z = dz; g.h_re = dh_re; g.h_im = dh_im;
+  return aussm_operator_bwd(&p, grad_y, grad_nh_re, grad_nh_im, nh_re, nh_im, &g, workspace, stream);
 }
 
 }  // extern "C"

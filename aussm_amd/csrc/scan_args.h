@@ -63,6 +63,9 @@ struct FwdArgs {
   int hs, ho;                // matrix-core kernels: h0 of pair b is entry b * hs + ho of the state array
   int urep;                  // generic kernels: u and delta are [B / urep, D, L], shared by urep consecutive batch elements
   uint32_t auxtag;           // what a kernel that fills aux writes behind it (aux_tag of the call)
+  // vector-ALU kernels: rows per batch element of the tensors z and B_t / C_t lie in (0: D and N, tensors of their own),
+  // and whether the scan's input is silu(u)
+  int zrows, bcrows, u_act;
 };
 
 struct UniBwdArgs {
@@ -87,6 +90,7 @@ struct UniBwdArgs {
   int tag_mode;         // matrix-core kernels: 0 use the auxiliary buffer if its tag is valid; 1 leave at once
                         // unless it is; 2 leave at once if it is
   uint32_t auxtag;      // the tag a forward call of the same arguments leaves behind aux (aux_tag)
+  int g16;              // du and ddelta leave in bf16 (inputs in bf16)
 };
 
 struct RecBwdArgs {
@@ -103,7 +107,7 @@ struct RecBwdArgs {
   const float* delta_bias;  // [D] or null (real)
   const float* h0;          // [B,D,N,C] or null
   const float* hck;         // [B,nck,N,C,D], ck == 16
-  float *du, *ddelta;       // [B,D,L]
+  float *du, *ddelta;       // [B,D,L] (bf16 with g16)
   float *dtheta, *drho;     // [B,D,L] (complex)
   float* dA;                // [D,N] (real), accumulated into
   float *dB, *dC;           // [B,N,L(,2)], accumulated into
@@ -121,6 +125,10 @@ struct RecBwdArgs {
   // (du, ddelta, dtheta, drho) are added to what the earlier blocks wrote, and the terms that do not
   // depend on the state (the D skip, dD) are left out.
   int nbase, accum;
+  int zrows, bcrows, u_act;  // as FwdArgs, for z / dz, B_t / C_t / dB / dC and u / du
+  float* dbias;              // [D] or null (real): dbias_scale times the sum of ddelta over (batch, step) is added
+  float dbias_scale;
+  int g16;                   // du and ddelta leave in bf16 (inputs in bf16, states in one launch)
 };
 
 // Adjoint of the state entering a segment, from a zero adjoint at its end (complex and real scans)
@@ -136,6 +144,7 @@ struct AdjSegArgs {
   float* out;               // [B*ns,D,N,C]
   float* ptot;              // [B*ns,D,2]  as FwdArgs::ptot
   int D, N, L, ld, ns, ncg, delta_softplus;   // L: segment length (the last one may be shorter)
+  int zrows, bcrows;        // as FwdArgs
 };
 
 struct SegArgs {

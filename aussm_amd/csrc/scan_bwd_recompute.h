@@ -153,7 +153,9 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   float* red = s_red + (VALU_SUMS ? 0 : wave * 64 * (WIDE ? RED16_RS : RED_RS));
   float4* part = s_part + (WIDE ? 0 : wave * RT * TS);
   float* slab = s_slab + (WIDE ? wave * SLAB : 0);
-  const size_t row_base = ((size_t)b * N + n0) * ld + lbeg;
+  const size_t row_base = ((size_t)b * ((VAR == VAR_REAL && p.bcrows) ? p.bcrows : N) + n0) * ld + lbeg;
+  // z and dz may be rows of a wider tensor: every address below is formed for rows of their own
+  const size_t zoff = (VAR == VAR_REAL && p.zrows) ? (size_t)b * (p.zrows - p.D) * ld : 0;
 
   // ---- per-lane constants and accumulators
   float a2[NW], an[NW], dAacc[NW], gr[NW], gi[NW];
@@ -200,7 +202,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   const int col = tid % RT, row0 = tid / RT;
   struct RawTile { Tin u[E], dl[E]; float th[E], rho[E], gy[E], zz[E]; };
   RawTile rdy, fly;
-  float dsk[E], dbias[E], accD[E];
+  float dsk[E], dbias[E], accD[E], accB[E];
   size_t goff[E];
   bool rowok[E];
 #pragma unroll
@@ -210,7 +212,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
     goff[k] = ((size_t)b * D + (rowok[k] ? dd : 0)) * ld + lbeg;
     dsk[k] = (p.Dskip && rowok[k]) ? p.Dskip[dd] : 0.f;
     dbias[k] = (VAR == VAR_REAL && p.delta_bias && rowok[k]) ? p.delta_bias[dd] : 0.f;
-    accD[k] = 0.f;
+    accD[k] = 0.f; accB[k] = 0.f;
     rdy.u[k] = rdy.dl[k] = fly.u[k] = fly.dl[k] = Tin(0);
     rdy.th[k] = rdy.rho[k] = rdy.gy[k] = fly.th[k] = fly.rho[k] = fly.gy[k] = 0.f;
     rdy.zz[k] = fly.zz[k] = 0.f;
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       r.u[k] = gu[o];
       r.dl[k] = gdl[o];
       r.gy[k] = p.dy[o];
-      if (p.z) r.zz[k] = p.z[o];
+      if (p.z) r.zz[k] = p.z[o + zoff];
       if (VAR == VAR_COMPLEX) { r.th[k] = p.theta[o]; r.rho[k] = p.rho[o]; }
     }
   };
@@ -271,11 +273,15 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
     if (warm_next) warm.issue(gB, gC, row_base + l0 - RT, ld);
 
     // ---- stage
-    float eu[E], edl[E], egy[E], eraw[E], egz[E];       // egz: dy silu'(z), for dz
+    float eu[E], edl[E], egy[E], eraw[E], egz[E], eact[E];   // egz: dy silu'(z), for dz; eact: silu'(u)
 #pragma unroll
     for (int k = 0; k < E; ++k) {
       const bool ok = rowok[k] && l0 + col < L;
       eu[k] = ok ? to_f32(rdy.u[k]) : 0.f;
+      if (VAR == VAR_REAL && p.u_act) {                    // uniform
+        eact[k] = dsiluf_(eu[k]);
+        eu[k] = siluf_(eu[k]);
+      }
       egy[k] = ok ? rdy.gy[k] : 0.f;
       egz[k] = 0.f;
       if (p.z) {                                           // uniform
@@ -548,19 +554,28 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       if (rowok[k] && ll < L) {
         const size_t o = goff[k] + ll;
         const bool acc = p.accum != 0;                   // uniform
-        p.du[o] = acc ? fmaf(kk, edl[k], p.du[o]) : fmaf(kk, edl[k], dsk[k] * egy[k]);
+        float duv = acc ? kk * edl[k] : fmaf(kk, edl[k], dsk[k] * egy[k]);
+        float dd = kk * eu[k];
+        if (VAR == VAR_REAL && p.u_act) duv *= eact[k];
         if (VAR == VAR_REAL) {
-          float dd = fmaf(kk, eu[k], xx);
+          dd += xx;
           if (p.delta_softplus) dd *= (eraw[k] > 20.0f) ? 1.0f : sigmoidf_(eraw[k]);
-          p.ddelta[o] = acc ? p.ddelta[o] + dd : dd;
+          accB[k] += dd;
+        }
+        if (sizeof(Tin) == 2 && p.g16) {                   // uniform
+          reinterpret_cast<bf16_t*>(p.du)[o] = to_bf16(duv);
+          reinterpret_cast<bf16_t*>(p.ddelta)[o] = to_bf16(dd);
         } else {
-          p.ddelta[o] = acc ? fmaf(kk, eu[k], p.ddelta[o]) : kk * eu[k];
+          p.du[o] = acc ? p.du[o] + duv : duv;
+          p.ddelta[o] = acc ? p.ddelta[o] + dd : dd;
+        }
+        if (VAR == VAR_COMPLEX) {
           p.dtheta[o] = acc ? p.dtheta[o] + xx : xx;
           p.drho[o] = acc ? p.drho[o] + zz : zz;
         }
         if (p.dz) {                                        // y_pre = sum over the states + D u (the latter once)
           const float dzv = egz[k] * (acc ? yy : fmaf(dsk[k], eu[k], yy));
-          p.dz[o] = acc ? p.dz[o] + dzv : dzv;
+          p.dz[o + zoff] = acc ? p.dz[o + zoff] + dzv : dzv;
         }
         accD[k] = fmaf(egy[k], eu[k], accD[k]);
       }
@@ -589,6 +604,15 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
 #pragma unroll
       for (int o = RT / 2; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
       if (col == 0 && rowok[k]) atomicAdd(p.dD + d0 + row0 + k * RSTEP, s);
+    }
+  }
+  if (VAR == VAR_REAL && p.dbias) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      float s = accB[k];
+#pragma unroll
+      for (int o = RT / 2; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (col == 0 && rowok[k]) atomicAdd(p.dbias + d0 + row0 + k * RSTEP, p.dbias_scale * s);
     }
   }
 }

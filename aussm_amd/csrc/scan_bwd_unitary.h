@@ -383,8 +383,14 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
       for (int w = 0; w < NWV; ++w) { kk += pv[k][w].x; qq += pv[k][w].y; }
       if (rowok[k] && ll < L) {
         const size_t o = goff[k] + ll;
-        p.du[o] = fmaf(kk, edl[k], dsk[k] * egy[k]);
-        p.ddelta[o] = kk * eu[k];
+        const float duv = fmaf(kk, edl[k], dsk[k] * egy[k]), ddv = kk * eu[k];
+        if (sizeof(Tin) == 2 && p.g16) {                   // uniform
+          reinterpret_cast<bf16_t*>(p.du)[o] = to_bf16(duv);
+          reinterpret_cast<bf16_t*>(p.ddelta)[o] = to_bf16(ddv);
+        } else {
+          p.du[o] = duv;
+          p.ddelta[o] = ddv;
+        }
         p.dtheta[o] = qq;
         accD[k] = fmaf(egy[k], eu[k], accD[k]);
       }

@@ -682,8 +682,8 @@ __global__ __launch_bounds__(256) void unitary_bwd_xdl_kernel(const UniBwdArgs p
       for (int st = 0; st < 2; ++st) {
         const int l = l0 + 16 * st + 4 * g;
         if (l < L) {
-          *reinterpret_cast<f4*>(p.du + row + l) = o_du[st];
-          *reinterpret_cast<f4*>(p.ddelta + row + l) = o_dd[st];
+          store_grad4<Tin>(p.du, 4 * (row + l), o_du[st], p.g16);
+          store_grad4<Tin>(p.ddelta, 4 * (row + l), o_dd[st], p.g16);
           *reinterpret_cast<f4*>(p.dtheta + row + l) = o_dt[st];
         }
       }

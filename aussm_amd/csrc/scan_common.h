@@ -29,6 +29,12 @@ typedef uint16_t bf16_t;
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(bf16_t v) { return __uint_as_float(((uint32_t)v) << 16); }
 
+// round to nearest even (finite values; a NaN keeps its sign and stays one)
+__device__ __forceinline__ bf16_t to_bf16(float v) {
+  typedef __bf16 b1;
+  return __builtin_bit_cast(bf16_t, (b1)v);
+}
+
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
 // Workgroups are dealt round-robin to the XCDs (workgroup i runs on XCD i % 8).  Remap so that
@@ -320,6 +326,18 @@ __device__ __forceinline__ void store4(float* __restrict__ p, size_t o, const fl
 }
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+// four consecutive results at byte offset ob (of a float tensor): float, or bf16 at half the offset (g16, uniform)
+template <typename Tin>
+__device__ __forceinline__ void store_grad4(float* p, size_t ob, const f4& v, int g16) {
+  if (sizeof(Tin) == 2 && g16) {
+    uint2 w;
+    w.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
+    w.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
+    *reinterpret_cast<uint2*>(reinterpret_cast<char*>(p) + ob / 2) = w;
+  } else {
+    *reinterpret_cast<f4*>(reinterpret_cast<char*>(p) + ob) = v;
+  }
+}
 
 // sin and cos without the large-argument branch: the caller keeps |x| below ~150.
 __device__ __forceinline__ void sincos_small(float x, float* sn, float* cs) {

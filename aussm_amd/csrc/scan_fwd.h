@@ -46,6 +46,9 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
   const Tbc* __restrict__ gB = static_cast<const Tbc*>(p.Bm);
   const Tbc* __restrict__ gC = static_cast<const Tbc*>(p.Cm);
 
+  // z may be rows of a wider tensor: every address below is formed for rows of its own
+  const float* __restrict__ gz = p.z ? p.z + ((VAR == VAR_REAL && p.zrows) ? (size_t)b * (p.zrows - p.D) * ld : 0) : nullptr;
+
   // ---- scan-side state (lane == channel)
   float hr[NW], hi[NW], a2[NW];
 #pragma unroll
@@ -109,7 +112,7 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
       r.dl[k].load(gdl, o, vec, idx);
       if (VAR != VAR_REAL) r.th[k].load(p.theta, o, vec, idx);
       if (VAR == VAR_COMPLEX) r.rho[k].load(p.rho, o, vec, idx);
-      if (p.z) r.z[k].load(p.z, o, vec, idx);
+      if (p.z) r.z[k].load(gz, o, vec, idx);
     }
   };
   // A use of every register of a set: the compiler puts its wait for the loads here.
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
   constexpr int RB = (int)sizeof(Tbc) * C;
   const bool full_group = active && n0 + NW <= N;
   TileWarm<WARM ? NW : 1, RB> warm;
-  const size_t bc_row = ((size_t)b * N + n0) * ld + lbeg;   // B_t / C_t: row n0, first step of the segment
+  const size_t bc_row = ((size_t)b * ((VAR == VAR_REAL && p.bcrows) ? p.bcrows : N) + n0) * ld + lbeg;   // B_t / C_t: row n0, first step of the segment
   if (WARM && full_group && T <= L) {
     warm.issue(gB, gC, bc_row, ld);
     warm.retire();
@@ -161,7 +164,8 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const bool ok = rowok[k] && l0 + t0 + i < L;
-        const float uu = ok ? rdy.u[k].get(i) : 0.f;
+        float uu = ok ? rdy.u[k].get(i) : 0.f;
+        if (VAR == VAR_REAL && p.u_act) uu = siluf_(uu);
         float dl = ok ? rdy.dl[k].get(i) : 0.f;
         float4 rec;
         if (VAR == VAR_REAL) {

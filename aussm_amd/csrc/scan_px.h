@@ -984,8 +984,8 @@ __global__ __launch_bounds__(512) void unitary_bwd_px_kernel(const UniBwdArgs p,
               o_dt[k] = gth[e] + (st ? offb : offa);
             }
             const size_t ob = (size_t)(rowf + (uint32_t)l * 4);
-            *reinterpret_cast<f4*>(reinterpret_cast<char*>(p.du) + ob) = o_du;
-            *reinterpret_cast<f4*>(reinterpret_cast<char*>(p.ddelta) + ob) = o_dd;
+            store_grad4<Tin>(p.du, ob, o_du, p.g16);
+            store_grad4<Tin>(p.ddelta, ob, o_dd, p.g16);
             *reinterpret_cast<f4*>(reinterpret_cast<char*>(p.dtheta) + ob) = o_dt;
           }
         }

@@ -68,6 +68,9 @@ __global__ __launch_bounds__(256) void adjoint_seg_kernel(const AdjSegArgs p) {
     dbias[k] = (VAR == VAR_REAL && p.delta_bias && rowok[k]) ? p.delta_bias[dd] : 0.f;
   }
 
+  const size_t zoff = p.zrows ? (size_t)b * (p.zrows - p.D) * ld : 0;   // (z may be rows of a wider tensor)
+  const int bcrows = p.bcrows ? p.bcrows : N;
+
   const int ntiles = (L + RT - 1) / RT;
   for (int it = ntiles - 1; it >= 0; --it) {
     const int l0 = it * RT;
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(256) void adjoint_seg_kernel(const AdjSegArgs p) {
       const bool ok = rowok[k] && l0 + col < L;
       const size_t o = goff[k] + ((l0 + col < L) ? l0 + col : L - 1);
       float gy = ok ? p.dy[o] : 0.f;
-      if (p.z) gy *= siluf_(p.z[o]);
+      if (p.z) gy *= siluf_(p.z[o + zoff]);
       float4 rec;
       if (VAR == VAR_REAL) {
         float dl = to_f32(gdl[o]) + dbias[k];
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(256) void adjoint_seg_kernel(const AdjSegArgs p) {
       for (int k = 0; k < ADJ_NSW; ++k) {
         const int n = wave + 4 * k;
         if (n < N) {                             // wave-uniform
-          const size_t row = ((size_t)b * N + n) * ld + lbeg;
+          const size_t row = ((size_t)b * bcrows + n) * ld + lbeg;
           if constexpr (VAR == VAR_REAL) {
             const f32x8 cc = ld_r8_safe(gC, row, l0 + g * TG, L);
 #pragma unroll

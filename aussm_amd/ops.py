@@ -258,6 +258,12 @@ def ssm_adaptive_interface(u: Tensor, dt: Tensor, x: Tensor, x_bias: Tensor, B: 
         raise ValueError("max_parallel_length must be positive")
     b, d, l = u.shape
     n = x.shape[1]
+    if (l <= max_parallel_length and not save_intermediates and u.is_cuda and B.dtype is torch.complex64
+            and C.dtype is torch.complex64 and not torch.compiler.is_compiling() and type(u) is Tensor):
+        # one launch sequence: the operator as one graph node, its softplus and zero start state inside the kernels
+        host = L.host()
+        if host.operator_supported(b, d, n, l):
+            return host.adaptive_operator(u, dt, x, x_bias, B, C, D, z)
     B_r = F.softplus(B.real).contiguous()
     B_theta = B.imag.contiguous()
     C_r = F.softplus(C.real).contiguous()

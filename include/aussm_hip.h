@@ -38,6 +38,13 @@ extern "C" {
 
 #define AUSSM_F32 0
 #define AUSSM_BF16 1
+/* Flags or-ed into in_dtype of the backward calls:
+ *  AUSSM_GRADS_IN_DTYPE  du and ddelta are tensors of the input type (bf16 inputs; complex and real scans: N <= 16)
+ *  AUSSM_AUX_FILLED      (aussm_unitary_bwd_aux) the caller made the forward call on the same tensors with this aux and ck,
+ *                        every tensor is 16-byte aligned and aussm_unitary_kernel_mode() answers 6 in both directions:
+ *                        the launches that check what the buffer holds are left out */
+#define AUSSM_GRADS_IN_DTYPE 0x100
+#define AUSSM_AUX_FILLED 0x200
 
 #define AUSSM_OK 0
 #define AUSSM_E_NULL (-1)      /* a required pointer is NULL                         */
@@ -321,6 +328,96 @@ int aussm_swap_last2_act(const float* x, const float* bias, const float* pre, fl
  * gradients runs these two around them (in place is allowed: y may be y_pre, dy_pre may be dy). */
 int aussm_gate_fwd(const float* y_pre, const float* z, float* y, size_t n, void* stream);
 int aussm_gate_bwd(const float* dy, const float* y_pre, const float* z, float* dy_pre, float* dz, size_t n, void* stream);
+
+/* The operator above with the conventions of its callers (ai-modules/wavesAI/model/aussm.py:808-902) taken into the
+ * kernels, so that nothing is converted or copied around it:
+ *   polar_stride    elements between consecutive states of B_r, B_theta, C_r, C_theta (2: the parts of a complex tensor)
+ *   radius_raw      B_r and C_r are given before their softplus (and so are their gradients)
+ *   x_state_major   x is [n, d, d] and x_bias [n, d] (rows of the xA projection's weight) instead of [d, n, ..]
+ *   x_scale         x enters multiplied by it
+ *   z_batch_stride  elements between batch elements of z and of its gradient (0: d L)
+ *   dt_softplus     dt is a softplus: the backward call returns the gradient of its argument and, in dt_bias
+ *                   (optional), dt_bias_scale times the sum of that gradient over batch and sequence, per channel
+ * h_re / h_im may be NULL (zero start state).  Workspace: aussm_ssm_adaptive_unitary_workspace_floats. */
+typedef struct aussm_operator_args {
+  const float *u, *dt, *x, *x_bias, *B_r, *B_theta, *C_r, *C_theta, *D, *z, *h_re, *h_im;
+  int b, d, n, L;
+  int polar_stride, radius_raw, x_state_major, dt_softplus;
+  float x_scale, dt_bias_scale;
+  long long z_batch_stride;
+} aussm_operator_args;
+typedef struct aussm_operator_grads {
+  float *u, *dt, *x, *x_bias, *B_r, *B_theta, *C_r, *C_theta, *D, *z, *h_re, *h_im, *dt_bias;
+} aussm_operator_grads;
+int aussm_operator_fwd(const aussm_operator_args* op, float* y, float* nh_re, float* nh_im, float* workspace, void* stream);
+int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const float* grad_nh_re, const float* grad_nh_im,
+                       const float* nh_re, const float* nh_im, const aussm_operator_grads* grads, float* workspace, void* stream);
+
+/* ---------------------------------------------------------------------------------------
+ * fp32-accurate matrix products of the blocks' linear layers (bf16 matrix cores on operands split into three exact
+ * pieces, fp32 sums): nn.Linear of ai-modules/wavesAI/model/aussm.py:725-737, :813-828 and its gradients.
+ *     C(m, n) = act( alpha sum_k A(m, k) B(k, n) + bias_scale bias[m] + add(m, n) )
+ * Column n lies in batch n / nper, at position n % nper: B and C move by sbb / scb per batch and by sbn / scn per
+ * position (one A for a batch of products).  With Z > 1 the product is also summed over z (A, B move by saz, sbz).
+ * reduce != 0: C is added to, and a long sum over few tiles is cut over workgroups (float atomics; no bias, add, act).
+ * Strides count elements; one of sam / sak, one of sbk / sbn and one of scm / scn is 1.  act: 0 none, 1 softplus.
+ * ------------------------------------------------------------------------------------- */
+typedef struct aussm_gemm_args {
+  const float* A;
+  const float* B;
+  float* C;
+  const float* bias;      /* [M] or NULL */
+  const float* add;       /* laid out as C (may be C) or NULL */
+  float alpha, bias_scale;
+  int act, reduce;
+  long long sam, sak, saz, sbk, sbn, sbb, sbz, scm, scn, scb;
+  int M, N, K, Z, nper;
+} aussm_gemm_args;
+int aussm_gemm(const aussm_gemm_args* args, void* stream);
+
+/* ---------------------------------------------------------------------------------------
+ * What the blocks do around the scans, on channel rows (rows of L elements, the scans' layout).
+ * Depthwise causal convolution (aussm.py:762, :863) of rows (b, i) at x + b xs_b + i L; y, dy [B, D, L], the gradient of
+ * x at dx + b dxs_b + i L; dw, dbias accumulated into.  K <= 8; D rows per batch element.
+ * Root-mean-square norm (aussm.py:905-916) over rows of d <= 1024 elements; rstd [rows] is what the backward call takes;
+ * res (optional) is added to dx; dw accumulated into.
+ * Sums of columns / rows: out[c] += scale sum_r x[r, c];  out[r % d] += scale sum_l x[r, l].
+ * aussm_neg_exp: dA NULL: out = -exp(a_log), else out = dA * -exp(a_log).
+ * aussm_zero_many: up to 12 buffers set to zero with one launch.
+ * ------------------------------------------------------------------------------------- */
+int aussm_conv_rows_fwd(const float* x, const float* w, const float* bias, float* y, int B, int D, int L, int K, long long xs_b, void* stream);
+int aussm_conv_rows_bwd(const float* dy, const float* x, const float* w, float* dx, float* dw, float* dbias, int B, int D, int L, int K,
+                        long long xs_b, long long dxs_b, void* stream);
+int aussm_rms_norm_fwd(const float* x, const float* w, float* y, float* rstd, size_t rows, int d, float eps, void* stream);
+int aussm_rms_norm_bwd(const float* dy, const float* x, const float* w, const float* rstd, const float* res, float* dx, float* dw,
+                       size_t rows, int d, void* stream);
+int aussm_col_sum(const float* x, float* out, size_t rows, int d, float scale, void* stream);
+int aussm_row_sum(const float* x, float* out, size_t rows, int d, int L, float scale, void* stream);
+int aussm_neg_exp(const float* a_log, const float* dA, float* out, int n, void* stream);
+int aussm_zero_many(float* const* p, const size_t* n, int count, void* stream);
+
+/* The real scan as the Mamba block calls it, tensors that are rows of wider ones included (all fields 0: the plain call):
+ *   z_rows, bc_rows  rows per batch element of the tensors that z (dz) and B, C (dB, dC) are rows of
+ *   u_silu           the scan's input is silu(u); du is the gradient of u
+ *   ddelta_bias      (backward) [D]: ddelta_bias_scale times the sum of ddelta over batch and sequence is added to it */
+typedef struct aussm_real_rows {
+  int z_rows, bc_rows, u_silu;
+  float* ddelta_bias;
+  float ddelta_bias_scale;
+} aussm_real_rows;
+int aussm_real_fwd_rows(const void* u, const void* delta, const float* A,
+                        const void* Bm, const void* Cm, const float* Dskip, const float* z,
+                        const float* delta_bias, int delta_softplus,
+                        const float* h0, float* y, float* hL, float* hck, float* workspace, const aussm_real_rows* rows,
+                        int B, int D, int N, int L, int ck, int in_dtype, void* stream);
+int aussm_real_bwd_rows(const float* dy, const float* dhL,
+                        const void* u, const void* delta, const float* A,
+                        const void* Bm, const void* Cm, const float* Dskip,
+                        const float* delta_bias, int delta_softplus,
+                        const float* h0, const float* hck,
+                        float* du, float* ddelta, float* dA, float* dB, float* dC,
+                        float* dD, float* dh0, const float* z, float* dz, float* workspace, const aussm_real_rows* rows,
+                        int B, int D, int N, int L, int ck, int in_dtype, void* stream);
 
 /* Sets n floats to zero with one launch (a kernel, not a memory-set node, so a call may be recorded in a graph):
  * the buffers that the backward calls above accumulate into. */

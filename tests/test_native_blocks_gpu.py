@@ -1,0 +1,135 @@
+"""The native route of the blocks: its products, convolution and norm against float64, and whole blocks against the
+same layers composed one by one (which tests/test_blocks.py holds to the oracle)."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, want):
+    return float((a.double() - want).norm() / want.norm())
+
+
+def _gemm(A, B, C, M, N, K, sa, sb, sc, **kw):
+    from aussm_amd import _lib, scan
+    a = dict(alpha=1.0, bias_scale=1.0, Z=1, nper=N, sam=sa[0], sak=sa[1], sbk=sb[0], sbn=sb[1], scm=sc[0], scn=sc[1])
+    a.update({k: (v.data_ptr() if torch.is_tensor(v) else v) for k, v in kw.items()})
+    g = _lib.GemmArgs(A=A.data_ptr(), B=B.data_ptr(), C=C.data_ptr(), M=M, N=N, K=K, **a)
+    _lib.check(_lib.load().aussm_gemm(ctypes.byref(g), ctypes.c_void_p(scan._stream())), "aussm_gemm")
+
+
+# (batch, length, inner, outer): one step and partial steps along k, partial tiles, batches smaller than a tile and
+# not a multiple of four, K not a multiple of four
+SHAPES = [(1, 1, 1, 1), (3, 5, 7, 3), (2, 128, 32, 128), (2, 129, 33, 65), (5, 77, 21, 130), (2, 720, 64, 200), (9, 10, 260, 31)]
+
+
+@pytest.mark.parametrize("b,l,i,o", SHAPES)
+def test_products_of_a_linear_layer(b, l, i, o):
+    """All operand orders the blocks use.  Three bf16 pieces per operand drop less than 2^-26 of a product, the sums
+    are fp32: relative error below 1e-6 for sums of up to a few thousand terms."""
+    print(f"case gemm b={b} l={l} i={i} o={o}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(b * l + i)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    X, W, bias, dY = rn(b, l, i), rn(o, i), rn(o), rn(b, o, l)
+    # rows of the output: Y[b] = softplus(W X[b]^T + 2 bias)
+    Y = torch.full((b, o, l), float("nan"), device="cuda")
+    kw = dict(nper=l, sbb=l * i, scb=o * l)
+    _gemm(W, X, Y, o, b * l, i, (i, 1), (1, i), (l, 1), bias=bias, bias_scale=2.0, act=1, **kw)
+    pre = (X.double() @ W.double().t() + 2 * bias.double()).transpose(1, 2)
+    assert _rel(Y, torch.nn.functional.softplus(pre)) < 2e-6
+    # ... added to what is there
+    Z = rn(b, o, l)
+    want = Z.double() + pre - 2 * bias.double()[:, None]
+    _gemm(W, X, Z, o, b * l, i, (i, 1), (1, i), (l, 1), add=Z, **kw)
+    assert _rel(Z, want) < 1e-6
+    # gradient of the input from channel rows: dX[b] = dY[b]^T W, contiguous along the product's rows
+    dX = torch.full((b, l, i), float("nan"), device="cuda")
+    _gemm(W, dY, dX, i, b * l, o, (1, i), (l, 1), (1, i), nper=l, sbb=o * l, scb=l * i)
+    assert _rel(dX, dY.double().transpose(1, 2) @ W.double()) < 1e-6
+    # weight gradient, summed over the batch: from channel rows, and from sequence rows
+    want = torch.einsum("bol,bli->oi", dY.double(), X.double())
+    dW = torch.zeros(o, i, device="cuda")
+    _gemm(dY, X, dW, o, i, l, (l, 1), (i, 1), (i, 1), Z=b, saz=o * l, sbz=l * i, reduce=1)
+    assert _rel(dW, want) < 2e-6
+    dW.zero_()
+    dYs = dY.transpose(1, 2).contiguous()
+    _gemm(dYs, X, dW, o, i, b * l, (1, o), (i, 1), (i, 1), reduce=1)
+    assert _rel(dW, want) < 2e-6
+
+
+@pytest.mark.parametrize("B,D,L,K", [(1, 1, 1, 4), (2, 5, 3, 4), (3, 70, 130, 4), (2, 9, 2050, 4), (2, 8, 33, 3), (1, 4, 7, 8)])
+def test_convolution_of_channel_rows(B, D, L, K):
+    from aussm_amd import _lib, scan
+    lib, P = _lib.load(), _lib.ptr
+    print(f"case conv rows B={B} D={D} L={L} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(L)
+    wide = torch.randn(B, 2 * D, L, generator=g, device="cuda")
+    w, bias, dy = (torch.randn(*s, generator=g, device="cuda") for s in ((D, K), (D,), (B, D, L)))
+    y = torch.empty(B, D, L, device="cuda")
+    _lib.check(lib.aussm_conv_rows_fwd(P(wide), P(w), P(bias), P(y), B, D, L, K, 2 * D * L, scan._stream()), "fwd")
+    leaves = [t.double().requires_grad_(True) for t in (wide[:, :D], w, bias)]
+    ref = torch.nn.functional.conv1d(leaves[0], leaves[1][:, None], leaves[2], padding=K - 1, groups=D)[:, :, :L]
+    ref.backward(dy.double())
+    torch.testing.assert_close(y.double(), ref.detach(), atol=1e-5, rtol=1e-5)
+    dx, dw, db = torch.zeros_like(wide), torch.zeros_like(w), torch.zeros_like(bias)
+    _lib.check(lib.aussm_conv_rows_bwd(P(dy), P(wide), P(w), P(dx), P(dw), P(db), B, D, L, K, 2 * D * L, 2 * D * L, scan._stream()), "bwd")
+    torch.testing.assert_close(dx[:, :D].double(), leaves[0].grad, atol=1e-5, rtol=1e-5)
+    assert dx[:, D:].abs().max() == 0
+    for a, r in ((dw, leaves[1].grad), (db, leaves[2].grad)):
+        scale = max(1.0, float(r.abs().max()))
+        torch.testing.assert_close(a.double() / scale, r / scale, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("rows,d", [(1, 1), (65, 3), (130, 64), (7, 65), (64, 200), (33, 513), (5, 1024)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_norm_and_its_gradient(rows, d, residual):
+    from aussm_amd import _lib, scan
+    lib, P = _lib.load(), _lib.ptr
+    print(f"case norm rows={rows} d={d} residual={residual}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(d)
+    x, w, dy, res = (torch.randn(*s, generator=g, device="cuda") for s in ((rows, d), (d,), (rows, d), (rows, d)))
+    y, rstd, dx, dw = torch.empty_like(x), torch.empty(rows, device="cuda"), torch.empty_like(x), torch.zeros_like(w)
+    _lib.check(lib.aussm_rms_norm_fwd(P(x), P(w), P(y), P(rstd), rows, d, 1e-5, scan._stream()), "fwd")
+    _lib.check(lib.aussm_rms_norm_bwd(P(dy), P(x), P(w), P(rstd), P(res) if residual else None, P(dx), P(dw), rows, d, scan._stream()), "bwd")
+    xd, wd = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    ref = xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1e-5) * wd
+    ref.backward(dy.double())
+    torch.testing.assert_close(y.double(), ref.detach(), atol=1e-5, rtol=1e-5)
+    torch.testing.assert_close(dx.double(), xd.grad + (res.double() if residual else 0), atol=1e-5, rtol=1e-5)
+    torch.testing.assert_close(dw.double(), wd.grad, atol=1e-4, rtol=1e-5)      # up to 130 terms of size <= 10
+
+
+@pytest.mark.parametrize("kind,d,n,b,l,kw", [("a", 8, 4, 2, 33, {}), ("a", 40, 16, 3, 70, {"bias": True}), ("a", 24, 20, 1, 130, {"d_conv": 3}),
+                                             ("m", 8, 4, 2, 33, {}), ("m", 40, 16, 3, 70, {"bias": True}), ("m", 33, 20, 2, 131, {"d_conv": 3})])
+@pytest.mark.parametrize("residual", [False, True])
+def test_native_block_matches_the_composed_layers(kind, d, n, b, l, kw, residual, monkeypatch):
+    """Output, input gradient and every parameter gradient: two fp32 evaluations of the same block, within 1e-4 of
+    each tensor's scale."""
+    from aussm_amd import blocks
+    torch.manual_seed(d + l)
+    args = (blocks.ModelArgsSSMau if kind == "a" else blocks.ModelArgsMamba)(d_model=d, d_state=n, **kw)
+    print(f"case native block {kind} d={d} n={n} b={b} l={l} {kw} residual={residual}", flush=True)
+    net = (blocks.ResidualBlock(args) if residual else args.block(args)).cuda()
+    with torch.no_grad():
+        for p in net.parameters():
+            p.add_(0.1 * torch.randn_like(p))
+    x, dy = torch.randn(b, l, d, device="cuda"), torch.randn(b, l, d, device="cuda")
+
+    def step():
+        xi = x.clone().requires_grad_(True)
+        net.zero_grad(set_to_none=True)
+        y = net(xi)
+        y.backward(dy)
+        return [y.detach(), xi.grad] + [p.grad for p in net.parameters()]
+    got = step()
+    assert net(x).grad_fn.name() == ("AussmBlockBackward" if kind == "a" else "AussmMambaBlockBackward")
+    mixer = net.mixer if residual else net
+    if kind == "a":
+        assert mixer.ssm_args["u"].shape == (b, d, l)
+    monkeypatch.setattr(blocks, "_native", lambda x: False)
+    for name, a, w in zip(["y", "x"] + [k for k, _ in net.named_parameters()], got, step()):
+        a, w = (torch.view_as_real(t) if t.is_complex() else t for t in (a, w))
+        scale = max(1e-3, float(w.abs().max()))
+        torch.testing.assert_close(a / scale, w / scale, atol=1e-4, rtol=1e-4, msg=lambda m, k=name: f"{k}: {m}")
