@@ -49,12 +49,23 @@ Tensor check_h0(const Tensor& h0, int64_t b, int64_t d, int64_t n) {
 // gradient of a (b, n, l[, 2]) float buffer in the type and shape of the tensor it belongs to
 Tensor as_like(const Tensor& g, bool complex, at::ScalarType dtype) {
   if (complex) return at::view_as_complex(g);
-  return dtype == at::kFloat ? g : g.to(dtype);
+  return g.scalar_type() == dtype ? g : g.to(dtype);
 }
 
 Tensor workspace(int variant, const Tensor& u, int b, int d, int n, int l, int ck, int dt) {
   const size_t f = aussm_scan_workspace_floats(variant, b, d, n, l, ck, dt);
   return f ? empty_f32({(int64_t)f}, u) : Tensor();
+}
+
+// gradient of a (b, d, l) input: in the input's type where the kernel writes that (flag AUSSM_GRADS_IN_DTYPE)
+Tensor empty_grad(const Tensor& u, int64_t b, int64_t d, int64_t l, bool in_dtype) {
+  return at::empty({b, d, l}, at::TensorOptions().dtype(in_dtype ? u.scalar_type() : at::kFloat).device(u.device()));
+}
+
+bool aligned16(std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t->defined() && (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15)) return false;
+  return true;
 }
 
 // ---- buffers that the backward kernels accumulate into: one allocation and one clearing launch
@@ -84,6 +95,7 @@ struct Acc {
 struct UnitaryNode : SavingNode {
   int b, d, n, l, ck, dt;
   bool bc_complex;
+  bool filled;                   // the forward call left what the backward kernel wants in `aux`
   std::string name() const override { return "AussmUnitaryScanBackward"; }
   variable_list apply(variable_list&& g) override;
 };
@@ -108,7 +120,8 @@ variable_list UnitaryNode::apply(variable_list&& g) {
     dy = dpre;
     out[U_Z] = dz;
   }
-  Tensor du = empty_f32({b, d, l}, u), ddelta = empty_f32({b, d, l}, u), dtheta = empty_f32({b, d, l}, u);
+  const bool g16 = dt == AUSSM_BF16 && u.size(0) == b;
+  Tensor du = empty_grad(u, b, d, l, g16), ddelta = empty_grad(u, b, d, l, g16), dtheta = empty_f32({b, d, l}, u);
   const bool want_dD = D.defined() && task_should_compute_output(U_D);
   const bool want_dh0 = task_should_compute_output(U_H0);
   Acc acc;
@@ -117,7 +130,8 @@ variable_list UnitaryNode::apply(variable_list&& g) {
   Tensor dB = acc.part(iB, {b, n, l, 2}), dC = acc.part(iC, {b, n, l, 2}), dD = want_dD ? acc.part(iD, {d}) : Tensor();
   Tensor dh0 = want_dh0 ? empty_f32({b, d, n, 2}, u) : Tensor();
   check(aussm_unitary_bwd_aux(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(hck), ptr(aux),
-                              ptr(du), ptr(ddelta), ptr(dtheta), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), b, d, n, l, ck, dt,
+                              ptr<float>(du), ptr<float>(ddelta), ptr(dtheta), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), b, d, n, l, ck,
+                              dt | (g16 ? AUSSM_GRADS_IN_DTYPE : 0) | (filled && aligned16({&dy}) ? AUSSM_AUX_FILLED : 0),
                               b / (int)u.size(0), cur_stream()),
         "aussm_unitary_bwd_aux");
   if (u.size(0) != b) {                          // u, delta shared by consecutive batch elements
@@ -193,6 +207,8 @@ std::pair<Tensor, Tensor> unitary_scan(const Tensor& u_, const Tensor& delta_, c
       node->save({u, delta, theta, B, C, D, z, hck, aux, ypre});
       node->b = b; node->d = d; node->n = n; node->l = l; node->ck = ck; node->dt = dt;
       node->bc_complex = Bc.is_complex();
+      node->filled = aux.defined() && aussm_unitary_kernel_mode(0, b, d, n, l, ck, dt, urep, 1) == 6 &&
+                     aussm_unitary_kernel_mode(1, b, d, n, l, ck, dt, urep, 1) == 6 && aligned16({&u, &delta, &theta, &B, &C});
     } else {
       // no backward pass: the buffer serves as workspace only (prepared operands of the matrix-core kernels, segment
       // states of a launch that is split along L) and no checkpoints are kept.  (The buffer of a shape that the
@@ -236,7 +252,8 @@ variable_list ComplexNode::apply(variable_list&& g) {
   const c10::DeviceGuard guard(u.device());
   const Tensor dy = g[0].defined() ? dense(g[0]) : at::zeros({b, d, l}, theta.options());
   const Tensor dhL = g.size() > 1 ? dense(g[1]) : Tensor();
-  Tensor du = empty_f32({b, d, l}, u), ddelta = empty_f32({b, d, l}, u), drho = empty_f32({b, d, l}, u),
+  const bool g16 = dt == AUSSM_BF16 && n <= 16;
+  Tensor du = empty_grad(u, b, d, l, g16), ddelta = empty_grad(u, b, d, l, g16), drho = empty_f32({b, d, l}, u),
          dtheta = empty_f32({b, d, l}, u), dz = z.defined() ? empty_f32({b, d, l}, u) : Tensor();
   const bool want_dD = D.defined() && task_should_compute_output(X_D);
   const bool want_dh0 = h0.defined() && task_should_compute_output(X_H0);
@@ -248,7 +265,7 @@ variable_list ComplexNode::apply(variable_list&& g) {
   const Tensor ws = workspace(VAR_COMPLEX, u, b, d, n, l, REC_CK, dt);
   check(aussm_complex_bwd(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(rho), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(h0), ptr(hck),
                           ptr(du), ptr(ddelta), ptr(drho), ptr(dtheta), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), ptr(z), ptr(dz), ptr(ws),
-                          b, d, n, l, REC_CK, dt, cur_stream()),
+                          b, d, n, l, REC_CK, dt | (g16 ? AUSSM_GRADS_IN_DTYPE : 0), cur_stream()),
         "aussm_complex_bwd");
   out[X_U] = as_like(du, false, u.scalar_type());
   out[X_DELTA] = as_like(ddelta, false, u.scalar_type());
@@ -331,20 +348,28 @@ variable_list RealNode::apply(variable_list&& g) {
   const c10::DeviceGuard guard(u.device());
   const Tensor dy = g[0].defined() ? dense(g[0]) : at::zeros({b, d, l}, A.options());
   const Tensor dhL = g.size() > 1 ? dense(g[1]) : Tensor();
-  Tensor du = empty_f32({b, d, l}, u), ddelta = empty_f32({b, d, l}, u), dz = z.defined() ? empty_f32({b, d, l}, u) : Tensor();
+  const bool g16 = dt == AUSSM_BF16 && n <= 16;
+  Tensor du = empty_grad(u, b, d, l, g16), ddelta = empty_grad(u, b, d, l, g16), dz = z.defined() ? empty_f32({b, d, l}, u) : Tensor();
   const bool want_dD = D.defined() && task_should_compute_output(R_D);
   const bool want_dh0 = h0.defined() && task_should_compute_output(R_H0);
   Acc acc;
-  const int iA = acc.add((int64_t)d * n), iB = acc.add((int64_t)b * n * l), iC = acc.add((int64_t)b * n * l), iD = want_dD ? acc.add(d) : 0;
+  const bool want_bias = bias.defined() && task_should_compute_output(R_BIAS);
+  const int iA = acc.add((int64_t)d * n), iB = acc.add((int64_t)b * n * l), iC = acc.add((int64_t)b * n * l), iD = want_dD ? acc.add(d) : 0,
+            iBias = want_bias ? acc.add(d) : 0;
   acc.make(u);
   Tensor dA = acc.part(iA, {d, n}), dB = acc.part(iB, {b, n, l}), dC = acc.part(iC, {b, n, l}), dD = want_dD ? acc.part(iD, {d}) : Tensor();
   Tensor dh0 = want_dh0 ? empty_f32({b, d, n}, u) : Tensor();
   const Tensor ws = workspace(VAR_REAL, u, b, d, n, l, REC_CK, dt);
-  check(aussm_real_bwd(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(A), ptr(B), ptr(C), ptr(D), ptr(bias), softplus, ptr(h0), ptr(hck),
-                       ptr(du), ptr(ddelta), ptr(dA), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), ptr(z), ptr(dz), ptr(ws), b, d, n, l, REC_CK, dt,
-                       cur_stream()),
-        "aussm_real_bwd");
-  if (bias.defined() && task_should_compute_output(R_BIAS)) out[R_BIAS] = ddelta.sum(at::IntArrayRef({0, 2}));
+  aussm_real_rows rows{};
+  if (want_bias) {
+    out[R_BIAS] = acc.part(iBias, {d});
+    rows.ddelta_bias = ptr(out[R_BIAS]);
+    rows.ddelta_bias_scale = 1.0f;
+  }
+  check(aussm_real_bwd_rows(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(A), ptr(B), ptr(C), ptr(D), ptr(bias), softplus, ptr(h0), ptr(hck),
+                            ptr(du), ptr(ddelta), ptr(dA), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), ptr(z), ptr(dz), ptr(ws), &rows, b, d, n, l,
+                            REC_CK, dt | (g16 ? AUSSM_GRADS_IN_DTYPE : 0), cur_stream()),
+        "aussm_real_bwd_rows");
   out[R_U] = as_like(du, false, u.scalar_type());
   out[R_DELTA] = as_like(ddelta, false, u.scalar_type());
   out[R_A] = dA;
