@@ -9,6 +9,9 @@ import ctypes
 import os
 from ctypes import c_char_p, c_int, c_void_p
 
+import torch
+from torch.autograd import forward_ad
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libaussm_hip.so")
 
@@ -135,6 +138,14 @@ def host():
         loader.exec_module(module)
         _host = module
     return _host
+
+
+def plain_call() -> bool:
+    """Nothing but reverse-mode autograd follows this call: no tracer, compiler, dispatch mode, forward-mode level or
+    function transform."""
+    return (torch._C._get_tracing_state() is None and forward_ad._current_level < 0
+            and not torch._C._are_functorch_transforms_active() and torch._C._len_torch_dispatch_stack() == 0
+            and not torch.compiler.is_compiling())
 
 
 def check(code: int, what: str) -> None:

@@ -112,9 +112,11 @@ def _plain(module: nn.Module, cls) -> bool:
 
 
 def _native(x: torch.Tensor) -> bool:
-    """Tensors the native route takes at all (it checks the rest itself)."""
+    """Calls the native route takes at all (it checks the rest itself): plain tensors, and nobody who follows the layers
+    one by one (tracer, compiler, dispatch modes, forward-mode and function transforms)."""
     m = torch.nn.modules.module
-    return (x.is_cuda and x.dtype is torch.float32 and not torch.is_autocast_enabled()
+    return (x.is_cuda and x.dtype is torch.float32 and type(x) in (torch.Tensor, nn.Parameter) and _lib.plain_call()
+            and not torch.is_autocast_enabled()
             and not (m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
                      or m._global_backward_pre_hooks))
 

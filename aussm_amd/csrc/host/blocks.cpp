@@ -218,7 +218,7 @@ OptTensor aussm_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
                       const Tensor& B, const Tensor& C, const Tensor& D, const Tensor& W_out, const OptTensor& b_out, double scale) {
   const Tensor raw[A_INPUTS] = {x_, opt(nw_), W_in, opt(b_in), cw, opt(cb), W_xp, W_dt, b_dt, xA_w, xA_b, B, C, D, W_out, opt(b_out)};
   BlockDims s{};
-  if (!front_ok(x_, raw[A_NW], nw_.has_value(), W_in, raw[A_BIN], cw, raw[A_CB], W_out, raw[A_BOUT], s)) return std::nullopt;
+  if (!front_ok(x_, raw[A_NW], nw_.has_value(), W_in, raw[A_BIN], cw, raw[A_CB], W_out, raw[A_BOUT], s) || !same_device(x_, raw)) return std::nullopt;
   s.residual = residual; s.eps = (float)eps;
   const int64_t n = B.numel(), r = W_xp.size(0), e = s.e;
   for (int i : {A_WXP, A_WDT, A_BDT, A_XAW, A_XAB, A_D})
@@ -334,7 +334,7 @@ OptTensor mamba_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
                       const Tensor& W_out, const OptTensor& b_out) {
   const Tensor raw[M_INPUTS] = {x_, opt(nw_), W_in, opt(b_in), cw, opt(cb), W_xp, W_dt, b_dt, A_log, D, W_out, opt(b_out)};
   BlockDims s{};
-  if (!front_ok(x_, raw[M_NW], nw_.has_value(), W_in, raw[M_BIN], cw, raw[M_CB], W_out, raw[M_BOUT], s)) return std::nullopt;
+  if (!front_ok(x_, raw[M_NW], nw_.has_value(), W_in, raw[M_BIN], cw, raw[M_CB], W_out, raw[M_BOUT], s) || !same_device(x_, raw)) return std::nullopt;
   s.residual = residual; s.eps = (float)eps;
   for (int i : {M_WXP, M_WDT, M_BDT, M_ALOG, M_D})
     if (!f32_cuda(raw[i])) return std::nullopt;
@@ -439,7 +439,9 @@ variable_list LinearNode::apply(variable_list&& g) {
 
 OptTensor norm_linear(const Tensor& x_, const OptTensor& nw_, double eps, const Tensor& W_, const OptTensor& b_) {
   const Tensor nwv = opt(nw_), bv = opt(b_);
-  if (!f32_cuda(x_) || !f32_cuda(W_) || !f32_or_none(nwv) || !f32_or_none(bv) || x_.dim() < 2 || x_.numel() == 0) return std::nullopt;
+  if (!f32_cuda(x_) || !f32_cuda(W_) || !f32_or_none(nwv) || !f32_or_none(bv) || x_.dim() < 2 || x_.numel() == 0 ||
+      !same_device(x_, {W_, nwv, bv}))
+    return std::nullopt;
   const int64_t i = x_.size(-1), rows = x_.numel() / i, o = W_.size(0);
   if (W_.dim() != 2 || W_.size(1) != i || rows >= (1ll << 30) || i >= (1 << 24) || o >= (1 << 24)) return std::nullopt;
   if (nw_.has_value() && (nwv.numel() != i || i > 1024)) return std::nullopt;

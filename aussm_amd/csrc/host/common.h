@@ -90,6 +90,17 @@ inline Tensor f32(const Tensor& t, const char* name, at::IntArrayRef shape) {
   return dense(t);
 }
 
+// every tensor of a call lies on one device (a kernel must not be handed an address of another)
+inline bool same_device(const Tensor& ref, at::ArrayRef<Tensor> ts) {
+  for (const Tensor& t : ts)
+    if (t.defined() && t.device() != ref.device()) return false;
+  return true;
+}
+inline void check_devices(const Tensor& ref, at::ArrayRef<Tensor> ts) {
+  for (const Tensor& t : ts)
+    if (t.defined() && t.device() != ref.device()) fail("expected all tensors of the call on ", ref.device(), ", got one on ", t.device());
+}
+
 // A graph node over saved tensors: `saved` are released together, and unpacking them after that raises torch's
 // usual error about a second backward pass.
 struct SavingNode : Node {

@@ -44,7 +44,7 @@ PYBIND11_MODULE(_aussm_host, m) {
     return result(complex_scan(u, delta, rho, theta, Bc, Cc, D, z, h0, want_state), want_state);
   });
   m.def("selective_scan", [](const Tensor& u, const Tensor& delta, const Tensor& A, const Tensor& B, const Tensor& C, const OptTensor& D,
-                             const OptTensor& z, const OptTensor& bias, bool softplus, bool want_state, const OptTensor& h0) {
+                             const OptTensor& z, const OptTensor& bias, const OptTensor& h0, bool softplus, bool want_state) {
     return result(selective_scan(u, delta, A, B, C, D, z, bias, softplus, want_state, h0), want_state);
   });
   m.def("operator_supported", &operator_supported);

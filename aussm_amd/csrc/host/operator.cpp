@@ -73,6 +73,7 @@ Tensor adaptive_operator(const Tensor& u_, const Tensor& dt_, const Tensor& x_, 
   want(C_, "C", at::kComplexFloat, {n});
   want(D_, "D", at::kFloat, {d});
   want(z_, "z", at::kFloat, {b, d, l});
+  check_devices(u_, {dt_, x_, xb_, B_, C_, D_, z_});
   const c10::DeviceGuard guard(u_.device());
   const bool needs_grad = at::GradMode::is_enabled() && (wants_grad(u_) || wants_grad(dt_) || wants_grad(x_) || wants_grad(xb_) ||
                                                          wants_grad(B_) || wants_grad(C_) || wants_grad(D_) || wants_grad(z_));

@@ -166,6 +166,7 @@ std::pair<Tensor, Tensor> unitary_scan(const Tensor& u_, const Tensor& delta_, c
   check_bdl(u_, delta_);
   const c10::DeviceGuard guard(u_.device());
   const Tensor Dv = opt(D_), zv = opt(z_), hv = opt(h0_);
+  check_devices(u_, {delta_, theta_, Bc, Cc, Dv, zv, hv});
   const bool needs_grad = at::GradMode::is_enabled() && (wants_grad(u_) || wants_grad(delta_) || wants_grad(theta_) || wants_grad(Bc) ||
                                                          wants_grad(Cc) || wants_grad(Dv) || wants_grad(zv) || wants_grad(hv));
   Tensor y, hL;
@@ -286,6 +287,7 @@ std::pair<Tensor, Tensor> complex_scan(const Tensor& u_, const Tensor& delta_, c
   check_bdl(u_, delta_);
   const c10::DeviceGuard guard(u_.device());
   const Tensor Dv = opt(D_), zv = opt(z_), hv = opt(h0_);
+  check_devices(u_, {delta_, rho_, theta_, Bc, Cc, Dv, zv, hv});
   const bool needs_grad = at::GradMode::is_enabled() &&
                           (wants_grad(u_) || wants_grad(delta_) || wants_grad(rho_) || wants_grad(theta_) || wants_grad(Bc) ||
                            wants_grad(Cc) || wants_grad(Dv) || wants_grad(zv) || wants_grad(hv));
@@ -389,6 +391,7 @@ std::pair<Tensor, Tensor> selective_scan(const Tensor& u_, const Tensor& delta_,
   check_bdl(u_, delta_);
   const c10::DeviceGuard guard(u_.device());
   const Tensor Dv = opt(D_), zv = opt(z_), bv = opt(bias_), hv = opt(h0_);
+  check_devices(u_, {delta_, A_, B_, C_, Dv, zv, bv, hv});
   const bool needs_grad = at::GradMode::is_enabled() &&
                           (wants_grad(u_) || wants_grad(delta_) || wants_grad(A_) || wants_grad(B_) || wants_grad(C_) ||
                            wants_grad(Dv) || wants_grad(zv) || wants_grad(bv) || wants_grad(hv));

@@ -259,7 +259,7 @@ def ssm_adaptive_interface(u: Tensor, dt: Tensor, x: Tensor, x_bias: Tensor, B: 
     b, d, l = u.shape
     n = x.shape[1]
     if (l <= max_parallel_length and not save_intermediates and u.is_cuda and B.dtype is torch.complex64
-            and C.dtype is torch.complex64 and not torch.compiler.is_compiling() and type(u) is Tensor):
+            and C.dtype is torch.complex64 and L.plain_call() and type(u) in (Tensor, torch.nn.Parameter)):
         # one launch sequence: the operator as one graph node, its softplus and zero start state inside the kernels
         host = L.host()
         if host.operator_supported(b, d, n, l):

@@ -26,6 +26,7 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._lib import check, ptr
@@ -141,6 +142,36 @@ def unitary_bwd_raw(dy, dhL, u, delta, theta, Bri, Cri, D, hck, ck, want_dD=True
     return du, ddelta, dtheta, dB, dC, dD, dh0
 
 
+class _ScanFn(torch.autograd.Function):
+    """A scan as an autograd function of Python, for the callers that need one: the tracer records it as an operator of
+    its own, and forward-mode differentiation refuses it.  Its backward pass runs the scan again."""
+
+    @staticmethod
+    def forward(ctx, call, args, *tensors):
+        ctx.call, ctx.args = call, args
+        ctx.save_for_backward(*tensors)
+        with torch.no_grad():
+            return call(*tensors, *args)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        with torch.enable_grad():
+            leaves = [None if t is None else t.detach().requires_grad_(need)
+                      for t, need in zip(ctx.saved_tensors, ctx.needs_input_grad[2:])]
+            out = ctx.call(*leaves, *ctx.args)
+            wanted = [t for t in leaves if t is not None and t.requires_grad]
+            got = iter(torch.autograd.grad(out, wanted, grads, allow_unused=True))
+        return (None, None, *(next(got) if t is not None and t.requires_grad else None for t in leaves))
+
+
+def _call(fn, tensors, *args):
+    """`fn(*tensors, *args)` of the native host path.  Its graph nodes are invisible to the tracer and know no tangents,
+    so a call under either goes through `_ScanFn`."""
+    if torch._C._get_tracing_state() is None and forward_ad._current_level < 0:
+        return fn(*tensors, *args)
+    return _ScanFn.apply(fn, args, *tensors)
+
+
 def unitary_scan(u: Tensor, delta: Tensor, theta: Tensor, Bc: Tensor, Cc: Tensor, D: Optional[Tensor] = None,
                  z: Optional[Tensor] = None, h0: Optional[Tensor] = None, return_last_state: bool = False):
     """Adaptive-unitary scan.  u, delta, theta, z: (b, d, l); Bc, Cc: (b, n, l) complex64 (or
@@ -148,7 +179,7 @@ def unitary_scan(u: Tensor, delta: Tensor, theta: Tensor, Bc: Tensor, Cc: Tensor
     state (b, d, n) complex64 if return_last_state.  u and delta may be (b / r, d, l): batch element i
     of theirs then serves the r consecutive batch elements i r .. i r + r - 1 of everything else
     (one input, r phase sequences)."""
-    return _lib.host().unitary_scan(u, delta, theta, Bc, Cc, D, z, h0, return_last_state)
+    return _call(_lib.host().unitary_scan, (u, delta, theta, Bc, Cc, D, z, h0), return_last_state)
 
 
 # --------------------------------------------------------------------------------------------
@@ -205,7 +236,7 @@ def complex_scan(u: Tensor, delta: Tensor, rho: Tensor, theta: Tensor, Bc: Tenso
                  D: Optional[Tensor] = None, z: Optional[Tensor] = None, h0: Optional[Tensor] = None,
                  return_last_state: bool = False):
     """Complex scan, a_l = exp(rho_l + i theta_l).  Shapes as unitary_scan plus rho (b, d, l)."""
-    return _lib.host().complex_scan(u, delta, rho, theta, Bc, Cc, D, z, h0, return_last_state)
+    return _call(_lib.host().complex_scan, (u, delta, rho, theta, Bc, Cc, D, z, h0), return_last_state)
 
 
 # --------------------------------------------------------------------------------------------
@@ -261,4 +292,4 @@ def selective_scan_fn(u: Tensor, delta: Tensor, A: Tensor, B: Tensor, C: Tensor,
 
     Returns y (b, d, l) float32, plus the last state (b, d, n) if return_last_state.
     `h0` (b, d, n), a start state, is an extension over the reference's signature."""
-    return _lib.host().selective_scan(u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus), return_last_state, h0)
+    return _call(_lib.host().selective_scan, (u, delta, A, B, C, D, z, delta_bias, h0), bool(delta_softplus), return_last_state)
