@@ -2,8 +2,8 @@
 // the phase adjoints of the fused operator.
 //
 // Both operands are fp32 in memory and split EXACTLY into three bf16 pieces while they are staged into LDS (scan_fwd_xdl.h:
-// split8, xmm<3>): what a product drops is below 2^-26 of it, the sums are fp32.  Workgroup tile 128 x (64 TNH), four
-// wavefronts of 64 x (32 TNH), 32 of k per step; the values of the next step are requested before the products of
+// split8, xmm<3>): what a product drops is below 2^-26 of it, the sums are fp32.  Workgroup tile 128 x (32 EN), four
+// wavefronts of 64 x (16 EN), 32 of k per step; the values of the next step are requested before the products of
 // the current one, and two workgroups per compute unit cover each other's barriers.
 //
 // Operands may be contiguous along k or along their other index (AK1 / BK1), so no transposed copy is ever made:
@@ -14,6 +14,8 @@
 #pragma once
 #include "gemm_args.h"
 #include "scan_fwd_xdl.h"
+
+#include <type_traits>
 
 namespace aussm {
 
@@ -28,23 +30,41 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// One thread's share of an operand tile of 64 H rows x 32 k: H records of 8 k each.
-//   K1:  row tid / 4 (+ 64), k group tid % 4
-//   else rows H lane .. H lane + H - 1 (one load for two rows), k group = wavefront: the k index, its bound and the
-//        stride along k are scalars, and a load instruction is a scalar base plus the row's offset
+// split8<3> with the residuals taken by an unpack and a subtract instead of the dot instruction: the same pieces.  Beside
+// a busy matrix pipe the dot instruction costs more than the two (256 x 23040, K = 4096 382 us with it, 331 us without).
+__device__ __forceinline__ void split8_sub(const float (&x)[8], u4 (&out)[3]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    float a = x[2 * q], b = x[2 * q + 1];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const uint32_t pk = pk_bf16(a, b);
+      out[p][q] = pk;
+      if (p < 2) {
+        a -= __uint_as_float(pk << 16);
+        b -= __uint_as_float(pk & 0xffff0000u);
+      }
+    }
+  }
+}
+
+// One thread's share of an operand tile of H NT / 4 rows x 32 k (NT threads): H records of 8 k each.
+//   K1:  row tid / 4 (+ NT / 4), k group tid % 4
+//   else rows H lane .. H lane + H - 1 (one load for two rows) of the wavefront's 64 H rows, k group = wavefront % 4: the
+//        k index, its bound and the stride along k are scalars, and a load instruction is a scalar base plus the row's offset
 // Loads are unconditional (no branch may hide from the compiler how many are in flight): in the last, partial step
 // along k they repeat valid elements, and stage() clears what lies past K.  QUAD: K is a multiple of four.
-template <bool K1, bool QUAD, int H>
+template <bool K1, bool QUAD, int H, int NT>
 struct XgOperand {
   const float* row[H];       // K1: this thread's rows; else row[0]: its first row (the second one is next to it)
   long sk;
   int r0, kq;
   struct Vals { float v[H][8]; };
   __device__ __forceinline__ void place(int tid) {
-    r0 = K1 ? tid >> 2 : H * (tid & 63);
-    kq = 8 * (K1 ? tid & 3 : wave_index());
+    r0 = K1 ? tid >> 2 : H * (tid & 63) + 64 * H * (wave_index() >> 2);
+    kq = 8 * (K1 ? tid & 3 : wave_index() & 3);
   }
-  __device__ __forceinline__ int local_row(int h) const { return K1 ? r0 + 64 * h : r0 + h; }
+  __device__ __forceinline__ int local_row(int h) const { return K1 ? r0 + (NT / 4) * h : r0 + h; }
   __device__ __forceinline__ int slot(int h) const {
     const int r = local_row(h);
     return (r >> 4) * (3 * 64) + xg_slot(r & 15, kq >> 3);
@@ -78,7 +98,7 @@ struct XgOperand {
       }
     }
   }
-  __device__ __forceinline__ void stage(const SplitK& sk_, Vals& x, int k0, int K, u4* __restrict__ lds) const {
+  __device__ __forceinline__ void stage(Vals& x, int k0, int K, u4* __restrict__ lds) const {
     if (k0 + 32 > K) {                                  // uniform
 #pragma unroll
       for (int c = 0; c < 8; ++c)
@@ -88,7 +108,7 @@ struct XgOperand {
 #pragma unroll
     for (int h = 0; h < H; ++h) {
       u4 pc[3];
-      split8<3>(sk_, x.v[h], pc);
+      split8_sub(x.v[h], pc);
 #pragma unroll
       for (int c = 0; c < 3; ++c) lds[slot(h) + c * 64] = pc[c];
     }
@@ -100,24 +120,31 @@ struct XgOperand {
 // borders, atomics).  Unrolled stores straight from the registers, each with its own bounds and offset, made the
 // code several times the size of the main loop and covered 64 bytes at a time: 32 x 720 columns, 256 rows, K = 16
 // 19.5 us, now 13 us.
-template <bool AK1, bool BK1, bool TR, int TNH, bool QUAD>
-__global__ __launch_bounds__(256, 2) void xgemm_kernel(const XGemmArgs p) {
-  constexpr int NP = 3, TN = 64 * TNH, EN = 2 * TNH;        // EN: 16-wide column tiles per wavefront
+//
+// WIDE: eight wavefronts on a tile of 256 x (32 EN), both operand tiles twice in LDS, the values two steps ahead.  While the
+// wavefronts multiply step s they also split the values of step s + 1 into the other pair of tiles: one barrier a step, and
+// a value is split for twice as many products as in the narrow tile.  The first four wavefronts split before they
+// multiply, the others after it.  256 x 23040, K = 1024: 94 us narrow, 80 us wide (96 columns: see run_xgemm); of these,
+// the matrix instructions alone take 55 us and everything but them 58 us: the two overlap by half.
+template <bool AK1, bool BK1, bool TR, int EN, bool QUAD, bool WIDE>
+__global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 1 : 2) void xgemm_kernel(const XGemmArgs p) {
+  static_assert(WIDE ? EN == 3 || EN == 4 : EN == 2 || EN == 4, "column tiles");
+  constexpr int NT = WIDE ? 512 : 256, TM = WIDE ? XG_TM_WIDE : XG_TM;
+  constexpr int HB = WIDE ? 1 : EN / 2;                     // records of B per thread
+  constexpr int NP = 3, TN = 32 * EN;                       // EN: 16-wide column tiles per wavefront
   constexpr int WN = 16 * EN;                               // columns of a wavefront's block
   constexpr int LD = (TR ? 64 : WN) + 4;                    // row stride of its slice in LDS: 64 rows x WN columns, or transposed
   constexpr int SLICE = (TR ? WN : 64) * LD;
-  constexpr int TILES = (8 + 4 * TNH) * NP * 64;            // records of both operand tiles
-  constexpr int LDS16 = TILES > SLICE ? TILES : SLICE;      // (four slices of SLICE floats = SLICE 16-byte records)
+  constexpr int ATILE = (TM / 16) * NP * 64, TILES = ATILE + HB * (NT / 64) * NP * 64;   // records of both operand tiles
+  constexpr int SLICES = (NT / 256) * SLICE;                // (four slices of SLICE floats = SLICE 16-byte records)
+  constexpr int LDS16 = (WIDE ? 2 : 1) * TILES > SLICES ? (WIDE ? 2 : 1) * TILES : SLICES;
   __shared__ u4 s_mem[LDS16];
-  u4* const s_a = s_mem;
-  u4* const s_b = s_mem + 8 * NP * 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   // consecutive logical workgroups share their columns (B is the large operand) and an XCD
-  const int tm = (p.M + XG_TM - 1) / XG_TM, tn = (p.N + TN - 1) / TN;
+  const int tm = (p.M + TM - 1) / TM, tn = (p.N + TN - 1) / TN;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
-  const int m0 = (wg % tm) * XG_TM, n0 = (wg / tm % tn) * TN, sl = wg / (tm * tn);
+  const int m0 = (wg % tm) * TM, n0 = (wg / tm % tn) * TN, sl = wg / (tm * tn);
   const int wm = (wave >> 1) * 4, wn = (wave & 1) * EN;     // this wavefront's first 16-wide tiles
-  const SplitK sk = make_splitk();
   f4 acc[4][EN];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
@@ -127,41 +154,43 @@ __global__ __launch_bounds__(256, 2) void xgemm_kernel(const XGemmArgs p) {
   const int nb0 = n0 / p.nper, np0 = n0 - nb0 * p.nper;
   const bool one = np0 + TN <= p.nper || p.nper >= p.N;
   // rows past M / N are fetched from the last valid one (they only reach results that are not stored)
-  XgOperand<AK1, QUAD, 2> oa;
-  XgOperand<BK1, QUAD, TNH> ob;
+  XgOperand<AK1, QUAD, 2, NT> oa;
+  XgOperand<BK1, QUAD, HB, NT> ob;
   oa.place(tid); ob.place(tid);
   oa.sk = p.sak; ob.sk = p.sbk;
 #pragma unroll
   for (int h = 0; h < 2; ++h) oa.row[h] = p.A + (long)min(m0 + oa.local_row(h), p.M - 1) * p.sam;
 #pragma unroll
-  for (int h = 0; h < TNH; ++h) {
-    const int dn = min(ob.local_row(h), p.N - 1 - n0) + np0, nb = one ? 0 : dn / p.nper;
+  for (int h = 0; h < HB; ++h) {
+    const int dn = min(min(ob.local_row(h), TN - 1), p.N - 1 - n0) + np0, nb = one ? 0 : dn / p.nper;
     ob.row[h] = p.B + ((long)(nb0 + nb) * p.sbb + (long)(dn - nb * p.nper) * p.sbn);
   }
   // two neighbouring rows in one load: every pair of the tile exists and lies in one batch (uniform)
-  const bool pa = m0 + XG_TM <= p.M, pb = one && n0 + TN <= p.N;
+  const bool pa = m0 + TM <= p.M, pb = one && n0 + TN <= p.N;
   const int nk = (p.K + 31) / 32, steps = nk * p.Z, per = (steps + p.slices - 1) / p.slices;
   const int s0 = sl * per, s1 = s0 + per < steps ? s0 + per : steps;
   int fz = s0 / nk, fit = s0 - fz * nk;                     // (z, k step) of the next fetch
-  typename XgOperand<AK1, QUAD, 2>::Vals va;
-  typename XgOperand<BK1, QUAD, TNH>::Vals vb;
+  typename XgOperand<AK1, QUAD, 2, NT>::Vals va[2];
+  typename XgOperand<BK1, QUAD, HB, NT>::Vals vb[2];
+  int sfit = fit;
   const int rslot = xg_slot(lane & 15, lane >> 4);          // the record of (row lane % 16, g lane / 16)
-  if (s0 < s1) {
-    oa.fetch(va, (long)fz * p.saz, fit * 32, p.K, pa);
-    ob.fetch(vb, (long)fz * p.sbz, fit * 32, p.K, pb);
-  }
-#pragma unroll 1
-  for (int s = s0; s < s1; ++s) {
-    const int k0 = fit * 32;
-    if (s > s0) __syncthreads();
-    oa.stage(sk, va, k0, p.K, s_a);
-    ob.stage(sk, vb, k0, p.K, s_b);
-    __syncthreads();
+  auto fetch = [&](auto st) {
+    constexpr int S = decltype(st)::value;
+    oa.fetch(va[S], (long)fz * p.saz, fit * 32, p.K, pa);
+    ob.fetch(vb[S], (long)fz * p.sbz, fit * 32, p.K, pb);
     if (++fit == nk) { fit = 0; ++fz; }
-    if (s + 1 < s1) {                                       // in flight during the products
-      oa.fetch(va, (long)fz * p.saz, fit * 32, p.K, pa);
-      ob.fetch(vb, (long)fz * p.sbz, fit * 32, p.K, pb);
-    }
+  };
+  auto stage = [&](auto st, int buf) {
+    constexpr int S = decltype(st)::value;
+    oa.stage(va[S], sfit * 32, p.K, s_mem + buf * TILES);
+    ob.stage(vb[S], sfit * 32, p.K, s_mem + buf * TILES + ATILE);
+    if (++sfit == nk) sfit = 0;
+  };
+  typedef std::integral_constant<int, 0> I0;
+  typedef std::integral_constant<int, 1> I1;
+  auto multiply = [&](int buf) {
+    const u4* const s_a = s_mem + buf * TILES;
+    const u4* const s_b = s_a + ATILE;
     u4 rB[EN][NP];
 #pragma unroll
     for (int f = 0; f < EN; ++f)
@@ -175,9 +204,49 @@ __global__ __launch_bounds__(256, 2) void xgemm_kernel(const XGemmArgs p) {
 #pragma unroll
       for (int f = 0; f < EN; ++f) acc[e][f] = xmm<NP>(rA, rB[f], acc[e][f]);
     }
+  };
+  if (s0 < s1) fetch(I0{});
+  if constexpr (WIDE) {
+    if (s0 + 1 < s1) fetch(I1{});
+    if (s0 < s1) stage(I0{}, 0);
+    if (s0 + 2 < s1) fetch(I0{});
+    __syncthreads();
+    auto run = [&](auto first_tag) {
+      constexpr bool FIRST = decltype(first_tag)::value;
+      auto step = [&](int s, auto q) {
+        constexpr int Q = decltype(q)::value;
+        typedef std::integral_constant<int, Q ^ 1> O;
+        auto next = [&]() {
+          if (s + 1 < s1) {
+            stage(O{}, Q ^ 1);
+            if (s + 3 < s1) fetch(O{});
+          }
+        };
+        if constexpr (FIRST) next();
+        multiply(Q);
+        if constexpr (!FIRST) next();
+        __syncthreads();
+      };
+#pragma unroll 1
+      for (int s = s0; s < s1; s += 2) {
+        step(s, I0{});
+        if (s + 1 < s1) step(s + 1, I1{});
+      }
+    };
+    if (wave < 4) run(std::true_type{});
+    else run(std::false_type{});
+  } else {
+#pragma unroll 1
+    for (int s = s0; s < s1; ++s) {
+      if (s > s0) __syncthreads();
+      stage(I0{}, 0);
+      __syncthreads();
+      if (s + 1 < s1) fetch(I0{});
+      multiply(0);
+    }
+    __syncthreads();
   }
   // result tile (e, f), register a: row 16 e + 4 (lane / 16) + a, column 16 f + lane % 16 of the wavefront's block
-  __syncthreads();                                          // (the operand tiles are read no more)
   float* const sw = reinterpret_cast<float*>(s_mem) + wave * SLICE;
   const int c = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -197,7 +266,7 @@ __global__ __launch_bounds__(256, 2) void xgemm_kernel(const XGemmArgs p) {
   if (p.slices > 1) {                                       // uniform: summed into C (TR: one batch, nper = N)
     constexpr int RA = 64 / COLS;                           // lane = column (two rows at a time where 32 fill the row)
     const int q = lane % COLS;
-    const bool cok = TR ? mw + q < p.M : nw + q < p.N;
+    const bool cok = lane < RA * COLS && (TR ? mw + q < p.M : nw + q < p.N);
     const int dq = nw + q - n0 + np0, bq = (TR || one) ? 0 : dq / p.nper;
     float* const dst = p.C + (TR ? (long)(mw + q) * p.scm : (long)(nb0 + bq) * p.scb + (long)(dq - bq * p.nper) * p.scn);
 #pragma unroll 4
@@ -210,7 +279,7 @@ __global__ __launch_bounds__(256, 2) void xgemm_kernel(const XGemmArgs p) {
   constexpr int PR = COLS / 4, RR = 64 / PR;                // lanes per row, rows per iteration
   const int q = 4 * (lane % PR);
   // the other index's bounds and strides; four elements that exist, in one batch and aligned, leave as 16 bytes
-  const int cnt = min(4, TR ? p.M - (mw + q) : p.N - (nw + q));
+  const int cnt = lane < RR * PR ? min(4, TR ? p.M - (mw + q) : p.N - (nw + q)) : 0;
   const int dnq = nw + q - n0 + np0, nbq = (TR || one) ? 0 : dnq / p.nper, npq = dnq - nbq * p.nper;
   const bool ptr16 = ((reinterpret_cast<uintptr_t>(p.C) | (add ? reinterpret_cast<uintptr_t>(add) : 0)) & 15) == 0;
   const bool quad = cnt == 4 && (TR || one || npq + 4 <= p.nper);

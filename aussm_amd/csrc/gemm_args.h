@@ -25,5 +25,6 @@ struct XGemmArgs {
 };
 
 constexpr int XG_TM = 128;      // rows of a workgroup tile
+constexpr int XG_TM_WIDE = 256; // ... of the tile of eight wavefronts
 
 }  // namespace aussm

@@ -59,6 +59,13 @@ def test_products_of_a_linear_layer(b, l, i, o):
     assert _rel(dW, want) < 2e-6
 
 
+# ... and shapes large enough for the tiles of eight wavefronts, none a multiple of a tile: 96 columns (both operand orders,
+# results along either index), 128 columns, and slices of a long sum
+@pytest.mark.parametrize("b,l,i,o", [(23, 721, 200, 130), (31, 1027, 256, 200), (64, 2048, 70, 300)])
+def test_products_on_wide_tiles(b, l, i, o):
+    test_products_of_a_linear_layer(b, l, i, o)
+
+
 @pytest.mark.parametrize("B,D,L,K", [(1, 1, 1, 4), (2, 5, 3, 4), (3, 70, 130, 4), (2, 9, 2050, 4), (2, 8, 33, 3), (1, 4, 7, 8)])
 def test_convolution_of_channel_rows(B, D, L, K):
     from aussm_amd import _lib, scan
