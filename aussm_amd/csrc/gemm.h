@@ -126,16 +126,18 @@ struct XgOperand {
 // a value is split for twice as many products as in the narrow tile.  The first four wavefronts split before they
 // multiply, the others after it.  256 x 23040, K = 1024: 94 us narrow, 80 us wide (96 columns: see run_xgemm); of these,
 // the matrix instructions alone take 55 us and everything but them 58 us: the two overlap by half.
-template <bool AK1, bool BK1, bool TR, int EN, bool QUAD, bool WIDE>
+template <bool AK1, bool BK1, bool TR, int WM, int EM, int EN, bool QUAD, bool WIDE>
 __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 1 : 2) void xgemm_kernel(const XGemmArgs p) {
-  static_assert(WIDE ? EN == 3 || EN == 4 : EN == 2 || EN == 4, "column tiles");
-  constexpr int NT = WIDE ? 512 : 256, TM = WIDE ? XG_TM_WIDE : XG_TM;
-  constexpr int HB = WIDE ? 1 : EN / 2;                     // records of B per thread
-  constexpr int NP = 3, TN = 32 * EN;                       // EN: 16-wide column tiles per wavefront
+  constexpr int NT = WIDE ? 512 : 256, NWN = NT / 64 / WM;  // wavefronts: WM along the rows, NWN along the columns
+  constexpr int TM = 16 * EM * WM, TN = 16 * EN * NWN;      // EM, EN: 16-wide row and column tiles per wavefront
+  constexpr int HA = TM > NT / 4 ? 2 : 1, HB = TN > NT / 4 ? 2 : 1;    // records of A and B per thread
+  static_assert(TM <= HA * NT / 4 && TN <= HB * NT / 4, "a thread stages at most two records of an operand");
+  constexpr int NP = 3;
   constexpr int WN = 16 * EN;                               // columns of a wavefront's block
-  constexpr int LD = (TR ? 64 : WN) + 4;                    // row stride of its slice in LDS: 64 rows x WN columns, or transposed
-  constexpr int SLICE = (TR ? WN : 64) * LD;
-  constexpr int ATILE = (TM / 16) * NP * 64, TILES = ATILE + HB * (NT / 64) * NP * 64;   // records of both operand tiles
+  constexpr int WR = 16 * EM;                               // ... and rows
+  constexpr int LD = (TR ? WR : WN) + 4;                    // row stride of its slice in LDS: WR rows x WN columns, or transposed
+  constexpr int SLICE = (TR ? WN : WR) * LD;
+  constexpr int ATILE = HA * (NT / 64) * NP * 64, TILES = ATILE + HB * (NT / 64) * NP * 64;   // records of both operand tiles
   constexpr int SLICES = (NT / 256) * SLICE;                // (four slices of SLICE floats = SLICE 16-byte records)
   constexpr int LDS16 = (WIDE ? 2 : 1) * TILES > SLICES ? (WIDE ? 2 : 1) * TILES : SLICES;
   __shared__ u4 s_mem[LDS16];
@@ -144,33 +146,33 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 1 : 2) void xgemm_kernel(c
   const int tm = (p.M + TM - 1) / TM, tn = (p.N + TN - 1) / TN;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
   const int m0 = (wg % tm) * TM, n0 = (wg / tm % tn) * TN, sl = wg / (tm * tn);
-  const int wm = (wave >> 1) * 4, wn = (wave & 1) * EN;     // this wavefront's first 16-wide tiles
-  f4 acc[4][EN];
+  const int wm = (wave / NWN) * EM, wn = (wave % NWN) * EN;     // this wavefront's first 16-wide tiles
+  f4 acc[EM][EN];
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
+  for (int e = 0; e < EM; ++e)
 #pragma unroll
     for (int f = 0; f < EN; ++f) acc[e][f] = f4{0, 0, 0, 0};
   // batch and position of the tile's first column; most tiles lie in one batch (no division per column)
   const int nb0 = n0 / p.nper, np0 = n0 - nb0 * p.nper;
   const bool one = np0 + TN <= p.nper || p.nper >= p.N;
   // rows past M / N are fetched from the last valid one (they only reach results that are not stored)
-  XgOperand<AK1, QUAD, 2, NT> oa;
+  XgOperand<AK1, QUAD, HA, NT> oa;
   XgOperand<BK1, QUAD, HB, NT> ob;
   oa.place(tid); ob.place(tid);
   oa.sk = p.sak; ob.sk = p.sbk;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) oa.row[h] = p.A + (long)min(m0 + oa.local_row(h), p.M - 1) * p.sam;
+  for (int h = 0; h < HA; ++h) oa.row[h] = p.A + (long)min(m0 + oa.local_row(h), p.M - 1) * p.sam;
 #pragma unroll
   for (int h = 0; h < HB; ++h) {
     const int dn = min(min(ob.local_row(h), TN - 1), p.N - 1 - n0) + np0, nb = one ? 0 : dn / p.nper;
     ob.row[h] = p.B + ((long)(nb0 + nb) * p.sbb + (long)(dn - nb * p.nper) * p.sbn);
   }
   // two neighbouring rows in one load: every pair of the tile exists and lies in one batch (uniform)
-  const bool pa = m0 + TM <= p.M, pb = one && n0 + TN <= p.N;
+  const bool pa = m0 + HA * NT / 4 <= p.M, pb = one && n0 + TN <= p.N;
   const int nk = (p.K + 31) / 32, steps = nk * p.Z, per = (steps + p.slices - 1) / p.slices;
   const int s0 = sl * per, s1 = s0 + per < steps ? s0 + per : steps;
   int fz = s0 / nk, fit = s0 - fz * nk;                     // (z, k step) of the next fetch
-  typename XgOperand<AK1, QUAD, 2, NT>::Vals va[2];
+  typename XgOperand<AK1, QUAD, HA, NT>::Vals va[2];
   typename XgOperand<BK1, QUAD, HB, NT>::Vals vb[2];
   int sfit = fit;
   const int rslot = xg_slot(lane & 15, lane >> 4);          // the record of (row lane % 16, g lane / 16)
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 1 : 2) void xgemm_kernel(c
 #pragma unroll
       for (int c = 0; c < NP; ++c) rB[f][c] = s_b[((wn + f) * NP + c) * 64 + rslot];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < EM; ++e) {
       u4 rA[NP];
 #pragma unroll
       for (int c = 0; c < NP; ++c) rA[c] = s_a[((wm + e) * NP + c) * 64 + rslot];
@@ -250,7 +252,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 1 : 2) void xgemm_kernel(c
   float* const sw = reinterpret_cast<float*>(s_mem) + wave * SLICE;
   const int c = lane & 15, g = lane >> 4;
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
+  for (int e = 0; e < EM; ++e)
 #pragma unroll
     for (int f = 0; f < EN; ++f) {
       if constexpr (TR) *reinterpret_cast<f4*>(sw + (16 * f + c) * LD + 16 * e + 4 * g) = acc[e][f];
@@ -262,7 +264,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 1 : 2) void xgemm_kernel(c
   __builtin_amdgcn_wave_barrier();                          // (a slice belongs to one wavefront)
   const float* const add = p.add ? p.add : p.reduce ? p.C : nullptr;
   const int mw = m0 + 16 * wm, nw = n0 + 16 * wn;
-  constexpr int ROWS = TR ? WN : 64, COLS = TR ? 64 : WN;   // rows of the slice run along the contiguous index of C
+  constexpr int ROWS = TR ? WN : WR, COLS = TR ? WR : WN;   // rows of the slice run along the contiguous index of C
   if (p.slices > 1) {                                       // uniform: summed into C (TR: one batch, nper = N)
     constexpr int RA = 64 / COLS;                           // lane = column (two rows at a time where 32 fill the row)
     const int q = lane % COLS;

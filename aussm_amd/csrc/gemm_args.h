@@ -24,7 +24,4 @@ struct XGemmArgs {
   int reduce;             // C holds the addend of the sum (zero for a plain product): slices may be more than one
 };
 
-constexpr int XG_TM = 128;      // rows of a workgroup tile
-constexpr int XG_TM_WIDE = 256; // ... of the tile of eight wavefronts
-
 }  // namespace aussm

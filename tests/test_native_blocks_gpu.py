@@ -66,6 +66,12 @@ def test_products_on_wide_tiles(b, l, i, o):
     test_products_of_a_linear_layer(b, l, i, o)
 
 
+# ... and tiles of few rows or few columns (rows: 32 and 64, columns: 32 and 64) over several tiles of the other index
+@pytest.mark.parametrize("b,l,i,o", [(3, 130, 32, 32), (3, 133, 33, 17), (2, 300, 140, 64), (2, 301, 65, 48), (2, 96, 32, 300)])
+def test_products_on_small_tiles(b, l, i, o):
+    test_products_of_a_linear_layer(b, l, i, o)
+
+
 @pytest.mark.parametrize("B,D,L,K", [(1, 1, 1, 4), (2, 5, 3, 4), (3, 70, 130, 4), (2, 9, 2050, 4), (2, 8, 33, 3), (1, 4, 7, 8)])
 def test_convolution_of_channel_rows(B, D, L, K):
     from aussm_amd import _lib, scan
