@@ -5,7 +5,7 @@
 namespace aussm {
 
 constexpr int CONV_PIECE = 2048;   // steps of a row per wavefront of the backward kernel
-constexpr int NORM_ROWS = 64;      // rows per workgroup of the norm's backward kernel
+constexpr int NORM_ROWS = 32;      // rows per workgroup of the norm's backward kernel
 constexpr int NORM_MAX_D = 1024;
 constexpr int COLSUM_ROWS = 256;
 

@@ -294,16 +294,17 @@ __device__ __forceinline__ float row_sum(float v) {     // total of the row in i
 }
 
 // The share of a tile's phase product that goes with state group a of 4: its steps k = a KS / 4 .. (KS < 4: all with a = 0).
-// Two accumulators, for the even and the odd steps, halve the chain of dependent matrix instructions.
+// One accumulator, in the order of the forward kernel: the states are recovered from its end state with these phases, and
+// phases that differ in their last bit would add up from tile to tile (gradients off by 1e-5 with two accumulators).
 template <int KS>
-__device__ __forceinline__ void phase_part(int a, const u4 (&xa)[KS][3], const u4* __restrict__ su, int lane, f4 (&acc)[2]) {
+__device__ __forceinline__ void phase_part(int a, const u4 (&xa)[KS][3], const u4* __restrict__ su, int lane, f4& acc) {
   constexpr int STEP = (KS + 3) / 4;
 #pragma unroll
   for (int k = a * STEP; k < (a + 1) * STEP && k < KS; ++k) {
     u4 ubk[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) ubk[q] = su[(k * 3 + q) * 64 + lane];
-    acc[k & 1] = xmm<3>(xa[k], ubk, acc[k & 1]);
+    acc = xmm<3>(xa[k], ubk, acc);
   }
 }
 
@@ -375,13 +376,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
   tile_load<NT, NREC, KS>(upb + (size_t)max(t_last - 1, t_first) * (KS * 3 * 64), sv, tid);
   tile_store<NT, NREC, KS>(sv, s_u[(t_last + 1) & 1], tid);
   __syncthreads();
-  f4 th;
-  {
-    f4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+  f4 th = {0, 0, 0, 0};
 #pragma unroll
-    for (int a = 0; a < 4; ++a) phase_part<KS>(a, xa, s_u[t_last & 1], lane, acc);
-    th = acc[0] + acc[1];
-  }
+  for (int a = 0; a < 4; ++a) phase_part<KS>(a, xa, s_u[t_last & 1], lane, th);
   __syncthreads();                                     // (the first iteration overwrites that tile)
   // the wavefront's own inputs, requested one tile ahead
   float un, dtn, zn, gyn;
@@ -404,7 +401,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
       gyn = q.gy[row + l - DT];
     }
     tile_load<NT, NREC, KS>(upb + (size_t)max(t - 2, t_first) * (KS * 3 * 64), sv, tid);
-    f4 nx[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};           // the next tile's phases, formed between the states of this one
+    f4 nx = {0, 0, 0, 0};                              // the next tile's phases, formed between the states of this one
     const u4* su = s_u[(t + 1) & 1];
     const float ut = silu_fast(uv), w = dtv * ut, sz = silu_fast(zv), av = gyv * sz;
     const float cnt = (float)(min(l_ + 1, L - l0));      // timesteps of the tile up to this one that exist
@@ -456,7 +453,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     ysum = rows_sum(ysum);
     wsum = rows_sum(wsum);
     if (nb > 1 && g == 0) s_yw[t & 1][wave][l_] = make_float2(ysum, wsum);
-    th = nx[0] + nx[1];
+    th = nx;
     tile_store<NT, NREC, KS>(sv, s_u[t & 1], tid);
     if (nb > 1) {                                      // the channel's first wavefront adds the shares up
       __syncthreads();

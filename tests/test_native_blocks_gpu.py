@@ -95,6 +95,12 @@ def test_convolution_of_channel_rows(B, D, L, K):
         torch.testing.assert_close(a.double() / scale, r / scale, atol=1e-5, rtol=1e-5)
 
 
+# rows of whole groups of four (16-byte loads): one group, a piece of the backward kernel and one group more, several pieces
+@pytest.mark.parametrize("B,D,L,K", [(1, 2, 4, 4), (2, 3, 8, 4), (3, 5, 720, 4), (1, 3, 2052, 4), (1, 2, 4100, 4), (2, 3, 64, 3)])
+def test_convolution_of_aligned_rows(B, D, L, K):
+    test_convolution_of_channel_rows(B, D, L, K)
+
+
 @pytest.mark.parametrize("rows,d", [(1, 1), (65, 3), (130, 64), (7, 65), (64, 200), (33, 513), (5, 1024)])
 @pytest.mark.parametrize("residual", [False, True])
 def test_norm_and_its_gradient(rows, d, residual):
@@ -112,6 +118,13 @@ def test_norm_and_its_gradient(rows, d, residual):
     torch.testing.assert_close(y.double(), ref.detach(), atol=1e-5, rtol=1e-5)
     torch.testing.assert_close(dx.double(), xd.grad + (res.double() if residual else 0), atol=1e-5, rtol=1e-5)
     torch.testing.assert_close(dw.double(), wd.grad, atol=1e-4, rtol=1e-5)      # up to 130 terms of size <= 10
+
+
+# ... and rows of whole groups of four, more of them than one workgroup takes, the last turn of a workgroup not full
+@pytest.mark.parametrize("rows,d", [(1, 132), (35, 256), (97, 200), (33, 260), (70, 512), (5, 516), (34, 1024)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_norm_of_aligned_rows(rows, d, residual):
+    test_norm_and_its_gradient(rows, d, residual)
 
 
 @pytest.mark.parametrize("kind,d,n,b,l,kw", [("a", 8, 4, 2, 33, {}), ("a", 40, 16, 3, 70, {"bias": True}), ("a", 24, 20, 1, 130, {"d_conv": 3}),
