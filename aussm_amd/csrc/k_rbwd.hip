@@ -25,7 +25,10 @@ static int rec_bwd_t(const RecBwdArgs& args, hipStream_t s) {
     // a full block of 16 states: eight wavefronts of two states, two wavefronts per SIMD (the complex scan with a
     // gate gradient to return keeps a fourth partial sum per wavefront)
     if (left > 8) {
-      if constexpr (VAR == VAR_COMPLEX) {
+      const bool plain = !a.z && !a.dz && !a.u_act && !a.delta_softplus && !a.delta_bias && !a.dbias && !a.accum;
+      if (plain) {
+        hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, false, true>), grid, dim3(512), 0, s, a);
+      } else if constexpr (VAR == VAR_COMPLEX) {
         if (a.dz) hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, true>), grid, dim3(512), 0, s, a);
         else hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, false>), grid, dim3(512), 0, s, a);
       } else {

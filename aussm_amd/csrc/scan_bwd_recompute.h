@@ -105,7 +105,9 @@ struct LaneTranspose16 {
 // two wavefronts into one slab with LDS float atomics instead made the kernel 2.5 times slower: those run far below
 // the rate of plain LDS writes.)
 // PLANE4: the complex scan's workgroups of eight wavefronts with the fourth plane (calls that want dz).
-template <int VAR, int NW, int NT, typename Tin, typename Tbc = Tin, bool PLANE4 = false>
+// PLAIN: calls without a gate, activations or a step bias on their first block of states: what those options keep in scalar
+// registers across the tile loop (90 of them spilled to vector lanes, 270 moves back) is not there.
+template <int VAR, int NW, int NT, typename Tin, typename Tbc = Tin, bool PLANE4 = false, bool PLAIN = false>
 __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   static_assert(VAR == VAR_COMPLEX || VAR == VAR_REAL, "unitary has its own kernel");
   constexpr int C = (VAR == VAR_REAL) ? 1 : 2;
@@ -155,7 +157,8 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   float* slab = s_slab + (WIDE ? wave * SLAB : 0);
   const size_t row_base = ((size_t)b * ((VAR == VAR_REAL && p.bcrows) ? p.bcrows : N) + n0) * ld + lbeg;
   // z and dz may be rows of a wider tensor: every address below is formed for rows of their own
-  const size_t zoff = (VAR == VAR_REAL && p.zrows) ? (size_t)b * (p.zrows - p.D) * ld : 0;
+  const bool gated = !PLAIN && p.z != nullptr;
+  const size_t zoff = (VAR == VAR_REAL && !PLAIN && p.zrows) ? (size_t)b * (p.zrows - p.D) * ld : 0;
 
   // ---- per-lane constants and accumulators
   float a2[NW], an[NW], dAacc[NW], gr[NW], gi[NW];
@@ -211,7 +214,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
     rowok[k] = dd < D;
     goff[k] = ((size_t)b * D + (rowok[k] ? dd : 0)) * ld + lbeg;
     dsk[k] = (p.Dskip && rowok[k]) ? p.Dskip[dd] : 0.f;
-    dbias[k] = (VAR == VAR_REAL && p.delta_bias && rowok[k]) ? p.delta_bias[dd] : 0.f;
+    dbias[k] = (VAR == VAR_REAL && !PLAIN && p.delta_bias && rowok[k]) ? p.delta_bias[dd] : 0.f;
     accD[k] = 0.f; accB[k] = 0.f;
     rdy.u[k] = rdy.dl[k] = fly.u[k] = fly.dl[k] = Tin(0);
     rdy.th[k] = rdy.rho[k] = rdy.gy[k] = fly.th[k] = fly.rho[k] = fly.gy[k] = 0.f;
@@ -225,14 +228,15 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       r.u[k] = gu[o];
       r.dl[k] = gdl[o];
       r.gy[k] = p.dy[o];
-      if (p.z) r.zz[k] = p.z[o + zoff];
+      if (gated) r.zz[k] = p.z[o + zoff];
       if (VAR == VAR_COMPLEX) { r.th[k] = p.theta[o]; r.rho[k] = p.rho[o]; }
     }
   };
   auto collect_tile = [&](RawTile& r) {
 #pragma unroll
     for (int k = 0; k < E; ++k) {
-      touch_vgpr(r.u[k]); touch_vgpr(r.dl[k]); touch_vgpr(r.gy[k]); touch_vgpr(r.zz[k]);
+      touch_vgpr(r.u[k]); touch_vgpr(r.dl[k]); touch_vgpr(r.gy[k]);
+      if (!PLAIN) touch_vgpr(r.zz[k]);
       if (VAR == VAR_COMPLEX) { touch_vgpr(r.th[k]); touch_vgpr(r.rho[k]); }
     }
   };
@@ -278,13 +282,13 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
     for (int k = 0; k < E; ++k) {
       const bool ok = rowok[k] && l0 + col < L;
       eu[k] = ok ? to_f32(rdy.u[k]) : 0.f;
-      if (VAR == VAR_REAL && p.u_act) {                    // uniform
+      if (VAR == VAR_REAL && !PLAIN && p.u_act) {          // uniform
         eact[k] = dsiluf_(eu[k]);
         eu[k] = siluf_(eu[k]);
       }
       egy[k] = ok ? rdy.gy[k] : 0.f;
       egz[k] = 0.f;
-      if (p.z) {                                           // uniform
+      if (gated) {                                         // uniform
         egz[k] = egy[k] * dsiluf_(rdy.zz[k]);
         egy[k] *= siluf_(rdy.zz[k]);
       }
@@ -293,7 +297,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       if (VAR == VAR_REAL) {
         dl += dbias[k];
         eraw[k] = dl;
-        if (p.delta_softplus) dl = softplusf_(dl);
+        if (!PLAIN && p.delta_softplus) dl = softplusf_(dl);
         if (!ok) dl = 0.f;                         // out-of-range steps: a = 1, w = 0
         rec = make_float4(dl, dl * eu[k], egy[k], 0.f);
       } else {
@@ -553,13 +557,13 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       for (int w = 0; w < NSLAB; ++w) { kk += pv[k][w].x; xx += pv[k][w].y; zz += pv[k][w].z; yy += pv[k][w].w; }
       if (rowok[k] && ll < L) {
         const size_t o = goff[k] + ll;
-        const bool acc = p.accum != 0;                   // uniform
+        const bool acc = !PLAIN && p.accum != 0;         // uniform
         float duv = acc ? kk * edl[k] : fmaf(kk, edl[k], dsk[k] * egy[k]);
         float dd = kk * eu[k];
-        if (VAR == VAR_REAL && p.u_act) duv *= eact[k];
+        if (VAR == VAR_REAL && !PLAIN && p.u_act) duv *= eact[k];
         if (VAR == VAR_REAL) {
           dd += xx;
-          if (p.delta_softplus) dd *= (eraw[k] > 20.0f) ? 1.0f : sigmoidf_(eraw[k]);
+          if (!PLAIN && p.delta_softplus) dd *= (eraw[k] > 20.0f) ? 1.0f : sigmoidf_(eraw[k]);
           accB[k] += dd;
         }
         if (sizeof(Tin) == 2 && p.g16) {                   // uniform
@@ -573,7 +577,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
           p.dtheta[o] = acc ? p.dtheta[o] + xx : xx;
           p.drho[o] = acc ? p.drho[o] + zz : zz;
         }
-        if (p.dz) {                                        // y_pre = sum over the states + D u (the latter once)
+        if (!PLAIN && p.dz) {                              // y_pre = sum over the states + D u (the latter once)
           const float dzv = egz[k] * (acc ? yy : fmaf(dsk[k], eu[k], yy));
           p.dz[o + zoff] = acc ? p.dz[o + zoff] + dzv : dzv;
         }
@@ -606,7 +610,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       if (col == 0 && rowok[k]) atomicAdd(p.dD + d0 + row0 + k * RSTEP, s);
     }
   }
-  if (VAR == VAR_REAL && p.dbias) {
+  if (VAR == VAR_REAL && !PLAIN && p.dbias) {
 #pragma unroll
     for (int k = 0; k < E; ++k) {
       float s = accB[k];
