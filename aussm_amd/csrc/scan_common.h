@@ -46,12 +46,33 @@ __device__ __forceinline__ int xcd_remap(int i, int G) {
   return x * q + (x < r ? x : r) + k;
 }
 
-__device__ __forceinline__ float sigmoidf_(float v) { return 1.0f / (1.0f + __expf(-v)); }
+// (reciprocal: the hardware's and one Newton step, 4 instructions where an IEEE division takes 11 and the same error; the
+// maximum takes the step away, 0 * inf, where 1 + e^-v is infinite)
+__device__ __forceinline__ float sigmoidf_(float v) {
+  const float x = 1.0f + __expf(-v), r = __builtin_amdgcn_rcpf(x);
+  return fmaf(r, fmaxf(fmaf(-x, r, 1.0f), -1.0f), r);
+}
 __device__ __forceinline__ float siluf_(float v) { return v * sigmoidf_(v); }
 // d/dv silu(v) = s + v s (1 - s)
 __device__ __forceinline__ float dsiluf_(float v) { float s = sigmoidf_(v); return s * (1.0f + v * (1.0f - s)); }
-// softplus with torch's threshold of 20 (F.softplus default)
-__device__ __forceinline__ float softplusf_(float v) { return v > 20.0f ? v : log1pf(__expf(v)); }
+// softplus with torch's threshold of 20 (F.softplus default), 33 vector instructions; log1pf(__expf(v)) takes 118, which was
+// a fifth of the gated S6 forward kernel.  Root mean square of the relative error for N(0, 1) 3.6e-8 against 4.3e-8, for
+// -20 .. 20 3.5e-8 against 2.3e-7.
+//   t = e^v, with the rounding of v log2(e) made up for (the maximum: v = -inf);  w = fl(1 + t) = 2^k m, m in
+//   [1 / sqrt 2, sqrt 2);  f = m - 1 plus what 1 + t was rounded by;  log(1 + f) = f - s (f - R), s = f / (2 + f),
+//   R = s^2 (2/3 + 2/5 s^2 + ..): the series of 2 artanh(s)
+__device__ __forceinline__ float softplusf_(float v) {
+  const float h = v * 1.44269504088896341f;
+  const float lo = fmaxf(fmaf(v, 1.92596299112661746887e-8f, fmaf(v, 1.44269504088896341f, -h)), -1.0f);
+  const float e = __builtin_amdgcn_exp2f(h);
+  const float t = fmaf(e, lo * 0.693147180559945309f, e), w = 1.0f + t;
+  const int u = __float_as_int(w) - 0x3f3504f3, k = u >> 23;
+  const float f = __builtin_amdgcn_ldexpf(t - (w - 1.0f), -k) + (__int_as_float((u & 0x7fffff) + 0x3f3504f3) - 1.0f);
+  const float s = f * __builtin_amdgcn_rcpf(2.0f + f), z = s * s;
+  const float R = z * fmaf(fmaf(fmaf(0.22222222f, z, 0.28571429f), z, 0.4f), z, 0.66666667f);
+  const float r = fmaf((float)k, 0.693147180559945309f, fmaf(-s, f - R, f));
+  return v > 20.0f ? v : r;
+}
 
 // sin and cos of one argument, about 25 VALU instructions and no branch on the common path.
 // Cody-Waite reduction by pi/2 in three fused steps, then minimax polynomials on [-pi/4, pi/4]

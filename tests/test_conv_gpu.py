@@ -99,3 +99,18 @@ def test_swap_last2_with_activation(b, r, c, sliced, act, with_bias):
         torch.testing.assert_close(a.double() / scale, w / scale, atol=1e-5, rtol=1e-5)
     with pytest.raises(ValueError):
         conv.swap_last2(x, act="tanh")
+
+
+def test_softplus_over_its_range():
+    """Relative error within three units in the last place (hardware exponential and reciprocal: one each, the last
+    rounding: half of one) wherever e^v is no denormal, the threshold of 20, and the special values."""
+    from aussm_amd import conv
+    print("case softplus range", flush=True)
+    x = torch.cat([torch.linspace(-87.0, 25.0, 200001), torch.tensor([0.0, 20.0, 20.001, -1e-7, 1e-7, -16.6, 15.9])]).cuda()
+    y = conv.swap_last2(x.view(1, 1, -1), act="softplus").flatten()
+    xd = x.double()
+    want = torch.where(xd > 20, xd, torch.log1p(torch.exp(xd)))
+    assert float(((y.double() - want).abs() / want).max()) < 3 * 2 ** -23
+    inf = float("inf")
+    y = conv.swap_last2(torch.tensor([inf, -inf, 1e30, -1e30, float("nan")]).cuda().view(1, 1, -1), act="softplus").flatten().tolist()
+    assert y[:4] == [inf, 0.0, torch.tensor(1e30).item(), 0.0] and y[4] != y[4]
