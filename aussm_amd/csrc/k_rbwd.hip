@@ -26,14 +26,21 @@ static int rec_bwd_t(const RecBwdArgs& args, hipStream_t s) {
     // gate gradient to return keeps a fourth partial sum per wavefront)
     if (left > 8) {
       const bool plain = !a.z && !a.dz && !a.u_act && !a.delta_softplus && !a.delta_bias && !a.dbias && !a.accum;
-      if (plain) {
-        hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, false, true>), grid, dim3(512), 0, s, a);
-      } else if constexpr (VAR == VAR_COMPLEX) {
-        if (a.dz) hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, true>), grid, dim3(512), 0, s, a);
-        else hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, false>), grid, dim3(512), 0, s, a);
-      } else {
-        hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float>), grid, dim3(512), 0, s, a);
-      }
+      // (a launch that is split along the sequence has segments of whole tiles, the last one may end earlier)
+      const bool whole = left >= 16 && a.D % CH == 0 && a.ld % RT == 0 && a.L % RT == 0;
+      auto go = [&](auto whole_tag) {
+        constexpr bool W = decltype(whole_tag)::value;
+        if (plain) {
+          hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, false, true, W>), grid, dim3(512), 0, s, a);
+        } else if constexpr (VAR == VAR_COMPLEX) {
+          if (a.dz) hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, true, false, W>), grid, dim3(512), 0, s, a);
+          else hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, false, false, W>), grid, dim3(512), 0, s, a);
+        } else {
+          hipLaunchKernelGGL((recompute_bwd_kernel<VAR, 2, 512, Tin, float, false, false, W>), grid, dim3(512), 0, s, a);
+        }
+      };
+      if (whole) go(std::true_type{});
+      else go(std::false_type{});
       done = true;
     }
 #endif

@@ -107,7 +107,9 @@ struct LaneTranspose16 {
 // PLANE4: the complex scan's workgroups of eight wavefronts with the fourth plane (calls that want dz).
 // PLAIN: calls without a gate, activations or a step bias on their first block of states: what those options keep in scalar
 // registers across the tile loop (90 of them spilled to vector lanes, 270 moves back) is not there.
-template <int VAR, int NW, int NT, typename Tin, typename Tbc = Tin, bool PLANE4 = false, bool PLAIN = false>
+// WHOLE: channels in whole groups of 64, whole tiles, and all states of the workgroup exist: no bounds (nor masks that hold
+// their outcome), no second form of the tile.
+template <int VAR, int NW, int NT, typename Tin, typename Tbc = Tin, bool PLANE4 = false, bool PLAIN = false, bool WHOLE = false>
 __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   static_assert(VAR == VAR_COMPLEX || VAR == VAR_REAL, "unitary has its own kernel");
   constexpr int C = (VAR == VAR_REAL) ? 1 : 2;
@@ -144,9 +146,9 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   const int N = p.N, D = p.D;
   const int L = (ld - lbeg < p.L) ? ld - lbeg : p.L;        // steps of this segment
   const int n0 = p.nbase + wave * NW;
-  const bool active = n0 < N;
+  const bool active = WHOLE || n0 < N;
   const int d = d0 + lane;
-  const bool dok = d < D;
+  const bool dok = WHOLE || d < D;
 
   const Tin* __restrict__ gu = static_cast<const Tin*>(p.u);
   const Tin* __restrict__ gdl = static_cast<const Tin*>(p.delta);
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   for (int k = 0; k < NW; ++k) {
     const int n = n0 + k;
     a2[k] = 0.f; an[k] = 0.f; dAacc[k] = 0.f; gr[k] = 0.f; gi[k] = 0.f;
-    if (dok && n < N) {
+    if (WHOLE || (dok && n < N)) {
       if (VAR == VAR_REAL) { an[k] = p.A[(size_t)d * N + n]; a2[k] = an[k] * LOG2E; }
       if (p.dhL) {
         const size_t o = (((size_t)vb * D + d) * N + n) * C;
@@ -183,7 +185,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
     for (int k = 0; k < NW; ++k) {
       const int n = n0 + k;
       s.r[k] = 0.f; s.i[k] = 0.f;
-      if (dok && n < N) {
+      if (WHOLE || (dok && n < N)) {
         if (tile0 + it > 0) {
           const size_t o = ((((size_t)b * p.nck + (tile0 + it - 1)) * N + n) * C) * D + d;
           s.r[k] = p.hck[o];
@@ -211,7 +213,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
 #pragma unroll
   for (int k = 0; k < E; ++k) {
     const int dd = d0 + row0 + k * RSTEP;
-    rowok[k] = dd < D;
+    rowok[k] = WHOLE || dd < D;
     goff[k] = ((size_t)b * D + (rowok[k] ? dd : 0)) * ld + lbeg;
     dsk[k] = (p.Dskip && rowok[k]) ? p.Dskip[dd] : 0.f;
     dbias[k] = (VAR == VAR_REAL && !PLAIN && p.delta_bias && rowok[k]) ? p.delta_bias[dd] : 0.f;
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   auto load_tile = [&](RawTile& r, int l0) {
 #pragma unroll
     for (int k = 0; k < E; ++k) {
-      const int ll = (l0 + col < L) ? l0 + col : L - 1;
+      const int ll = (WHOLE || l0 + col < L) ? l0 + col : L - 1;
       const size_t o = goff[k] + ll;
       r.u[k] = gu[o];
       r.dl[k] = gdl[o];
@@ -254,9 +256,9 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
   // lines of the tile that comes next are touched a tile ahead, during the staging maths, so that those loads
   // find them in the scalar cache.
   constexpr int RB = (int)sizeof(Tbc) * C;
-  const bool full_group = active && n0 + NW <= N;          // wave-uniform
+  const bool full_group = WHOLE || (active && n0 + NW <= N);   // wave-uniform
   TileWarm<NW, RB, RT> warm;
-  if (full_group && ntiles * RT == L) {
+  if (WHOLE || (full_group && ntiles * RT == L)) {
     warm.issue(gB, gC, row_base + (size_t)(ntiles - 1) * RT, ld);
     warm.retire();
   }
@@ -280,7 +282,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
     float eu[E], edl[E], egy[E], eraw[E], egz[E], eact[E];   // egz: dy silu'(z), for dz; eact: silu'(u)
 #pragma unroll
     for (int k = 0; k < E; ++k) {
-      const bool ok = rowok[k] && l0 + col < L;
+      const bool ok = WHOLE || (rowok[k] && l0 + col < L);
       eu[k] = ok ? to_f32(rdy.u[k]) : 0.f;
       if (VAR == VAR_REAL && !PLAIN && p.u_act) {          // uniform
         eact[k] = dsiluf_(eu[k]);
@@ -471,8 +473,12 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
     if (active) {
       // (bf16 rows start at even element offsets when L is even: wide loads stay 4-byte aligned)
       const bool full = (l0 + RT <= L) && (n0 + NW <= N) && (sizeof(Tbc) == 4 || (ld & 1) == 0);
-      if (full) tile_body(std::true_type{});
-      else tile_body(std::false_type{});
+      if constexpr (WHOLE) {
+        tile_body(std::true_type{});
+      } else {
+        if (full) tile_body(std::true_type{});
+        else tile_body(std::false_type{});
+      }
     }
     __syncthreads();
 
@@ -500,10 +506,10 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
               const float v = rres[(g * NW + k) * C + h];
               if (VAR == VAR_REAL) {
                 float* dst = (c >> 3) ? p.dC : p.dB;
-                if (mine && n0 + k < N && t + (c & 7) < L) atomicAdd(dst + row_base + (size_t)k * ld + t + (c & 7), v);
+                if (mine && (WHOLE || (n0 + k < N && t + (c & 7) < L))) atomicAdd(dst + row_base + (size_t)k * ld + t + (c & 7), v);
               } else {
                 float* dst = h ? p.dC : p.dB;
-                if (mine && n0 + k < N && t + (c >> 1) < L) atomicAdd(dst + 2 * (row_base + (size_t)k * ld + t) + c, v);
+                if (mine && (WHOLE || (n0 + k < N && t + (c >> 1) < L))) atomicAdd(dst + 2 * (row_base + (size_t)k * ld + t) + c, v);
               }
             }
       } else {
@@ -555,7 +561,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       float kk = 0.f, xx = 0.f, zz = 0.f, yy = 0.f;
 #pragma unroll
       for (int w = 0; w < NSLAB; ++w) { kk += pv[k][w].x; xx += pv[k][w].y; zz += pv[k][w].z; yy += pv[k][w].w; }
-      if (rowok[k] && ll < L) {
+      if (WHOLE || (rowok[k] && ll < L)) {
         const size_t o = goff[k] + ll;
         const bool acc = !PLAIN && p.accum != 0;         // uniform
         float duv = acc ? kk * edl[k] : fmaf(kk, edl[k], dsk[k] * egy[k]);
@@ -591,7 +597,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
 #pragma unroll
     for (int k = 0; k < NW; ++k) {
       const int n = n0 + k;
-      if (n < N) {
+      if (WHOLE || n < N) {
         if (p.dh0) {
           const size_t o = (((size_t)vb * D + d) * N + n) * C;
           p.dh0[o] = gr[k];
@@ -607,7 +613,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       float s = accD[k];
 #pragma unroll
       for (int o = RT / 2; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-      if (col == 0 && rowok[k]) atomicAdd(p.dD + d0 + row0 + k * RSTEP, s);
+      if (col == 0 && (WHOLE || rowok[k])) atomicAdd(p.dD + d0 + row0 + k * RSTEP, s);
     }
   }
   if (VAR == VAR_REAL && !PLAIN && p.dbias) {
@@ -616,7 +622,7 @@ __global__ __launch_bounds__(NT) void recompute_bwd_kernel(const RecBwdArgs p) {
       float s = accB[k];
 #pragma unroll
       for (int o = RT / 2; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-      if (col == 0 && rowok[k]) atomicAdd(p.dbias + d0 + row0 + k * RSTEP, p.dbias_scale * s);
+      if (col == 0 && (WHOLE || rowok[k])) atomicAdd(p.dbias + d0 + row0 + k * RSTEP, p.dbias_scale * s);
     }
   }
 }
