@@ -58,7 +58,7 @@ BWD_KERNELS = {0: ["unitary_bwd_kernel"], 2: ["unitary_bwd_xdl_kernel<2"], 3: ["
 def source_digest() -> str:
     """Digest of the kernel sources: a traffic record is only valid for the sources it was taken with."""
     h = hashlib.sha256()
-    for f in sorted(glob.glob(os.path.join(ROOT, "aussm_amd", "csrc", "*"))):
+    for f in sorted(glob.glob(os.path.join(ROOT, "aussm_amd", "csrc", "*.h")) + glob.glob(os.path.join(ROOT, "aussm_amd", "csrc", "*.hip"))):
         h.update(os.path.basename(f).encode())
         h.update(open(f, "rb").read())
     return h.hexdigest()[:16]

@@ -85,3 +85,16 @@ def test_scanner_on_hand_made_listings():
 
 def test_kernels_keep_loads_in_flight_intact():
     build.check_px_listing(verbose=False)
+
+
+def test_benchmark_digests_the_kernel_sources():
+    """The record of measured traffic is tied to the kernel sources, whatever else lies beside them."""
+    import os
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    sys.path.insert(0, root)
+    try:
+        import bench
+    finally:
+        sys.path.remove(root)
+    assert os.path.isdir(os.path.join(root, "aussm_amd", "csrc", "host")) and len(bench.source_digest()) == 16
