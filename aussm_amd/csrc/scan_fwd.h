@@ -12,7 +12,10 @@ namespace aussm {
 // VAR: variant.  NW: states per wavefront.  NT: threads per workgroup.  Tin: float or bf16_t (u, delta).
 // Tbc: type of B_t / C_t (bf16 rows cost scalar-ALU conversions in the scan; the complex and real entry
 // points convert them to float once per call instead).
-template <int VAR, int NW, int NT, typename Tin, typename Tbc = Tin>
+// PLAIN: no gate, activation or step bias, nothing kept for a split launch; channels in whole groups of 64, whole tiles, all
+// states of the workgroup exist, 16-byte accesses: no bounds, no options, and none of the scalar registers that hold them
+// (S6 B32 D512 N16 L2048, bf16: 240 -> 210 us).
+template <int VAR, int NW, int NT, typename Tin, typename Tbc = Tin, bool PLAIN = false>
 __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
   constexpr int C = (VAR == VAR_REAL) ? 1 : 2;   // floats per state
   constexpr int NWV = NT / 64;                   // wavefronts per workgroup
@@ -34,9 +37,9 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
   const int N = p.N, D = p.D;
   const int L = (ld - lbeg < p.L) ? ld - lbeg : p.L;      // steps of this segment
   const int n0 = wave * NW;
-  const bool active = n0 < N;                    // wave-uniform
+  const bool active = PLAIN || n0 < N;           // wave-uniform
   const int d = d0 + lane;
-  const bool dok = d < D;
+  const bool dok = PLAIN || d < D;
 
   // u and delta may be shared by p.urep consecutive batch elements (tensors [B / urep, D, L]): every
   // address below is formed for batch element b, so their base steps back by the difference
@@ -47,7 +50,8 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
   const Tbc* __restrict__ gC = static_cast<const Tbc*>(p.Cm);
 
   // z may be rows of a wider tensor: every address below is formed for rows of its own
-  const float* __restrict__ gz = p.z ? p.z + ((VAR == VAR_REAL && p.zrows) ? (size_t)b * (p.zrows - p.D) * ld : 0) : nullptr;
+  const bool gated = !PLAIN && p.z != nullptr;
+  const float* __restrict__ gz = gated ? p.z + ((VAR == VAR_REAL && p.zrows) ? (size_t)b * (p.zrows - p.D) * ld : 0) : nullptr;
 
   // ---- scan-side state (lane == channel)
   float hr[NW], hi[NW], a2[NW];
@@ -55,7 +59,7 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
   for (int k = 0; k < NW; ++k) {
     const int n = n0 + k;
     hr[k] = 0.f; hi[k] = 0.f; a2[k] = 0.f;
-    if (dok && n < N) {
+    if (PLAIN || (dok && n < N)) {
       if (p.h0) {
         const size_t o = (((size_t)vb * D + d) * N + n) * C;
         hr[k] = p.h0[o];
@@ -84,17 +88,17 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
     srow[k] = row0 + k * SG::RP;
     inrow[k] = srow[k] < CH;                     // this thread has a row in this pass
     const int dd = d0 + srow[k];
-    rowok[k] = inrow[k] && dd < D;
+    rowok[k] = inrow[k] && (PLAIN || dd < D);
     goff[k] = ((size_t)b * D + (rowok[k] ? dd : 0)) * ld + lbeg;
     dsk[k] = (p.Dskip && rowok[k]) ? p.Dskip[dd] : 0.f;
-    dbias[k] = (VAR == VAR_REAL && p.delta_bias && rowok[k]) ? p.delta_bias[dd] : 0.f;
+    dbias[k] = (VAR == VAR_REAL && !PLAIN && p.delta_bias && rowok[k]) ? p.delta_bias[dd] : 0.f;
     rdy.u[k].zero(); rdy.dl[k].zero(); rdy.th[k].zero(); rdy.rho[k].zero(); rdy.z[k].zero();
     fly.u[k].zero(); fly.dl[k].zero(); fly.th[k].zero(); fly.rho[k].zero(); fly.z[k].zero();
   }
   // 16-byte accesses need every row start (L % 4 == 0) and every tensor base aligned
   auto al = [](const void* q, size_t a) { return q == nullptr || (reinterpret_cast<uintptr_t>(q) % a) == 0; };
-  const bool vec = (ld % 4 == 0) && (L % 4 == 0) && al(p.u, 4 * sizeof(Tin)) && al(p.delta, 4 * sizeof(Tin)) && al(p.theta, 16) &&
-                   al(p.rho, 16) && al(p.z, 16) && al(p.y, 16);
+  const bool vec = PLAIN || ((ld % 4 == 0) && (L % 4 == 0) && al(p.u, 4 * sizeof(Tin)) && al(p.delta, 4 * sizeof(Tin)) && al(p.theta, 16) &&
+                   al(p.rho, 16) && al(p.z, 16) && al(p.y, 16));
 
   auto load_tile = [&](RawTile& r, int l0) {
 #pragma unroll
@@ -106,13 +110,13 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
       const int ll = l0 + t0;
       int idx[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) idx[i] = (ll + i < L) ? ll + i : L - 1;
-      const size_t o = goff[k] + (vec ? ((ll < L) ? ll : L - 4) : 0);
+      for (int i = 0; i < 4; ++i) idx[i] = (PLAIN || ll + i < L) ? ll + i : L - 1;
+      const size_t o = goff[k] + (vec ? ((PLAIN || ll < L) ? ll : L - 4) : 0);
       r.u[k].load(gu, o, vec, idx);
       r.dl[k].load(gdl, o, vec, idx);
       if (VAR != VAR_REAL) r.th[k].load(p.theta, o, vec, idx);
       if (VAR == VAR_COMPLEX) r.rho[k].load(p.rho, o, vec, idx);
-      if (p.z) r.z[k].load(gz, o, vec, idx);
+      if (gated) r.z[k].load(gz, o, vec, idx);
     }
   };
   // A use of every register of a set: the compiler puts its wait for the loads here.
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
       r.u[k].touch(); r.dl[k].touch();
       if (VAR != VAR_REAL) r.th[k].touch();
       if (VAR == VAR_COMPLEX) r.rho[k].touch();
-      if (p.z) r.z[k].touch();
+      if (gated) r.z[k].touch();
     }
   };
   load_tile(rdy, 0);
@@ -134,7 +138,7 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
   // touched here, a whole tile ahead, while the vector ALUs are busy with the staging maths.
   constexpr bool WARM = NW <= 4;
   constexpr int RB = (int)sizeof(Tbc) * C;
-  const bool full_group = active && n0 + NW <= N;
+  const bool full_group = PLAIN || (active && n0 + NW <= N);
   TileWarm<WARM ? NW : 1, RB> warm;
   const size_t bc_row = ((size_t)b * ((VAR == VAR_REAL && p.bcrows) ? p.bcrows : N) + n0) * ld + lbeg;   // B_t / C_t: row n0, first step of the segment
   if (WARM && full_group && T <= L) {
@@ -144,7 +148,7 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
 
   // product of the a_l over the segment (complex) or sum of the step sizes (real), kept by wavefront 0
   // of a launch that wants it (a split launch chains its segments with it)
-  const bool want_tot = p.ptot != nullptr && wave == 0;   // wave-uniform
+  const bool want_tot = !PLAIN && p.ptot != nullptr && wave == 0;   // wave-uniform
   float fr = (VAR == VAR_REAL) ? 0.f : 1.f, fi = 0.f;
 
   // a wavefront that owns no state never writes its slab of partial read-outs: it clears it once, so that the
@@ -163,14 +167,14 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
     for (int k = 0; k < PASS; ++k) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const bool ok = rowok[k] && l0 + t0 + i < L;
+        const bool ok = PLAIN || (rowok[k] && l0 + t0 + i < L);
         float uu = ok ? rdy.u[k].get(i) : 0.f;
-        if (VAR == VAR_REAL && p.u_act) uu = siluf_(uu);
+        if (VAR == VAR_REAL && !PLAIN && p.u_act) uu = siluf_(uu);
         float dl = ok ? rdy.dl[k].get(i) : 0.f;
         float4 rec;
         if (VAR == VAR_REAL) {
           dl += dbias[k];
-          if (p.delta_softplus) dl = softplusf_(dl);
+          if (!PLAIN && p.delta_softplus) dl = softplusf_(dl);
           rec = make_float4(dl, dl * uu, 0.f, 0.f);
         } else {
           float sn, cs;
@@ -187,12 +191,11 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
     __syncthreads();
 
     // ---- scan: lane == channel, sequential over the tile's timesteps
-    const int tmax = (L - l0 < T) ? (L - l0) : T;
+    const int tmax = (PLAIN || L - l0 >= T) ? T : (L - l0);
     const size_t brow = bc_row + l0;
     // fast path: a full tile and a full group of states.  (bf16 real rows need an even offset
     // so that the 8-element scalar load is 4-byte aligned.)
-    const bool fast = tmax == T && n0 + NW <= N &&
-                      !(VAR == VAR_REAL && sizeof(Tbc) == 2 && (ld & 1));
+    const bool fast = PLAIN || (tmax == T && n0 + NW <= N && !(VAR == VAR_REAL && sizeof(Tbc) == 2 && (ld & 1)));
     float mr[NW], mi[NW];                        // state after the first half of the tile
 #pragma unroll
     for (int k = 0; k < NW; ++k) { mr[k] = 0.f; mi[k] = 0.f; }
@@ -388,10 +391,10 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
           acc[i] = yin[k][i];
 #pragma unroll
           for (int w = 0; w < NWV; ++w) acc[i] += pv[k][i][w];
-          if (p.z) acc[i] *= siluf_(gate[k][i]);
+          if (gated) acc[i] *= siluf_(gate[k][i]);
         }
         const int nvalid = L - (l0 + t0);
-        if (rowok[k] && nvalid > 0) store4(p.y, goff[k] + l0 + t0, acc, vec, nvalid);
+        if (PLAIN ? inrow[k] : rowok[k] && nvalid > 0) store4(p.y, goff[k] + l0 + t0, acc, vec, nvalid);
       }
     }
     // ---- checkpoint at the end of every ck-step block (and at the end of the sequence).
@@ -402,7 +405,7 @@ __global__ __launch_bounds__(NT) void core_fwd_kernel(const FwdArgs p) {
 #pragma unroll
         for (int k = 0; k < NW; ++k) {
           const int n = n0 + k;
-          if (n < N) {
+          if (PLAIN || n < N) {
             const size_t o = ((((size_t)b * p.nck + sg * (p.L / p.ck) + kb) * N + n) * C) * D + d;
             p.hck[o] = xr[k];
             if (C == 2) p.hck[o + D] = xi[k];

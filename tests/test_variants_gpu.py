@@ -148,6 +148,31 @@ def test_real_gradients(B, D, N, L, softplus, gate):
         _close(got[k], want[k], f"d{k}")
 
 
+# whole groups of 64 channels, whole tiles of 16 (backward) or 32 (forward) steps, 16 states: the instances without bounds;
+# two blocks of states, whole backward but not whole forward tiles, and a split launch of whole segments
+WHOLE = [(1, 64, 16, 16), (2, 128, 16, 64), (3, 64, 32, 48), (2, 64, 16, 96), (1, 64, 16, 512)]
+
+
+@pytest.mark.parametrize("B,D,N,L", WHOLE)
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("variant", ["complex", "real"])
+def test_whole_shapes(B, D, N, L, gate, variant):
+    from aussm_amd import scan
+    print(f"case whole {variant} B={B} D={D} N={N} L={L} gate={gate}", flush=True)
+    (test_complex_gradients if variant == "complex" else lambda *a: test_real_gradients(*a[:4], gate, gate))(B, D, N, L, gate)
+    p = O.make_core_inputs(B, D, N, L, seed=L + N, variant=variant, gate=gate)
+    q = {k: v.cuda() for k, v in p.items()}
+    if variant == "complex":
+        args = ("u", "delta", "rho", "theta", "Bc", "Cc", "Dskip")
+        want, _ = O.complex_core_loop(*(p[k] for k in args), p.get("z"))
+        y = scan.complex_scan(*(q[k] for k in args), q.get("z"))
+    else:
+        args = ("u", "delta", "A", "Bm", "Cm", "Dskip")
+        want, _ = O.real_core_loop(*(p[k] for k in args), p.get("z"))
+        y = scan.selective_scan_fn(*(q[k] for k in args), q.get("z"))
+    _close(y, want, "y")
+
+
 def test_state_limit():
     """64 states per channel is the limit of both directions (AUSSM_MAX_STATE)."""
     from aussm_amd import scan
