@@ -25,7 +25,7 @@ __device__ __forceinline__ void divide(size_t a, unsigned d, size_t* q, unsigned
 // aussm.py:762, :863, along rows of L elements.  Thread = four consecutive steps of one row.  Memory bound: 8 bytes per
 // element.
 // V4: K = 4, rows of whole, aligned groups of four: the four steps and the four before them are two 16-byte loads
-// (32 x 256 rows of 720 steps 24 -> 11 us; with one load per tap and step the loads were what took the time).
+// (32 x 256 and 32 x 512 rows of 720 steps, mean 37 -> 14 us; one load per tap and step and 64-bit divisions took the time).
 template <int K, bool V4>
 __global__ __launch_bounds__(256) void conv_rows_fwd_kernel(const ConvRowsArgs p) {
   const int nq = (p.L + 3) / 4;
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void conv_rows_fwd_kernel(const ConvRowsArgs p
 
 // dx[b,i,l] = sum_k w[i,k] dy[b,i,l + (K-1) - k];  dw[i,k] += sum dy[l] x[l - (K-1) + k];  dbias[i] += sum dy.
 // One wavefront per (row, piece of CONV_PIECE steps): dx and the weight sums in one pass over dy and x.
-// V4: as in the forward kernel, four steps per lane and turn from four 16-byte loads.
+// V4: as in the forward kernel, four steps per lane and turn from four 16-byte loads (the same rows, mean 35 -> 27 us).
 template <int K, bool V4>
 __global__ __launch_bounds__(256) void conv_rows_bwd_kernel(const ConvRowsArgs p) {
   const int lane = threadIdx.x & 63;
@@ -175,8 +175,8 @@ __device__ __forceinline__ float lanes_sum(float v) {
 // A workgroup of four wavefronts walks NORM_ROWS rows, R rows per wavefront and turn, all their loads in flight together; the
 // sums for dw stay in registers until the end, meet in LDS and leave as one atomic per column and workgroup.
 // V4: rows of whole, aligned groups of four; lane = four neighbouring columns of every 256.
-// Memory bound: 12 bytes per element (16 with the residual).  23040 rows of 256 with the residual: 61 us with one row at a
-// time and 4-byte loads.
+// Memory bound: 12 bytes per element (16 with the residual).  23040 rows of 256 with the residual: 27 us; 61 us with one
+// row at a time and 4-byte loads.
 template <int NJ, bool V4>
 __global__ __launch_bounds__(256) void rms_norm_bwd_kernel(const NormArgs p) {
   static_assert(!V4 || NJ % 4 == 0, "four columns per lane");
