@@ -8,6 +8,8 @@
 #include "common.h"
 #include "host.h"
 
+#include <torch/csrc/autograd/autograd.h>
+
 namespace aussm_host {
 
 namespace {
@@ -138,6 +140,48 @@ bool front_ok(const Tensor& x, const Tensor& nw, bool norm, const Tensor& W_in, 
   return s.b * s.l < (1ll << 31) / 2 && s.l < (1 << 24) && s.b * (s.e + 3) / 4 < 0x7fffffffll;
 }
 
+// ---- the same from differentiable operators, for a backward pass that is recorded (create_graph) ----------
+Tensor composed_norm(const Tensor& x, const Tensor& w, double eps) {
+  return w.defined() ? x * (x.square().mean({-1}, true) + eps).rsqrt() * w : x;
+}
+// channel rows (u behind the convolution, z) of the input projection of x
+std::pair<Tensor, Tensor> composed_front(const BlockDims& s, const Tensor& x, const Tensor& nw, const Tensor& W_in, const Tensor& b_in,
+                                         const Tensor& cw, const Tensor& cb) {
+  const Tensor xz = at::linear(composed_norm(x, nw, s.eps), W_in, b_in).transpose(1, 2);
+  const Tensor in = at::constant_pad_nd(xz.narrow(1, 0, s.e), {s.K - 1, 0}), w = cw.reshape({s.e, s.K, 1});
+  Tensor u = in.narrow(2, 0, s.l) * w.select(1, 0);
+  for (int64_t k = 1; k < s.K; ++k) u = u + in.narrow(2, k, s.l) * w.select(1, k);
+  return {cb.defined() ? u + cb.unsqueeze(1) : u, xz.narrow(1, s.e, s.e)};
+}
+Tensor composed_back(const BlockDims& s, const Tensor& y, const Tensor& W_out, const Tensor& b_out, const Tensor& x) {
+  const Tensor out = at::linear(y.transpose(1, 2), W_out, b_out);
+  return s.residual ? out + x : out;
+}
+// Gradients of compose(inputs) for the first `count` saved tensors, recorded.  The operators get an alias of each input: what
+// an input owes to another one (one tensor handed in twice, a weight formed from x) is the outer graph's to follow.
+template <typename F>
+variable_list recorded_gradients(SavingNode& node, std::mutex& m, int count, const Tensor& g, const F& compose) {
+  variable_list in(count), out(count), wanted;
+  if (!g.defined()) return out;
+  {
+    std::lock_guard<std::mutex> lock(m);
+    for (int i = 0; i < count; ++i) in[i] = node.saved[i].unpack();
+  }
+  std::vector<int> at;
+  for (int i = 0; i < count; ++i) {
+    if (!in[i].defined() || !in[i].requires_grad()) continue;
+    in[i] = in[i].alias();
+    if (!node.task_should_compute_output(i)) continue;
+    wanted.push_back(in[i]);
+    at.push_back(i);
+  }
+  if (wanted.empty()) return out;
+  const c10::DeviceGuard guard(in[0].device());
+  const variable_list got = torch::autograd::grad({compose(in)}, wanted, {g}, true, true, true);
+  for (size_t k = 0; k < at.size(); ++k) out[at[k]] = got[k];
+  return out;
+}
+
 }  // namespace
 
 // ============================================================================ AUSSM block
@@ -151,7 +195,8 @@ struct AussmBlockNode : SavingNode {
   int64_t n, r;
   float scale;
   std::string name() const override { return "AussmBlockBackward"; }
-  variable_list apply(variable_list&& g) override;
+  variable_list gradients(const variable_list& g) override;
+  variable_list recorded(variable_list&& g) override;
 };
 
 aussm_operator_args block_operator(const BlockDims& s, int64_t n, float scale, const Tensor& u, const Tensor& dt, const Tensor* in, const Tensor& xz) {
@@ -164,13 +209,11 @@ aussm_operator_args block_operator(const BlockDims& s, int64_t n, float scale, c
   return p;
 }
 
-variable_list AussmBlockNode::apply(variable_list&& g) {
-  std::lock_guard<std::mutex> lock(mutex_);
-  at::NoGradGuard no_grad;
+variable_list AussmBlockNode::gradients(const variable_list& g) {
   variable_list out(A_INPUTS);
   if (!g[0].defined()) return out;
   Tensor in[A_INPUTS];
-  for (int i = 0; i < A_INPUTS; ++i) in[i] = saved[i].unpack();
+  for (int i = 0; i < A_INPUTS; ++i) in[i] = dense(saved[i].unpack());
   const Tensor xn = saved[A_INPUTS].unpack(), rstd = saved[A_INPUTS + 1].unpack(), xz = saved[A_INPUTS + 2].unpack(),
                u = saved[A_INPUTS + 3].unpack(), dt0 = saved[A_INPUTS + 4].unpack(), dt = saved[A_INPUTS + 5].unpack(),
                y = saved[A_INPUTS + 6].unpack(), nh_re = saved[A_INPUTS + 7].unpack(), nh_im = saved[A_INPUTS + 8].unpack();
@@ -209,6 +252,16 @@ variable_list AussmBlockNode::apply(variable_list&& g) {
   for (int i : {A_NW, A_WIN, A_BIN, A_CW, A_CB, A_WXP, A_WDT, A_WOUT, A_BOUT})
     if (need(i)) out[i] = acc.like(id[i], in[i]);
   return out;
+}
+
+variable_list AussmBlockNode::recorded(variable_list&& g) {
+  return recorded_gradients(*this, mutex_, A_INPUTS, g[0], [&](const variable_list& in) {
+    const auto [u, z] = composed_front(s, in[A_X], in[A_NW], in[A_WIN], in[A_BIN], in[A_CW], in[A_CB]);
+    const Tensor dt = at::linear(at::linear(u.transpose(1, 2), in[A_WXP]), in[A_WDT], in[A_BDT]) + in[A_BDT];
+    const Tensor y = adaptive_operator(u, at::softplus(dt).transpose(1, 2), in[A_XAW].reshape({n, s.e, s.e}).transpose(0, 1) * (double)scale,
+                                       in[A_XAB].reshape({n, s.e}).t(), in[A_B], in[A_C], in[A_D], z);
+    return composed_back(s, y, in[A_WOUT], in[A_BOUT], in[A_X]);
+  });
 }
 
 }  // namespace
@@ -253,8 +306,8 @@ OptTensor aussm_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
       node = make_node<AussmBlockNode>();
       node->set_next_edges(torch::autograd::collect_next_edges(raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9],
                                                                raw[10], raw[11], raw[12], raw[13], raw[14], raw[15]));
-      node->save({in[0], in[1], in[2], in[3], in[4], in[5], in[6], in[7], in[8], in[9], in[10], in[11], in[12], in[13], in[14], in[15], f.xn,
-                  f.rstd, f.xz, f.u, dt0, dt, y, nh_re, nh_im});
+      node->save({raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9], raw[10], raw[11], raw[12], raw[13], raw[14],
+                  raw[15], f.xn, f.rstd, f.xz, f.u, dt0, dt, y, nh_re, nh_im});
       node->s = s; node->n = n; node->r = r; node->scale = (float)scale;
     }
   }
@@ -273,16 +326,15 @@ struct MambaBlockNode : SavingNode {
   BlockDims s;
   int64_t n, r;
   std::string name() const override { return "AussmMambaBlockBackward"; }
-  variable_list apply(variable_list&& g) override;
+  variable_list gradients(const variable_list& g) override;
+  variable_list recorded(variable_list&& g) override;
 };
 
-variable_list MambaBlockNode::apply(variable_list&& g) {
-  std::lock_guard<std::mutex> lock(mutex_);
-  at::NoGradGuard no_grad;
+variable_list MambaBlockNode::gradients(const variable_list& g) {
   variable_list out(M_INPUTS);
   if (!g[0].defined()) return out;
   Tensor in[M_INPUTS];
-  for (int i = 0; i < M_INPUTS; ++i) in[i] = saved[i].unpack();
+  for (int i = 0; i < M_INPUTS; ++i) in[i] = dense(saved[i].unpack());
   const Tensor xn = saved[M_INPUTS].unpack(), rstd = saved[M_INPUTS + 1].unpack(), xz = saved[M_INPUTS + 2].unpack(),
                u = saved[M_INPUTS + 3].unpack(), dbc = saved[M_INPUTS + 4].unpack(), dt = saved[M_INPUTS + 5].unpack(),
                A = saved[M_INPUTS + 6].unpack(), hck = saved[M_INPUTS + 7].unpack(), y = saved[M_INPUTS + 8].unpack();
@@ -325,6 +377,17 @@ variable_list MambaBlockNode::apply(variable_list&& g) {
     check(aussm_neg_exp(ptr(in[M_ALOG]), acc.p(iA), ptr(out[M_ALOG]), e * n, cur_stream()), "aussm_neg_exp");
   }
   return out;
+}
+
+variable_list MambaBlockNode::recorded(variable_list&& g) {
+  return recorded_gradients(*this, mutex_, M_INPUTS, g[0], [&](const variable_list& in) {
+    const auto [c, z] = composed_front(s, in[M_X], in[M_NW], in[M_WIN], in[M_BIN], in[M_CW], in[M_CB]);
+    const Tensor u = at::silu(c), dbc = at::linear(c.transpose(1, 2), in[M_WXP]);    // (x_proj reads the rows before their SiLU)
+    const Tensor dt = at::linear(dbc.narrow(2, 0, r), in[M_WDT], in[M_BDT]).transpose(1, 2);
+    const Tensor y = selective_scan(u, dt, -in[M_ALOG].exp(), dbc.narrow(2, r, n).transpose(1, 2), dbc.narrow(2, r + n, n).transpose(1, 2),
+                                    in[M_D], z, in[M_BDT], true, false, std::nullopt).first;
+    return composed_back(s, y, in[M_WOUT], in[M_BOUT], in[M_X]);
+  });
 }
 
 }  // namespace
@@ -375,8 +438,8 @@ OptTensor mamba_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
       node = make_node<MambaBlockNode>();
       node->set_next_edges(torch::autograd::collect_next_edges(raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9],
                                                                raw[10], raw[11], raw[12]));
-      node->save({in[0], in[1], in[2], in[3], in[4], in[5], in[6], in[7], in[8], in[9], in[10], in[11], in[12], f.xn, f.rstd, f.xz, f.u, dbc, dt,
-                  A, hck, y});
+      node->save({raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9], raw[10], raw[11], raw[12], f.xn, f.rstd, f.xz,
+                  f.u, dbc, dt, A, hck, y});
       node->s = s; node->n = n; node->r = r;
     }
   }
@@ -393,17 +456,17 @@ enum { L_X, L_NW, L_W, L_B, L_INPUTS };
 struct LinearNode : SavingNode {
   int64_t rows, i, o;
   bool norm;
+  double eps;
   std::string name() const override { return "AussmLinearBackward"; }
-  variable_list apply(variable_list&& g) override;
+  variable_list gradients(const variable_list& g) override;
+  variable_list recorded(variable_list&& g) override;
 };
 
-variable_list LinearNode::apply(variable_list&& g) {
-  std::lock_guard<std::mutex> lock(mutex_);
-  at::NoGradGuard no_grad;
+variable_list LinearNode::gradients(const variable_list& g) {
   variable_list out(L_INPUTS);
   if (!g[0].defined()) return out;
   Tensor in[L_INPUTS];
-  for (int k = 0; k < L_INPUTS; ++k) in[k] = saved[k].unpack();
+  for (int k = 0; k < L_INPUTS; ++k) in[k] = dense(saved[k].unpack());
   const Tensor xn = saved[L_INPUTS].unpack(), rstd = saved[L_INPUTS + 1].unpack();
   const Tensor& x = in[L_X];
   const c10::DeviceGuard guard(x.device());
@@ -433,6 +496,12 @@ variable_list LinearNode::apply(variable_list&& g) {
     }
   }
   return out;
+}
+
+variable_list LinearNode::recorded(variable_list&& g) {
+  return recorded_gradients(*this, mutex_, L_INPUTS, g[0], [&](const variable_list& in) {
+    return at::linear(composed_norm(in[L_X], in[L_NW], eps), in[L_W], in[L_B]);
+  });
 }
 
 }  // namespace
@@ -465,8 +534,8 @@ OptTensor norm_linear(const Tensor& x_, const OptTensor& nw_, double eps, const 
     if (needs_grad) {
       node = make_node<LinearNode>();
       node->set_next_edges(torch::autograd::collect_next_edges(x_, nwv, W_, bv));
-      node->save({x, nw, W, b, xn, rstd});
-      node->rows = rows; node->i = i; node->o = o; node->norm = nw.defined();
+      node->save({x_, nwv, W_, bv, xn, rstd});
+      node->rows = rows; node->i = i; node->o = o; node->norm = nw.defined(); node->eps = eps;
     }
   }
   if (node) torch::autograd::set_history(y, node);

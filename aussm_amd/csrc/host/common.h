@@ -7,6 +7,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 
@@ -112,6 +113,34 @@ struct SavingNode : Node {
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
     for (auto& s : saved) s.reset_data();
+  }
+  variable_list apply(variable_list&& g) override {
+    if (at::GradMode::is_enabled()) return recorded(std::move(g));
+    return launched(g);
+  }
+  // gradients of the inputs from the kernels, called with gradient recording off
+  virtual variable_list gradients(const variable_list& g) = 0;
+  variable_list launched(const variable_list& g) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    at::NoGradGuard no_grad;
+    return gradients(g);
+  }
+  // ... and for a backward pass that is recorded itself (create_graph).  The kernels' gradients carry no graph: they can
+  // be used, and differentiating them raises.  (The error hangs on the edges of this node and of the gradients
+  // it got, so that every derivative that should pass through it does.)
+  virtual variable_list recorded(variable_list&& g) {
+    variable_list out = launched(g);
+    torch::autograd::edge_list edges = torch::autograd::collect_next_edges(g);
+    edges.insert(edges.end(), next_edges().begin(), next_edges().end());
+    std::shared_ptr<Node> refusal(new torch::autograd::Error(cat(name(), ": second derivatives of this operator are not implemented"),
+                                                             std::move(edges)),
+                                  torch::autograd::deleteNode);
+    for (Tensor& t : out)
+      if (t.defined()) {
+        t = t.detach();
+        torch::autograd::set_history(t, refusal);
+      }
+    return out;
   }
 };
 

@@ -12,7 +12,7 @@ enum { O_U, O_DT, O_X, O_XB, O_B, O_C, O_D, O_Z, O_INPUTS };
 struct OperatorNode : SavingNode {
   int b, d, n, l;
   std::string name() const override { return "AussmOperatorBackward"; }
-  variable_list apply(variable_list&& g) override;
+  variable_list gradients(const variable_list& g) override;
 };
 
 aussm_operator_args arguments(const Tensor& u, const Tensor& dt, const Tensor& x, const Tensor& xb, const Tensor& B, const Tensor& C,
@@ -25,9 +25,7 @@ aussm_operator_args arguments(const Tensor& u, const Tensor& dt, const Tensor& x
   return p;
 }
 
-variable_list OperatorNode::apply(variable_list&& g) {
-  std::lock_guard<std::mutex> lock(mutex_);
-  at::NoGradGuard no_grad;
+variable_list OperatorNode::gradients(const variable_list& g) {
   variable_list out(O_INPUTS);
   if (!g[0].defined()) return out;
   Tensor t[10];

@@ -97,14 +97,12 @@ struct UnitaryNode : SavingNode {
   bool bc_complex;
   bool filled;                   // the forward call left what the backward kernel wants in `aux`
   std::string name() const override { return "AussmUnitaryScanBackward"; }
-  variable_list apply(variable_list&& g) override;
+  variable_list gradients(const variable_list& g) override;
 };
 
 enum { U_U, U_DELTA, U_THETA, U_B, U_C, U_D, U_Z, U_H0, U_INPUTS };
 
-variable_list UnitaryNode::apply(variable_list&& g) {
-  std::lock_guard<std::mutex> lock(mutex_);
-  at::NoGradGuard no_grad;
+variable_list UnitaryNode::gradients(const variable_list& g) {
   variable_list out(U_INPUTS);
   if (!g[0].defined() && !(g.size() > 1 && g[1].defined())) return out;
   const Tensor u = saved[0].unpack(), delta = saved[1].unpack(), theta = saved[2].unpack(), B = saved[3].unpack(),
@@ -237,14 +235,12 @@ struct ComplexNode : SavingNode {
   int b, d, n, l, dt;
   bool bc_complex;
   std::string name() const override { return "AussmComplexScanBackward"; }
-  variable_list apply(variable_list&& g) override;
+  variable_list gradients(const variable_list& g) override;
 };
 
 enum { X_U, X_DELTA, X_RHO, X_THETA, X_B, X_C, X_D, X_H0, X_Z, X_INPUTS };
 
-variable_list ComplexNode::apply(variable_list&& g) {
-  std::lock_guard<std::mutex> lock(mutex_);
-  at::NoGradGuard no_grad;
+variable_list ComplexNode::gradients(const variable_list& g) {
   variable_list out(X_INPUTS);
   if (!g[0].defined() && !(g.size() > 1 && g[1].defined())) return out;
   const Tensor u = saved[0].unpack(), delta = saved[1].unpack(), rho = saved[2].unpack(), theta = saved[3].unpack(),
@@ -335,14 +331,12 @@ namespace {
 struct RealNode : SavingNode {
   int b, d, n, l, dt, softplus;
   std::string name() const override { return "AussmSelectiveScanBackward"; }
-  variable_list apply(variable_list&& g) override;
+  variable_list gradients(const variable_list& g) override;
 };
 
 enum { R_U, R_DELTA, R_A, R_B, R_C, R_D, R_BIAS, R_H0, R_Z, R_INPUTS };
 
-variable_list RealNode::apply(variable_list&& g) {
-  std::lock_guard<std::mutex> lock(mutex_);
-  at::NoGradGuard no_grad;
+variable_list RealNode::gradients(const variable_list& g) {
   variable_list out(R_INPUTS);
   if (!g[0].defined() && !(g.size() > 1 && g[1].defined())) return out;
   const Tensor u = saved[0].unpack(), delta = saved[1].unpack(), A = saved[2].unpack(), B = saved[3].unpack(), C = saved[4].unpack(),

@@ -155,12 +155,13 @@ class _ScanFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *grads):
+        record = torch.is_grad_enabled()                 # create_graph: the gradients refuse to be differentiated
         with torch.enable_grad():
-            leaves = [None if t is None else t.detach().requires_grad_(need)
+            leaves = [t if t is None else t.view_as(t) if record and need else t.detach().requires_grad_(need)
                       for t, need in zip(ctx.saved_tensors, ctx.needs_input_grad[2:])]
             out = ctx.call(*leaves, *ctx.args)
             wanted = [t for t in leaves if t is not None and t.requires_grad]
-            got = iter(torch.autograd.grad(out, wanted, grads, allow_unused=True))
+            got = iter(torch.autograd.grad(out, wanted, grads, allow_unused=True, create_graph=record))
         return (None, None, *(next(got) if t is not None and t.requires_grad else None for t in leaves))
 
 

@@ -1,0 +1,168 @@
+"""What callers do with the graph behind a scan, a block or a linear layer: second derivatives, graphs kept or recomputed,
+hooks on what is saved, frozen parameters, gradients and states changed in place."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _scan_inputs(kind, b=2, d=8, n=8, l=64, seed=0, dtype=torch.float32):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    u, delta = rn(b, d, l), torch.nn.functional.softplus(rn(b, d, l))
+    if kind == "s6":
+        t = [u, delta, -torch.exp(rn(d, n)), rn(b, n, l), rn(b, n, l), rn(d)]
+    else:
+        t = [u, delta, *([-delta] if kind == "complex" else []), rn(b, d, l) * 0.5, torch.complex(rn(b, n, l), rn(b, n, l)),
+             torch.complex(rn(b, n, l), rn(b, n, l)), rn(d)]
+    return [v.clone().requires_grad_(True) for v in t]
+
+
+def _scan(kind):
+    from aussm_amd import scan
+    return {"unitary": scan.unitary_scan, "complex": scan.complex_scan, "s6": scan.selective_scan_fn}[kind]
+
+
+def _model(layers="a|m", d=24, **kw):
+    from aussm_amd import blocks
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        net = blocks.SSMTS(d_model=d, input_dim=5, output_dim=3, layers=layers, d_state=4, **kw)
+    with torch.no_grad():
+        for p in net.parameters():
+            p.add_(0.05 * torch.randn_like(p))
+    return net
+
+
+def _both_routes(monkeypatch, fn):
+    """`fn()` on the native route and on the composed layers."""
+    from aussm_amd import blocks
+    got = fn()
+    with monkeypatch.context() as m:
+        m.setattr(blocks, "_native", lambda *a: False)
+        return got, fn()
+
+
+def _close(got, want, tol=2e-4):
+    for k, (a, w) in enumerate(zip(got, want)):
+        assert (a is None) == (w is None), k
+        if a is None:
+            continue
+        a, w = (torch.view_as_real(t) if t.is_complex() else t for t in (a.detach(), w.detach()))
+        scale = max(1e-3, float(w.abs().max()))
+        torch.testing.assert_close(a / scale, w / scale, atol=tol, rtol=tol, msg=lambda m, k=k: f"{k}: {m}")
+
+
+# ---- second derivatives -----------------------------------------------------------------------
+
+@pytest.mark.parametrize("target", ["norm_f.weight", "output.weight", "embedding.weight"])
+def test_penalty_on_the_gradient_of_an_outer_layer(target, monkeypatch):
+    """Gradient of loss + |d loss / d w|^2, the inner gradient recorded.  Behind the blocks the recorded gradient holds
+    their first derivatives only; the embedding's also passes their second ones, which are refused."""
+    print("case penalty", target, flush=True)
+    net = _model()
+    x, tgt = torch.randn(2, 33, 5, device="cuda"), torch.randn(2, 33, 3, device="cuda")
+    params = dict(net.named_parameters())
+
+    def step():
+        net.zero_grad(set_to_none=True)
+        loss = (net(x) - tgt).square().mean()
+        g, = torch.autograd.grad(loss, params[target], create_graph=True)
+        (loss + g.square().sum()).backward()
+        return [p.grad for p in params.values()]
+    if target == "embedding.weight":
+        with pytest.raises(RuntimeError, match="second derivatives"):
+            step()
+        return
+    got, want = _both_routes(monkeypatch, step)
+    _close(got, want)
+
+
+@pytest.mark.parametrize("kind", ["a", "m"])
+@pytest.mark.parametrize("residual", [False, True])
+def test_penalty_on_the_gradient_of_a_block_s_output_projection(kind, residual, monkeypatch):
+    from aussm_amd import blocks
+    print("case block penalty", kind, residual, flush=True)
+    torch.manual_seed(5)
+    args = blocks.ModelArgsSSMau(24, 4, bias=True) if kind == "a" else blocks.ModelArgsMamba(24, 4, bias=True)
+    net = (blocks.ResidualBlock(args) if residual else args.block(args)).cuda()
+    out = (net.mixer if residual else net).out_proj
+    x, dy = torch.randn(2, 40, 24, device="cuda"), torch.randn(2, 40, 24, device="cuda")
+
+    def step():
+        net.zero_grad(set_to_none=True)
+        xi = x.clone().requires_grad_(True)
+        loss = (net(xi) * dy).sum() / 80
+        g = torch.autograd.grad(loss, [out.weight, out.bias], create_graph=True)
+        (loss + sum(t.square().sum() for t in g)).backward()
+        return [xi.grad] + [p.grad for p in net.parameters()]
+    _close(*_both_routes(monkeypatch, step))
+
+
+@pytest.mark.parametrize("norm", [False, True])
+def test_linear_layer_is_twice_differentiable(norm):
+    """Against the same two layers in float64."""
+    from aussm_amd import blocks
+    print("case linear twice", norm, flush=True)
+    torch.manual_seed(1)
+    lin, rms = torch.nn.Linear(12, 7), blocks.RMSNorm(12)
+    x, v = torch.randn(3, 9, 12), torch.randn(3, 9, 7)
+
+    def step(dev, dt):
+        leaves = [t.detach().to(dev, dt).requires_grad_(True) for t in (x, rms.weight, lin.weight, lin.bias)]
+        if dt is torch.float32:
+            l2, r2 = torch.nn.Linear(12, 7).to(dev), blocks.RMSNorm(12).to(dev)
+            l2.weight, l2.bias, r2.weight = (torch.nn.Parameter(t.detach()) for t in (leaves[2], leaves[3], leaves[1]))
+            leaves[1:] = [r2.weight, l2.weight, l2.bias]
+            y = blocks._norm_linear(l2, leaves[0], r2 if norm else None)
+            assert y.grad_fn.name() == "AussmLinearBackward"
+        else:
+            h = leaves[0]
+            if norm:
+                h = h * torch.rsqrt(h.square().mean(-1, keepdim=True) + rms.eps) * leaves[1]
+            y = torch.nn.functional.linear(h, leaves[2], leaves[3])
+        used = leaves if norm else [leaves[0], *leaves[2:]]
+        g = torch.autograd.grad((y.tanh() * v.to(dev, dt)).sum(), used, create_graph=True)
+        return torch.autograd.grad(sum(t.square().sum() for t in g), used)
+    for a, w in zip(step("cuda", torch.float32), step("cpu", torch.float64)):
+        scale = float(w.abs().max())
+        torch.testing.assert_close(a.cpu().double() / scale, w / scale, atol=1e-5, rtol=1e-5)
+
+
+def test_one_tensor_as_two_inputs_of_a_block_counts_once(monkeypatch):
+    """Recorded gradients where two weights of a block are one tensor and the input depends on a third."""
+    from aussm_amd import blocks
+    torch.manual_seed(5)
+    net = blocks.SSMauBlock(blocks.ModelArgsSSMau(8, 8)).cuda()
+    net.dt_proj.weight = net.x_proj.weight = net.out_proj.weight        # 8 x 8, three times
+    x = torch.randn(2, 24, 8, device="cuda")
+
+    def step():
+        net.zero_grad(set_to_none=True)
+        xi = (x * net.D).tanh()
+        net(xi).square().mean().backward(create_graph=True)
+        return [p.grad.detach() for p in net.parameters()]
+    _close(*_both_routes(monkeypatch, step))
+
+
+@pytest.mark.parametrize("kind", ["unitary", "complex", "s6"])
+def test_recorded_gradients_of_a_scan_are_values_and_refuse_to_be_differentiated(kind):
+    print("case scan create_graph", kind, flush=True)
+    t = _scan_inputs(kind)
+    want = torch.autograd.grad(_scan(kind)(*t).square().sum(), t)
+    y = _scan(kind)(*t)
+    got = torch.autograd.grad(y.square().sum(), t, create_graph=True)
+    _close(got, want, 1e-6)
+    with pytest.raises(RuntimeError, match="second derivatives"):
+        torch.autograd.grad(got[1].square().sum(), t)
+
+
+def test_recorded_gradients_of_the_operator_refuse_to_be_differentiated():
+    from aussm_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    t = [v.requires_grad_(True) for v in (rn(2, 8, 40), rn(2, 8, 40).abs(), rn(8, 4, 8) * 0.3, rn(8, 4), torch.complex(rn(4), rn(4)),
+                                          torch.complex(rn(4), rn(4)), rn(8), rn(2, 8, 40))]
+    got = torch.autograd.grad(ops.ssm_adaptive_interface(*t).square().sum(), t, create_graph=True)
+    with pytest.raises(RuntimeError, match="second derivatives"):
+        torch.autograd.grad(got[0].square().sum(), t)
