@@ -174,6 +174,7 @@ std::pair<Tensor, Tensor> unitary_scan(const Tensor& u_, const Tensor& delta_, c
     const Tensor u = dense(u_), delta = dense(delta_);
     const int64_t bu = u.size(0), d = u.size(1), l = u.size(2);
     const int64_t b = theta_.dim() == 3 ? theta_.size(0) : bu;
+    if (u.numel() == 0) check(AUSSM_E_SHAPE, "unitary_scan");     // (before anything is divided by a size)
     if (b % bu != 0) fail("batch size of theta (", b, ") must be a multiple of that of u (", bu, ")");
     const Tensor theta = f32(theta_, "theta", {b, d, l});
     const Tensor B = complex_rows(Bc, "B", b, l, u.scalar_type()), C = complex_rows(Cc, "C", b, l, u.scalar_type());

@@ -66,3 +66,14 @@ def test_blocks_show_their_layers_to_a_dispatch_mode(kind):
             y = net(x)
     assert counter.get_total_flops() > 0
     torch.testing.assert_close(y, want, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("kind", ["unitary", "complex", "s6"])
+@pytest.mark.parametrize("empty", [{"b": 0}, {"d": 0}, {"l": 0}])
+@pytest.mark.parametrize("grad", [False, True])
+def test_empty_inputs_are_refused(kind, empty, grad):
+    """As an error, before any launch (an empty batch once divided by its size in the host code)."""
+    print("case empty", kind, empty, grad, flush=True)
+    t = [v.requires_grad_(grad) for v in _inputs(kind, **empty)]
+    with pytest.raises(RuntimeError, match="out of the supported range"):
+        _fn(kind)(*t)
