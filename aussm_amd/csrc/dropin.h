@@ -47,9 +47,23 @@ __device__ __forceinline__ float op_radius(const DropinArgs& p, const float* r, 
   return p.raw ? softplusf_(v) : v;
 }
 __device__ __forceinline__ float op_phase(const DropinArgs& p, const float* th, int j) { return th[(size_t)j * p.bcs]; }
-// derivative of the softplus behind dt, from dt itself: 1 - e^-dt (by its series where that would cancel)
+// Derivative of the softplus behind dt, from dt itself: 1 - e^-dt, below 1 by its Taylor series (the next term is below
+// 2^-28 of the value).  Measured through the gradient of dt's argument, the rounding of the product included: root mean
+// square of the relative error 4.0e-8 below 0.3, 4.5e-8 up to 1, 3.7e-8 from there on.  (The difference alone cancels:
+// 2.7e-7 for dt between 0.05 and 0.1.)
 __device__ __forceinline__ float dsoftplus_of(float dt) {
-  return dt < 0.05f ? dt * fmaf(-dt, fmaf(-dt, fmaf(dt, -0.041666668f, 0.16666667f), 0.5f), 1.0f) : 1.0f - __expf(-dt);
+  float p = 2.5052108e-8f;                             // 1 / 11!
+  p = fmaf(-dt, p, 2.7557319e-7f);
+  p = fmaf(-dt, p, 2.7557319e-6f);
+  p = fmaf(-dt, p, 2.4801587e-5f);
+  p = fmaf(-dt, p, 1.9841270e-4f);
+  p = fmaf(-dt, p, 1.3888889e-3f);
+  p = fmaf(-dt, p, 8.3333333e-3f);
+  p = fmaf(-dt, p, 4.1666667e-2f);
+  p = fmaf(-dt, p, 1.6666667e-1f);
+  p = fmaf(-dt, p, 0.5f);
+  p = fmaf(-dt, p, 1.0f);
+  return dt < 1.0f ? dt * p : 1.0f - __expf(-dt);
 }
 
 // ---- prefix / suffix sums along a row of 16 lanes
