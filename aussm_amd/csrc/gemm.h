@@ -32,6 +32,7 @@ typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 
 // split8<3> with the residuals taken by an unpack and a subtract instead of the dot instruction: the same pieces.  Beside
 // a busy matrix pipe the dot instruction costs more than the two (256 x 23040, K = 4096 382 us with it, 331 us without).
+// (Values that are not finite, or round to infinity in bf16, have no such pieces: xg_plain.)
 __device__ __forceinline__ void split8_sub(const float (&x)[8], u4 (&out)[3]) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -114,6 +115,37 @@ struct XgOperand {
     }
   }
 };
+
+// An infinity, and a finite value that rounds to one in bf16, leaves a NaN in its pieces (inf - inf) and in every sum that it
+// enters.  Sums that came out as an infinity or a NaN are formed again here from the values themselves, in fp32 steps: of a wavefront's slice `sw` (rows
+// mw .., columns nw ..) those of the steps of its slice of the sum.  A sum that has become a NaN ends early.
+// (The arguments are read again: kept in scalar registers across the main loop for this they cost every product.)
+template <bool TR, int TM, int TN, int WR, int WN, int LD>
+__device__ __forceinline__ void xg_plain(float* __restrict__ sw, int mw, int nw, int lane) {
+  typedef const __attribute__((address_space(4))) XGemmArgs* Args;
+  Args p = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  const int tiles = ((p->M + TM - 1) / TM) * ((p->N + TN - 1) / TN), sl = xcd_remap(blockIdx.x, gridDim.x) / tiles;
+  const int nk = (p->K + 31) / 32, steps = nk * p->Z, per = (steps + p->slices - 1) / p->slices;
+  const int s0 = sl * per, s1 = s0 + per < steps ? s0 + per : steps;
+#pragma unroll 1
+  for (int i = lane; i < WR * WN; i += 64) {
+    const int r = TR ? i % WR : i / WN, q = TR ? i / WR : i % WN, m = mw + r, n = nw + q;
+    float* const v = sw + (TR ? q * LD + r : r * LD + q);
+    if (m >= p->M || n >= p->N || *v * 0.0f == 0.0f) continue;
+    const int nb = n / p->nper;
+    const float* a = p->A + (long)m * p->sam;
+    const float* b = p->B + ((long)nb * p->sbb + (long)(n - nb * p->nper) * p->sbn);
+    float t = 0.0f;
+#pragma unroll 1
+    for (int s = s0; s < s1 && t == t; ++s) {
+      const int z = s / nk, k0 = (s - z * nk) * 32, k1 = min(k0 + 32, p->K);
+#pragma unroll 1
+      for (int k = k0; k < k1; ++k) t = fmaf(a[(long)z * p->saz + (long)k * p->sak], b[(long)z * p->sbz + (long)k * p->sbk], t);
+    }
+    *v = t;
+  }
+}
 
 // The results go through LDS to the memory: 64 registers written with fixed offsets, then rolled loops over the rows
 // along the contiguous index of C - 16 bytes a lane for whole, aligned tiles, else one element a lane (bounds, batch
@@ -251,10 +283,13 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 1 : 2) void xgemm_kernel(c
   // result tile (e, f), register a: row 16 e + 4 (lane / 16) + a, column 16 f + lane % 16 of the wavefront's block
   float* const sw = reinterpret_cast<float*>(s_mem) + wave * SLICE;
   const int c = lane & 15, g = lane >> 4;
+  float probe[2] = {0.0f, 0.0f};                            // a NaN if a result is one
 #pragma unroll
   for (int e = 0; e < EM; ++e)
 #pragma unroll
     for (int f = 0; f < EN; ++f) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) probe[a] = fmaf(acc[e][f][a], acc[e][f][a + 2], probe[a]);
       if constexpr (TR) *reinterpret_cast<f4*>(sw + (16 * f + c) * LD + 16 * e + 4 * g) = acc[e][f];
       else {
 #pragma unroll
@@ -262,8 +297,12 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 1 : 2) void xgemm_kernel(c
       }
     }
   __builtin_amdgcn_wave_barrier();                          // (a slice belongs to one wavefront)
-  const float* const add = p.add ? p.add : p.reduce ? p.C : nullptr;
   const int mw = m0 + 16 * wm, nw = n0 + 16 * wn;
+  if (__builtin_expect(__ballot(probe[0] + probe[1] != probe[0] + probe[1]) != 0, 0)) {
+    xg_plain<TR, TM, TN, WR, WN, LD>(sw, mw, nw, lane);
+    __builtin_amdgcn_wave_barrier();
+  }
+  const float* const add = p.add ? p.add : p.reduce ? p.C : nullptr;
   constexpr int ROWS = TR ? WN : WR, COLS = TR ? WR : WN;   // rows of the slice run along the contiguous index of C
   if (p.slices > 1) {                                       // uniform: summed into C (TR: one batch, nper = N)
     constexpr int RA = 64 / COLS;                           // lane = column (two rows at a time where 32 fill the row)

@@ -72,6 +72,44 @@ def test_products_on_small_tiles(b, l, i, o):
     test_products_of_a_linear_layer(b, l, i, o)
 
 
+# one step and one tile, partial tiles, small tiles, wide tiles of 96 and 128 columns, slices of a long sum
+@pytest.mark.parametrize("b,l,i,o", [(1, 1, 1, 1), (2, 129, 33, 65), (3, 133, 33, 17), (2, 96, 32, 300), (23, 721, 200, 130), (31, 1027, 256, 200),
+                                     (64, 256, 70, 300)])
+def test_products_of_values_that_are_not_finite(b, l, i, o):
+    """Infinities, NaN and finite values beyond bf16's largest in either operand: the same infinities and NaN as the sums in
+    float64, and the other results untouched (a huge term is one of 3.4e38 x 2^-10: no partial sum overflows)."""
+    print(f"case gemm not finite b={b} l={l} i={i} o={o}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(b + l)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    X, W, dY = rn(b, l, i), rn(o, i) * 2.0 ** -10, rn(b, o, l)
+    inf, nan, huge = float("inf"), float("nan"), 3.4e38
+    X[0, 0, 0], X[b - 1, l - 1, i - 1], X[0, l // 2, i // 2], X[0, l - 1, 0] = inf, -inf, nan, huge
+    X[b // 2, l // 3, 0], X[b // 2, l // 3, i - 1] = inf, -inf
+    dY[0, o // 2, l // 2], dY[b - 1, 0, 0] = inf, huge
+    W[o - 1, i - 1] = inf
+
+    def check(got, want):
+        want32 = want.float()
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(got.isinf() & (got > 0), want32.isinf() & (want32 > 0)) and torch.equal(got.isinf(), want32.isinf())
+        m = want32.isfinite()
+        if m.any():
+            # (huge terms, where they are, outweigh the rest of their sum)
+            assert float(((got.double() - want)[m].abs() / want[m].abs().clamp(min=1.0)).max()) < 1e-4
+
+    Y = torch.empty(b, o, l, device="cuda")
+    _gemm(W, X, Y, o, b * l, i, (i, 1), (1, i), (l, 1), nper=l, sbb=l * i, scb=o * l)
+    check(Y, (X.double().reshape(b * l, i) @ W.double().t()).reshape(b, l, o).transpose(1, 2))
+    dX = torch.empty(b, l, i, device="cuda")
+    Wt = W.t().contiguous()
+    _gemm(Wt, dY, dX, i, b * l, o, (o, 1), (l, 1), (1, i), nper=l, sbb=o * l, scb=l * i)
+    check(dX, (dY.double().transpose(1, 2).reshape(b * l, o) @ Wt.double().t()).reshape(b, l, i))
+    dW = torch.zeros(o, i, device="cuda")
+    X = X * 2.0 ** -10
+    _gemm(dY, X, dW, o, i, l, (l, 1), (i, 1), (i, 1), Z=b, saz=o * l, sbz=l * i, reduce=1)
+    check(dW, dY.double().transpose(0, 1).reshape(o, b * l) @ X.double().reshape(b * l, i))
+
+
 @pytest.mark.parametrize("B,D,L,K", [(1, 1, 1, 4), (2, 5, 3, 4), (3, 70, 130, 4), (2, 9, 2050, 4), (2, 8, 33, 3), (1, 4, 7, 8)])
 def test_convolution_of_channel_rows(B, D, L, K):
     from aussm_amd import _lib, scan
