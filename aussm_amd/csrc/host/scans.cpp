@@ -62,6 +62,11 @@ Tensor empty_grad(const Tensor& u, int64_t b, int64_t d, int64_t l, bool in_dtyp
   return at::empty({b, d, l}, at::TensorOptions().dtype(in_dtype ? u.scalar_type() : at::kFloat).device(u.device()));
 }
 
+// final state, complex: a tensor of its own (a view formed while gradients are not recorded could not be changed in place)
+Tensor empty_state(const Tensor& u, int64_t b, int64_t d, int64_t n) {
+  return at::empty({b, d, n}, at::TensorOptions().dtype(at::kComplexFloat).device(u.device()));
+}
+
 bool aligned16(std::initializer_list<const Tensor*> ts) {
   for (const Tensor* t : ts)
     if (t->defined() && (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15)) return false;
@@ -183,7 +188,7 @@ std::pair<Tensor, Tensor> unitary_scan(const Tensor& u_, const Tensor& delta_, c
     const Tensor D = f32(Dv, "D", {d}), z = f32(zv, "z", {b, d, l}), h0 = check_h0(hv, b, d, n);
     const int dt = in_dtype(u), urep = (int)(b / bu), ck = unitary_ck(b, d, n, l);
     y = empty_f32({b, d, l}, u);
-    if (want_state) hL = empty_f32({b, d, n, 2}, u);
+    if (want_state) hL = empty_state(u, b, d, n);
     const size_t aux_floats = aussm_unitary_aux_floats(b, d, n, l, ck);
     Tensor aux;
     if (needs_grad) {
@@ -219,7 +224,6 @@ std::pair<Tensor, Tensor> unitary_scan(const Tensor& u_, const Tensor& delta_, c
                                   ptr(aux), b, d, n, l, aux.defined() ? ck : TILE, dt, urep, cur_stream()),
             "aussm_unitary_fwd_aux");
     }
-    if (want_state) hL = at::view_as_complex(hL);
   }
   if (node) {
     torch::autograd::set_history(y, node);
@@ -303,7 +307,7 @@ std::pair<Tensor, Tensor> complex_scan(const Tensor& u_, const Tensor& delta_, c
       fail("the complex backward pass supports at most ", AUSSM_MAX_STATE, " states per channel");
     const int dt = in_dtype(u), ck = needs_grad ? REC_CK : TILE;
     y = empty_f32({b, d, l}, u);
-    if (want_state) hL = empty_f32({b, d, n, 2}, u);
+    if (want_state) hL = empty_state(u, b, d, n);
     const Tensor hck = needs_grad ? empty_f32({b, (l + ck - 1) / ck, n, 2, d}, u) : Tensor();
     const Tensor ws = workspace(VAR_COMPLEX, u, b, d, n, l, ck, dt);
     check(aussm_complex_fwd(ptr(u), ptr(delta), ptr(rho), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(z), ptr(h0), ptr(y), ptr(hL), ptr(hck),
@@ -316,7 +320,6 @@ std::pair<Tensor, Tensor> complex_scan(const Tensor& u_, const Tensor& delta_, c
       node->b = b; node->d = d; node->n = n; node->l = l; node->dt = dt;
       node->bc_complex = Bc.is_complex();
     }
-    if (want_state) hL = at::view_as_complex(hL);
   }
   if (node) {
     torch::autograd::set_history(y, node);

@@ -166,3 +166,28 @@ def test_recorded_gradients_of_the_operator_refuse_to_be_differentiated():
     got = torch.autograd.grad(ops.ssm_adaptive_interface(*t).square().sum(), t, create_graph=True)
     with pytest.raises(RuntimeError, match="second derivatives"):
         torch.autograd.grad(got[0].square().sum(), t)
+
+
+# ---- results changed in place -------------------------------------------------------------------
+
+@pytest.mark.parametrize("kind", ["unitary", "complex", "s6"])
+@pytest.mark.parametrize("gate", [False, True])
+def test_outputs_of_a_training_call_may_be_changed_in_place(kind, gate):
+    """A stream that resets the state of the requests that are done, between two calls of one graph."""
+    print("case in place", kind, gate, flush=True)
+    t = _scan_inputs(kind)
+    kw = {"z": torch.randn(2, 8, 64, device="cuda")} if gate else {}
+    done = torch.tensor([True, False], device="cuda")
+
+    def step(in_place):
+        y, h = _scan(kind)(*t, **kw, return_last_state=True)
+        if in_place:
+            h[done] = 0
+            h.mul_(0.5)
+            y.add_(1.0)
+        else:
+            h = torch.where(done[:, None, None], torch.zeros_like(h), h) * 0.5
+            y = y + 1.0
+        y2 = _scan(kind)(*t, **kw, h0=h)
+        return torch.autograd.grad(y.square().sum() + y2.square().sum(), t)
+    _close(step(True), step(False), 1e-5)
