@@ -104,11 +104,29 @@ def _swap(x: torch.Tensor) -> torch.Tensor:
 
 # ---- the native route -------------------------------------------------------------------------
 
-def _plain(module: nn.Module, cls) -> bool:
-    """A layer whose forward is exactly its class's: what it computes may be done without calling it."""
+_PLAIN_TYPES = (nn.Parameter, torch.Tensor, type(None))
+
+
+def _plain(module: nn.Module, cls, names=("weight", "bias")) -> bool:
+    """A layer whose forward is exactly its class's, on registered parameters `names` that are plain tensors: what it computes
+    may be done without calling it."""
     d = module.__dict__
-    return type(module) is cls and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-                                        or d["_backward_pre_hooks"]) and "forward" not in d
+    if type(module) is not cls or (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                                   or d["_backward_pre_hooks"]) or "forward" in d:
+        return False
+    p = d["_parameters"]
+    for k in names:
+        if k not in p or type(p[k]) not in _PLAIN_TYPES:
+            return False
+    return True
+
+
+def _plain_norm(norm: Optional[nn.Module]) -> bool:
+    return norm is None or _plain(norm, RMSNorm, ("weight",))
+
+
+def _plain_tensors(*ts: torch.Tensor) -> bool:
+    return all(type(t) in _PLAIN_TYPES for t in ts)
 
 
 def _native(x: torch.Tensor) -> bool:
@@ -123,7 +141,7 @@ def _native(x: torch.Tensor) -> bool:
 
 def _norm_linear(layer: nn.Linear, x: torch.Tensor, norm: Optional[nn.Module] = None) -> torch.Tensor:
     """`layer(norm(x))`."""
-    if _native(x) and _plain(layer, nn.Linear) and (norm is None or _plain(norm, RMSNorm)):
+    if _native(x) and _plain(layer, nn.Linear) and _plain_norm(norm):
         p = layer._parameters
         y = _lib.host().norm_linear(x, None if norm is None else norm.weight, 0.0 if norm is None else norm.eps,
                                     p["weight"], p["bias"])
@@ -205,7 +223,8 @@ class MambaBlock(nn.Module):
 
     def native(self, x: torch.Tensor, norm: Optional[nn.Module] = None, residual: bool = False) -> Optional[torch.Tensor]:
         """The block (behind `norm`, plus x with `residual`) on the native route, or None where that does not apply."""
-        if (self.scan_impl is not scan.selective_scan_fn or not _native(x) or (norm is not None and not _plain(norm, RMSNorm))):
+        if (self.scan_impl is not scan.selective_scan_fn or not _native(x) or not _plain_norm(norm)
+                or not _plain_tensors(self.A_log, self.D)):
             return None
         mods = self._modules
         ip, cv, op, xp, dp = (mods[k] for k in ("in_proj", "conv1d", "out_proj", "x_proj", "dt_proj"))
@@ -290,7 +309,7 @@ class SSMauBlock(nn.Module):
     def native(self, x: torch.Tensor, norm: Optional[nn.Module] = None, residual: bool = False) -> Optional[torch.Tensor]:
         """The block (behind `norm`, plus x with `residual`) on the native route, or None where that does not apply."""
         if (self._default_scan is None or self.optimized_SSMa_function is not self._default_scan or not self.args.conv_1d
-                or not _native(x) or (norm is not None and not _plain(norm, RMSNorm))):
+                or not _native(x) or not _plain_norm(norm) or not _plain_tensors(self.B, self.C, self.D)):
             return None
         mods = self._modules
         ip, cv, op, xp, dp, xa = (mods[k] for k in ("in_proj", "conv1d", "out_proj", "x_proj", "dt_proj", "xA_proj"))
@@ -354,7 +373,7 @@ class ResidualBlock(nn.Module):
 
     def forward(self, x):
         # norm, block and residual as one: the block itself must not be hooked either
-        if type(self.mixer) in (SSMauBlock, MambaBlock) and _plain(self.mixer, type(self.mixer)):
+        if type(self.mixer) in (SSMauBlock, MambaBlock) and _plain(self.mixer, type(self.mixer), ()):
             y = self.mixer.native(x, self.norm, True)
             if y is not None:
                 if type(self.mixer) is SSMauBlock:

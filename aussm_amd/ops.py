@@ -259,7 +259,8 @@ def ssm_adaptive_interface(u: Tensor, dt: Tensor, x: Tensor, x_bias: Tensor, B: 
     b, d, l = u.shape
     n = x.shape[1]
     if (l <= max_parallel_length and not save_intermediates and u.is_cuda and B.dtype is torch.complex64
-            and C.dtype is torch.complex64 and L.plain_call() and type(u) in (Tensor, torch.nn.Parameter)):
+            and C.dtype is torch.complex64 and L.plain_call()
+            and all(type(t) in (Tensor, torch.nn.Parameter) for t in (u, dt, x, x_bias, B, C, D, z))):
         # one launch sequence: the operator as one graph node, its softplus and zero start state inside the kernels
         host = L.host()
         if host.operator_supported(b, d, n, l):

@@ -197,3 +197,72 @@ def test_native_block_matches_the_composed_layers(kind, d, n, b, l, kw, residual
         a, w = (torch.view_as_real(t) if t.is_complex() else t for t in (a, w))
         scale = max(1e-3, float(w.abs().max()))
         torch.testing.assert_close(a / scale, w / scale, atol=1e-4, rtol=1e-4, msg=lambda m, k=name: f"{k}: {m}")
+
+
+# ---- calls that leave the native route ------------------------------------------------------------
+
+class _Marked(torch.Tensor):
+    """A tensor subclass that notes the functions it meets."""
+    seen = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(getattr(func, "__name__", str(func)))
+        return super().__torch_function__(func, types, args, kwargs)
+
+
+def _layer(net, path):
+    m = net
+    for k in path.split("."):
+        m = getattr(m, k)
+    return m
+
+
+BLOCKS = [("a", "mixer.in_proj"), ("a", "mixer.xA_proj"), ("a", "norm"), ("m", "mixer.x_proj"), ("m", "mixer.out_proj"),
+          ("m", "mixer.conv1d")]
+
+
+def _residual(kind):
+    from aussm_amd import blocks
+    torch.manual_seed(11)
+    args = blocks.ModelArgsSSMau(16, 4, bias=True) if kind == "a" else blocks.ModelArgsMamba(16, 4, bias=True)
+    return blocks.ResidualBlock(args).cuda()
+
+
+@pytest.mark.parametrize("kind,path", BLOCKS)
+@pytest.mark.parametrize("how", ["tensor", "subclass", "hook", "forward"])
+def test_replaced_and_hooked_layers(kind, path, how):
+    """A layer whose weight is no parameter of its own any more or is a subclass, or that is hooked or has another forward: the
+    block's result and the gradients of what it still has are those of the plain block."""
+    print("case replaced", kind, path, how, flush=True)
+    net, want = _residual(kind), _residual(kind)
+    layer, calls = _layer(net, path), []
+    w = layer.weight
+    if how == "tensor":
+        del layer.weight
+        layer.weight = w.detach().clone().requires_grad_(True)
+    elif how == "subclass":
+        layer.weight = torch.nn.Parameter(w.detach().clone().as_subclass(_Marked))
+    elif how == "hook":
+        layer.register_forward_hook(lambda m, a, y: calls.append(1))
+    else:
+        old = layer.forward
+        layer.forward = lambda x: (calls.append(1), old(x))[1]
+    x, dy = torch.randn(2, 24, 16, device="cuda"), torch.randn(2, 24, 16, device="cuda")
+    res = []
+    for m in (net, want):
+        xi = x.clone().requires_grad_(True)
+        if m is net:
+            _Marked.seen.clear()
+        y = m(xi)
+        if m is net:
+            assert bool(_Marked.seen) == (how == "subclass")
+        y.backward(dy)
+        res.append([y.detach(), xi.grad, _layer(m, path).weight.grad])
+    # (a GPU convolution and the weight of xA_proj are read by their block, not called: the block of composed layers either way)
+    if how == "hook" and not path.endswith(("conv1d", "xA_proj")):
+        assert calls
+    for a, b in zip(*res):
+        a, b = a.as_subclass(torch.Tensor), b.as_subclass(torch.Tensor)
+        scale = max(1e-3, float(b.abs().max()))
+        torch.testing.assert_close(a / scale, b / scale, atol=1e-4, rtol=1e-4)
