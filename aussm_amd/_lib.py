@@ -56,6 +56,7 @@ _SIGNATURES = {
     "aussm_gate_fwd": [_P] * 3 + [ctypes.c_size_t, _P],
     "aussm_gate_bwd": [_P] * 5 + [ctypes.c_size_t, _P],
     "aussm_operator_fwd": [_P] * 6,
+    "aussm_operator_fwd_keep": [_P] * 8,
     "aussm_operator_bwd": [_P] * 9,
     "aussm_gemm": [_P, _P],
     "aussm_conv_rows_fwd": [_P] * 4 + [_I] * 4 + [_LL, _P],

@@ -104,29 +104,22 @@ def _swap(x: torch.Tensor) -> torch.Tensor:
 
 # ---- the native route -------------------------------------------------------------------------
 
-_PLAIN_TYPES = (nn.Parameter, torch.Tensor, type(None))
+_PLAIN_TENSOR = frozenset((nn.Parameter, torch.Tensor))
+_PLAIN_BIAS = _PLAIN_TENSOR | {type(None)}
 
 
-def _plain(module: nn.Module, cls, names=("weight", "bias")) -> bool:
-    """A layer whose forward is exactly its class's, on registered parameters `names` that are plain tensors: what it computes
-    may be done without calling it."""
+def _unhooked(module: nn.Module, cls) -> bool:
     d = module.__dict__
-    if type(module) is not cls or (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-                                   or d["_backward_pre_hooks"]) or "forward" in d:
-        return False
-    p = d["_parameters"]
-    for k in names:
-        if k not in p or type(p[k]) not in _PLAIN_TYPES:
-            return False
-    return True
+    return type(module) is cls and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                                        or d["_backward_pre_hooks"]) and "forward" not in d
 
 
-def _plain_norm(norm: Optional[nn.Module]) -> bool:
-    return norm is None or _plain(norm, RMSNorm, ("weight",))
-
-
-def _plain_tensors(*ts: torch.Tensor) -> bool:
-    return all(type(t) in _PLAIN_TYPES for t in ts)
+def _plain(module: nn.Module, cls) -> bool:
+    """A layer whose forward is exactly its class's, on a registered weight (and bias, or None) that are plain tensors: what
+    it computes may be done without calling it."""
+    p = module.__dict__["_parameters"]
+    return (_unhooked(module, cls) and type(p.get("weight")) in _PLAIN_TENSOR
+            and (cls is RMSNorm or type(p.get("bias", 0)) in _PLAIN_BIAS))
 
 
 def _native(x: torch.Tensor) -> bool:
@@ -141,7 +134,7 @@ def _native(x: torch.Tensor) -> bool:
 
 def _norm_linear(layer: nn.Linear, x: torch.Tensor, norm: Optional[nn.Module] = None) -> torch.Tensor:
     """`layer(norm(x))`."""
-    if _native(x) and _plain(layer, nn.Linear) and _plain_norm(norm):
+    if _native(x) and _plain(layer, nn.Linear) and (norm is None or _plain(norm, RMSNorm)):
         p = layer._parameters
         y = _lib.host().norm_linear(x, None if norm is None else norm.weight, 0.0 if norm is None else norm.eps,
                                     p["weight"], p["bias"])
@@ -223,8 +216,8 @@ class MambaBlock(nn.Module):
 
     def native(self, x: torch.Tensor, norm: Optional[nn.Module] = None, residual: bool = False) -> Optional[torch.Tensor]:
         """The block (behind `norm`, plus x with `residual`) on the native route, or None where that does not apply."""
-        if (self.scan_impl is not scan.selective_scan_fn or not _native(x) or not _plain_norm(norm)
-                or not _plain_tensors(self.A_log, self.D)):
+        if (self.scan_impl is not scan.selective_scan_fn or not _native(x) or (norm is not None and not _plain(norm, RMSNorm))
+                or not (type(self.A_log) in _PLAIN_TENSOR and type(self.D) in _PLAIN_TENSOR)):
             return None
         mods = self._modules
         ip, cv, op, xp, dp = (mods[k] for k in ("in_proj", "conv1d", "out_proj", "x_proj", "dt_proj"))
@@ -296,20 +289,27 @@ class SSMauBlock(nn.Module):
 
     @property
     def ssm_args(self):
-        """What the last forward pass handed to the scan operator."""
-        if self._ssm_args is None and self._last_input is not None:
-            x, norm = self._last_input
-            x_and_z = _linear(self.in_proj, x if norm is None else norm(x))
-            x, z = x_and_z.split(self.args.d_model, dim=-1)
-            self._ssm_args = self._scan_args(_causal_conv(self.conv1d, x, x.shape[1]), z)
+        """What the last forward pass handed to the scan operator.  (From the native route: values outside the graph, put
+        together when they are asked for from what that pass left.)"""
+        if self._ssm_args is None:
+            if self._handed is None:
+                raise AttributeError("ssm_args")
+            u, dt, xz, x, x_bias, B, C, D = self._handed
+            self.ssm_args = {"u": u, "dt": dt, "x": x, "x_bias": x_bias, "B": B, "C": C, "D": D,
+                             "z": xz[:, u.shape[1]:].contiguous()}
         return self._ssm_args
 
-    _ssm_args = _last_input = None
+    @ssm_args.setter
+    def ssm_args(self, value):
+        self._ssm_args, self._handed = value, None
+
+    _ssm_args = _handed = None
 
     def native(self, x: torch.Tensor, norm: Optional[nn.Module] = None, residual: bool = False) -> Optional[torch.Tensor]:
         """The block (behind `norm`, plus x with `residual`) on the native route, or None where that does not apply."""
         if (self._default_scan is None or self.optimized_SSMa_function is not self._default_scan or not self.args.conv_1d
-                or not _native(x) or not _plain_norm(norm) or not _plain_tensors(self.B, self.C, self.D)):
+                or not _native(x) or (norm is not None and not _plain(norm, RMSNorm))
+                or not {type(self.B), type(self.C), type(self.D)} <= _PLAIN_TENSOR):
             return None
         mods = self._modules
         ip, cv, op, xp, dp, xa = (mods[k] for k in ("in_proj", "conv1d", "out_proj", "x_proj", "dt_proj", "xA_proj"))
@@ -318,16 +318,19 @@ class SSMauBlock(nn.Module):
                 or xa.bias is None or cv.padding[0] != cv.kernel_size[0] - 1:
             return None
         i, c, o, a = ip._parameters, cv._parameters, op._parameters, xa._parameters
-        return _lib.host().aussm_block(x, None if norm is None else norm.weight, 0.0 if norm is None else norm.eps, residual,
-                                       i["weight"], i["bias"], c["weight"], c["bias"], xp._parameters["weight"],
-                                       dp._parameters["weight"], dp._parameters["bias"], a["weight"], a["bias"], self.B, self.C,
-                                       self.D, o["weight"], o["bias"], 1 / math.sqrt(self.args.d_model))
+        B, C, D = self.B, self.C, self.D
+        out = _lib.host().aussm_block(x, None if norm is None else norm.weight, 0.0 if norm is None else norm.eps, residual,
+                                      i["weight"], i["bias"], c["weight"], c["bias"], xp._parameters["weight"],
+                                      dp._parameters["weight"], dp._parameters["bias"], a["weight"], a["bias"], B, C, D,
+                                      o["weight"], o["bias"], 1 / math.sqrt(self.args.d_model))
+        if out is None:
+            return None
+        self.__dict__.update(_ssm_args=None, _handed=(*out[1:], B, C, D))
+        return out[0]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         y = self.native(x)
         if y is not None:
-            # (the operator's arguments never exist as tensors of their own here: ssm_args forms them when asked)
-            self._ssm_args, self._last_input = None, (x, None)
             return y
         (b, l, d) = x.shape
         x_and_z = _linear(self.in_proj, x)
@@ -357,8 +360,8 @@ class SSMauBlock(nn.Module):
         }
 
     def ssm_au(self, x, z):
-        self._ssm_args, self._last_input = self._scan_args(x, z), None
-        y = self.optimized_SSMa_function(**self._ssm_args)
+        self.ssm_args = self._scan_args(x, z)
+        y = self.optimized_SSMa_function(**self.ssm_args)
         return _swap(y)
 
 
@@ -373,11 +376,9 @@ class ResidualBlock(nn.Module):
 
     def forward(self, x):
         # norm, block and residual as one: the block itself must not be hooked either
-        if type(self.mixer) in (SSMauBlock, MambaBlock) and _plain(self.mixer, type(self.mixer), ()):
+        if type(self.mixer) in (SSMauBlock, MambaBlock) and _unhooked(self.mixer, type(self.mixer)):
             y = self.mixer.native(x, self.norm, True)
             if y is not None:
-                if type(self.mixer) is SSMauBlock:
-                    self.mixer._ssm_args, self.mixer._last_input = None, (x, self.norm)
                 return y
         return self.mixer(self.norm(x)) + x
 

@@ -93,8 +93,10 @@ __device__ __forceinline__ float row_first(float v, int) { return dpp_perm<0x150
 
 // x (rows of d: (channel i, state j) at row i xsi + j xsj), times scale -> operand records.  Record (v = i nb + sb, ks, piece, lane = (row = lane % 16, g = lane / 16))
 // holds x[i, 16 sb + row, 32 ks + 8 g .. + 7] (zero past the ends).  One thread per (v, ks, lane).
+// x_out [d, n, d], xb_out [d, n] (or null): scale x and x_bias in the operator's own order, for a caller that keeps them.
 __global__ __launch_bounds__(256) void dropin_xprep_kernel(const float* __restrict__ x, u4* __restrict__ xp, int d, int n, int ks, int nb,
-                                                           int xsi, int xsj, float scale) {
+                                                           int xsi, int xsj, float scale, const float* __restrict__ x_bias,
+                                                           float* __restrict__ x_out, float* __restrict__ xb_out) {
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (size_t)d * nb * ks * 64) return;
   const int lane = (int)(idx & 63);
@@ -107,6 +109,19 @@ __global__ __launch_bounds__(256) void dropin_xprep_kernel(const float* __restri
     const int r = 32 * k + 8 * g + q;
     v[q] = (j < n && r < d) ? x[((size_t)i * xsi + (size_t)j * xsj) * d + r] * scale : 0.0f;
   }
+  const int r0 = 32 * k + 8 * g;
+  if (x_out && j < n) {
+    float* const o = x_out + ((size_t)i * n + j) * d + r0;
+    if (r0 + 8 <= d) {
+      *reinterpret_cast<f4u*>(o) = f4u{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<f4u*>(o + 4) = f4u{v[4], v[5], v[6], v[7]};
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (r0 + q < d) o[q] = v[q];
+    }
+  }
+  if (xb_out && j < n && k == 0 && g == 0) xb_out[(size_t)i * n + j] = x_bias[(size_t)i * xsi + (size_t)j * xsj];
   u4 pc[3];
   split8<3>(sk, v, pc);
 #pragma unroll

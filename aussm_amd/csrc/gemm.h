@@ -24,10 +24,6 @@ namespace aussm {
 // neighbouring lanes = 16 rows of one g) both free of bank conflicts.
 __device__ __forceinline__ int xg_slot(int r, int g) { return 16 * g + ((r + 4 * g) & 15); }
 
-// 16-byte loads that are only known to be 4-byte aligned (rows start anywhere when the row length is not a
-// multiple of four): the memory pipeline takes them, the type tells the compiler so
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 
 // split8<3> with the residuals taken by an unpack and a subtract instead of the dot instruction: the same pieces.  Beside

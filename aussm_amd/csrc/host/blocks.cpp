@@ -266,9 +266,10 @@ variable_list AussmBlockNode::recorded(variable_list&& g) {
 
 }  // namespace
 
-OptTensor aussm_block(const Tensor& x_, const OptTensor& nw_, double eps, bool residual, const Tensor& W_in, const OptTensor& b_in, const Tensor& cw,
-                      const OptTensor& cb, const Tensor& W_xp, const Tensor& W_dt, const Tensor& b_dt, const Tensor& xA_w, const Tensor& xA_b,
-                      const Tensor& B, const Tensor& C, const Tensor& D, const Tensor& W_out, const OptTensor& b_out, double scale) {
+std::optional<AussmBlockResult> aussm_block(const Tensor& x_, const OptTensor& nw_, double eps, bool residual, const Tensor& W_in,
+                                            const OptTensor& b_in, const Tensor& cw, const OptTensor& cb, const Tensor& W_xp, const Tensor& W_dt,
+                                            const Tensor& b_dt, const Tensor& xA_w, const Tensor& xA_b, const Tensor& B, const Tensor& C,
+                                            const Tensor& D, const Tensor& W_out, const OptTensor& b_out, double scale) {
   const Tensor raw[A_INPUTS] = {x_, opt(nw_), W_in, opt(b_in), cw, opt(cb), W_xp, W_dt, b_dt, xA_w, xA_b, B, C, D, W_out, opt(b_out)};
   BlockDims s{};
   if (!front_ok(x_, raw[A_NW], nw_.has_value(), W_in, raw[A_BIN], cw, raw[A_CB], W_out, raw[A_BOUT], s) || !same_device(x_, raw)) return std::nullopt;
@@ -283,7 +284,7 @@ OptTensor aussm_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
   bool needs_grad = false;
   if (at::GradMode::is_enabled())
     for (const Tensor& t : raw) needs_grad = needs_grad || wants_grad(t);
-  Tensor out;
+  AussmBlockResult res;
   std::shared_ptr<AussmBlockNode> node;
   {
     at::NoGradGuard no_grad;
@@ -299,9 +300,13 @@ OptTensor aussm_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
     {
       const Tensor ws = empty_f32({(int64_t)aussm_ssm_adaptive_unitary_workspace_floats(s.b, e, n, s.l, 0)}, x);
       const aussm_operator_args p = block_operator(s, n, (float)scale, f.u, dt, in, f.xz);
-      check(aussm_operator_fwd(&p, ptr(y), ptr(nh_re), ptr(nh_im), ptr(ws), cur_stream()), "aussm_operator_fwd");
+      res.x = empty_f32({e, n, e}, x);
+      res.x_bias = empty_f32({e, n}, x);
+      check(aussm_operator_fwd_keep(&p, ptr(y), ptr(nh_re), ptr(nh_im), ptr(ws), ptr(res.x), ptr(res.x_bias), cur_stream()),
+            "aussm_operator_fwd_keep");
     }
-    out = back_projection(s, y, in[A_WOUT], in[A_BOUT], x);
+    res.u = f.u; res.dt = dt; res.xz = f.xz;
+    res.out = back_projection(s, y, in[A_WOUT], in[A_BOUT], x);
     if (needs_grad) {
       node = make_node<AussmBlockNode>();
       node->set_next_edges(torch::autograd::collect_next_edges(raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9],
@@ -311,8 +316,8 @@ OptTensor aussm_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
       node->s = s; node->n = n; node->r = r; node->scale = (float)scale;
     }
   }
-  if (node) torch::autograd::set_history(out, node);
-  return out;
+  if (node) torch::autograd::set_history(res.out, node);
+  return res;
 }
 
 // ============================================================================ Mamba block

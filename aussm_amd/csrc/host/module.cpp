@@ -49,7 +49,14 @@ PYBIND11_MODULE(_aussm_host, m) {
   });
   m.def("operator_supported", &operator_supported);
   m.def("adaptive_operator", &adaptive_operator);
-  m.def("aussm_block", &aussm_block);
+  m.def("aussm_block", [](const Tensor& x, const OptTensor& nw, double eps, bool residual, const Tensor& W_in, const OptTensor& b_in,
+                          const Tensor& cw, const OptTensor& cb, const Tensor& W_xp, const Tensor& W_dt, const Tensor& b_dt, const Tensor& xA_w,
+                          const Tensor& xA_b, const Tensor& B, const Tensor& C, const Tensor& D, const Tensor& W_out, const OptTensor& b_out,
+                          double scale) -> py::object {
+    const auto r = aussm_block(x, nw, eps, residual, W_in, b_in, cw, cb, W_xp, W_dt, b_dt, xA_w, xA_b, B, C, D, W_out, b_out, scale);
+    if (!r) return py::none();
+    return py::make_tuple(r->out, r->u, r->dt, r->xz, r->x, r->x_bias);
+  });
   m.def("mamba_block", &mamba_block);
   m.def("norm_linear", &norm_linear);
 }

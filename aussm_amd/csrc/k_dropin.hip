@@ -4,10 +4,11 @@
 
 namespace aussm {
 
-int run_dropin_xprep(const float* x, u4* xp, int d, int n, int ks, int nb, int xsi, int xsj, float scale, hipStream_t s) {
+int run_dropin_xprep(const float* x, u4* xp, int d, int n, int ks, int nb, int xsi, int xsj, float scale, const float* x_bias, float* x_out,
+                     float* xb_out, hipStream_t s) {
   const size_t total = (size_t)d * nb * ks * 64;
   hipLaunchKernelGGL(dropin_xprep_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, x, xp, d, n, ks, nb, xsi, xsj,
-                     scale);
+                     scale, x_bias, x_out, xb_out);
   return launch_status();
 }
 

@@ -901,6 +901,10 @@ static DropinArgs dropin_args(const aussm_operator_args& p) {
 }
 
 int aussm_operator_fwd(const aussm_operator_args* op, float* y, float* nh_re, float* nh_im, float* workspace, void* stream) {
+  return aussm_operator_fwd_keep(op, y, nh_re, nh_im, workspace, nullptr, nullptr, stream);
+}
+int aussm_operator_fwd_keep(const aussm_operator_args* op, float* y, float* nh_re, float* nh_im, float* workspace, float* x_out, float* x_bias_out,
+                            void* stream) {
   if (int e = operator_check(op)) return e;
   if (!y || !nh_re || !nh_im || !workspace) return AUSSM_E_NULL;
   if (misaligned(workspace, 16)) return AUSSM_E_ALIGN;
@@ -910,7 +914,7 @@ int aussm_operator_fwd(const aussm_operator_args* op, float* y, float* nh_re, fl
   DropinArgs a = dropin_args(*op);
   u4* xp = (u4*)workspace;
   u4* up = (u4*)(workspace + dropin_xp_floats(d, n));
-  if (int e = run_dropin_xprep(op->x, xp, d, n, a.ks, a.nb, a.xsi, a.xsj, op->x_scale, s)) return e;
+  if (int e = run_dropin_xprep(op->x, xp, d, n, a.ks, a.nb, a.xsi, a.xsj, op->x_scale, op->x_bias, x_out, x_bias_out, s)) return e;
   a.y = y; a.nh_re = nh_re; a.nh_im = nh_im; a.xp = xp; a.up = up; a.b = b;
   // the sequence in chunks of ct tiles (one chunk unless it is long): prepared tiles of u for the chunk, then the
   // scan over it, the state handed from chunk to chunk in the output buffers
@@ -954,7 +958,7 @@ int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const
   u4* up = (u4*)(dth + (size_t)blk.bg * ct * DT * d * n);
   DropinArgs f = dropin_args(*op);
   f.xp = xp; f.up = up;
-  if (int e = run_dropin_xprep(op->x, xp, d, n, f.ks, f.nb, f.xsi, f.xsj, op->x_scale, s)) return e;
+  if (int e = run_dropin_xprep(op->x, xp, d, n, f.ks, f.nb, f.xsi, f.xsj, op->x_scale, nullptr, nullptr, nullptr, s)) return e;
   FillArgs fa{};
   auto fill = [&](float* dst, const float* src, size_t cnt) {
     fa.dst[fa.count] = dst; fa.src[fa.count] = src; fa.n[fa.count] = cnt; ++fa.count;

@@ -350,6 +350,10 @@ typedef struct aussm_operator_grads {
   float *u, *dt, *x, *x_bias, *B_r, *B_theta, *C_r, *C_theta, *D, *z, *h_re, *h_im, *dt_bias;
 } aussm_operator_grads;
 int aussm_operator_fwd(const aussm_operator_args* op, float* y, float* nh_re, float* nh_im, float* workspace, void* stream);
+/* ... and leaves x_scale x [d, n, d] and x_bias [d, n] in the operator's own order in x_out and x_bias_out (each may be
+ * NULL): a record of the call that later changes of the weights do not reach, written by a launch that reads x anyway. */
+int aussm_operator_fwd_keep(const aussm_operator_args* op, float* y, float* nh_re, float* nh_im, float* workspace, float* x_out,
+                            float* x_bias_out, void* stream);
 int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const float* grad_nh_re, const float* grad_nh_im,
                        const float* nh_re, const float* nh_im, const aussm_operator_grads* grads, float* workspace, void* stream);
 

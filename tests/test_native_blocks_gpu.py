@@ -266,3 +266,34 @@ def test_replaced_and_hooked_layers(kind, path, how):
         a, b = a.as_subclass(torch.Tensor), b.as_subclass(torch.Tensor)
         scale = max(1e-3, float(b.abs().max()))
         torch.testing.assert_close(a / scale, b / scale, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("d,n,l", [(8, 4, 33), (40, 20, 70), (33, 40, 17)])
+def test_arguments_handed_to_the_operator(d, n, l, monkeypatch):
+    """ssm_args is what the last forward pass handed on: also after the weights have changed, and what is assigned to it."""
+    from aussm_amd import blocks
+    print("case ssm_args", d, n, l, flush=True)
+    torch.manual_seed(d)
+    net = blocks.SSMauBlock(blocks.ModelArgsSSMau(d, n)).cuda()
+    with pytest.raises(AttributeError):
+        net.ssm_args
+    x = torch.randn(2, l, d, device="cuda")
+    with monkeypatch.context() as m:
+        m.setattr(blocks, "_native", lambda *a: False)
+        net(x)
+        want = {k: v.detach().clone() for k, v in net.ssm_args.items()}
+    y = net(x)
+    assert y.grad_fn.name() == "AussmBlockBackward"
+    with torch.no_grad():
+        for k, p in net.named_parameters():
+            if k not in ("B", "C", "D"):                 # (those are handed on themselves)
+                p.add_(1.0)
+    got = net.ssm_args
+    assert got.keys() == want.keys() and got is net.ssm_args
+    for k in want:
+        assert got[k].shape == want[k].shape and got[k].dtype == want[k].dtype and got[k].is_contiguous()
+        torch.testing.assert_close(got[k].detach(), want[k], atol=1e-5, rtol=1e-5)
+    net.ssm_args = {"u": 1}
+    assert net.ssm_args == {"u": 1}
+    net(x)
+    assert net.ssm_args["u"].shape == (2, d, l)
