@@ -74,8 +74,7 @@ int run_xgemm(XGemmArgs a, hipStream_t s) {
   }
   if (steps > 0x7fffffffL || tiles * sl > 0x7fffffffL) return -2;
   a.slices = (int)sl;
-  // (offsets inside a tile of C are 32-bit)
-  if (a.scm < 0 || a.scn < 0 || a.scm >= (1l << 24) || a.scn >= (1l << 24)) return -2;
+  if (a.scm < 0 || a.scn < 0) return -2;
   const unsigned grid = (unsigned)(tiles * sl);
   return a.K % 4 == 0 ? launch_xgemm<true>(tile, a, grid, s) : launch_xgemm<false>(tile, a, grid, s);
 }

@@ -72,6 +72,26 @@ def test_products_on_small_tiles(b, l, i, o):
     test_products_of_a_linear_layer(b, l, i, o)
 
 
+@pytest.mark.parametrize("rows", [False, True])
+@pytest.mark.parametrize("reduce", [0, 1])
+def test_results_far_apart(rows, reduce):
+    """Rows or columns of C more than 2^24 elements apart, as the operator's gradients of a sequence that long are."""
+    print("case gemm far apart", rows, reduce, flush=True)
+    far, M, N, K = (1 << 24) + 20, 3, 40, 260
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    A, B = rn(M, K), rn(K, N)
+    C = torch.zeros(2 * far + N, device="cuda")
+    if rows:                                            # C(m, n) at m far + n
+        _gemm(A, B, C, M, N, K, (K, 1), (N, 1), (far, 1), reduce=reduce)
+        got = torch.stack([C[m * far:m * far + N] for m in range(M)])
+    else:                                               # the product's columns far apart: C^T = B^T A^T
+        _gemm(B.t().contiguous(), A.t().contiguous(), C, N, M, K, (K, 1), (M, 1), (1, far), reduce=reduce)
+        got = torch.stack([C[m * far:m * far + N] for m in range(M)])
+    assert _rel(got, A.double() @ B.double()) < 1e-6
+    assert int(torch.count_nonzero(C)) == M * N
+
+
 # one step and one tile, partial tiles, small tiles, wide tiles of 96 and 128 columns, slices of a long sum
 @pytest.mark.parametrize("b,l,i,o", [(1, 1, 1, 1), (2, 129, 33, 65), (3, 133, 33, 17), (2, 96, 32, 300), (23, 721, 200, 130), (31, 1027, 256, 200),
                                      (64, 256, 70, 300)])
