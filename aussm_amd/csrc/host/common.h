@@ -110,6 +110,12 @@ struct SavingNode : Node {
     saved.reserve(ts.size());
     for (const Tensor& t : ts) saved.emplace_back(t, false);
   }
+  // hooks stood between the forward pass and what `saved` hands out: it need not be what was saved, nor lie where it lay
+  bool hooked() const {
+    for (const auto& s : saved)
+      if (s.has_hooks()) return true;
+    return false;
+  }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
     for (auto& s : saved) s.reset_data();

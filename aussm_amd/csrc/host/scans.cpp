@@ -134,7 +134,7 @@ variable_list UnitaryNode::gradients(const variable_list& g) {
   Tensor dh0 = want_dh0 ? empty_f32({b, d, n, 2}, u) : Tensor();
   check(aussm_unitary_bwd_aux(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(hck), ptr(aux),
                               ptr<float>(du), ptr<float>(ddelta), ptr(dtheta), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), b, d, n, l, ck,
-                              dt | (g16 ? AUSSM_GRADS_IN_DTYPE : 0) | (filled && aligned16({&dy}) ? AUSSM_AUX_FILLED : 0),
+                              dt | (g16 ? AUSSM_GRADS_IN_DTYPE : 0) | (filled && !hooked() && aligned16({&dy}) ? AUSSM_AUX_FILLED : 0),
                               b / (int)u.size(0), cur_stream()),
         "aussm_unitary_bwd_aux");
   if (u.size(0) != b) {                          // u, delta shared by consecutive batch elements

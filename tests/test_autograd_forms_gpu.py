@@ -191,3 +191,70 @@ def test_outputs_of_a_training_call_may_be_changed_in_place(kind, gate):
         y2 = _scan(kind)(*t, **kw, h0=h)
         return torch.autograd.grad(y.square().sum() + y2.square().sum(), t)
     _close(step(True), step(False), 1e-5)
+
+
+# ---- what is saved between the passes -----------------------------------------------------------
+
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_hooks_that_round_what_the_scan_saves(gate, dtype):
+    """The scan's operand images are bf16 pairs in a float buffer: rounded by a hook they are no images any more, and the backward
+    pass forms its own.  The inputs survive the hook (they are bf16 values); the checkpoint and the ungated output are
+    rounded to 2^-9, the gradients follow within a few times that."""
+    from aussm_amd import scan
+    print("case rounding hooks", gate, dtype, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16().float()
+    b, d, n, l = 2, 64, 16, 256
+    t = [rn(b, d, l).to(dtype), rn(b, d, l).abs().to(dtype), rn(b, d, l), rn(b, n, l, 2).to(dtype), rn(b, n, l, 2).to(dtype), rn(d)]
+    if gate:
+        t.append(rn(b, d, l))
+    t = [v.requires_grad_(True) for v in t]
+    dy = rn(b, d, l)
+    want = torch.autograd.grad(scan.unitary_scan(*t), t, dy)
+    packed = []
+
+    def pack(v):
+        packed.append(v.numel())
+        return v.bfloat16().to(v.dtype)
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda v: v):
+        y = scan.unitary_scan(*t)
+    got = torch.autograd.grad(y, t, dy)
+    assert len(packed) >= 8
+    for k, (a, w) in enumerate(zip(got, want)):
+        rel = float((a.double() - w.double()).norm() / w.double().norm())
+        assert rel < 2e-2, (k, rel)
+
+
+@pytest.mark.parametrize("what", ["unitary", "complex", "s6", "a", "m", "linear"])
+@pytest.mark.parametrize("how", ["cpu", "checkpoint", "retain"])
+def test_saved_tensors_moved_recomputed_and_kept(what, how):
+    """save_on_cpu, activation checkpointing and a graph used twice: the gradients of a plain pass."""
+    from torch.utils.checkpoint import checkpoint
+    from aussm_amd import blocks
+    print("case saved", what, how, flush=True)
+    if what in ("unitary", "complex", "s6"):
+        t = _scan_inputs(what, d=64, n=16, l=256)
+        fn = lambda: _scan(what)(*t).square().sum()
+    else:
+        torch.manual_seed(2)
+        net = (torch.nn.Linear(24, 9) if what == "linear" else
+               (blocks.ModelArgsSSMau(24, 8) if what == "a" else blocks.ModelArgsMamba(24, 8)).block(
+                   blocks.ModelArgsSSMau(24, 8) if what == "a" else blocks.ModelArgsMamba(24, 8))).cuda()
+        x = torch.randn(2, 50, 24, device="cuda", requires_grad=True)
+        t = [x, *net.parameters()]
+        fn = lambda: (blocks._norm_linear(net, x) if what == "linear" else net(x)).square().sum()
+    want = torch.autograd.grad(fn(), t)
+    if how == "cpu":
+        with torch.autograd.graph.save_on_cpu():
+            y = fn()
+        got = torch.autograd.grad(y, t)
+    elif how == "checkpoint":
+        got = torch.autograd.grad(checkpoint(fn, use_reentrant=False), t)
+    else:
+        y = fn()
+        torch.autograd.grad(y, t, retain_graph=True)
+        got = torch.autograd.grad(y, t)
+        with pytest.raises(RuntimeError, match="second time"):
+            torch.autograd.grad(y, t)
+    _close(got, want, 1e-5)
