@@ -558,12 +558,20 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
   }
 }
 
-// Several small buffers set in one launch (blockIdx.y picks the buffer): dst[i] = src ? src[i] : 0.
+// Several buffers set in one launch (blockIdx.y picks the buffer), 16 bytes a lane where both sides allow it.
 __global__ __launch_bounds__(256) void fill_kernel(const FillArgs a) {
-  float* __restrict__ dst = a.dst[blockIdx.y];
-  const float* __restrict__ src = a.src[blockIdx.y];
-  const size_t n = a.n[blockIdx.y];
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = src ? src[i] : 0.0f;
+  const int i = blockIdx.y;
+  float* __restrict__ dst = a.dst[i];
+  const float* __restrict__ src = a.src[i];
+  const size_t at = (size_t)blockIdx.x * FILL_BLOCK, end = min((size_t)a.n[i], at + FILL_BLOCK);
+  const bool vec = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0;
+  for (size_t j = at + 4 * threadIdx.x; j < end; j += 1024) {
+    if (vec && j + 4 <= end) {
+      *reinterpret_cast<f4*>(dst + j) = src ? *reinterpret_cast<const f4*>(src + j) : f4{0, 0, 0, 0};
+    } else {
+      for (size_t k = j; k < end && k < j + 4; ++k) dst[k] = src ? src[k] : 0.0f;
+    }
+  }
 }
 
 }  // namespace aussm

@@ -60,11 +60,13 @@ struct DropinBwdArgs {
   float ddtb_scale;
 };
 
-// Up to 12 buffers set in one launch: dst[i] = src ? src[i] : 0 for i < n.
+// Up to FILL_MAX buffers set in one launch: dst[i] = src ? src[i] : 0 for i < n.
+constexpr int FILL_MAX = 16;
+constexpr int FILL_BLOCK = 4096;    // floats per workgroup
 struct FillArgs {
-  float* dst[12];
-  const float* src[12];
-  unsigned long long n[12];
+  float* dst[FILL_MAX];
+  const float* src[FILL_MAX];
+  unsigned long long n[FILL_MAX];
   int count;
 };
 

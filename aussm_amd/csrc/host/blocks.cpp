@@ -42,33 +42,6 @@ Gemm rows_from_rows_t(const float* W, const float* in, float* out, int64_t b, in
   return Gemm(o, b * l, i).A(W, 1, o).B(in, l, 1, in_rows * l).batch(l).C(out, l, 1, out_rows * l);
 }
 
-// ---- parameter gradients that the kernels accumulate into: one buffer, cleared by one launch ---------------
-struct Grads {
-  Tensor all;
-  std::vector<int64_t> at_;
-  int64_t total = 0;
-  int add(int64_t n) {
-    at_.push_back(total);
-    total += (n + 3) / 4 * 4;
-    return (int)at_.size() - 1;
-  }
-  // `also`: another buffer to clear with the same launch
-  void make(const Tensor& like, const Tensor& also = Tensor()) {
-    all = empty_f32({std::max<int64_t>(total, 4)}, like);
-    float* p[2] = {ptr(all), ptr(also)};
-    const size_t n[2] = {(size_t)all.numel(), also.defined() ? (size_t)also.numel() : 0};
-    check(aussm_zero_many(p, n, also.defined() ? 2 : 1, cur_stream()), "aussm_zero_many");
-  }
-  float* p(int i) const { return ptr(all) + at_[i]; }
-  Tensor view(int i, at::IntArrayRef shape) const {
-    std::vector<int64_t> st(shape.size());
-    int64_t s = 1;
-    for (size_t k = shape.size(); k-- > 0;) { st[k] = s; s *= shape[k]; }
-    return all.as_strided(shape, st, at_[i]);
-  }
-  Tensor like(int i, const Tensor& t) const { return view(i, t.sizes()); }
-};
-
 bool f32_cuda(const Tensor& t) { return t.defined() && t.is_cuda() && t.scalar_type() == at::kFloat; }
 bool f32_or_none(const Tensor& t) { return !t.defined() || f32_cuda(t); }
 
@@ -222,11 +195,12 @@ variable_list AussmBlockNode::gradients(const variable_list& g) {
   const Tensor dout = dense(g[0]);
   const int64_t b = s.b, l = s.l, e = s.e;
   auto need = [&](int i) { return in[i].defined() && task_should_compute_output(i); };
-  Grads acc;
-  int id[A_INPUTS];
-  for (int i : {A_NW, A_WIN, A_BIN, A_CW, A_CB, A_WXP, A_WDT, A_WOUT, A_BOUT}) id[i] = in[i].defined() ? acc.add(in[i].numel()) : -1;
-  acc.make(x);
-  auto gp = [&](int i) { return need(i) ? acc.p(id[i]) : nullptr; };
+  Cleared acc;
+  int id[A_INPUTS];            // (norm and convolution add to theirs in any case)
+  for (int i : {A_NW, A_WIN, A_BIN, A_CW, A_CB, A_WXP, A_WDT, A_WOUT, A_BOUT})
+    id[i] = need(i) || (in[i].defined() && (i == A_NW || i == A_CW)) ? acc.part(in[i].numel()) : -1;
+  acc.clear(x);
+  auto gp = [&](int i) { return id[i] < 0 ? nullptr : acc.data(id[i]); };
   Tensor dy = empty_f32({b, e, l}, x);
   out_grads(s, dout, y, in[A_WOUT], ptr(dy), gp(A_WOUT), gp(A_BOUT));
   // the operator
@@ -247,10 +221,10 @@ variable_list AussmBlockNode::gradients(const variable_list& g) {
   if (float* w = gp(A_WDT)) Gemm(e, r, l).A(ptr(ddt), l, 1, e * l).Bz(ptr(dt0), 1, l, r * l).C(w, r, 1).sum(b).run();
   rows_from_rows_t(ptr(in[A_WXP]), ptr(ddt0), ptr(du), b, l, r, e, r, e).add(ptr(du)).run();
   if (float* w = gp(A_WXP)) Gemm(r, e, l).A(ptr(ddt0), l, 1, r * l).Bz(ptr(u), 1, l, e * l).C(w, e, 1).sum(b).run();
-  out[A_X] = front_grads(s, x, xn, rstd, in[A_NW], xz, in[A_WIN], in[A_CW], du, dxz, dout, s.norm ? acc.p(id[A_NW]) : nullptr, gp(A_WIN),
-                         gp(A_BIN), acc.p(id[A_CW]), in[A_CB].defined() ? acc.p(id[A_CB]) : nullptr, need(A_X) || need(A_NW));
+  out[A_X] = front_grads(s, x, xn, rstd, in[A_NW], xz, in[A_WIN], in[A_CW], du, dxz, dout, gp(A_NW), gp(A_WIN), gp(A_BIN),
+                         gp(A_CW), gp(A_CB), need(A_X) || need(A_NW));
   for (int i : {A_NW, A_WIN, A_BIN, A_CW, A_CB, A_WXP, A_WDT, A_WOUT, A_BOUT})
-    if (need(i)) out[i] = acc.like(id[i], in[i]);
+    if (need(i)) out[i] = acc.view(id[i], in[i].sizes());
   return out;
 }
 
@@ -348,13 +322,13 @@ variable_list MambaBlockNode::gradients(const variable_list& g) {
   const Tensor dout = dense(g[0]);
   const int64_t b = s.b, l = s.l, e = s.e, R = r + 2 * n;
   auto need = [&](int i) { return in[i].defined() && task_should_compute_output(i); };
-  Grads acc;
-  int id[M_INPUTS];
-  for (int i : {M_NW, M_WIN, M_BIN, M_CW, M_CB, M_WXP, M_WDT, M_BDT, M_D, M_WOUT, M_BOUT}) id[i] = in[i].defined() ? acc.add(in[i].numel()) : -1;
-  const int iA = acc.add(e * n);
-  Tensor ddbc = empty_f32({b, R, l}, x);            // (the kernels add to its rows of B and C)
-  acc.make(x, ddbc);
-  auto gp = [&](int i) { return need(i) ? acc.p(id[i]) : nullptr; };
+  Cleared acc;
+  int id[M_INPUTS];            // (norm and convolution add to theirs in any case)
+  for (int i : {M_NW, M_WIN, M_BIN, M_CW, M_CB, M_WXP, M_WDT, M_BDT, M_ALOG, M_D, M_WOUT, M_BOUT})
+    id[i] = need(i) || (in[i].defined() && (i == M_NW || i == M_CW)) ? acc.part(in[i].numel()) : -1;
+  const Tensor ddbc = acc.own(x, {b, R, l});        // (the scan adds to its rows of B and C)
+  acc.clear(x);
+  auto gp = [&](int i) { return id[i] < 0 ? nullptr : acc.data(id[i]); };
   Tensor dy = empty_f32({b, e, l}, x);
   out_grads(s, dout, y, in[M_WOUT], ptr(dy), gp(M_WOUT), gp(M_BOUT));
   Tensor du = empty_f32({b, e, l}, x), ddt = empty_f32({b, e, l}, x), dxz = empty_f32({b, 2 * e, l}, x);
@@ -362,9 +336,9 @@ variable_list MambaBlockNode::gradients(const variable_list& g) {
     const size_t wf = aussm_scan_workspace_floats(2, b, e, n, l, CK, AUSSM_F32);
     const Tensor ws = wf ? empty_f32({(int64_t)wf}, x) : Tensor();
     aussm_real_rows rows{};
-    rows.z_rows = 2 * e; rows.bc_rows = R; rows.u_silu = 1; rows.ddelta_bias = acc.p(id[M_BDT]); rows.ddelta_bias_scale = 2.0f;
+    rows.z_rows = 2 * e; rows.bc_rows = R; rows.u_silu = 1; rows.ddelta_bias = gp(M_BDT); rows.ddelta_bias_scale = 2.0f;
     check(aussm_real_bwd_rows(ptr(dy), nullptr, ptr(u), ptr(dt), ptr(A), ptr(dbc) + r * l, ptr(dbc) + (r + n) * l, ptr(in[M_D]), ptr(in[M_BDT]), 1,
-                              nullptr, ptr(hck), ptr(du), ptr(ddt), acc.p(iA), ptr(ddbc) + r * l, ptr(ddbc) + (r + n) * l, acc.p(id[M_D]),
+                              nullptr, ptr(hck), ptr(du), ptr(ddt), gp(M_ALOG), ptr(ddbc) + r * l, ptr(ddbc) + (r + n) * l, gp(M_D),
                               nullptr, ptr(xz) + e * l, ptr(dxz) + e * l, ptr(ws), &rows, b, e, n, l, CK, AUSSM_F32, cur_stream()),
           "aussm_real_bwd_rows");
   }
@@ -373,13 +347,13 @@ variable_list MambaBlockNode::gradients(const variable_list& g) {
   if (float* w = gp(M_WDT)) Gemm(e, r, l).A(ptr(ddt), l, 1, e * l).Bz(ptr(dbc), 1, l, R * l).C(w, r, 1).sum(b).run();
   rows_from_rows_t(ptr(in[M_WXP]), ptr(ddbc), ptr(du), b, l, R, e, R, e).add(ptr(du)).run();
   if (float* w = gp(M_WXP)) Gemm(R, e, l).A(ptr(ddbc), l, 1, R * l).Bz(ptr(u), 1, l, e * l).C(w, e, 1).sum(b).run();
-  out[M_X] = front_grads(s, x, xn, rstd, in[M_NW], xz, in[M_WIN], in[M_CW], du, dxz, dout, s.norm ? acc.p(id[M_NW]) : nullptr, gp(M_WIN),
-                         gp(M_BIN), acc.p(id[M_CW]), in[M_CB].defined() ? acc.p(id[M_CB]) : nullptr, need(M_X) || need(M_NW));
+  out[M_X] = front_grads(s, x, xn, rstd, in[M_NW], xz, in[M_WIN], in[M_CW], du, dxz, dout, gp(M_NW), gp(M_WIN), gp(M_BIN),
+                         gp(M_CW), gp(M_CB), need(M_X) || need(M_NW));
   for (int i : {M_NW, M_WIN, M_BIN, M_CW, M_CB, M_WXP, M_WDT, M_BDT, M_D, M_WOUT, M_BOUT})
-    if (need(i)) out[i] = acc.like(id[i], in[i]);
+    if (need(i)) out[i] = acc.view(id[i], in[i].sizes());
   if (need(M_ALOG)) {
     out[M_ALOG] = empty_f32({e, n}, x);
-    check(aussm_neg_exp(ptr(in[M_ALOG]), acc.p(iA), ptr(out[M_ALOG]), e * n, cur_stream()), "aussm_neg_exp");
+    check(aussm_neg_exp(ptr(in[M_ALOG]), gp(M_ALOG), ptr(out[M_ALOG]), e * n, cur_stream()), "aussm_neg_exp");
   }
   return out;
 }
@@ -477,27 +451,28 @@ variable_list LinearNode::gradients(const variable_list& g) {
   const c10::DeviceGuard guard(x.device());
   const Tensor dy = dense(g[0]);
   auto need = [&](int k) { return in[k].defined() && task_should_compute_output(k); };
-  Grads acc;
-  const int iN = norm ? acc.add(i) : -1, iW = acc.add(o * i), iB = in[L_B].defined() ? acc.add(o) : -1;
-  if (norm || need(L_W) || need(L_B)) acc.make(x);
+  const bool below = need(L_X) || need(L_NW);
+  Cleared acc;
+  const int iN = norm && below ? acc.part(i) : -1, iW = need(L_W) ? acc.part(o * i) : -1, iB = need(L_B) ? acc.part(o) : -1;
+  acc.clear(x);
   if (need(L_W)) {
-    Gemm(o, i, rows).A(ptr(dy), 1, o).Bz(ptr(xn), i, 1, 0).C(acc.p(iW), i, 1).sum(1).run();
-    out[L_W] = acc.like(iW, in[L_W]);
+    Gemm(o, i, rows).A(ptr(dy), 1, o).Bz(ptr(xn), i, 1, 0).C(acc.data(iW), i, 1).sum(1).run();
+    out[L_W] = acc.view(iW, in[L_W].sizes());
   }
   if (need(L_B)) {
-    check(aussm_col_sum(ptr(dy), acc.p(iB), (size_t)rows, o, 1.0f, cur_stream()), "aussm_col_sum");
-    out[L_B] = acc.like(iB, in[L_B]);
+    check(aussm_col_sum(ptr(dy), acc.data(iB), (size_t)rows, o, 1.0f, cur_stream()), "aussm_col_sum");
+    out[L_B] = acc.view(iB, in[L_B].sizes());
   }
-  if (need(L_X) || need(L_NW)) {
+  if (below) {
     Tensor dxn = at::empty(x.sizes(), x.options());
     Gemm(i, rows, o).A(ptr(in[L_W]), 1, i).B(ptr(dy), 1, o).C(ptr(dxn), 1, i).run();
     out[L_X] = dxn;
     if (norm) {
       Tensor dx = at::empty(x.sizes(), x.options());
-      check(aussm_rms_norm_bwd(ptr(dxn), ptr(x), ptr(in[L_NW]), ptr(rstd), nullptr, ptr(dx), acc.p(iN), (size_t)rows, i, cur_stream()),
+      check(aussm_rms_norm_bwd(ptr(dxn), ptr(x), ptr(in[L_NW]), ptr(rstd), nullptr, ptr(dx), acc.data(iN), (size_t)rows, i, cur_stream()),
             "aussm_rms_norm_bwd");
       out[L_X] = dx;
-      if (need(L_NW)) out[L_NW] = acc.like(iN, in[L_NW]);
+      if (need(L_NW)) out[L_NW] = acc.view(iN, in[L_NW].sizes());
     }
   }
   return out;

@@ -102,6 +102,42 @@ inline void check_devices(const Tensor& ref, at::ArrayRef<Tensor> ts) {
     if (t.defined() && t.device() != ref.device()) fail("expected all tensors of the call on ", ref.device(), ", got one on ", t.device());
 }
 
+// Buffers that kernels add into, cleared by one launch: own() is an allocation of its own, part() a piece of one that the
+// parameter gradients of the call share (they are small and go together; a view takes half the time of an allocation).
+// What a caller keeps so holds no gradient of an activation's size but itself.
+struct Cleared {
+  std::vector<float*> p;
+  std::vector<size_t> n;
+  Tensor parts;
+  std::vector<int64_t> at;
+  int64_t total = 0;
+  void entry(const Tensor& t, int64_t floats) { p.push_back(ptr(t)); n.push_back((size_t)floats); }
+  Tensor own(const Tensor& like, at::IntArrayRef shape, at::ScalarType type = at::kFloat) {
+    const Tensor t = at::empty(shape, at::TensorOptions().dtype(type).device(like.device()));
+    entry(t, t.numel() * (type == at::kComplexFloat ? 2 : 1));
+    return t;
+  }
+  int part(int64_t floats) {
+    at.push_back(total);
+    total += (floats + 3) / 4 * 4;              // every part starts on 16 bytes
+    return (int)at.size() - 1;
+  }
+  void clear(const Tensor& like) {
+    if (total) {
+      parts = empty_f32({total}, like);
+      entry(parts, total);
+    }
+    if (!p.empty()) check(aussm_zero_many(p.data(), n.data(), (int)p.size(), cur_stream()), "aussm_zero_many");
+  }
+  float* data(int i) const { return ptr(parts) + at[i]; }
+  Tensor view(int i, at::IntArrayRef shape) const {
+    std::vector<int64_t> strides(shape.size());
+    int64_t s = 1;
+    for (size_t k = shape.size(); k-- > 0;) { strides[k] = s; s *= shape[k]; }
+    return parts.as_strided(shape, strides, at[i]);
+  }
+};
+
 // A graph node over saved tensors: `saved` are released together, and unpacking them after that raises torch's
 // usual error about a second backward pass.
 struct SavingNode : Node {

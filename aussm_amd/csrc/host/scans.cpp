@@ -46,12 +46,6 @@ Tensor check_h0(const Tensor& h0, int64_t b, int64_t d, int64_t n) {
   return dense(h0);
 }
 
-// gradient of a (b, n, l[, 2]) float buffer in the type and shape of the tensor it belongs to
-Tensor as_like(const Tensor& g, bool complex, at::ScalarType dtype) {
-  if (complex) return at::view_as_complex(g);
-  return g.scalar_type() == dtype ? g : g.to(dtype);
-}
-
 Tensor workspace(int variant, const Tensor& u, int b, int d, int n, int l, int ck, int dt) {
   const size_t f = aussm_scan_workspace_floats(variant, b, d, n, l, ck, dt);
   return f ? empty_f32({(int64_t)f}, u) : Tensor();
@@ -67,33 +61,18 @@ Tensor empty_state(const Tensor& u, int64_t b, int64_t d, int64_t n) {
   return at::empty({b, d, n}, at::TensorOptions().dtype(at::kComplexFloat).device(u.device()));
 }
 
+Tensor in_type(const Tensor& g, const Tensor& like) { return g.scalar_type() == like.scalar_type() ? g : g.to(like.scalar_type()); }
+
+// gradient rows of complex B / C that a kernel adds into: complex64 (b, n, l) or float (b, n, l, 2)
+Tensor add_rows(Cleared& acc, const Tensor& u, bool cplx, int64_t b, int64_t n, int64_t l) {
+  return cplx ? acc.own(u, {b, n, l}, at::kComplexFloat) : acc.own(u, {b, n, l, 2});
+}
+
 bool aligned16(std::initializer_list<const Tensor*> ts) {
   for (const Tensor* t : ts)
     if (t->defined() && (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15)) return false;
   return true;
 }
-
-// ---- buffers that the backward kernels accumulate into: one allocation and one clearing launch
-struct Acc {
-  Tensor all;
-  std::vector<int64_t> at_;
-  int64_t total = 0;
-  int add(int64_t n) {
-    at_.push_back(total);
-    total += (n + 3) / 4 * 4;                   // every part starts on 16 bytes
-    return (int)at_.size() - 1;
-  }
-  void make(const Tensor& like) {
-    all = empty_f32({total}, like);
-    check(aussm_zero_f32(ptr(all), (size_t)total, cur_stream()), "aussm_zero_f32");
-  }
-  Tensor part(int i, at::IntArrayRef shape) const {
-    std::vector<int64_t> strides(shape.size());
-    int64_t s = 1;
-    for (size_t k = shape.size(); k-- > 0;) { strides[k] = s; s *= shape[k]; }
-    return all.as_strided(shape, strides, at_[i]);
-  }
-};
 
 // ============================================================================ unitary
 
@@ -127,11 +106,10 @@ variable_list UnitaryNode::gradients(const variable_list& g) {
   Tensor du = empty_grad(u, b, d, l, g16), ddelta = empty_grad(u, b, d, l, g16), dtheta = empty_f32({b, d, l}, u);
   const bool want_dD = D.defined() && task_should_compute_output(U_D);
   const bool want_dh0 = task_should_compute_output(U_H0);
-  Acc acc;
-  const int iB = acc.add((int64_t)b * n * l * 2), iC = acc.add((int64_t)b * n * l * 2), iD = want_dD ? acc.add(d) : 0;
-  acc.make(u);
-  Tensor dB = acc.part(iB, {b, n, l, 2}), dC = acc.part(iC, {b, n, l, 2}), dD = want_dD ? acc.part(iD, {d}) : Tensor();
-  Tensor dh0 = want_dh0 ? empty_f32({b, d, n, 2}, u) : Tensor();
+  Cleared acc;
+  const Tensor dB = add_rows(acc, u, bc_complex, b, n, l), dC = add_rows(acc, u, bc_complex, b, n, l), dD = want_dD ? acc.own(u, {d}) : Tensor();
+  acc.clear(u);
+  const Tensor dh0 = want_dh0 ? empty_state(u, b, d, n) : Tensor();
   check(aussm_unitary_bwd_aux(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(hck), ptr(aux),
                               ptr<float>(du), ptr<float>(ddelta), ptr(dtheta), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), b, d, n, l, ck,
                               dt | (g16 ? AUSSM_GRADS_IN_DTYPE : 0) | (filled && !hooked() && aligned16({&dy}) ? AUSSM_AUX_FILLED : 0),
@@ -141,13 +119,13 @@ variable_list UnitaryNode::gradients(const variable_list& g) {
     du = du.view({u.size(0), -1, d, l}).sum(1);
     ddelta = ddelta.view({u.size(0), -1, d, l}).sum(1);
   }
-  out[U_U] = as_like(du, false, u.scalar_type());
-  out[U_DELTA] = as_like(ddelta, false, u.scalar_type());
+  out[U_U] = in_type(du, u);
+  out[U_DELTA] = in_type(ddelta, u);
   out[U_THETA] = dtheta;
-  out[U_B] = as_like(dB, bc_complex, u.scalar_type());
-  out[U_C] = as_like(dC, bc_complex, u.scalar_type());
+  out[U_B] = bc_complex ? dB : in_type(dB, u);
+  out[U_C] = bc_complex ? dC : in_type(dC, u);
   if (want_dD) out[U_D] = dD;
-  if (want_dh0) out[U_H0] = at::view_as_complex(dh0);
+  if (want_dh0) out[U_H0] = dh0;
   return out;
 }
 
@@ -259,24 +237,23 @@ variable_list ComplexNode::gradients(const variable_list& g) {
          dtheta = empty_f32({b, d, l}, u), dz = z.defined() ? empty_f32({b, d, l}, u) : Tensor();
   const bool want_dD = D.defined() && task_should_compute_output(X_D);
   const bool want_dh0 = h0.defined() && task_should_compute_output(X_H0);
-  Acc acc;
-  const int iB = acc.add((int64_t)b * n * l * 2), iC = acc.add((int64_t)b * n * l * 2), iD = want_dD ? acc.add(d) : 0;
-  acc.make(u);
-  Tensor dB = acc.part(iB, {b, n, l, 2}), dC = acc.part(iC, {b, n, l, 2}), dD = want_dD ? acc.part(iD, {d}) : Tensor();
-  Tensor dh0 = want_dh0 ? empty_f32({b, d, n, 2}, u) : Tensor();
+  Cleared acc;
+  const Tensor dB = add_rows(acc, u, bc_complex, b, n, l), dC = add_rows(acc, u, bc_complex, b, n, l), dD = want_dD ? acc.own(u, {d}) : Tensor();
+  acc.clear(u);
+  const Tensor dh0 = want_dh0 ? empty_state(u, b, d, n) : Tensor();
   const Tensor ws = workspace(VAR_COMPLEX, u, b, d, n, l, REC_CK, dt);
   check(aussm_complex_bwd(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(rho), ptr(theta), ptr(B), ptr(C), ptr(D), ptr(h0), ptr(hck),
                           ptr(du), ptr(ddelta), ptr(drho), ptr(dtheta), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), ptr(z), ptr(dz), ptr(ws),
                           b, d, n, l, REC_CK, dt | (g16 ? AUSSM_GRADS_IN_DTYPE : 0), cur_stream()),
         "aussm_complex_bwd");
-  out[X_U] = as_like(du, false, u.scalar_type());
-  out[X_DELTA] = as_like(ddelta, false, u.scalar_type());
+  out[X_U] = in_type(du, u);
+  out[X_DELTA] = in_type(ddelta, u);
   out[X_RHO] = drho;
   out[X_THETA] = dtheta;
-  out[X_B] = as_like(dB, bc_complex, u.scalar_type());
-  out[X_C] = as_like(dC, bc_complex, u.scalar_type());
+  out[X_B] = bc_complex ? dB : in_type(dB, u);
+  out[X_C] = bc_complex ? dC : in_type(dC, u);
   if (want_dD) out[X_D] = dD;
-  if (want_dh0) out[X_H0] = at::view_as_complex(dh0);
+  if (want_dh0) out[X_H0] = dh0;
   if (z.defined()) out[X_Z] = dz;
   return out;
 }
@@ -352,29 +329,29 @@ variable_list RealNode::gradients(const variable_list& g) {
   Tensor du = empty_grad(u, b, d, l, g16), ddelta = empty_grad(u, b, d, l, g16), dz = z.defined() ? empty_f32({b, d, l}, u) : Tensor();
   const bool want_dD = D.defined() && task_should_compute_output(R_D);
   const bool want_dh0 = h0.defined() && task_should_compute_output(R_H0);
-  Acc acc;
+  Cleared acc;
   const bool want_bias = bias.defined() && task_should_compute_output(R_BIAS);
-  const int iA = acc.add((int64_t)d * n), iB = acc.add((int64_t)b * n * l), iC = acc.add((int64_t)b * n * l), iD = want_dD ? acc.add(d) : 0,
-            iBias = want_bias ? acc.add(d) : 0;
-  acc.make(u);
-  Tensor dA = acc.part(iA, {d, n}), dB = acc.part(iB, {b, n, l}), dC = acc.part(iC, {b, n, l}), dD = want_dD ? acc.part(iD, {d}) : Tensor();
+  const int iA = acc.part((int64_t)d * n), iD = want_dD ? acc.part(d) : 0, iBias = want_bias ? acc.part(d) : 0;
+  const Tensor dB = acc.own(u, {b, n, l}), dC = acc.own(u, {b, n, l});
+  acc.clear(u);
+  const Tensor dA = acc.view(iA, {d, n}), dD = want_dD ? acc.view(iD, {d}) : Tensor(), dbias = want_bias ? acc.view(iBias, {d}) : Tensor();
   Tensor dh0 = want_dh0 ? empty_f32({b, d, n}, u) : Tensor();
   const Tensor ws = workspace(VAR_REAL, u, b, d, n, l, REC_CK, dt);
   aussm_real_rows rows{};
   if (want_bias) {
-    out[R_BIAS] = acc.part(iBias, {d});
-    rows.ddelta_bias = ptr(out[R_BIAS]);
+    out[R_BIAS] = dbias;
+    rows.ddelta_bias = ptr(dbias);
     rows.ddelta_bias_scale = 1.0f;
   }
   check(aussm_real_bwd_rows(ptr(dy), ptr(dhL), ptr(u), ptr(delta), ptr(A), ptr(B), ptr(C), ptr(D), ptr(bias), softplus, ptr(h0), ptr(hck),
                             ptr(du), ptr(ddelta), ptr(dA), ptr(dB), ptr(dC), ptr(dD), ptr(dh0), ptr(z), ptr(dz), ptr(ws), &rows, b, d, n, l,
                             REC_CK, dt | (g16 ? AUSSM_GRADS_IN_DTYPE : 0), cur_stream()),
         "aussm_real_bwd_rows");
-  out[R_U] = as_like(du, false, u.scalar_type());
-  out[R_DELTA] = as_like(ddelta, false, u.scalar_type());
+  out[R_U] = in_type(du, u);
+  out[R_DELTA] = in_type(ddelta, u);
   out[R_A] = dA;
-  out[R_B] = as_like(dB, false, u.scalar_type());
-  out[R_C] = as_like(dC, false, u.scalar_type());
+  out[R_B] = in_type(dB, u);
+  out[R_C] = in_type(dC, u);
   if (want_dD) out[R_D] = dD;
   if (want_dh0) out[R_H0] = dh0;
   if (z.defined()) out[R_Z] = dz;

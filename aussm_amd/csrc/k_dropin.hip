@@ -15,9 +15,9 @@ int run_dropin_xprep(const float* x, u4* xp, int d, int n, int ks, int nb, int x
 int run_fill(const FillArgs& a, hipStream_t s) {
   size_t most = 0;
   for (int i = 0; i < a.count; ++i) most = a.n[i] > most ? a.n[i] : most;
-  if (!a.count || !most) return 0;
-  size_t blocks = (most + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
+  const size_t blocks = (most + FILL_BLOCK - 1) / FILL_BLOCK;
+  if (blocks > 0x7fffffffULL) return -2;
+  if (!blocks) return 0;
   hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks, (unsigned)a.count), dim3(256), 0, s, a);
   return launch_status();
 }

@@ -145,13 +145,6 @@ int run_conv_bwd(const ConvArgs& a, hipStream_t s) {
   return launch_status();
 }
 
-int run_zero(float* p, size_t n, hipStream_t s) {
-  const size_t blocks = (n + 1023) / 1024;
-  hipLaunchKernelGGL(zero_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, s, p, n,
-                     (reinterpret_cast<uintptr_t>(p) & 15) == 0);
-  return launch_status();
-}
-
 int run_gate(const float* dy, const float* ypre, const float* z, float* out, float* dz, size_t n, hipStream_t s) {
   const size_t blocks = (n + 1023) / 1024;
   const dim3 grid((unsigned)(blocks < 8192 ? blocks : 8192));

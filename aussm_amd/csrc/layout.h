@@ -47,18 +47,6 @@ __global__ __launch_bounds__(256) void swap_last2_kernel(const SwapArgs p) {
   }
 }
 
-// n floats set to zero (vec: p is 16-byte aligned)
-__global__ __launch_bounds__(256) void zero_kernel(float* __restrict__ p, size_t n, int vec) {
-  const size_t stride = (size_t)gridDim.x * 256 * 4;
-  for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += stride) {
-    if (vec && i + 4 <= n) {
-      *reinterpret_cast<float4*>(p + i) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    } else {
-      for (size_t j = i; j < n && j < i + 4; ++j) p[j] = 0.0f;
-    }
-  }
-}
-
 // The scans' output gate  y = y_pre silu(z)  (extension-cpp/extension_cpp/ops.py:226) and its two gradients
 //     dy_pre = dy silu(z),   dz = dy y_pre silu'(z)
 // as one pass each over contiguous tensors of n floats (vec: all of them 16-byte aligned), for the scan

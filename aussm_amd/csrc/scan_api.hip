@@ -792,11 +792,12 @@ int aussm_neg_exp(const float* a_log, const float* dA, float* out, int n, void* 
 }
 int aussm_zero_many(float* const* p, const size_t* n, int count, void* stream) {
   if (!p || !n) return AUSSM_E_NULL;
-  if (count < 0 || count > 12) return AUSSM_E_SHAPE;
+  if (count < 0 || count > FILL_MAX) return AUSSM_E_SHAPE;
   FillArgs f{};
   for (int i = 0; i < count; ++i) {
     if (!n[i]) continue;
     if (!p[i]) return AUSSM_E_NULL;
+    if (misaligned(p[i], 4)) return AUSSM_E_ALIGN;
     f.dst[f.count] = p[i]; f.src[f.count] = nullptr; f.n[f.count] = n[i]; ++f.count;
   }
   return run_fill(f, (hipStream_t)stream);
@@ -805,7 +806,7 @@ int aussm_zero_many(float* const* p, const size_t* n, int count, void* stream) {
 int aussm_zero_f32(float* p, size_t n, void* stream) {
   if (!p) return AUSSM_E_NULL;
   if (misaligned(p, 4)) return AUSSM_E_ALIGN;
-  return n ? run_zero(p, n, (hipStream_t)stream) : AUSSM_OK;
+  return aussm_zero_many(&p, &n, 1, stream);
 }
 
 // ---- the reference's operator extension_cpp::ssm_adaptive_unitary as fused kernels (dropin.h)

@@ -387,7 +387,8 @@ int aussm_gemm(const aussm_gemm_args* args, void* stream);
  * res (optional) is added to dx; dw accumulated into.
  * Sums of columns / rows: out[c] += scale sum_r x[r, c];  out[r % d] += scale sum_l x[r, l].
  * aussm_neg_exp: dA NULL: out = -exp(a_log), else out = dA * -exp(a_log).
- * aussm_zero_many: up to 12 buffers set to zero with one launch.
+ * aussm_zero_many: up to 16 buffers set to zero with one launch (a kernel, not a memory-set node, so that a call may be
+ * recorded in a graph): the buffers that the backward calls add into.
  * ------------------------------------------------------------------------------------- */
 int aussm_conv_rows_fwd(const float* x, const float* w, const float* bias, float* y, int B, int D, int L, int K, long long xs_b, void* stream);
 int aussm_conv_rows_bwd(const float* dy, const float* x, const float* w, float* dx, float* dw, float* dbias, int B, int D, int L, int K,
@@ -423,8 +424,7 @@ int aussm_real_bwd_rows(const float* dy, const float* dhL,
                         float* dD, float* dh0, const float* z, float* dz, float* workspace, const aussm_real_rows* rows,
                         int B, int D, int N, int L, int ck, int in_dtype, void* stream);
 
-/* Sets n floats to zero with one launch (a kernel, not a memory-set node, so a call may be recorded in a graph):
- * the buffers that the backward calls above accumulate into. */
+/* aussm_zero_many of one buffer. */
 int aussm_zero_f32(float* p, size_t n, void* stream);
 
 /* ---------------------------------------------------------------------------------------

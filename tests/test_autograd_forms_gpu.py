@@ -258,3 +258,31 @@ def test_saved_tensors_moved_recomputed_and_kept(what, how):
         with pytest.raises(RuntimeError, match="second time"):
             torch.autograd.grad(y, t)
     _close(got, want, 1e-5)
+
+
+# ---- what a gradient keeps alive ------------------------------------------------------------------
+
+@pytest.mark.parametrize("what", ["unitary", "complex", "s6", "a", "m", "linear"])
+def test_a_gradient_holds_its_own_memory_only(what):
+    """Keeping D.grad, or any other one, keeps no gradient of an activation alive: those lie in allocations of their own, the
+    parameters' of one call at most in one with each other (parts padded to 16 bytes)."""
+    from aussm_amd import blocks
+    print("case memory of gradients", what, flush=True)
+    if what in ("unitary", "complex", "s6"):
+        t = _scan_inputs(what, d=33, n=5, l=100)
+        params = [v for v in t if v.shape[0] == 33]              # A, D
+        y = _scan(what)(*t)
+    else:
+        torch.manual_seed(2)
+        net = (torch.nn.Linear(24, 9) if what == "linear" else
+               blocks.ResidualBlock(blocks.ModelArgsSSMau(24, 8) if what == "a" else blocks.ModelArgsMamba(24, 8))).cuda()
+        x = torch.randn(2, 50, 24, device="cuda", requires_grad=True)
+        params = list(net.parameters())
+        t = [x, *params]
+        y = blocks._norm_linear(net, x) if what == "linear" else net(x)
+    y.square().sum().backward()
+    most = sum((v.numel() + 3) // 4 * 4 * v.element_size() for v in params)
+    for v in t:
+        own = v.numel() * v.element_size()
+        held = v.grad.untyped_storage().nbytes()
+        assert held <= most if any(v is p for p in params) else held == own, tuple(v.shape)
