@@ -10,6 +10,8 @@
 
 #include <torch/csrc/autograd/autograd.h>
 
+#include <algorithm>
+
 namespace aussm_host {
 
 namespace {
@@ -74,9 +76,9 @@ Tensor back_projection(const BlockDims& s, const Tensor& y, const Tensor& W_out,
       .bias(ptr(b_out)).add(s.residual ? ptr(x) : nullptr).run();
   return out;
 }
-// gradient of the rows y behind the output projection, its weight gradient
+// gradient of the rows y behind the output projection (dy null: not wanted), its weight gradient
 void out_grads(const BlockDims& s, const Tensor& dout, const Tensor& y, const Tensor& W_out, float* dy, float* dW, float* db) {
-  Gemm(s.e, s.b * s.l, s.d).A(ptr(W_out), 1, s.e).B(ptr(dout), 1, s.d, s.l * s.d).batch(s.l).C(dy, s.l, 1, s.e * s.l).run();
+  if (dy) Gemm(s.e, s.b * s.l, s.d).A(ptr(W_out), 1, s.e).B(ptr(dout), 1, s.d, s.l * s.d).batch(s.l).C(dy, s.l, 1, s.e * s.l).run();
   if (dW) Gemm(s.d, s.e, s.l).A(ptr(dout), 1, s.d, s.l * s.d).Bz(ptr(y), 1, s.l, s.e * s.l).C(dW, s.e, 1).sum(s.b).run();
   if (db) check(aussm_col_sum(ptr(dout), db, (size_t)(s.b * s.l), s.d, 1.0f, cur_stream()), "aussm_col_sum");
 }
@@ -195,14 +197,24 @@ variable_list AussmBlockNode::gradients(const variable_list& g) {
   const Tensor dout = dense(g[0]);
   const int64_t b = s.b, l = s.l, e = s.e;
   auto need = [&](int i) { return in[i].defined() && task_should_compute_output(i); };
+  auto any = [&](std::initializer_list<int> is) { return std::any_of(is.begin(), is.end(), need); };
+  // how far down the block something wants a gradient: past the convolution, past the operator
+  const bool front = any({A_X, A_NW, A_WIN, A_BIN, A_CW, A_CB});
+  const bool op = front || any({A_WXP, A_WDT, A_BDT, A_XAW, A_XAB, A_B, A_C, A_D});
   Cleared acc;
   int id[A_INPUTS];            // (norm and convolution add to theirs in any case)
   for (int i : {A_NW, A_WIN, A_BIN, A_CW, A_CB, A_WXP, A_WDT, A_WOUT, A_BOUT})
-    id[i] = need(i) || (in[i].defined() && (i == A_NW || i == A_CW)) ? acc.part(in[i].numel()) : -1;
+    id[i] = need(i) || (front && in[i].defined() && (i == A_NW || i == A_CW)) ? acc.part(in[i].numel()) : -1;
   acc.clear(x);
   auto gp = [&](int i) { return id[i] < 0 ? nullptr : acc.data(id[i]); };
-  Tensor dy = empty_f32({b, e, l}, x);
+  auto parts = [&] {
+    for (int i : {A_NW, A_WIN, A_BIN, A_CW, A_CB, A_WXP, A_WDT, A_WOUT, A_BOUT})
+      if (need(i)) out[i] = acc.view(id[i], in[i].sizes());
+    return std::move(out);
+  };
+  const Tensor dy = op ? empty_f32({b, e, l}, x) : Tensor();
   out_grads(s, dout, y, in[A_WOUT], ptr(dy), gp(A_WOUT), gp(A_BOUT));
+  if (!op) return parts();
   // the operator
   Tensor du = empty_f32({b, e, l}, x), ddt = empty_f32({b, e, l}, x), dxz = empty_f32({b, 2 * e, l}, x), dh = empty_f32({2, b, e, n}, x);
   for (int i : {A_BDT, A_XAW, A_XAB, A_B, A_C, A_D}) out[i] = at::empty_like(in[i], at::MemoryFormat::Contiguous);
@@ -216,16 +228,17 @@ variable_list AussmBlockNode::gradients(const variable_list& g) {
     check(aussm_operator_bwd(&p, ptr(dy), nullptr, nullptr, ptr(nh_re), ptr(nh_im), &q, ptr(ws), cur_stream()), "aussm_operator_bwd");
   }
   // dt = softplus(W_dt (W_xp u) + 2 b_dt): ddt is the gradient of the softplus' argument
-  Tensor ddt0 = empty_f32({b, r, l}, x);
-  rows_from_rows_t(ptr(in[A_WDT]), ptr(ddt), ptr(ddt0), b, l, e, r, e, r).run();
   if (float* w = gp(A_WDT)) Gemm(e, r, l).A(ptr(ddt), l, 1, e * l).Bz(ptr(dt0), 1, l, r * l).C(w, r, 1).sum(b).run();
-  rows_from_rows_t(ptr(in[A_WXP]), ptr(ddt0), ptr(du), b, l, r, e, r, e).add(ptr(du)).run();
-  if (float* w = gp(A_WXP)) Gemm(r, e, l).A(ptr(ddt0), l, 1, r * l).Bz(ptr(u), 1, l, e * l).C(w, e, 1).sum(b).run();
-  out[A_X] = front_grads(s, x, xn, rstd, in[A_NW], xz, in[A_WIN], in[A_CW], du, dxz, dout, gp(A_NW), gp(A_WIN), gp(A_BIN),
-                         gp(A_CW), gp(A_CB), need(A_X) || need(A_NW));
-  for (int i : {A_NW, A_WIN, A_BIN, A_CW, A_CB, A_WXP, A_WDT, A_WOUT, A_BOUT})
-    if (need(i)) out[i] = acc.view(id[i], in[i].sizes());
-  return out;
+  if (front || need(A_WXP)) {
+    const Tensor ddt0 = empty_f32({b, r, l}, x);
+    rows_from_rows_t(ptr(in[A_WDT]), ptr(ddt), ptr(ddt0), b, l, e, r, e, r).run();
+    if (float* w = gp(A_WXP)) Gemm(r, e, l).A(ptr(ddt0), l, 1, r * l).Bz(ptr(u), 1, l, e * l).C(w, e, 1).sum(b).run();
+    if (front) rows_from_rows_t(ptr(in[A_WXP]), ptr(ddt0), ptr(du), b, l, r, e, r, e).add(ptr(du)).run();
+  }
+  if (front)
+    out[A_X] = front_grads(s, x, xn, rstd, in[A_NW], xz, in[A_WIN], in[A_CW], du, dxz, dout, gp(A_NW), gp(A_WIN), gp(A_BIN),
+                           gp(A_CW), gp(A_CB), need(A_X) || need(A_NW));
+  return parts();
 }
 
 variable_list AussmBlockNode::recorded(variable_list&& g) {
@@ -255,9 +268,13 @@ std::optional<AussmBlockResult> aussm_block(const Tensor& x_, const OptTensor& n
   if (e != s.d || W_xp.size(1) != e || W_dt.size(0) != e || W_dt.size(1) != r || b_dt.numel() != e || D.numel() != e) return std::nullopt;
   if (xA_w.size(0) != e * n || xA_w.size(1) != e || xA_b.numel() != e * n || !operator_supported(s.b, e, n, s.l)) return std::nullopt;
   const c10::DeviceGuard guard(x_.device());
-  bool needs_grad = false;
+  bool needs_grad = false, op_grad = false;        // of anything; of more than the output projection
   if (at::GradMode::is_enabled())
-    for (const Tensor& t : raw) needs_grad = needs_grad || wants_grad(t);
+    for (int i = 0; i < A_INPUTS; ++i) {
+      needs_grad = needs_grad || wants_grad(raw[i]);
+      op_grad = op_grad || (i != A_WOUT && i != A_BOUT && wants_grad(raw[i]));
+    }
+  auto keep = [&](const Tensor& t) { return op_grad ? t : Tensor(); };
   AussmBlockResult res;
   std::shared_ptr<AussmBlockNode> node;
   {
@@ -286,7 +303,7 @@ std::optional<AussmBlockResult> aussm_block(const Tensor& x_, const OptTensor& n
       node->set_next_edges(torch::autograd::collect_next_edges(raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9],
                                                                raw[10], raw[11], raw[12], raw[13], raw[14], raw[15]));
       node->save({raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9], raw[10], raw[11], raw[12], raw[13], raw[14],
-                  raw[15], f.xn, f.rstd, f.xz, f.u, dt0, dt, y, nh_re, nh_im});
+                  raw[15], keep(f.xn), keep(f.rstd), keep(f.xz), keep(f.u), keep(dt0), keep(dt), y, keep(nh_re), keep(nh_im)});
       node->s = s; node->n = n; node->r = r; node->scale = (float)scale;
     }
   }
@@ -322,15 +339,25 @@ variable_list MambaBlockNode::gradients(const variable_list& g) {
   const Tensor dout = dense(g[0]);
   const int64_t b = s.b, l = s.l, e = s.e, R = r + 2 * n;
   auto need = [&](int i) { return in[i].defined() && task_should_compute_output(i); };
+  auto any = [&](std::initializer_list<int> is) { return std::any_of(is.begin(), is.end(), need); };
+  // how far down the block something wants a gradient: past the convolution, past the scan
+  const bool front = any({M_X, M_NW, M_WIN, M_BIN, M_CW, M_CB});
+  const bool op = front || any({M_WXP, M_WDT, M_BDT, M_ALOG, M_D});
   Cleared acc;
   int id[M_INPUTS];            // (norm and convolution add to theirs in any case)
   for (int i : {M_NW, M_WIN, M_BIN, M_CW, M_CB, M_WXP, M_WDT, M_BDT, M_ALOG, M_D, M_WOUT, M_BOUT})
-    id[i] = need(i) || (in[i].defined() && (i == M_NW || i == M_CW)) ? acc.part(in[i].numel()) : -1;
-  const Tensor ddbc = acc.own(x, {b, R, l});        // (the scan adds to its rows of B and C)
+    id[i] = need(i) || (front && in[i].defined() && (i == M_NW || i == M_CW)) ? acc.part(in[i].numel()) : -1;
+  const Tensor ddbc = op ? acc.own(x, {b, R, l}) : Tensor();        // (the scan adds to its rows of B and C)
   acc.clear(x);
   auto gp = [&](int i) { return id[i] < 0 ? nullptr : acc.data(id[i]); };
-  Tensor dy = empty_f32({b, e, l}, x);
+  auto parts = [&] {
+    for (int i : {M_NW, M_WIN, M_BIN, M_CW, M_CB, M_WXP, M_WDT, M_BDT, M_D, M_WOUT, M_BOUT})
+      if (need(i)) out[i] = acc.view(id[i], in[i].sizes());
+    return std::move(out);
+  };
+  const Tensor dy = op ? empty_f32({b, e, l}, x) : Tensor();
   out_grads(s, dout, y, in[M_WOUT], ptr(dy), gp(M_WOUT), gp(M_BOUT));
+  if (!op) return parts();
   Tensor du = empty_f32({b, e, l}, x), ddt = empty_f32({b, e, l}, x), dxz = empty_f32({b, 2 * e, l}, x);
   {
     const size_t wf = aussm_scan_workspace_floats(2, b, e, n, l, CK, AUSSM_F32);
@@ -343,19 +370,18 @@ variable_list MambaBlockNode::gradients(const variable_list& g) {
           "aussm_real_bwd_rows");
   }
   // dt = W_dt dbc[:r] + b_dt, dbc = W_xp u
-  rows_from_rows_t(ptr(in[M_WDT]), ptr(ddt), ptr(ddbc), b, l, e, r, e, R).run();
   if (float* w = gp(M_WDT)) Gemm(e, r, l).A(ptr(ddt), l, 1, e * l).Bz(ptr(dbc), 1, l, R * l).C(w, r, 1).sum(b).run();
-  rows_from_rows_t(ptr(in[M_WXP]), ptr(ddbc), ptr(du), b, l, R, e, R, e).add(ptr(du)).run();
+  if (front || need(M_WXP)) rows_from_rows_t(ptr(in[M_WDT]), ptr(ddt), ptr(ddbc), b, l, e, r, e, R).run();
   if (float* w = gp(M_WXP)) Gemm(R, e, l).A(ptr(ddbc), l, 1, R * l).Bz(ptr(u), 1, l, e * l).C(w, e, 1).sum(b).run();
-  out[M_X] = front_grads(s, x, xn, rstd, in[M_NW], xz, in[M_WIN], in[M_CW], du, dxz, dout, gp(M_NW), gp(M_WIN), gp(M_BIN),
-                         gp(M_CW), gp(M_CB), need(M_X) || need(M_NW));
-  for (int i : {M_NW, M_WIN, M_BIN, M_CW, M_CB, M_WXP, M_WDT, M_BDT, M_D, M_WOUT, M_BOUT})
-    if (need(i)) out[i] = acc.view(id[i], in[i].sizes());
+  if (front) rows_from_rows_t(ptr(in[M_WXP]), ptr(ddbc), ptr(du), b, l, R, e, R, e).add(ptr(du)).run();
+  if (front)
+    out[M_X] = front_grads(s, x, xn, rstd, in[M_NW], xz, in[M_WIN], in[M_CW], du, dxz, dout, gp(M_NW), gp(M_WIN), gp(M_BIN),
+                           gp(M_CW), gp(M_CB), need(M_X) || need(M_NW));
   if (need(M_ALOG)) {
     out[M_ALOG] = empty_f32({e, n}, x);
     check(aussm_neg_exp(ptr(in[M_ALOG]), gp(M_ALOG), ptr(out[M_ALOG]), e * n, cur_stream()), "aussm_neg_exp");
   }
-  return out;
+  return parts();
 }
 
 variable_list MambaBlockNode::recorded(variable_list&& g) {
@@ -384,9 +410,13 @@ OptTensor mamba_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
   if (A_log.size(0) != e || n > AUSSM_MAX_STATE || W_xp.size(0) != R || W_xp.size(1) != e || W_dt.size(0) != e || b_dt.numel() != e || D.numel() != e)
     return std::nullopt;
   const c10::DeviceGuard guard(x_.device());
-  bool needs_grad = false;
+  bool needs_grad = false, op_grad = false;        // of anything; of more than the output projection
   if (at::GradMode::is_enabled())
-    for (const Tensor& t : raw) needs_grad = needs_grad || wants_grad(t);
+    for (int i = 0; i < M_INPUTS; ++i) {
+      needs_grad = needs_grad || wants_grad(raw[i]);
+      op_grad = op_grad || (i != M_WOUT && i != M_BOUT && wants_grad(raw[i]));
+    }
+  auto keep = [&](const Tensor& t) { return op_grad ? t : Tensor(); };
   Tensor out;
   std::shared_ptr<MambaBlockNode> node;
   {
@@ -399,8 +429,8 @@ OptTensor mamba_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
     rows_from_rows(ptr(in[M_WXP]), ptr(f.u), ptr(dbc), s.b, s.l, e, R, e, R).run();
     rows_from_rows(ptr(in[M_WDT]), ptr(dbc), ptr(dt), s.b, s.l, r, e, R, e).bias(ptr(in[M_BDT])).run();
     check(aussm_neg_exp(ptr(in[M_ALOG]), nullptr, ptr(A), e * n, cur_stream()), "aussm_neg_exp");
-    const int ck = needs_grad ? CK : AUSSM_TILE;
-    const Tensor hck = needs_grad ? empty_f32({s.b, (s.l + ck - 1) / ck, n, 1, e}, x) : Tensor();
+    const int ck = op_grad ? CK : AUSSM_TILE;
+    const Tensor hck = op_grad ? empty_f32({s.b, (s.l + ck - 1) / ck, n, 1, e}, x) : Tensor();
     {
       const size_t wf = aussm_scan_workspace_floats(2, s.b, e, n, s.l, ck, AUSSM_F32);
       const Tensor ws = wf ? empty_f32({(int64_t)wf}, x) : Tensor();
@@ -417,8 +447,8 @@ OptTensor mamba_block(const Tensor& x_, const OptTensor& nw_, double eps, bool r
       node = make_node<MambaBlockNode>();
       node->set_next_edges(torch::autograd::collect_next_edges(raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9],
                                                                raw[10], raw[11], raw[12]));
-      node->save({raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9], raw[10], raw[11], raw[12], f.xn, f.rstd, f.xz,
-                  f.u, dbc, dt, A, hck, y});
+      node->save({raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9], raw[10], raw[11], raw[12], keep(f.xn), keep(f.rstd),
+                  keep(f.xz), keep(f.u), keep(dbc), keep(dt), keep(A), hck, y});
       node->s = s; node->n = n; node->r = r;
     }
   }

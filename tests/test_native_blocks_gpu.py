@@ -317,3 +317,46 @@ def test_arguments_handed_to_the_operator(d, n, l, monkeypatch):
     assert net.ssm_args == {"u": 1}
     net(x)
     assert net.ssm_args["u"].shape == (2, d, l)
+
+
+# ---- blocks of which only a part is trained ---------------------------------------------------------
+
+TRAINED = {"a": ["out_proj", "D", "xA_proj", "dt_proj.bias", "dt_proj.weight", "x_proj", "conv1d.bias", "conv1d", "in_proj.bias", "norm", ""],
+           "m": ["out_proj", "D", "A_log", "dt_proj.bias", "dt_proj.weight", "x_proj", "conv1d.bias", "conv1d", "in_proj.bias", "norm", ""]}
+
+
+@pytest.mark.parametrize("kind,trained", [(k, t) for k in "am" for t in TRAINED[k]])
+@pytest.mark.parametrize("with_x", [False, True])
+def test_partly_frozen_blocks(kind, trained, with_x):
+    """The gradients that are left are those of the whole block; with the output projection alone nothing of an activation's
+    size is formed for the backward pass."""
+    print("case frozen", kind, trained, with_x, flush=True)
+    net = _residual(kind)
+    x, dy = torch.randn(3, 130, 16, device="cuda"), torch.randn(3, 130, 16, device="cuda")
+    xi = x.clone().requires_grad_(True)
+    net(xi).backward(dy)
+    want = {k: p.grad for k, p in net.named_parameters()}
+    net.zero_grad(set_to_none=True)
+    for k, p in net.named_parameters():
+        p.requires_grad_(bool(trained) and k.removeprefix("mixer.").startswith(trained))
+    xf = x.clone().requires_grad_(with_x)
+    before = torch.cuda.memory_allocated()
+    y = net(xf)
+    (net.mixer if hasattr(net, "mixer") else net).__dict__.update(_handed=None, _ssm_args=None)
+    if trained == "out_proj" and not with_x:            # its input (d_inner = 2 d for "m") and the block's output
+        assert torch.cuda.memory_allocated() - before <= (2 if kind == "a" else 3) * x.numel() * 4 + 4096
+    if not y.requires_grad:
+        assert not trained and not with_x
+        return
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    y.backward(dy)
+    if trained == "out_proj" and not with_x:
+        assert torch.cuda.max_memory_allocated() - before < x.numel() * 4
+    named = [(k, p.grad, want[k]) for k, p in net.named_parameters() if p.requires_grad]
+    assert all(g is not None for _, g, _ in named) and all(p.grad is None for p in net.parameters() if not p.requires_grad)
+    for k, g, w in named + ([("x", xf.grad, xi.grad)] if with_x else []):
+        g, w = (torch.view_as_real(t) if t.is_complex() else t for t in (g, w))
+        scale = max(1e-3, float(w.abs().max()))
+        torch.testing.assert_close(g / scale, w / scale, atol=1e-5, rtol=1e-5, msg=lambda m, k=k: f"{k}: {m}")
