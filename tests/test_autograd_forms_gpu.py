@@ -260,6 +260,20 @@ def test_saved_tensors_moved_recomputed_and_kept(what, how):
     _close(got, want, 1e-5)
 
 
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("off", [1, 2])
+def test_upstream_gradient_that_is_not_aligned(gate, off):
+    """A gradient that does not start on 16 bytes behind a forward pass whose auxiliary buffer is filled: another kernel."""
+    print("case misaligned", gate, off, flush=True)
+    t = _scan_inputs("unitary", d=64, n=16, l=256)
+    kw = {"z": torch.randn(2, 64, 256, device="cuda")} if gate else {}
+    dy = torch.randn(2 * 64 * 256 + off, device="cuda")[off:].view(2, 64, 256)
+    assert dy.data_ptr() % 16
+    y = _scan("unitary")(*t, **kw)
+    got = torch.autograd.grad(y, t, dy, retain_graph=True)
+    _close(got, torch.autograd.grad(y, t, dy.clone()), 2e-5)
+
+
 # ---- what a gradient keeps alive ------------------------------------------------------------------
 
 @pytest.mark.parametrize("what", ["unitary", "complex", "s6", "a", "m", "linear"])

@@ -219,6 +219,13 @@ def test_native_block_matches_the_composed_layers(kind, d, n, b, l, kw, residual
         torch.testing.assert_close(a / scale, w / scale, atol=1e-4, rtol=1e-4, msg=lambda m, k=name: f"{k}: {m}")
 
 
+# widths and row counts at which the products of the blocks run on the tiles of eight wavefronts (256 x 96 and 256 x 128, and
+# for "a" a sliced sum), whole groups of four along k and not; two evaluations in fp32 with sums of up to 12320 terms
+@pytest.mark.parametrize("kind,d,n,b,l", [("a", 256, 16, 16, 770), ("a", 130, 4, 16, 690), ("m", 256, 16, 12, 721), ("m", 130, 16, 10, 701)])
+def test_native_block_on_wide_tiles(kind, d, n, b, l, monkeypatch):
+    test_native_block_matches_the_composed_layers(kind, d, n, b, l, {}, True, monkeypatch)
+
+
 # ---- calls that leave the native route ------------------------------------------------------------
 
 class _Marked(torch.Tensor):
