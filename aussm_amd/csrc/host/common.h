@@ -30,11 +30,8 @@ typedef std::optional<Tensor> OptTensor;
 struct AussmError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
-// raised in Python as RuntimeError / ValueError, without the C++ call stack that TORCH_CHECK appends
+// raised in Python as RuntimeError, without the C++ call stack that TORCH_CHECK appends
 struct ArgError : std::runtime_error {
-  using std::runtime_error::runtime_error;
-};
-struct ValueArgError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
 

@@ -28,8 +28,6 @@ PYBIND11_MODULE(_aussm_host, m) {
       if (p) std::rethrow_exception(p);
     } catch (const AussmError& e) {
       PyErr_SetString(aussm_error_class(), e.what());
-    } catch (const ValueArgError& e) {
-      PyErr_SetString(PyExc_ValueError, e.what());
     } catch (const ArgError& e) {
       PyErr_SetString(PyExc_RuntimeError, e.what());
     }

@@ -132,8 +132,10 @@ variable_list UnitaryNode::gradients(const variable_list& g) {
 }  // namespace
 
 // Checkpoint interval of the unitary scan for a shape: 256, or half of it where that lets a launch with few (batch,
-// channel) pairs be split into more segments along L (a segment is a whole number of checkpoint blocks); calls
-// that are not split at all checkpoint every 4096 steps (one checkpoint, at the end, for shorter sequences).
+// channel) pairs be split into more segments along L (a segment is a whole number of checkpoint blocks).  Where the call
+// is not split nothing ties the interval to a segment length, and against the float64 oracle the gradients do not change
+// between 256 and one checkpoint at the end of 2048 or 8192 steps (the reverse recurrence is norm-preserving): every
+// 4096 steps then (one checkpoint, at the end, for shorter sequences).
 int unitary_ck(int b, int d, int n, int l) {
   constexpr int CK = 256, CK_LONG = 4096;
   const int s_half = aussm_unitary_split_segments(b, d, n, l, CK / 2), s_full = aussm_unitary_split_segments(b, d, n, l, CK);

@@ -60,7 +60,8 @@ __device__ __forceinline__ float dsiluf_(float v) { float s = sigmoidf_(v); retu
 // -20 .. 20 3.5e-8 against 2.3e-7.
 //   t = e^v, with the rounding of v log2(e) made up for (the maximum: v = -inf);  w = fl(1 + t) = 2^k m, m in
 //   [1 / sqrt 2, sqrt 2);  f = m - 1 plus what 1 + t was rounded by;  log(1 + f) = f - s (f - R), s = f / (2 + f),
-//   R = s^2 (2/3 + 2/5 s^2 + ..): the series of 2 artanh(s)
+//   R = s^2 (2/3 + 2/5 s^2 + ..): the series of 2 artanh(s) (Abramowitz and Stegun, 4.1.27; the reduction to one octave
+//   around 1 is that of Cody and Waite, Software Manual for the Elementary Functions, chapter 5)
 __device__ __forceinline__ float softplusf_(float v) {
   const float h = v * 1.44269504088896341f;
   const float lo = fmaxf(fmaf(v, 1.92596299112661746887e-8f, fmaf(v, 1.44269504088896341f, -h)), -1.0f);

@@ -33,27 +33,16 @@ from ._lib import check, ptr
 
 Tensor = torch.Tensor
 
-# Checkpoint interval (timesteps) of the forward pass.  The unitary backward pass regenerates the
+# Checkpoint interval (timesteps) of a unitary scan that is split along L.  The unitary backward pass regenerates the
 # states by running the recurrence in reverse and only uses checkpoints to stop rounding drift,
 # so a long interval is enough; the complex and real backward passes recompute every tile from
 # its checkpoint and need one per tile.
 UNITARY_CK = 256
-# ... and where the launch is not split along L nothing ties the interval to a segment length: measured
-# against the float64 oracle the gradients do not change between an interval of 256 and one checkpoint at
-# the end of 2048 or 8192 steps (the reverse recurrence is norm-preserving), so such a call keeps a
-# checkpoint every UNITARY_CK_LONG steps only
-UNITARY_CK_LONG = 4096
 
 
 def unitary_ck(b: int, d: int, n: int, l: int) -> int:
-    """Checkpoint interval of the unitary scan for a shape: UNITARY_CK, or half of it where that
-    lets a launch with few (batch, channel) pairs be split into more segments along L (a segment
-    is a whole number of checkpoint blocks); calls that are not split at all checkpoint every
-    UNITARY_CK_LONG steps (one checkpoint, at the end, for shorter sequences)."""
+    """Checkpoint interval of the unitary scan for a shape (csrc/host/scans.cpp has the rule)."""
     return _lib.host().unitary_ck(b, d, n, l)
-
-
-TILE_CK = _lib.TILE
 
 
 def _stream() -> int:
@@ -85,16 +74,6 @@ def unitary_aux(u, n: int, ck: int) -> Tensor:
     b, d, l = u.shape
     return torch.empty((lib.aussm_unitary_aux_floats(b, d, n, l, ck or _lib.TILE),), device=u.device,
                        dtype=torch.float32)
-
-
-def unitary_aux_useful(b: int, d: int, n: int, l: int, ck: int, in_dtype: int, urep: int = 1) -> bool:
-    """False when neither direction of the scan would touch an auxiliary buffer for this shape (the
-    vector-ALU kernels use it only for the segment states of a call that is split along the sequence), so
-    that the autograd wrapper does not allocate and keep a buffer for nothing."""
-    lib = _lib.load()
-    return bool(lib.aussm_unitary_kernel_mode(0, b, d, n, l, ck, in_dtype, urep, 1)
-                or lib.aussm_unitary_kernel_mode(1, b, d, n, l, ck, in_dtype, urep, 1)
-                or lib.aussm_unitary_split_segments(b, d, n, l, ck) > 1)
 
 
 def unitary_fwd_raw(u, delta, theta, Bri, Cri, D=None, z=None, h0=None, want_state=False, ck=0, aux=None, ck_arg=0):
@@ -188,7 +167,6 @@ def unitary_scan(u: Tensor, delta: Tensor, theta: Tensor, Bc: Tensor, Cc: Tensor
 # --------------------------------------------------------------------------------------------
 
 REC_CK = 16          # checkpoint interval the recomputing backward kernels (complex, real) need
-REC_MAX_STATE = _lib.MAX_STATE   # largest state size those kernels take (16 states per launch, one launch per block)
 
 
 def _scan_workspace(variant: int, u: Tensor, n: int, ck: int) -> Optional[Tensor]:
