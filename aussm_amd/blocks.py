@@ -294,9 +294,10 @@ class SSMauBlock(nn.Module):
         if self._ssm_args is None:
             if self._handed is None:
                 raise AttributeError("ssm_args")
-            u, dt, xz, x, x_bias, B, C, D = self._handed
-            self.ssm_args = {"u": u, "dt": dt, "x": x, "x_bias": x_bias, "B": B, "C": C, "D": D,
-                             "z": xz[:, u.shape[1]:].contiguous()}
+            u, dt, xz, xs, B, C, D = self._handed
+            d, n = u.shape[1], B.numel()
+            self.ssm_args = {"u": u, "dt": dt, "x": xs[:d * n * d].view(d, n, d), "x_bias": xs[d * n * d:].view(d, n),
+                             "B": B, "C": C, "D": D, "z": xz[:, d:].contiguous()}
         return self._ssm_args
 
     @ssm_args.setter

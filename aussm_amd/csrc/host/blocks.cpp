@@ -191,7 +191,7 @@ variable_list AussmBlockNode::gradients(const variable_list& g) {
   for (int i = 0; i < A_INPUTS; ++i) in[i] = dense(saved[i].unpack());
   const Tensor xn = saved[A_INPUTS].unpack(), rstd = saved[A_INPUTS + 1].unpack(), xz = saved[A_INPUTS + 2].unpack(),
                u = saved[A_INPUTS + 3].unpack(), dt0 = saved[A_INPUTS + 4].unpack(), dt = saved[A_INPUTS + 5].unpack(),
-               y = saved[A_INPUTS + 6].unpack(), nh_re = saved[A_INPUTS + 7].unpack(), nh_im = saved[A_INPUTS + 8].unpack();
+               y = saved[A_INPUTS + 6].unpack(), nh = saved[A_INPUTS + 7].unpack();
   const Tensor& x = in[A_X];
   const c10::DeviceGuard guard(x.device());
   const Tensor dout = dense(g[0]);
@@ -225,7 +225,7 @@ variable_list AussmBlockNode::gradients(const variable_list& g) {
     q.u = ptr(du); q.dt = ptr(ddt); q.x = ptr(out[A_XAW]); q.x_bias = ptr(out[A_XAB]); q.D = ptr(out[A_D]);
     q.B_r = ptr(out[A_B]); q.B_theta = q.B_r + 1; q.C_r = ptr(out[A_C]); q.C_theta = q.C_r + 1;
     q.z = ptr(dxz) + e * l; q.h_re = ptr(dh); q.h_im = q.h_re + b * e * n; q.dt_bias = ptr(out[A_BDT]);
-    check(aussm_operator_bwd(&p, ptr(dy), nullptr, nullptr, ptr(nh_re), ptr(nh_im), &q, ptr(ws), cur_stream()), "aussm_operator_bwd");
+    check(aussm_operator_bwd(&p, ptr(dy), nullptr, nullptr, ptr(nh), ptr(nh) + b * e * n, &q, ptr(ws), cur_stream()), "aussm_operator_bwd");
   }
   // dt = softplus(W_dt (W_xp u) + 2 b_dt): ddt is the gradient of the softplus' argument
   if (float* w = gp(A_WDT)) Gemm(e, r, l).A(ptr(ddt), l, 1, e * l).Bz(ptr(dt0), 1, l, r * l).C(w, r, 1).sum(b).run();
@@ -287,13 +287,13 @@ std::optional<AussmBlockResult> aussm_block(const Tensor& x_, const OptTensor& n
     rows_from_rows(ptr(in[A_WXP]), ptr(f.u), ptr(dt0), s.b, s.l, e, r, e, r).run();
     // (the reference adds the bias of dt_proj twice, aussm.py:878-880)
     rows_from_rows(ptr(in[A_WDT]), ptr(dt0), ptr(dt), s.b, s.l, r, e, r, e).bias(ptr(in[A_BDT]), 2.0f).softplus().run();
-    const Tensor nh_re = empty_f32({s.b, e, n}, x), nh_im = empty_f32({s.b, e, n}, x);
+    const Tensor nh = empty_f32({2, s.b, e, n}, x);         // (real, then imaginary parts)
     {
       const Tensor ws = empty_f32({(int64_t)aussm_ssm_adaptive_unitary_workspace_floats(s.b, e, n, s.l, 0)}, x);
       const aussm_operator_args p = block_operator(s, n, (float)scale, f.u, dt, in, f.xz);
-      res.x = empty_f32({e, n, e}, x);
-      res.x_bias = empty_f32({e, n}, x);
-      check(aussm_operator_fwd_keep(&p, ptr(y), ptr(nh_re), ptr(nh_im), ptr(ws), ptr(res.x), ptr(res.x_bias), cur_stream()),
+      res.x_and_bias = empty_f32({e * n * (e + 1)}, x);
+      float* const kept = ptr(res.x_and_bias);
+      check(aussm_operator_fwd_keep(&p, ptr(y), ptr(nh), ptr(nh) + s.b * e * n, ptr(ws), kept, kept + e * n * e, cur_stream()),
             "aussm_operator_fwd_keep");
     }
     res.u = f.u; res.dt = dt; res.xz = f.xz;
@@ -303,7 +303,7 @@ std::optional<AussmBlockResult> aussm_block(const Tensor& x_, const OptTensor& n
       node->set_next_edges(torch::autograd::collect_next_edges(raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9],
                                                                raw[10], raw[11], raw[12], raw[13], raw[14], raw[15]));
       node->save({raw[0], raw[1], raw[2], raw[3], raw[4], raw[5], raw[6], raw[7], raw[8], raw[9], raw[10], raw[11], raw[12], raw[13], raw[14],
-                  raw[15], keep(f.xn), keep(f.rstd), keep(f.xz), keep(f.u), keep(dt0), keep(dt), y, keep(nh_re), keep(nh_im)});
+                  raw[15], keep(f.xn), keep(f.rstd), keep(f.xz), keep(f.u), keep(dt0), keep(dt), y, keep(nh)});
       node->s = s; node->n = n; node->r = r; node->scale = (float)scale;
     }
   }

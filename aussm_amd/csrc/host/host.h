@@ -19,9 +19,9 @@ Tensor adaptive_operator(const Tensor& u, const Tensor& dt, const Tensor& x, con
 
 // The blocks and linear layers answer nothing where they do not take the tensors (another type or device, sizes
 // beyond the kernels): the caller then composes the layer from separate operators.
-// (the AUSSM block also returns what it handed to its operator, outside the graph: u, dt, the rows whose second half is z, and
-// the projection's weight and bias as the operator's x and x_bias)
-struct AussmBlockResult { Tensor out, u, dt, xz, x, x_bias; };
+// (the AUSSM block also returns what it handed to its operator, outside the graph: u, dt, the rows whose second half is z, and,
+// one after the other in one buffer, the projection's weight and bias as the operator's x and x_bias)
+struct AussmBlockResult { Tensor out, u, dt, xz, x_and_bias; };
 std::optional<AussmBlockResult> aussm_block(const Tensor& x, const OptTensor& norm_w, double eps, bool residual, const Tensor& W_in, const OptTensor& b_in,
                       const Tensor& conv_w, const OptTensor& conv_b, const Tensor& W_xp, const Tensor& W_dt, const Tensor& b_dt, const Tensor& xA_w,
                       const Tensor& xA_b, const Tensor& B, const Tensor& C, const Tensor& D, const Tensor& W_out, const OptTensor& b_out, double scale);

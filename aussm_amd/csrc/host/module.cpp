@@ -53,7 +53,7 @@ PYBIND11_MODULE(_aussm_host, m) {
                           double scale) -> py::object {
     const auto r = aussm_block(x, nw, eps, residual, W_in, b_in, cw, cb, W_xp, W_dt, b_dt, xA_w, xA_b, B, C, D, W_out, b_out, scale);
     if (!r) return py::none();
-    return py::make_tuple(r->out, r->u, r->dt, r->xz, r->x, r->x_bias);
+    return py::make_tuple(r->out, r->u, r->dt, r->xz, r->x_and_bias);
   });
   m.def("mamba_block", &mamba_block);
   m.def("norm_linear", &norm_linear);
