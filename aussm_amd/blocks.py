@@ -361,8 +361,8 @@ class SSMauBlock(nn.Module):
         }
 
     def ssm_au(self, x, z):
-        self.ssm_args = self._scan_args(x, z)
-        y = self.optimized_SSMa_function(**self.ssm_args)
+        self._ssm_args, self._handed = self._scan_args(x, z), None
+        y = self.optimized_SSMa_function(**self._ssm_args)
         return _swap(y)
 
 

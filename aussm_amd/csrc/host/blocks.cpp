@@ -115,7 +115,8 @@ bool front_ok(const Tensor& x, const Tensor& nw, bool norm, const Tensor& W_in, 
   return s.b * s.l < (1ll << 31) / 2 && s.l < (1 << 24) && s.b * (s.e + 3) / 4 < 0x7fffffffll;
 }
 
-// ---- the same from differentiable operators, for a backward pass that is recorded (create_graph) ----------
+// ---- the same from differentiable operators, for a backward pass that is recorded (create_graph) or that more than one
+// plain gradient follows (a batch of them under vmap, one with a tangent) -----------------------------------
 Tensor composed_norm(const Tensor& x, const Tensor& w, double eps) {
   return w.defined() ? x * (x.square().mean({-1}, true) + eps).rsqrt() * w : x;
 }
@@ -132,7 +133,7 @@ Tensor composed_back(const BlockDims& s, const Tensor& y, const Tensor& W_out, c
   const Tensor out = at::linear(y.transpose(1, 2), W_out, b_out);
   return s.residual ? out + x : out;
 }
-// Gradients of compose(inputs) for the first `count` saved tensors, recorded.  The operators get an alias of each input: what
+// Gradients of compose(inputs) for the first `count` saved tensors, recorded if the pass is.  The operators get an alias of each input: what
 // an input owes to another one (one tensor handed in twice, a weight formed from x) is the outer graph's to follow.
 template <typename F>
 variable_list recorded_gradients(SavingNode& node, std::mutex& m, int count, const Tensor& g, const F& compose) {
@@ -142,6 +143,8 @@ variable_list recorded_gradients(SavingNode& node, std::mutex& m, int count, con
     std::lock_guard<std::mutex> lock(m);
     for (int i = 0; i < count; ++i) in[i] = node.saved[i].unpack();
   }
+  const bool record = at::GradMode::is_enabled();
+  at::AutoGradMode with_graph(true);
   std::vector<int> at;
   for (int i = 0; i < count; ++i) {
     if (!in[i].defined() || !in[i].requires_grad()) continue;
@@ -152,7 +155,7 @@ variable_list recorded_gradients(SavingNode& node, std::mutex& m, int count, con
   }
   if (wanted.empty()) return out;
   const c10::DeviceGuard guard(in[0].device());
-  const variable_list got = torch::autograd::grad({compose(in)}, wanted, {g}, true, true, true);
+  const variable_list got = torch::autograd::grad({compose(in)}, wanted, {g}, true, record, true);
   for (size_t k = 0; k < at.size(); ++k) out[at[k]] = got[k];
   return out;
 }
@@ -171,7 +174,7 @@ struct AussmBlockNode : SavingNode {
   float scale;
   std::string name() const override { return "AussmBlockBackward"; }
   variable_list gradients(const variable_list& g) override;
-  variable_list recorded(variable_list&& g) override;
+  variable_list composed(variable_list&& g) override;
 };
 
 aussm_operator_args block_operator(const BlockDims& s, int64_t n, float scale, const Tensor& u, const Tensor& dt, const Tensor* in, const Tensor& xz) {
@@ -241,7 +244,7 @@ variable_list AussmBlockNode::gradients(const variable_list& g) {
   return parts();
 }
 
-variable_list AussmBlockNode::recorded(variable_list&& g) {
+variable_list AussmBlockNode::composed(variable_list&& g) {
   return recorded_gradients(*this, mutex_, A_INPUTS, g[0], [&](const variable_list& in) {
     const auto [u, z] = composed_front(s, in[A_X], in[A_NW], in[A_WIN], in[A_BIN], in[A_CW], in[A_CB]);
     const Tensor dt = at::linear(at::linear(u.transpose(1, 2), in[A_WXP]), in[A_WDT], in[A_BDT]) + in[A_BDT];
@@ -323,7 +326,7 @@ struct MambaBlockNode : SavingNode {
   int64_t n, r;
   std::string name() const override { return "AussmMambaBlockBackward"; }
   variable_list gradients(const variable_list& g) override;
-  variable_list recorded(variable_list&& g) override;
+  variable_list composed(variable_list&& g) override;
 };
 
 variable_list MambaBlockNode::gradients(const variable_list& g) {
@@ -384,7 +387,7 @@ variable_list MambaBlockNode::gradients(const variable_list& g) {
   return parts();
 }
 
-variable_list MambaBlockNode::recorded(variable_list&& g) {
+variable_list MambaBlockNode::composed(variable_list&& g) {
   return recorded_gradients(*this, mutex_, M_INPUTS, g[0], [&](const variable_list& in) {
     const auto [c, z] = composed_front(s, in[M_X], in[M_NW], in[M_WIN], in[M_BIN], in[M_CW], in[M_CB]);
     const Tensor u = at::silu(c), dbc = at::linear(c.transpose(1, 2), in[M_WXP]);    // (x_proj reads the rows before their SiLU)
@@ -468,7 +471,7 @@ struct LinearNode : SavingNode {
   double eps;
   std::string name() const override { return "AussmLinearBackward"; }
   variable_list gradients(const variable_list& g) override;
-  variable_list recorded(variable_list&& g) override;
+  variable_list composed(variable_list&& g) override;
 };
 
 variable_list LinearNode::gradients(const variable_list& g) {
@@ -508,7 +511,7 @@ variable_list LinearNode::gradients(const variable_list& g) {
   return out;
 }
 
-variable_list LinearNode::recorded(variable_list&& g) {
+variable_list LinearNode::composed(variable_list&& g) {
   return recorded_gradients(*this, mutex_, L_INPUTS, g[0], [&](const variable_list& in) {
     return at::linear(composed_norm(in[L_X], in[L_NW], eps), in[L_W], in[L_B]);
   });

@@ -135,6 +135,10 @@ struct Cleared {
   }
 };
 
+// tensors that stand for others: wrapped by a function transform, or handled by Python
+constexpr c10::DispatchKeySet WRAPPED{c10::DispatchKey::Batched, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                      c10::DispatchKey::Functionalize, c10::DispatchKey::Python};
+
 // A graph node over saved tensors: `saved` are released together, and unpacking them after that raises torch's
 // usual error about a second backward pass.
 struct SavingNode : Node {
@@ -154,8 +158,9 @@ struct SavingNode : Node {
     for (auto& s : saved) s.reset_data();
   }
   variable_list apply(variable_list&& g) override {
-    if (at::GradMode::is_enabled()) return recorded(std::move(g));
-    return launched(g);
+    bool more = at::GradMode::is_enabled();            // create_graph
+    for (const Tensor& t : g) more = more || (t.defined() && (t._fw_grad(0).defined() || t.key_set().has_any(WRAPPED)));
+    return more ? composed(std::move(g)) : launched(g);
   }
   // gradients of the inputs from the kernels, called with gradient recording off
   virtual variable_list gradients(const variable_list& g) = 0;
@@ -166,9 +171,12 @@ struct SavingNode : Node {
   }
   // ... and for a backward pass that is recorded itself (create_graph).  The kernels' gradients carry no graph: they can
   // be used, and differentiating them raises.  (The error hangs on the edges of this node and of the gradients
-  // it got, so that every derivative that should pass through it does.)
-  virtual variable_list recorded(variable_list&& g) {
+  // it got, so that every derivative that should pass through it does.)  Tangents and batches have no kernel.
+  virtual variable_list composed(variable_list&& g) {
+    for (const Tensor& t : g)
+      if (t.defined() && t._fw_grad(0).defined()) fail(name(), ": forward-mode derivatives of this operator are not implemented");
     variable_list out = launched(g);
+    if (!at::GradMode::is_enabled()) return out;
     torch::autograd::edge_list edges = torch::autograd::collect_next_edges(g);
     edges.insert(edges.end(), next_edges().begin(), next_edges().end());
     std::shared_ptr<Node> refusal(new torch::autograd::Error(cat(name(), ": second derivatives of this operator are not implemented"),

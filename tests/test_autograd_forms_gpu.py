@@ -145,12 +145,50 @@ def test_one_tensor_as_two_inputs_of_a_block_counts_once(monkeypatch):
     _close(*_both_routes(monkeypatch, step))
 
 
+@pytest.mark.parametrize("target", ["norm_f.weight", "output.weight", "layers.1.mixer.out_proj.weight"])
+@pytest.mark.parametrize("how", ["vmap", "tangent"])
+def test_a_batch_of_gradients_and_one_with_a_tangent(target, how):
+    """What follows a gradient through the layers behind the last scan: several at once, or its derivative."""
+    from torch.autograd import forward_ad
+    print("case batched gradients", target, how, flush=True)
+    net = _model()
+    x, v = torch.randn(2, 33, 5, device="cuda"), torch.randn(3, 2, 33, 3, device="cuda")
+    w = dict(net.named_parameters())[target]
+    y = net(x)
+    want = [torch.autograd.grad(y, w, g, retain_graph=True)[0] for g in v]
+    if how == "vmap":
+        got, = torch.autograd.grad(y, w, v, is_grads_batched=True, retain_graph=True)
+        _close(got, want, 1e-5)
+        return
+    with forward_ad.dual_level():
+        got, = torch.autograd.grad(y, w, forward_ad.make_dual(v[0], v[1]), retain_graph=True)
+        primal, tangent = forward_ad.unpack_dual(got)
+        _close([primal, tangent], want[:2], 1e-5)
+
+
 @pytest.mark.parametrize("kind", ["unitary", "complex", "s6"])
-def test_recorded_gradients_of_a_scan_are_values_and_refuse_to_be_differentiated(kind):
-    print("case scan create_graph", kind, flush=True)
+def test_tangents_behind_a_scan_are_refused(kind):
+    from torch.autograd import forward_ad
+    t = _scan_inputs(kind)
+    y = _scan(kind)(*t)
+    with forward_ad.dual_level(), pytest.raises(RuntimeError, match="forward-mode"):
+        torch.autograd.grad(y, t, forward_ad.make_dual(torch.ones_like(y), torch.ones_like(y)))
+
+
+@pytest.mark.parametrize("kind", ["unitary", "complex", "s6"])
+@pytest.mark.parametrize("python", [False, True])
+def test_recorded_gradients_of_a_scan_are_values_and_refuse_to_be_differentiated(kind, python):
+    """... also through the autograd function of Python that stands for the scan under a tracer."""
+    from aussm_amd import _lib, scan
+    print("case scan create_graph", kind, python, flush=True)
     t = _scan_inputs(kind)
     want = torch.autograd.grad(_scan(kind)(*t).square().sum(), t)
-    y = _scan(kind)(*t)
+    if not python:
+        y = _scan(kind)(*t)
+    elif kind == "s6":
+        y = scan._ScanFn.apply(_lib.host().selective_scan, (False, False), *t, None, None, None)
+    else:
+        y = scan._ScanFn.apply(getattr(_lib.host(), kind + "_scan"), (False,), *t, None, None)
     got = torch.autograd.grad(y.square().sum(), t, create_graph=True)
     _close(got, want, 1e-6)
     with pytest.raises(RuntimeError, match="second derivatives"):
