@@ -2,9 +2,10 @@
 // the phase adjoints of the fused operator.
 //
 // Both operands are fp32 in memory and split EXACTLY into three bf16 pieces while they are staged into LDS (scan_fwd_xdl.h:
-// split8, xmm<3>): what a product drops is below 2^-26 of it, the sums are fp32.  Workgroup tile 128 x (32 EN), four
-// wavefronts of 64 x (16 EN), 32 of k per step; the values of the next step are requested before the products of
-// the current one, and two workgroups per compute unit cover each other's barriers.
+// split8, xmm<3>): what a product drops is below 2^-26 of it, the sums are fp32; infinities and NaN come out as fp32 sums
+// give them (xg_plain).  Workgroup tile 128 x (32 EN), four wavefronts of 64 x (16 EN), 32 of k per step; the values of the
+// next step are requested before the products of the current one, and two workgroups per compute unit cover each
+// other's barriers.
 //
 // Operands may be contiguous along k or along their other index (AK1 / BK1), so no transposed copy is ever made:
 //   along k: four neighbouring lanes fetch the 32 values of a row (one 128-byte line), 16 bytes at a time;
@@ -113,8 +114,11 @@ struct XgOperand {
 };
 
 // An infinity, and a finite value that rounds to one in bf16, leaves a NaN in its pieces (inf - inf) and in every sum that it
-// enters.  Sums that came out as an infinity or a NaN are formed again here from the values themselves, in fp32 steps: of a wavefront's slice `sw` (rows
-// mw .., columns nw ..) those of the steps of its slice of the sum.  A sum that has become a NaN ends early.
+// enters.  Sums that came out as an infinity or a NaN are formed again here from the values themselves, in fp32 steps: of a
+// wavefront's slice `sw` (rows mw .., columns nw ..) those of the steps of its slice of the sum.  64 results at a time: few that
+// are not finite one after the other by all lanes, four terms a lane and turn, else one by each lane, which ends
+// early where its sum has become a NaN.  256 x 23040, K = 1024, 77 us of finite values: 257 us with one infinity (one lane to
+// a sum: 3.3 ms), 114 us of NaN, 11 ms with an infinity in every sum.
 // (The arguments are read again: kept in scalar registers across the main loop for this they cost every product.)
 template <bool TR, int TM, int TN, int WR, int WN, int LD>
 __device__ __forceinline__ void xg_plain(float* __restrict__ sw, int mw, int nw, int lane) {
@@ -124,22 +128,42 @@ __device__ __forceinline__ void xg_plain(float* __restrict__ sw, int mw, int nw,
   const int tiles = ((p->M + TM - 1) / TM) * ((p->N + TN - 1) / TN), sl = xcd_remap(blockIdx.x, gridDim.x) / tiles;
   const int nk = (p->K + 31) / 32, steps = nk * p->Z, per = (steps + p->slices - 1) / p->slices;
   const int s0 = sl * per, s1 = s0 + per < steps ? s0 + per : steps;
+  const long terms = 32l * (s1 - s0);
 #pragma unroll 1
-  for (int i = lane; i < WR * WN; i += 64) {
-    const int r = TR ? i % WR : i / WN, q = TR ? i / WR : i % WN, m = mw + r, n = nw + q;
-    float* const v = sw + (TR ? q * LD + r : r * LD + q);
-    if (m >= p->M || n >= p->N || *v * 0.0f == 0.0f) continue;
-    const int nb = n / p->nper;
-    const float* a = p->A + (long)m * p->sam;
-    const float* b = p->B + ((long)nb * p->sbb + (long)(n - nb * p->nper) * p->sbn);
-    float t = 0.0f;
+  for (int base = 0; base < WR * WN; base += 64) {
+    auto row = [](int i) { return TR ? i % WR : i / WN; };
+    auto col = [](int i) { return TR ? i / WR : i % WN; };
+    auto at = [&](int i) { return sw + (TR ? col(i) * LD + row(i) : row(i) * LD + col(i)); };
+    const int own = base + lane;
+    const bool bad = mw + row(own) < p->M && nw + col(own) < p->N && !(*at(own) * 0.0f == 0.0f);
+    unsigned long long left = __ballot(bad);
+    const bool few = __popcll(left) <= 8;
 #pragma unroll 1
-    for (int s = s0; s < s1 && t == t; ++s) {
-      const int z = s / nk, k0 = (s - z * nk) * 32, k1 = min(k0 + 32, p->K);
+    while (left) {                                          // (uniform; at most eight turns)
+      const int i = few ? base + __ffsll(left) - 1 : own, step = few ? 256 : 4;
+      left = few ? left & (left - 1) : 0;
+      const int m = min(mw + row(i), p->M - 1), n = min(nw + col(i), p->N - 1), nb = n / p->nper;
+      const float* a = p->A + (long)m * p->sam;
+      const float* b = p->B + ((long)nb * p->sbb + (long)(n - nb * p->nper) * p->sbn);
+      float sum = 0.0f;
 #pragma unroll 1
-      for (int k = k0; k < k1; ++k) t = fmaf(a[(long)z * p->saz + (long)k * p->sak], b[(long)z * p->sbz + (long)k * p->sbk], t);
+      for (long t = few ? 4 * lane : bad ? 0 : terms; t < terms && sum == sum; t += step) {
+        const int s = s0 + (int)(t >> 5), z = s / nk, k = (s - z * nk) * 32 + (int)(t & 31);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const long kk = min(k + j, p->K - 1);
+          const float f = fmaf(a[z * p->saz + kk * p->sak], b[z * p->sbz + kk * p->sbk], sum);
+          sum = k + j < p->K ? f : sum;
+        }
+      }
+      if (few) {
+#pragma unroll
+        for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o);
+        if (lane == 0) *at(i) = sum;
+      } else if (bad) {
+        *at(i) = sum;
+      }
     }
-    *v = t;
   }
 }
 

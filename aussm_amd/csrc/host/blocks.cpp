@@ -4,7 +4,12 @@
 // Activations stay channel rows (b, d, l) between the two projections, whose products read and write that layout
 // themselves, so nothing is transposed, and what the reference does between two layers - bias, softplus, SiLU, gate,
 // residual - happens inside the kernel of one of them.  The forward pass of a block is 8-9 launches, the backward pass
-// 12-14, without Python or a framework operator between them.
+// 16-17 (AUSSM) or 12-13 (Mamba), without Python or a framework operator between them; of a block that is trained in part it
+// runs as far down as a gradient is wanted.
+//
+// The kernels' gradients are not differentiable themselves.  A backward pass that needs more than their values (create_graph,
+// vmap, tangents) recomputes the block from differentiable operators, the scan operators of this library among them:
+// what they refuse, the block refuses.
 #include "common.h"
 #include "host.h"
 

@@ -442,7 +442,7 @@ int aussm_zero_f32(float* p, size_t n, void* stream);
  * The phase tensor theta (b, d, n, L) is never stored: the forward call forms it tile by tile on
  * the matrix cores inside the scan kernel.  The backward call recomputes from the twelve inputs,
  * as the reference does, and needs the phase adjoints of a few batch elements at a time (for the
- * product that sums over all channels); they live in the workspace, at most about 50 MiB.
+ * product that sums over all channels); they live in the workspace, at most about 100 MiB.
  * Limits: n <= 64, d <= 512 (AUSSM_E_SHAPE beyond).  L is arbitrary (the reference needs a
  * multiple of 16 and pads).  `workspace` holds aussm_ssm_adaptive_unitary_workspace_floats(...)
  * floats, 16-byte aligned; nothing in it has to be initialised, nothing in it is kept between calls.
