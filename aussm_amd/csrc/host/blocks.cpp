@@ -150,6 +150,8 @@ variable_list recorded_gradients(SavingNode& node, std::mutex& m, int count, con
   }
   const bool record = at::GradMode::is_enabled();
   at::AutoGradMode with_graph(true);
+  // (the forward pass was in fp32, whatever the backward pass is called under)
+  c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
   std::vector<int> at;
   for (int i = 0; i < count; ++i) {
     if (!in[i].defined() || !in[i].requires_grad()) continue;

@@ -129,6 +129,20 @@ def test_linear_layer_is_twice_differentiable(norm):
         torch.testing.assert_close(a.cpu().double() / scale, w / scale, atol=1e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("kind", ["a", "m"])
+def test_recorded_backward_under_autocast_stays_in_fp32(kind):
+    from aussm_amd import blocks
+    torch.manual_seed(5)
+    args = blocks.ModelArgsSSMau(24, 4) if kind == "a" else blocks.ModelArgsMamba(24, 4)
+    net = blocks.ResidualBlock(args).cuda()
+    x, w = torch.randn(2, 40, 24, device="cuda"), list(net.parameters())
+    want = torch.autograd.grad(net(x).square().mean(), w)
+    loss = net(x).square().mean()
+    with torch.autocast("cuda", torch.bfloat16):
+        got = torch.autograd.grad(loss, w, create_graph=True)
+    _close(got, want)
+
+
 def test_one_tensor_as_two_inputs_of_a_block_counts_once(monkeypatch):
     """Recorded gradients where two weights of a block are one tensor and the input depends on a third."""
     from aussm_amd import blocks
