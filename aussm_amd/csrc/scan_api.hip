@@ -84,6 +84,7 @@ constexpr int SPLIT_MIN_WGS = 129;     // launches of at least this many workgro
 constexpr int SPLIT_TARGET_WGS = 256;
 constexpr int SPLIT_MAX = 32;
 constexpr int SPLIT_MIN_LEN = 128;
+constexpr int GSPLIT_MAX = 64;         // segments of unequal runs of blocks, of the vector-ALU kernels' split
 inline bool matrix_shape(int N, int L, int ck) { return N <= XN && L % 4 == 0 && ck >= XT && ck % XT == 0; }
 inline int seg_capacity(int B, int D, int N, int L, int ck) {
   if (N < MATRIX_MIN_STATE || !matrix_shape(N, L, ck) || L % ck != 0) return 1;
@@ -92,13 +93,6 @@ inline int seg_capacity(int B, int D, int N, int L, int ck) {
   const int nblk = L / ck, target = (int)(SPLIT_TARGET_WGS / wgs);
   int ns = 1;
   while (ns * 2 <= target && ns * 2 <= SPLIT_MAX && nblk % (ns * 2) == 0 && L / (ns * 2) >= SPLIT_MIN_LEN) ns *= 2;
-  return ns;
-}
-inline int seg_count(int B, int D, int N, int L, int ck) {
-  int ns = seg_capacity(B, D, N, L, ck);
-  const int cap = opt(AUSSM_OPT_SPLIT_CAP);
-  if (cap >= 0)
-    while (ns > 1 && ns > cap) ns /= 2;
   return ns;
 }
 // The segment states are computed on finer segments than the scan proper uses (the kernel that
@@ -110,13 +104,44 @@ inline int seg_fine(int L, int ns) {
     if (Ls % (r * XT) == 0 && Ls / r >= SPLIT_MIN_LEN) return r;
   return 1;
 }
+// Segments of a call on the matrix-core kernels: ns of ls steps (whole checkpoint blocks, the last one possibly shorter),
+// each of r fine ones, nf fine ones per sequence.  Sequences that halve into equal segments do so (seg_capacity).  Others -
+// a length that is no multiple of the checkpoint interval, a number of blocks that is no power of two - take as many equal
+// runs of blocks as bring the launch near one workgroup per compute unit, where that makes at least twice as many segments;
+// their fine segments are the segments, so that the states fit the area the vector-ALU kernels' split needs
+// (generic_split: as many segments or more).  B6 D28 N16 L11312, bf16, training pass: 1918 us on 6 workgroups.
+struct USplit { int ns, ls, r, nf; };
+// room: floats there are for the states of unequal segments.
+inline USplit unitary_split(int B, int D, int N, int L, int ck, bool use_cap, size_t room = ~(size_t)0) {
+  const USplit whole{1, L, 1, 1};
+  const int cap = use_cap ? opt(AUSSM_OPT_SPLIT_CAP) : -1;
+  if (cap == 0 || cap == 1 || N < MATRIX_MIN_STATE || !matrix_shape(N, L, ck)) return whole;
+  int ns = seg_capacity(B, D, N, L, ck);
+  const int fine = ns * seg_fine(L, ns);
+  if (cap > 1)
+    while (ns > 1 && ns > cap) ns /= 2;
+  const long long wgs = (long long)B * ((D + CH - 1) / CH);
+  if (wgs < SPLIT_MIN_WGS && L >= 4 * SPLIT_MIN_LEN) {
+    const int nblk = (L + ck - 1) / ck;
+    int want = (int)(SPLIT_TARGET_WGS / wgs);
+    if (want > GSPLIT_MAX) want = GSPLIT_MAX;
+    if (cap > 1 && want > cap) want = cap;
+    int bps = (nblk + want - 1) / want;
+    if (bps * ck < SPLIT_MIN_LEN) bps = (SPLIT_MIN_LEN + ck - 1) / ck;
+    const int nr = (nblk + bps - 1) / bps;
+    if (nr >= 2 * ns && (size_t)B * nr * D * (2 * N + 2) <= room) return USplit{nr, bps * ck, 1, nr};
+  }
+  if (ns <= 1) return whole;
+  int r = seg_fine(L, ns);
+  while (r > 1 && ns * r > fine) r /= 2;      // (fewer segments by option: no more fine ones than the area is sized for)
+  return USplit{ns, L / ns, r, ns * r};
+}
 inline size_t round64(size_t n) { return (n + 63) & ~(size_t)63; }
 inline size_t seg_floats(int B, int D, int N, int L, int ns) {
   return ns > 1 ? round64((size_t)B * ns * seg_fine(L, ns) * D * (2 * N + 2)) : 0;
 }
 // The complex and the real scan split the same way (scan_seg_generic.h) when the call brings a workspace:
 // ns segments of ls steps (whole tiles and checkpoint blocks), the last one possibly shorter.
-constexpr int GSPLIT_MAX = 64;
 struct GSplit { int ns, ls; };
 inline GSplit generic_split(int B, int D, int L, int ck, bool use_cap) {
   const long long wgs = (long long)B * ((D + CH - 1) / CH);
@@ -169,14 +194,15 @@ inline size_t aux_seg_floats(int B, int D, int N, int L, int ck) {
   const size_t m = seg_floats(B, D, N, L, seg_capacity(B, D, N, L, ck)), g = generic_split_floats(VAR_COMPLEX, B, D, N, L, ck);
   return m > g ? m : g;
 }
-struct AuxLayout { float* seg; u4* img; u4* fimg; uint32_t* stamp; float* pad; float* gseg; };
+struct AuxLayout { float* seg; u4* img; u4* fimg; uint32_t* stamp; float* pad; float* gseg; size_t seg_room; };
 inline AuxLayout aux_layout(float* aux, int B, int D, int N, int L, int ck) {
-  if (!aux) return AuxLayout{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  if (!aux) return AuxLayout{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
   float* pad = aux + aux_im_floats(B, D, N, L, ck);
   float* seg = pad + AUX_PAD;
   u4* img = reinterpret_cast<u4*>(seg + aux_seg_floats(B, D, N, L, ck));
-  if (!img_floats(B, N, L, ck)) return AuxLayout{seg, nullptr, nullptr, nullptr, pad, seg};
-  return AuxLayout{seg, img, img + img_chunks(B, L) * PXB_REC, reinterpret_cast<uint32_t*>(pad) + AUX_IMG_FP, pad, seg};
+  if (!img_floats(B, N, L, ck)) return AuxLayout{seg, nullptr, nullptr, nullptr, pad, seg, aux_seg_floats(B, D, N, L, ck)};
+  return AuxLayout{seg, img, img + img_chunks(B, L) * PXB_REC, reinterpret_cast<uint32_t*>(pad) + AUX_IMG_FP, pad, seg,
+                   aux_seg_floats(B, D, N, L, ck)};
 }
 
 // Kernel family of a call whose tensors are 16-byte aligned: 0 vector ALU, 2 / 3 / 5 matrix-core kernels
@@ -240,17 +266,16 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
   }
   const int B = a.B, L = a.L;
   if ((mode == 2 || mode == 3 || mode == 6) && ws.seg) {
-    const int ns = seg_count(B, a.D, a.N, L, a.ck);
-    if (ns > 1) {
+    const USplit sp = unitary_split(B, a.D, a.N, L, a.ck, true, ws.seg_room);
+    if (sp.ns > 1) {
       // 1. end state of every segment from a zero start and its rotation; 2. chain them;
       // 3. the scan proper over (batch, segment) pairs, each from its true incoming state
-      const int Ls = L / ns, r = seg_fine(L, ns), nf = ns * r;
       float* seg = ws.seg;
-      float* ptot = seg + (size_t)B * nf * a.D * a.N * 2;
-      SegArgs sa{a.delta, a.u, a.theta, a.Bm, seg, ptot, a.D, a.N, Ls / r, L, nf, a.ncg};
-      if (int e = run_seg_state(false, sa, in_dtype, (unsigned)(B * nf * a.ncg), s)) return e;
-      if (int e = run_seg_carry_fwd(seg, ptot, a.h0, a.hL, B, a.D, a.N, nf, s)) return e;
-      a.B = B * ns; a.L = Ls; a.ns = ns; a.nck = Ls / a.ck; a.h0 = seg; a.hL = nullptr; a.hs = r; a.ho = 0;
+      float* ptot = seg + (size_t)B * sp.nf * a.D * a.N * 2;
+      SegArgs sa{a.delta, a.u, a.theta, a.Bm, seg, ptot, a.D, a.N, sp.ls / sp.r, L, sp.nf, a.ncg};
+      if (int e = run_seg_state(false, sa, in_dtype, (unsigned)(B * sp.nf * a.ncg), s)) return e;
+      if (int e = run_seg_carry_fwd(seg, ptot, a.h0, a.hL, B, a.D, a.N, sp.nf, s)) return e;
+      a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.h0 = seg; a.hL = nullptr; a.hs = sp.r; a.ho = 0; a.nf = sp.nf;
     }
   }
   if (mode == 6) {
@@ -380,7 +405,7 @@ int aussm_bwd_checkpoint_interval(int variant) { return variant == VAR_UNITARY ?
 
 int aussm_unitary_split_segments(int B, int D, int N, int L, int ck) {
   if (B < 1 || D < 1 || N < 1 || L < 1 || ck < 1) return 0;
-  int ns = seg_capacity(B, D, N, L, ck);
+  int ns = unitary_split(B, D, N, L, ck, false).ns;
   // shapes that the vector-ALU kernels serve by default split their way
   if (!(matrix_shape(N, L, ck) && N >= MATRIX_MIN_STATE)) {
     const int g = generic_split(B, D, L, ck, false).ns;
@@ -435,7 +460,7 @@ int aussm_unitary_fwd_aux(const void* u, const void* delta, const float* theta, 
   a.u = u; a.delta = delta; a.theta = theta; a.Bm = Bc; a.Cm = Cc; a.Dskip = Dskip; a.z = z;
   a.h0 = h0; a.y = y; a.hL = hL; a.hck = hck; a.aux = aux;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.urep = urep;
+  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = urep;
   a.auxtag = aux_tag(u, delta, theta, Bc, Cc, B, D, N, L, in_dtype);
   return launch_unitary_fwd(a, in_dtype, (hipStream_t)stream, aux_layout(aux, B, D, N, L, ck));
 }
@@ -454,8 +479,10 @@ int aussm_unitary_fwd_static(const void* u, const void* delta, const float* thet
   if (misaligned(Bc, ca) || misaligned(Cc, ca)) return AUSSM_E_ALIGN;
   // the only workspace a forward call without checkpoints uses: the segment states of a launch
   // that is split along L
-  const size_t need = seg_floats(B, D, N, L, seg_capacity(B, D, N, L, ck));
+  size_t need = seg_floats(B, D, N, L, seg_capacity(B, D, N, L, ck));
   if (need > STATIC_SCRATCH_FLOATS) return AUSSM_E_SCRATCH;
+  // (unequal segments are taken only where their states fit: such a call is not refused)
+  if (unitary_split(B, D, N, L, ck, false, STATIC_SCRATCH_FLOATS).ns > 1) need = STATIC_SCRATCH_FLOATS;
   float* scratch = nullptr;
   if (need > 0)
     if (int e = static_scratch(&scratch)) return e;
@@ -463,11 +490,11 @@ int aussm_unitary_fwd_static(const void* u, const void* delta, const float* thet
   a.u = u; a.delta = delta; a.theta = theta; a.Bm = Bc; a.Cm = Cc; a.Dskip = Dskip; a.z = z;
   a.h0 = h0; a.y = y; a.hL = hL; a.hck = nullptr; a.aux = nullptr;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.urep = 1;
+  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = 1;
   // (every segment state the scan reads is written earlier in the same call: nothing in the
   // scratch has to start at zero)
   // (the vector-ALU kernels do not split here: no gseg)
-  return launch_unitary_fwd(a, in_dtype, (hipStream_t)stream, AuxLayout{scratch, nullptr, nullptr, nullptr, nullptr, nullptr});
+  return launch_unitary_fwd(a, in_dtype, (hipStream_t)stream, AuxLayout{scratch, nullptr, nullptr, nullptr, nullptr, nullptr, STATIC_SCRATCH_FLOATS});
 }
 
 int aussm_complex_fwd(const void* u, const void* delta, const float* rho, const float* theta, const void* Bc,
@@ -481,7 +508,7 @@ int aussm_complex_fwd(const void* u, const void* delta, const float* rho, const 
   a.u = u; a.delta = delta; a.rho = rho; a.theta = theta; a.Bm = Bc; a.Cm = Cc; a.Dskip = Dskip; a.z = z;
   a.h0 = h0; a.y = y; a.hL = hL; a.hck = hck;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.urep = 1;
+  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = 1;
   return launch_generic_fwd(VAR_COMPLEX, a, in_dtype, workspace, (hipStream_t)stream);
 }
 
@@ -513,7 +540,7 @@ int aussm_real_fwd_rows(const void* u, const void* delta, const float* A, const 
   if (int e = real_rows_check(rows, D, N, in_dtype)) return e;
   if (rows) { a.zrows = rows->z_rows; a.bcrows = rows->bc_rows; a.u_act = rows->u_silu; }
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.urep = 1;
+  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = 1;
   return launch_generic_fwd(VAR_REAL, a, in_dtype, workspace, (hipStream_t)stream);
 }
 
@@ -542,7 +569,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
   a.dy = dy; a.dhL = dhL; a.u = u; a.delta = delta; a.theta = theta; a.Bm = Bc; a.Cm = Cc; a.Dskip = Dskip;
   a.hck = hck; a.aux = aux; a.du = du; a.ddelta = ddelta; a.dtheta = dtheta; a.dB = dB; a.dC = dC; a.dD = dD; a.dh0 = dh0;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.urep = 1;
+  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = 1;
   a.urep = urep;
   a.g16 = g16 && in_dtype == AUSSM_BF16;
   a.auxtag = aux_tag(u, delta, theta, Bc, Cc, B, D, N, L, in_dtype);
@@ -552,17 +579,16 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
       !(misaligned(dy, 16) || misaligned(u, 16) || misaligned(delta, 16) || misaligned(theta, 16) ||
         misaligned(du, 16) || misaligned(ddelta, 16) || misaligned(dtheta, 16) || misaligned(Bc, 16) ||
         misaligned(Cc, 16))) {
-    const int ns = aux ? seg_count(B, D, N, L, ck) : 1;
-    if (ns > 1) {
+    const USplit sp = aux ? unitary_split(B, D, N, L, ck, true, ws.seg_room) : USplit{1, L, 1, 1};
+    if (sp.ns > 1) {
       // adjoint at the start of every segment from a zero adjoint at its end, chained last to first
-      const int Ls = L / ns, r = seg_fine(L, ns), nf = ns * r;
       float* seg = ws.seg;
-      float* ptot = seg + (size_t)B * nf * D * N * 2;
-      SegArgs sa{dy, nullptr, theta, Cc, seg, ptot, D, N, Ls / r, L, nf, a.ncg};
-      if (int e = run_seg_state(true, sa, in_dtype, (unsigned)(B * nf * a.ncg), s)) return e;
-      if (int e = run_seg_carry_bwd(seg, ptot, dhL, dh0, B, D, N, nf, s)) return e;
+      float* ptot = seg + (size_t)B * sp.nf * D * N * 2;
+      SegArgs sa{dy, nullptr, theta, Cc, seg, ptot, D, N, sp.ls / sp.r, L, sp.nf, a.ncg};
+      if (int e = run_seg_state(true, sa, in_dtype, (unsigned)(B * sp.nf * a.ncg), s)) return e;
+      if (int e = run_seg_carry_bwd(seg, ptot, dhL, dh0, B, D, N, sp.nf, s)) return e;
       // a segment of the scan ends where its last fine segment ends
-      a.B = B * ns; a.L = Ls; a.ns = ns; a.nck = Ls / ck; a.dhL = seg; a.dh0 = nullptr; a.hs = r; a.ho = r - 1;
+      a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.dhL = seg; a.dh0 = nullptr; a.hs = sp.r; a.ho = sp.r - 1; a.nf = sp.nf;
     }
     if (mode == 6) {
       // The prepared-operand kernel needs Im(P S) from the forward call in the auxiliary buffer; its

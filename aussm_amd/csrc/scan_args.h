@@ -57,10 +57,11 @@ struct FwdArgs {
                             // (complex: re, im; real: the sum of delta after bias / softplus, 0)
   int B, D, N, L, ck, nck, ncg, delta_softplus;
   int ld, ns;                // row stride of the [.., L] tensors and segments per sequence: B then counts
-                             // (batch, segment) pairs and L is the segment length.  The vector-ALU kernels take a
-                             // shorter last segment (ld not a multiple of L) and keep nck = checkpoints of a whole
-                             // sequence; h0 / hL / ptot are indexed by the pair
-  int hs, ho;                // matrix-core kernels: h0 of pair b is entry b * hs + ho of the state array
+                             // (batch, segment) pairs and L is the segment length (the last one may be shorter: ld
+                             // not a multiple of L); nck stays the number of checkpoints of a whole sequence;
+                             // vector-ALU kernels: h0 / hL / ptot are indexed by the pair
+  int hs, ho, nf;            // matrix-core kernels: h0 of segment sg of batch element bb is entry bb * nf + min(sg * hs + ho,
+                             // nf - 1) of the state array (nf entries per batch element)
   int urep;                  // generic kernels: u and delta are [B / urep, D, L], shared by urep consecutive batch elements
   uint32_t auxtag;           // what a kernel that fills aux writes behind it (aux_tag of the call)
   // vector-ALU kernels: rows per batch element of the tensors z and B_t / C_t lie in (0: D and N, tensors of their own),
@@ -84,8 +85,8 @@ struct UniBwdArgs {
   float* dD;            // [D] or null, accumulated into
   float* dh0;           // [B,D,N,2] or null
   int B, D, N, L, ck, nck, ncg;
-  int ld, ns;           // matrix-core kernel: row stride of the [.., L] tensors, segments per sequence
-  int hs, ho;           // ... and dhL of (batch, segment) pair b is entry b * hs + ho of the adjoint array
+  int ld, ns;           // row stride of the [.., L] tensors, segments per sequence (as FwdArgs)
+  int hs, ho, nf;       // ... and which entry of the adjoint array is a pair's dhL (as FwdArgs)
   int urep;             // generic kernel: u and delta are [B / urep, D, L], shared by urep consecutive batch elements
   int tag_mode;         // matrix-core kernels: 0 use the auxiliary buffer if its tag is valid; 1 leave at once
                         // unless it is; 2 leave at once if it is
@@ -154,7 +155,7 @@ struct SegArgs {
   const void* M;        // forward: B_t, adjoint: C_t (Tin)            [B, N, ld, 2]
   float* out;           // Z or Y                             [B * ns, D, N, 2]
   float* ptot;          // rotation of the segment            [B * ns, D, 2]
-  int D, N, L, ld, ns, ncg;   // L: segment length
+  int D, N, L, ld, ns, ncg;   // L: segment length (the last one may be shorter)
 };
 
 // Prepared operands ("images") of the matrix-core kernels, in 16-byte records per (batch, chunk)

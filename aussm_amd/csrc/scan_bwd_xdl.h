@@ -158,14 +158,15 @@ __global__ __launch_bounds__(256) void unitary_bwd_xdl_kernel(const UniBwdArgs p
   const int b = wg / p.ncg, d0 = (wg % p.ncg) * CH;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int dl = lane & 15, g = lane >> 4;
-  const int D = p.D, N = p.N, L = p.L;
+  const int D = p.D, N = p.N;
   const int d = d0 + wave * 16 + dl;
   const bool dok = d < D;
   const int dc = dok ? d : D - 1;
-  // b counts (batch element, segment of L steps) pairs when the launcher has split the sequence:
-  // states and checkpoints are indexed by b, the [.., ld] tensors by (bb, segment offset so)
-  const int bb = b / p.ns;
-  const size_t so = (size_t)(b - bb * p.ns) * L;
+  // b counts (batch element, segment of p.L steps) pairs when the launcher has split the sequence; the last segment may
+  // be shorter
+  const int bb = b / p.ns, sg = b - bb * p.ns;
+  const size_t so = (size_t)sg * p.L;
+  const int L = p.ld - (int)so < p.L ? p.ld - (int)so : p.L;
   const size_t row = ((size_t)bb * D + dc) * p.ld + so;
   const Tin* __restrict__ gu = static_cast<const Tin*>(p.u) + row;
   const Tin* __restrict__ gdl = static_cast<const Tin*>(p.delta) + row;
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(256) void unitary_bwd_xdl_kernel(const UniBwdArgs p
   constexpr int NPA = sizeof(Tin) == 2 ? 1 : NP, NPAC = sizeof(Tin) == 2 ? 1 : NPC;
   // Im(P_t S_t) left by the forward kernel (if it filled the buffer): saves recomputing S here
   const bool use_phi = p.aux != nullptr &&
-      __builtin_amdgcn_readfirstlane(__float_as_uint(p.aux[(size_t)p.B * D * L])) == p.auxtag;
+      __builtin_amdgcn_readfirstlane(__float_as_uint(p.aux[(size_t)(p.B / p.ns) * D * p.ld])) == p.auxtag;
   if (p.tag_mode == 2 && use_phi) return;      // the kernel that needs the buffer's contents has done the work
   // (always a valid address: the load below is unconditional, its result unused without the tag)
   const float* __restrict__ gph = use_phi ? p.aux + row : gth;
@@ -355,12 +356,12 @@ __global__ __launch_bounds__(256) void unitary_bwd_xdl_kernel(const UniBwdArgs p
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int n = 4 * g + i;
-    ck_row[i] = p.hck + ((((size_t)b * p.nck) * N + (n < N ? n : 0)) * 2) * D + dc;
+    ck_row[i] = p.hck + ((((size_t)bb * p.nck + sg * (p.L / p.ck)) * N + (n < N ? n : 0)) * 2) * D + dc;
   }
   const size_t ck_stride = (size_t)N * 2 * D;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {                      // the state at the end of the sequence
-    const size_t o = (size_t)(p.nck - 1) * ck_stride;
+    const size_t o = (size_t)((L + p.ck - 1) / p.ck - 1) * ck_stride;
     const float vr = ck_row[i][o], vi = ck_row[i][o + D];
     Hr[i] = 4 * g + i < N ? vr : 0.0f;
     Hi[i] = 4 * g + i < N ? vi : 0.0f;
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(256) void unitary_bwd_xdl_kernel(const UniBwdArgs p
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
       if (n < N) {
-        const size_t o = ((((size_t)b * p.hs + p.ho) * D + d) * N + n) * 2;
+        const size_t o = ((seg_entry(bb, sg, p) * D + d) * N + n) * 2;
         Ar[i] = p.dhL[o];
         Ai[i] = p.dhL[o + 1];
       }

@@ -39,6 +39,13 @@ typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 
 
+// entry of the array of segment states (or adjoints) that segment sg of batch element bb starts from
+template <typename Args>
+__device__ __forceinline__ size_t seg_entry(int bb, int sg, const Args& p) {
+  const int e = sg * p.hs + p.ho;
+  return (size_t)bb * p.nf + (e < p.nf ? e : p.nf - 1);
+}
+
 __device__ __forceinline__ f4 xdl(const u4& a, const u4& b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8v, a), __builtin_bit_cast(bf8v, b), c, 0, 0, 0);
 }
@@ -221,14 +228,15 @@ __global__ __launch_bounds__(256) void unitary_fwd_xdl_kernel(const FwdArgs p) {
   const int b = wg / p.ncg, d0 = (wg % p.ncg) * CH;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int dl = lane & 15, g = lane >> 4;
-  const int D = p.D, N = p.N, L = p.L;
+  const int D = p.D, N = p.N;
   const int d = d0 + wave * 16 + dl;
   const bool dok = d < D;
   const int dc = dok ? d : D - 1;
-  // b counts (batch element, segment of L steps) pairs when the launcher has split the sequence:
-  // states and checkpoints are indexed by b, the [.., ld] tensors by (bb, segment offset so)
-  const int bb = b / p.ns;
-  const size_t so = (size_t)(b - bb * p.ns) * L;
+  // b counts (batch element, segment of p.L steps) pairs when the launcher has split the sequence; the last segment may
+  // be shorter
+  const int bb = b / p.ns, sg = b - bb * p.ns;
+  const size_t so = (size_t)sg * p.L;
+  const int L = p.ld - (int)so < p.L ? p.ld - (int)so : p.L;
   const size_t row = ((size_t)bb * D + dc) * p.ld + so;
   const Tin* __restrict__ gu = static_cast<const Tin*>(p.u) + row;
   const Tin* __restrict__ gdl = static_cast<const Tin*>(p.delta) + row;
@@ -440,7 +448,7 @@ __global__ __launch_bounds__(256) void unitary_fwd_xdl_kernel(const FwdArgs p) {
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
       if (n < N) {
-        const size_t o = ((((size_t)b * p.hs + p.ho) * D + d) * N + n) * 2;
+        const size_t o = ((seg_entry(bb, sg, p) * D + d) * N + n) * 2;
         Hr[i] = p.h0[o];
         Hi[i] = p.h0[o + 1];
       }
@@ -451,7 +459,7 @@ __global__ __launch_bounds__(256) void unitary_fwd_xdl_kernel(const FwdArgs p) {
   const int ck_chunks = p.ck / XT;
   int ck_left = ck_chunks;           // chunks to the next checkpoint
   // this lane's rows n = 4 g .. 4 g + 3 of checkpoint 0; one checkpoint further = N * 2 * D floats
-  float* __restrict__ hck_ptr = p.hck ? p.hck + (((size_t)b * p.nck * N + 4 * g) * 2) * D + dc : nullptr;
+  float* __restrict__ hck_ptr = p.hck ? p.hck + ((((size_t)bb * p.nck + sg * (p.L / p.ck)) * N + 4 * g) * 2) * D + dc : nullptr;
   const size_t hck_stride = (size_t)N * 2 * D;
 
   // One chunk.  pc: vector work of chunk c (ready); pn: receives that of chunk c + 1, computed from
@@ -725,7 +733,7 @@ __global__ __launch_bounds__(256) void unitary_fwd_xdl_kernel(const FwdArgs p) {
     step(c + 1, inB, inA, P1, P0);
   }
 
-  if (p.aux && blockIdx.x == 0 && tid == 0) p.aux[(size_t)p.B * D * L] = __uint_as_float(p.auxtag);
+  if (p.aux && blockIdx.x == 0 && tid == 0) p.aux[(size_t)(p.B / p.ns) * D * p.ld] = __uint_as_float(p.auxtag);
   if (p.hL && dok) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

@@ -263,12 +263,13 @@ __global__ __launch_bounds__(512) void unitary_fwd_px_kernel(const FwdArgs p, co
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int cg = wave & 3, hf = wave >> 2;
   const int dl = lane & 15, g = lane >> 4;
-  const int D = p.D, N = p.N, L = p.L;
+  const int D = p.D, N = p.N;
   const int d = d0 + cg * 16 + dl;
   const bool dok = d < D;
   const int dc = dok ? d : D - 1;
-  const int bb = b / p.ns;
-  const size_t so = (size_t)(b - bb * p.ns) * L;
+  const int bb = b / p.ns, sg = b - bb * p.ns;              // (batch element, segment): the last segment may be shorter
+  const size_t so = (size_t)sg * p.L;
+  const int L = p.ld - (int)so < p.L ? p.ld - (int)so : p.L;
   const size_t row = ((size_t)bb * D + dc) * p.ld + so;
   const Tin* __restrict__ gu = static_cast<const Tin*>(p.u) + row;
   const Tin* __restrict__ gdl = static_cast<const Tin*>(p.delta) + row;
@@ -401,7 +402,7 @@ __global__ __launch_bounds__(512) void unitary_fwd_px_kernel(const FwdArgs p, co
       for (int i = 0; i < 4; ++i) {
         const int n = 4 * g + i;
         if (n < N) {
-          const size_t o = ((((size_t)b * p.hs + p.ho) * D + d) * N + n) * 2;
+          const size_t o = ((seg_entry(bb, sg, p) * D + d) * N + n) * 2;
           hr[i] = p.h0[o];
           hi[i] = p.h0[o + 1];
         }
@@ -499,7 +500,7 @@ __global__ __launch_bounds__(512) void unitary_fwd_px_kernel(const FwdArgs p, co
     s_h[(c + 1) & 1][cg][1][lane] = ni;
     // ---- checkpoint: state at the end of every ck-step block and at the end of the sequence
     if (p.hck && dok && c < nchunks && ((c + 1) % ck_chunks == 0 || c == nchunks - 1)) {
-      float* __restrict__ hp = p.hck + ((((size_t)b * p.nck + c / ck_chunks) * N + 4 * g) * 2) * D + dc;
+      float* __restrict__ hp = p.hck + ((((size_t)bb * p.nck + sg * (p.L / p.ck) + c / ck_chunks) * N + 4 * g) * 2) * D + dc;
 #pragma unroll
       for (int k = 0; k < 4; ++k)
         if (4 * g + k < N) { hp[(size_t)k * 2 * D] = nr[k]; hp[(size_t)k * 2 * D + D] = ni[k]; }
@@ -669,12 +670,13 @@ __global__ __launch_bounds__(512) void unitary_bwd_px_kernel(const UniBwdArgs p,
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int cg = wave & 3, hf = wave >> 2;
   const int dl = lane & 15, g = lane >> 4;
-  const int D = p.D, N = p.N, L = p.L;
+  const int D = p.D, N = p.N;
   const int d = d0 + cg * 16 + dl;
   const bool dok = d < D;
   const int dc = dok ? d : D - 1;
-  const int bb = b / p.ns;
-  const size_t so = (size_t)(b - bb * p.ns) * L;
+  const int bb = b / p.ns, sg = b - bb * p.ns;              // (batch element, segment): the last segment may be shorter
+  const size_t so = (size_t)sg * p.L;
+  const int L = p.ld - (int)so < p.L ? p.ld - (int)so : p.L;
   const size_t row = ((size_t)bb * D + dc) * p.ld + so;
   const size_t tagpos = (size_t)(p.B / p.ns) * D * p.ld;
   if (p.tag_mode == 1 &&
@@ -813,7 +815,7 @@ __global__ __launch_bounds__(512) void unitary_bwd_px_kernel(const UniBwdArgs p,
     const bool ck_here = c > 0 && c % ck_chunks == 0;     // (uniform)
     float ckv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (ck_here) {
-      const float* __restrict__ cp = p.hck + ((size_t)b * p.nck + (c / ck_chunks - 1)) * ck_stride + dc;
+      const float* __restrict__ cp = p.hck + ((size_t)bb * p.nck + sg * (p.L / p.ck) + (c / ck_chunks - 1)) * ck_stride + dc;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int n = 4 * g + i;
@@ -1152,7 +1154,7 @@ __global__ __launch_bounds__(512) void unitary_bwd_px_kernel(const UniBwdArgs p,
   // ---- prologue: end state and its adjoint into the carry, first images, first inputs
   if (hf == 0) {
     f4 hr = {0, 0, 0, 0}, hi = hr, ar = hr, ai = hr;
-    const float* __restrict__ cp = p.hck + ((size_t)b * p.nck + (p.nck - 1)) * ck_stride + dc;
+    const float* __restrict__ cp = p.hck + ((size_t)bb * p.nck + sg * (p.L / p.ck) + ((L + p.ck - 1) / p.ck - 1)) * ck_stride + dc;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
@@ -1160,7 +1162,7 @@ __global__ __launch_bounds__(512) void unitary_bwd_px_kernel(const UniBwdArgs p,
         hr[i] = cp[(size_t)n * 2 * D];
         hi[i] = cp[(size_t)n * 2 * D + D];
         if (p.dhL && dok) {
-          const size_t o = ((((size_t)b * p.hs + p.ho) * D + d) * N + n) * 2;
+          const size_t o = ((seg_entry(bb, sg, p) * D + d) * N + n) * 2;
           ar[i] = p.dhL[o];
           ai[i] = p.dhL[o + 1];
         }

@@ -34,12 +34,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   const int vb = wg / p.ncg, d0 = (wg % p.ncg) * CH;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int dl = lane & 15, g = lane >> 4;
-  const int D = p.D, N = p.N, L = p.L;
+  const int D = p.D, N = p.N;
   const int d = d0 + wave * 16 + dl;
   const bool dok = d < D;
   const int dc = dok ? d : D - 1;
   const int bb = vb / p.ns;
-  const size_t so = (size_t)(vb - bb * p.ns) * L;
+  const size_t so = (size_t)(vb - bb * p.ns) * p.L;
+  const int L = p.ld - (int)so < p.L ? p.ld - (int)so : p.L;   // (the last segment may be shorter)
   const size_t row = ((size_t)bb * D + dc) * p.ld + so;
   using TA = typename std::conditional<ADJ, float, Tin>::type;   // dy is always float
   const TA* __restrict__ gx1 = static_cast<const TA*>(p.x1) + row;

@@ -155,6 +155,22 @@ def test_sequence_split_over_workgroups(B, D, N, L, cap):
         _close(gt, wh.cpu(), k + " (split vs whole)", tol=2e-5)
 
 
+@pytest.mark.parametrize("B,D,N,L,cap", [
+    (1, 40, 16, 1100, None),       # a last segment shorter than the others, its last chunk not full
+    (2, 70, 7, 772, None),         # ... of one run of four steps
+    (1, 64, 16, 1536, None),       # twelve checkpoint blocks: no power of two
+    (2, 64, 16, 1088, "3"),        # fewer segments by option
+    (26, 70, 16, 516, None),       # a launch of 52 workgroups, a last segment of four steps
+])
+def test_sequence_split_into_unequal_segments(B, D, N, L, cap):
+    """Lengths that do not halve into equal segments of whole checkpoint blocks."""
+    from aussm_amd import scan, _lib
+    ck = scan.unitary_ck(B, D, N, L)
+    ns = _lib.load().aussm_unitary_split_segments(B, D, N, L, ck)
+    assert ns > 2 and ns & (ns - 1) or L % (ns * ck) != 0
+    test_sequence_split_over_workgroups(B, D, N, L, cap)
+
+
 @pytest.mark.parametrize("B,D,N,L,force", [
     (1, 64, 32, 1024, False),      # more than 16 states
     (2, 70, 24, 1000, False),      # ... ragged channel group, a last segment shorter than the others
