@@ -26,8 +26,8 @@ LIBNAME = "libaussm_hip.so"
 
 # One translation unit per kernel family: they compile side by side, and a change in one family
 # does not recompile the others' objects by hand (`--only k_px` rebuilds one unit and relinks).
-SOURCES = ["scan_api.hip", "k_fwd.hip", "k_ubwd.hip", "k_rbwd.hip", "k_generic.hip", "k_xdl.hip", "k_px.hip", "k_dropin.hip", "k_gemm.hip",
-           "k_blocks.hip"]
+SOURCES = ["scan_api.hip", "k_oct_fwd.hip", "k_oct_bwd.hip", "k_ubwd.hip", "k_generic.hip", "k_xdl.hip", "k_px.hip", "k_dropin.hip",
+           "k_gemm.hip", "k_blocks.hip"]
 
 # Packed-FP32 instructions are switched off on purpose (see the flag): the kernels are written
 # with scalar float arithmetic only.

@@ -3,31 +3,9 @@
 #include "conv1d.h"
 #include "launch.h"
 #include "layout.h"
-#include "scan_seg_generic.h"
+#include "scan_seg_real.h"
 
 namespace aussm {
-
-int run_adjoint_seg(int variant, const AdjSegArgs& a, int in_dtype, unsigned grid, hipStream_t s) {
-  // (B_t / C_t are float in every instance of the complex and real scans; the complex kernel reads no u / delta
-  // at all.  The unitary scan runs the complex instance without rho, with C_t in the type of its inputs.)
-  if (variant == VAR_UNITARY) {
-    if (in_dtype == 1) hipLaunchKernelGGL((adjoint_seg_kernel<VAR_COMPLEX, float, bf16_t>), dim3(grid), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((adjoint_seg_kernel<VAR_COMPLEX, float, float>), dim3(grid), dim3(256), 0, s, a);
-  } else if (variant == VAR_COMPLEX) {
-    hipLaunchKernelGGL((adjoint_seg_kernel<VAR_COMPLEX, float, float>), dim3(grid), dim3(256), 0, s, a);
-  } else {
-    if (in_dtype) hipLaunchKernelGGL((adjoint_seg_kernel<VAR_REAL, bf16_t, float>), dim3(grid), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((adjoint_seg_kernel<VAR_REAL, float, float>), dim3(grid), dim3(256), 0, s, a);
-  }
-  return launch_status();
-}
-
-int run_bc_to_f32(const void* Bm, const void* Cm, float* oB, float* oC, size_t n, hipStream_t s) {
-  const size_t blocks = (n + 255) / 256;
-  hipLaunchKernelGGL(bc_to_f32_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, s,
-                     static_cast<const bf16_t*>(Bm), static_cast<const bf16_t*>(Cm), oB, oC, n);
-  return launch_status();
-}
 
 int run_seg_carry_real(bool adjoint, float* seg, const float* ptot, const float* A, const float* first, float* last,
                         int B, int D, int N, int ns, hipStream_t s) {

@@ -1,0 +1,44 @@
+// Translation unit of the recomputing reverse scans, complex and real (scan_oct.h).
+#include "launch.h"
+#include "scan_oct.h"
+
+namespace aussm {
+
+// One launch per block of states (stream order makes the later blocks' additions safe): as many groups of eight as the
+// registers for the recomputed states and the slabs in LDS hold - complex 16 states, real 24.
+template <int VAR, typename Tin>
+static int oct_bwd_t(const RecBwdArgs& args, hipStream_t s) {
+  const dim3 grid((unsigned)(args.B * args.ncg)), block(512);
+  constexpr int BLOCK = VAR == VAR_REAL ? 24 : 16;
+  for (int nbase = 0; nbase < args.N; nbase += BLOCK) {
+    RecBwdArgs a = args;
+    a.nbase = nbase;
+    a.accum = nbase > 0;
+    const int left = a.N - nbase, S = left >= BLOCK ? BLOCK / 8 : (left + 7) / 8;
+    auto go = [&](auto sc, auto full) {
+      constexpr int S_ = decltype(sc)::value;
+      constexpr bool F = decltype(full)::value;
+      if (a.z) hipLaunchKernelGGL((oct_bwd_kernel<VAR, S_, F, Tin, Tin, true>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((oct_bwd_kernel<VAR, S_, F, Tin, Tin, false>), grid, block, 0, s, a);
+    };
+    using std::integral_constant;
+    if (S == 1) go(integral_constant<int, 1>{}, std::false_type{});
+    else if (S == 2) {
+      if (left >= 16) go(integral_constant<int, 2>{}, std::true_type{});
+      else go(integral_constant<int, 2>{}, std::false_type{});
+    } else {
+      if constexpr (VAR == VAR_REAL) {
+        go(integral_constant<int, 3>{}, std::false_type{});
+      }
+    }
+    if (int e = launch_status()) return e;
+  }
+  return 0;
+}
+
+int run_oct_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s) {
+  if (variant == VAR_COMPLEX) return in_dtype ? oct_bwd_t<VAR_COMPLEX, bf16_t>(a, s) : oct_bwd_t<VAR_COMPLEX, float>(a, s);
+  return in_dtype ? oct_bwd_t<VAR_REAL, bf16_t>(a, s) : oct_bwd_t<VAR_REAL, float>(a, s);
+}
+
+}  // namespace aussm

@@ -16,21 +16,17 @@ inline int launch_status() {
   return e == hipSuccess ? 0 : (int)e;
 }
 
-// A workgroup of nt threads (nt / 64 wavefronts) of the vector-ALU kernels owns 64 channels; each
-// wavefront owns nw states.
+// A workgroup of nt threads (nt / 64 wavefronts) of unitary_bwd_kernel owns 64 channels; each wavefront owns nw states.
 struct Cfg { int nw, nt; };
 
-// ---- k_fwd.hip, k_ubwd.hip, k_rbwd.hip: vector-ALU scans; k_generic.hip: their split along L, convolution, layout swap
-// in_dtype: 0 float, 1 bf16 (unitary only), 2 = u / delta bf16 and B_t / C_t float (complex and real only, whose
-// kernels take no bf16 B_t / C_t: converted to float once per call)
-constexpr int IN_BF16_BC32 = 2;
-int run_core_fwd(int variant, const FwdArgs& a, int in_dtype, Cfg c, hipStream_t s);
+// ---- k_oct_fwd.hip, k_oct_bwd.hip, k_ubwd.hip: vector-ALU scans; k_generic.hip: chain of the S6 segments, convolution,
+// layout swap.  in_dtype: 0 float, 1 bf16
+int run_oct_fwd(int variant, const FwdArgs& a, int in_dtype, hipStream_t s);
+int run_oct_adj(int variant, const AdjSegArgs& a, int in_dtype, unsigned grid, hipStream_t s);   // adjoint entering every segment
+int run_oct_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s);
 int run_unitary_bwd_generic(const UniBwdArgs& a, int in_dtype, Cfg c, hipStream_t s);
-int run_rec_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s);
 int run_aux_invalidate(float* tag, bool fill_tag, bool images_tag, hipStream_t s);   // clears tag(s) in the buffer's pad
-// split of the complex / real scans along L: adjoint entering every segment, chain of the real scan's segments
-int run_adjoint_seg(int variant, const AdjSegArgs& a, int in_dtype, unsigned grid, hipStream_t s);
-int run_bc_to_f32(const void* Bm, const void* Cm, float* oB, float* oC, size_t n, hipStream_t s);   // bf16 -> float
+// split along L: chain of the real scan's segments
 int run_seg_carry_real(bool adjoint, float* seg, const float* ptot, const float* A, const float* first, float* last,
                         int B, int D, int N, int ns, hipStream_t s);
 int run_hbm_probe(const float* a, const float* b, const float* c, float* o1, float* o2, int rows, int L, int pattern,

@@ -18,7 +18,7 @@ std::atomic<int> g_opt[AUSSM_OPT_COUNT] = {{-1}, {-1}, {-1}, {-1}, {-1}, {-1}};
 static_assert(AUSSM_OPT_COUNT == 6, "one initialiser per option");
 inline int opt(int key) { return g_opt[key].load(std::memory_order_relaxed); }
 
-// ---- configuration of the vector-ALU kernels --------------------------------------------------
+// ---- configuration of unitary_bwd_kernel -------------------------------------------------------
 // The scalar loads of B_t/C_t are issued one "turn" ahead; with two or more wavefronts per SIMD
 // the turn of another wavefront doubles that distance, so for a given N the configuration with
 // MORE wavefronts (smaller NW) is preferred as long as the launch still fits one workgroup.
@@ -51,8 +51,7 @@ inline int check_common(int B, int D, int N, int L, int ck, int in_dtype) {
   return AUSSM_OK;
 }
 
-// The recomputing backward kernels (complex, real) keep a tile of states in registers: four
-// wavefronts of at most four states each.
+// Checkpoint interval of the recomputing backward kernels (complex, real)
 constexpr int REC_CK = AUSSM_TILE / 2;
 
 inline bool misaligned(const void* p, size_t a) { return p && (reinterpret_cast<uintptr_t>(p) % a) != 0; }
@@ -140,7 +139,7 @@ inline size_t round64(size_t n) { return (n + 63) & ~(size_t)63; }
 inline size_t seg_floats(int B, int D, int N, int L, int ns) {
   return ns > 1 ? round64((size_t)B * ns * seg_fine(L, ns) * D * (2 * N + 2)) : 0;
 }
-// The complex and the real scan split the same way (scan_seg_generic.h) when the call brings a workspace:
+// The complex and the real scan split the same way (scan_seg_real.h) when the call brings a workspace:
 // ns segments of ls steps (whole tiles and checkpoint blocks), the last one possibly shorter.
 struct GSplit { int ns, ls; };
 inline GSplit generic_split(int B, int D, int L, int ck, bool use_cap) {
@@ -161,18 +160,10 @@ inline size_t generic_split_floats(int variant, int B, int D, int N, int L, int 
   const int C = variant == VAR_REAL ? 1 : 2;
   return sp.ns > 1 ? round64((size_t)B * sp.ns * D * (N * C + 2)) : 0;
 }
-// ... and their kernels take B_t / C_t as float: bf16 rows are converted once per call, behind the segments
+// (bf16 inputs: the kernels read B_t / C_t as they are; the room for float copies of them stays part of the size that callers
+// allocate by, and of what a call without a workspace is refused for)
 inline size_t generic_bc_floats(int variant, int B, int N, int L, int in_dtype) {
   return in_dtype == AUSSM_BF16 ? round64((size_t)B * N * L * (variant == VAR_REAL ? 1 : 2)) : 0;
-}
-struct BcF32 { const void* Bm; const void* Cm; int in_dtype; int err; };
-inline BcF32 generic_bc(int variant, const void* Bm, const void* Cm, float* ws, int B, int D, int N, int L, int ck,
-                        int in_dtype, hipStream_t s) {
-  if (in_dtype != AUSSM_BF16) return BcF32{Bm, Cm, 0, 0};
-  const size_t n = generic_bc_floats(variant, B, N, L, in_dtype);
-  float* fB = ws + generic_split_floats(variant, B, D, N, L, ck);
-  const int err = run_bc_to_f32(Bm, Cm, fB, fB + n, (size_t)B * N * L * (variant == VAR_REAL ? 1 : 2), s);
-  return BcF32{fB, fB + n, 2, err};
 }
 
 // Workspace of the prepared operands: per (batch element, chunk) one backward image and, behind
@@ -246,7 +237,6 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
   if (!fill) a.aux = nullptr;
   if (!mode) {
     // vector-ALU kernel; with a segment area and few (batch, channel group) pairs, split along the sequence
-    const Cfg cfg = pick_cfg(a.N, 8);
     const GSplit sp = ws.gseg ? generic_split(a.B, a.D, a.L, a.ck, true) : GSplit{1, a.L};
     if (sp.ns > 1) {
       const int B = a.B;
@@ -256,13 +246,13 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
       FwdArgs z = a;
       z.B = B * sp.ns; z.L = sp.ls; z.ns = sp.ns;
       z.y = nullptr; z.z = nullptr; z.Dskip = nullptr; z.h0 = nullptr; z.hL = seg; z.hck = nullptr; z.ptot = ptot;
-      if (int e = run_core_fwd(VAR_UNITARY, z, in_dtype, cfg, s)) return e;
+      if (int e = run_oct_fwd(VAR_UNITARY, z, in_dtype, s)) return e;
       // 2. the state that enters every segment; the state after the last one is the call's hL
       if (int e = run_seg_carry_fwd(seg, ptot, a.h0, a.hL, B, a.D, a.N, sp.ns, s)) return e;
       // 3. the scan proper over (batch, segment) pairs
       a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.h0 = seg; a.hL = nullptr;
     }
-    return run_core_fwd(VAR_UNITARY, a, in_dtype, cfg, s);
+    return run_oct_fwd(VAR_UNITARY, a, in_dtype, s);
   }
   const int B = a.B, L = a.L;
   if ((mode == 2 || mode == 3 || mode == 6) && ws.seg) {
@@ -294,10 +284,6 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
 int launch_generic_fwd(int variant, FwdArgs a, int in_dtype, float* ws, hipStream_t s) {
   if (in_dtype == AUSSM_BF16 && !ws) return AUSSM_E_NULL;
   if (misaligned(ws, 16)) return AUSSM_E_ALIGN;
-  const BcF32 bc = generic_bc(variant, a.Bm, a.Cm, ws, a.B, a.D, a.N, a.L, a.ck, in_dtype, s);
-  if (bc.err) return bc.err;
-  a.Bm = bc.Bm; a.Cm = bc.Cm; in_dtype = bc.in_dtype;
-  const Cfg cfg = pick_cfg(a.N, 8);
   const GSplit sp = ws ? generic_split(a.B, a.D, a.L, a.ck, true) : GSplit{1, a.L};
   if (sp.ns > 1) {
     const int B = a.B, C = variant == VAR_REAL ? 1 : 2;
@@ -307,7 +293,7 @@ int launch_generic_fwd(int variant, FwdArgs a, int in_dtype, float* ws, hipStrea
     FwdArgs z = a;
     z.B = B * sp.ns; z.L = sp.ls; z.ns = sp.ns;
     z.y = nullptr; z.z = nullptr; z.Dskip = nullptr; z.h0 = nullptr; z.hL = seg; z.hck = nullptr; z.ptot = ptot;
-    if (int e = run_core_fwd(variant, z, in_dtype, cfg, s)) return e;
+    if (int e = run_oct_fwd(variant, z, in_dtype, s)) return e;
     // 2. the state that enters every segment; the state after the last one is the call's hL
     if (int e = variant == VAR_COMPLEX ? run_seg_carry_fwd(seg, ptot, a.h0, a.hL, B, a.D, a.N, sp.ns, s)
                                        : run_seg_carry_real(false, seg, ptot, a.A, a.h0, a.hL, B, a.D, a.N, sp.ns, s))
@@ -315,15 +301,12 @@ int launch_generic_fwd(int variant, FwdArgs a, int in_dtype, float* ws, hipStrea
     // 3. the scan proper over (batch, segment) pairs
     a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.h0 = seg; a.hL = nullptr;
   }
-  return run_core_fwd(variant, a, in_dtype, cfg, s);
+  return run_oct_fwd(variant, a, in_dtype, s);
 }
 
 int launch_generic_bwd(int variant, RecBwdArgs a, int in_dtype, float* ws, hipStream_t s) {
   if (in_dtype == AUSSM_BF16 && !ws) return AUSSM_E_NULL;
   if (misaligned(ws, 16)) return AUSSM_E_ALIGN;
-  const BcF32 bc = generic_bc(variant, a.Bm, a.Cm, ws, a.B, a.D, a.N, a.L, REC_CK, in_dtype, s);
-  if (bc.err) return bc.err;
-  a.Bm = bc.Bm; a.Cm = bc.Cm; in_dtype = bc.in_dtype;
   const GSplit sp = ws ? generic_split(a.B, a.D, a.L, REC_CK, true) : GSplit{1, a.L};
   if (sp.ns > 1) {
     const int B = a.B, C = variant == VAR_REAL ? 1 : 2;
@@ -334,13 +317,13 @@ int launch_generic_bwd(int variant, RecBwdArgs a, int in_dtype, float* ws, hipSt
     g.delta_bias = a.delta_bias; g.out = seg; g.ptot = ptot;
     g.D = a.D; g.N = a.N; g.L = sp.ls; g.ld = a.L; g.ns = sp.ns; g.ncg = a.ncg; g.delta_softplus = a.delta_softplus;
     g.zrows = a.zrows; g.bcrows = a.bcrows;
-    if (int e = run_adjoint_seg(variant, g, in_dtype, (unsigned)(B * sp.ns * a.ncg), s)) return e;
+    if (int e = run_oct_adj(variant, g, in_dtype, (unsigned)(B * sp.ns * a.ncg), s)) return e;
     if (int e = variant == VAR_COMPLEX ? run_seg_carry_bwd(seg, ptot, a.dhL, a.dh0, B, a.D, a.N, sp.ns, s)
                                        : run_seg_carry_real(true, seg, ptot, a.A, a.dhL, a.dh0, B, a.D, a.N, sp.ns, s))
       return e;
     a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.dhL = seg; a.dh0 = nullptr;
   }
-  return run_rec_bwd(variant, a, in_dtype, s);
+  return run_oct_bwd(variant, a, in_dtype, s);
 }
 
 // ---- static workspace of aussm_unitary_fwd_static ---------------------------------------------
@@ -618,7 +601,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
     AdjSegArgs g{};
     g.dy = dy; g.theta = theta; g.Cm = Cc; g.out = seg; g.ptot = ptot;
     g.D = D; g.N = N; g.L = sp.ls; g.ld = L; g.ns = sp.ns; g.ncg = a.ncg;
-    if (int e = run_adjoint_seg(VAR_UNITARY, g, in_dtype, (unsigned)(B * sp.ns * a.ncg), s)) return e;
+    if (int e = run_oct_adj(VAR_UNITARY, g, in_dtype, (unsigned)(B * sp.ns * a.ncg), s)) return e;
     if (int e = run_seg_carry_bwd(seg, ptot, dhL, dh0, B, D, N, sp.ns, s)) return e;
     a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.dhL = seg; a.dh0 = nullptr;
   }
@@ -645,7 +628,7 @@ int aussm_complex_bwd(const float* dy, const float* dhL, const void* u, const vo
   a.du = du; a.ddelta = ddelta; a.dtheta = dtheta; a.drho = drho; a.dB = dB; a.dC = dC; a.dD = dD; a.dh0 = dh0;
   if ((z == nullptr) != (dz == nullptr)) return AUSSM_E_NULL;
   a.z = z; a.dz = dz;
-  a.B = B; a.D = D; a.N = N; a.L = L; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
+  a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
   // (several blocks of states add up in du and ddelta: those stay float)
   if (g16 && in_dtype == AUSSM_BF16 && N > 16) return AUSSM_E_DTYPE;
   a.g16 = g16 && in_dtype == AUSSM_BF16;
@@ -684,7 +667,7 @@ int aussm_real_bwd_rows(const float* dy, const float* dhL, const void* u, const 
     a.dbias = rows->ddelta_bias; a.dbias_scale = rows->ddelta_bias_scale;
   }
   a.z = z; a.dz = dz;
-  a.B = B; a.D = D; a.N = N; a.L = L; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
+  a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
   // (several blocks of states add up in du and ddelta: those stay float)
   if (g16 && in_dtype == AUSSM_BF16 && N > 16) return AUSSM_E_DTYPE;
   a.g16 = g16 && in_dtype == AUSSM_BF16;

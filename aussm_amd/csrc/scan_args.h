@@ -116,13 +116,12 @@ struct RecBwdArgs {
   float* dh0;               // [B,D,N,C] or null
   const float* z;           // [B,D,L] or null: the output was gated, y = y_pre silu(z); dy is the gradient of y
   float* dz;                // [B,D,L] (with z)
-  int B, D, N, L, nck, ncg, delta_softplus;
+  int B, D, N, L, ck, nck, ncg, delta_softplus;   // ck: 16
   // Split along the sequence: ld = row stride of the [.., L] tensors (the whole sequence), ns segments per
   // sequence, B counts (batch, segment) pairs, L is the segment length (a multiple of 16; the last segment may
   // be shorter), nck the checkpoints of a whole sequence; dhL / dh0 are indexed by the pair, h0 by the batch element.
   int ld, ns;
-  // A launch handles the states nbase .. nbase + 15 (a workgroup's four wavefronts of up to four states);
-  // larger N takes one launch per block of 16 states.  accum: a later block - the sums over the states
+  // A launch handles a block of states from nbase on (complex 16, real 24); larger N takes one launch per block.  accum: a later block - the sums over the states
   // (du, ddelta, dtheta, drho) are added to what the earlier blocks wrote, and the terms that do not
   // depend on the state (the D skip, dD) are left out.
   int nbase, accum;

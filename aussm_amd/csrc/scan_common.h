@@ -78,9 +78,8 @@ __device__ __forceinline__ float softplusf_(float v) {
 // sin and cos of one argument, about 25 VALU instructions and no branch on the common path.
 // Cody-Waite reduction by pi/2 in three fused steps, then minimax polynomials on [-pi/4, pi/4]
 // (max error ~1 ulp of 1.0 for |x| < 1e4, which covers accumulated phases of practical length).
-// Larger arguments take the library routine.
-__device__ __forceinline__ void fast_sincosf(float x, float* sn, float* cs) {
-  if (__builtin_expect(fabsf(x) > 1.0e4f, 0)) { sincosf(x, sn, cs); return; }
+// Larger arguments take the library routine (fast_sincosf; sincos_1e4 leaves the check to its caller).
+__device__ __forceinline__ void sincos_1e4(float x, float* sn, float* cs) {
   const float kf = rintf(x * 0.636619772367581343f);
   float r = fmaf(-kf, 1.57079637050628662109375f, x);
   r = fmaf(-kf, -4.37113900018624283e-8f, r);
@@ -97,6 +96,10 @@ __device__ __forceinline__ void fast_sincosf(float x, float* sn, float* cs) {
   const float c1 = (q & 1) ? s : c;
   *sn = (q & 2) ? -s1 : s1;
   *cs = ((q + 1) & 2) ? -c1 : c1;
+}
+__device__ __forceinline__ void fast_sincosf(float x, float* sn, float* cs) {
+  if (__builtin_expect(fabsf(x) > 1.0e4f, 0)) sincosf(x, sn, cs);
+  else sincos_1e4(x, sn, cs);
 }
 
 // wave-uniform loads of B_t / C_t.  idx is uniform across the wavefront.  The tensors are inputs

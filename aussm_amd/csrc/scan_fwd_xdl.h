@@ -28,7 +28,6 @@
 // split into pieces) are staged once per workgroup in LDS as 16-byte records [row][g].
 #pragma once
 #include "scan_common.h"
-#include "scan_fwd.h"
 #include <type_traits>
 
 namespace aussm {
