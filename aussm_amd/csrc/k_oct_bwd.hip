@@ -41,4 +41,33 @@ int run_oct_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s) {
   return in_dtype ? oct_bwd_t<VAR_REAL, bf16_t>(a, s) : oct_bwd_t<VAR_REAL, float>(a, s);
 }
 
+// The unitary scan's, up to 32 states in one launch.
+template <typename Tin>
+static int oct_ubwd_t(const RecBwdArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)(a.B * a.ncg)), block(512);
+  auto go = [&](auto sc, auto full) {
+    constexpr int S = decltype(sc)::value;
+    constexpr bool F = decltype(full)::value;
+    hipLaunchKernelGGL((oct_bwd_kernel<VAR_UNITARY, S, F, Tin, Tin, false>), grid, block, 0, s, a);
+  };
+  using std::integral_constant;
+  const int S = (a.N + 7) / 8;
+  if (S == 1) go(integral_constant<int, 1>{}, std::false_type{});
+  else if (S == 2 && a.N == 16) go(integral_constant<int, 2>{}, std::true_type{});
+  else if (S == 2) go(integral_constant<int, 2>{}, std::false_type{});
+  else if (S == 3) go(integral_constant<int, 3>{}, std::false_type{});
+  else if (S == 4) go(integral_constant<int, 4>{}, std::false_type{});
+  else return -2;
+  return launch_status();
+}
+
+int run_oct_ubwd(const UniBwdArgs& u, int in_dtype, hipStream_t s) {
+  RecBwdArgs a{};
+  a.dy = u.dy; a.dhL = u.dhL; a.u = u.u; a.delta = u.delta; a.theta = u.theta; a.Bm = u.Bm; a.Cm = u.Cm; a.Dskip = u.Dskip; a.hck = u.hck;
+  a.du = u.du; a.ddelta = u.ddelta; a.dtheta = u.dtheta; a.dB = u.dB; a.dC = u.dC; a.dD = u.dD; a.dh0 = u.dh0;
+  a.B = u.B; a.D = u.D; a.N = u.N; a.L = u.L; a.ck = u.ck; a.nck = u.nck; a.ncg = u.ncg; a.ld = u.ld; a.ns = u.ns;
+  a.urep = u.urep; a.g16 = u.g16;
+  return in_dtype ? oct_ubwd_t<bf16_t>(a, s) : oct_ubwd_t<float>(a, s);
+}
+
 }  // namespace aussm

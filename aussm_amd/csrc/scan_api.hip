@@ -605,6 +605,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
     if (int e = run_seg_carry_bwd(seg, ptot, dhL, dh0, B, D, N, sp.ns, s)) return e;
     a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.dhL = seg; a.dh0 = nullptr;
   }
+  if (N <= 32) return run_oct_ubwd(a, in_dtype, s);
   return run_unitary_bwd_generic(a, in_dtype, pick_cfg(a.N, 8), s);
 }
 

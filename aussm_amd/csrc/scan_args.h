@@ -129,6 +129,7 @@ struct RecBwdArgs {
   float* dbias;              // [D] or null (real): dbias_scale times the sum of ddelta over (batch, step) is added
   float dbias_scale;
   int g16;                   // du and ddelta leave in bf16 (inputs in bf16, states in one launch)
+  int urep;                  // unitary: u and delta are [B / urep, D, L], shared by urep consecutive batch elements
 };
 
 // Adjoint of the state entering a segment, from a zero adjoint at its end (complex and real scans)

@@ -704,7 +704,7 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
   }
 }
 
-// Reverse scan of the complex and the real (S6) variant.  With |a_l| < 1 the recurrence cannot be run backwards (dividing by
+// Reverse scan.  Complex and real (S6) variant: with |a_l| < 1 the recurrence cannot be run backwards (dividing by
 // a_l amplifies rounding errors without bound): the states of HT steps are recomputed from the checkpoint before them and
 // kept in registers, then the steps are walked backwards with the adjoint state g_l = dLoss/dh_l
 //     g_l = conj(C_l) dy_l + conj(a_{l+1}) g_{l+1},
@@ -715,23 +715,29 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
 //     real:    x = g_l a_l h_{l-1};  dA[d,n] += x delta_l;  ddelta_l = sum_n x A[d,n] + dw_l u_l.
 // Gate: with z given the forward output was y = y_pre silu(z); dy is scaled by silu(z) on the way in, y_pre = sum_n Re(C h) +
 // D u is recomputed with the states, and dz = dy y_pre silu'(z) leaves with the other gradients (GATED).
-// Checkpoints every OH = 16 steps.  States nbase .. nbase + 8 S - 1 (RecBwdArgs).
+// Checkpoints every 16 steps.
+// Unitary variant: |a_l| = 1, the recurrence runs backwards from the checkpoint at the end, h_{l-1} = conj(a_l) (h_l - B_l w_l),
+// and takes every checkpoint it passes (ck a multiple of 32) instead of what it has come to;
+//     dtheta_l = -sum_n Im(conj(g_l) p_l),  p_l = h_l - B_l w_l.
+// 30 vector instructions per state and step, no states kept; B5 D200 N24 L1001 85 -> 68 us.
+// States nbase .. nbase + 8 S - 1 (RecBwdArgs).
 //
-// Time is cut into intervals of 16 steps with one barrier each; 32 steps are staged at a time, at the end of every other
+// Time is cut into intervals of OH steps (16, or 8 where the slabs of more than 16 complex states need the room) with one barrier each; 32 steps are staged at a time, at the end of every other
 // interval.  (Tiles 16 steps apart in the two wavefronts of a SIMD, so that one computes while the other stages: no faster, and
 // a third more HBM reads where a tile no longer starts on a 128-byte line.)
-constexpr int OH = 16;
 template <int VAR, int S, bool FULLN, typename Tin, typename Tbc, bool GATED>
 __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
-  static_assert(VAR == VAR_COMPLEX || VAR == VAR_REAL, "the unitary scan runs backwards");
   constexpr int C = VAR == VAR_REAL ? 1 : 2;
+  constexpr bool UNI = VAR == VAR_UNITARY;
+  constexpr int OH = UNI && S > 2 ? 8 : 16;
+  static_assert(!(UNI && GATED), "the unitary scan's gate has kernels of its own");
   // planes [channel][step] of a wavefront: what the steps read - real (delta, w, dy), complex (Re a, Im a, w, dy) -, the
   // sums over the states (the first in the place of w), and what the end of the tile wants back and registers have no room for
   constexpr int PX = 0, PW = C, PG = C + 1, PKA = PW, PXA = C + 2;
   constexpr int PZA = PXA + 1;                              // complex: sum behind drho, dtheta (imaginary part)
   constexpr int PU = PXA + 1, PRAW = PXA + 2, PACT = PXA + 3;   // real: u, delta before the softplus, silu'(u)
   constexpr int PYA = VAR == VAR_REAL ? PACT + 1 : PZA + 1, PGZ = PYA + 1;
-  constexpr int NPL = VAR == VAR_REAL ? (GATED ? PGZ + 1 : PACT + 1) : (GATED ? PYA + 1 : PZA + 1);
+  constexpr int NPL = VAR == VAR_REAL ? (GATED ? PGZ + 1 : PACT + 1) : UNI ? PXA + 1 : (GATED ? PYA + 1 : PZA + 1);
   constexpr int PL = 8 * OP;
   using Rows = OctRows<C, S, 2, OT, Tbc>;
   // a wavefront's sums over its channels of 16 steps: [dB, dC][state row][step], rows 4 floats apart from a power of two
@@ -755,8 +761,9 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   const bool dok = d < D, live = d0 + 8 * wave < D;
   const int dd = dok ? d : D - 1;
 
-  const Tin* __restrict__ gu = static_cast<const Tin*>(p.u);
-  const Tin* __restrict__ gdl = static_cast<const Tin*>(p.delta);
+  const size_t uback = UNI ? (size_t)(b - b / p.urep) * D * ld : 0;   // (u, delta of [B / urep, D, L])
+  const Tin* __restrict__ gu = static_cast<const Tin*>(p.u) - uback;
+  const Tin* __restrict__ gdl = static_cast<const Tin*>(p.delta) - uback;
   const size_t goff = ((size_t)b * D + dd) * ld + lbeg;
   const size_t zoff = (VAR == VAR_REAL && p.zrows) ? (size_t)b * (p.zrows - D) * ld : 0;   // (z, dz: rows of a wider tensor)
   const size_t bc_row = ((size_t)b * ((VAR == VAR_REAL && p.bcrows) ? p.bcrows : NT_) + p.nbase) * ld + lbeg;
@@ -779,11 +786,12 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   }
   const bool has_last = FULLN || 8 * (S - 1) + g < N;
 
-  // ---- state before step l (a multiple of 16) of the segment: the checkpoint there, or the initial state
+  // ---- state before step l of the segment (a multiple of 16; unitary: of ck, or its end): the checkpoint there, or the initial
+  // state
   struct Start { float r[S], i[S]; };
   auto load_start = [&](Start& st, int l) {
     const int lg = lbeg + l;
-    const size_t base = fresh((((size_t)b * p.nck + (lg > 0 ? lg / p.ck - 1 : 0)) * NT_ + p.nbase + g) * C * D + d);
+    const size_t base = fresh((((size_t)b * p.nck + (lg > 0 ? (lg - 1) / p.ck : 0)) * NT_ + p.nbase + g) * C * D + d);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int n = p.nbase + 8 * s + g;
@@ -819,14 +827,16 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
     raw.dl.load(gdl, o, vec, idx);
     raw.dy.load(p.dy, o, vec, idx);
     if (GATED) raw.z.load(p.z + zoff, o, vec, idx);
-    if (VAR == VAR_COMPLEX) { raw.th.load(p.theta, o, vec, idx); raw.rho.load(p.rho, o, vec, idx); }
+    if (C == 2) raw.th.load(p.theta, o, vec, idx);
+    if (VAR == VAR_COMPLEX) raw.rho.load(p.rho, o, vec, idx);
   };
   Rows rows;
   Start st, st_next;                                        // of this interval, of the next (its loads in flight)
   auto land = [&]() {
     raw.u.touch(); raw.dl.touch(); raw.dy.touch();
     if (GATED) raw.z.touch();
-    if (VAR == VAR_COMPLEX) { raw.th.touch(); raw.rho.touch(); }
+    if (C == 2) raw.th.touch();
+    if (VAR == VAR_COMPLEX) raw.rho.touch();
   };
   auto land_start = [&]() {
 #pragma unroll
@@ -841,7 +851,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   float accD = 0.f, accB = 0.f;
   float* __restrict__ in = &s_in[wave][0][0];
 
-  // what the eight wavefronts left of the 16 steps from lh on: added up, one atomic per element
+  // what the eight wavefronts left of the OH steps from lh on: added up, one atomic per element
   auto flush = [&](int buf, int lh) {
     constexpr int TOT = 2 * 8 * S * OH * C;
 #pragma unroll
@@ -860,7 +870,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   };
 
   const int last = (L - 1) / OH;                             // index of the last interval
-  const int lastb = last >> 1;                               // ... of the block of rows it lies in
+  const int lastb = (L - 1) / OT;                            // ... of the block of rows it lies in
   int tile0 = lastb * OT;                                    // first step of the staged tile
   float eu[4], edl[4], egz[4];                               // of the staged tile (complex: kept in registers; egz: dy silu'(z))
   // (whole: all of the tile's steps and of the wavefront's channels exist)
@@ -873,9 +883,9 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       ok[i] = WHOLE || (dok && l0 + 4 * g + i < L);
-      th[i] = VAR == VAR_COMPLEX && ok[i] ? raw.th.get(i) : 0.f;
+      th[i] = C == 2 && ok[i] ? raw.th.get(i) : 0.f;
     }
-    if constexpr (VAR == VAR_COMPLEX) sincos4(th, sn, cs);
+    if constexpr (C == 2) sincos4(th, sn, cs);
     float u4_[4], d4[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -906,7 +916,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
       if (VAR == VAR_REAL) {
         o0[i] = dl;
       } else {
-        const float r = expf(ok[i] ? raw.rho.get(i) : 0.f);
+        const float r = VAR == VAR_COMPLEX ? expf(ok[i] ? raw.rho.get(i) : 0.f) : 1.f;
         o0[i] = cs[i] * r; o1[i] = sn[i] * r;
       }
       ow[i] = dl * uu; og[i] = gy; ou[i] = uu;
@@ -949,9 +959,10 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   Steps sp[2];
   RowsAt rw[2];
 
-  // Steps lh .. lh + 15 from the start state st; t0: their place in the staged tile, bc: in the rows.  TAIL: some of them lie
+  // Steps lh .. lh + OH - 1 from the start state st; t0: their place in the staged tile, bc: in the rows.  TAIL: some of them lie
   // past the end; state and adjoint pass through those unchanged.
-  float hsr[OH][S], hsi[OH][S];                              // states; real: hsi holds the decay factors of the steps
+  // states; real: hsi holds the decay factors of the steps; unitary: the state behind the step being worked on
+  float hsr[UNI ? 1 : OH][S], hsi[UNI ? 1 : OH][S];
   auto recompute = [&](int lh, int t0, const float* __restrict__ bc, auto tail_tag) {
     constexpr bool TAIL = decltype(tail_tag)::value;
     float xr[S], xi[S];
@@ -1011,14 +1022,33 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
         sched_fence();
         const Steps& x = sp[qq & 1];
         const RowsAt& r = rw[turn & 1];
-        float vb_r[G], vb_i[G];
+        float vb_r[G], vb_i[G], vc_r[G], vc_i[G];
 #pragma unroll
         for (int t = G - 1; t >= 0; --t) {
           const int tt = qq * G + t;
           const bool mine = s < S - 1 || has_last;
           const float wt = mine ? x.w[t] : 0.f, gy = mine ? x.gy[t] : 0.f;
-          const float hpr = tt > 0 ? hsr[tt > 0 ? tt - 1 : 0][s] : st.r[s];
-          if constexpr (VAR == VAR_REAL) {
+          const float hpr = !UNI && tt > 0 ? hsr[!UNI && tt > 0 ? tt - 1 : 0][s] : st.r[s];
+          if constexpr (UNI) {
+            float& hr = hsr[0][s];
+            float& hi = hsi[0][s];
+            gr[s] = fmaf(r.cr[t], gy, gr[s]);
+            gi[s] = fmaf(-r.ci[t], gy, gi[s]);
+            vb_r[t] = wt * gr[s];
+            vb_i[t] = wt * gi[s];
+            vc_r[t] = gy * hr;
+            vc_i[t] = -gy * hi;
+            ka[t] = fmaf(r.br[t], gr[s], ka[t]);
+            ka[t] = fmaf(r.bi[t], gi[s], ka[t]);
+            const float pr = fmaf(-r.br[t], wt, hr), pi = fmaf(-r.bi[t], wt, hi);
+            xa[t] = fmaf(gr[s], pi, xa[t]);                  // Im(conj(g) p)
+            xa[t] = fmaf(-gi[s], pr, xa[t]);
+            const float tg = fmaf(x.x0[t], gr[s], x.x1[t] * gi[s]);
+            gi[s] = fmaf(x.x0[t], gi[s], -x.x1[t] * gr[s]);
+            gr[s] = tg;
+            hr = fmaf(x.x0[t], pr, x.x1[t] * pi);
+            hi = fmaf(x.x0[t], pi, -x.x1[t] * pr);
+          } else if constexpr (VAR == VAR_REAL) {
             gr[s] = fmaf(r.cr[t], gy, gr[s]);
             vb_r[t] = wt * gr[s];
             if (GATED) ya[t] = fmaf(r.cr[t], hsr[tt][s], ya[t]);
@@ -1059,8 +1089,8 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
 #pragma unroll
         for (int t = 0; t < G; ++t) {
           const float gy = (s < S - 1 || has_last) ? x.gy[t] : 0.f;
-          vb_r[t] = gy * hsr[qq * G + t][s];
-          if (C == 2) vb_i[t] = -gy * hsi[qq * G + t][s];
+          vb_r[t] = UNI ? vc_r[t] : gy * hsr[UNI ? 0 : qq * G + t][s];
+          if (C == 2) vb_i[t] = UNI ? vc_i[t] : -gy * hsi[UNI ? 0 : qq * G + t][s];
         }
         put(o + 8 * S * SR);
         sched_fence();
@@ -1069,7 +1099,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
       float* o = in + c * OP + t0 + qq * G + gs_;
       o[PKA * PL] = state_sums(ka, bit2, bit1, bit0);
       o[PXA * PL] = state_sums(xa, bit2, bit1, bit0);
-      if constexpr (C == 2) o[PZA * PL] = state_sums(za, bit2, bit1, bit0);
+      if constexpr (VAR == VAR_COMPLEX) o[PZA * PL] = state_sums(za, bit2, bit1, bit0);
       if constexpr (GATED) o[PYA * PL] = state_sums(ya, bit2, bit1, bit0);
     }
   };
@@ -1087,7 +1117,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
     f4 x1 = {0, 0, 0, 0}, za = x1, ya = x1, uu = {eu[0], eu[1], eu[2], eu[3]}, dl = {edl[0], edl[1], edl[2], edl[3]};
     f4 act = {1, 1, 1, 1}, pre = x1, gz = {egz[0], egz[1], egz[2], egz[3]};
     const f4 x0 = plane(0);
-    if constexpr (C == 2) { x1 = plane(1); za = plane(PZA); }
+    if constexpr (VAR == VAR_COMPLEX) { x1 = plane(1); za = plane(PZA); }
     if constexpr (VAR == VAR_REAL) {
       dl = x0; uu = plane(PU);
       if (p.u_act) act = plane(PACT);
@@ -1114,6 +1144,8 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
         dd_[i] += xa[i];
         dd_[i] *= dsp[i];
         if (i < nvalid) accB += dd_[i];
+      } else if (UNI) {
+        dth[i] = -xa[i];
       } else {
         drh[i] = fmaf(x0[i], xa[i], -x1[i] * za[i]);       // Re(a s)
         dth[i] = -fmaf(x0[i], za[i], x1[i] * xa[i]);       // -Im(a s)
@@ -1151,7 +1183,8 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
         put(p.du + o, duv);
         put(p.ddelta + o, dd_);
       }
-      if (VAR == VAR_COMPLEX) { put(p.dtheta + o, dth); put(p.drho + o, drh); }
+      if (C == 2) put(p.dtheta + o, dth);
+      if (VAR == VAR_COMPLEX) put(p.drho + o, drh);
       if (GATED) put(p.dz + o + zoff, dzv);
     }
     if (more) {
@@ -1166,7 +1199,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   rows.load(gB, gC, bc_row, ld, lastb * OT, L, N, tid);
   if (live) {
     load_tile(tile0);
-    load_start(st_next, last * OH);
+    load_start(st_next, UNI ? L : last * OH);
   } else {
     for (int i = lane; i < SLAB; i += 64) { s_slab[0][wave][i] = 0.f; s_slab[1][wave][i] = 0.f; }
   }
@@ -1175,6 +1208,10 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   if (live) {
     stage(tile0);
     land_start();
+    if constexpr (UNI) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) { hsr[0][s] = st.r[s]; hsi[0][s] = st.i[s]; }
+    }
     if (tile0 > 0) load_tile(tile0 - OT);
   }
   oct_barrier();
@@ -1182,21 +1219,32 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   for (int j = last; j >= 0; --j) {
     const int lh = j * OH;
     // ---- the rows of the next block, whose loads are two intervals old, into the other buffer; request the ones after
-    const int rb = j >> 1;
-    if (((j & 1) || j == last) && rb > 0) {
+    const int rb = lh / OT;
+    if ((lh % OT == OT - OH || j == last) && rb > 0) {
       rows.put(s_bc[(rb - 1) & 1], (rb - 1) * OT, L, N, tid);
       if (rb > 1) rows.load(gB, gC, bc_row, ld, (rb - 2) * OT, L, N, tid);
     }
     if (live) {
-      if (j > 0) load_start(st_next, lh - OH);
+      if (!UNI && j > 0) load_start(st_next, lh - OH);
       const int t0 = lh - tile0;
       const float* __restrict__ bc = s_bc[rb & 1] + g * Rows::RS + (lh & (OT - 1)) * C;
       oct_wave_fence();
-      if (lh + OH <= L) recompute(lh, t0, bc, std::false_type{});
-      else recompute(lh, t0, bc, std::true_type{});
+      if constexpr (!UNI) {
+        if (lh + OH <= L) recompute(lh, t0, bc, std::false_type{});
+        else recompute(lh, t0, bc, std::true_type{});
+      }
       if (j < last) flush((j + 1) & 1, lh + OH);
       walk(t0, bc, j & 1);
-      land_start();
+      if constexpr (UNI) {
+        // a checkpoint: its state instead of the one run back to (plain loads, once per block)
+        if (lh > 0 && lh % p.ck == 0) {
+          load_start(st, lh);
+#pragma unroll
+          for (int s = 0; s < S; ++s) { hsr[0][s] = st.r[s]; hsi[0][s] = st.i[s]; }
+        }
+      } else {
+        land_start();
+      }
       rows.touch();
       if (t0 == 0) finish(j > 0);
     } else if (j < last) {
