@@ -1,20 +1,10 @@
-// Translation unit of the kernels around the vector-ALU scans: their split along the sequence, the causal convolution,
-// the layout swap, the gate.
+// Translation unit of the kernels around the scans: the causal convolution, the layout swap, the gate.
 #include "conv1d.h"
 #include "launch.h"
 #include "layout.h"
-#include "scan_seg_real.h"
+#include "scan_common.h"
 
 namespace aussm {
-
-int run_seg_carry_real(bool adjoint, float* seg, const float* ptot, const float* A, const float* first, float* last,
-                        int B, int D, int N, int ns, hipStream_t s) {
-  const size_t n = (size_t)B * D * N;
-  const dim3 grid((unsigned)((n + 255) / 256));
-  if (adjoint) hipLaunchKernelGGL(seg_carry_real_kernel<true>, grid, dim3(256), 0, s, seg, ptot, A, first, last, B, D, N, ns);
-  else hipLaunchKernelGGL(seg_carry_real_kernel<false>, grid, dim3(256), 0, s, seg, ptot, A, first, last, B, D, N, ns);
-  return launch_status();
-}
 
 // ---- what the memory system gives for the scans' access pattern (no arithmetic to speak of): o1 = a + b c,
 // o2 = 2 o1 over [rows, L] tensors.  PATTERN 0: every thread streams consecutive 16-byte pieces (a plain

@@ -65,7 +65,7 @@ int run_oct_ubwd(const UniBwdArgs& u, int in_dtype, hipStream_t s) {
   RecBwdArgs a{};
   a.dy = u.dy; a.dhL = u.dhL; a.u = u.u; a.delta = u.delta; a.theta = u.theta; a.Bm = u.Bm; a.Cm = u.Cm; a.Dskip = u.Dskip; a.hck = u.hck;
   a.du = u.du; a.ddelta = u.ddelta; a.dtheta = u.dtheta; a.dB = u.dB; a.dC = u.dC; a.dD = u.dD; a.dh0 = u.dh0;
-  a.B = u.B; a.D = u.D; a.N = u.N; a.L = u.L; a.ck = u.ck; a.nck = u.nck; a.ncg = u.ncg; a.ld = u.ld; a.ns = u.ns;
+  a.B = u.B; a.D = u.D; a.N = u.N; a.L = u.L; a.ck = u.ck; a.nck = u.nck; a.ncg = u.ncg; a.ld = u.ld; a.ns = u.ns; a.seg = u.seg; a.segq = u.segq;
   a.urep = u.urep; a.g16 = u.g16;
   return in_dtype ? oct_ubwd_t<bf16_t>(a, s) : oct_ubwd_t<float>(a, s);
 }

@@ -16,6 +16,13 @@ int run_px_prep(const PrepArgs& a, int B, int in_dtype, hipStream_t s) {
   return launch_status();
 }
 
+int run_prep_seg(const PrepArgs& a, int B, const SegArgs& sa, unsigned nseg, int in_dtype, hipStream_t s) {
+  const dim3 grid((unsigned)(B * a.nch) + nseg);
+  if (in_dtype == 1) hipLaunchKernelGGL((unitary_prep_seg_kernel<bf16_t>), grid, dim3(256), 0, s, a, sa, (int)nseg);
+  else hipLaunchKernelGGL((unitary_prep_seg_kernel<float>), grid, dim3(256), 0, s, a, sa, (int)nseg);
+  return launch_status();
+}
+
 int run_px_fwd(const FwdArgs& a, const u4* img, const ImgNote& note, int in_dtype, hipStream_t s) {
   const dim3 grid((unsigned)(a.B * a.ncg));
   if (in_dtype == 1) {

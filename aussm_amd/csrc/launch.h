@@ -19,17 +19,13 @@ inline int launch_status() {
 // A workgroup of nt threads (nt / 64 wavefronts) of unitary_bwd_kernel owns 64 channels; each wavefront owns nw states.
 struct Cfg { int nw, nt; };
 
-// ---- k_oct_fwd.hip, k_oct_bwd.hip, k_ubwd.hip: vector-ALU scans; k_generic.hip: chain of the S6 segments, convolution,
-// layout swap.  in_dtype: 0 float, 1 bf16
+// ---- k_oct_fwd.hip, k_oct_bwd.hip, k_ubwd.hip: vector-ALU scans; k_generic.hip: convolution, layout swap.  in_dtype: 0 float, 1 bf16
 int run_oct_fwd(int variant, const FwdArgs& a, int in_dtype, hipStream_t s);
 int run_oct_adj(int variant, const AdjSegArgs& a, int in_dtype, unsigned grid, hipStream_t s);   // adjoint entering every segment
 int run_oct_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s);
 int run_oct_ubwd(const UniBwdArgs& a, int in_dtype, hipStream_t s);                              // N <= 32
 int run_unitary_bwd_generic(const UniBwdArgs& a, int in_dtype, Cfg c, hipStream_t s);
 int run_aux_invalidate(float* tag, bool fill_tag, bool images_tag, hipStream_t s);   // clears tag(s) in the buffer's pad
-// split along L: chain of the real scan's segments
-int run_seg_carry_real(bool adjoint, float* seg, const float* ptot, const float* A, const float* first, float* last,
-                        int B, int D, int N, int ns, hipStream_t s);
 int run_hbm_probe(const float* a, const float* b, const float* c, float* o1, float* o2, int rows, int L, int pattern,
                   int write, hipStream_t s);
 int run_conv_fwd(const ConvArgs& a, hipStream_t s);
@@ -43,11 +39,10 @@ int run_gate(const float* dy, const float* ypre, const float* z, float* out, flo
 int run_xdl_fwd(int mode, const FwdArgs& a, int in_dtype, hipStream_t s);
 int run_xdl_bwd(int mode, const UniBwdArgs& a, int in_dtype, hipStream_t s);
 int run_seg_state(bool adjoint, const SegArgs& a, int in_dtype, unsigned grid, hipStream_t s);
-int run_seg_carry_fwd(float* seg, const float* ptot, const float* h0, float* hL, int B, int D, int N, int nf, hipStream_t s);
-int run_seg_carry_bwd(float* seg, const float* ptot, const float* dhL, float* dh0, int B, int D, int N, int nf, hipStream_t s);
 
 // ---- k_px.hip: matrix-core unitary scans on operands prepared by a pre-pass
 int run_px_prep(const PrepArgs& a, int B, int in_dtype, hipStream_t s);
+int run_prep_seg(const PrepArgs& a, int B, const SegArgs& sa, unsigned nseg, int in_dtype, hipStream_t s);   // both in one launch
 int run_px_fwd(const FwdArgs& a, const u4* img, const ImgNote& note, int in_dtype, hipStream_t s);
 int run_px_bwd(const UniBwdArgs& a, const u4* img, int in_dtype, hipStream_t s);
 

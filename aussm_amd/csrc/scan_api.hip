@@ -132,26 +132,32 @@ inline USplit unitary_split(int B, int D, int N, int L, int ck, bool use_cap, si
   }
   if (ns <= 1) return whole;
   int r = seg_fine(L, ns);
-  while (r > 1 && ns * r > fine) r /= 2;      // (fewer segments by option: no more fine ones than the area is sized for)
+  // (no more fine ones than the area is sized for - fewer segments by option -, and few: a workgroup of the scan walks those
+  // ahead of its segment.  B4 D256 N16 L16384 training pass with 64 / 32 / 16 of them 435 / 415 / 422 us, B8 L4096 with
+  // 32 / 16 / 8 212 / 198 / 201, B2 L8192 with 64 / 32 136 / 124)
+  while (r > 1 && (ns * r > fine || r > 2 || ns * r > 32)) r /= 2;
   return USplit{ns, L / ns, r, ns * r};
 }
 inline size_t round64(size_t n) { return (n + 63) & ~(size_t)63; }
 inline size_t seg_floats(int B, int D, int N, int L, int ns) {
   return ns > 1 ? round64((size_t)B * ns * seg_fine(L, ns) * D * (2 * N + 2)) : 0;
 }
-// The complex and the real scan split the same way (scan_seg_real.h) when the call brings a workspace:
+// The complex and the real scan split the same way (scan_oct.h) when the call brings a workspace:
 // ns segments of ls steps (whole tiles and checkpoint blocks), the last one possibly shorter.
+// (segments of 64 steps, forward passes, us: S6 B1 D512 L300 28 -> 20 against 128, B2 D64 L256 27 -> 19; sequences of fewer than
+// 256 steps stay whole: what is left to gain there is less than the launches of the first pass cost)
+constexpr int GSPLIT_MIN_LEN = 64, GSPLIT_FROM = 256;
 struct GSplit { int ns, ls; };
 inline GSplit generic_split(int B, int D, int L, int ck, bool use_cap) {
   const long long wgs = (long long)B * ((D + CH - 1) / CH);
   const int cap = use_cap ? opt(AUSSM_OPT_SPLIT_CAP) : -1;
-  if (wgs >= SPLIT_MIN_WGS || cap == 0 || cap == 1) return GSplit{1, L};
+  if (wgs >= SPLIT_MIN_WGS || L < GSPLIT_FROM || cap == 0 || cap == 1) return GSplit{1, L};
   int want = (int)((SPLIT_TARGET_WGS + wgs - 1) / wgs);
   if (want > GSPLIT_MAX) want = GSPLIT_MAX;
   if (cap > 1 && want > cap) want = cap;
   const int unit = ck > XT ? ck : XT;
   int ls = ((L + want - 1) / want + unit - 1) / unit * unit;
-  if (ls < SPLIT_MIN_LEN) ls = (SPLIT_MIN_LEN + unit - 1) / unit * unit;
+  if (ls < GSPLIT_MIN_LEN) ls = (GSPLIT_MIN_LEN + unit - 1) / unit * unit;
   const int ns = (L + ls - 1) / ls;
   return ns > 1 ? GSplit{ns, ls} : GSplit{1, L};
 }
@@ -232,8 +238,10 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
   const bool fill = a.aux && a.hck && mode >= 2;
   // (the prepared-operand kernel clears the fill tag itself, at its end: one launch less for a forward-only call)
   const bool clear_in_kernel = a.aux && !fill && mode == 6;
-  if (a.aux)
+  // (the vector-ALU kernels do that too, at theirs)
+  if (a.aux && mode)
     if (int e = run_aux_invalidate(ws.pad, !fill && !clear_in_kernel, mode != 6 && ws.stamp, s)) return e;
+  const bool had_aux = a.aux != nullptr;
   if (!fill) a.aux = nullptr;
   if (!mode) {
     // vector-ALU kernel; with a segment area and few (batch, channel group) pairs, split along the sequence
@@ -247,25 +255,27 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
       z.B = B * sp.ns; z.L = sp.ls; z.ns = sp.ns;
       z.y = nullptr; z.z = nullptr; z.Dskip = nullptr; z.h0 = nullptr; z.hL = seg; z.hck = nullptr; z.ptot = ptot;
       if (int e = run_oct_fwd(VAR_UNITARY, z, in_dtype, s)) return e;
-      // 2. the state that enters every segment; the state after the last one is the call's hL
-      if (int e = run_seg_carry_fwd(seg, ptot, a.h0, a.hL, B, a.D, a.N, sp.ns, s)) return e;
-      // 3. the scan proper over (batch, segment) pairs
-      a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.h0 = seg; a.hL = nullptr;
+      // 2. the scan proper over (batch, segment) pairs, each from what those before it make of the state
+      a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.seg = seg; a.segq = ptot;
     }
+    a.clear = had_aux ? ws.pad : nullptr;
     return run_oct_fwd(VAR_UNITARY, a, in_dtype, s);
   }
   const int B = a.B, L = a.L;
+  SegArgs sa{};
+  unsigned nseg = 0;                           // workgroups of the segment-state pass, run with the pre-pass (mode 6)
   if ((mode == 2 || mode == 3 || mode == 6) && ws.seg) {
     const USplit sp = unitary_split(B, a.D, a.N, L, a.ck, true, ws.seg_room);
     if (sp.ns > 1) {
-      // 1. end state of every segment from a zero start and its rotation; 2. chain them;
-      // 3. the scan proper over (batch, segment) pairs, each from its true incoming state
+      // 1. end state of every segment from a zero start and its rotation; 2. the scan proper over (batch, segment) pairs,
+      // each from what the segments before it make of the state
       float* seg = ws.seg;
       float* ptot = seg + (size_t)B * sp.nf * a.D * a.N * 2;
-      SegArgs sa{a.delta, a.u, a.theta, a.Bm, seg, ptot, a.D, a.N, sp.ls / sp.r, L, sp.nf, a.ncg};
-      if (int e = run_seg_state(false, sa, in_dtype, (unsigned)(B * sp.nf * a.ncg), s)) return e;
-      if (int e = run_seg_carry_fwd(seg, ptot, a.h0, a.hL, B, a.D, a.N, sp.nf, s)) return e;
-      a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.h0 = seg; a.hL = nullptr; a.hs = sp.r; a.ho = 0; a.nf = sp.nf;
+      sa = SegArgs{a.delta, a.u, a.theta, a.Bm, seg, ptot, a.D, a.N, sp.ls / sp.r, L, sp.nf, a.ncg};
+      nseg = (unsigned)(B * sp.nf * a.ncg);
+      if (mode != 6)
+        if (int e = run_seg_state(false, sa, in_dtype, nseg, s)) return e;
+      a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.seg = seg; a.segq = ptot; a.hs = sp.r; a.nf = sp.nf;
     }
   }
   if (mode == 6) {
@@ -273,7 +283,7 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
     // checkpoints, so a call without them is not followed by one)
     const bool with_bwd = a.hck != nullptr;
     PrepArgs pa{a.Bm, a.Cm, ws.fimg, with_bwd ? ws.img : nullptr, a.N, L, (L + XT - 1) / XT, nullptr, ImgStamp{}};
-    if (int e = run_px_prep(pa, B, in_dtype, s)) return e;
+    if (int e = nseg ? run_prep_seg(pa, B, sa, nseg, in_dtype, s) : run_px_prep(pa, B, in_dtype, s)) return e;
     const ImgNote note{ws.stamp, img_stamp(a.Bm, a.Cm, B, a.N, L, in_dtype, with_bwd), clear_in_kernel ? ws.pad : nullptr};
     return run_px_fwd(a, ws.fimg, note, in_dtype, s);
   }
@@ -294,12 +304,8 @@ int launch_generic_fwd(int variant, FwdArgs a, int in_dtype, float* ws, hipStrea
     z.B = B * sp.ns; z.L = sp.ls; z.ns = sp.ns;
     z.y = nullptr; z.z = nullptr; z.Dskip = nullptr; z.h0 = nullptr; z.hL = seg; z.hck = nullptr; z.ptot = ptot;
     if (int e = run_oct_fwd(variant, z, in_dtype, s)) return e;
-    // 2. the state that enters every segment; the state after the last one is the call's hL
-    if (int e = variant == VAR_COMPLEX ? run_seg_carry_fwd(seg, ptot, a.h0, a.hL, B, a.D, a.N, sp.ns, s)
-                                       : run_seg_carry_real(false, seg, ptot, a.A, a.h0, a.hL, B, a.D, a.N, sp.ns, s))
-      return e;
-    // 3. the scan proper over (batch, segment) pairs
-    a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.h0 = seg; a.hL = nullptr;
+    // 2. the scan proper over (batch, segment) pairs, each from what those before it make of the state
+    a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.seg = seg; a.segq = ptot;
   }
   return run_oct_fwd(variant, a, in_dtype, s);
 }
@@ -318,10 +324,7 @@ int launch_generic_bwd(int variant, RecBwdArgs a, int in_dtype, float* ws, hipSt
     g.D = a.D; g.N = a.N; g.L = sp.ls; g.ld = a.L; g.ns = sp.ns; g.ncg = a.ncg; g.delta_softplus = a.delta_softplus;
     g.zrows = a.zrows; g.bcrows = a.bcrows;
     if (int e = run_oct_adj(variant, g, in_dtype, (unsigned)(B * sp.ns * a.ncg), s)) return e;
-    if (int e = variant == VAR_COMPLEX ? run_seg_carry_bwd(seg, ptot, a.dhL, a.dh0, B, a.D, a.N, sp.ns, s)
-                                       : run_seg_carry_real(true, seg, ptot, a.A, a.dhL, a.dh0, B, a.D, a.N, sp.ns, s))
-      return e;
-    a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.dhL = seg; a.dh0 = nullptr;
+    a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.seg = seg; a.segq = ptot;
   }
   return run_oct_bwd(variant, a, in_dtype, s);
 }
@@ -443,7 +446,7 @@ int aussm_unitary_fwd_aux(const void* u, const void* delta, const float* theta, 
   a.u = u; a.delta = delta; a.theta = theta; a.Bm = Bc; a.Cm = Cc; a.Dskip = Dskip; a.z = z;
   a.h0 = h0; a.y = y; a.hL = hL; a.hck = hck; a.aux = aux;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = urep;
+  a.ld = L; a.ns = 1; a.urep = urep;
   a.auxtag = aux_tag(u, delta, theta, Bc, Cc, B, D, N, L, in_dtype);
   return launch_unitary_fwd(a, in_dtype, (hipStream_t)stream, aux_layout(aux, B, D, N, L, ck));
 }
@@ -473,7 +476,7 @@ int aussm_unitary_fwd_static(const void* u, const void* delta, const float* thet
   a.u = u; a.delta = delta; a.theta = theta; a.Bm = Bc; a.Cm = Cc; a.Dskip = Dskip; a.z = z;
   a.h0 = h0; a.y = y; a.hL = hL; a.hck = nullptr; a.aux = nullptr;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = 1;
+  a.ld = L; a.ns = 1; a.urep = 1;
   // (every segment state the scan reads is written earlier in the same call: nothing in the
   // scratch has to start at zero)
   // (the vector-ALU kernels do not split here: no gseg)
@@ -491,7 +494,7 @@ int aussm_complex_fwd(const void* u, const void* delta, const float* rho, const 
   a.u = u; a.delta = delta; a.rho = rho; a.theta = theta; a.Bm = Bc; a.Cm = Cc; a.Dskip = Dskip; a.z = z;
   a.h0 = h0; a.y = y; a.hL = hL; a.hck = hck;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = 1;
+  a.ld = L; a.ns = 1; a.urep = 1;
   return launch_generic_fwd(VAR_COMPLEX, a, in_dtype, workspace, (hipStream_t)stream);
 }
 
@@ -523,7 +526,7 @@ int aussm_real_fwd_rows(const void* u, const void* delta, const float* A, const 
   if (int e = real_rows_check(rows, D, N, in_dtype)) return e;
   if (rows) { a.zrows = rows->z_rows; a.bcrows = rows->bc_rows; a.u_act = rows->u_silu; }
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = 1;
+  a.ld = L; a.ns = 1; a.urep = 1;
   return launch_generic_fwd(VAR_REAL, a, in_dtype, workspace, (hipStream_t)stream);
 }
 
@@ -552,7 +555,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
   a.dy = dy; a.dhL = dhL; a.u = u; a.delta = delta; a.theta = theta; a.Bm = Bc; a.Cm = Cc; a.Dskip = Dskip;
   a.hck = hck; a.aux = aux; a.du = du; a.ddelta = ddelta; a.dtheta = dtheta; a.dB = dB; a.dC = dC; a.dD = dD; a.dh0 = dh0;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  a.ld = L; a.ns = 1; a.hs = 1; a.ho = 0; a.nf = 1; a.urep = 1;
+  a.ld = L; a.ns = 1; a.urep = 1;
   a.urep = urep;
   a.g16 = g16 && in_dtype == AUSSM_BF16;
   a.auxtag = aux_tag(u, delta, theta, Bc, Cc, B, D, N, L, in_dtype);
@@ -564,14 +567,12 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
         misaligned(Cc, 16))) {
     const USplit sp = aux ? unitary_split(B, D, N, L, ck, true, ws.seg_room) : USplit{1, L, 1, 1};
     if (sp.ns > 1) {
-      // adjoint at the start of every segment from a zero adjoint at its end, chained last to first
+      // adjoint at the start of every segment from a zero adjoint at its end
       float* seg = ws.seg;
       float* ptot = seg + (size_t)B * sp.nf * D * N * 2;
       SegArgs sa{dy, nullptr, theta, Cc, seg, ptot, D, N, sp.ls / sp.r, L, sp.nf, a.ncg};
       if (int e = run_seg_state(true, sa, in_dtype, (unsigned)(B * sp.nf * a.ncg), s)) return e;
-      if (int e = run_seg_carry_bwd(seg, ptot, dhL, dh0, B, D, N, sp.nf, s)) return e;
-      // a segment of the scan ends where its last fine segment ends
-      a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.dhL = seg; a.dh0 = nullptr; a.hs = sp.r; a.ho = sp.r - 1; a.nf = sp.nf;
+      a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.seg = seg; a.segq = ptot; a.hs = sp.r; a.nf = sp.nf;
     }
     if (mode == 6) {
       // The prepared-operand kernel needs Im(P S) from the forward call in the auxiliary buffer; its
@@ -602,8 +603,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
     g.dy = dy; g.theta = theta; g.Cm = Cc; g.out = seg; g.ptot = ptot;
     g.D = D; g.N = N; g.L = sp.ls; g.ld = L; g.ns = sp.ns; g.ncg = a.ncg;
     if (int e = run_oct_adj(VAR_UNITARY, g, in_dtype, (unsigned)(B * sp.ns * a.ncg), s)) return e;
-    if (int e = run_seg_carry_bwd(seg, ptot, dhL, dh0, B, D, N, sp.ns, s)) return e;
-    a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.dhL = seg; a.dh0 = nullptr;
+    a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.seg = seg; a.segq = ptot;
   }
   if (N <= 32) return run_oct_ubwd(a, in_dtype, s);
   return run_unitary_bwd_generic(a, in_dtype, pick_cfg(a.N, 8), s);

@@ -58,10 +58,14 @@ struct FwdArgs {
   int B, D, N, L, ck, nck, ncg, delta_softplus;
   int ld, ns;                // row stride of the [.., L] tensors and segments per sequence: B then counts
                              // (batch, segment) pairs and L is the segment length (the last one may be shorter: ld
-                             // not a multiple of L); nck stays the number of checkpoints of a whole sequence;
-                             // vector-ALU kernels: h0 / hL / ptot are indexed by the pair
-  int hs, ho, nf;            // matrix-core kernels: h0 of segment sg of batch element bb is entry bb * nf + min(sg * hs + ho,
-                             // nf - 1) of the state array (nf entries per batch element)
+                             // not a multiple of L); nck stays the number of checkpoints of a whole sequence
+  // ... and what the segments make of a zero state (seg_chain): nf entries per sequence, hs per segment.  Null: not split.
+  // h0 and hL are indexed by the batch element; a launch that forms the entries (ptot) starts from zero and leaves
+  // them in hL and ptot by the pair.
+  const float* seg;          // [B / ns * nf, D, N, C]
+  const float* segq;         // [B / ns * nf, D, 2]
+  int hs, nf;
+  float* clear;              // vector-ALU kernels: words 0 and AUX_IMG_FP .. + 7 here are set to zero, or null
   int urep;                  // generic kernels: u and delta are [B / urep, D, L], shared by urep consecutive batch elements
   uint32_t auxtag;           // what a kernel that fills aux writes behind it (aux_tag of the call)
   // vector-ALU kernels: rows per batch element of the tensors z and B_t / C_t lie in (0: D and N, tensors of their own),
@@ -86,7 +90,8 @@ struct UniBwdArgs {
   float* dh0;           // [B,D,N,2] or null
   int B, D, N, L, ck, nck, ncg;
   int ld, ns;           // row stride of the [.., L] tensors, segments per sequence (as FwdArgs)
-  int hs, ho, nf;       // ... and which entry of the adjoint array is a pair's dhL (as FwdArgs)
+  const float *seg, *segq;   // adjoints of the segments (as FwdArgs); dhL and dh0 are indexed by the batch element
+  int hs, nf;
   int urep;             // generic kernel: u and delta are [B / urep, D, L], shared by urep consecutive batch elements
   int tag_mode;         // matrix-core kernels: 0 use the auxiliary buffer if its tag is valid; 1 leave at once
                         // unless it is; 2 leave at once if it is
@@ -118,9 +123,11 @@ struct RecBwdArgs {
   float* dz;                // [B,D,L] (with z)
   int B, D, N, L, ck, nck, ncg, delta_softplus;   // ck: 16
   // Split along the sequence: ld = row stride of the [.., L] tensors (the whole sequence), ns segments per
-  // sequence, B counts (batch, segment) pairs, L is the segment length (a multiple of 16; the last segment may
-  // be shorter), nck the checkpoints of a whole sequence; dhL / dh0 are indexed by the pair, h0 by the batch element.
+  // sequence, B counts (batch, segment) pairs, L is the segment length (a multiple of 32; the last segment may
+  // be shorter), nck the checkpoints of a whole sequence; seg, segq: adjoints of the segments (as FwdArgs, one entry per
+  // segment); dhL, dh0 and h0 are indexed by the batch element.
   int ld, ns;
+  const float *seg, *segq;
   // A launch handles a block of states from nbase on (complex 16, real 24); larger N takes one launch per block.  accum: a later block - the sums over the states
   // (du, ddelta, dtheta, drho) are added to what the earlier blocks wrote, and the terms that do not
   // depend on the state (the D skip, dD) are left out.

@@ -126,9 +126,18 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
     const int n = n0 + k;
     gr[k] = 0.f; gi[k] = 0.f;
     if (p.dhL && dok && n < N) {
-      const size_t o = (((size_t)vb * D + d) * N + n) * 2;
+      const size_t o = (((size_t)b * D + d) * N + n) * 2;
       gr[k] = p.dhL[o]; gi[k] = p.dhL[o + 1];
     }
+  }
+  if (p.seg) {
+    int nn[NW];
+    float a2[NW];
+    const int dc = dok ? d : D - 1;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) { nn[k] = n0 + k < N ? n0 + k : N - 1; a2[k] = 0.f; }
+    const size_t e = ((size_t)b * p.ns + p.ns - 1) * D + dc;
+    seg_chain<VAR_UNITARY, true, NW>(p.seg + e * N * 2, p.segq + e * 2, -(ptrdiff_t)D * N * 2, -(ptrdiff_t)D * 2, p.ns - 1 - sg, nn, a2, gr, gi);
   }
 
   // ---- staging-side mapping (lanes run along time)
@@ -399,12 +408,12 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
     // and the next scan writes s_part only after the next barrier.
   }
 
-  if (p.dh0 && active && dok) {
+  if (p.dh0 && active && dok && sg == 0) {
 #pragma unroll
     for (int k = 0; k < NW; ++k) {
       const int n = n0 + k;
       if (n < N) {
-        const size_t o = (((size_t)vb * D + d) * N + n) * 2;
+        const size_t o = (((size_t)b * D + d) * N + n) * 2;
         p.dh0[o] = gr[k]; p.dh0[o + 1] = gi[k];
       }
     }

@@ -371,12 +371,13 @@ __global__ __launch_bounds__(256) void unitary_bwd_xdl_kernel(const UniBwdArgs p
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
       if (n < N) {
-        const size_t o = ((seg_entry(bb, sg, p) * D + d) * N + n) * 2;
+        const size_t o = (((size_t)bb * D + d) * N + n) * 2;
         Ar[i] = p.dhL[o];
         Ai[i] = p.dhL[o + 1];
       }
     }
   }
+  if (p.seg) seg_enter<true>(p, bb, sg, dc, g, Ar, Ai);
   float accD = 0.0f;
   // dB / dC output: lane (at_n, at_x) of a closing wavefront adds element (row n = 2 k + at_n,
   // timestep at_x / 2, part at_x % 2) of its tile, k = 0..7
@@ -742,12 +743,12 @@ __global__ __launch_bounds__(256) void unitary_bwd_xdl_kernel(const UniBwdArgs p
   }
   flush_dbc(0);
 
-  if (p.dh0 && dok) {
+  if (p.dh0 && dok && sg == 0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
       if (n < N) {
-        const size_t o = (((size_t)b * D + d) * N + n) * 2;
+        const size_t o = (((size_t)bb * D + d) * N + n) * 2;
         p.dh0[o] = Ar[i];
         p.dh0[o + 1] = Ai[i];
       }

@@ -367,6 +367,53 @@ __device__ __forceinline__ void store_grad4(float* p, size_t ob, const f4& v, in
   }
 }
 
+// A call that is split along the sequence: what enters a segment, from what the segments before it (ADJ: behind it) make of a
+// zero state.  Each of them acts on the state as h -> q h + Z with Z [entry][D][N][C] and q from [entry][D][2] (complex: the
+// product of the a_l; real: the sum of the step sizes, q = exp(A sum)); the adjoint takes conj(q).  Every workgroup walks the
+// entries ahead of its segment itself, K states per lane, four entries in flight: a chain kernel between the two passes took
+// 5 - 9 us and a launch gap (B16 D128 N16 L1024 unitary forward: chain 6.5, scan 16.4 -> 17.4 us without).  z, q: first entry, at the lane's channel; zs, qs: floats from one entry to the next walked;
+// n: the lane's states (valid indices); a2: real, A log2(e).
+template <int VAR, bool ADJ, int K>
+__device__ __forceinline__ void seg_chain(const float* __restrict__ z, const float* __restrict__ q, ptrdiff_t zs, ptrdiff_t qs, int cnt,
+                                          const int (&n)[K], const float (&a2)[K], float (&hr)[K], float (&hi)[K]) {
+  constexpr int U = 4;
+#pragma unroll 1
+  for (int j = 0; j < cnt; j += U) {
+    float zr[U][K], zi[U][K], qr[U], qi[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const ptrdiff_t e = j + i < cnt ? j + i : cnt - 1;
+      const float2 qq = *reinterpret_cast<const float2*>(q + e * qs);
+      qr[i] = qq.x; qi[i] = qq.y;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        if (VAR == VAR_REAL) {
+          zr[i][k] = z[e * zs + n[k]]; zi[i][k] = 0.f;
+        } else {
+          const float2 v = *reinterpret_cast<const float2*>(z + e * zs + 2 * n[k]);
+          zr[i][k] = v.x; zi[i][k] = v.y;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      if (j + i < cnt) {                                     // uniform
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (VAR == VAR_REAL) {
+            hr[k] = fmaf(__builtin_amdgcn_exp2f(qr[i] * a2[k]), hr[k], zr[i][k]);
+          } else {
+            const float x = qr[i], y = ADJ ? -qi[i] : qi[i];
+            const float nr = fmaf(x, hr[k], fmaf(-y, hi[k], zr[i][k]));
+            hi[k] = fmaf(x, hi[k], fmaf(y, hr[k], zi[i][k]));
+            hr[k] = nr;
+          }
+        }
+      }
+    }
+  }
+}
+
 // sin and cos without the large-argument branch: the caller keeps |x| below ~150.
 __device__ __forceinline__ void sincos_small(float x, float* sn, float* cs) {
   const float kf = rintf(x * 0.636619772367581343f);

@@ -38,11 +38,63 @@ typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 
 
-// entry of the array of segment states (or adjoints) that segment sg of batch element bb starts from
-template <typename Args>
-__device__ __forceinline__ size_t seg_entry(int bb, int sg, const Args& p) {
-  const int e = sg * p.hs + p.ho;
-  return (size_t)bb * p.nf + (e < p.nf ? e : p.nf - 1);
+// State (ADJ: adjoint) that enters segment sg of batch element bb of a split call: lane (dl, g) holds n = 4 g + i of channel d.
+// part of parts: the entries in as many runs; part 0 applies the first to (hr, hi), any other starts from zero and
+// composes its run, whose product goes to (pr, pi).
+template <bool ADJ, typename Args>
+__device__ __forceinline__ void seg_enter(const Args& p, int bb, int sg, int d, int g, f4& hr, f4& hi, int part = 0, int parts = 1,
+                                          float* pr = nullptr, float* pi = nullptr) {
+  const int own = (sg + (ADJ ? 1 : 0)) * p.hs;
+  const int all = ADJ ? (p.nf > own ? p.nf - own : 0) : own, per = (all + parts - 1) / parts, from = part * per;
+  const int cnt = all - from < per ? all - from : per;
+  const size_t e = ((size_t)bb * p.nf + (ADJ ? p.nf - 1 : 0)) * p.D + d;
+  const ptrdiff_t st = ADJ ? -(ptrdiff_t)p.D : (ptrdiff_t)p.D;
+  const float* z = p.seg + e * p.N * 2 + from * st * p.N * 2;
+  const float* q = p.segq + e * 2 + from * st * 2;
+  const ptrdiff_t zs = st * p.N * 2, qs = st * 2;
+  float xr = 1.0f, xi = 0.0f;
+  constexpr int U = 4;
+#pragma unroll 1
+  for (int j = 0; j < cnt; j += U) {
+    f4 za[U], zb[U];
+    float2 qq[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const ptrdiff_t o = j + i < cnt ? j + i : cnt - 1;
+      qq[i] = *reinterpret_cast<const float2*>(q + o * qs);
+      if (p.N == XN) {                                       // (uniform; the entries lie on 16 bytes)
+        const f4* zz = reinterpret_cast<const f4*>(z + o * zs + 8 * g);
+        za[i] = zz[0]; zb[i] = zz[1];
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int n = 4 * g + k < p.N ? 4 * g + k : p.N - 1;
+          const float2 v = *reinterpret_cast<const float2*>(z + o * zs + 2 * n);
+          (k < 2 ? za : zb)[i][2 * (k & 1)] = v.x;
+          (k < 2 ? za : zb)[i][2 * (k & 1) + 1] = v.y;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      if (j + i < cnt) {                                     // uniform
+        const float x = qq[i].x, y = ADJ ? -qq[i].y : qq[i].y, t = fmaf(x, xr, -y * xi);
+        xi = fmaf(x, xi, y * xr);
+        xr = t;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const f4& v = k < 2 ? za[i] : zb[i];
+          const float nr = fmaf(x, hr[k], fmaf(-y, hi[k], v[2 * (k & 1)]));
+          hi[k] = fmaf(x, hi[k], fmaf(y, hr[k], v[2 * (k & 1) + 1]));
+          hr[k] = nr;
+        }
+      }
+    }
+  }
+  if (pr) { *pr = xr; *pi = xi; }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (4 * g + i >= p.N) { hr[i] = 0.f; hi[i] = 0.f; }
 }
 
 __device__ __forceinline__ f4 xdl(const u4& a, const u4& b, f4 c) {
@@ -447,12 +499,14 @@ __global__ __launch_bounds__(256) void unitary_fwd_xdl_kernel(const FwdArgs p) {
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
       if (n < N) {
-        const size_t o = ((seg_entry(bb, sg, p) * D + d) * N + n) * 2;
+        const size_t o = (((size_t)bb * D + d) * N + n) * 2;
         Hr[i] = p.h0[o];
         Hi[i] = p.h0[o + 1];
       }
     }
   }
+
+  if (p.seg) seg_enter<false>(p, bb, sg, dc, g, Hr, Hi);
 
   int i0 = 0, i1 = 1, i2 = 2;   // LDS slots of chunks c, c+1, c+2
   const int ck_chunks = p.ck / XT;
@@ -733,12 +787,12 @@ __global__ __launch_bounds__(256) void unitary_fwd_xdl_kernel(const FwdArgs p) {
   }
 
   if (p.aux && blockIdx.x == 0 && tid == 0) p.aux[(size_t)(p.B / p.ns) * D * p.ld] = __uint_as_float(p.auxtag);
-  if (p.hL && dok) {
+  if (p.hL && dok && sg == p.ns - 1) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
       if (n < N) {
-        const size_t o = (((size_t)b * D + d) * N + n) * 2;
+        const size_t o = (((size_t)bb * D + d) * N + n) * 2;
         p.hL[o] = Hr[i];
         p.hL[o + 1] = Hi[i];
       }

@@ -271,12 +271,22 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
     hr[s] = 0.f; hi[s] = 0.f; a2[s] = 0.f; mr[s] = 0.f; mi[s] = 0.f;
     if (dok && n < N) {
       if (p.h0) {
-        const size_t o = (((size_t)vb * D + d) * N + n) * C;
+        const size_t o = (((size_t)b * D + d) * N + n) * C;
         hr[s] = p.h0[o];
         if (C == 2) hi[s] = p.h0[o + C - 1];
       }
       if (VAR == VAR_REAL) a2[s] = p.A[(size_t)d * N + n] * LOG2E;
     }
+  }
+  if (!LEAN && p.seg && live) {
+    int nn[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) nn[s] = 8 * s + g < N ? 8 * s + g : N - 1;
+    const size_t e = (size_t)b * p.ns * D + dd;
+    seg_chain<VAR, false, S>(p.seg + e * N * C, p.segq + e * 2, (ptrdiff_t)D * N * C, (ptrdiff_t)D * 2, sg, nn, a2, hr, hi);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (8 * s + g >= N) { hr[s] = 0.f; hi[s] = 0.f; }
   }
   // the last group's lanes without a state: their w is zero (an infinite w times B = 0 would not be)
   const bool has_last = FULLN || 8 * (S - 1) + g < N;
@@ -527,12 +537,13 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
       }
     }
   }
-  if (p.hL && dok) {
+  if (p.clear && blockIdx.x == 0 && (tid == 0 || (tid >= AUX_IMG_FP && tid < AUX_IMG_FP + 8))) p.clear[tid] = 0.f;
+  if (p.hL && dok && (LEAN || sg == p.ns - 1)) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int n = 8 * s + g;
       if (n < N) {
-        const size_t o = (((size_t)vb * D + d) * N + n) * C;
+        const size_t o = (((size_t)(LEAN ? vb : b) * D + d) * N + n) * C;
         p.hL[o] = hr[s];
         if (C == 2) p.hL[o + 1] = hi[s];
       }
@@ -540,6 +551,16 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
   }
 }
 
+// ---- Splitting along the sequence.  With few (batch, channel group) pairs a launch leaves most of the chip idle, so the sequence
+// is cut into ns segments and the scan runs over (batch, segment) pairs:
+//   forward   1. oct_fwd_kernel over the pairs from a zero state, outputs off (LEAN): end state Z_k of every segment and the
+//                product q_k of its a_l (FwdArgs::ptot),
+//             2. oct_fwd_kernel over the pairs, each from  h <- q_k h + Z_k  over the segments before it (seg_chain);
+//   backward  1. oct_adj_kernel: adjoint Y_k of the state entering every segment from a zero adjoint at its end (the reverse
+//                recurrence alone - no states are needed for it), and q_k,
+//             2. oct_bwd_kernel over the pairs, each from  g <- conj(q_k) g + Y_k  over the segments behind it.
+// The reference itself does not split.
+//
 // Adjoint of the state that enters a segment, from a zero adjoint at its end, and the product of its a_l: the reverse
 // recurrence  g <- conj(a_l) (g + conj(C_l) dy_l silu(z_l))  alone.
 template <int VAR, int S, bool FULLN, typename Tin, typename Tbc>
@@ -778,11 +799,21 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
     if (dok && n < NT_) {
       if (VAR == VAR_REAL) { an[s] = p.A[(size_t)d * NT_ + n]; a2[s] = an[s] * LOG2E; }
       if (p.dhL) {
-        const size_t o = (((size_t)vb * D + d) * NT_ + n) * C;
+        const size_t o = (((size_t)b * D + d) * NT_ + n) * C;
         gr[s] = p.dhL[o];
         if (C == 2) gi[s] = p.dhL[o + 1];
       }
     }
+  }
+  if (p.seg && live) {
+    int nn[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) nn[s] = p.nbase + (8 * s + g < N ? 8 * s + g : N - 1);
+    const size_t e = ((size_t)b * p.ns + p.ns - 1) * D + dd;
+    seg_chain<VAR, true, S>(p.seg + e * NT_ * C, p.segq + e * 2, -(ptrdiff_t)D * NT_ * C, -(ptrdiff_t)D * 2, p.ns - 1 - sg, nn, a2, gr, gi);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (8 * s + g >= N) { gr[s] = 0.f; gi[s] = 0.f; }
   }
   const bool has_last = FULLN || 8 * (S - 1) + g < N;
 
@@ -1261,8 +1292,8 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
       for (int s = 0; s < S; ++s) {
         const int n = p.nbase + 8 * s + g;
         if (n < NT_) {
-          if (p.dh0) {
-            const size_t o = (((size_t)vb * D + d) * NT_ + n) * C;
+          if (p.dh0 && sg == 0) {
+            const size_t o = (((size_t)b * D + d) * NT_ + n) * C;
             p.dh0[o] = gr[s];
             if (C == 2) p.dh0[o + 1] = gi[s];
           }

@@ -25,28 +25,30 @@
 #pragma once
 #include "scan_bwd_xdl.h"
 #include "scan_fwd_xdl.h"
+#include "scan_seg_xdl.h"
 
 namespace aussm {
 
 // One workgroup (256 threads) per (batch element, chunk).  CHECK: the launch of a backward call, which has
 // nothing to do when the forward call of the same tensors has left the images (its own instance, so that a
 // profile tells the two launches of a training step apart).
+// (the records the images do not hold - [Ci, Cr] and [-Bi, Br] - are formed in registers where the products
+// need them: 48 KiB instead of 60 per workgroup, three workgroups per compute unit instead of two, so that one
+// workgroup's stores - half of its life - overlap the others' loads and products)
+struct PrepLds {
+  u4 cs_r[PX_NP][XT * 4];   // row t: [ Cr[4g..], -Ci[4g..] ]
+  u4 bs[PX_NP][XT * 4];     // row s: [ Br[4g..],  Bi[4g..] ]
+  u4 bt_r[PX_NP][XN * 4];   // row n: Br[t(g,e)][n]
+  u4 bt_i[PX_NP][XN * 4];
+  u4 ct_r[PX_NP][XN * 4];   // row n: Cr[t(g,e)][n]
+  u4 ct_i[PX_NP][XN * 4];
+  XbG<PX_NP> g;
+};
 template <typename Tin, bool CHECK>
-__global__ __launch_bounds__(256) void unitary_px_prep_kernel(const PrepArgs p) {
+__device__ __forceinline__ void px_prep_body(const PrepArgs& p, char* mem, int block) {
   constexpr int NP = PX_NP;
-  // (the records the images do not hold - [Ci, Cr] and [-Bi, Br] - are formed in registers where the products
-  // need them: 48 KiB instead of 60 per workgroup, three workgroups per compute unit instead of two, so that one
-  // workgroup's stores - half of its life - overlap the others' loads and products)
-  struct PrepBC {
-    u4 cs_r[NP][XT * 4];   // row t: [ Cr[4g..], -Ci[4g..] ]
-    u4 bs[NP][XT * 4];     // row s: [ Br[4g..],  Bi[4g..] ]
-    u4 bt_r[NP][XN * 4];   // row n: Br[t(g,e)][n]
-    u4 bt_i[NP][XN * 4];
-    u4 ct_r[NP][XN * 4];   // row n: Cr[t(g,e)][n]
-    u4 ct_i[NP][XN * 4];
-  };
-  __shared__ PrepBC s_bc;
-  __shared__ XbG<NP> s_g;
+  PrepLds& s_bc = *reinterpret_cast<PrepLds*>(mem);
+  XbG<NP>& s_g = s_bc.g;
 
   // the images a forward call left behind are still those of these tensors: nothing to do
   if (CHECK && p.have) {
@@ -55,7 +57,7 @@ __global__ __launch_bounds__(256) void unitary_px_prep_kernel(const PrepArgs p) 
     for (int i = 0; i < 8; ++i) same &= __builtin_amdgcn_readfirstlane(p.have[i]) == p.want.w[i];
     if (same) return;
   }
-  const int bb = blockIdx.x / p.nch, c = blockIdx.x % p.nch;
+  const int bb = block / p.nch, c = block % p.nch;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int dl = lane & 15, g = lane >> 4;
   const int N = p.N, L = p.ld;
@@ -189,6 +191,22 @@ __global__ __launch_bounds__(256) void unitary_px_prep_kernel(const PrepArgs p) 
   }
 }
 
+template <typename Tin, bool CHECK>
+__global__ __launch_bounds__(256) void unitary_px_prep_kernel(const PrepArgs p) {
+  __shared__ __align__(16) char s_mem[sizeof(PrepLds)];
+  px_prep_body<Tin, CHECK>(p, s_mem, blockIdx.x);
+}
+
+// The forward call of a sequence that is split along L: segment states (the first nseg workgroups, the longer ones) and images
+// in one launch, neither needs the other's results.  B16 D128 N16 L1024 forward: 9.7 + 6.5 us and a launch gap -> 10.6 us.
+template <typename Tin>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void unitary_prep_seg_kernel(const PrepArgs p, const SegArgs sa,
+                                                                                                     int nseg) {
+  __shared__ __align__(16) char s_mem[sizeof(PrepLds) > SEG_STATE_LDS ? sizeof(PrepLds) : SEG_STATE_LDS];
+  if ((int)blockIdx.x < nseg) seg_state_body<3, false, Tin>(sa, s_mem, blockIdx.x, nseg);
+  else px_prep_body<Tin, false>(p, s_mem, blockIdx.x - nseg);
+}
+
 // ---- global memory -> LDS without passing through registers: a wavefront moves 64 records (1 KiB)
 // per instruction, lane i's record to lds + i.  The data is in LDS once the wavefront's vector-memory
 // counter says so (px_loads_done / px_wait) and a barrier has published it.  The instruction is
@@ -240,6 +258,16 @@ template <> struct PxRaw4<bf16_t> {
     return (i & 1) ? bf16_hi(w) : bf16_lo(w);
   }
 };
+
+// (hr, hi) <- q (hr, hi) + (zr, zi)
+__device__ __forceinline__ void seg_compose(const f4& q, const f4& zr, const f4& zi, f4& hr, f4& hi) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float x = fmaf(q[0], hr[i], fmaf(-q[1], hi[i], zr[i]));
+    hi[i] = fmaf(q[0], hi[i], fmaf(q[1], hr[i], zi[i]));
+    hr[i] = x;
+  }
+}
 
 // [x0..x3, y0..y3] with (x, y) = (Cr, -Ci)  ->  (Ci, Cr): the imaginary-part record of C from the real-part one
 template <int NP>
@@ -395,21 +423,34 @@ __global__ __launch_bounds__(512) void unitary_fwd_px_kernel(const FwdArgs p, co
   };
 
   // ---- prologue: start state, first images, inputs of this wavefront's first chunk
-  if (hf == 0) {
+  {
     f4 hr = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
-    if (p.h0 && dok) {
+    if (p.h0 && dok && hf == 0) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int n = 4 * g + i;
         if (n < N) {
-          const size_t o = ((seg_entry(bb, sg, p) * D + d) * N + n) * 2;
+          const size_t o = (((size_t)bb * D + d) * N + n) * 2;
           hr[i] = p.h0[o];
           hi[i] = p.h0[o + 1];
         }
       }
     }
-    s_h[0][cg][0][lane] = hr;
-    s_h[0][cg][1][lane] = hi;
+    if (p.seg) {                                     // a split call: the partners of a channel group walk half of the entries each
+      float qr, qi;
+      seg_enter<false>(p, bb, sg, dc, g, hr, hi, hf, 2, &qr, &qi);
+      if (hf == 1) {
+        s_h[0][cg][0][lane] = f4{qr, qi, 0, 0};
+        s_h[1][cg][0][lane] = hr;
+        s_h[1][cg][1][lane] = hi;
+      }
+      __syncthreads();
+      if (hf == 0) seg_compose(s_h[0][cg][0][lane], s_h[1][cg][0][lane], s_h[1][cg][1][lane], hr, hi);
+    }
+    if (hf == 0) {
+      s_h[0][cg][0][lane] = hr;
+      s_h[0][cg][1][lane] = hi;
+    }
   }
   img_load(0, 0);
   img_store(0, 0, std::integral_constant<int, 0>{});
@@ -607,13 +648,13 @@ __global__ __launch_bounds__(512) void unitary_fwd_px_kernel(const FwdArgs p, co
   // (the pre-pass that wrote the images has finished: this kernel read them)
   if (note.dst && blockIdx.x == 0 && tid < 8) note.dst[tid] = note.stamp.w[tid];
   if (note.clear && blockIdx.x == 0 && tid == 0) *note.clear = 0.0f;
-  if (p.hL && dok && hf == 0) {
+  if (p.hL && dok && hf == 0 && sg == p.ns - 1) {
     const f4 hr = s_h[0][cg][0][lane], hi = s_h[0][cg][1][lane];    // state after the last (possibly padding) chunk
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
       if (n < N) {
-        const size_t o = (((size_t)b * D + d) * N + n) * 2;
+        const size_t o = (((size_t)bb * D + d) * N + n) * 2;
         p.hL[o] = hr[i];
         p.hL[o + 1] = hi[i];
       }
@@ -1152,23 +1193,38 @@ __global__ __launch_bounds__(512) void unitary_bwd_px_kernel(const UniBwdArgs p,
   auto idle = [&](int i) { flush_acc(i); lds_barrier(); lds_barrier(); };
 
   // ---- prologue: end state and its adjoint into the carry, first images, first inputs
-  if (hf == 0) {
+  {
     f4 hr = {0, 0, 0, 0}, hi = hr, ar = hr, ai = hr;
     const float* __restrict__ cp = p.hck + ((size_t)bb * p.nck + sg * (p.L / p.ck) + ((L + p.ck - 1) / p.ck - 1)) * ck_stride + dc;
+    if (hf == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int n = 4 * g + i;
-      if (n < N) {
-        hr[i] = cp[(size_t)n * 2 * D];
-        hi[i] = cp[(size_t)n * 2 * D + D];
-        if (p.dhL && dok) {
-          const size_t o = ((seg_entry(bb, sg, p) * D + d) * N + n) * 2;
-          ar[i] = p.dhL[o];
-          ai[i] = p.dhL[o + 1];
+      for (int i = 0; i < 4; ++i) {
+        const int n = 4 * g + i;
+        if (n < N) {
+          hr[i] = cp[(size_t)n * 2 * D];
+          hi[i] = cp[(size_t)n * 2 * D + D];
+          if (p.dhL && dok) {
+            const size_t o = (((size_t)bb * D + d) * N + n) * 2;
+            ar[i] = p.dhL[o];
+            ai[i] = p.dhL[o + 1];
+          }
         }
       }
     }
-    s_x[cg][0][lane] = hr; s_x[cg][1][lane] = hi; s_x[cg][2][lane] = ar; s_x[cg][3][lane] = ai;
+    if (p.seg) {                                     // a split call: the partners of a channel group walk half of the entries each
+      float qr, qi;
+      seg_enter<true>(p, bb, sg, dc, g, ar, ai, hf, 2, &qr, &qi);
+      if (hf == 1) {
+        s_x[cg][0][lane] = f4{qr, qi, 0, 0};
+        s_x[cg][2][lane] = ar;
+        s_x[cg][3][lane] = ai;
+      }
+      __syncthreads();
+      if (hf == 0) seg_compose(s_x[cg][0][lane], s_x[cg][2][lane], s_x[cg][3][lane], ar, ai);
+    }
+    if (hf == 0) {
+      s_x[cg][0][lane] = hr; s_x[cg][1][lane] = hi; s_x[cg][2][lane] = ar; s_x[cg][3][lane] = ai;
+    }
   }
   // images of chunk indices 0 and 1 (all eight wavefronts take part, here only)
   {
@@ -1203,13 +1259,13 @@ __global__ __launch_bounds__(512) void unitary_bwd_px_kernel(const UniBwdArgs p,
     flush_acc(2 * npairs + 1);          // (what the second half accumulated in the last interval)
   }
 
-  if (p.dh0 && dok && hf == 0) {
+  if (p.dh0 && dok && hf == 0 && sg == 0) {
     const f4 ar = s_x[cg][2][lane], ai = s_x[cg][3][lane];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * g + i;
       if (n < N) {
-        const size_t o = (((size_t)b * D + d) * N + n) * 2;
+        const size_t o = (((size_t)bb * D + d) * N + n) * 2;
         p.dh0[o] = ar[i];
         p.dh0[o + 1] = ai[i];
       }

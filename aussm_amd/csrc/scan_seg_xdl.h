@@ -8,9 +8,8 @@
 //      parallel; only the sums  Z = P sum_s conj(P_s) delta_s u_s B_s,  Y = sum_t conj(P_t) dy_t conj(C_t)
 //      are formed: per chunk one product with the channel as free index, on the matrix cores in
 //      the layout of the scan kernels),
-//   2. chains the segments of each (batch, channel, state) with seg_carry_*_kernel (ns steps),
-//   3. runs the scan kernel proper with (batch, segment) pairs as its batch index, every segment
-//      starting from its true incoming state or adjoint.
+//   2. runs the scan kernel proper with (batch, segment) pairs as its batch index, every segment
+//      starting from what the segments before it make of the state (seg_chain).
 #pragma once
 #include <type_traits>
 
@@ -22,15 +21,16 @@ namespace aussm {
 // ADJ = false: Z of each segment, chunks in forward order,  H <- P_T (H + B^T V).
 // ADJ = true:  Y of each segment, chunks in reverse order,  A <- conj(P_T) A + conj(C)^T Q.
 // Requires N <= 16, L % 4 == 0, 16-byte aligned tensors.  Tin: float or bf16_t (u, delta, B, C).
-// Four wavefronts per SIMD (128 registers): the launch of a split call (1024 light workgroups for 64 fine segments
-// of a batch of 4 x 4 channel groups) then fits the chip in one round instead of one and a third.
+// mem: SEG_STATE_LDS bytes of LDS; block of blocks: the workgroup's index in this part of the launch.
+constexpr int SEG_STATE_LDS = 2 * 2 * 3 * XN * 4 * 16;
 template <int NP, bool ADJ, typename Tin = float>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void unitary_seg_state_kernel(const SegArgs p) {
+__device__ __forceinline__ void seg_state_body(const SegArgs& p, char* mem, int block, int blocks) {
   // row n: M[t(g, e)][n], real and imaginary parts (the imaginary part negated for ADJ: conj(C))
-  __shared__ u4 s_mr[2][NP][XN * 4];
-  __shared__ u4 s_mi[2][NP][XN * 4];
+  static_assert(NP <= 3, "LDS is sized for three pieces");
+  u4 (*s_mr)[NP][XN * 4] = reinterpret_cast<u4 (*)[NP][XN * 4]>(mem);
+  u4 (*s_mi)[NP][XN * 4] = s_mr + 2;
 
-  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int wg = xcd_remap(block, blocks);
   const int vb = wg / p.ncg, d0 = (wg % p.ncg) * CH;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int dl = lane & 15, g = lane >> 4;
@@ -206,69 +206,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   }
 }
 
-// Chains the segments of one (batch, channel, state).  Forward (ADJ false): on entry seg[k] holds Z_k, on return the
-// state that enters segment k; the state after the last segment goes to `last` (if wanted); `first` is the state
-// before the first one (or null).  ADJ: on entry seg[k] holds Y_k, on return the adjoint that enters segment k at
-// its end, walking from the last segment with conj(q_k); `first` is the adjoint after the last segment, `last`
-// receives the adjoint of the initial state.
-// The chain is short and there are few of them (B D N), so one thread per chain leaves the chip waiting on its
-// loads: CARRY_SUBS threads share a chain - each composes its run of consecutive segments into one affine map
-// h -> Q h + Z, the maps of the runs before it (LDS) give the state that enters its run, and it walks the run
-// again writing every segment's incoming state.
-constexpr int CARRY_SUBS = 8;          // threads per chain
-constexpr int CARRY_RUN = 16;          // segments per thread at most: chains of up to 128 segments
-template <bool ADJ>
-__global__ __launch_bounds__(32 * CARRY_SUBS) void seg_carry_kernel(float* __restrict__ seg, const float* __restrict__ ptot,
-                                                                    const float* __restrict__ first, float* __restrict__ last,
-                                                                    int B, int D, int N, int ns) {
-  __shared__ float4 s_map[CARRY_SUBS][32];          // (Re Q, Im Q, Re Z, Im Z) of every run
-  const int cl = threadIdx.x & 31, sub = threadIdx.x >> 5;
-  const size_t idx = (size_t)blockIdx.x * 32 + cl;
-  const bool ok = idx < (size_t)B * D * N;
-  const size_t ic = ok ? idx : 0;
-  const int n = (int)(ic % N);
-  const int d = (int)((ic / N) % D);
-  const int b = (int)(ic / ((size_t)N * D));
-  const int per = (ns + CARRY_SUBS - 1) / CARRY_SUBS;
-  auto mul = [](float2 q, float hr, float hi) {          // q h, or conj(q) h for the adjoint
-    return ADJ ? make_float2(q.x * hr + q.y * hi, q.x * hi - q.y * hr) : make_float2(q.x * hr - q.y * hi, q.x * hi + q.y * hr);
-  };
-  float2 z[CARRY_RUN], q[CARRY_RUN];
-  size_t off[CARRY_RUN];
-#pragma unroll
-  for (int j = 0; j < CARRY_RUN; ++j) {
-    const int pos = sub * per + j;
-    const bool valid = j < per && pos < ns;
-    const int k = valid ? (ADJ ? ns - 1 - pos : pos) : 0;
-    const size_t v = ((size_t)b * ns + k) * D + d;
-    off[j] = valid ? (v * N + n) * 2 : ~(size_t)0;
-    z[j] = valid ? *reinterpret_cast<const float2*>(seg + (v * N + n) * 2) : make_float2(0.f, 0.f);
-    q[j] = valid ? *reinterpret_cast<const float2*>(ptot + v * 2) : make_float2(1.f, 0.f);
-  }
-  float Qr = 1.f, Qi = 0.f, Zr = 0.f, Zi = 0.f;
-#pragma unroll
-  for (int j = 0; j < CARRY_RUN; ++j) {
-    const float2 a = mul(q[j], Qr, Qi), c = mul(q[j], Zr, Zi);
-    Qr = a.x; Qi = a.y; Zr = c.x + z[j].x; Zi = c.y + z[j].y;
-  }
-  s_map[sub][cl] = make_float4(Qr, Qi, Zr, Zi);
-  __syncthreads();
-  float hr = first ? first[ic * 2] : 0.0f, hi = first ? first[ic * 2 + 1] : 0.0f;
-  for (int s_ = 0; s_ < sub; ++s_) {
-    const float4 m = s_map[s_][cl];
-    // (the maps hold q's products already conjugated for the adjoint: plain complex multiplication here)
-    const float nr = m.x * hr - m.y * hi + m.z, ni = m.x * hi + m.y * hr + m.w;
-    hr = nr; hi = ni;
-  }
-#pragma unroll
-  for (int j = 0; j < CARRY_RUN; ++j) {
-    if (off[j] != ~(size_t)0) {
-      if (ok) *reinterpret_cast<float2*>(seg + off[j]) = make_float2(hr, hi);
-      const float2 a = mul(q[j], hr, hi);
-      hr = a.x + z[j].x; hi = a.y + z[j].y;
-    }
-  }
-  if (last && ok && sub == CARRY_SUBS - 1) { last[idx * 2] = hr; last[idx * 2 + 1] = hi; }
+// Four wavefronts per SIMD (128 registers): the launch of a split call (1024 light workgroups for 64 fine segments
+// of a batch of 4 x 4 channel groups) then fits the chip in one round instead of one and a third.
+template <int NP, bool ADJ, typename Tin = float>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void unitary_seg_state_kernel(const SegArgs p) {
+  __shared__ __align__(16) char s_mem[SEG_STATE_LDS];
+  seg_state_body<NP, ADJ, Tin>(p, s_mem, blockIdx.x, gridDim.x);
 }
 
 }  // namespace aussm
