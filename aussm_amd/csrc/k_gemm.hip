@@ -22,19 +22,28 @@ static int launch_tile(const XGemmArgs& a, unsigned grid, hipStream_t s) {
 struct Tile { int wm, em, en; };        // wavefronts along the rows; 16-wide row and column tiles per wavefront
 constexpr int rows_of(const Tile& t) { return 16 * t.em * t.wm; }
 constexpr int cols_of(const Tile& t) { return 16 * t.en * (t.wm == 4 ? 2 : 4 / t.wm); }
-constexpr Tile NARROW{2, 4, 4}, COLS64{2, 4, 2}, COLS32{2, 4, 1}, ROWS64{1, 4, 2}, ROWS32{1, 2, 2}, WIDE128{4, 4, 4}, WIDE96{4, 4, 3};
+constexpr Tile NARROW{2, 4, 4}, COLS64{2, 4, 2}, COLS32{2, 4, 1}, ROWS32{1, 2, 2}, WIDE128{4, 4, 4}, WIDE96{4, 4, 3};
+constexpr Tile T64{2, 2, 2}, R32C64{1, 2, 1}, R64C32{2, 2, 1}, T32{2, 1, 1};       // 64 x 64, 32 x 64, 64 x 32, 32 x 32
 
 template <bool QUAD>
 static int launch_xgemm(const Tile& t, const XGemmArgs& a, unsigned grid, hipStream_t s) {
 #define XT(T_) if (t.wm == T_.wm && t.em == T_.em && t.en == T_.en) return launch_tile<T_.wm, T_.em, T_.en, QUAD>(a, grid, s);
-  XT(NARROW) XT(COLS64) XT(COLS32) XT(ROWS64) XT(ROWS32) XT(WIDE128) XT(WIDE96)
+  XT(NARROW) XT(COLS64) XT(COLS32) XT(ROWS32) XT(WIDE128) XT(WIDE96) XT(T64) XT(R32C64) XT(R64C32) XT(T32)
 #undef XT
   return -2;
 }
 
-// Tiles of few rows or few columns where the product has no more: the matrix instructions and the staging of a 128-row
-// tile would mostly work on repeated rows.  (Columns 23040, K = 512: 48 rows 39 -> 30 us, 16 rows 42 -> 27 us; 32 rows,
-// 11264 columns, K = 2048 in slices 44 -> 28 us; 2048 x 32, sums of 11264, 28 -> 23 us.)
+// Small tiles where a product has few of them.  What a step of 32 costs a workgroup is mostly waiting - for the values, for the
+// other wavefronts -, 2.3 us with 128 x 128, 1.4 with 64 x 64, 0.95 with 32 x 32, so a product that leaves the chip
+// part empty is done sooner in many small ones: the smallest tile of which there are at most 256, else 64 x 64 up to 1024 of
+// them.  us, 128-wide tile / the one taken: 256 x 5760, K = 1024 74 / 45; 1000 x 1000, K = 250 31 / 16; 137 x 1008, K = 548
+// 51 / 20; 384 x 954, K = 96 23 / 7.4; 54 x 1320, K = 27 11 / 5.1; 48 x 23040, K = 512 30 / 24; 16 x 131072, K = 32 9.3 with 32 x 64, 8.0
+// with 32 x 128; 512 x 8192, K = 256 (1024 tiles of 64 x 64) 23.9 / 23.2, 1024 x 8192 (2048) 27.4 with the wide tile against 34.8.  Sums over z alike, by the work there is:
+// 64 x 64 up to 18000 tile steps (256 x 512, 736 steps, 23500 of them: 53 against 62; 1024 x 256, 256 steps, 16400: 49 against
+// 45; 512 x 128, 512 steps 56 / 27; 96 x 192, 30 steps 20 / 6.8), for 32 columns or rows up to 4500 (512 x 16, 736 steps, 5900:
+// 13.7 against 15.0; 256 x 16 11.8 / 10.0).  Past that few rows take 32 x 128 (32 x 32768, sums of 2048: 62, 128 x 128 111), or 64 x 64
+// and twice the slices (64 x 23040, 1024: 34.7, with 64 x 128 42.6; 64 x 32768, 4096: 156, 151).
+//
 // Else the wide ones for more rows than the narrow one has, by the rounds that the tiles make on the chip (256 compute
 // units, one wide or two narrow workgroups each) times what a round takes: 1 for 256 x 128, 0.88 for 256 x 96, 1.2 for two of
 // 128 x 128, 0.72 for one.  23040 columns, us narrow / 96 / 128: 256 rows, K = 1024 93 / 70 / 78; 512 rows, K = 256 46 / 43 /
@@ -42,16 +51,34 @@ static int launch_xgemm(const Tile& t, const XGemmArgs& a, unsigned grid, hipStr
 //
 // Slices: a sum over many steps with few tiles is cut into as many workgroups as run at once (more would start a second
 // round: 540 workgroups 140 us, 450 workgroups 91 us for the product with 90 tiles and 128 steps), at least four steps of
-// 32 per slice (shorter ones would spend their time on the atomics of the tile).  The wide tile from 24 steps a slice on:
-// 4096 x 256, sums of 23040, 281 -> 248 us; 256 x 5760, K = 4096 93 -> 81 us; 512 x 256 (12 steps) 56 against 58 us.
+// 32 per slice (shorter ones would spend their time on the atomics of the tile), of small tiles two unless four leave 200
+// workgroups (548 x 137, 36 steps: 10.2 against 11.7 us; 96 x 192, 30 steps: 9.6 against 6.8).  The wide tile from 24 steps a
+// slice on: 4096 x 256, sums of 23040, 281 -> 248 us; 256 x 5760, K = 4096 93 -> 81 us; 512 x 256 (12 steps) 56 against 58 us.
 int run_xgemm(XGemmArgs a, hipStream_t s) {
   if (a.M < 1 || a.N < 1 || a.K < 1 || a.Z < 1 || a.nper < 1) return -2;
   if (a.reduce && a.scm == 1 && a.scn != 1 && a.nper < a.N) return -2;
   const long steps = (long)((a.K + 31) / 32) * a.Z;
   const bool sliced = a.reduce && !a.bias && !a.add && !a.act;
   auto tiles_of = [&](const Tile& t) { return (long)((a.M + rows_of(t) - 1) / rows_of(t)) * ((a.N + cols_of(t) - 1) / cols_of(t)); };
-  Tile tile = a.N <= 32 ? COLS32 : a.N <= 64 ? COLS64 : a.M <= 32 ? ROWS32 : a.M <= 64 ? ROWS64 : NARROW;
-  if (a.M > rows_of(NARROW) && a.N > 64) {
+  Tile tile = a.N <= 32 ? COLS32 : a.N <= 64 ? COLS64 : NARROW;
+  bool small = true;
+  int slots = 512;
+  const Tile half = tiles_of(R64C32) < tiles_of(R32C64) ? R64C32 : R32C64;
+  if (sliced) {
+    if (a.M <= 32 && a.N <= 32) tile = T32;
+    else if ((a.M <= 32 || a.N <= 32) && tiles_of(half) * steps <= 4500) tile = half;
+    else if (a.M > 32 && a.N > 32 && tiles_of(T64) * steps <= 18000) tile = T64;
+    else if (a.M <= 32 && a.N > 64) tile = ROWS32;
+    else if (a.M <= 64 && a.N > 64) tile = T64, slots = 1024;
+    else small = false;
+  } else {
+    if (tiles_of(T32) <= 256) tile = T32;
+    else if (tiles_of(half) <= 256) tile = half;
+    else if (a.M <= 32) tile = tiles_of(half) <= 512 ? half : ROWS32;
+    else if (tiles_of(T64) <= 1024 || a.M <= 64) tile = T64;
+    else small = false;
+  }
+  if (!small && a.M > rows_of(NARROW) && a.N > 64) {
     if (sliced) {
       const long t = tiles_of(WIDE128);
       if (steps >= 24 * (t < 256 ? 256 / t : 1)) tile = WIDE128;
@@ -66,8 +93,9 @@ int run_xgemm(XGemmArgs a, hipStream_t s) {
   const long tiles = tiles_of(tile);
   long sl = 1;
   if (sliced) {
-    sl = (tile.wm == 4 ? 256 : 512) / tiles;
-    if (sl > steps / 4) sl = steps / 4;
+    sl = (tile.wm == 4 ? 256 : slots) / tiles;
+    const long least = small && tiles * (steps / 4) < 200 ? 2 : 4;
+    if (sl > steps / least) sl = steps / least;
     if (sl < 1) sl = 1;
     const long per = (steps + sl - 1) / sl;
     sl = (steps + per - 1) / per;

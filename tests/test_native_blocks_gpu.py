@@ -59,6 +59,14 @@ def test_products_of_a_linear_layer(b, l, i, o):
     assert _rel(dW, want) < 2e-6
 
 
+# tiles of 32 x 32, 64 x 32, 32 x 64 and 64 x 64: whole, one over and one under, few rows of many columns (32 x 64 and
+# 32 x 128), sums over z in slices of two and four steps
+@pytest.mark.parametrize("b,l,i,o", [(1, 32, 32, 32), (1, 33, 31, 33), (3, 65, 63, 64), (6, 150, 97, 66), (8, 400, 128, 256), (5, 401, 129, 127),
+                                     (2, 2001, 6, 31), (10, 4000, 9, 16), (16, 1024, 33, 64), (3, 700, 300, 192)])
+def test_products_on_tiles_of_32_and_64(b, l, i, o):
+    test_products_of_a_linear_layer(b, l, i, o)
+
+
 # ... and shapes large enough for the tiles of eight wavefronts, none a multiple of a tile: 96 columns (both operand orders,
 # results along either index), 128 columns, and slices of a long sum
 @pytest.mark.parametrize("b,l,i,o", [(23, 721, 200, 130), (31, 1027, 256, 200), (64, 2048, 70, 300)])
