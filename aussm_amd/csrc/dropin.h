@@ -14,7 +14,7 @@
 //     three bf16 pieces (scan_fwd_xdl.h), i.e. fp32-accurate, where U is the tile of u[b] prefix-summed along
 //     the tile (sum_{l' <= l} x.u_{l'} = x.U_l), plus (l + 1) x_bias.  The wavefront keeps its rows of x in
 //     registers for the whole launch; the tiles of U, which all wavefronts of a batch element share, are
-//     prepared once per call by a pre-pass (dropin_uprep_kernel) and copied into LDS once per workgroup;
+//     prepared once per call by a pre-pass (dropin_prep_kernel) and copied into LDS once per workgroup;
 //   * the product lands with the timestep along the lanes of a 16-lane row (lane = (timestep l,
 //     state group g), states 4 g .. 4 g + 3 in registers), so the rest of the recurrence is prefix sums
 //     along the row (DPP row shifts, no LDS): E = e^{iG}, p = conj(E) Bt w, R = h_in + prefix(p), h = E R.
@@ -47,6 +47,20 @@ __device__ __forceinline__ float op_radius(const DropinArgs& p, const float* r, 
   return p.raw ? softplusf_(v) : v;
 }
 __device__ __forceinline__ float op_phase(const DropinArgs& p, const float* th, int j) { return th[(size_t)j * p.bcs]; }
+// (Re Bt, Im Bt, Re Ct, Im Ct) of every state, 0 past n, and with UNIT (e^{i B_theta}, e^{i C_theta}), made by the first 128 threads of a
+// workgroup, one polar number each: a sine with its branches in every lane for its own four states, at either end of a kernel,
+// was half of the kernels' code and 3 to 4 us of every launch, mostly fetching it (5 x 48 pairs, 64 steps: 10.9 -> 9.0 us
+// forward, 21.5 -> 15.8 backward).
+template <bool UNIT>
+__device__ __forceinline__ void polar_params(const DropinArgs& p, f4* s_par, f4* s_unit, int tid) {
+  if (tid >= 2 * D_MAXN) return;
+  const int j = tid & (D_MAXN - 1), c = tid / D_MAXN, jc = j < p.n ? j : 0;
+  float sn, cs;
+  fast_sincosf(op_phase(p, c ? p.C_th : p.B_th, jc), &sn, &cs);
+  const float r = j < p.n ? op_radius(p, c ? p.C_r : p.B_r, jc) : 0.0f;
+  reinterpret_cast<float2*>(s_par)[2 * j + c] = make_float2(r * cs, r * sn);
+  if (UNIT) reinterpret_cast<float2*>(s_unit)[2 * j + c] = make_float2(cs, sn);
+}
 // Derivative of the softplus behind dt, from dt itself: 1 - e^-dt, below 1 by its Taylor series (the next term is below
 // 2^-28 of the value).  Measured through the gradient of dt's argument, the rounding of the product included: root mean
 // square of the relative error 4.0e-8 below 0.3, 4.5e-8 up to 1, 3.7e-8 from there on.  (The difference alone cancels:
@@ -94,10 +108,13 @@ __device__ __forceinline__ float row_first(float v, int) { return dpp_perm<0x150
 // x (rows of d: (channel i, state j) at row i xsi + j xsj), times scale -> operand records.  Record (v = i nb + sb, ks, piece, lane = (row = lane % 16, g = lane / 16))
 // holds x[i, 16 sb + row, 32 ks + 8 g .. + 7] (zero past the ends).  One thread per (v, ks, lane).
 // x_out [d, n, d], xb_out [d, n] (or null): scale x and x_bias in the operator's own order, for a caller that keeps them.
-__global__ __launch_bounds__(256) void dropin_xprep_kernel(const float* __restrict__ x, u4* __restrict__ xp, int d, int n, int ks, int nb,
-                                                           int xsi, int xsj, float scale, const float* __restrict__ x_bias,
-                                                           float* __restrict__ x_out, float* __restrict__ xb_out) {
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void xprep_block(const DropinPrepArgs& a, unsigned block) {
+  const int d = a.d, n = a.n, ks = a.ks, nb = a.nb, xsi = a.xsi, xsj = a.xsj;
+  const float scale = a.scale;
+  const float* __restrict__ x = a.x;
+  float* __restrict__ x_out = a.x_out;
+  u4* __restrict__ xp = a.xp;
+  const size_t idx = (size_t)block * 256 + threadIdx.x;
   if (idx >= (size_t)d * nb * ks * 64) return;
   const int lane = (int)(idx & 63);
   const int k = (int)((idx >> 6) % ks), vc = (int)((idx >> 6) / ks);
@@ -121,24 +138,23 @@ __global__ __launch_bounds__(256) void dropin_xprep_kernel(const float* __restri
         if (r0 + q < d) o[q] = v[q];
     }
   }
-  if (xb_out && j < n && k == 0 && g == 0) xb_out[(size_t)i * n + j] = x_bias[(size_t)i * xsi + (size_t)j * xsj];
+  if (a.xb_out && j < n && k == 0 && g == 0) a.xb_out[(size_t)i * n + j] = a.x_bias[(size_t)i * xsi + (size_t)j * xsj];
   u4 pc[3];
   split8<3>(sk, v, pc);
 #pragma unroll
   for (int q = 0; q < 3; ++q) xp[(((size_t)vc * ks + k) * 3 + q) * 64 + lane] = pc[q];
 }
 
-// Tiles of u as the second operand of the phase product, prepared once per call (one workgroup of 256
-// threads per (batch element, tile)): record (k, piece, lane = (column l = lane % 16, g)) holds
+// Tiles of u as the second operand of the phase product, one workgroup of 256 threads per (batch element, tile): record (k, piece, lane = (column l = lane % 16, g)) holds
 // U[32 k + 8 g .. + 7][l], U[r][l] = sum_{l' <= l} u[b, r, l0 + l'] - the prefix sum along the tile - so that
 // the matrix product hands the scan kernels the running phase G = prefix(theta) directly
 // (sum_{l' <= l} sum_r x[i,j,r] u[r,l'] = sum_r x[i,j,r] U[r,l]); timesteps past L count as zero.  All KS steps the
 // kernels are compiled for are written, the ones past ceil(d / 32) as zeros.
-__global__ __launch_bounds__(256) void dropin_uprep_kernel(const float* __restrict__ u, u4* __restrict__ up, int d, int L,
-                                                           int KS, int b0, int t0, int nt) {
-  const int zb = blockIdx.x / nt, t = t0 + blockIdx.x % nt;
-  const float* __restrict__ ub = u + (size_t)(b0 + zb) * d * L;
-  u4* __restrict__ dst = up + (size_t)blockIdx.x * KS * 3 * 64;
+__device__ __forceinline__ void uprep_block(const DropinPrepArgs& a, unsigned block) {
+  const int d = a.d, L = a.L, KS = a.KS;
+  const int zb = block / a.nt, t = a.t0 + block % a.nt;
+  const float* __restrict__ ub = a.u + (size_t)(a.b0 + zb) * d * L;
+  u4* __restrict__ dst = a.up + (size_t)block * KS * 3 * 64;
   const SplitK sk = make_splitk();
   for (int rec = threadIdx.x; rec < KS * 64; rec += 256) {        // (whole wavefronts: 64 records per k)
     const int lane = rec & 63, k = rec >> 6;
@@ -175,16 +191,73 @@ __device__ __forceinline__ void tile_store(const u4 (&v)[NREC], u4* __restrict__
   }
 }
 
-// Workgroup = (batch b, NW consecutive (channel, state block) pairs), one pair per wavefront; the nb
-// wavefronts of a channel are neighbours (nb divides NW) and add their shares of y through LDS.
-// KS: 32-wide steps of the contraction over r (d <= 32 KS).
-template <int KS, int NW>
-__global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p) {
+// ---- the sequence in segments
+//
+// A call of few (batch, channel) pairs leaves most of the chip idle while each pair walks its sequence alone (64 pairs of 2048
+// steps: 163 us forward, 262 backward, on 8 compute units).  Its tiles are cut into nseg segments of sl, walked side by side.
+// What a segment makes of the state that enters it is linear, h -> E h + F: dropin_seg_kernel finds E and F first, for the
+// backward sweep also what it adds to the adjoint, and every wavefront of the scan composes the segments before (behind) its own.
+
+// The states (and with ADJ their adjoints) of a lane's four rows after `cnt` segments, whose maps are `step` apart from `mp` (`ma`)
+// + off[a] on in the order of the walk.  Lane l of a row takes map l, four shifts compose the row's sixteen in order into its
+// last lane.  All lanes of a row return the same.
+template <bool ADJ>
+__device__ __forceinline__ void seg_enter_row(const f4* __restrict__ mp, const float2* __restrict__ ma, const int (&off)[4], ptrdiff_t step, int cnt,
+                                              int l_, float (&hr)[4], float (&hi)[4], float* ar, float* ai) {
+  for (int k0 = 0; k0 < cnt; k0 += 16) {
+    const int k = k0 + l_;
+    f4 m[4];
+    float2 c[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      m[a] = k < cnt ? mp[k * step + off[a]] : f4{1, 0, 0, 0};
+      c[a] = ADJ && k < cnt ? ma[k * step + off[a]] : make_float2(0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      float Er = m[a][0], Ei = m[a][1], Fr = m[a][2], Fi = m[a][3], Ar = c[a].x, Ai = c[a].y;
+      auto fold = [&](float er, float ei, float fr, float fi, float cr, float ci) {   // the earlier map comes first
+        Fr += Er * fr - Ei * fi;
+        Fi += Er * fi + Ei * fr;
+        if (ADJ) {
+          Ar += Er * cr - Ei * ci;
+          Ai += Er * ci + Ei * cr;
+        }
+        const float t = Er * er - Ei * ei;
+        Ei = Er * ei + Ei * er;
+        Er = t;
+      };
+#define SEG_FOLD(C_) fold(dpp_mov0<C_>(Er), dpp_mov0<C_>(Ei), dpp_mov0<C_>(Fr), dpp_mov0<C_>(Fi), ADJ ? dpp_mov0<C_>(Ar) : 0.0f, ADJ ? dpp_mov0<C_>(Ai) : 0.0f)
+      SEG_FOLD(0x111); SEG_FOLD(0x112); SEG_FOLD(0x114); SEG_FOLD(0x118);   // row_shr:1, 2, 4, 8: the last lane's sources are all in its row
+#undef SEG_FOLD
+      Er = row_last(Er, 0); Ei = row_last(Ei, 0);
+      const float h = Er * hr[a] - Ei * hi[a] + row_last(Fr, 0);
+      hi[a] = Er * hi[a] + Ei * hr[a] + row_last(Fi, 0);
+      hr[a] = h;
+      if (ADJ) {
+        const float t = Er * ar[a] - Ei * ai[a] + row_last(Ar, 0);
+        ai[a] = Er * ai[a] + Ei * ar[a] + row_last(Ai, 0);
+        ar[a] = t;
+      }
+    }
+  }
+}
+
+// The maps of the segments: all but the last one's for the forward kernel, all but the first one's for the backward one
+// (blockIdx.x = segment, batch element, channel group).  With Q_l the rotation from the segment's start to step l - tile by
+// tile, from the phases that the scans form, in their order -, S = sum w conj(Q) and T = sum a conj(Q):
+//     E = Q_end,  F = E Bt S;        towards the front M = conj(E),  N = -Bt S,  A = conj(Ct) T.
+// The sums stay with their lanes until the end, so a tile costs its phases, one sincos and eight operations a (state, step):
+// of 256 pairs and 512 steps 7 us in segments of two tiles (forward) and 9 of four (backward), before scans of 9.7 and 28 us.
+template <int KS, int NW, bool BWD>
+__global__ __launch_bounds__(NW * 64) void dropin_seg_kernel(const DropinBwdArgs q) {
   __shared__ u4 s_u[2][KS * 3 * 64];
-  __shared__ float s_y[2][NW][DT];                     // shares of y of the tile, by tile parity (nb > 1)
+  __shared__ f4 s_par[D_MAXN];
+  const DropinArgs& p = q.f;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int nb = p.nb, ncg = (p.d * nb + NW - 1) / NW;
-  const int b = p.b0 + blockIdx.x / ncg, v = (blockIdx.x % ncg) * NW + wave;
+  const int sq = blockIdx.x / (q.bg * ncg), cell = blockIdx.x - sq * q.bg * ncg, sg = sq + (BWD ? 1 : 0);
+  const int zb = cell / ncg, b = q.b0 + zb, v = (cell % ncg) * NW + wave;
   const int i = v / nb, sb = v % nb, j0 = 16 * sb;
   const bool iok = i < p.d;
   const int ic = iok ? i : p.d - 1, vc = ic * nb + sb;
@@ -192,6 +265,120 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
   const int d = p.d, n = p.n, L = p.L;
   const size_t row = ((size_t)b * d + ic) * L, zrow = (size_t)b * p.zs + (size_t)ic * L;
   const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * (KS * 3 * 64);   // + tile * (KS 3 64)
+  const int tb = q.t0 + sg * p.sl, te = min(tb + p.sl, q.t1);
+
+  u4 xa[KS][3];
+#pragma unroll
+  for (int k = 0; k < KS; ++k)
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      xa[k][c] = (k < p.ks) ? p.xp[(((size_t)vc * p.ks + k) * 3 + c) * 64 + lane] : u4{0, 0, 0, 0};
+  float xb[4], Qr[4], Qi[4], Sr[4], Si[4], Tr[4], Ti[4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int j = j0 + 4 * g + a;
+    xb[a] = j < n ? p.x_bias[(size_t)ic * p.xsi + (size_t)j * p.xsj] : 0.0f;
+    Qr[a] = 1.0f;
+    Qi[a] = Sr[a] = Si[a] = Tr[a] = Ti[a] = 0.0f;
+  }
+  constexpr int NT = NW * 64, NREC = (KS * 3 * 64 + NT - 1) / NT;
+  u4 sv[NREC];
+  tile_load<NT, NREC, KS>(upb + (size_t)tb * (KS * 3 * 64), sv, tid);
+  tile_store<NT, NREC, KS>(sv, s_u[tb & 1], tid);
+  polar_params<false>(p, s_par, nullptr, tid);
+  __syncthreads();
+  float un = 0.0f, dtn = 0.0f, zn = 0.0f, gyn = 0.0f;
+  auto inputs = [&](int l) {                           // a tile ahead; steps past the end count as zero
+    const bool ok = l < L;
+    un = ok ? p.u[row + l] : 0.0f;
+    dtn = ok ? p.dt[row + l] : 0.0f;
+    if (BWD) {
+      zn = ok ? p.z[zrow + l] : 0.0f;
+      gyn = ok ? q.gy[row + l] : 0.0f;
+    }
+  };
+  inputs(tb * DT + l_);
+  for (int t = tb; t < te; ++t) {
+    const int l0 = t * DT;
+    const float w = dtn * silu_fast(un), av = BWD ? gyn * silu_fast(zn) : 0.0f;
+    if (t + 1 < te) {
+      inputs(l0 + DT + l_);
+      tile_load<NT, NREC, KS>(upb + (size_t)(t + 1) * (KS * 3 * 64), sv, tid);
+    }
+    f4 th = {0, 0, 0, 0};
+    const u4* su = s_u[t & 1];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      u4 ubk[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) ubk[c] = su[(k * 3 + c) * 64 + lane];
+      th = xmm<3>(xa[k], ubk, th);
+    }
+    const float cnt = (float)(min(l_ + 1, L - l0));
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      float sn, cs;
+      sincos_any(fmaf(xb[a], cnt, th[a]), &sn, &cs);
+      const float qr = Qr[a] * cs - Qi[a] * sn, qi = Qr[a] * sn + Qi[a] * cs;
+      Sr[a] += w * qr;
+      Si[a] -= w * qi;
+      if (BWD) {
+        Tr[a] += av * qr;
+        Ti[a] -= av * qi;
+      }
+      Qr[a] = row_last(qr, lane);
+      Qi[a] = row_last(qi, lane);
+    }
+    if (t + 1 < te) tile_store<NT, NREC, KS>(sv, s_u[(t + 1) & 1], tid);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int j = j0 + 4 * g + a;
+    const float sr = row_last(row_prefix(Sr[a]), lane), si = row_last(row_prefix(Si[a]), lane);
+    float tr = 0.0f, ti = 0.0f;
+    if (BWD) {
+      tr = row_last(row_prefix(Tr[a]), lane);
+      ti = row_last(row_prefix(Ti[a]), lane);
+    }
+    if (iok && l_ == 0 && j < n) {
+      const size_t at = ((size_t)zb * d + i) * n + j, to = (size_t)sg * q.bg * d * n + at;
+      const f4 par = s_par[j];
+      const float Nr = par[0] * sr - par[1] * si, Ni = par[0] * si + par[1] * sr;    // Bt S
+      if (BWD) {
+        p.seg[to] = f4{Qr[a], -Qi[a], -Nr, -Ni};
+        q.sega[to] = make_float2(par[2] * tr + par[3] * ti, par[2] * ti - par[3] * tr);
+        if (sg == 1) {
+          const size_t sidx = ((size_t)b * d + i) * n + j;
+          q.ent[at] = f4{q.hc_re[sidx], q.hc_im[sidx], q.dh_re[sidx], q.dh_im[sidx]};
+        }
+      } else {
+        p.seg[to] = f4{Qr[a], Qi[a], Qr[a] * Nr - Qi[a] * Ni, Qr[a] * Ni + Qi[a] * Nr};
+      }
+    }
+  }
+}
+
+// Workgroup = (batch b, NW consecutive (channel, state block) pairs), one pair per wavefront; the nb
+// wavefronts of a channel are neighbours (nb divides NW) and add their shares of y through LDS.
+// KS: 32-wide steps of the contraction over r (d <= 32 KS).
+template <int KS, int NW>
+__global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p) {
+  __shared__ u4 s_u[2][KS * 3 * 64];
+  __shared__ f4 s_par[D_MAXN];
+  __shared__ float s_y[2][NW][DT];                     // shares of y of the tile, by tile parity (nb > 1)
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
+  const int nb = p.nb, ncg = (p.d * nb + NW - 1) / NW;
+  const int sg = blockIdx.x / (p.b * ncg), cell = blockIdx.x - sg * p.b * ncg;
+  const int b = p.b0 + cell / ncg, v = (cell % ncg) * NW + wave;
+  const int i = v / nb, sb = v % nb, j0 = 16 * sb;
+  const bool iok = i < p.d;
+  const int ic = iok ? i : p.d - 1, vc = ic * nb + sb;
+  const int l_ = lane & 15, g = lane >> 4;
+  const int d = p.d, n = p.n, L = p.L;
+  const size_t row = ((size_t)b * d + ic) * L, zrow = (size_t)b * p.zs + (size_t)ic * L;
+  const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * (KS * 3 * 64);   // + tile * (KS 3 64)
+  const int tb = p.nseg > 1 ? p.t0 + sg * p.sl : p.t0, ntiles = p.nseg > 1 ? min(tb + p.sl, p.t1) : p.t1;
 
   // this wavefront's rows of x, split, for the whole launch
   u4 xa[KS][3];
@@ -202,35 +389,41 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
       xa[k][q] = (k < p.ks) ? p.xp[(((size_t)vc * p.ks + k) * 3 + q) * 64 + lane] : u4{0, 0, 0, 0};
   // per state j = j0 + 4 g + a: bias, Bt, Ct, carried state
   float xb[4], btr[4], bti[4], ctr[4], cti[4], hr[4], hi[4];
+  int at[4];
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
     const int j = j0 + 4 * g + a;
     const bool ok = j < n;
     const int jc = ok ? j : 0;
+    const size_t cell_ = ((size_t)(b - p.b0) * d + ic) * n + jc;
     xb[a] = ok ? p.x_bias[(size_t)ic * p.xsi + (size_t)jc * p.xsj] : 0.0f;
-    float s, c;
-    const float br = op_radius(p, p.B_r, jc), cr = op_radius(p, p.C_r, jc);
-    fast_sincosf(op_phase(p, p.B_th, jc), &s, &c);
-    btr[a] = ok ? br * c : 0.0f;
-    bti[a] = ok ? br * s : 0.0f;
-    fast_sincosf(op_phase(p, p.C_th, jc), &s, &c);
-    ctr[a] = ok ? cr * c : 0.0f;
-    cti[a] = ok ? cr * s : 0.0f;
-    hr[a] = ok && p.h_re ? p.h_re[((size_t)b * d + ic) * n + jc] : 0.0f;
-    hi[a] = ok && p.h_im ? p.h_im[((size_t)b * d + ic) * n + jc] : 0.0f;
+    hr[a] = ok && p.h_re ? p.h_re[(size_t)p.b0 * d * n + cell_] : 0.0f;
+    hi[a] = ok && p.h_im ? p.h_im[(size_t)p.b0 * d * n + cell_] : 0.0f;
+    at[a] = (int)cell_;                                // (of use with segments, where there are few)
+  }
+  if (sg > 0) {                                        // through the segments in front
+    seg_enter_row<false>(p.seg, nullptr, at, (ptrdiff_t)p.b * d * n, sg, l_, hr, hi, nullptr, nullptr);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+      if (j0 + 4 * g + a >= n) hr[a] = hi[a] = 0.0f;
   }
   const float Di = p.Dp[ic];
-  const int ntiles = p.t1;
 
   constexpr int NT = NW * 64, NREC = (KS * 3 * 64 + NT - 1) / NT;
   u4 sv[NREC];
-  tile_load<NT, NREC, KS>(upb + (size_t)p.t0 * (KS * 3 * 64), sv, tid);
-  tile_store<NT, NREC, KS>(sv, s_u[p.t0 & 1], tid);
+  tile_load<NT, NREC, KS>(upb + (size_t)tb * (KS * 3 * 64), sv, tid);
+  tile_store<NT, NREC, KS>(sv, s_u[tb & 1], tid);
+  polar_params<false>(p, s_par, nullptr, tid);
   __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const f4 par = s_par[j0 + 4 * g + a];
+    btr[a] = par[0]; bti[a] = par[1]; ctr[a] = par[2]; cti[a] = par[3];
+  }
   // the wavefront's own inputs, requested one tile ahead
-  const int lf = p.t0 * DT + l_;
+  const int lf = tb * DT + l_;
   float un = lf < L ? p.u[row + lf] : 0.0f, dtn = lf < L ? p.dt[row + lf] : 0.0f, zn = lf < L ? p.z[zrow + lf] : 0.0f;
-  for (int t = p.t0; t < ntiles; ++t) {
+  for (int t = tb; t < ntiles; ++t) {
     const int l0 = t * DT, l = l0 + l_;
     const bool lok = l < L;
     const float uv = un, dtv = dtn, zv = zn;
@@ -282,7 +475,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
       p.y[row + l] = silu_fast(zv) * (tot + Di * ut);
     }
   }
-  if (p.nh_re && iok && l_ == 0) {
+  if (p.nh_re && iok && l_ == 0 && ntiles == p.t1) {
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       const int j = j0 + 4 * g + a;
@@ -350,7 +543,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
   const DropinArgs& p = q.f;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int nb = p.nb, ncg = (p.d * nb + NW - 1) / NW;
-  const int zb = blockIdx.x / ncg, b = q.b0 + zb, v = (blockIdx.x % ncg) * NW + wave;
+  const int sg = blockIdx.x / (q.bg * ncg), cell = blockIdx.x - sg * q.bg * ncg;
+  const int zb = cell / ncg, b = q.b0 + zb, v = (cell % ncg) * NW + wave;
   const int i = v / nb, sb = v % nb, j0 = 16 * sb;
   const bool iok = i < p.d;
   const int ic = iok ? i : p.d - 1, vc = ic * nb + sb;
@@ -367,36 +561,44 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
       xa[k][c] = (k < p.ks) ? p.xp[(((size_t)vc * p.ks + k) * 3 + c) * 64 + lane] : u4{0, 0, 0, 0};
   // per state: (Re Bt, Im Bt, Re Ct, Im Ct), shared by the workgroup, and the bias of this wavefront's channel.
   // They are read from LDS where they are used: in registers they would push the kernel over 256.
-  __shared__ f4 s_par[D_MAXN];
+  __shared__ f4 s_par[D_MAXN], s_unit[D_MAXN];
   __shared__ float s_xb[NW][16];
-  if (tid < D_MAXN) {
-    const bool ok = tid < n;
-    const int jc = ok ? tid : 0;
-    float sb, cb, sc, cc;
-    fast_sincosf(op_phase(p, p.B_th, jc), &sb, &cb);
-    fast_sincosf(op_phase(p, p.C_th, jc), &sc, &cc);
-    const float br = op_radius(p, p.B_r, jc), cr = op_radius(p, p.C_r, jc);
-    s_par[tid] = ok ? f4{br * cb, br * sb, cr * cc, cr * sc} : f4{0, 0, 0, 0};
-  }
+  polar_params<true>(p, s_par, s_unit, tid);
   if (lane < 16) s_xb[wave][lane] = j0 + lane < n ? p.x_bias[(size_t)ic * p.xsi + (size_t)(j0 + lane) * p.xsj] : 0.0f;
-  float hr[4], hi[4], ar[4], ai[4];
+  float hr[4], hi[4], ar[4], ai[4];                    // state at the end of the tile being processed, its adjoint
   float gBr[4], gBi[4], gCr[4], gCi[4], gxb[4];
+  int at[4];
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
     const int j = j0 + 4 * g + a;
-    const bool ok = j < n;
-    const int jc = ok ? j : 0;
-    const size_t sidx = ((size_t)b * d + ic) * n + jc;
-    hr[a] = ok ? q.hc_re[sidx] : 0.0f;             // state at the end of the tile being processed
-    hi[a] = ok ? q.hc_im[sidx] : 0.0f;
-    ar[a] = ok ? q.dh_re[sidx] : 0.0f;             // its adjoint
-    ai[a] = ok ? q.dh_im[sidx] : 0.0f;
+    at[a] = (zb * d + ic) * n + (j < n ? j : 0);
     gBr[a] = gBi[a] = gCr[a] = gCi[a] = gxb[a] = 0.0f;
   }
+  if (p.nseg > 1) {
+    const ptrdiff_t per = (ptrdiff_t)q.bg * d * n;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const f4 en = q.ent[at[a]];
+      hr[a] = en[0]; hi[a] = en[1]; ar[a] = en[2]; ai[a] = en[3];
+    }
+    seg_enter_row<true>(p.seg + (p.nseg - 1) * per, q.sega + (p.nseg - 1) * per, at, -per, p.nseg - 1 - sg, l_, hr, hi, ar, ai);
+  } else {
+    const size_t base = (size_t)q.b0 * d * n;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      hr[a] = q.hc_re[base + at[a]];
+      hi[a] = q.hc_im[base + at[a]];
+      ar[a] = q.dh_re[base + at[a]];
+      ai[a] = q.dh_im[base + at[a]];
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+    if (j0 + 4 * g + a >= n) hr[a] = hi[a] = ar[a] = ai[a] = 0.0f;
   const float Di = p.Dp[ic];
   float gD = 0.0f, gdtb = 0.0f;
-  const int t_first = q.t0, t_last = q.t1 - 1;
-  float* __restrict__ dth = q.dth + ((size_t)zb * d * n + (size_t)ic * p.xsi) * q.lc - (size_t)t_first * DT;   // + state j: j xsj rows
+  const int t_first = q.t0 + sg * p.sl, t_last = (p.nseg > 1 ? min(t_first + p.sl, q.t1) : q.t1) - 1;
+  float* __restrict__ dth = q.dth + ((size_t)zb * d * n + (size_t)ic * p.xsi) * q.lc - (size_t)q.t0 * DT;   // + state j: j xsj rows
 
   constexpr int NT = NW * 64, NREC = (KS * 3 * 64 + NT - 1) / NT;
   u4 sv[NREC];
@@ -506,6 +708,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
   // ---- reductions over the timesteps (lanes of a row) and hand-off.  The gradients of the 4 n shared
   // parameters are first summed over the workgroup's channels in LDS: every workgroup of the launch adds
   // to the same few addresses.
+  // What only this part needs is fetched here: with all arguments at hand from the start the kernel spills scalar registers
+  // (d = 256, four launches over 8 batch elements of 45 tiles: 511 us, 504 now).
+  const __attribute__((address_space(4))) DropinBwdArgs* e = (const __attribute__((address_space(4))) DropinBwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(e));
   __shared__ float s_red[4][D_MAXN];
   if (tid < 4 * D_MAXN) (&s_red[0][0])[tid] = 0.0f;
   __syncthreads();
@@ -525,45 +731,42 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
       const int j = j0 + 4 * g + a;
       if (j < n) {
         const size_t sidx = ((size_t)b * d + i) * n + j;
-        q.dh_re[sidx] = ar[a];
-        q.dh_im[sidx] = ai[a];
-        q.hc_re[sidx] = hr[a];
-        q.hc_im[sidx] = hi[a];
-        atomicAdd(q.dxb + (size_t)i * p.xsi + (size_t)j * p.xsj, gxb[a]);
-        // polar parameters: Bt = B_r e^{i B_theta}
-        float ebr, ebi, ecr, eci;
-        fast_sincosf(op_phase(p, p.B_th, j), &ebi, &ebr);
-        fast_sincosf(op_phase(p, p.C_th, j), &eci, &ecr);
-        const f4 par = s_par[j];
-        atomicAdd(&s_red[0][j], gBr[a] * ebr + gBi[a] * ebi);
+        if (sg == 0) {
+          e->dh_re[sidx] = ar[a];
+          e->dh_im[sidx] = ai[a];
+          e->hc_re[sidx] = hr[a];
+          e->hc_im[sidx] = hi[a];
+        }
+        atomicAdd(e->dxb + (size_t)i * e->f.xsi + (size_t)j * e->f.xsj, gxb[a]);
+        const f4 par = s_par[j], un_ = s_unit[j];      // polar parameters: Bt = B_r e^{i B_theta}
+        atomicAdd(&s_red[0][j], gBr[a] * un_[0] + gBi[a] * un_[1]);
         atomicAdd(&s_red[1][j], gBi[a] * par[0] - gBr[a] * par[1]);
-        atomicAdd(&s_red[2][j], gCr[a] * ecr + gCi[a] * eci);
+        atomicAdd(&s_red[2][j], gCr[a] * un_[2] + gCi[a] * un_[3]);
         atomicAdd(&s_red[3][j], gCi[a] * par[2] - gCr[a] * par[3]);
       }
     }
     if (g == 0 && sb == 0) {
-      atomicAdd(q.dD + i, gD);
-      if (q.ddtb) atomicAdd(q.ddtb + i, q.ddtb_scale * gdtb);
+      atomicAdd(e->dD + i, gD);
+      if (e->ddtb) atomicAdd(e->ddtb + i, e->ddtb_scale * gdtb);
     }
   }
   __syncthreads();
   if (tid < 4 * D_MAXN && (tid & (D_MAXN - 1)) < n) {
     constexpr int SH = 6;                              // log2(D_MAXN)
-    float* dst = (tid >> SH) == 0 ? q.dB_r : (tid >> SH) == 1 ? q.dB_th : (tid >> SH) == 2 ? q.dC_r : q.dC_th;
+    float* dst = (tid >> SH) == 0 ? e->dB_r : (tid >> SH) == 1 ? e->dB_th : (tid >> SH) == 2 ? e->dC_r : e->dC_th;
     const int j = tid & (D_MAXN - 1);
     float v = (&s_red[0][0])[tid];
     // (raw radii: through the softplus)
-    if (p.raw && !((tid >> SH) & 1)) v *= sigmoidf_(((tid >> SH) == 0 ? p.B_r : p.C_r)[(size_t)j * p.bcs]);
-    atomicAdd(dst + (size_t)j * p.bcs, v);
+    if (e->f.raw && !((tid >> SH) & 1)) v *= sigmoidf_(((tid >> SH) == 0 ? e->f.B_r : e->f.C_r)[(size_t)j * e->f.bcs]);
+    atomicAdd(dst + (size_t)j * e->f.bcs, v);
   }
 }
 
-// Several buffers set in one launch (blockIdx.y picks the buffer), 16 bytes a lane where both sides allow it.
-__global__ __launch_bounds__(256) void fill_kernel(const FillArgs a) {
-  const int i = blockIdx.y;
+// A buffer set, FILL_BLOCK floats by one workgroup of 256, 16 bytes a lane where both sides allow it.
+__device__ __forceinline__ void fill_block(const FillArgs& a, int i, size_t block) {
   float* __restrict__ dst = a.dst[i];
   const float* __restrict__ src = a.src[i];
-  const size_t at = (size_t)blockIdx.x * FILL_BLOCK, end = min((size_t)a.n[i], at + FILL_BLOCK);
+  const size_t at = block * FILL_BLOCK, end = min((size_t)a.n[i], at + FILL_BLOCK);
   const bool vec = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0;
   for (size_t j = at + 4 * threadIdx.x; j < end; j += 1024) {
     if (vec && j + 4 <= end) {
@@ -571,6 +774,23 @@ __global__ __launch_bounds__(256) void fill_kernel(const FillArgs a) {
     } else {
       for (size_t k = j; k < end && k < j + 4; ++k) dst[k] = src ? src[k] : 0.0f;
     }
+  }
+}
+// Several buffers in one launch (blockIdx.y picks the buffer)
+__global__ __launch_bounds__(256) void fill_kernel(const FillArgs a) { fill_block(a, blockIdx.y, blockIdx.x); }
+
+// What a call prepares, in one launch: the records of x, the tiles of u, the buffers that start from zero or from a copy.  Each
+// alone takes 4 us, nearly all of it the launch; a call of 64 pairs and 256 steps spent 20 of 85 us (both directions) on five of them.
+__global__ __launch_bounds__(256) void dropin_prep_kernel(const DropinPrepArgs a, const FillArgs f) {
+  unsigned blk = blockIdx.x;
+  if (blk < a.xblocks) { xprep_block(a, blk); return; }
+  blk -= a.xblocks;
+  if (blk < a.ublocks) { uprep_block(a, blk); return; }
+  blk -= a.ublocks;
+  for (int i = 0; i < f.count; ++i) {
+    const unsigned own = (unsigned)((f.n[i] + FILL_BLOCK - 1) / FILL_BLOCK);
+    if (blk < own) { fill_block(f, i, blk); return; }
+    blk -= own;
   }
 }
 

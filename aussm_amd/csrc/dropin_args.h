@@ -33,6 +33,8 @@ struct DropinArgs {
   int xsi, xsj;          // row of (channel i, state j) in x, x_bias and the phase adjoints: i xsi + j xsj (n, 1 or 1, d)
   int bcs, raw;          // stride of the four polar parameters; raw: the radii are given before their softplus
   long zs;               // elements between the batch elements of z (d L for a tensor of its own)
+  int nseg, sl;          // segments of sl tiles that the launch works on side by side (nseg 0 or 1: none, one sweep)
+  f4* seg;               // [nseg][b][d][n] what a segment makes of the state: (E, F), h -> E h + F; backward (M, N), h -> M h + N towards the front
 };
 
 struct DropinBwdArgs {
@@ -58,6 +60,23 @@ struct DropinBwdArgs {
   int dt_act;              // dt = softplus(pre): ddt is the gradient of pre, and ddtb [d] (or null) sums it (atomics)
   float* ddtb;
   float ddtb_scale;
+  float2* sega;            // [nseg][bg][d][n] with nseg > 1: A of the adjoint, which becomes M hat h + A
+  f4* ent;                 // [bg][d][n] ... and the state and the adjoint after tile t1 - 1 (hc_*, dh_* are written by the first segment)
+};
+
+// The pre-pass of a call: records of x (xblocks workgroups, 0: none) and the tiles t0 .. t0 + nt - 1 of u (ublocks)
+struct DropinPrepArgs {
+  const float* x;          // rows of d, (channel i, state j) at row i xsi + j xsj
+  const float* x_bias;
+  const float* u;          // [b, d, L]
+  u4* xp;
+  u4* up;
+  float* x_out;            // scale x, and x_bias, in the operator's own order, or null
+  float* xb_out;
+  int d, n, L, ks, KS, nb, xsi, xsj;   // ks = ceil(d / 32), KS: compiled steps of the contraction
+  int b0, t0, nt;
+  float scale;
+  unsigned xblocks, ublocks;
 };
 
 // Up to FILL_MAX buffers set in one launch: dst[i] = src ? src[i] : 0 for i < n.

@@ -4,14 +4,6 @@
 
 namespace aussm {
 
-int run_dropin_xprep(const float* x, u4* xp, int d, int n, int ks, int nb, int xsi, int xsj, float scale, const float* x_bias, float* x_out,
-                     float* xb_out, hipStream_t s) {
-  const size_t total = (size_t)d * nb * ks * 64;
-  hipLaunchKernelGGL(dropin_xprep_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, x, xp, d, n, ks, nb, xsi, xsj,
-                     scale, x_bias, x_out, xb_out);
-  return launch_status();
-}
-
 int run_fill(const FillArgs& a, hipStream_t s) {
   size_t most = 0;
   for (int i = 0; i < a.count; ++i) most = a.n[i] > most ? a.n[i] : most;
@@ -31,14 +23,21 @@ constexpr int DROPIN_NW = DROPIN_NW_;     // channels (wavefronts) per workgroup
 template <int KS>
 static void launch_fwd(const DropinArgs& a, hipStream_t s) {
   constexpr int NW = KS > 8 ? 4 : DROPIN_NW;
-  const unsigned grid = (unsigned)(a.b * ((a.d * a.nb + NW - 1) / NW));
+  const unsigned grid = (unsigned)((a.nseg > 1 ? a.nseg : 1) * a.b * ((a.d * a.nb + NW - 1) / NW));
   hipLaunchKernelGGL((dropin_fwd_kernel<KS, NW>), dim3(grid), dim3(NW * 64), 0, s, a);
 }
 template <int KS>
 static void launch_bwd(const DropinBwdArgs& a, hipStream_t s) {
   constexpr int NW = KS > 8 ? 4 : DROPIN_NW;
-  const unsigned grid = (unsigned)(a.bg * ((a.f.d * a.f.nb + NW - 1) / NW));
+  const unsigned grid = (unsigned)((a.f.nseg > 1 ? a.f.nseg : 1) * a.bg * ((a.f.d * a.f.nb + NW - 1) / NW));
   hipLaunchKernelGGL((dropin_bwd_kernel<KS, NW>), dim3(grid), dim3(NW * 64), 0, s, a);
+}
+template <int KS>
+static void launch_seg(const DropinBwdArgs& a, hipStream_t s) {
+  constexpr int NW = KS > 8 ? 4 : DROPIN_NW;
+  const unsigned grid = (unsigned)((a.f.nseg - 1) * a.bg * ((a.f.d * a.f.nb + NW - 1) / NW));
+  if (a.sega) hipLaunchKernelGGL((dropin_seg_kernel<KS, NW, true>), dim3(grid), dim3(NW * 64), 0, s, a);
+  else hipLaunchKernelGGL((dropin_seg_kernel<KS, NW, false>), dim3(grid), dim3(NW * 64), 0, s, a);
 }
 
 int dropin_channels_per_workgroup(int ks) { return ks > 8 ? 4 : DROPIN_NW; }
@@ -46,8 +45,13 @@ int dropin_channels_per_workgroup(int ks) { return ks > 8 ? 4 : DROPIN_NW; }
 // the compiled size of the contraction (steps of 32) that serves ceil(d / 32) = ks
 int dropin_compiled_ks(int ks) { return ks <= 4 ? (ks < 1 ? 1 : ks) : ks <= 6 ? 6 : ks <= 8 ? 8 : ks <= 12 ? 12 : 16; }
 
-int run_dropin_uprep(const float* u, u4* up, int d, int L, int ks, int b0, int bg, int t0, int nt, hipStream_t s) {
-  hipLaunchKernelGGL(dropin_uprep_kernel, dim3((unsigned)(bg * nt)), dim3(256), 0, s, u, up, d, L, dropin_compiled_ks(ks), b0, t0, nt);
+int run_dropin_prep(DropinPrepArgs a, int bg, bool rows, const FillArgs& f, hipStream_t s) {
+  const size_t xb = rows ? ((size_t)a.d * a.nb * a.ks * 64 + 255) / 256 : 0, ub = (size_t)bg * a.nt;
+  size_t total = xb + ub;
+  for (int i = 0; i < f.count; ++i) total += (f.n[i] + FILL_BLOCK - 1) / FILL_BLOCK;
+  if (total > 0x7fffffffULL) return -2;
+  a.KS = dropin_compiled_ks(a.ks); a.xblocks = (unsigned)xb; a.ublocks = (unsigned)ub;
+  hipLaunchKernelGGL(dropin_prep_kernel, dim3((unsigned)total), dim3(256), 0, s, a, f);
   return launch_status();
 }
 
@@ -64,6 +68,11 @@ int run_dropin_uprep(const float* u, u4* up, int d, int L, int ks, int b0, int b
 
 int run_dropin_fwd(const DropinArgs& a, hipStream_t s) {
   DROPIN_KS_DISPATCH(launch_fwd, a.ks)
+  return launch_status();
+}
+
+int run_dropin_seg(const DropinBwdArgs& a, hipStream_t s) {
+  DROPIN_KS_DISPATCH(launch_seg, a.f.ks)
   return launch_status();
 }
 

@@ -47,12 +47,11 @@ int run_px_fwd(const FwdArgs& a, const u4* img, const ImgNote& note, int in_dtyp
 int run_px_bwd(const UniBwdArgs& a, const u4* img, int in_dtype, hipStream_t s);
 
 // ---- k_dropin.hip: the reference's 12-input operator as fused kernels
-int run_dropin_xprep(const float* x, u4* xp, int d, int n, int ks, int nb, int xsi, int xsj, float scale, const float* x_bias, float* x_out,
-                     float* xb_out, hipStream_t s);
 int dropin_channels_per_workgroup(int ks);
 int dropin_compiled_ks(int ks);
-int run_dropin_uprep(const float* u, u4* up, int d, int L, int ks, int b0, int bg, int t0, int nt, hipStream_t s);
+int run_dropin_prep(DropinPrepArgs a, int bg, bool rows, const FillArgs& f, hipStream_t s);   // rows: the records of x too
 int run_dropin_fwd(const DropinArgs& a, hipStream_t s);
+int run_dropin_seg(const DropinBwdArgs& a, hipStream_t s);   // maps of the segments (nseg > 1): backward with sega, else forward
 int run_dropin_bwd(const DropinBwdArgs& a, hipStream_t s);
 int run_fill(const FillArgs& a, hipStream_t s);   // several buffers set (zero or a copy) in one launch
 

@@ -872,14 +872,37 @@ static int dropin_fwd_chunk_tiles(int b, int d, int L, bool largest = false) {
   return (int)(((size_t)ntiles + nc - 1) / nc);
 }
 
+// Tiles of a segment of a launch over nt tiles of `bg` batch elements (nt: one sweep).  As many segments as one workgroup per
+// compute unit takes, two in the forward call up to d = 128, where registers leave room for them (16 x 64 pairs of 512 steps: 47 us
+// in one sweep, 23 and 6 for the maps in four segments; 3 x 200: 30 in three segments, 39 in six), but at least two tiles each.
+// The maps cost a third to a half of a sweep: two segments gain nothing (16 x 64 pairs, backward: 80 us, 60 and 22 in two), three
+// do (3 x 200, 500 steps: 87, 46 and 25), and under 16 tiles their launch eats the rest (2 x 32 pairs, 7 tiles: 39 us both ways, 47
+// in segments; 8 x 8, 16 tiles: 62, 49).
+static int dropin_segment_tiles(int bg, int d, int n, int nt, bool backward) {
+  const int nw = dropin_channels_per_workgroup((d + 31) / 32);
+  const long wgs = (long)bg * ((d * dropin_state_blocks(n) + nw - 1) / nw);
+  long most = (backward || d > 128 ? 256 : 512) / wgs;
+  if (most > nt / 2) most = nt / 2;
+  if (most < 3 || nt < 16) return nt;
+  return (int)((nt + most - 1) / most);
+}
+// floats per state of a launch's maps, (E, F) each, backward also A, and the state and adjoint at the end
+static size_t dropin_segment_floats(int bg, int d, int n, int nt, bool backward) {
+  const int sl = dropin_segment_tiles(bg, d, n, nt, backward), nseg = (nt + sl - 1) / sl;
+  return nseg < 2 ? 0 : (size_t)bg * d * n * (backward ? 6 * (size_t)nseg + 4 : 4 * (size_t)nseg);
+}
+
 size_t aussm_ssm_adaptive_unitary_workspace_floats(int b, int d, int n, int L, int backward) {
   if (dropin_check(b, d, n, L) != AUSSM_OK) return 0;
   size_t f = dropin_xp_floats(d, n);
   if (backward) {
     const DropinBlocks k = dropin_blocks(b, d, n, L, true);
     f += 2 * round4((size_t)b * d * n) + (size_t)k.bg * k.ct * DT * d * n + (size_t)k.bg * k.ct * dropin_tile_floats(d);
+    f += dropin_segment_floats(k.bg, d, n, k.ct, true);
   } else {
-    f += (size_t)b * dropin_fwd_chunk_tiles(b, d, L, true) * dropin_tile_floats(d);
+    const int ct = dropin_fwd_chunk_tiles(b, d, L, true);
+    f += (size_t)b * ct * dropin_tile_floats(d);
+    if (ct == (L + DT - 1) / DT) f += dropin_segment_floats(b, d, n, ct, false);
   }
   return f;
 }
@@ -911,6 +934,13 @@ static DropinArgs dropin_args(const aussm_operator_args& p) {
   return a;
 }
 
+static DropinPrepArgs dropin_prep_args(const aussm_operator_args& p, const DropinArgs& f, u4* xp, u4* up) {
+  DropinPrepArgs a{};
+  a.x = p.x; a.x_bias = p.x_bias; a.u = p.u; a.xp = xp; a.up = up; a.d = p.d; a.n = p.n; a.L = p.L; a.ks = f.ks; a.nb = f.nb;
+  a.xsi = f.xsi; a.xsj = f.xsj; a.scale = p.x_scale;
+  return a;
+}
+
 int aussm_operator_fwd(const aussm_operator_args* op, float* y, float* nh_re, float* nh_im, float* workspace, void* stream) {
   return aussm_operator_fwd_keep(op, y, nh_re, nh_im, workspace, nullptr, nullptr, stream);
 }
@@ -925,15 +955,32 @@ int aussm_operator_fwd_keep(const aussm_operator_args* op, float* y, float* nh_r
   DropinArgs a = dropin_args(*op);
   u4* xp = (u4*)workspace;
   u4* up = (u4*)(workspace + dropin_xp_floats(d, n));
-  if (int e = run_dropin_xprep(op->x, xp, d, n, a.ks, a.nb, a.xsi, a.xsj, op->x_scale, op->x_bias, x_out, x_bias_out, s)) return e;
+  DropinPrepArgs pa = dropin_prep_args(*op, a, xp, up);
+  pa.x_out = x_out; pa.xb_out = x_bias_out;
   a.y = y; a.nh_re = nh_re; a.nh_im = nh_im; a.xp = xp; a.up = up; a.b = b;
+  const size_t nstate = (size_t)b * d * n;
+  auto apart = [nstate](const float* p, const float* q) { return !p || p + nstate <= q || q + nstate <= p; };
+  if (ct == ntiles && apart(op->h_re, nh_re) && apart(op->h_re, nh_im) && apart(op->h_im, nh_re) && apart(op->h_im, nh_im)) {
+    // (the first segment still reads the state when the last one writes)
+    const int sl = dropin_segment_tiles(b, d, n, ntiles, false);
+    if (sl < ntiles) {
+      a.nseg = (ntiles + sl - 1) / sl; a.sl = sl;
+      a.seg = (f4*)((float*)up + (size_t)b * ct * dropin_tile_floats(d));
+    }
+  }
   // the sequence in chunks of ct tiles (one chunk unless it is long): prepared tiles of u for the chunk, then the
   // scan over it, the state handed from chunk to chunk in the output buffers
   for (int t0 = 0; t0 < ntiles; t0 += ct) {
     const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
-    if (int e = run_dropin_uprep(op->u, up, d, L, a.ks, 0, b, t0, t1 - t0, s)) return e;
+    pa.t0 = t0; pa.nt = t1 - t0;
+    if (int e = run_dropin_prep(pa, b, t0 == 0, FillArgs{}, s)) return e;
     if (t0) { a.h_re = nh_re; a.h_im = nh_im; }
     a.up_t0 = t0; a.up_nt = t1 - t0; a.t0 = t0; a.t1 = t1;
+    if (a.nseg > 1) {
+      DropinBwdArgs q{};
+      q.f = a; q.bg = b; q.t0 = t0; q.t1 = t1;
+      if (int e = run_dropin_seg(q, s)) return e;
+    }
     if (int e = run_dropin_fwd(a, s)) return e;
   }
   return AUSSM_OK;
@@ -967,9 +1014,10 @@ int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const
   float* hc_im = hc_re + round4(nstate);
   float* dth = hc_im + round4(nstate);
   u4* up = (u4*)(dth + (size_t)blk.bg * ct * DT * d * n);
+  f4* seg = (f4*)((float*)up + (size_t)blk.bg * ct * dropin_tile_floats(d));
   DropinArgs f = dropin_args(*op);
   f.xp = xp; f.up = up;
-  if (int e = run_dropin_xprep(op->x, xp, d, n, f.ks, f.nb, f.xsi, f.xsj, op->x_scale, nullptr, nullptr, nullptr, s)) return e;
+  DropinPrepArgs pa = dropin_prep_args(*op, f, xp, up);
   FillArgs fa{};
   auto fill = [&](float* dst, const float* src, size_t cnt) {
     fa.dst[fa.count] = dst; fa.src[fa.count] = src; fa.n[fa.count] = cnt; ++fa.count;
@@ -995,8 +1043,16 @@ int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const
   }
   fill(g->D, nullptr, d);
   if (g->dt_bias) fill(g->dt_bias, nullptr, d);
-  if (int e = run_fill(fa, s)) return e;
+  bool first = true;                                  // the call's first preparation sets the buffers and lays out x, too
+  auto prepare = [&](int b0, int bg, int t0, int nt) {
+    pa.b0 = b0; pa.t0 = t0; pa.nt = nt;
+    const int e = run_dropin_prep(pa, bg, first, first ? fa : FillArgs{}, s);
+    first = false;
+    return e;
+  };
   const long dn = (long)d * n;
+  const DropinBlocks blk_most = dropin_blocks(b, d, n, L, true);
+  const size_t segf = dropin_segment_floats(blk_most.bg, d, n, blk_most.ct, true);      // what the workspace has for segments
   for (int b0 = 0; b0 < b; b0 += blk.bg) {
     const int bg = b - b0 < blk.bg ? b - b0 : blk.bg;
     f.b = bg; f.b0 = b0; f.up_b0 = b0;
@@ -1004,7 +1060,7 @@ int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const
       // the state at the end of the sequence: a forward sweep without outputs over this group's chunks
       for (int t0 = 0; t0 < ntiles; t0 += ct) {
         const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
-        if (int e = run_dropin_uprep(op->u, up, d, L, f.ks, b0, bg, t0, t1 - t0, s)) return e;
+        if (int e = prepare(b0, bg, t0, t1 - t0)) return e;
         DropinArgs a = f;
         a.y = nullptr; a.nh_re = hc_re; a.nh_im = hc_im;
         if (t0) { a.h_re = hc_re; a.h_im = hc_im; }
@@ -1016,7 +1072,7 @@ int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const
     for (int t0 = ((ntiles - 1) / ct) * ct; t0 >= 0; t0 -= ct) {
       const int t1 = t0 + ct < ntiles ? t0 + ct : ntiles;
       const int l0 = t0 * DT, len = (t1 * DT < L ? t1 * DT : L) - l0;
-      if (int e = run_dropin_uprep(op->u, up, d, L, f.ks, b0, bg, t0, t1 - t0, s)) return e;
+      if (int e = prepare(b0, bg, t0, t1 - t0)) return e;
       DropinBwdArgs q{};
       q.f = f;
       q.f.up_t0 = t0; q.f.up_nt = t1 - t0;
@@ -1025,6 +1081,13 @@ int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const
       q.dB_r = g->B_r; q.dB_th = g->B_theta; q.dC_r = g->C_r; q.dC_th = g->C_theta; q.dD = g->D;
       q.dh_re = g->h_re; q.dh_im = g->h_im; q.b0 = b0; q.bg = bg; q.t0 = t0; q.t1 = t1; q.lc = lc;
       q.dt_act = op->dt_softplus; q.ddtb = g->dt_bias; q.ddtb_scale = op->dt_bias_scale;
+      const int nt = t1 - t0, sl = dropin_segment_tiles(bg, d, n, nt, true), nseg = (nt + sl - 1) / sl;
+      if (nseg > 1 && dropin_segment_floats(bg, d, n, nt, true) <= segf) {
+        const size_t per = (size_t)bg * d * n;
+        q.f.nseg = nseg; q.f.sl = sl; q.f.seg = seg;
+        q.ent = seg + nseg * per; q.sega = (float2*)(q.ent + per);
+        if (int e = run_dropin_seg(q, s)) return e;
+      }
       if (int e = run_dropin_bwd(q, s)) return e;
       // grad_u[b, r, l0 + l] += scale sum_(i j) x[(i j), r] hat theta[b, (i j), l]   (rows (i j) in the order of x)
       XGemmArgs gu{};

@@ -24,6 +24,7 @@ constexpr int AUX_PAD = 64;
 constexpr int AUX_IMG_FP = 8;
 
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef float f4 __attribute__((ext_vector_type(4)));
 
 // What the per-(b,d,l) part of an auxiliary buffer was computed from: the tensors (addresses), the shape
 // and the input type.  Never zero (zero is what an invalidated buffer holds).

@@ -350,7 +350,6 @@ __device__ __forceinline__ void store4(float* __restrict__ p, size_t o, const fl
   }
 }
 
-typedef float f4 __attribute__((ext_vector_type(4)));
 // 16-byte loads and stores that are only known to be 4-byte aligned (rows start anywhere when the row length is not a
 // multiple of four): the memory pipeline takes them, the type tells the compiler so
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));

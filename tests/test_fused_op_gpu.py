@@ -100,6 +100,32 @@ def test_small_blocks_walk_the_problem_in_many_launches(kfloats):
         _close(g2, w, "gradient (from state) wrt " + name)
 
 
+# Few pairs, 16 tiles and more: the sequence in segments.  A last tile of one step; a last segment that is shorter; more
+# segments than a row has lanes (75 tiles: 37); 48 states (four blocks); eight wavefronts with wide x; four (d > 256); chunks
+# of 25 tiles with segments of their own (kfloats 160: 1200 steps of 24 x 16 states in three)
+@pytest.mark.parametrize("b,d,n,l,kfloats", [(1, 16, 16, 241, 0), (3, 40, 5, 700, 0), (1, 12, 16, 1200, 0), (1, 24, 48, 530, 0), (2, 200, 8, 333, 0),
+                                             (1, 300, 16, 300, 0), (1, 24, 16, 1200, 160)])
+def test_segments_of_the_sequence(b, d, n, l, kfloats):
+    from aussm_amd import ops, _lib  # noqa: F401
+    print(f"case fused segments b={b} d={d} n={n} l={l}", flush=True)
+    args = _inputs(b, d, n, l, seed=21, xscale=d ** -0.5)
+    g = torch.Generator().manual_seed(22)
+    grads = [torch.randn(*s, generator=g, dtype=torch.float64) for s in ((b, d, l), (b, d, n), (b, d, n))]
+    leaves = [a.cuda().requires_grad_(True) for a in args]
+    outs = O.adaptive_unitary_op_loop(*leaves)
+    want = torch.autograd.grad(outs, leaves, [t.cuda() for t in grads])
+    dev, gdev = [a.float().cuda() for a in args], [t.float().cuda() for t in grads]
+    with _lib.options(block_kfloats=kfloats):
+        got = torch.ops.extension_cpp.ssm_adaptive_unitary(*dev)
+        got_b = torch.ops.extension_cpp.ssm_adaptive_backward_unitary(*gdev, *dev)
+        got_s = torch.ops.aussm_amd.ssm_adaptive_backward_unitary_from_state(*gdev, *dev, got[1], got[2])
+    for w, g_, name in zip(outs, got, ("y", "next_hid_real", "next_hid_imag")):
+        _close(g_, w.detach().cpu(), name)
+    for w, g1, g2, name in zip(want, got_b, got_s, IN_NAMES):
+        _close(g1, w.cpu(), "gradient wrt " + name)
+        _close(g2, w.cpu(), "gradient (from state) wrt " + name)
+
+
 def test_backward_from_saved_state_equals_backward_from_inputs():
     """The autograd formula hands the forward call's end state to the backward kernels; the reference-shaped
     backward operator recomputes it.  Same gradients either way."""
