@@ -39,8 +39,9 @@ static int launch_xgemm(const Tile& t, const XGemmArgs& a, unsigned grid, hipStr
 // them.  us, 128-wide tile / the one taken: 256 x 5760, K = 1024 74 / 45; 1000 x 1000, K = 250 31 / 16; 137 x 1008, K = 548
 // 51 / 20; 384 x 954, K = 96 23 / 7.4; 54 x 1320, K = 27 11 / 5.1; 48 x 23040, K = 512 30 / 24; 16 x 131072, K = 32 9.3 with 32 x 64, 8.0
 // with 32 x 128; 512 x 8192, K = 256 (1024 tiles of 64 x 64) 23.9 / 23.2, 1024 x 8192 (2048) 27.4 with the wide tile against 34.8.  Sums over z alike, by the work there is:
-// 64 x 64 up to 18000 tile steps (256 x 512, 736 steps, 23500 of them: 53 against 62; 1024 x 256, 256 steps, 16400: 49 against
-// 45; 512 x 128, 512 steps 56 / 27; 96 x 192, 30 steps 20 / 6.8), for 32 columns or rows up to 4500 (512 x 16, 736 steps, 5900:
+// 64 x 64 up to 18000 tile steps, past 8000 in twice the slices (512 x 128, 512 steps 56 / 27; 96 x 192, 30 steps 20 / 6.8;
+// 142 x 3960, 71 steps, 13206 of them: 42 / 39, 53 in half the slices; 200 x 3000, 100 steps, 18800: 51 / 50), where rows of K that do
+// not start on 16 bytes cost the small tile's loads more to 6000 (2272 x 142, 50 steps of 791, 5400: 41 / 38; 75 steps, 8100: 48 / 54), for 32 columns or rows up to 4500 (512 x 16, 736 steps, 5900:
 // 13.7 against 15.0; 256 x 16 11.8 / 10.0).  Past that few rows take 32 x 128 (32 x 32768, sums of 2048: 62, 128 x 128 111), or 64 x 64
 // and twice the slices (64 x 23040, 1024: 34.7, with 64 x 128 42.6; 64 x 32768, 4096: 156, 151).
 //
@@ -67,7 +68,10 @@ int run_xgemm(XGemmArgs a, hipStream_t s) {
   if (sliced) {
     if (a.M <= 32 && a.N <= 32) tile = T32;
     else if ((a.M <= 32 || a.N <= 32) && tiles_of(half) * steps <= 4500) tile = half;
-    else if (a.M > 32 && a.N > 32 && tiles_of(T64) * steps <= 18000) tile = T64;
+    else if (a.M > 32 && a.N > 32 && tiles_of(T64) * steps <= (a.K % 4 ? 6000 : 18000)) {
+      tile = T64;
+      if (tiles_of(T64) * steps > 8000) slots = 1024;
+    }
     else if (a.M <= 32 && a.N > 64) tile = ROWS32;
     else if (a.M <= 64 && a.N > 64) tile = T64, slots = 1024;
     else small = false;
