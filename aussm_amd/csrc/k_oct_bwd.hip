@@ -41,24 +41,29 @@ int run_oct_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s) {
   return in_dtype ? oct_bwd_t<VAR_REAL, bf16_t>(a, s) : oct_bwd_t<VAR_REAL, float>(a, s);
 }
 
-// The unitary scan's, up to 32 states in one launch.
+// The unitary scan's, blocks of 32 states.
 template <typename Tin>
-static int oct_ubwd_t(const RecBwdArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)(a.B * a.ncg)), block(512);
-  auto go = [&](auto sc, auto full) {
-    constexpr int S = decltype(sc)::value;
-    constexpr bool F = decltype(full)::value;
-    hipLaunchKernelGGL((oct_bwd_kernel<VAR_UNITARY, S, F, Tin, Tin, false>), grid, block, 0, s, a);
-  };
-  using std::integral_constant;
-  const int S = (a.N + 7) / 8;
-  if (S == 1) go(integral_constant<int, 1>{}, std::false_type{});
-  else if (S == 2 && a.N == 16) go(integral_constant<int, 2>{}, std::true_type{});
-  else if (S == 2) go(integral_constant<int, 2>{}, std::false_type{});
-  else if (S == 3) go(integral_constant<int, 3>{}, std::false_type{});
-  else if (S == 4) go(integral_constant<int, 4>{}, std::false_type{});
-  else return -2;
-  return launch_status();
+static int oct_ubwd_t(const RecBwdArgs& args, hipStream_t s) {
+  const dim3 grid((unsigned)(args.B * args.ncg)), block(512);
+  for (int nbase = 0; nbase < args.N; nbase += 32) {
+    RecBwdArgs a = args;
+    a.nbase = nbase;
+    a.accum = nbase > 0;
+    auto go = [&](auto sc, auto full) {
+      constexpr int S = decltype(sc)::value;
+      constexpr bool F = decltype(full)::value;
+      hipLaunchKernelGGL((oct_bwd_kernel<VAR_UNITARY, S, F, Tin, Tin, false>), grid, block, 0, s, a);
+    };
+    using std::integral_constant;
+    const int left = a.N - nbase, S = (left + 7) / 8;
+    if (S == 1) go(integral_constant<int, 1>{}, std::false_type{});
+    else if (S == 2 && left == 16) go(integral_constant<int, 2>{}, std::true_type{});
+    else if (S == 2) go(integral_constant<int, 2>{}, std::false_type{});
+    else if (S == 3) go(integral_constant<int, 3>{}, std::false_type{});
+    else go(integral_constant<int, 4>{}, std::false_type{});
+    if (int e = launch_status()) return e;
+  }
+  return 0;
 }
 
 int run_oct_ubwd(const UniBwdArgs& u, int in_dtype, hipStream_t s) {

@@ -4,7 +4,7 @@
 
 namespace aussm {
 
-// groups of eight states: S = 1 .. 4 (N <= 32) or 8
+// groups of eight states: S = 1 .. 4 (N <= 32), 6 or 8
 template <int VAR, typename Tin>
 static int oct_fwd_t(const FwdArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)(a.B * a.ncg)), block(512);
@@ -28,6 +28,7 @@ static int oct_fwd_t(const FwdArgs& a, hipStream_t s) {
   else if (S == 2) go(std::integral_constant<int, 2>{});
   else if (S == 3) go(std::integral_constant<int, 3>{});
   else if (S == 4) go(std::integral_constant<int, 4>{});
+  else if (S <= 6) go(std::integral_constant<int, 6>{});
   else if (S <= 8) go(std::integral_constant<int, 8>{});
   else return -2;
   return launch_status();
@@ -50,6 +51,7 @@ static int oct_adj_t(const AdjSegArgs& a, unsigned grid, hipStream_t s) {
   else if (S == 2) go(std::integral_constant<int, 2>{});
   else if (S == 3) go(std::integral_constant<int, 3>{});
   else if (S == 4) go(std::integral_constant<int, 4>{});
+  else if (S <= 6) go(std::integral_constant<int, 6>{});
   else if (S <= 8) go(std::integral_constant<int, 8>{});
   else return -2;
   return launch_status();

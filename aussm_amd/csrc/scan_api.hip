@@ -605,7 +605,8 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
     if (int e = run_oct_adj(VAR_UNITARY, g, in_dtype, (unsigned)(B * sp.ns * a.ncg), s)) return e;
     a.B = B * sp.ns; a.L = sp.ls; a.ns = sp.ns; a.seg = seg; a.segq = ptot;
   }
-  if (N <= 32) return run_oct_ubwd(a, in_dtype, s);
+  // (Blocks of 32 states add to what the first wrote, which bf16 would round.  8 x 72 x 37, 2957 steps: 237 us against 642.)
+  if (N <= 32 || !a.g16) return run_oct_ubwd(a, in_dtype, s);
   return run_unitary_bwd_generic(a, in_dtype, pick_cfg(a.N, 8), s);
 }
 

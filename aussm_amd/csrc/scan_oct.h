@@ -227,6 +227,10 @@ struct OctRows {
   }
 };
 
+// The states are worked out here.  (Without the sums' stores nothing kept a pass without outputs from reading a whole tile's
+// rows ahead: 220 spilled registers at 64 states.)
+__device__ __forceinline__ void pin(float& a, float& b) { asm volatile("" : "+v"(a), "+v"(b) : : "memory"); }
+
 // S: state groups of eight (8 S >= N).  FULLN: N = 8 S.  LEAN: no outputs but the end state and the product of the a_l (the
 // first pass of a call that is split along the sequence).
 template <int VAR, int S, bool FULLN, typename Tin, typename Tbc, bool LEAN>
@@ -439,6 +443,10 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
       };
       auto sums = [&](int q) {                               // (over what the group has read)
         if constexpr (!LEAN) in[q * G + (G == 8 ? g : g >> 1)] = state_sums(ya, bit2, bit1, bit0);
+        else {
+#pragma unroll
+          for (int s = 0; s < S; ++s) pin(hr[s], hi[s]);
+        }
       };
       constexpr int NQ = OT / G;
       const bool next = l0 + OT < L;

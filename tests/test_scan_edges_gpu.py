@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from oracle import scan_oracle as O
+from test_unitary_gpu import test_gradients_match_oracle as unitary_gradients
 from test_variants_gpu import test_complex_gradients as complex_gradients, test_real_gradients as real_gradients
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +43,35 @@ def test_an_infinity_stays_in_its_channel(N, D):
     others = torch.ones(B, D, dtype=torch.bool)
     others[1, 2] = False
     assert torch.equal(y[others.cuda()], y0[others.cuda()]) and torch.equal(h[others.cuda()], h0[others.cuda()])
+
+
+# More than 32 states: the reverse scan in two launches that add up, 48 and 64 states' worth of registers forward; split
+# along the sequence (260 steps) and not
+@pytest.mark.parametrize("B,D,N,L", [(2, 9, 33, 260), (1, 72, 48, 300), (1, 8, 49, 41), (1, 70, 64, 257)])
+def test_unitary_of_more_than_32_states(B, D, N, L):
+    unitary_gradients(B, D, N, L, False)
+    unitary_gradients(B, D, N, L, True)
+
+
+@pytest.mark.parametrize("N", [32, 40])
+def test_unitary_gradients_in_bf16_are_the_rounded_sums(N):
+    """bf16 inputs with du and ddelta in bf16 (the flag of the entry point): what the same call in float leaves, rounded once.
+    The two may take other kernels, whose sums differ by a few 2^-22 of the largest: one bf16 step where that crosses a tie."""
+    from aussm_amd import _lib, scan
+    B, D, L, ck = 2, 72, 100, 32
+    p = O.make_core_inputs(B, D, N, L, seed=N)
+    lo = lambda t: (torch.view_as_real(t).contiguous() if t.is_complex() else t).bfloat16().cuda()
+    u, delta, Bri, Cri = lo(p["u"]), lo(p["delta"]), lo(p["Bc"]), lo(p["Cc"])
+    theta, dy, Dsk = p["theta"].cuda(), p["dy"].cuda(), p["Dskip"].cuda()
+    _, _, hck = scan.unitary_fwd_raw(u, delta, theta, Bri, Cri, Dsk, ck=ck)
+    want = scan.unitary_bwd_raw(dy, None, u, delta, theta, Bri, Cri, Dsk, hck, ck)
+    du, dd = (torch.empty(B, D, L, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    dth, acc = torch.empty(B, D, L, device="cuda"), [torch.zeros(B, N, L, 2, device="cuda") for _ in range(2)]
+    _lib.check(_lib.load().aussm_unitary_bwd_aux(
+        *[_lib.ptr(t) for t in (dy, None, u, delta, theta, Bri, Cri, Dsk, hck, None, du, dd, dth, *acc, torch.zeros(D, device="cuda"), None)],
+        B, D, N, L, ck, _lib.BF16 | 0x100, 1, scan._stream()), "aussm_unitary_bwd_aux")
+    for got, w in ((du, want[0]), (dd, want[1])):
+        tie = float(w.abs().max()) * 2.0 ** -20
+        step = w.abs() * 2.0 ** -7 + tie                  # 2^-8 of rounding either way
+        assert bool(((got.float() - w).abs() <= step).all())
+        assert float((got != w.bfloat16()).float().mean()) < 1e-2
