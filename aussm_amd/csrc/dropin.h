@@ -457,7 +457,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
       const float Rr = hr[a] + row_prefix(pr), Ri = hi[a] + row_prefix(pi);
       // h = E R
       const float her = cs * Rr - sn * Ri, hei = cs * Ri + sn * Rr;
-      ysum += ctr[a] * her - cti[a] * hei;
+      ysum = fmaf(ctr[a], her, fmaf(-cti[a], hei, ysum));
       hr[a] = row_last(her, lane);
       hi[a] = row_last(hei, lane);
     }
@@ -634,9 +634,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     tile_load<NT, NREC, KS>(upb + (size_t)max(t - 2, t_first) * (KS * 3 * 64), sv, tid);
     f4 nx = {0, 0, 0, 0};                              // the next tile's phases, formed between the states of this one
     const u4* su = s_u[(t + 1) & 1];
+    const int lend = min(15, L - 1 - l0);               // the tile's last step that exists
     const float ut = silu_fast(uv), w = dtv * ut, sz = silu_fast(zv), av = gyv * sz;
     const float cnt = (float)(min(l_ + 1, L - l0));      // timesteps of the tile up to this one that exist
-    float ysum = 0.0f, wsum = 0.0f;
+    float ysum = 0.0f, wsum = 0.0f, thv[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       phase_part<KS>(a, xa, su, lane, nx);
@@ -654,33 +655,35 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
       const float hinr = Rer - Ptr, hini = Rei - Pti;
       const float Rr = hinr + Ppr, Ri = hini + Ppi;
       const float her = cs * Rr - sn * Ri, hei = cs * Ri + sn * Rr;                  // h_l
-      ysum += ctr_ * her - cti_ * hei;
+      ysum = fmaf(ctr_, her, fmaf(-cti_, hei, ysum));
       // adjoints
       const float hdr = av * ctr_, hdi = -av * cti_;                              // a conj(Ct)
       const float Rhr = cs * hdr + sn * hdi, Rhi = cs * hdi - sn * hdr;               // conj(E_l) (a conj(Ct))
       const float Kr = csl * ar[a] + snl * ai[a], Ki = csl * ai[a] - snl * ar[a];     // conj(E_last) hat h_out
       const float phr = row_suffix(Rhr) + Kr, phi = row_suffix(Rhi) + Ki;             // hat p_s
-      // hat w: Re(E conj(Bt) hat p)
-      const float ebr = cs * btr_ + sn * bti_, ebi = sn * btr_ - cs * bti_;   // E conj(Bt)
-      wsum += ebr * phr - ebi * phi;
+      // X = E hat p:  hat w = Re(conj(Bt) X),  hat Bt += w X
+      const float Xr = fmaf(cs, phr, -(sn * phi)), Xi = fmaf(cs, phi, sn * phr);
+      wsum = fmaf(btr_, Xr, fmaf(bti_, Xi, wsum));
+      gBr[a] = fmaf(w, Xr, gBr[a]);
+      gBi[a] = fmaf(w, Xi, gBi[a]);
       // hat G
-      float Gh = -(hdr * hei - hdi * her) + (phr * pi - phi * pr);
-      if (l_ == 15) Gh -= ar[a] * hi[a] - ai[a] * hr[a];                              // h at the last step is h_out
+      float Gh = fmaf(phr, pi, fmaf(-phi, pr, fmaf(hdi, her, -(hdr * hei))));
+      if (l_ == lend) Gh -= ar[a] * hi[a] - ai[a] * hr[a];                            // h at the last step is h_out
       const float thh = row_suffix(Gh);
-      if (lok && iok && j0 + 4 * g + a < n) dth[(size_t)(j0 + 4 * g + a) * p.xsj * q.lc + l] = thh;
-      gxb[a] += lok ? thh : 0.0f;
-      // hat Bt += E w hat p ; hat Ct += a conj(h)
-      const float ewr = cs * w, ewi = sn * w;
-      gBr[a] += ewr * phr - ewi * phi;
-      gBi[a] += ewr * phi + ewi * phr;
-      gCr[a] += av * her;
-      gCi[a] -= av * hei;
+      thv[a] = thh;
+      gxb[a] += thh;                                   // (zero past the end)
+      gCr[a] = fmaf(av, her, gCr[a]);                  // hat Ct += a conj(h)
+      gCi[a] = fmaf(-av, hei, gCi[a]);
       // hand over to the previous tile
       hr[a] = hinr;
       hi[a] = hini;
       ar[a] = row_first(phr, lane);
       ai[a] = row_first(phi, lane);
     }
+    // (stored here: a branch inside the loop cuts the four states into blocks that cannot hide each other's latencies)
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+      if (lok && iok && j0 + 4 * g + a < n) dth[(size_t)(j0 + 4 * g + a) * p.xsj * q.lc + l] = thv[a];
     ysum = rows_sum(ysum);
     wsum = rows_sum(wsum);
     if (nb > 1 && g == 0) s_yw[t & 1][wave][l_] = make_float2(ysum, wsum);
