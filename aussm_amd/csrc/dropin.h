@@ -679,7 +679,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
       hi[a] = hini;
       ar[a] = row_first(phr, lane);
       ai[a] = row_first(phi, lane);
+      // (Long phase products stay between the states: gathered by the scheduler, 32 x 256 x 16, 720 steps: 550 us, 540 so; 32 x
+      // 128, 220 gathered, 225.)
+      if (KS >= 8) __builtin_amdgcn_sched_barrier(0);
     }
+    // Loads and stores share one in-order counter: the wait for the tile, requested in front of the states, comes before this
+    // tile's stores, or it would see them out, too (32 x 128, 720 steps: 221 -> 219 us).
+    tile_store<NT, NREC, KS>(sv, s_u[t & 1], tid);
     // (stored here: a branch inside the loop cuts the four states into blocks that cannot hide each other's latencies)
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -688,7 +694,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     wsum = rows_sum(wsum);
     if (nb > 1 && g == 0) s_yw[t & 1][wave][l_] = make_float2(ysum, wsum);
     th = nx;
-    tile_store<NT, NREC, KS>(sv, s_u[t & 1], tid);
     if (nb > 1) {                                      // the channel's first wavefront adds the shares up
       __syncthreads();
       for (int k = 1; k < nb; ++k) {
