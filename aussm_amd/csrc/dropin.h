@@ -362,8 +362,12 @@ __global__ __launch_bounds__(NW * 64) void dropin_seg_kernel(const DropinBwdArgs
 // Workgroup = (batch b, NW consecutive (channel, state block) pairs), one pair per wavefront; the nb
 // wavefronts of a channel are neighbours (nb divides NW) and add their shares of y through LDS.
 // KS: 32-wide steps of the contraction over r (d <= 32 KS).
+// The tiles of U go straight to LDS up to d = 128 and in workgroups of four: without the registers in between, a workgroup of four wavefronts fits three
+// times on a compute unit at 128 < d (166 registers; the kernel waits more than it works, VALU 50 % with two wavefronts on a
+// SIMD): 32 x 256 x 16, 720 steps 342 -> 304 us, 32 x 180 214 -> 177, and 32 x 64 in workgroups of eight as before 73 -> 62.
+// One wavefront on a SIMD (d > 256) or two of wide x gain nothing from it: 8 x 300, 400 steps 109 -> 113, 8 x 250, 720 86 -> 90.
 template <int KS, int NW>
-__global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p) {
+__global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 3 : 1) void dropin_fwd_kernel(const DropinArgs p) {
   __shared__ u4 s_u[2][KS * 3 * 64];
   __shared__ f4 s_par[D_MAXN];
   __shared__ float s_y[2][NW][DT];                     // shares of y of the tile, by tile parity (nb > 1)
@@ -409,11 +413,24 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
   }
   const float Di = p.Dp[ic];
 
-  constexpr int NT = NW * 64, NREC = (KS * 3 * 64 + NT - 1) / NT;
+  constexpr bool DIRECT = KS <= 4 || (KS <= 8 && NW == 4);
+  constexpr int NT = NW * 64, NREC = DIRECT ? 1 : (KS * 3 * 64 + NT - 1) / NT;
   u4 sv[NREC];
-  tile_load<NT, NREC, KS>(upb + (size_t)tb * (KS * 3 * 64), sv, tid);
-  tile_store<NT, NREC, KS>(sv, s_u[tb & 1], tid);
+  auto fetch = [&](int t) {                            // a tile's records towards s_u[t & 1], directly 1 KiB at a time
+    const u4* __restrict__ src = upb + (size_t)t * (KS * 3 * 64);
+    if constexpr (DIRECT) {
+      for (int c = wave; c < KS * 3; c += NW) px_load_block(src + c * 64, s_u[t & 1] + c * 64, lane);
+    } else {
+      tile_load<NT, NREC, KS>(src, sv, tid);
+    }
+  };
+  auto landed = [&](int t) {
+    if constexpr (DIRECT) px_loads_done();
+    else tile_store<NT, NREC, KS>(sv, s_u[t & 1], tid);
+  };
+  fetch(tb);
   polar_params<false>(p, s_par, nullptr, tid);
+  landed(tb);
   __syncthreads();
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
@@ -433,7 +450,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
       dtn = nok ? p.dt[row + l + DT] : 0.0f;
       zn = nok ? p.z[zrow + l + DT] : 0.0f;
     }
-    if (t + 1 < ntiles) tile_load<NT, NREC, KS>(upb + (size_t)(t + 1) * (KS * 3 * 64), sv, tid);
+    if (t + 1 < ntiles) fetch(t + 1);
     // ---- running phases of the tile, less the bias: lane (column l, rows j = 4 g + a)
     f4 th = {0, 0, 0, 0};
     const u4* su = s_u[t & 1];
@@ -462,12 +479,12 @@ __global__ __launch_bounds__(NW * 64) void dropin_fwd_kernel(const DropinArgs p)
       hi[a] = row_last(hei, lane);
     }
     ysum = rows_sum(ysum);
+    if (t + 1 < ntiles) landed(t + 1);                 // (in front of this tile's store, which the counter would wait for, too)
     if (nb == 1) {
       if (p.y && iok && lok && g == 0) p.y[row + l] = silu_fast(zv) * (ysum + Di * ut);
     } else if (g == 0) {
       s_y[t & 1][wave][l_] = ysum;
     }
-    if (t + 1 < ntiles) tile_store<NT, NREC, KS>(sv, s_u[(t + 1) & 1], tid);
     __syncthreads();
     if (nb > 1 && sb == 0 && g == 0 && p.y && iok && lok) {      // the channel's first wavefront adds the shares up
       float tot = ysum;

@@ -20,11 +20,23 @@ int run_fill(const FillArgs& a, hipStream_t s) {
 constexpr int DROPIN_NW = DROPIN_NW_;     // channels (wavefronts) per workgroup
 
 // (d > 256: the rows of x take 192 registers, which leaves room for one wavefront per SIMD only)
-template <int KS>
-static void launch_fwd(const DropinArgs& a, hipStream_t s) {
-  constexpr int NW = KS > 8 ? 4 : DROPIN_NW;
+template <int KS, int NW>
+static void launch_fwd_nw(const DropinArgs& a, hipStream_t s) {
   const unsigned grid = (unsigned)((a.nseg > 1 ? a.nseg : 1) * a.b * ((a.d * a.nb + NW - 1) / NW));
   hipLaunchKernelGGL((dropin_fwd_kernel<KS, NW>), dim3(grid), dim3(NW * 64), 0, s, a);
+}
+// Past two wavefronts on every SIMD 128 < d takes workgroups of four, three to a compute unit (dropin.h); up to there they
+// would only read the tiles twice (8 x 250 x 16, 720 steps: 86 us in eights, 90 in fours; 20 x 130: 139, 87).
+template <int KS>
+static void launch_fwd(const DropinArgs& a, hipStream_t s) {
+  if constexpr (KS > 8) {
+    launch_fwd_nw<KS, 4>(a, s);
+  } else if constexpr (KS > 4) {
+    if ((a.nseg > 1 ? a.nseg : 1l) * a.b * a.d * a.nb > 256l * DROPIN_NW) launch_fwd_nw<KS, 4>(a, s);
+    else launch_fwd_nw<KS, DROPIN_NW>(a, s);
+  } else {
+    launch_fwd_nw<KS, DROPIN_NW>(a, s);
+  }
 }
 template <int KS>
 static void launch_bwd(const DropinBwdArgs& a, hipStream_t s) {

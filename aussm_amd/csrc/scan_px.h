@@ -207,18 +207,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void u
   else px_prep_body<Tin, false>(p, s_mem, blockIdx.x - nseg);
 }
 
-// ---- global memory -> LDS without passing through registers: a wavefront moves 64 records (1 KiB)
-// per instruction, lane i's record to lds + i.  The data is in LDS once the wavefront's vector-memory
-// counter says so (px_loads_done / px_wait) and a barrier has published it.  The instruction is
-// written out: left to the compiler, every later LDS read of the wavefront waits for ALL of its
-// outstanding loads of this kind, which would serialise the prefetch.
-__device__ __forceinline__ void px_load_block(const u4* __restrict__ src, u4* lds, int lane) {
-  const uint32_t dst = __builtin_amdgcn_readfirstlane(
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src + lane), "s"(dst) : "memory");
-}
-__device__ __forceinline__ void px_loads_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// ... or all but the K youngest vector-memory operations of the wavefront have completed
+// All but the K youngest vector-memory operations of the wavefront have completed
 template <int K>
 __device__ __forceinline__ void px_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(K) : "memory"); }
 // Workgroup barrier that publishes LDS contents only.  __syncthreads() also drains the

@@ -126,6 +126,13 @@ def test_segments_of_the_sequence(b, d, n, l, kfloats):
         _close(g2, w.cpu(), "gradient (from state) wrt " + name)
 
 
+# ... and more wavefronts than two for every SIMD, where 128 < d runs in workgroups of four: channels and states that do not fill
+# the last one, a last tile of one step
+@pytest.mark.parametrize("b,d,n,l", [(16, 130, 16, 17), (9, 251, 5, 40), (6, 178, 20, 33)])
+def test_forward_in_workgroups_of_four(b, d, n, l):
+    test_fused_forward_matches_oracle((b, d, n, l))
+
+
 def test_backward_from_saved_state_equals_backward_from_inputs():
     """The autograd formula hands the forward call's end state to the backward kernels; the reference-shaped
     backward operator recomputes it.  Same gradients either way."""
