@@ -1,4 +1,4 @@
-// Translation unit of the unitary reverse scan on the vector ALU (scan_bwd_unitary.h).
+// Translation unit of the unitary reverse scan of 33 to 64 states that leaves du and ddelta in bf16 (scan_bwd_unitary.h).
 #include "launch.h"
 #include "scan_bwd_unitary.h"
 
@@ -6,24 +6,12 @@ namespace aussm {
 
 // The backward workgroup keeps a (dw, dtheta) slab per wavefront in LDS: four wavefronts afford
 // 32-step tiles, eight wavefronts 16-step tiles.
-#define AUSSM_UBWD_CASE(NW_, NT_, TT_)                                                               \
-  if (c.nw == NW_ && c.nt == NT_) {                                                                  \
-    hipLaunchKernelGGL((unitary_bwd_kernel<NW_, NT_, TT_, Tin>), grid, dim3(NT_), 0, s, a);          \
-    return launch_status();                                                                          \
-  }
-
-template <typename Tin>
-static int unitary_bwd_t(const UniBwdArgs& a, Cfg c, hipStream_t s) {
-  const dim3 grid((unsigned)(a.B * a.ncg));
-  AUSSM_UBWD_CASE(1, 256, 32) AUSSM_UBWD_CASE(2, 256, 32) AUSSM_UBWD_CASE(4, 256, 32)
-  AUSSM_UBWD_CASE(8, 256, 32) AUSSM_UBWD_CASE(16, 256, 32)
-  AUSSM_UBWD_CASE(1, 512, 16) AUSSM_UBWD_CASE(2, 512, 16) AUSSM_UBWD_CASE(4, 512, 16)
-  AUSSM_UBWD_CASE(8, 512, 16)
-  return -2;
-}
-
-int run_unitary_bwd_generic(const UniBwdArgs& a, int in_dtype, Cfg c, hipStream_t s) {
-  return in_dtype == 1 ? unitary_bwd_t<bf16_t>(a, c, s) : unitary_bwd_t<float>(a, c, s);
+int run_unitary_bwd_generic(const UniBwdArgs& a, Cfg c, hipStream_t s) {
+  const dim3 grid((unsigned)(a.B * a.ncg)), block((unsigned)c.nt);
+  if (c.nw == 8 && c.nt == 512) hipLaunchKernelGGL((unitary_bwd_kernel<8, 512, 16, bf16_t>), grid, block, 0, s, a);
+  else if (c.nw == 16 && c.nt == 256) hipLaunchKernelGGL((unitary_bwd_kernel<16, 256, 32, bf16_t>), grid, block, 0, s, a);
+  else return -2;
+  return launch_status();
 }
 
 }  // namespace aussm

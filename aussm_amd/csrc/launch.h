@@ -24,7 +24,7 @@ int run_oct_fwd(int variant, const FwdArgs& a, int in_dtype, hipStream_t s);
 int run_oct_adj(int variant, const AdjSegArgs& a, int in_dtype, unsigned grid, hipStream_t s);   // adjoint entering every segment
 int run_oct_bwd(int variant, const RecBwdArgs& a, int in_dtype, hipStream_t s);
 int run_oct_ubwd(const UniBwdArgs& a, int in_dtype, hipStream_t s);   // N <= 32 where du leaves in bf16
-int run_unitary_bwd_generic(const UniBwdArgs& a, int in_dtype, Cfg c, hipStream_t s);
+int run_unitary_bwd_generic(const UniBwdArgs& a, Cfg c, hipStream_t s);   // N > 32, bf16 inputs, du and ddelta in bf16
 int run_aux_invalidate(float* tag, bool fill_tag, bool images_tag, hipStream_t s);   // clears tag(s) in the buffer's pad
 int run_hbm_probe(const float* a, const float* b, const float* c, float* o1, float* o2, int rows, int L, int pattern,
                   int write, hipStream_t s);

@@ -18,21 +18,10 @@ std::atomic<int> g_opt[AUSSM_OPT_COUNT] = {{-1}, {-1}, {-1}, {-1}, {-1}, {-1}};
 static_assert(AUSSM_OPT_COUNT == 6, "one initialiser per option");
 inline int opt(int key) { return g_opt[key].load(std::memory_order_relaxed); }
 
-// ---- configuration of unitary_bwd_kernel -------------------------------------------------------
-// The scalar loads of B_t/C_t are issued one "turn" ahead; with two or more wavefronts per SIMD
-// the turn of another wavefront doubles that distance, so for a given N the configuration with
-// MORE wavefronts (smaller NW) is preferred as long as the launch still fits one workgroup.
-inline Cfg pick_cfg(int N, int max_waves) {
-  // test/tuning override (must be one of the compiled configurations)
-  {
-    const Cfg c{opt(AUSSM_OPT_GENERIC_NW), opt(AUSSM_OPT_GENERIC_NT)};
-    if (c.nw > 0 && c.nt > 0 && c.nw * (c.nt / 64) >= N) return c;
-  }
-  const Cfg table[] = {{1, 256}, {1, 512}, {2, 512}, {4, 512}, {8, 512},
-                       {2, 256}, {4, 256}, {8, 256}, {16, 256}};
-  for (const Cfg& c : table)
-    if (c.nw * (c.nt / 64) >= N && c.nt / 64 <= max_waves) return c;
-  return Cfg{16, 256};
+// ---- configuration of unitary_bwd_kernel (33 to 64 states): eight wavefronts of eight states, unless the options force the four
+// of sixteen (two wavefronts on a SIMD hide each other's scalar loads: 64 states 10 % faster)
+inline Cfg pick_cfg() {
+  return opt(AUSSM_OPT_GENERIC_NW) == 16 && opt(AUSSM_OPT_GENERIC_NT) == 256 ? Cfg{16, 256} : Cfg{8, 512};
 }
 
 // flags that the backward entry points take beside the input type
@@ -607,7 +596,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
   }
   // (Blocks of 32 states add to what the first wrote, which bf16 would round.  8 x 72 x 37, 2957 steps: 237 us against 642.)
   if (N <= 32 || !a.g16) return run_oct_ubwd(a, in_dtype, s);
-  return run_unitary_bwd_generic(a, in_dtype, pick_cfg(a.N, 8), s);
+  return run_unitary_bwd_generic(a, pick_cfg(), s);
 }
 
 int aussm_complex_bwd(const float* dy, const float* dhL, const void* u, const void* delta, const float* rho,

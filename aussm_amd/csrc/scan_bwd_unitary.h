@@ -95,14 +95,12 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
   float2* part = s_part + wave * TT * TS;
   // lane -> element of the (row, 8 timesteps) output block of a turn: columns 0..15 are dB
   // (re, im interleaved), 16..31 dC; both halves of the wavefront add their half sum.
-  // The sums over the channels of a turn's dB / dC products: through the LDS lane transpose, whose latency hides
-  // behind the next turn, or on the vector ALU alone (`lanes_sum16`).  Measured at B=32, D=512, L=2048: with eight
-  // states per wavefront (N = 64) the vector-ALU form is 10 % faster, with four or two (N = 32, 16) 2-5 % slower.
-  // (With lanes_sum16: lane (g, c) holds column 4 (c % 4) + g of dB for c / 4 == 0, of dC for c / 4 == 1.)
-  constexpr bool VALU_SUMS = NW >= 8;
-  float* const red_dst = VALU_SUMS ? ((lane & 4) ? p.dC : p.dB) : (((lane & 31) < 2 * TG) ? p.dB : p.dC);
-  const int red_off = VALU_SUMS ? 4 * (lane & 3) + (lane >> 4) : (lane & (2 * TG - 1));
-  const bool red_mine = VALU_SUMS ? (lane & 8) == 0 : true;
+  // The sums over the channels of a turn's dB / dC products on the vector ALU (`lanes_sum16`; 10 % faster with eight states per
+  // wavefront than through the lane transpose, which the ragged path takes): lane (g, c) holds column 4 (c % 4) + g of dB
+  // for c / 4 == 0, of dC for c / 4 == 1.
+  float* const red_dst = (lane & 4) ? p.dC : p.dB;
+  const int red_off = 4 * (lane & 3) + (lane >> 4);
+  const bool red_mine = (lane & 8) == 0;
 
   auto load_ck = [&](int kb, float (&xr)[NW], float (&xi)[NW]) {
 #pragma unroll
@@ -183,15 +181,7 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
   collect_tile(rdy);
   if (ntiles > 1) load_tile(fly, (ntiles - 2) * TT);
 
-  // scalar-cache warm-up of the B_t/C_t lines, one tile ahead of the scan (see the forward kernel)
-  constexpr bool WARM = NW <= 4;
-  constexpr int RB = (int)sizeof(Tin) * 2;
   const size_t row_base = ((size_t)b * N + n0) * ld + lbeg;
-  TileWarm<WARM ? NW : 1, RB, TT> warm;
-  if (WARM && full_group && ntiles * TT == L) {
-    warm.issue(gB, gC, row_base + (size_t)(ntiles - 1) * TT, ld);
-    warm.retire();
-  }
 
   // a wavefront that owns no state never writes its slab of partial sums: it clears it once, so that the epilogue
   // can add the slabs of all wavefronts without asking which of them exist (the loop's first barrier orders the two)
@@ -202,8 +192,6 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
   for (int it = ntiles - 1; it >= 0; --it) {
     const int l0 = it * TT;
     const int tmax = (L - l0 < TT) ? (L - l0) : TT;
-    const bool warm_next = WARM && full_group && it > 0;
-    if (warm_next) warm.issue(gB, gC, row_base + l0 - TT, ld);
 
     // ---- stage
     float eu[E], edl[E], egy[E];
@@ -217,7 +205,6 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
       fast_sincosf(ok ? rdy.th[k] : 0.f, &sn, &cs);
       s_in[col * TS + row0 + k * RSTEP] = make_float4(cs, sn, edl[k] * eu[k], egy[k]);
     }
-    if (warm_next) warm.retire();
     __syncthreads();
 
     const size_t brow = row_base + l0;
@@ -226,8 +213,7 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
     if (fast) {
       // ---- fast path: groups of TG timesteps right to left; inside a group the wavefront's
       // state rows take turns, each turn consuming ONE scalar load of B_t and one of C_t that
-      // was issued a turn earlier.  The channel reduction of a turn's dB/dC products is started
-      // at the end of the turn and collected at the end of the NEXT turn.
+      // was issued a turn earlier.
       float rc[TG], rs[TG], rw[TG], rg[TG];
 #pragma unroll
       for (int t = 0; t < TG; ++t) {
@@ -235,7 +221,6 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
         rc[t] = v.x; rs[t] = v.y; rw[t] = v.z; rg[t] = v.w;
       }
       f32x16 bn = ld_c8(gB, brow + (TT - TG)), cn = ld_c8(gC, brow + (TT - TG));
-      LaneTranspose xp;
 #pragma unroll
       for (int g = NGRP - 1; g >= 0; --g) {
         float kacc[TG], qacc[TG], nc[TG], ns[TG], nw_[TG], ng[TG];
@@ -286,19 +271,12 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
             gr[k] = tg;
           }
           sched_fence();
-          if constexpr (VALU_SUMS) {
-            // the turn's 16 dB and 16 dC products summed over the channels on the vector ALU
-            float hb[16], hc[16];
+          // the turn's 16 dB and 16 dC products summed over the channels
+          float hb[16], hc[16];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) { hb[j] = vals[j]; hc[j] = vals[16 + j]; }
-            const float sb = lanes_sum16(hb, lane), sc = lanes_sum16(hc, lane);
-            rres[g * NW + k] = (lane & 4) ? sc : sb;
-          } else {
-            // collect the previous turn's sums (turn (g, k-1), or (g+1, NW-1) across a group)
-            if (k > 0) rres[g * NW + k - 1] = xp.finish();
-            else if (g < NGRP - 1) rres[(g + 1) * NW + NW - 1] = xp.finish();
-            xp.issue(vals, red, lane);
-          }
+          for (int j = 0; j < 16; ++j) { hb[j] = vals[j]; hc[j] = vals[16 + j]; }
+          const float sb = lanes_sum16(hb, lane), sc = lanes_sum16(hc, lane);
+          rres[g * NW + k] = (lane & 4) ? sc : sb;
         }
 #pragma unroll
         for (int t = 0; t < TG; ++t) {
@@ -306,7 +284,6 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
           if (g > 0) { rc[t] = nc[t]; rs[t] = ns[t]; rw[t] = nw_[t]; rg[t] = ng[t]; }
         }
       }
-      if constexpr (!VALU_SUMS) rres[NW - 1] = xp.finish();   // the last turn was (g = 0, k = NW-1)
     } else if (active) {
       // ---- general path (ragged tile or partial state group): one timestep at a time
       for (int t = tmax - 1; t >= 0; --t) {

@@ -1,15 +1,9 @@
 // Shared device helpers for the gfx950 selective-scan kernels.
 //
-// Work decomposition used by every kernel in this library
-//   * one workgroup owns (batch b, a group of CH = 64 consecutive channels);
-//   * inside the scan phase lane i of every wavefront IS channel d0 + i, and wavefront w owns the
-//     NW consecutive state indices n0 = w*NW ..; the state of (channel, n) lives in registers;
-//   * B_t[b,n,l] / C_t[b,n,l] do not depend on the channel, so inside a wavefront they are
-//     wave-uniform: they are fetched with scalar loads and used as SGPR operands of the FMAs;
-//   * u / delta / theta / dy are [B,D,L] with L fastest.  A tile of CH channels x T timesteps is
-//     loaded with lanes running along L (coalesced 128-byte row segments), converted
-//     (sincos / exp / products) once per (channel, timestep), and transposed through LDS into
-//     [t][channel] order so that the scan phase reads one 16-byte record per lane per timestep.
+// Two splits of the work: scan_oct.h and scan_bwd_unitary.h (vector ALU) give a workgroup CH = 64 channels of one batch element
+// - a wavefront eight of them with all their states, or a lane a channel and a wavefront a few states -, the matrix-core
+// kernels (scan_fwd_xdl.h, scan_bwd_xdl.h, scan_px.h) a wavefront 16 channels and chunks of 32 steps.  In all of them the
+// inputs [B, D, L], L fastest, are read along L and turned in LDS, and B_t, C_t, shared by the channels, once a workgroup.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -119,24 +113,13 @@ __device__ __forceinline__ float2 ld_c(const bf16_t* __restrict__ p, size_t idx)
   const uint32_t raw = const_as<uint32_t>(p)[idx];
   return make_float2(__uint_as_float(raw << 16), __uint_as_float(raw & 0xffff0000u));
 }
-__device__ __forceinline__ float ld_r(const float* __restrict__ p, size_t idx) { return const_as<float>(p)[idx]; }
-__device__ __forceinline__ float ld_r(const bf16_t* __restrict__ p, size_t idx) {
-  // 16-bit scalar loads do not exist: fetch the aligned 32-bit word and pick the half
-  const uint32_t raw = const_as<uint32_t>(p)[idx >> 1];
-  return __uint_as_float((idx & 1) ? (raw & 0xffff0000u) : (raw << 16));
-}
-
 // ---- eight consecutive timesteps of one state row in one scalar load (one 64-byte line for
 // complex fp32).  TG is the number of timesteps the scan consumes per row "turn".
 constexpr int TG = 8;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 struct __attribute__((aligned(8))) f32x16_a8 { f32x16 v; };
-struct __attribute__((aligned(4))) f32x8_a4 { f32x8 v; };
 struct __attribute__((aligned(4))) u32x8_a4 { u32x8 v; };
-struct __attribute__((aligned(4))) u32x4_a4 { u32x4 v; };
 
 // complex rows: idx counts (re, im) records; result = re0, im0, re1, im1, ...
 __device__ __forceinline__ f32x16 ld_c8(const float* __restrict__ p, size_t idx) {
@@ -152,21 +135,6 @@ __device__ __forceinline__ f32x16 ld_c8(const bf16_t* __restrict__ p, size_t idx
   }
   return r;
 }
-// real rows.  For bf16 the caller guarantees an even idx (4-byte aligned address).
-__device__ __forceinline__ f32x8 ld_r8(const float* __restrict__ p, size_t idx) {
-  return const_as<f32x8_a4>(p + idx)->v;
-}
-__device__ __forceinline__ f32x8 ld_r8(const bf16_t* __restrict__ p, size_t idx) {
-  const u32x4 raw = const_as<u32x4_a4>(p + idx)->v;
-  f32x8 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    r[2 * i] = __uint_as_float(raw[i] << 16);
-    r[2 * i + 1] = __uint_as_float(raw[i] & 0xffff0000u);
-  }
-  return r;
-}
-
 // Orders the instruction stream at this point: nothing is scheduled across it.
 __device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
 // A use of a wave-uniform value that emits no instruction: makes the compiler place its
@@ -179,37 +147,6 @@ __device__ __forceinline__ void touch_uniform(uint32_t v) { asm volatile("" ::"s
 // (or where nothing younger is in flight) keeps that wait from also draining recent stores.
 __device__ __forceinline__ void touch_vgpr(float v) { asm volatile("" ::"v"(v)); }
 __device__ __forceinline__ void touch_vgpr(bf16_t v) { asm volatile("" ::"v"((uint32_t)v)); }
-
-// One dword of record `idx` of a row tensor (REC_BYTES per record) through the scalar cache.  Its
-// only purpose is to pull the record's 64-byte line into the scalar cache well before the scan
-// asks for it; the value itself is discarded (pass it to touch_uniform before the next barrier).
-template <int REC_BYTES>
-__device__ __forceinline__ uint32_t ld_touch(const void* p, size_t idx) {
-  return *const_as<uint32_t>(static_cast<const char*>(p) + ((idx * REC_BYTES) & ~(size_t)3));
-}
-
-// Warm the scalar cache with the B_t/C_t lines of the NW state rows starting at record `row`
-// (row stride L records) for one tile of TT timesteps: one dword per 64-byte line (rows of real fp32 records
-// have 16 steps per line, of complex ones 8 = TG).
-template <int NW, int REC_BYTES, int TT = T>
-struct TileWarm {
-  static constexpr int STEP = (64 / REC_BYTES > TG) ? 64 / REC_BYTES : TG;   // records between touches
-  static constexpr int NTOUCH = (TT + STEP - 1) / STEP;                       // touches per row
-  uint32_t v[2 * NW * NTOUCH];
-  __device__ __forceinline__ void issue(const void* gB, const void* gC, size_t row, int L) {
-#pragma unroll
-    for (int k = 0; k < NW; ++k)
-#pragma unroll
-      for (int g = 0; g < NTOUCH; ++g) {
-        v[(2 * k) * NTOUCH + g] = ld_touch<REC_BYTES>(gB, row + (size_t)k * L + g * STEP);
-        v[(2 * k + 1) * NTOUCH + g] = ld_touch<REC_BYTES>(gC, row + (size_t)k * L + g * STEP);
-      }
-  }
-  __device__ __forceinline__ void retire() {
-#pragma unroll
-    for (int i = 0; i < 2 * NW * NTOUCH; ++i) touch_uniform(v[i]);
-  }
-};
 
 // ---- sums and moves across the four 16-lane rows of a wavefront (lane = 16 g + c) on the vector ALU.  gfx950 swaps
 // rows between two registers in one instruction (v_permlane16_swap: rows 1 and 3 of the first with rows 0 and 2 of
@@ -253,7 +190,7 @@ __device__ __forceinline__ float rows_sum(float x) {
   rows_swap32(c, d);
   return c + d;
 }
-// the value of row 3 (row 0) of the same column, in every row
+// the value of row 3 of the same column, in every row
 __device__ __forceinline__ float rows_last(float x) {
   float c = x, d = x;
   rows_swap32(c, d);                              // d = [x2 x3 x2 x3]
@@ -261,14 +198,6 @@ __device__ __forceinline__ float rows_last(float x) {
   rows_swap16(a, b);                              // b = [x3 x3 x3 x3]
   return b;
 }
-__device__ __forceinline__ float rows_first(float x) {
-  float c = x, d = x;
-  rows_swap32(c, d);                              // c = [x0 x1 x0 x1]
-  float a = c, b = c;
-  rows_swap16(a, b);                              // a = [x0 x0 x0 x0]
-  return a;
-}
-
 // DPP moves inside a row of 16 lanes (every lane has a source for the patterns used here)
 template <int CTRL>
 __device__ __forceinline__ float dpp_perm(float v) {
@@ -297,16 +226,6 @@ __device__ __forceinline__ float lanes_sum16(const float (&v)[16], int lane) {
   r += dpp_perm<0x128>(r);                                                    // row_ror:8
   return r;
 }
-
-// ---- staging geometry: a thread owns runs of FOUR consecutive timesteps of one channel row, so a
-// tile row of TT timesteps is covered by TT/4 neighbouring lanes with 16-byte accesses.
-template <int NT, int TT>
-struct StageGeom {
-  static constexpr int TPR = TT / 4;                        // threads per channel row
-  static constexpr int RW = 64 / TPR;                       // channel rows covered by one wavefront
-  static constexpr int RP = NT / TPR;                       // channel rows covered per pass
-  static constexpr int PASS = (CH + RP - 1) / RP;           // passes over the tile (1 if RP >= CH)
-};
 
 // Four consecutive raw input elements, kept exactly as loaded (no arithmetic may touch a loaded
 // register before the tile is collected, or the wait for the load moves up to the load).
@@ -444,13 +363,6 @@ __device__ __forceinline__ void sincos_small_hw(float x, float* sn, float* cs) {
 }
 
 __device__ __forceinline__ void touch4(const f4& v) { touch_vgpr(v[0]); touch_vgpr(v[1]); touch_vgpr(v[2]); touch_vgpr(v[3]); }
-
-// Sum `v` over the lanes of each aligned group of 32 lanes; result valid in every lane.
-__device__ __forceinline__ float half_wave_sum(float v) {
-#pragma unroll
-  for (int o = 16; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // ---- global memory -> LDS without passing through registers: a wavefront moves 64 records (1 KiB)
 // per instruction, lane i's record to lds + i.  The data is in LDS once the wavefront's vector-memory

@@ -84,8 +84,8 @@ const char* aussm_error_string(int code);
  *                          value 25600 = 100 MiB; the option can only lower it)
  * Workspace and auxiliary-buffer sizes do not depend on any option: a buffer sized by the query
  * functions below holds what a call of that shape uses under every setting.
- *   AUSSM_OPT_GENERIC_NW / AUSSM_OPT_GENERIC_NT   states per wavefront / threads per workgroup of
- *                          the vector-ALU kernels (both must be set; one of the built pairs) */
+ *   AUSSM_OPT_GENERIC_NW / AUSSM_OPT_GENERIC_NT   states per wavefront / threads per workgroup of the unitary
+ *                          reverse scan of more than 32 states with du in bf16: 8 / 512 (default) or 16 / 256 */
 #define AUSSM_OPT_UNITARY_FWD 0
 #define AUSSM_OPT_UNITARY_BWD 1
 #define AUSSM_OPT_SPLIT_CAP 2
@@ -157,8 +157,8 @@ int aussm_unitary_bwd(const float* dy, const float* dhL,
  *    autograd one: between a forward call and the backward call that is handed its buffer, Bc and
  *    Cc must not be modified in place, and no other call may be given the buffer;
  *  - a launch with few (batch, channel) pairs and a long sequence is split along L over more
- *    workgroups (per-segment end states from a zero start, a short chain over the segments, then
- *    the scan of every segment from its true incoming state - the two-level scan of
+ *    workgroups (per-segment end states from a zero start, then the scan of every segment, which first
+ *    composes the ones in front of it to its true incoming state - the two-level scan of
  *    ssm_adaptive_unitary_forward.cu:122-162 one level up); the segment states live behind the
  *    per-(b,d,l) part of the buffer, during the call only.  Each call writes there: two calls
  *    that share one buffer must not overlap.  aussm_set_option(AUSSM_OPT_SPLIT_CAP, 0) switches the split off.
@@ -228,12 +228,11 @@ int aussm_unitary_fwd_static(const void* u, const void* delta, const float* thet
  *
  * workspace (complex and real scans, forward and backward): aussm_scan_workspace_floats() floats of
  * device memory, 16-byte aligned, contents irrelevant on entry; may be NULL for float inputs, required
- * (AUSSM_E_NULL otherwise) for bf16 inputs, whose B_t / C_t rows the call first converts to float in it
- * (the scan consumes them as wave-uniform scalar operands; converting them there costs a scalar
- * instruction per value).  With it, a call with fewer
+ * (AUSSM_E_NULL otherwise) for bf16 inputs (its size there counts float copies of B_t / C_t, which
+ * the call no longer makes).  With it, a call with fewer
  * than 129 (batch, group of 64 channels) pairs is split along the sequence into up to 64 segments of
- * at least 128 steps that run side by side (end state / adjoint of every segment from zero, a chain
- * over the segments, then the scan proper from the true incoming states), so that short batches of
+ * at least 64 steps that run side by side (end state / adjoint of every segment from zero, then the
+ * scan proper, each segment from the composition of those in front of it), so that short batches of
  * long sequences fill the chip; results equal the unsplit call's up to fp32 rounding.  The function
  * answers 0 when the call needs none (pass NULL then).  No counterpart in the reference: its
  * complex kernel walks the sequence chunk after chunk inside one thread block
