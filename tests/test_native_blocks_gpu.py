@@ -234,6 +234,12 @@ def test_native_block_on_wide_tiles(kind, d, n, b, l, monkeypatch):
     test_native_block_matches_the_composed_layers(kind, d, n, b, l, {}, True, monkeypatch)
 
 
+# few channels of long sequences: the operator works on them in segments, with the block's strides and raw parameters
+@pytest.mark.parametrize("d,n,b,l", [(8, 4, 1, 257), (24, 20, 2, 400), (136, 4, 1, 300)])
+def test_native_block_in_segments(d, n, b, l, monkeypatch):
+    test_native_block_matches_the_composed_layers("a", d, n, b, l, {"bias": True}, True, monkeypatch)
+
+
 # ---- calls that leave the native route ------------------------------------------------------------
 
 class _Marked(torch.Tensor):
