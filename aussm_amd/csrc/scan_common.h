@@ -227,6 +227,11 @@ __device__ __forceinline__ float lanes_sum16(const float (&v)[16], int lane) {
   return r;
 }
 
+// 16-byte loads and stores that are only known to be 4-byte aligned, and 8-byte ones of four bf16 (rows start anywhere when the
+// row length is not a multiple of four): the memory pipeline takes them, the type tells the compiler so
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u2h __attribute__((ext_vector_type(2), aligned(2)));
+
 // Four consecutive raw input elements, kept exactly as loaded (no arithmetic may touch a loaded
 // register before the tile is collected, or the wait for the load moves up to the load).
 template <typename Tin> struct Quad;
@@ -235,10 +240,10 @@ template <> struct Quad<float> {
   __device__ __forceinline__ float get(int i) const { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
   __device__ __forceinline__ void touch() const { touch_vgpr(v.x); touch_vgpr(v.y); touch_vgpr(v.z); touch_vgpr(v.w); }
   __device__ __forceinline__ void zero() { v = make_float4(0.f, 0.f, 0.f, 0.f); }
-  // vec: one 16-byte load at element offset o (caller guarantees alignment and range);
+  // vec: one load of all four at element offset o (the caller guarantees the range; no alignment beyond the element's);
   // otherwise four element loads at o + idx[i].
   __device__ __forceinline__ void load(const float* __restrict__ p, size_t o, bool vec, const int (&idx)[4]) {
-    if (vec) v = *reinterpret_cast<const float4*>(p + o);
+    if (vec) { const f4u r = *reinterpret_cast<const f4u*>(p + o); v = make_float4(r[0], r[1], r[2], r[3]); }
     else v = make_float4(p[o + idx[0]], p[o + idx[1]], p[o + idx[2]], p[o + idx[3]]);
   }
 };
@@ -251,17 +256,17 @@ template <> struct Quad<bf16_t> {
   __device__ __forceinline__ void touch() const { touch_vgpr(__uint_as_float(v.x)); touch_vgpr(__uint_as_float(v.y)); }
   __device__ __forceinline__ void zero() { v = make_uint2(0u, 0u); }
   __device__ __forceinline__ void load(const bf16_t* __restrict__ p, size_t o, bool vec, const int (&idx)[4]) {
-    if (vec) v = *reinterpret_cast<const uint2*>(p + o);
+    if (vec) { const u2h r = *reinterpret_cast<const u2h*>(p + o); v = make_uint2(r[0], r[1]); }
     else v = make_uint2((uint32_t)p[o + idx[0]] | ((uint32_t)p[o + idx[1]] << 16),
                         (uint32_t)p[o + idx[2]] | ((uint32_t)p[o + idx[3]] << 16));
   }
 };
 
-// Four consecutive float32 outputs at element offset o: one 16-byte store when `vec`, else
+// Four consecutive float32 outputs at element offset o: one 16-byte store (on any element) when `vec`, else
 // element stores for the timesteps < nvalid.
 __device__ __forceinline__ void store4(float* __restrict__ p, size_t o, const float (&x)[4], bool vec, int nvalid) {
   if (vec && nvalid >= 4) {
-    *reinterpret_cast<float4*>(p + o) = make_float4(x[0], x[1], x[2], x[3]);
+    *reinterpret_cast<f4u*>(p + o) = f4u{x[0], x[1], x[2], x[3]};
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -269,9 +274,6 @@ __device__ __forceinline__ void store4(float* __restrict__ p, size_t o, const fl
   }
 }
 
-// 16-byte loads and stores that are only known to be 4-byte aligned (rows start anywhere when the row length is not a
-// multiple of four): the memory pipeline takes them, the type tells the compiler so
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 // four consecutive results at byte offset ob (of a float tensor): float, or bf16 at half the offset (g16, uniform)
 template <typename Tin>
 __device__ __forceinline__ void store_grad4(float* p, size_t ob, const f4& v, int g16) {

@@ -231,6 +231,11 @@ struct OctRows {
 // rows ahead: 220 spilled registers at 64 states.)
 __device__ __forceinline__ void pin(float& a, float& b) { asm volatile("" : "+v"(a), "+v"(b) : : "memory"); }
 
+// Inputs and results move four steps a lane at a time wherever a row starts; single elements are left to a last tile whose
+// length is no multiple of four.  (With a second path for rows that do not start on 16 bytes: 8 x 256 x 16, 2957 steps, bf16,
+// complex with the gate 395 us, now 342, S6 278 -> 246; and the longer code cost whole rows, too, 32 x 512 x 16, 2048 steps,
+// complex 1133 -> 1046.)
+
 // S: state groups of eight (8 S >= N).  FULLN: N = 8 S.  LEAN: no outputs but the end state and the product of the a_l (the
 // first pass of a call that is split along the sequence).
 template <int VAR, int S, bool FULLN, typename Tin, typename Tbc, bool LEAN>
@@ -297,10 +302,6 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
   const float dsk = (!LEAN && p.Dskip && dok) ? p.Dskip[dd] : 0.f;
   const float dbias = (VAR == VAR_REAL && p.delta_bias && dok) ? p.delta_bias[dd] : 0.f;
 
-  // 16-byte accesses need every row start (ld % 4 == 0) and every tensor base aligned
-  auto al = [](const void* q, size_t a) { return q == nullptr || (reinterpret_cast<uintptr_t>(q) % a) == 0; };
-  const bool vec = (ld % 4 == 0) && (L % 4 == 0) && al(p.u, 4 * sizeof(Tin)) && al(p.delta, 4 * sizeof(Tin)) && al(p.theta, 16) &&
-                   al(p.rho, 16) && al(p.z, 16) && al(p.y, 16);
   // two sets of loaded inputs: `rdy` has landed and is staged next, `fly` is a tile behind it
   struct Raw { Quad<Tin> u, dl; Quad<float> th, rho, z; } rdy, fly;
   fly.u.zero(); fly.dl.zero(); fly.th.zero(); fly.rho.zero(); fly.z.zero();
@@ -309,7 +310,8 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
     int idx[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) idx[i] = ll + i < L ? ll + i : L - 1;
-    const size_t o = fresh(goff + (vec ? (ll < L ? ll : L - 4) : 0));
+    const bool vec = l0 + OT <= L || L % 4 == 0;             // uniform: a lane's four steps exist or none
+    const size_t o = fresh(goff + (vec ? min(ll, L - 4) : 0));
     raw.u.load(gu, o, vec, idx);
     raw.dl.load(gdl, o, vec, idx);
     if (VAR != VAR_REAL) raw.th.load(p.theta, o, vec, idx);
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
             if (gated) acc[i] *= siluf_(gate[i]);
           }
           const int nvalid = L - (l0 + 4 * g);
-          if (dok && nvalid > 0) store4(p.y, fresh(goff + l0 + 4 * g), acc, vec, nvalid);
+          if (dok && nvalid > 0) store4(p.y, fresh(goff + l0 + 4 * g), acc, true, nvalid);
         }
         // checkpoint at the end of every ck-step block (and at the end of the sequence); ck: a multiple of the tile or half of it
         if (p.hck && dok) {
@@ -607,8 +609,6 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
   }
   const bool has_last = FULLN || 8 * (S - 1) + g < N;
   const float dbias = (VAR == VAR_REAL && p.delta_bias && dok) ? p.delta_bias[dd] : 0.f;
-  auto al = [](const void* q, size_t a) { return q == nullptr || (reinterpret_cast<uintptr_t>(q) % a) == 0; };
-  const bool vec = (ld % 4 == 0) && (L % 4 == 0) && al(p.dy, 16) && al(p.z, 16) && al(p.delta, 4 * sizeof(Tin)) && al(p.theta, 16) && al(p.rho, 16);
   struct Raw { Quad<Tin> dl; Quad<float> dy, th, rho, z; } raw;
   raw.dl.zero(); raw.dy.zero(); raw.th.zero(); raw.rho.zero(); raw.z.zero();
   auto load_tile = [&](int l0) {
@@ -616,7 +616,8 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
     int idx[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) idx[i] = ll + i < L ? ll + i : L - 1;
-    const size_t o = goff + (vec ? (ll < L ? ll : L - 4) : 0);
+    const bool vec = l0 + OT <= L || L % 4 == 0;
+    const size_t o = goff + (vec ? min(ll, L - 4) : 0);
     raw.dy.load(p.dy, o, vec, idx);
     if (VAR == VAR_REAL) raw.dl.load(gdl, o, vec, idx);
     else raw.th.load(p.theta, o, vec, idx);
@@ -849,11 +850,6 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
     }
   };
 
-  auto al = [](const void* q, size_t a) { return q == nullptr || (reinterpret_cast<uintptr_t>(q) % a) == 0; };
-  const size_t ga = sizeof(Tin) == 2 && p.g16 ? 8 : 16;
-  const bool vec = (ld % 4 == 0) && (L % 4 == 0) && al(p.u, 4 * sizeof(Tin)) && al(p.delta, 4 * sizeof(Tin)) && al(p.theta, 16) &&
-                   al(p.rho, 16) && al(p.z, 16) && al(p.dz, 16) && al(p.dy, 16) && al(p.du, ga) && al(p.ddelta, ga) && al(p.dtheta, 16) &&
-                   al(p.drho, 16);
   struct Raw { Quad<Tin> u, dl; Quad<float> dy, th, rho, z; } raw;
   raw.u.zero(); raw.dl.zero(); raw.dy.zero(); raw.th.zero(); raw.rho.zero(); raw.z.zero();
   auto load_tile = [&](int l0) {
@@ -861,7 +857,8 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
     int idx[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) idx[i] = ll + i < L ? ll + i : L - 1;
-    const size_t o = fresh(goff + (vec ? (ll < L ? ll : L - 4) : 0));
+    const bool vec = l0 + OT <= L || L % 4 == 0;             // uniform: a lane's four steps exist or none
+    const size_t o = fresh(goff + (vec ? min(ll, L - 4) : 0));
     raw.u.load(gu, o, vec, idx);
     raw.dl.load(gdl, o, vec, idx);
     raw.dy.load(p.dy, o, vec, idx);
@@ -1199,17 +1196,17 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
           float w[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) w[i] = i < nvalid ? dst[i] + v[i] : 0.f;
-          store4(dst, 0, w, vec, nvalid);
+          store4(dst, 0, w, true, nvalid);
         } else {
-          store4(dst, 0, v, vec, nvalid);
+          store4(dst, 0, v, true, nvalid);
         }
       };
       if (sizeof(Tin) == 2 && p.g16) {                     // uniform
         auto put16 = [&](float* base, const float (&v)[4]) {
           bf16_t* dst = reinterpret_cast<bf16_t*>(base) + o;
-          if (vec && nvalid >= 4) {
-            *reinterpret_cast<uint2*>(dst) = make_uint2((uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16),
-                                                        (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16));
+          if (nvalid >= 4) {
+            *reinterpret_cast<u2h*>(dst) = u2h{(uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16),
+                                               (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16)};
           } else {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
