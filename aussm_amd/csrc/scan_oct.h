@@ -14,11 +14,10 @@
 // In the split before this one (a wavefront = 64 channels x 2 states, B_t and C_t as scalar operands) every step's sums over
 // the states went through LDS, two barriers per 16 steps held all wavefronts of the compute unit together, and up to 118
 // scalar registers lived in vector lanes.  What bounds these kernels now is vector instructions: per state and step S6 7.5
-// forward and 22 backward, complex 14 and 40, the vector ALU busy 75-80 % of the time.  Two wavefronts per SIMD hide an LDS
+// forward and 22 backward, complex 14 and 40, the vector ALU busy 68-82 % of the time.  Two wavefronts per SIMD hide an LDS
 // read only if it is asked for a turn ahead of its use (forward kernel 213 -> 182 us, complex backward 967 -> 884).
-// B32 D512 N16 L2048, kernel times before and after, us: S6 bf16 forward 215 -> 182, backward 642 -> 451; complex forward
-// 414 -> 340, backward 1090 -> 786; S6 gated, softplus, L720 forward 107 -> 94, backward 273 -> 229.  Few channels, B11 D37
-// L1178 (split along L): forward 37 -> 21, adjoints 35 -> 13, backward 84 -> 45.
+// Forward and backward pass before and after, us, B32 D512 N16 L2048: S6 bf16 834 -> 630, complex 1493 -> 1040; S6 gated, softplus,
+// L720 377 -> 290; unitary gated, B5 D200 N24 L1001 228 -> 126.
 //
 // Reference semantics: extension-cpp/extension_cpp/ops.py:215-223 (unitary loop), :270-291 (complex loop), :349-356 (real
 // loop), the selective-scan call at ai-modules/wavesAI/model/aussm.py:791-802; gradient structure of
