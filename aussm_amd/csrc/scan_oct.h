@@ -296,8 +296,12 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
     for (int s = 0; s < S; ++s)
       if (8 * s + g >= N) { hr[s] = 0.f; hi[s] = 0.f; }
   }
-  // the last group's lanes without a state: their w is zero (an infinite w times B = 0 would not be)
-  const bool has_last = FULLN || 8 * (S - 1) + g < N;
+  // Lanes without a state take no part in the sums over the states (their C is zero, but their state, from infinite inputs or
+  // decays times zeros, may be a NaN).  They lie in the last group, with registers for 48 or 64 states in the last two.
+  constexpr int WHOLE_S = FULLN ? S : S > 4 ? S - 2 : S - 1;   // groups whose lanes all have a state
+  bool has[S - WHOLE_S > 0 ? S - WHOLE_S : 1];
+#pragma unroll
+  for (int s = WHOLE_S; s < S; ++s) has[s - WHOLE_S] = 8 * s + g < N;
   const float dsk = (!LEAN && p.Dskip && dok) ? p.Dskip[dd] : 0.f;
   const float dbias = (VAR == VAR_REAL && p.delta_bias && dok) ? p.delta_bias[dd] : 0.f;
 
@@ -422,20 +426,18 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
 #pragma unroll
         for (int t = 0; t < G; ++t) {
           if (t >= steps) break;                             // uniform
-          const float wt = (s < S - 1 || has_last) ? x.w[t] : 0.f;
+          float yt;
           if constexpr (VAR == VAR_REAL) {
             const float a = __builtin_amdgcn_exp2f(x.x0[t] * a2[s]);
-            hr[s] = fmaf(a, hr[s], r.br[t] * wt);
-            if constexpr (!LEAN) ya[t] = fmaf(r.cr[t], hr[s], ya[t]);
+            hr[s] = fmaf(a, hr[s], r.br[t] * x.w[t]);
+            if constexpr (!LEAN) yt = fmaf(r.cr[t], hr[s], ya[t]);
           } else {
-            const float nr = fmaf(x.x0[t], hr[s], fmaf(-x.x1[t], hi[s], r.br[t] * wt));
-            const float ni = fmaf(x.x0[t], hi[s], fmaf(x.x1[t], hr[s], r.bi[t] * wt));
+            const float nr = fmaf(x.x0[t], hr[s], fmaf(-x.x1[t], hi[s], r.br[t] * x.w[t]));
+            const float ni = fmaf(x.x0[t], hi[s], fmaf(x.x1[t], hr[s], r.bi[t] * x.w[t]));
             hr[s] = nr; hi[s] = ni;
-            if constexpr (!LEAN) {
-              ya[t] = fmaf(r.cr[t], nr, ya[t]);
-              ya[t] = fmaf(-r.ci[t], ni, ya[t]);
-            }
+            if constexpr (!LEAN) yt = fmaf(-r.ci[t], ni, fmaf(r.cr[t], nr, ya[t]));
           }
+          if constexpr (!LEAN) ya[t] = s < WHOLE_S || has[s < WHOLE_S ? 0 : s - WHOLE_S] ? yt : ya[t];
         }
       };
       auto clear = [&]() {
@@ -606,7 +608,6 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
     gr[s] = 0.f; gi[s] = 0.f;
     a2[s] = (VAR == VAR_REAL && dok && n < N) ? p.A[(size_t)d * N + n] * LOG2E : 0.f;
   }
-  const bool has_last = FULLN || 8 * (S - 1) + g < N;
   const float dbias = (VAR == VAR_REAL && p.delta_bias && dok) ? p.delta_bias[dd] : 0.f;
   struct Raw { Quad<Tin> dl; Quad<float> dy, th, rho, z; } raw;
   raw.dl.zero(); raw.dy.zero(); raw.th.zero(); raw.rho.zero(); raw.z.zero();
@@ -690,12 +691,11 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
 #pragma unroll
           for (int t = 7; t >= 0; --t) {
             if (TAIL && l0 + q * OG + t >= L) continue;                    // uniform
-            const float gy = (s < S - 1 || has_last) ? w[t] : 0.f;
-            const float yr = fmaf(cr[t], gy, gr[s]);
+            const float yr = fmaf(cr[t], w[t], gr[s]);       // (lanes without a state: whatever it is, nobody reads it)
             if constexpr (VAR == VAR_REAL) {
               gr[s] = yr * __builtin_amdgcn_exp2f(x0[t] * a2[s]);
             } else {
-              const float yi = fmaf(-ci[t], gy, gi[s]);
+              const float yi = fmaf(-ci[t], w[t], gi[s]);
               gr[s] = fmaf(x0[t], yr, x1[t] * yi);
               gi[s] = fmaf(x0[t], yi, -x1[t] * yr);
             }
@@ -821,9 +821,13 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
     seg_chain<VAR, true, S>(p.seg + e * NT_ * C, p.segq + e * 2, -(ptrdiff_t)D * NT_ * C, -(ptrdiff_t)D * 2, p.ns - 1 - sg, nn, a2, gr, gi);
 #pragma unroll
     for (int s = 0; s < S; ++s)
-      if (8 * s + g >= N) { gr[s] = 0.f; gi[s] = 0.f; }
+      if (!dok || 8 * s + g >= N) { gr[s] = 0.f; gi[s] = 0.f; }   // (lanes behind the last channel read that one's)
   }
+  // Lanes of the last group without a state.  Complex and unitary: nothing comes in there (w and dy count as zero), so state and
+  // adjoint stay zero wherever the other lanes' are not NaN.  Real: an infinite step makes a NaN of zero state and zero decay rate
+  // where the other lanes have a zero or an infinity, so what they add to the sums over the states is dropped (`mine`).
   const bool has_last = FULLN || 8 * (S - 1) + g < N;
+  auto seen = [&](float v, int s) { return C == 1 || s < S - 1 || has_last ? v : 0.f; };
 
   // ---- state before step l of the segment (a multiple of 16; unitary: of ck, or its end): the checkpoint there, or the initial
   // state
@@ -1020,7 +1024,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
         for (int t = 0; t < G; ++t) {
           const int tt = q * G + t;
           const bool skip = TAIL && lh + tt >= L;            // uniform
-          const float wt = (s < S - 1 || has_last) ? x.w[t] : 0.f;
+          const float wt = seen(x.w[t], s);
           if constexpr (VAR == VAR_REAL) {
             const float a = skip ? 1.f : __builtin_amdgcn_exp2f(x.x0[t] * a2[s]);
             xr[s] = fmaf(a, xr[s], r.br[t] * wt);
@@ -1061,8 +1065,8 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
 #pragma unroll
         for (int t = G - 1; t >= 0; --t) {
           const int tt = qq * G + t;
+          const float wt = seen(x.w[t], s), gy = seen(x.gy[t], s);
           const bool mine = s < S - 1 || has_last;
-          const float wt = mine ? x.w[t] : 0.f, gy = mine ? x.gy[t] : 0.f;
           const float hpr = !UNI && tt > 0 ? hsr[!UNI && tt > 0 ? tt - 1 : 0][s] : st.r[s];
           if constexpr (UNI) {
             float& hr = hsr[0][s];
@@ -1086,12 +1090,12 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
           } else if constexpr (VAR == VAR_REAL) {
             gr[s] = fmaf(r.cr[t], gy, gr[s]);
             vb_r[t] = wt * gr[s];
-            if (GATED) ya[t] = fmaf(r.cr[t], hsr[tt][s], ya[t]);
-            ka[t] = fmaf(r.br[t], gr[s], ka[t]);
+            if (GATED) ya[t] = mine ? fmaf(r.cr[t], hsr[tt][s], ya[t]) : ya[t];
+            ka[t] = mine ? fmaf(r.br[t], gr[s], ka[t]) : ka[t];
             gr[s] *= hsi[tt][s];
             const float xx = gr[s] * hpr;
             dAacc[s] = fmaf(xx, x.x0[t], dAacc[s]);
-            xa[t] = fmaf(xx, an[s], xa[t]);
+            xa[t] = mine ? fmaf(xx, an[s], xa[t]) : xa[t];
           } else {
             const float hpi = tt > 0 ? hsi[tt > 0 ? tt - 1 : 0][s] : st.i[s];
             gr[s] = fmaf(r.cr[t], gy, gr[s]);
@@ -1123,7 +1127,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
         sched_fence();
 #pragma unroll
         for (int t = 0; t < G; ++t) {
-          const float gy = (s < S - 1 || has_last) ? x.gy[t] : 0.f;
+          const float gy = seen(x.gy[t], s);
           vb_r[t] = UNI ? vc_r[t] : gy * hsr[UNI ? 0 : qq * G + t][s];
           if (C == 2) vb_i[t] = UNI ? vc_i[t] : -gy * hsi[UNI ? 0 : qq * G + t][s];
         }

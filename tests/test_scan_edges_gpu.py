@@ -75,3 +75,89 @@ def test_unitary_gradients_in_bf16_are_the_rounded_sums(N):
         step = w.abs() * 2.0 ** -7 + tie                  # 2^-8 of rounding either way
         assert bool(((got.float() - w).abs() <= step).all())
         assert float((got != w.bfloat16()).float().mean()) < 1e-2
+
+
+def _infinite(variant, N, L, which, at, seed=0):
+    """Inputs of three channels with one infinity at (1, 2, at).  The signs let the loop's output be an infinity there: no sum of
+    opposite ones."""
+    p = O.make_core_inputs(2, 3, N, L, seed=N + seed, variant=variant)
+    p["u"][1, 2, at] = p["u"][1, 2, at].abs() + 0.5
+    p["Dskip"] = p["Dskip"].abs()
+    if "A" in p:
+        p["A"] = p["A"].clamp(min=-0.5)                   # (no product of a segment's decays underflows: zero times infinity)
+    for k in ("Bm", "Cm", "Bc", "Cc"):
+        if k in p:
+            p[k] = torch.complex(p[k].real.abs(), (-1 if k == "Bc" else 1) * p[k].imag.abs()) if p[k].is_complex() else p[k].abs()
+    if which:
+        p[which][1, 2, at] = float("inf")
+    names = {"real": ("u", "delta", "A", "Bm", "Cm", "Dskip"), "complex": ("u", "delta", "rho", "theta", "Bc", "Cc", "Dskip"),
+             "unitary": ("u", "delta", "theta", "Bc", "Cc", "Dskip")}[variant]
+    return p, names
+
+
+def _scans(variant):
+    from aussm_amd import scan
+    loop, fn = {"real": (O.real_core_loop, scan.selective_scan_fn), "complex": (O.complex_core_loop, scan.complex_scan),
+                "unitary": (O.unitary_core_loop, scan.unitary_scan)}[variant]
+    return lambda *t: loop(*t)[0], fn
+
+
+# states in the middle of the last group of eight, in the group before the last (33 and 49 states take registers for 48 and 64), and
+# of a whole group that is not there; whole and split along the sequence
+STATES = [19, 33, 41, 49]
+
+
+@pytest.mark.parametrize("N", [5] + STATES)
+@pytest.mark.parametrize("which", ["u", "delta"])
+@pytest.mark.parametrize("L", [41, 290])
+def test_lanes_without_a_state_take_no_infinity(N, which, L):
+    """Outputs of the real scan: infinities where the loop has them, and no NaN where it has none."""
+    p, names = _infinite("real", N, L, which, 20)
+    loop, scan_fn = _scans("real")
+    want = loop(*(p[k] for k in names))
+    assert bool(torch.isinf(want[1, 2, 20]))
+    got = scan_fn(*(p[k].cuda() for k in names)).cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+
+
+@pytest.mark.parametrize("N", STATES)
+@pytest.mark.parametrize("variant", ["complex", "unitary"])
+def test_lanes_without_a_complex_state_take_no_infinity(variant, N):
+    """At the step itself every state is (inf, -inf) and every C has two positive parts, so the output is an infinity (from the next
+    step on the rotation takes differences of infinities)."""
+    p, names = _infinite(variant, N, 41, "u", 20)
+    y = _scans(variant)[1](*(p[k].cuda() for k in names)).cpu()
+    assert bool(torch.isposinf(y[1, 2, 20])) and bool(torch.isfinite(y[1, 2, :20]).all())
+
+
+def _gradients(fn, p, names, dev, dtype):
+    to = lambda t: t.to(torch.complex128 if t.is_complex() and dtype == torch.float64 else t.dtype if t.is_complex() else dtype)
+    lv = [to(p[k]).to(dev, copy=True).requires_grad_(True) for k in names]
+    y = fn(*lv)
+    y.backward(to(p["dy"]).to(dev))
+    return dict(zip(names, (t.grad.cpu() for t in lv)))
+
+
+@pytest.mark.parametrize("N", [5, 19, 33, 41])
+@pytest.mark.parametrize("L", [41, 290])
+def test_gradients_before_an_infinite_step_size_are_finite(N, L):
+    """exp(delta A) is zero at that step: what lies in front of it does not see what lies behind.  Where the loop's gradients
+    are finite, so are these, and equal to rounding (float64 against float32: a few hundred sums of terms of order one)."""
+    p, names = _infinite("real", N, L, "delta", 20)
+    loop, scan_fn = _scans("real")
+    want, got = _gradients(loop, p, names, "cpu", torch.float64), _gradients(scan_fn, p, names, "cuda", torch.float32)
+    assert bool(torch.isfinite(want["u"][1, 2, :20]).all()) and bool(torch.isfinite(want["delta"][1, 2, :20]).all())
+    for k in ("u", "delta"):
+        ok = torch.isfinite(want[k])
+        assert bool(torch.isfinite(got[k][ok]).all()), k
+        assert float((got[k][ok] - want[k][ok]).norm() / want[k][ok].norm()) < 1e-4, k
+
+
+def test_an_infinite_gradient_in_the_last_channel_of_a_split_call():
+    """Lanes behind the last channel take part in the sums over the channels with nothing, not with 0 times the last one's adjoint."""
+    p, names = _infinite("real", 19, 290, None, 0)
+    p["dy"][1, 2, 250] = float("inf")
+    loop, scan_fn = _scans("real")
+    want, got = (_gradients(f, p, names, dev, torch.float32)["Bm"] for f, dev in ((loop, "cpu"), (scan_fn, "cuda")))
+    assert bool(torch.isinf(want[1, :, :251]).all())
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
