@@ -43,6 +43,9 @@ inline int check_common(int B, int D, int N, int L, int ck, int in_dtype) {
 // Checkpoint interval of the recomputing backward kernels (complex, real)
 constexpr int REC_CK = AUSSM_TILE / 2;
 
+// A state handed out over the one handed in: such a call is not split along the sequence, since its first segments would still
+// read what its last one writes (the adjoint of the state alike).
+inline bool overlap(const float* p, const float* q, size_t n) { return p && q && p < q + n && q < p + n; }
 inline bool misaligned(const void* p, size_t a) { return p && (reinterpret_cast<uintptr_t>(p) % a) != 0; }
 
 // The matrix-core kernels cover the common unitary case (fp32 or bf16 inputs, 6 <= N <= 16, L a multiple of 4,
@@ -232,9 +235,10 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
     if (int e = run_aux_invalidate(ws.pad, !fill && !clear_in_kernel, mode != 6 && ws.stamp, s)) return e;
   const bool had_aux = a.aux != nullptr;
   if (!fill) a.aux = nullptr;
+  const bool in_place = overlap(a.h0, a.hL, (size_t)a.B * a.D * a.N * 2);
   if (!mode) {
     // vector-ALU kernel; with a segment area and few (batch, channel group) pairs, split along the sequence
-    const GSplit sp = ws.gseg ? generic_split(a.B, a.D, a.L, a.ck, true) : GSplit{1, a.L};
+    const GSplit sp = ws.gseg && !in_place ? generic_split(a.B, a.D, a.L, a.ck, true) : GSplit{1, a.L};
     if (sp.ns > 1) {
       const int B = a.B;
       float* seg = ws.gseg;
@@ -253,7 +257,7 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
   const int B = a.B, L = a.L;
   SegArgs sa{};
   unsigned nseg = 0;                           // workgroups of the segment-state pass, run with the pre-pass (mode 6)
-  if ((mode == 2 || mode == 3 || mode == 6) && ws.seg) {
+  if ((mode == 2 || mode == 3 || mode == 6) && ws.seg && !in_place) {
     const USplit sp = unitary_split(B, a.D, a.N, L, a.ck, true, ws.seg_room);
     if (sp.ns > 1) {
       // 1. end state of every segment from a zero start and its rotation; 2. the scan proper over (batch, segment) pairs,
@@ -283,7 +287,8 @@ int launch_unitary_fwd(FwdArgs a, int in_dtype, hipStream_t s, AuxLayout ws) {
 int launch_generic_fwd(int variant, FwdArgs a, int in_dtype, float* ws, hipStream_t s) {
   if (in_dtype == AUSSM_BF16 && !ws) return AUSSM_E_NULL;
   if (misaligned(ws, 16)) return AUSSM_E_ALIGN;
-  const GSplit sp = ws ? generic_split(a.B, a.D, a.L, a.ck, true) : GSplit{1, a.L};
+  const bool in_place = overlap(a.h0, a.hL, (size_t)a.B * a.D * a.N * (variant == VAR_REAL ? 1 : 2));
+  const GSplit sp = ws && !in_place ? generic_split(a.B, a.D, a.L, a.ck, true) : GSplit{1, a.L};
   if (sp.ns > 1) {
     const int B = a.B, C = variant == VAR_REAL ? 1 : 2;
     float* seg = ws;
@@ -302,7 +307,8 @@ int launch_generic_fwd(int variant, FwdArgs a, int in_dtype, float* ws, hipStrea
 int launch_generic_bwd(int variant, RecBwdArgs a, int in_dtype, float* ws, hipStream_t s) {
   if (in_dtype == AUSSM_BF16 && !ws) return AUSSM_E_NULL;
   if (misaligned(ws, 16)) return AUSSM_E_ALIGN;
-  const GSplit sp = ws ? generic_split(a.B, a.D, a.L, REC_CK, true) : GSplit{1, a.L};
+  const bool in_place = overlap(a.dhL, a.dh0, (size_t)a.B * a.D * a.N * (variant == VAR_REAL ? 1 : 2));
+  const GSplit sp = ws && !in_place ? generic_split(a.B, a.D, a.L, REC_CK, true) : GSplit{1, a.L};
   if (sp.ns > 1) {
     const int B = a.B, C = variant == VAR_REAL ? 1 : 2;
     float* seg = ws;
@@ -550,11 +556,12 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
   a.auxtag = aux_tag(u, delta, theta, Bc, Cc, B, D, N, L, in_dtype);
   const AuxLayout ws = aux_layout(aux, B, D, N, L, ck);
   const int mode = bwd_mode_for(B, D, N, L, ck, urep, ws.img != nullptr);
+  const bool in_place = overlap(dhL, dh0, (size_t)B * D * N * 2);
   if (mode > 0 &&
       !(misaligned(dy, 16) || misaligned(u, 16) || misaligned(delta, 16) || misaligned(theta, 16) ||
         misaligned(du, 16) || misaligned(ddelta, 16) || misaligned(dtheta, 16) || misaligned(Bc, 16) ||
         misaligned(Cc, 16))) {
-    const USplit sp = aux ? unitary_split(B, D, N, L, ck, true, ws.seg_room) : USplit{1, L, 1, 1};
+    const USplit sp = aux && !in_place ? unitary_split(B, D, N, L, ck, true, ws.seg_room) : USplit{1, L, 1, 1};
     if (sp.ns > 1) {
       // adjoint at the start of every segment from a zero adjoint at its end
       float* seg = ws.seg;
@@ -584,7 +591,7 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL, const void* u, cons
     return run_xdl_bwd(mode, a, in_dtype, s);
   }
   // vector-ALU kernel; split along the sequence like the forward call
-  const GSplit sp = ws.gseg ? generic_split(B, D, L, ck, true) : GSplit{1, L};
+  const GSplit sp = ws.gseg && !in_place ? generic_split(B, D, L, ck, true) : GSplit{1, L};
   if (sp.ns > 1) {
     float* seg = ws.gseg;
     float* ptot = seg + (size_t)B * sp.ns * D * N * 2;

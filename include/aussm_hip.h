@@ -111,6 +111,8 @@ int aussm_bwd_checkpoint_interval(int variant);
  * the device scan of extension-cpp/extension_cpp/csrc/cuda/ssm_adaptive_unitary_forward.cu:113-181
  * for a phase that is given per (b,d,l).
  * Optional (NULL allowed): Dskip, z, h0, y (NULL = states only), hL, hck.
+ * The final state may be handed out over the initial one (hL == h0), here and in every scan below, and the adjoint of the
+ * initial state over that of the final one (dh0 == dhL); such a call is not split along the sequence.
  * Kernel choice is internal: calls with 6 <= N <= 16, L a multiple of 4, 16-byte aligned
  * tensors and ck a multiple of AUSSM_TILE run on the matrix cores (fp32-accurate, see the
  * kernel headers); every other accepted call runs on the vector ALU.  Results agree to

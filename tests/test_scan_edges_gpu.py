@@ -161,3 +161,59 @@ def test_an_infinite_gradient_in_the_last_channel_of_a_split_call():
     want, got = (_gradients(f, p, names, dev, torch.float32)["Bm"] for f, dev in ((loop, "cpu"), (scan_fn, "cuda")))
     assert bool(torch.isinf(want[1, :, :251]).all())
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+
+
+# on the vector ALU and on the matrix cores, shapes that split along the sequence when the two states lie apart
+@pytest.mark.parametrize("variant,N,L", [("real", 16, 1500), ("complex", 16, 1500), ("unitary", 24, 1500), ("unitary", 16, 1536)])
+def test_the_state_in_place(variant, N, L):
+    """h0 and hL, dhL and dh0 of the C entry points in one buffer: what separate buffers give (to the rounding of a split call)."""
+    from aussm_amd import _lib, scan
+    B, D = 2, 70
+    p = {k: v.cuda() for k, v in O.make_core_inputs(B, D, N, L, seed=N, variant=variant).items()}
+    g = torch.Generator().manual_seed(1)
+    h0, dhL = (torch.randn(B, D, N, *([] if variant == "real" else [2]), generator=g).cuda() for _ in range(2))
+    ri = lambda t: torch.view_as_real(t).contiguous()
+    lib, stream, ptr, f32 = _lib.load(), scan._stream(), _lib.ptr, _lib.F32
+    if variant == "real":
+        ck, v = scan.REC_CK, _lib.VAR_REAL
+        first, Bm, Cm = (p["u"], p["delta"], p["A"]), p["Bm"], p["Cm"]
+    else:
+        ck, v = (scan.REC_CK, _lib.VAR_COMPLEX) if variant == "complex" else (scan.unitary_ck(B, D, N, L), 0)
+        first = (p["u"], p["delta"], *([p["rho"]] if variant == "complex" else []), p["theta"])
+        Bm, Cm = ri(p["Bc"]), ri(p["Cc"])
+    if variant == "unitary":
+        assert lib.aussm_unitary_split_segments(B, D, N, L, ck) > 1
+        room = lib.aussm_unitary_aux_floats(B, D, N, L, ck)
+    else:
+        room = lib.aussm_scan_workspace_floats(v, B, D, N, L, ck, f32)
+        assert room
+    ws, sizes = torch.zeros(room, device="cuda"), (B, D, N, L, ck, f32)
+
+    def run(start, end, adj_in, adj_out):
+        y, hck = torch.empty(B, D, L, device="cuda"), torch.empty(B, scan.num_checkpoints(L, ck), Bm[0, :, 0].numel(), D, device="cuda")
+        du, dd, dth, drh = (torch.empty(B, D, L, device="cuda") for _ in range(4))
+        dB, dC, dD = torch.zeros_like(Bm), torch.zeros_like(Cm), torch.zeros(D, device="cuda")
+        t = lambda *a: [ptr(x) if torch.is_tensor(x) else x for x in a]
+        kept = start.clone()                              # (the reverse scan's own h0)
+        if variant == "real":
+            _lib.check(lib.aussm_real_fwd(*t(*first, Bm, Cm, p["Dskip"], None, None, 0, start, y, end, hck, ws), *sizes, stream), "fwd")
+            dA = torch.zeros_like(p["A"])
+            _lib.check(lib.aussm_real_bwd(*t(p["dy"], adj_in, *first, Bm, Cm, p["Dskip"], None, 0, kept, hck, du, dd, dA, dB, dC, dD, adj_out,
+                                             None, None, ws), *sizes, stream), "bwd")
+            grads = [du, dd, dA]
+        elif variant == "complex":
+            _lib.check(lib.aussm_complex_fwd(*t(*first, Bm, Cm, p["Dskip"], None, start, y, end, hck, ws), *sizes, stream), "fwd")
+            _lib.check(lib.aussm_complex_bwd(*t(p["dy"], adj_in, *first, Bm, Cm, p["Dskip"], kept, hck, du, dd, drh, dth, dB, dC, dD, adj_out,
+                                                None, None, ws), *sizes, stream), "bwd")
+            grads = [du, dd, drh, dth]
+        else:
+            _lib.check(lib.aussm_unitary_fwd_aux(*t(*first, Bm, Cm, p["Dskip"], None, start, y, end, hck, ws), *sizes, 1, stream), "fwd")
+            _lib.check(lib.aussm_unitary_bwd_aux(*t(p["dy"], adj_in, *first, Bm, Cm, p["Dskip"], hck, ws, du, dd, dth, dB, dC, dD, adj_out),
+                                                 *sizes, 1, stream), "bwd")
+            grads = [du, dd, dth]
+        return [y, end, *grads, dB, dC, dD, adj_out]
+
+    want = run(h0, torch.empty_like(h0), dhL, torch.empty_like(h0))
+    state, adj = h0.clone(), dhL.clone()
+    for got, w in zip(run(state, state, adj, adj), want):
+        assert float((got - w).norm() / w.norm()) < 2e-5
