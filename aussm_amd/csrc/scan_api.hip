@@ -460,10 +460,8 @@ int aussm_unitary_fwd_static(const void* u, const void* delta, const float* thet
   if (misaligned(Bc, ca) || misaligned(Cc, ca)) return AUSSM_E_ALIGN;
   // the only workspace a forward call without checkpoints uses: the segment states of a launch
   // that is split along L
-  size_t need = seg_floats(B, D, N, L, seg_capacity(B, D, N, L, ck));
+  const size_t need = seg_floats(B, D, N, L, seg_capacity(B, D, N, L, ck));
   if (need > STATIC_SCRATCH_FLOATS) return AUSSM_E_SCRATCH;
-  // (unequal segments are taken only where their states fit: such a call is not refused)
-  if (unitary_split(B, D, N, L, ck, false, STATIC_SCRATCH_FLOATS).ns > 1) need = STATIC_SCRATCH_FLOATS;
   float* scratch = nullptr;
   if (need > 0)
     if (int e = static_scratch(&scratch)) return e;
@@ -474,8 +472,9 @@ int aussm_unitary_fwd_static(const void* u, const void* delta, const float* thet
   a.ld = L; a.ns = 1; a.urep = 1;
   // (every segment state the scan reads is written earlier in the same call: nothing in the
   // scratch has to start at zero)
-  // (the vector-ALU kernels do not split here: no gseg)
-  return launch_unitary_fwd(a, in_dtype, (hipStream_t)stream, AuxLayout{scratch, nullptr, nullptr, nullptr, nullptr, nullptr, STATIC_SCRATCH_FLOATS});
+  // (Neither the vector-ALU kernels, no gseg, nor sequences that do not halve into equal segments, no room, split here: all calls
+  // on a GPU share one array, and those that need none of it may run on several streams at once.)
+  return launch_unitary_fwd(a, in_dtype, (hipStream_t)stream, AuxLayout{scratch, nullptr, nullptr, nullptr, nullptr, nullptr, 0});
 }
 
 int aussm_complex_fwd(const void* u, const void* delta, const float* rho, const float* theta, const void* Bc,

@@ -209,7 +209,8 @@ int aussm_unitary_bwd_aux(const float* dy, const float* dhL,
  * inside the library, which every GPU the library runs on holds from the first use to the end of
  * the process.  Same arguments and results (to rounding) as aussm_unitary_fwd_aux with a buffer
  * sized for (B, D, N, L, ck); it runs the kernels that build their operands themselves, since it
- * has no room for prepared ones.  A call whose segment states do not fit returns AUSSM_E_SCRATCH.
+ * has no room for prepared ones.  A call whose segment states do not fit returns AUSSM_E_SCRATCH.  Only sequences that halve into
+ * equal segments are split here and use the array.
  * All calls on one GPU share that GPU's array: calls that overlap there (different streams,
  * different threads) race; calls in one stream are ordered and safe.  Nothing in the array has
  * to start at zero (every state read is written earlier in the same call).

@@ -58,6 +58,19 @@ def test_static_entry_point_matches_the_workspace_one_twice_in_a_row():
         assert torch.equal(y, y_ref) and torch.equal(hL, h_ref), "same kernels on the same inputs: bit for bit"
 
 
+# a last segment shorter than the others, one of four steps, a number of checkpoint blocks that is no power of two
+@pytest.mark.parametrize("B,D,N,L,equal", [(1, 40, 16, 1100, 1), (26, 70, 16, 516, 1), (1, 64, 16, 1536, 4)])
+def test_static_entry_point_leaves_the_shared_array_alone(B, D, N, L, equal):
+    """The workspace call cuts these lengths into unequal segments.  The static one does not, so that calls that need no array stay
+    independent of each other: it does what the workspace call does with as many segments as halving gives, bit for bit."""
+    from aussm_amd import _lib
+    (y, hL), _, ns = _run_both(B, D, N, L, 31, False, fwd_mode=3)
+    assert ns >= 2 * equal
+    with _lib.options(split_cap=equal):
+        _, (y_ref, h_ref), _ = _run_both(B, D, N, L, 31, False, fwd_mode=3)
+    assert torch.equal(y, y_ref) and torch.equal(hL, h_ref)
+
+
 def test_static_entry_point_rejects_what_does_not_fit():
     import ctypes
     from aussm_amd import _lib
