@@ -50,7 +50,7 @@ TRAFFIC_JSON = os.path.join(ROOT, "profiles", "traffic.json")
 # it - <float, true> - finds them and leaves at once, as does the recomputing kernel launched behind the scan kernel)
 FWD_KERNELS = {0: ["oct_fwd_kernel<0"], 2: ["unitary_fwd_xdl_kernel<2"], 3: ["unitary_fwd_xdl_kernel<3"],
                6: ["unitary_px_prep_kernel<float, false", "unitary_fwd_px_kernel"]}
-BWD_KERNELS = {0: ["unitary_bwd_kernel"], 2: ["unitary_bwd_xdl_kernel<2"], 3: ["unitary_bwd_xdl_kernel<3, 2"],
+BWD_KERNELS = {0: ["oct_bwd_kernel<0"], 2: ["unitary_bwd_xdl_kernel<2"], 3: ["unitary_bwd_xdl_kernel<3, 2"],
                5: ["unitary_bwd_xdl_kernel<3, 3"],
                6: ["unitary_bwd_px_kernel", "unitary_px_prep_kernel<float, true", "unitary_bwd_xdl_kernel<3, 2"]}
 

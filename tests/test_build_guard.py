@@ -98,3 +98,21 @@ def test_benchmark_digests_the_kernel_sources():
     finally:
         sys.path.remove(root)
     assert os.path.isdir(os.path.join(root, "aussm_amd", "csrc", "host")) and len(bench.source_digest()) == 16
+
+
+def test_benchmark_names_kernels_that_a_float_call_runs():
+    """Traffic records are looked up by these names: each has an instance in the library, and not of bf16 inputs alone."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    sys.path.insert(0, root)
+    try:
+        import bench
+    finally:
+        sys.path.remove(root)
+    symbols = [s for s in subprocess.run(["nm", "-C", build.lib_path()], capture_output=True, text=True, check=True).stdout.splitlines()
+               if "_kernel<" in s and "unsigned short" not in s]
+    for names in [*bench.FWD_KERNELS.values(), *bench.BWD_KERNELS.values()]:
+        for name in names:
+            assert any(f"::{name}" in s for s in symbols), name
