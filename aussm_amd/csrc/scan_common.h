@@ -230,6 +230,7 @@ __device__ __forceinline__ float lanes_sum16(const float (&v)[16], int lane) {
 // 16-byte loads and stores that are only known to be 4-byte aligned, and 8-byte ones of four bf16 (rows start anywhere when the
 // row length is not a multiple of four): the memory pipeline takes them, the type tells the compiler so
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t u2h __attribute__((ext_vector_type(2), aligned(2)));
 
 // Four consecutive raw input elements, kept exactly as loaded (no arithmetic may touch a loaded
@@ -303,8 +304,8 @@ __device__ __forceinline__ void seg_chain(const float* __restrict__ z, const flo
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const ptrdiff_t e = j + i < cnt ? j + i : cnt - 1;
-      const float2 qq = *reinterpret_cast<const float2*>(q + e * qs);
-      qr[i] = qq.x; qi[i] = qq.y;
+      const f2u qq = *reinterpret_cast<const f2u*>(q + e * qs);      // (real: behind an odd number of floats, maybe)
+      qr[i] = qq[0]; qi[i] = qq[1];
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         if (VAR == VAR_REAL) {
