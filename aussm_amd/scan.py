@@ -171,10 +171,12 @@ REC_CK = 16          # checkpoint interval the recomputing backward kernels (com
 
 def _scan_workspace(variant: int, u: Tensor, n: int, ck: int) -> Optional[Tensor]:
     """Workspace of a complex / real call for inputs shaped like u (aussm_scan_workspace_floats): segment
-    states that let a call with few (batch, channel group) pairs split along the sequence, and the float
-    copies of bfloat16 B_t / C_t.  None when the call needs neither."""
+    states that let a call with few (batch, channel group) pairs split along the sequence.  None when the call
+    needs none; bfloat16 calls need one in any case, of the float call's size or four floats."""
     b, d, l = u.shape
-    floats = _lib.load().aussm_scan_workspace_floats(variant, b, d, n, l, ck, _in_dtype(u))
+    floats = _lib.load().aussm_scan_workspace_floats(variant, b, d, n, l, ck, _lib.F32)
+    if _in_dtype(u) == _lib.BF16:
+        floats = max(floats, 4)
     return torch.empty((floats,), device=u.device, dtype=torch.float32) if floats else None
 
 

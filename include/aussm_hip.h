@@ -231,8 +231,8 @@ int aussm_unitary_fwd_static(const void* u, const void* delta, const float* thet
  *
  * workspace (complex and real scans, forward and backward): aussm_scan_workspace_floats() floats of
  * device memory, 16-byte aligned, contents irrelevant on entry; may be NULL for float inputs, required
- * (AUSSM_E_NULL otherwise) for bf16 inputs (its size there counts float copies of B_t / C_t, which
- * the call no longer makes).  With it, a call with fewer
+ * (AUSSM_E_NULL otherwise) for bf16 inputs.  Their size counts room for float copies of B_t / C_t, which the call
+ * does not make: the float call's size, and at least 16 bytes, is all that it uses.  With it, a call with fewer
  * than 129 (batch, group of 64 channels) pairs is split along the sequence into up to 64 segments of
  * at least 64 steps that run side by side (end state / adjoint of every segment from zero, then the
  * scan proper, each segment from the composition of those in front of it), so that short batches of

@@ -217,3 +217,23 @@ def test_the_state_in_place(variant, N, L):
     state, adj = h0.clone(), dhL.clone()
     for got, w in zip(run(state, state, adj, adj), want):
         assert float((got - w).norm() / w.norm()) < 2e-5
+
+
+@pytest.mark.parametrize("variant", ["real", "complex"])
+def test_bf16_calls_allocate_their_results_only(variant):
+    """A call that is not split needs no room beside what it returns (bf16 B_t and C_t are read as they are)."""
+    B, D, N, L = 32, 320, 16, 512
+    p = O.make_core_inputs(B, D, N, L, seed=3, variant=variant)
+    names = ("u", "delta", "A", "Bm", "Cm") if variant == "real" else ("u", "delta", "rho", "theta", "Bc", "Cc")
+    low = lambda t: (torch.view_as_real(t).contiguous() if t.is_complex() else t).bfloat16()
+    args = [(low(p[k]) if k in ("u", "delta", "Bm", "Cm", "Bc", "Cc") else p[k]).cuda() for k in names]
+    scan_fn = _scans(variant)[1]
+    with torch.no_grad():
+        scan_fn(*args)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        y = scan_fn(*args)
+        used = torch.cuda.max_memory_allocated() - before
+    copies = 2 * args[-1].numel() * 4
+    assert copies >= 1 << 21 and y.numel() * 4 <= used < y.numel() * 4 + copies // 4
