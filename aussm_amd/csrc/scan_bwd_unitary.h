@@ -136,6 +136,9 @@ __global__ __launch_bounds__(NT) void unitary_bwd_kernel(const UniBwdArgs p) {
     for (int k = 0; k < NW; ++k) { nn[k] = n0 + k < N ? n0 + k : N - 1; a2[k] = 0.f; }
     const size_t e = ((size_t)b * p.ns + p.ns - 1) * D + dc;
     seg_chain<VAR_UNITARY, true, NW>(p.seg + e * N * 2, p.segq + e * 2, -(ptrdiff_t)D * N * 2, -(ptrdiff_t)D * 2, p.ns - 1 - sg, nn, a2, gr, gi);
+#pragma unroll
+    for (int k = 0; k < NW; ++k)
+      if (!dok || n0 + k >= N) { gr[k] = 0.f; gi[k] = 0.f; }    // (those read the last channel's, the last state's)
   }
 
   // ---- staging-side mapping (lanes run along time)

@@ -237,3 +237,36 @@ def test_bf16_calls_allocate_their_results_only(variant):
         used = torch.cuda.max_memory_allocated() - before
     copies = 2 * args[-1].numel() * 4
     assert copies >= 1 << 21 and y.numel() * 4 <= used < y.numel() * 4 + copies // 4
+
+
+# Both configurations of the kernel that serves these calls (states per wavefront / threads), with groups of states that are whole, in
+# part and not there, more channels than a workgroup has; whole and split along the sequence, whose last segment is shorter
+@pytest.mark.parametrize("cfg", [(8, 512), (16, 256)])
+@pytest.mark.parametrize("N,L", [(33, 100), (40, 300), (61, 1001), (64, 512)])
+def test_unitary_gradients_in_bf16_of_more_than_32_states(N, L, cfg):
+    """What the float call on the same values leaves, with the adjoint of the state in and out; du and ddelta rounded once."""
+    from aussm_amd import _lib, scan
+    B, D, ck = 2, 70, 128
+    lib = _lib.load()
+    p = O.make_core_inputs(B, D, N, L, seed=N)
+    lo = lambda t: (torch.view_as_real(t).contiguous() if t.is_complex() else t).bfloat16().cuda()
+    u, delta, Bri, Cri = lo(p["u"]), lo(p["delta"]), lo(p["Bc"]), lo(p["Cc"])
+    theta, dy, Dsk = p["theta"].cuda(), p["dy"].cuda(), p["Dskip"].cuda()
+    dhL = torch.randn(B, D, N, 2, generator=torch.Generator().manual_seed(L)).cuda()
+    assert (lib.aussm_unitary_split_segments(B, D, N, L, ck) > 1) == (L >= 256)
+    aux = scan.unitary_aux(u, N, ck)
+    _, _, hck = scan.unitary_fwd_raw(u, delta, theta, Bri, Cri, Dsk, ck=ck, aux=aux)
+    want = scan.unitary_bwd_raw(dy, dhL, *[t.float() for t in (u, delta)], theta, Bri.float(), Cri.float(), Dsk, hck, ck, want_dh0=True)
+    du, dd = (torch.empty(B, D, L, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    dth, acc = torch.empty(B, D, L, device="cuda"), [torch.zeros(B, N, L, 2, device="cuda") for _ in range(2)]
+    dD, dh0 = torch.zeros(D, device="cuda"), torch.empty(B, D, N, 2, device="cuda")
+    with _lib.options(generic_nw=cfg[0], generic_nt=cfg[1]):
+        _lib.check(lib.aussm_unitary_bwd_aux(
+            *[_lib.ptr(t) for t in (dy, dhL, u, delta, theta, Bri, Cri, Dsk, hck, aux, du, dd, dth, *acc, dD, dh0)],
+            B, D, N, L, ck, _lib.BF16 | 0x100, 1, scan._stream()), "aussm_unitary_bwd_aux")
+    for got, w in ((du, want[0]), (dd, want[1])):
+        tie = float(w.abs().max()) * 2.0 ** -20           # (as in the test of the rounded sums above)
+        assert bool(((got.float() - w).abs() <= w.abs() * 2.0 ** -7 + tie).all())
+        assert float((got != w.bfloat16()).float().mean()) < 1e-2
+    for got, w in zip((dth, *acc, dD, dh0), want[2:]):    # two orders of the same float sums, of which the split adds a few
+        assert float((got - w).norm() / w.norm()) < 2e-5
