@@ -127,8 +127,7 @@ def test_sequence_split_over_workgroups(B, D, N, L, cap):
     the CPU oracle and against the same call with the split switched off."""
     from aussm_amd import scan, _lib
     lib = _lib.load()
-    # the shapes are chosen so that the split happens: its states need room behind the per-(b,d,l) part
-    assert lib.aussm_unitary_aux_floats(B, D, N, L, scan.UNITARY_CK) > B * D * L + 64
+    assert lib.aussm_unitary_split_segments(B, D, N, L, scan.unitary_ck(B, D, N, L)) > 1, "the shape is meant to split"
     p = _inputs(B, D, N, L, 3 + L + D, big_theta=(D == 80))
     g = torch.Generator().manual_seed(9)
     dh = torch.complex(torch.randn(B, D, N, generator=g), torch.randn(B, D, N, generator=g))
@@ -167,7 +166,8 @@ def test_sequence_split_into_unequal_segments(B, D, N, L, cap):
     from aussm_amd import scan, _lib
     ck = scan.unitary_ck(B, D, N, L)
     ns = _lib.load().aussm_unitary_split_segments(B, D, N, L, ck)
-    assert ns > 2 and ns & (ns - 1) or L % (ns * ck) != 0
+    assert ns > 1, "the shape is meant to split"
+    assert ns & (ns - 1) or L % (ns * ck) != 0, "... into segments that halving does not give"
     test_sequence_split_over_workgroups(B, D, N, L, cap)
 
 
