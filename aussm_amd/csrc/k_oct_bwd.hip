@@ -15,11 +15,17 @@ static int oct_bwd_t(const RecBwdArgs& args, hipStream_t s) {
     a.nbase = nbase;
     a.accum = nbase > 0;
     const int left = a.N - nbase, S = left >= BLOCK ? BLOCK / 8 : (left + 7) / 8;
-    auto go = [&](auto sc, auto full) {
+    auto launch = [&](auto sc, auto full, auto ragged) {
       constexpr int S_ = decltype(sc)::value;
-      constexpr bool F = decltype(full)::value;
-      if (a.z) hipLaunchKernelGGL((oct_bwd_kernel<VAR, S_, F, Tin, Tin, true>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((oct_bwd_kernel<VAR, S_, F, Tin, Tin, false>), grid, block, 0, s, a);
+      constexpr bool F = decltype(full)::value, R = decltype(ragged)::value;
+      if (a.z) hipLaunchKernelGGL((oct_bwd_kernel<VAR, S_, F, R, Tin, Tin, true>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((oct_bwd_kernel<VAR, S_, F, R, Tin, Tin, false>), grid, block, 0, s, a);
+    };
+    auto go = [&](auto sc, auto full) {
+      if constexpr (VAR == VAR_REAL) {
+        if (a.ld % 16 == 0) return launch(sc, full, std::false_type{});
+      }
+      launch(sc, full, std::true_type{});
     };
     using std::integral_constant;
     if (S == 1) go(integral_constant<int, 1>{}, std::false_type{});
@@ -52,7 +58,8 @@ static int oct_ubwd_t(const RecBwdArgs& args, hipStream_t s) {
     auto go = [&](auto sc, auto full) {
       constexpr int S = decltype(sc)::value;
       constexpr bool F = decltype(full)::value;
-      hipLaunchKernelGGL((oct_bwd_kernel<VAR_UNITARY, S, F, Tin, Tin, false>), grid, block, 0, s, a);
+      if (a.ld % 16 == 0) hipLaunchKernelGGL((oct_bwd_kernel<VAR_UNITARY, S, F, false, Tin, Tin, false>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((oct_bwd_kernel<VAR_UNITARY, S, F, true, Tin, Tin, false>), grid, block, 0, s, a);
     };
     using std::integral_constant;
     const int left = a.N - nbase, S = (left + 7) / 8;

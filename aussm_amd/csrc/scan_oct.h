@@ -750,14 +750,18 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
 //     dtheta_l = -sum_n Im(conj(g_l) p_l),  p_l = h_l - B_l w_l.
 // 30 vector instructions per state and step, no states kept; B5 D200 N24 L1001 85 -> 68 us.
 // States nbase .. nbase + 8 S - 1 (RecBwdArgs).
+// RAGGED: the sequence may end inside an interval, whose steps past the end the walk then leaves out.  Real and unitary, that walk is
+// a second copy of the code with 5 to 20 registers more, so lengths that are a multiple of 16 have an instance without it: in one
+// instance for all, S6 gated, 32 x 512 x 16, 720 steps 290.5 -> 292.7 us; apart 290.5, and 8 x 256 x 16, 1001 steps (unitary) 96.7 -> 98.3.
 //
 // Time is cut into intervals of OH steps (16, or 8 where the slabs of more than 16 complex states need the room) with one barrier each; 32 steps are staged at a time, at the end of every other
 // interval.  (Tiles 16 steps apart in the two wavefronts of a SIMD, so that one computes while the other stages: no faster, and
 // a third more HBM reads where a tile no longer starts on a 128-byte line.)
-template <int VAR, int S, bool FULLN, typename Tin, typename Tbc, bool GATED>
+template <int VAR, int S, bool FULLN, bool RAGGED, typename Tin, typename Tbc, bool GATED>
 __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
   constexpr int C = VAR == VAR_REAL ? 1 : 2;
   constexpr bool UNI = VAR == VAR_UNITARY;
+  constexpr bool WALK_TAIL = RAGGED && VAR != VAR_COMPLEX;   // (complex: what passes by stays in its step)
   constexpr int OH = UNI && S > 2 ? 8 : 16;
   static_assert(!(UNI && GATED), "the unitary scan's gate has kernels of its own");
   // planes [channel][step] of a wavefront: what the steps read - real (delta, w, dy), complex (Re a, Im a, w, dy) -, the
@@ -1041,8 +1045,10 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
       }
     }
   };
-  // walk back over those steps; the sums over the channels go to slab `buf`
-  auto walk = [&](int t0, const float* __restrict__ bc, int buf) {
+  // walk back over those steps; the sums over the channels go to slab `buf`.  TAIL: steps past the end are left out (their
+  // zeros times an infinite last state would be NaN)
+  auto walk = [&](int lh, int t0, const float* __restrict__ bc, int buf, auto tail_tag) {
+    constexpr bool TAIL = decltype(tail_tag)::value;
     float* __restrict__ slab = &s_slab[buf][wave][0];
     // the step of a group whose sums the lane holds (four at a time: two lanes hold, and write, the same)
     const int cs_ = G == 8 ? c : c >> 1, gs_ = G == 8 ? g : g >> 1;
@@ -1065,6 +1071,10 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
 #pragma unroll
         for (int t = G - 1; t >= 0; --t) {
           const int tt = qq * G + t;
+          if (TAIL && lh + tt >= L) {                        // uniform
+            vb_r[t] = vb_i[t] = vc_r[t] = vc_i[t] = 0.f;
+            continue;
+          }
           const float wt = seen(x.w[t], s), gy = seen(x.gy[t], s);
           const bool mine = s < S - 1 || has_last;
           const float hpr = !UNI && tt > 0 ? hsr[!UNI && tt > 0 ? tt - 1 : 0][s] : st.r[s];
@@ -1273,7 +1283,8 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
         else recompute(lh, t0, bc, std::true_type{});
       }
       if (j < last) flush((j + 1) & 1, lh + OH);
-      walk(t0, bc, j & 1);
+      if (!WALK_TAIL || lh + OH <= L) walk(lh, t0, bc, j & 1, std::false_type{});
+      else walk(lh, t0, bc, j & 1, std::integral_constant<bool, WALK_TAIL>{});
       if constexpr (UNI) {
         // a checkpoint: its state instead of the one run back to (plain loads, once per block)
         if (lh > 0 && lh % p.ck == 0) {

@@ -270,3 +270,21 @@ def test_unitary_gradients_in_bf16_of_more_than_32_states(N, L, cfg):
         assert float((got != w.bfloat16()).float().mean()) < 1e-2
     for got, w in zip((dth, *acc, dD, dh0), want[2:]):    # two orders of the same float sums, of which the split adds a few
         assert float((got - w).norm() / w.norm()) < 2e-5
+
+
+@pytest.mark.parametrize("variant,N", [("real", 16), ("real", 19), ("complex", 16), ("unitary", 24), ("unitary", 19)])
+@pytest.mark.parametrize("L", [41, 290])
+def test_an_infinity_in_the_last_step(variant, N, L):
+    """Steps past the end, which the last tile is filled up with, do not take 0 times the state that the sequence ends in: the decay
+    rates' gradient is finite, as the loop's, and C's is an infinity at that step alone."""
+    p, names = _infinite(variant, N, L, "u", L - 1)
+    loop, scan_fn = _scans(variant)
+    got = _gradients(scan_fn, p, names, "cuda", torch.float32)
+    if variant == "real":
+        want = _gradients(loop, p, names, "cpu", torch.float32)
+        for k in ("u", "A", "Bm", "Cm"):
+            assert torch.equal(torch.isnan(got[k]), torch.isnan(want[k])) and torch.equal(torch.isinf(got[k]), torch.isinf(want[k])), k
+        assert bool(torch.isfinite(want["A"]).all())
+    else:
+        dC = torch.view_as_real(got["Cc"])[1]             # (complex products of the loop make NaN of an infinity and a zero part)
+        assert bool(torch.isinf(dC[:, L - 1]).all())
