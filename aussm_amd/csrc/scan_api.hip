@@ -57,8 +57,12 @@ inline bool misaligned(const void* p, size_t a) { return p && (reinterpret_cast<
 // AUSSM_OPT_UNITARY_BWD: 0 vector ALU, 2 two pieces everywhere, 3 three pieces along the sequence
 // and two in the sums over the channel (dB, dC), 5 three pieces everywhere, 6 prepared operands.
 //
-// The matrix-core kernels cost the same for every N <= 16 while the vector-ALU ones scale with N:
-// measured, the crossover is between N = 4 (vector ALU 15 % faster) and N = 8 (matrix 30 % faster).
+// By time alone the matrix-core kernels would take every N: us, vector ALU / matrix cores, forward and backward pass and forward
+// alone, 32 x 512 channels of 2048 steps: N = 2 591 / 526, 194 / 161; 4 595 / 535, 197 / 160; 6 603 / 546, 197 / 161; 8 603 / 553,
+// 193 / 164; 8 x 256 of 1024: N = 4 97 / 90, 26.2 / 24.4; 8 96 / 93, 26.0 / 25.4.  But they take the channel sums behind dB and dC
+// in two pieces, 4.6e-6 of their norm from a float64 scan where the vector ALU's are 1.1e-6 (2 x 64 x 4, 2048 steps; the other
+// results agree to 20 %), so calls of fewer states, which the vector ALU has always served, stay there.  (The line is where the two
+// took the same time when it was drawn.)
 constexpr int MATRIX_MIN_STATE = 6;
 constexpr int DEFAULT_FWD_MODE = 6, DEFAULT_BWD_MODE = 6;   // (6 falls back to 3 where the call brings no workspace)
 inline int kernel_mode(int key, int dflt, int N) {
@@ -68,9 +72,10 @@ inline int kernel_mode(int key, int dflt, int N) {
 }
 // Splitting the sequence (scan_seg_xdl.h): with few (batch, channel group) pairs the launch would
 // leave most of the chip idle, so the sequence is cut into ns segments of whole checkpoint blocks
-// until about one workgroup per compute unit exists.  Only the matrix-core kernels take part,
-// and only the *_aux entry points (the segment states live behind the auxiliary buffer).
-// aussm_set_option(AUSSM_OPT_SPLIT_CAP, c): 0 or 1 switches it off, a power of two caps ns.
+// until about one workgroup per compute unit exists: here in equal ones by halving, below in others (unitary_split), on the
+// vector-ALU kernels by generic_split.  The segment states live behind the auxiliary buffer or in the call's workspace;
+// aussm_unitary_fwd_static has room for equal segments only.
+// aussm_set_option(AUSSM_OPT_SPLIT_CAP, c): 0 or 1 switches it off, more caps ns.
 constexpr int SPLIT_MIN_WGS = 129;     // launches of at least this many workgroups are left alone
 constexpr int SPLIT_TARGET_WGS = 256;
 constexpr int SPLIT_MAX = 32;
@@ -873,7 +878,9 @@ static int dropin_fwd_chunk_tiles(int b, int d, int L, bool largest = false) {
 // in one sweep, 23 and 6 for the maps in four segments; 3 x 200: 30 in three segments, 39 in six), but at least two tiles each.
 // The maps cost a third to a half of a sweep: two segments gain nothing (16 x 64 pairs, backward: 80 us, 60 and 22 in two), three
 // do (3 x 200, 500 steps: 87, 46 and 25), and under 16 tiles their launch eats the rest (2 x 32 pairs, 7 tiles: 39 us both ways, 47
-// in segments; 8 x 8, 16 tiles: 62, 49).
+// in segments; 8 x 8, 16 tiles: 62, 49).  Those are kernels; whole passes, in one sweep / in segments, of 16 tiles: forward 8 x 16 22.6 /
+// 15.1 us, 4 x 128 31.3 / 21.6, 16 x 64 28.0 / 25.7, but 3 x 200 41.0 / 42.0 (25 tiles of it: 55.5 / 52.5); with the gradients, where
+// the host's launches set the time, 8 x 16 113-115 / 121, 2 x 32, 19 tiles 111-115 / 119-121, 31 tiles 117-122 / 119.
 static int dropin_segment_tiles(int bg, int d, int n, int nt, bool backward) {
   const int nw = dropin_channels_per_workgroup((d + 31) / 32);
   const long wgs = (long)bg * ((d * dropin_state_blocks(n) + nw - 1) / nw);

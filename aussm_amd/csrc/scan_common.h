@@ -70,8 +70,8 @@ __device__ __forceinline__ float softplusf_(float v) {
 }
 
 // sin and cos of one argument, about 25 VALU instructions and no branch on the common path.
-// Cody-Waite reduction by pi/2 in three fused steps, then minimax polynomials on [-pi/4, pi/4]
-// (max error ~1 ulp of 1.0 for |x| < 1e4, which covers accumulated phases of practical length).
+// Cody-Waite reduction by pi/2 in three fused steps, then the minimax polynomials on [-pi/4, pi/4] of sinf and cosf in
+// S. L. Moshier's Cephes library (max error ~1 ulp of 1.0 for |x| < 1e4, which covers accumulated phases of practical length).
 // Larger arguments take the library routine (fast_sincosf; sincos_1e4 leaves the check to its caller).
 __device__ __forceinline__ void sincos_1e4(float x, float* sn, float* cs) {
   const float kf = rintf(x * 0.636619772367581343f);

@@ -754,7 +754,7 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
 // a second copy of the code with 5 to 20 registers more, so lengths that are a multiple of 16 have an instance without it: in one
 // instance for all, S6 gated, 32 x 512 x 16, 720 steps 290.5 -> 292.7 us; apart 290.5, and 8 x 256 x 16, 1001 steps (unitary) 96.7 -> 98.3.
 //
-// Time is cut into intervals of OH steps (16, or 8 where the slabs of more than 16 complex states need the room) with one barrier each; 32 steps are staged at a time, at the end of every other
+// Time is cut into intervals of OH steps (16, or 8 where the slabs of the unitary scan's 24 and 32 states need the room) with one barrier each; 32 steps are staged at a time, at the end of every other
 // interval.  (Tiles 16 steps apart in the two wavefronts of a SIMD, so that one computes while the other stages: no faster, and
 // a third more HBM reads where a tile no longer starts on a 128-byte line.)
 template <int VAR, int S, bool FULLN, bool RAGGED, typename Tin, typename Tbc, bool GATED>

@@ -22,7 +22,7 @@ resident in HBM.  Prints ONE JSON line.
                  --copy-probe adds to the run.  It is read from profiles/traffic.json, which
                  `bench.py --summarize-traffic FETCH_DIR WRITE_DIR` writes from the two passes'
                  output; the file records the kernels it saw and a digest of the kernel sources,
-                 and the figure is reported as null when either no longer matches this build.
+                 and the figure is reported as null when either no longer matches the library.
   cpu_baseline   the CPU oracle (sequential-loop PyTorch scan + autograd) timed on this host's
                  cores on a bounded slice of the batch: one warm-up run, then the median of three
 
@@ -101,7 +101,7 @@ def summarize_traffic(fetch_dir: str, write_dir: str) -> None:
 
 def recorded_traffic(kernel_substrings):
     """(bytes per call, note): sum over the named kernels of read + written bytes in profiles/traffic.json, or
-    (None, why) when the record does not cover this build or these kernels."""
+    (None, why) when the record does not cover the library's sources or these kernels."""
     if not os.path.exists(TRAFFIC_JSON):
         return None, "profiles/traffic.json missing"
     rec = json.load(open(TRAFFIC_JSON))
@@ -209,7 +209,7 @@ def main():
         summarize_traffic(*args.summarize_traffic)
         return
     if args.gpus != 1:
-        print("bench.py: this build runs on ONE GPU; --gpus must be 1 (no multi-GPU path exists)", file=sys.stderr)
+        print("bench.py runs on ONE GPU; --gpus must be 1 (no multi-GPU path exists)", file=sys.stderr)
         sys.exit(2)
 
     import torch
@@ -321,8 +321,7 @@ def main():
         "vs_baseline": None,
         "dtype": "f32",
         "data": "synthetic",
-        "config": {"workload": (f"unitary core scan fwd+bwd, B={B} D={D} N={N} L={L}, fp32"
-                                + (" (BASELINE configs[3], unitary, fp32)" if headline else "")),
+        "config": {"workload": f"unitary core scan fwd+bwd, B={B} D={D} N={N} L={L}, fp32",
                    "B": B, "D": D, "N": N, "L": L, "checkpoint_interval": ck},
         "state_updates_per_s": B * D * N * L / dt,
         "fwd_bwd_algorithmic_GBps": (bytes_fwd + bytes_bwd) / ((t_fwd + t_bwd) * 1e-6) / 1e9,

@@ -250,7 +250,8 @@ int aussm_complex_fwd(const void* u, const void* delta, const float* rho, const 
 
 /* z / dz of the two backward calls below (both NULL, or both given): the forward call was gated with this z
  * (y = y_pre silu(z)); dy is then the gradient of the gated y, the kernel applies the gate's derivative
- * itself and writes dz = dy y_pre silu'(z).  N <= 64 (one launch per block of 16 states). */
+ * itself and writes dz = dy y_pre silu'(z).  N <= 64 (one launch per block of 16 states here,
+ * of 24 in the real scan). */
 int aussm_complex_bwd(const float* dy, const float* dhL,
                       const void* u, const void* delta, const float* rho, const float* theta,
                       const void* Bc, const void* Cc, const float* Dskip,
