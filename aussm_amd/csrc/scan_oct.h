@@ -752,7 +752,8 @@ __global__ __launch_bounds__(512) void oct_adj_kernel(const AdjSegArgs p) {
 // States nbase .. nbase + 8 S - 1 (RecBwdArgs).
 // RAGGED: the sequence may end inside an interval, whose steps past the end the walk then leaves out.  Real and unitary, that walk is
 // a second copy of the code with 5 to 20 registers more, so lengths that are a multiple of 16 have an instance without it: in one
-// instance for all, S6 gated, 32 x 512 x 16, 720 steps 290.5 -> 292.7 us; apart 290.5, and 8 x 256 x 16, 1001 steps (unitary) 96.7 -> 98.3.
+// instance for all, S6 gated, 32 x 512 x 16, 720 steps 290.5 -> 292.7 us; apart 290.5, and 8 x 256 x 16, 1001 steps (unitary) 96.7 -> 98.3,
+// 32 x 512 x 24, 721 steps (S6 gated, where it costs two spilled registers) 389.8 -> 400.1.
 //
 // Time is cut into intervals of OH steps (16, or 8 where the slabs of the unitary scan's 24 and 32 states need the room) with one barrier each; 32 steps are staged at a time, at the end of every other
 // interval.  (Tiles 16 steps apart in the two wavefronts of a SIMD, so that one computes while the other stages: no faster, and
