@@ -505,7 +505,7 @@ int aussm_real_fwd(const void* u, const void* delta, const float* A, const void*
                              in_dtype, stream);
 }
 
-// (rows of wider tensors: float inputs only, whose B_t / C_t are not copied on the way)
+// (B_t / C_t as rows of wider tensors: float inputs only, as the Mamba block calls it; bf16 ones have never been taken)
 static int real_rows_check(const aussm_real_rows* r, int D, int N, int in_dtype) {
   if (!r) return AUSSM_OK;
   if ((r->z_rows && r->z_rows < D) || (r->bc_rows && r->bc_rows < N)) return AUSSM_E_SHAPE;
@@ -670,7 +670,7 @@ int aussm_real_bwd_rows(const float* dy, const float* dhL, const void* u, const 
   }
   a.z = z; a.dz = dz;
   a.B = B; a.D = D; a.N = N; a.L = L; a.ck = ck; a.nck = (L + ck - 1) / ck; a.ncg = (D + CH - 1) / CH;
-  // (several blocks of states add up in du and ddelta: those stay float)
+  // (several launches add up in du and ddelta: those stay float, 17 to 24 states, which one launch holds here, like more)
   if (g16 && in_dtype == AUSSM_BF16 && N > 16) return AUSSM_E_DTYPE;
   a.g16 = g16 && in_dtype == AUSSM_BF16;
   a.ld = L; a.ns = 1;

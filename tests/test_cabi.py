@@ -125,7 +125,7 @@ def test_argument_checks_without_a_device():
     assert lib.aussm_scan_workspace_floats(0, 4, 256, 16, 16384, 16, 0) == 0       # the unitary scan has its own
     assert lib.aussm_scan_workspace_floats(2, 4, 256, 16, 16384, 16, 0) >= 4 * 16 * 256 * 18
     assert lib.aussm_scan_workspace_floats(1, 4, 256, 16, 16384, 16, 0) >= 4 * 16 * 256 * 34
-    # bf16 inputs: float copies of B_t and C_t, and no call without the workspace that holds them
+    # bf16 inputs: the size has room for float copies of B_t and C_t, and no call goes without a workspace
     assert lib.aussm_scan_workspace_floats(1, 32, 512, 16, 2048, 16, 1) == 2 * 32 * 16 * 2048 * 2
     assert lib.aussm_real_bwd(*args, 1, 1, 1, 32, 16, 1, null) == -1
     # the blocks' causal convolution: kernel length limit, overlapping rows, required pointers
