@@ -10,8 +10,8 @@
 // A wavefront owns one (batch, channel) pair - with more than 16 states per channel, one block of 16
 // states of it - and walks the sequence in tiles of 16 timesteps:
 //   * the tile's RUNNING phases G = prefix(theta), a (16 states) x (16 timesteps) block, are one small matrix
-//     product x[i] (16 x d) . U (d x 16) on the bf16 matrix cores with both operands split exactly into
-//     three bf16 pieces (scan_fwd_xdl.h), i.e. fp32-accurate, where U is the tile of u[b] prefix-summed along
+//     product x[i] (16 x d) . U (d x 16) on the 16-bit matrix cores with both operands split, fp32-accurate
+//     (Phase below), where U is the tile of u[b] prefix-summed along
 //     the tile (sum_{l' <= l} x.u_{l'} = x.U_l), plus (l + 1) x_bias.  The wavefront keeps its rows of x in
 //     registers for the whole launch; the tiles of U, which all wavefronts of a batch element share, are
 //     prepared once per call by a pre-pass (dropin_prep_kernel) and copied into LDS once per workgroup;
@@ -25,9 +25,55 @@
 #pragma once
 #include "dropin_args.h"
 #include "scan_fwd_xdl.h"
+#include "split_half.h"
 
 namespace aussm {
 
+// How the operands of the phase product are split, by the steps of 32 that the contraction takes.  Up to two (d <= 64) three bf16
+// pieces and six partial products (scan_fwd_xdl.h); from three on two f16 pieces and three partial products (split_half.h), the
+// rows of x and the columns of U scaled by powers of two of their own: half the matrix instructions, which no vector instruction
+// of the other wavefronts hides.  Two accumulators, the pieces' product and the mixed ones: 2^11 apart, and two chains of matrix
+// instructions instead of one.  Relative error of sums of N(0, 1) products against 64 bits, six bf16 / three f16 products: 32 terms
+// 3.8e-8 / 9.1e-8, 64 9.3e-8 / 9.8e-8, 128 1.53e-7 / 1.11e-7, 256 2.3e-7 / 1.3e-7, 512 3.4e-7 / 1.7e-7 - hence where the line lies.
+// Records: [step][piece][64 lanes], behind them (f16) the exponent of each of the 16 rows or columns.
+template <int KS>
+struct Phase {
+  static constexpr bool HALF = KS >= PHASE_HALF_KS;
+  static constexpr int NP = HALF ? 2 : 3, REC = KS * NP * 64, TILE = REC + (HALF ? 4 : 0);   // 16-byte records of a tile of U
+  f4 hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
+  __device__ __forceinline__ void step(const u4 (&x)[NP], const u4* __restrict__ s, int lane) {
+    u4 v[NP];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) v[q] = s[q * 64 + lane];
+    if constexpr (HALF) {
+      hi = xdl_half(x[0], v[0], hi);
+      lo = xdl_half(x[1], v[0], lo);
+      lo = xdl_half(x[0], v[1], lo);
+    } else {
+      hi = xmm<3>(x, v, hi);
+    }
+  }
+  // exponents e of the row and of the column together
+  __device__ __forceinline__ float value(int a, int e) const {
+    return HALF ? __builtin_amdgcn_ldexpf(fmaf(lo[a], HALF_LO_INV, hi[a]), e) : hi[a];
+  }
+};
+// the exponents of the columns of tile t
+template <int KS>
+__device__ __forceinline__ const int* phase_columns(const u4* __restrict__ upb, int t) {
+  return reinterpret_cast<const int*>(upb + (size_t)t * Phase<KS>::TILE + Phase<KS>::REC);
+}
+// the rows of x of (channel, state block) vc, ks steps of them, into registers; what stands behind them
+template <int KS>
+__device__ __forceinline__ const int* phase_rows(const u4* __restrict__ xp, int ks, int vc, int lane, u4 (&xa)[KS][Phase<KS>::NP]) {
+  constexpr int NP = Phase<KS>::NP;
+  const u4* const r = xp + (size_t)vc * (ks * NP * 64 + (Phase<KS>::HALF ? 4 : 0));
+#pragma unroll
+  for (int k = 0; k < KS; ++k)
+#pragma unroll
+    for (int q = 0; q < NP; ++q) xa[k][q] = k < ks ? r[(k * NP + q) * 64 + lane] : u4{0, 0, 0, 0};
+  return reinterpret_cast<const int*>(r + ks * NP * 64);
+}
 
 // sin and cos of any argument without a branch: reduction by 2 pi in two fused steps (the result is as exact
 // as the fp32 argument itself), then the hardware sine and cosine of the reduced argument (sincos_small_hw).  A
@@ -105,89 +151,117 @@ __device__ __forceinline__ float row_last(float v, int) { return dpp_perm<0x15F>
 __device__ __forceinline__ float row_first(float v, int) { return dpp_perm<0x150>(v); }   // row_newbcast:0
 
 
-// x (rows of d: (channel i, state j) at row i xsi + j xsj), times scale -> operand records.  Record (v = i nb + sb, ks, piece, lane = (row = lane % 16, g = lane / 16))
-// holds x[i, 16 sb + row, 32 ks + 8 g .. + 7] (zero past the ends).  One thread per (v, ks, lane).
+// Operand records of 16 rows (or columns) of ks steps of 32, by a workgroup of 256 threads: v(k, lane, out) gives the eight values of lane
+// (row = lane % 16, g = lane / 16) of step k, terms 32 k + 8 g .. + 7.  A row is scaled by one power of two, found from its largest
+// value first: a thread keeps its records of up to 512 terms between the two passes.
+template <typename Values>
+__device__ __forceinline__ void phase_records(Values&& values, int ks, bool half, u4* __restrict__ dst) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (!half) {
+    const SplitK sk = make_splitk();
+    for (int k = wave; k < ks; k += 4) {
+      float v[8];
+      values(k, lane, v);
+      u4 pc[3];
+      split8<3>(sk, v, pc);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) dst[(k * 3 + q) * 64 + lane] = pc[q];
+    }
+    return;
+  }
+  __shared__ float s_most[4][16];
+  constexpr int R = D_MAXKS / 4;
+  float v[R][8], most = 0.0f;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (wave + 4 * r < ks) values(wave + 4 * r, lane, v[r]);
+    else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[r][q] = 0.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) most = fmaxf(most, fabsf(v[r][q]));
+  }
+  most = rows_max(most);
+  if (lane < 16) s_most[wave][lane] = most;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) most = fmaxf(most, s_most[w][lane & 15]);
+  const int e = half_exponent(most);
+  if (threadIdx.x < 16) reinterpret_cast<int*>(dst + ks * 2 * 64)[threadIdx.x] = -e;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = wave + 4 * r;
+    if (k >= ks) break;
+    u4 pc[2];
+    split8_half<true>(v[r], exp2_of(e), pc);
+    dst[(k * 2) * 64 + lane] = pc[0];
+    dst[(k * 2 + 1) * 64 + lane] = pc[1];
+  }
+}
+
+// x (rows of d: (channel i, state j) at row i xsi + j xsj), times scale -> operand records of (channel, state block) v = i nb + sb: row j - 16 sb.
 // x_out [d, n, d], xb_out [d, n] (or null): scale x and x_bias in the operator's own order, for a caller that keeps them.
-__device__ __forceinline__ void xprep_block(const DropinPrepArgs& a, unsigned block) {
-  const int d = a.d, n = a.n, ks = a.ks, nb = a.nb, xsi = a.xsi, xsj = a.xsj;
+__device__ __forceinline__ void xprep_block(const DropinPrepArgs& a, unsigned vc) {
+  const int d = a.d, n = a.n, nb = a.nb, xsi = a.xsi, xsj = a.xsj;
   const float scale = a.scale;
   const float* __restrict__ x = a.x;
   float* __restrict__ x_out = a.x_out;
-  u4* __restrict__ xp = a.xp;
-  const size_t idx = (size_t)block * 256 + threadIdx.x;
-  if (idx >= (size_t)d * nb * ks * 64) return;
-  const int lane = (int)(idx & 63);
-  const int k = (int)((idx >> 6) % ks), vc = (int)((idx >> 6) / ks);
-  const int i = vc / nb, j = 16 * (vc % nb) + (lane & 15), g = lane >> 4;
-  const SplitK sk = make_splitk();
-  float v[8];
+  const int i = vc / nb, jb = 16 * (vc % nb);
+  auto values = [&](int k, int lane, float (&v)[8]) {
+    const int j = jb + (lane & 15), r0 = 32 * k + 8 * (lane >> 4);
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int r = 32 * k + 8 * g + q;
-    v[q] = (j < n && r < d) ? x[((size_t)i * xsi + (size_t)j * xsj) * d + r] * scale : 0.0f;
-  }
-  const int r0 = 32 * k + 8 * g;
-  if (x_out && j < n) {
-    float* const o = x_out + ((size_t)i * n + j) * d + r0;
-    if (r0 + 8 <= d) {
-      *reinterpret_cast<f4u*>(o) = f4u{v[0], v[1], v[2], v[3]};
-      *reinterpret_cast<f4u*>(o + 4) = f4u{v[4], v[5], v[6], v[7]};
-    } else {
+    for (int q = 0; q < 8; ++q) v[q] = (j < n && r0 + q < d) ? x[((size_t)i * xsi + (size_t)j * xsj) * d + r0 + q] * scale : 0.0f;
+    if (x_out && j < n) {
+      float* const o = x_out + ((size_t)i * n + j) * d + r0;
+      if (r0 + 8 <= d) {
+        *reinterpret_cast<f4u*>(o) = f4u{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f4u*>(o + 4) = f4u{v[4], v[5], v[6], v[7]};
+      } else {
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
-        if (r0 + q < d) o[q] = v[q];
+        for (int q = 0; q < 8; ++q)
+          if (r0 + q < d) o[q] = v[q];
+      }
     }
-  }
-  if (a.xb_out && j < n && k == 0 && g == 0) a.xb_out[(size_t)i * n + j] = a.x_bias[(size_t)i * xsi + (size_t)j * xsj];
-  u4 pc[3];
-  split8<3>(sk, v, pc);
-#pragma unroll
-  for (int q = 0; q < 3; ++q) xp[(((size_t)vc * ks + k) * 3 + q) * 64 + lane] = pc[q];
+    if (a.xb_out && j < n && r0 == 0) a.xb_out[(size_t)i * n + j] = a.x_bias[(size_t)i * xsi + (size_t)j * xsj];
+  };
+  const bool half = a.KS >= PHASE_HALF_KS;
+  phase_records(values, a.ks, half, a.xp + (size_t)vc * (a.ks * (half ? 2 : 3) * 64 + (half ? 4 : 0)));
 }
 
-// Tiles of u as the second operand of the phase product, one workgroup of 256 threads per (batch element, tile): record (k, piece, lane = (column l = lane % 16, g)) holds
-// U[32 k + 8 g .. + 7][l], U[r][l] = sum_{l' <= l} u[b, r, l0 + l'] - the prefix sum along the tile - so that
+// Tiles of u as the second operand of the phase product, one workgroup per (batch element, tile): column l holds U[r][l],
+// U[r][l] = sum_{l' <= l} u[b, r, l0 + l'] - the prefix sum along the tile - so that
 // the matrix product hands the scan kernels the running phase G = prefix(theta) directly
 // (sum_{l' <= l} sum_r x[i,j,r] u[r,l'] = sum_r x[i,j,r] U[r,l]); timesteps past L count as zero.  All KS steps the
 // kernels are compiled for are written, the ones past ceil(d / 32) as zeros.
 __device__ __forceinline__ void uprep_block(const DropinPrepArgs& a, unsigned block) {
-  const int d = a.d, L = a.L, KS = a.KS;
-  const int zb = block / a.nt, t = a.t0 + block % a.nt;
-  const float* __restrict__ ub = a.u + (size_t)(a.b0 + zb) * d * L;
-  u4* __restrict__ dst = a.up + (size_t)block * KS * 3 * 64;
-  const SplitK sk = make_splitk();
-  for (int rec = threadIdx.x; rec < KS * 64; rec += 256) {        // (whole wavefronts: 64 records per k)
-    const int lane = rec & 63, k = rec >> 6;
-    const int l = t * DT + (lane & 15), g = lane >> 4;
-    float v[8];
+  const int d = a.d, L = a.L, t = a.t0 + block % a.nt;
+  const float* __restrict__ ub = a.u + (size_t)(a.b0 + block / a.nt) * d * L;
+  auto values = [&](int k, int lane, float (&v)[8]) {
+    const int l = t * DT + (lane & 15), r0 = 32 * k + 8 * (lane >> 4);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int r = 32 * k + 8 * g + q;
-      v[q] = row_prefix((r < d && l < L) ? ub[(size_t)r * L + l] : 0.0f);
-    }
-    u4 pc[3];
-    split8<3>(sk, v, pc);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) dst[(k * 3 + q) * 64 + lane] = pc[q];
-  }
+    for (int q = 0; q < 8; ++q) v[q] = row_prefix((r0 + q < d && l < L) ? ub[(size_t)(r0 + q) * L + l] : 0.0f);
+  };
+  const bool half = a.KS >= PHASE_HALF_KS;
+  phase_records(values, a.KS, half, a.up + (size_t)block * (a.KS * (half ? 2 : 3) * 64 + (half ? 4 : 0)));
 }
 
 // A tile's records, global memory -> registers -> LDS, in two steps so that the loads of the next tile fly
 // while the current one is computed.
-template <int NT, int NREC, int KS>
+template <int NT, int NREC, int REC>
 __device__ __forceinline__ void tile_load(const u4* __restrict__ src, u4 (&v)[NREC], int tid) {
 #pragma unroll
   for (int e = 0; e < NREC; ++e) {
     const int rec = tid + e * NT;
-    if (rec < KS * 3 * 64) v[e] = src[rec];
+    if (rec < REC) v[e] = src[rec];
   }
 }
-template <int NT, int NREC, int KS>
+template <int NT, int NREC, int REC>
 __device__ __forceinline__ void tile_store(const u4 (&v)[NREC], u4* __restrict__ dst, int tid) {
 #pragma unroll
   for (int e = 0; e < NREC; ++e) {
     const int rec = tid + e * NT;
-    if (rec < KS * 3 * 64) dst[rec] = v[e];
+    if (rec < REC) dst[rec] = v[e];
   }
 }
 
@@ -251,7 +325,8 @@ __device__ __forceinline__ void seg_enter_row(const f4* __restrict__ mp, const f
 // of 256 pairs and 512 steps 7 us in segments of two tiles (forward) and 9 of four (backward), before scans of 9.7 and 28 us.
 template <int KS, int NW, bool BWD>
 __global__ __launch_bounds__(NW * 64) void dropin_seg_kernel(const DropinBwdArgs q) {
-  __shared__ u4 s_u[2][KS * 3 * 64];
+  typedef Phase<KS> P;
+  __shared__ u4 s_u[2][P::REC];
   __shared__ f4 s_par[D_MAXN];
   const DropinArgs& p = q.f;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
@@ -264,31 +339,31 @@ __global__ __launch_bounds__(NW * 64) void dropin_seg_kernel(const DropinBwdArgs
   const int l_ = lane & 15, g = lane >> 4;
   const int d = p.d, n = p.n, L = p.L;
   const size_t row = ((size_t)b * d + ic) * L, zrow = (size_t)b * p.zs + (size_t)ic * L;
-  const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * (KS * 3 * 64);   // + tile * (KS 3 64)
+  const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * P::TILE;   // + tile * TILE
   const int tb = q.t0 + sg * p.sl, te = min(tb + p.sl, q.t1);
 
-  u4 xa[KS][3];
-#pragma unroll
-  for (int k = 0; k < KS; ++k)
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-      xa[k][c] = (k < p.ks) ? p.xp[(((size_t)vc * p.ks + k) * 3 + c) * 64 + lane] : u4{0, 0, 0, 0};
+  u4 xa[KS][P::NP];
+  const int* const xe = phase_rows<KS>(p.xp, p.ks, vc, lane, xa);
   float xb[4], Qr[4], Qi[4], Sr[4], Si[4], Tr[4], Ti[4];
+  int ex[4];
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
     const int j = j0 + 4 * g + a;
     xb[a] = j < n ? p.x_bias[(size_t)ic * p.xsi + (size_t)j * p.xsj] : 0.0f;
+    ex[a] = P::HALF ? xe[4 * g + a] : 0;
     Qr[a] = 1.0f;
     Qi[a] = Sr[a] = Si[a] = Tr[a] = Ti[a] = 0.0f;
   }
-  constexpr int NT = NW * 64, NREC = (KS * 3 * 64 + NT - 1) / NT;
+  constexpr int NT = NW * 64, NREC = (P::REC + NT - 1) / NT;
   u4 sv[NREC];
-  tile_load<NT, NREC, KS>(upb + (size_t)tb * (KS * 3 * 64), sv, tid);
-  tile_store<NT, NREC, KS>(sv, s_u[tb & 1], tid);
+  tile_load<NT, NREC, P::REC>(upb + (size_t)tb * P::TILE, sv, tid);
+  tile_store<NT, NREC, P::REC>(sv, s_u[tb & 1], tid);
   polar_params<false>(p, s_par, nullptr, tid);
   __syncthreads();
   float un = 0.0f, dtn = 0.0f, zn = 0.0f, gyn = 0.0f;
+  int en = 0;                                          // exponent of the tile's column
   auto inputs = [&](int l) {                           // a tile ahead; steps past the end count as zero
+    if (P::HALF) en = phase_columns<KS>(upb, l / DT)[l_];
     const bool ok = l < L;
     un = ok ? p.u[row + l] : 0.0f;
     dtn = ok ? p.dt[row + l] : 0.0f;
@@ -301,24 +376,20 @@ __global__ __launch_bounds__(NW * 64) void dropin_seg_kernel(const DropinBwdArgs
   for (int t = tb; t < te; ++t) {
     const int l0 = t * DT;
     const float w = dtn * silu_fast(un), av = BWD ? gyn * silu_fast(zn) : 0.0f;
+    const int eu = en;
     if (t + 1 < te) {
       inputs(l0 + DT + l_);
-      tile_load<NT, NREC, KS>(upb + (size_t)(t + 1) * (KS * 3 * 64), sv, tid);
+      tile_load<NT, NREC, P::REC>(upb + (size_t)(t + 1) * P::TILE, sv, tid);
     }
-    f4 th = {0, 0, 0, 0};
+    P th;
     const u4* su = s_u[t & 1];
 #pragma unroll
-    for (int k = 0; k < KS; ++k) {
-      u4 ubk[3];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) ubk[c] = su[(k * 3 + c) * 64 + lane];
-      th = xmm<3>(xa[k], ubk, th);
-    }
+    for (int k = 0; k < KS; ++k) th.step(xa[k], su + k * P::NP * 64, lane);
     const float cnt = (float)(min(l_ + 1, L - l0));
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       float sn, cs;
-      sincos_any(fmaf(xb[a], cnt, th[a]), &sn, &cs);
+      sincos_any(fmaf(xb[a], cnt, th.value(a, ex[a] + eu)), &sn, &cs);
       const float qr = Qr[a] * cs - Qi[a] * sn, qi = Qr[a] * sn + Qi[a] * cs;
       Sr[a] += w * qr;
       Si[a] -= w * qi;
@@ -329,7 +400,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_seg_kernel(const DropinBwdArgs
       Qr[a] = row_last(qr, lane);
       Qi[a] = row_last(qi, lane);
     }
-    if (t + 1 < te) tile_store<NT, NREC, KS>(sv, s_u[(t + 1) & 1], tid);
+    if (t + 1 < te) tile_store<NT, NREC, P::REC>(sv, s_u[(t + 1) & 1], tid);
     __syncthreads();
   }
 #pragma unroll
@@ -362,13 +433,15 @@ __global__ __launch_bounds__(NW * 64) void dropin_seg_kernel(const DropinBwdArgs
 // Workgroup = (batch b, NW consecutive (channel, state block) pairs), one pair per wavefront; the nb
 // wavefronts of a channel are neighbours (nb divides NW) and add their shares of y through LDS.
 // KS: 32-wide steps of the contraction over r (d <= 32 KS).
-// The tiles of U go straight to LDS up to d = 128 and in workgroups of four: without the registers in between, a workgroup of four wavefronts fits three
-// times on a compute unit at 128 < d (166 registers; the kernel waits more than it works, VALU 50 % with two wavefronts on a
-// SIMD): 32 x 256 x 16, 720 steps 342 -> 304 us, 32 x 180 214 -> 177, and 32 x 64 in workgroups of eight as before 73 -> 62.
+// The kernel waits more than it works, so it takes the registers of four workgroups of four wavefronts to a compute unit at 128 < d:
+// the tiles of U go straight to LDS (there and up to d = 128, in workgroups of eight), and at d > 192 the polar parameters are read
+// from LDS where they are used.  Whole call of 32 x 256 x 16, 720 steps: 339 us with three bf16 pieces and three workgroups, now
+// 234 (249 with three workgroups, 307 in workgroups of eight); 32 x 180 198 -> 167, 32 x 128 107 -> 99.
 // One wavefront on a SIMD (d > 256) or two of wide x gain nothing from it: 8 x 300, 400 steps 109 -> 113, 8 x 250, 720 86 -> 90.
 template <int KS, int NW>
-__global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 3 : 1) void dropin_fwd_kernel(const DropinArgs p) {
-  __shared__ u4 s_u[2][KS * 3 * 64];
+__global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 4 : 1) void dropin_fwd_kernel(const DropinArgs p) {
+  typedef Phase<KS> P;
+  __shared__ u4 s_u[2][P::REC];
   __shared__ f4 s_par[D_MAXN];
   __shared__ float s_y[2][NW][DT];                     // shares of y of the tile, by tile parity (nb > 1)
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
@@ -381,19 +454,15 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 3 : 1) void dropin_fw
   const int l_ = lane & 15, g = lane >> 4;
   const int d = p.d, n = p.n, L = p.L;
   const size_t row = ((size_t)b * d + ic) * L, zrow = (size_t)b * p.zs + (size_t)ic * L;
-  const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * (KS * 3 * 64);   // + tile * (KS 3 64)
+  const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * P::TILE;   // + tile * TILE
   const int tb = p.nseg > 1 ? p.t0 + sg * p.sl : p.t0, ntiles = p.nseg > 1 ? min(tb + p.sl, p.t1) : p.t1;
 
   // this wavefront's rows of x, split, for the whole launch
-  u4 xa[KS][3];
-#pragma unroll
-  for (int k = 0; k < KS; ++k)
-#pragma unroll
-    for (int q = 0; q < 3; ++q)
-      xa[k][q] = (k < p.ks) ? p.xp[(((size_t)vc * p.ks + k) * 3 + q) * 64 + lane] : u4{0, 0, 0, 0};
+  u4 xa[KS][P::NP];
+  const int* const xe = phase_rows<KS>(p.xp, p.ks, vc, lane, xa);
   // per state j = j0 + 4 g + a: bias, Bt, Ct, carried state
-  float xb[4], btr[4], bti[4], ctr[4], cti[4], hr[4], hi[4];
-  int at[4];
+  float xb[4], hr[4], hi[4];
+  int at[4], ex[4];
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
     const int j = j0 + 4 * g + a;
@@ -401,6 +470,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 3 : 1) void dropin_fw
     const int jc = ok ? j : 0;
     const size_t cell_ = ((size_t)(b - p.b0) * d + ic) * n + jc;
     xb[a] = ok ? p.x_bias[(size_t)ic * p.xsi + (size_t)jc * p.xsj] : 0.0f;
+    ex[a] = P::HALF ? xe[4 * g + a] : 0;
     hr[a] = ok && p.h_re ? p.h_re[(size_t)p.b0 * d * n + cell_] : 0.0f;
     hi[a] = ok && p.h_im ? p.h_im[(size_t)p.b0 * d * n + cell_] : 0.0f;
     at[a] = (int)cell_;                                // (of use with segments, where there are few)
@@ -413,68 +483,70 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 3 : 1) void dropin_fw
   }
   const float Di = p.Dp[ic];
 
+  constexpr bool PAR_LDS = NW == 4 && KS == 8;
   constexpr bool DIRECT = KS <= 4 || (KS <= 8 && NW == 4);
-  constexpr int NT = NW * 64, NREC = DIRECT ? 1 : (KS * 3 * 64 + NT - 1) / NT;
+  constexpr int NT = NW * 64, NREC = DIRECT ? 1 : (P::REC + NT - 1) / NT;
   u4 sv[NREC];
   auto fetch = [&](int t) {                            // a tile's records towards s_u[t & 1], directly 1 KiB at a time
-    const u4* __restrict__ src = upb + (size_t)t * (KS * 3 * 64);
+    const u4* __restrict__ src = upb + (size_t)t * P::TILE;
     if constexpr (DIRECT) {
-      for (int c = wave; c < KS * 3; c += NW) px_load_block(src + c * 64, s_u[t & 1] + c * 64, lane);
+      for (int c = wave; c < KS * P::NP; c += NW) px_load_block(src + c * 64, s_u[t & 1] + c * 64, lane);
     } else {
-      tile_load<NT, NREC, KS>(src, sv, tid);
+      tile_load<NT, NREC, P::REC>(src, sv, tid);
     }
   };
   auto landed = [&](int t) {
     if constexpr (DIRECT) px_loads_done();
-    else tile_store<NT, NREC, KS>(sv, s_u[t & 1], tid);
+    else tile_store<NT, NREC, P::REC>(sv, s_u[t & 1], tid);
   };
   fetch(tb);
   polar_params<false>(p, s_par, nullptr, tid);
   landed(tb);
   __syncthreads();
+  f4 par[4];
+  if constexpr (!PAR_LDS) {
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const f4 par = s_par[j0 + 4 * g + a];
-    btr[a] = par[0]; bti[a] = par[1]; ctr[a] = par[2]; cti[a] = par[3];
+    for (int a = 0; a < 4; ++a) par[a] = s_par[j0 + 4 * g + a];
   }
   // the wavefront's own inputs, requested one tile ahead
   const int lf = tb * DT + l_;
   float un = lf < L ? p.u[row + lf] : 0.0f, dtn = lf < L ? p.dt[row + lf] : 0.0f, zn = lf < L ? p.z[zrow + lf] : 0.0f;
+  int en = P::HALF ? phase_columns<KS>(upb, tb)[l_] : 0;   // exponent of the tile's column
   for (int t = tb; t < ntiles; ++t) {
     const int l0 = t * DT, l = l0 + l_;
     const bool lok = l < L;
     const float uv = un, dtv = dtn, zv = zn;
+    const int eu = en;
     {
       const bool nok = l + DT < L;
       un = nok ? p.u[row + l + DT] : 0.0f;
       dtn = nok ? p.dt[row + l + DT] : 0.0f;
       zn = nok ? p.z[zrow + l + DT] : 0.0f;
     }
-    if (t + 1 < ntiles) fetch(t + 1);
+    if (t + 1 < ntiles) {
+      if (P::HALF) en = phase_columns<KS>(upb, t + 1)[l_];
+      fetch(t + 1);
+    }
     // ---- running phases of the tile, less the bias: lane (column l, rows j = 4 g + a)
-    f4 th = {0, 0, 0, 0};
+    P th;
     const u4* su = s_u[t & 1];
 #pragma unroll
-    for (int k = 0; k < KS; ++k) {
-      u4 ubk[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) ubk[q] = su[(k * 3 + q) * 64 + lane];
-      th = xmm<3>(xa[k], ubk, th);
-    }
+    for (int k = 0; k < KS; ++k) th.step(xa[k], su + k * P::NP * 64, lane);
     const float ut = silu_fast(uv), w = dtv * ut;
     const float cnt = (float)(min(l_ + 1, L - l0));      // timesteps of the tile up to this one that exist
     float ysum = 0.0f;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
-      const float G = fmaf(xb[a], cnt, th[a]);
+      const float G = fmaf(xb[a], cnt, th.value(a, ex[a] + eu));
       float sn, cs;
       sincos_any(G, &sn, &cs);
       // p = conj(E) Bt w
-      const float pr = (cs * btr[a] + sn * bti[a]) * w, pi = (cs * bti[a] - sn * btr[a]) * w;
+      const f4 pa = PAR_LDS ? s_par[j0 + 4 * g + a] : par[a];
+      const float pr = (cs * pa[0] + sn * pa[1]) * w, pi = (cs * pa[1] - sn * pa[0]) * w;
       const float Rr = hr[a] + row_prefix(pr), Ri = hi[a] + row_prefix(pi);
       // h = E R
       const float her = cs * Rr - sn * Ri, hei = cs * Ri + sn * Rr;
-      ysum = fmaf(ctr[a], her, fmaf(-cti[a], hei, ysum));
+      ysum = fmaf(pa[2], her, fmaf(-pa[3], hei, ysum));
       hr[a] = row_last(her, lane);
       hi[a] = row_last(hei, lane);
     }
@@ -533,29 +605,26 @@ __device__ __forceinline__ float row_sum(float v) {     // total of the row in i
 }
 
 // The share of a tile's phase product that goes with state group a of 4: its steps k = a KS / 4 .. (KS < 4: all with a = 0).
-// One accumulator, in the order of the forward kernel: the states are recovered from its end state with these phases, and
-// phases that differ in their last bit would add up from tile to tile (gradients off by 1e-5 with two accumulators).
+// The sums run in the order of the forward kernel: the states are recovered from its end state with these phases, and
+// phases that differ in their last bit would add up from tile to tile (gradients off by 1e-5 where the order differed).
 template <int KS>
-__device__ __forceinline__ void phase_part(int a, const u4 (&xa)[KS][3], const u4* __restrict__ su, int lane, f4& acc) {
+__device__ __forceinline__ void phase_part(int a, const u4 (&xa)[KS][Phase<KS>::NP], const u4* __restrict__ su, int lane, Phase<KS>& acc) {
   constexpr int STEP = (KS + 3) / 4;
 #pragma unroll
-  for (int k = a * STEP; k < (a + 1) * STEP && k < KS; ++k) {
-    u4 ubk[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) ubk[q] = su[(k * 3 + q) * 64 + lane];
-    acc = xmm<3>(xa[k], ubk, acc);
-  }
+  for (int k = a * STEP; k < (a + 1) * STEP && k < KS; ++k) acc.step(xa[k], su + k * Phase<KS>::NP * 64, lane);
 }
 
 // The phases of the tile that comes next are formed between the states of the current one: an operand tile is in LDS a tile
 // ahead, and no wavefront waits for its chain of matrix instructions before it can start on the states (a launch over 8 x
-// 256 pairs of 45 tiles, d = 256: 145 -> 136 us).  The forward kernel, whose states take less, runs 10 % slower that way.
+// 256 pairs of 45 tiles, d = 256: 145 -> 136 us; 128 before two f16 pieces, 115 with them).  The forward kernel, whose states take
+// less, runs 10 % slower that way.
 #ifndef DROPIN_BWD_WAVES
 #define DROPIN_BWD_WAVES 1
 #endif
 template <int KS, int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_BWD_WAVES, DROPIN_BWD_WAVES))) void dropin_bwd_kernel(const DropinBwdArgs q) {
-  __shared__ u4 s_u[2][KS * 3 * 64];
+  typedef Phase<KS> P;
+  __shared__ u4 s_u[2][P::REC];
   __shared__ float2 s_yw[2][NW][DT];                   // shares of (sum_j Re(Ct h), sum_j hat w) of the tile (nb > 1)
   const DropinArgs& p = q.f;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
@@ -568,20 +637,18 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
   const int l_ = lane & 15, g = lane >> 4;
   const int d = p.d, n = p.n, L = p.L;
   const size_t row = ((size_t)b * d + ic) * L, zrow = (size_t)b * p.zs + (size_t)ic * L;
-  const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * (KS * 3 * 64);   // + tile * (KS 3 64)
+  const u4* __restrict__ upb = p.up + ((size_t)(b - p.up_b0) * p.up_nt - p.up_t0) * P::TILE;   // + tile * TILE
 
-  u4 xa[KS][3];
-#pragma unroll
-  for (int k = 0; k < KS; ++k)
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-      xa[k][c] = (k < p.ks) ? p.xp[(((size_t)vc * p.ks + k) * 3 + c) * 64 + lane] : u4{0, 0, 0, 0};
+  u4 xa[KS][P::NP];
+  const int* const xe = phase_rows<KS>(p.xp, p.ks, vc, lane, xa);
   // per state: (Re Bt, Im Bt, Re Ct, Im Ct), shared by the workgroup, and the bias of this wavefront's channel.
   // They are read from LDS where they are used: in registers they would push the kernel over 256.
   __shared__ f4 s_par[D_MAXN], s_unit[D_MAXN];
   __shared__ float s_xb[NW][16];
+  __shared__ int s_ex[NW][16];                         // ... and the exponents of its rows of x
   polar_params<true>(p, s_par, s_unit, tid);
   if (lane < 16) s_xb[wave][lane] = j0 + lane < n ? p.x_bias[(size_t)ic * p.xsi + (size_t)(j0 + lane) * p.xsj] : 0.0f;
+  if (P::HALF && lane < 16) s_ex[wave][lane] = xe[lane];
   float hr[4], hi[4], ar[4], ai[4];                    // state at the end of the tile being processed, its adjoint
   float gBr[4], gBi[4], gCr[4], gCi[4], gxb[4];
   int at[4];
@@ -617,19 +684,20 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
   const int t_first = q.t0 + sg * p.sl, t_last = (p.nseg > 1 ? min(t_first + p.sl, q.t1) : q.t1) - 1;
   float* __restrict__ dth = q.dth + ((size_t)zb * d * n + (size_t)ic * p.xsi) * q.lc - (size_t)q.t0 * DT;   // + state j: j xsj rows
 
-  constexpr int NT = NW * 64, NREC = (KS * 3 * 64 + NT - 1) / NT;
+  constexpr int NT = NW * 64, NREC = (P::REC + NT - 1) / NT;
   u4 sv[NREC];
-  tile_load<NT, NREC, KS>(upb + (size_t)t_last * (KS * 3 * 64), sv, tid);
-  tile_store<NT, NREC, KS>(sv, s_u[t_last & 1], tid);
-  tile_load<NT, NREC, KS>(upb + (size_t)max(t_last - 1, t_first) * (KS * 3 * 64), sv, tid);
-  tile_store<NT, NREC, KS>(sv, s_u[(t_last + 1) & 1], tid);
+  tile_load<NT, NREC, P::REC>(upb + (size_t)t_last * P::TILE, sv, tid);
+  tile_store<NT, NREC, P::REC>(sv, s_u[t_last & 1], tid);
+  tile_load<NT, NREC, P::REC>(upb + (size_t)max(t_last - 1, t_first) * P::TILE, sv, tid);
+  tile_store<NT, NREC, P::REC>(sv, s_u[(t_last + 1) & 1], tid);
   __syncthreads();
-  f4 th = {0, 0, 0, 0};
+  P th;
 #pragma unroll
   for (int a = 0; a < 4; ++a) phase_part<KS>(a, xa, s_u[t_last & 1], lane, th);
   __syncthreads();                                     // (the first iteration overwrites that tile)
   // the wavefront's own inputs, requested one tile ahead
   float un, dtn, zn, gyn;
+  int en = P::HALF ? phase_columns<KS>(upb, t_last)[l_] : 0;   // exponent of the tile's column
   {
     const int l = t_last * DT + l_;
     const bool ok = l < L;
@@ -642,14 +710,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     const int l0 = t * DT, l = l0 + l_;
     const bool lok = l < L;
     const float uv = un, dtv = dtn, zv = zn, gyv = gyn;
+    const int eu = en;
     if (t > t_first) {                 // l - DT < L holds
       un = p.u[row + l - DT];
       dtn = p.dt[row + l - DT];
       zn = p.z[zrow + l - DT];
       gyn = q.gy[row + l - DT];
+      if (P::HALF) en = phase_columns<KS>(upb, t - 1)[l_];
     }
-    tile_load<NT, NREC, KS>(upb + (size_t)max(t - 2, t_first) * (KS * 3 * 64), sv, tid);
-    f4 nx = {0, 0, 0, 0};                              // the next tile's phases, formed between the states of this one
+    tile_load<NT, NREC, P::REC>(upb + (size_t)max(t - 2, t_first) * P::TILE, sv, tid);
+    P nx;                                              // the next tile's phases, formed between the states of this one
     const u4* su = s_u[(t + 1) & 1];
     const int lend = min(15, L - 1 - l0);               // the tile's last step that exists
     const float ut = silu_fast(uv), w = dtv * ut, sz = silu_fast(zv), av = gyv * sz;
@@ -660,7 +730,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
       phase_part<KS>(a, xa, su, lane, nx);
       const f4 par = s_par[j0 + 4 * g + a];
       const float btr_ = par[0], bti_ = par[1], ctr_ = par[2], cti_ = par[3];
-      const float G = fmaf(s_xb[wave][4 * g + a], cnt, th[a]);
+      const float G = fmaf(s_xb[wave][4 * g + a], cnt, th.value(a, P::HALF ? s_ex[wave][4 * g + a] + eu : 0));
       float sn, cs;
       sincos_any(G, &sn, &cs);
       const float csl = row_last(cs, lane), snl = row_last(sn, lane);
@@ -702,7 +772,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     }
     // Loads and stores share one in-order counter: the wait for the tile, requested in front of the states, comes before this
     // tile's stores, or it would see them out, too (32 x 128, 720 steps: 221 -> 219 us).
-    tile_store<NT, NREC, KS>(sv, s_u[t & 1], tid);
+    tile_store<NT, NREC, P::REC>(sv, s_u[t & 1], tid);
     // (stored here: a branch inside the loop cuts the four states into blocks that cannot hide each other's latencies)
 #pragma unroll
     for (int a = 0; a < 4; ++a)

@@ -6,6 +6,7 @@ namespace aussm {
 
 constexpr int DT = 16;            // timesteps per tile
 constexpr int D_MAXKS = 16;       // 32-wide steps of the contraction over r held in registers: d <= 512
+constexpr int PHASE_HALF_KS = 3;  // from so many of them on the phase product takes two f16 pieces instead of three bf16 ones
 constexpr int D_MAXN = 64;        // states per channel: up to four blocks of 16, one block per wavefront
 
 struct DropinArgs {
@@ -23,8 +24,8 @@ struct DropinArgs {
   float* y;              // [b, d, L] or null (states only)
   float* nh_re;          // [b, d, n] or null: state after tile t1 - 1 (may be the same buffer as h_*)
   float* nh_im;
-  const u4* xp;          // rows of x as matrix operands: [d nb][ks][piece][64 lanes]
-  const u4* up;          // tiles of u, prefix-summed along the tile, as matrix operands: [b][tile - up_t0][KS][piece][64 lanes]
+  const u4* xp;          // rows of x as matrix operands: [d nb][ks][piece][64 lanes] (f16 pieces: 16 exponents behind each [ks])
+  const u4* up;          // tiles of u, prefix-summed along the tile, as matrix operands: [b][tile - up_t0][KS][piece][64 lanes] (likewise)
   int up_b0, up_t0, up_nt;   // up holds the batch elements from up_b0 on and the tiles up_t0 .. up_t0 + up_nt - 1
   int b, d, n, L, ks;    // b: batch elements of this launch; ks = ceil(d / 32)
   int nb;                // blocks of 16 states per channel: 1, 2 or 4 (>= ceil(n / 16))

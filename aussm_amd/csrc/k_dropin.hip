@@ -19,14 +19,14 @@ int run_fill(const FillArgs& a, hipStream_t s) {
 #endif
 constexpr int DROPIN_NW = DROPIN_NW_;     // channels (wavefronts) per workgroup
 
-// (d > 256: the rows of x take 192 registers, which leaves room for one wavefront per SIMD only)
+// (d > 256: the rows of x take up to 128 registers, in workgroups of four)
 template <int KS, int NW>
 static void launch_fwd_nw(const DropinArgs& a, hipStream_t s) {
   const unsigned grid = (unsigned)((a.nseg > 1 ? a.nseg : 1) * a.b * ((a.d * a.nb + NW - 1) / NW));
   hipLaunchKernelGGL((dropin_fwd_kernel<KS, NW>), dim3(grid), dim3(NW * 64), 0, s, a);
 }
-// Past two wavefronts on every SIMD 128 < d takes workgroups of four, three to a compute unit (dropin.h); up to there they
-// would only read the tiles twice (8 x 250 x 16, 720 steps: 86 us in eights, 90 in fours; 20 x 130: 139, 87).
+// Past two wavefronts on every SIMD 128 < d takes workgroups of four, four to a compute unit (dropin.h); up to there they
+// would only read the tiles twice (8 x 250 x 16, 720 steps: 86 us in eights, 90 in fours; past it 20 x 256: 233, 174).
 template <int KS>
 static void launch_fwd(const DropinArgs& a, hipStream_t s) {
   if constexpr (KS > 8) {
@@ -57,8 +57,13 @@ int dropin_channels_per_workgroup(int ks) { return ks > 8 ? 4 : DROPIN_NW; }
 // the compiled size of the contraction (steps of 32) that serves ceil(d / 32) = ks
 int dropin_compiled_ks(int ks) { return ks <= 4 ? (ks < 1 ? 1 : ks) : ks <= 6 ? 6 : ks <= 8 ? 8 : ks <= 12 ? 12 : 16; }
 
+// 16-byte records of `steps` steps of 16 rows or columns (Phase in dropin.h), by the compiled size of the contraction
+size_t dropin_records(int ks, int steps) {
+  return dropin_compiled_ks(ks) >= PHASE_HALF_KS ? (size_t)steps * 2 * 64 + 4 : (size_t)steps * 3 * 64;
+}
+
 int run_dropin_prep(DropinPrepArgs a, int bg, bool rows, const FillArgs& f, hipStream_t s) {
-  const size_t xb = rows ? ((size_t)a.d * a.nb * a.ks * 64 + 255) / 256 : 0, ub = (size_t)bg * a.nt;
+  const size_t xb = rows ? (size_t)a.d * a.nb : 0, ub = (size_t)bg * a.nt;
   size_t total = xb + ub;
   for (int i = 0; i < f.count; ++i) total += (f.n[i] + FILL_BLOCK - 1) / FILL_BLOCK;
   if (total > 0x7fffffffULL) return -2;

@@ -49,6 +49,7 @@ int run_px_bwd(const UniBwdArgs& a, const u4* img, int in_dtype, hipStream_t s);
 // ---- k_dropin.hip: the reference's 12-input operator as fused kernels
 int dropin_channels_per_workgroup(int ks);
 int dropin_compiled_ks(int ks);
+size_t dropin_records(int ks, int steps);
 int run_dropin_prep(DropinPrepArgs a, int bg, bool rows, const FillArgs& f, hipStream_t s);   // rows: the records of x too
 int run_dropin_fwd(const DropinArgs& a, hipStream_t s);
 int run_dropin_seg(const DropinBwdArgs& a, hipStream_t s);   // maps of the segments (nseg > 1): backward with sega, else forward

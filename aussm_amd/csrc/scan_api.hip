@@ -824,7 +824,7 @@ int aussm_zero_f32(float* p, size_t n, void* stream) {
 
 // blocks of 16 states per channel, one per wavefront: 1, 2 or 4 (they have to divide the wavefronts of a workgroup)
 static int dropin_state_blocks(int n) { const int k = (n + 15) / 16; return k == 3 ? 4 : k; }
-static size_t dropin_xp_floats(int d, int n) { return (size_t)d * dropin_state_blocks(n) * ((d + 31) / 32) * 3 * 64 * 4; }
+static size_t dropin_xp_floats(int d, int n) { return (size_t)d * dropin_state_blocks(n) * dropin_records((d + 31) / 32, (d + 31) / 32) * 4; }
 // The backward call works through the (batch, sequence) plane in blocks of bg batch elements x ct tiles
 // of 16 timesteps: the workspace holds the phase adjoints of one block (about 100 MiB at most:
 // at b = 32, d = 256, n = 16, L = 720 a block of 8 batch elements then spans the whole sequence, 1.39 ms per backward
@@ -862,8 +862,8 @@ static int dropin_check(int b, int d, int n, int L) {
   return AUSSM_OK;
 }
 
-// floats of one prepared tile of u (all compiled steps of the contraction, three pieces, 64 lanes of 16 bytes)
-static size_t dropin_tile_floats(int d) { return (size_t)dropin_compiled_ks((d + 31) / 32) * 3 * 64 * 4; }
+// floats of one prepared tile of u (all compiled steps of the contraction)
+static size_t dropin_tile_floats(int d) { return dropin_records((d + 31) / 32, dropin_compiled_ks((d + 31) / 32)) * 4; }
 // tiles per launch of the forward call: its prepared tiles of u (all batch elements) stay within the block budget
 static int dropin_fwd_chunk_tiles(int b, int d, int L, bool largest = false) {
   const int ntiles = (L + DT - 1) / DT;

@@ -183,6 +183,13 @@ __device__ __forceinline__ void rows_suffix(float x, int g, float* incl, float* 
   if (g < 2) y += d;
   *incl = y; *tot = c + d;
 }
+__device__ __forceinline__ float rows_max(float x) {
+  float a = x, b = x;
+  rows_swap16(a, b);
+  float c = fmaxf(a, b), d = c;
+  rows_swap32(c, d);
+  return fmaxf(c, d);
+}
 __device__ __forceinline__ float rows_sum(float x) {
   float a = x, b = x;
   rows_swap16(a, b);
