@@ -4,13 +4,12 @@
 
 namespace aussm {
 
-template <int WM, int EM, int EN, bool QUAD>
+template <int NW, int WM, int EM, int EN, bool QUAD, bool HALF>
 static int launch_tile(const XGemmArgs& a, unsigned grid, hipStream_t s) {
-  constexpr bool WIDE = WM == 4;
   const bool ak1 = a.sak == 1, bk1 = a.sbk == 1, tr = a.scm == 1 && a.scn != 1;
 #define XG(A_, B_, T_)                                                                       \
   if (ak1 == A_ && bk1 == B_ && tr == T_) {                                                  \
-    hipLaunchKernelGGL((xgemm_kernel<A_, B_, T_, WM, EM, EN, QUAD, WIDE>), dim3(grid), dim3(WIDE ? 512 : 256), 0, s, a);     \
+    hipLaunchKernelGGL((xgemm_kernel<A_, B_, T_, NW, WM, EM, EN, QUAD, HALF>), dim3(grid), dim3(64 * NW), 0, s, a);     \
     return launch_status();                                                                  \
   }
   XG(false, false, false) XG(false, false, true) XG(false, true, false) XG(false, true, true)
@@ -19,18 +18,27 @@ static int launch_tile(const XGemmArgs& a, unsigned grid, hipStream_t s) {
   return -2;
 }
 
-struct Tile { int wm, em, en; };        // wavefronts along the rows; 16-wide row and column tiles per wavefront
+struct Tile { int nw, wm, em, en; };    // wavefronts, of them along the rows; 16-wide row and column tiles per wavefront
 constexpr int rows_of(const Tile& t) { return 16 * t.em * t.wm; }
-constexpr int cols_of(const Tile& t) { return 16 * t.en * (t.wm == 4 ? 2 : 4 / t.wm); }
-constexpr Tile NARROW{2, 4, 4}, COLS64{2, 4, 2}, COLS32{2, 4, 1}, ROWS32{1, 2, 2}, WIDE128{4, 4, 4}, WIDE96{4, 4, 3};
-constexpr Tile T64{2, 2, 2}, R32C64{1, 2, 1}, R64C32{2, 2, 1}, T32{2, 1, 1};       // 64 x 64, 32 x 64, 64 x 32, 32 x 32
+constexpr int cols_of(const Tile& t) { return 16 * t.en * (t.nw / t.wm); }
+constexpr Tile NARROW{4, 2, 4, 4}, COLS64{4, 2, 4, 2}, COLS32{4, 2, 4, 1}, ROWS32{4, 1, 2, 2}, WIDE128{8, 4, 4, 4}, WIDE96{8, 4, 4, 3};
+constexpr Tile T64{4, 2, 2, 2}, R32C64{4, 1, 2, 1}, R64C32{4, 2, 2, 1}, T32{4, 2, 1, 1};       // 64 x 64, 32 x 64, 64 x 32, 32 x 32
 
-template <bool QUAD>
+template <bool QUAD, bool HALF>
 static int launch_xgemm(const Tile& t, const XGemmArgs& a, unsigned grid, hipStream_t s) {
-#define XT(T_) if (t.wm == T_.wm && t.em == T_.em && t.en == T_.en) return launch_tile<T_.wm, T_.em, T_.en, QUAD>(a, grid, s);
-  XT(NARROW) XT(COLS64) XT(COLS32) XT(ROWS32) XT(WIDE128) XT(WIDE96) XT(T64) XT(R32C64) XT(R64C32) XT(T32)
+#define XT(T_) if (t.nw == T_.nw && t.wm == T_.wm && t.em == T_.em && t.en == T_.en) return launch_tile<T_.nw, T_.wm, T_.em, T_.en, QUAD, HALF>(a, grid, s);
+  XT(NARROW) XT(COLS64) XT(COLS32) XT(ROWS32) XT(T64) XT(R32C64) XT(R64C32) XT(T32)
+  if constexpr (HALF) { XT(WIDE128) XT(WIDE96) }
 #undef XT
   return -2;
+}
+
+// f16 pieces: offsets of 32 bits inside a tile, whatever its position, and along k (XgHalfOperand)
+static bool near(const XGemmArgs& a) {
+  constexpr long most = 1l << 28, rows = 256;              // elements; a tile's rows or columns, at most
+  auto fits = [](long n, long stride) { return stride >= 0 && (stride == 0 || n < most / stride); };
+  return fits(rows, a.sam) && fits(a.K, a.sak) && fits(a.K, a.sbk) && fits(a.nper < a.N ? a.nper : rows, a.sbn) &&
+         (a.nper >= a.N || fits(rows / a.nper + 2, a.sbb));
 }
 
 // Small tiles where a product has few of them.  What a step of 32 costs a workgroup is mostly waiting - for the values, for the
@@ -46,28 +54,34 @@ static int launch_xgemm(const Tile& t, const XGemmArgs& a, unsigned grid, hipStr
 // and twice the slices (64 x 23040, 1024: 34.7, with 64 x 128 42.6; 64 x 32768, 4096: 156, 151).
 //
 // Else the wide ones for more rows than the narrow one has, by the rounds that the tiles make on the chip (256 compute
-// units, one wide or two narrow workgroups each) times what a round takes: 1 for 256 x 128, 0.88 for 256 x 96, 1.2 for two of
-// 128 x 128, 0.72 for one.  23040 columns, us narrow / 96 / 128: 256 rows, K = 1024 93 / 70 / 78; 512 rows, K = 256 46 / 43 /
-// 50; 1024 rows, K = 256 77 / 80 / 73; 512 rows, K = 16 17.1 / 17.1 / 19.2.
+// units, one wide or two narrow workgroups each) times what a round takes: 1 for 256 x 128, 0.9 for 256 x 96, 1.2 for two of
+// 128 x 128, 0.72 for one.  23040 columns, us narrow / 96 / 128: 256 rows, K = 1024 66 / 57 / 59; K = 512 41 / 34 / 38; 512 rows, K = 256
+// 39 / 39 / 42; 1024 rows, K = 256 68 / 77 / 65.
 //
 // Slices: a sum over many steps with few tiles is cut into as many workgroups as run at once (more would start a second
 // round: 540 workgroups 140 us, 450 workgroups 91 us for the product with 90 tiles and 128 steps), at least four steps of
 // 32 per slice (shorter ones would spend their time on the atomics of the tile), of small tiles two unless four leave 200
 // workgroups (548 x 137, 36 steps: 10.2 against 11.7 us; 96 x 192, 30 steps: 9.6 against 6.8).  The wide tile from 24 steps a
 // slice on: 4096 x 256, sums of 23040, 281 -> 248 us; 256 x 5760, K = 4096 93 -> 81 us; 512 x 256 (12 steps) 56 against 58 us.
+//
+// f16 pieces from six steps a workgroup on, from eight in the tiles of 32 x 32 to 64 x 32: finding the scales costs 1 to 2 us.  us bf16 / f16:
+// 256 x 256 in tiles of 32 x 32, K = 128 5.2 / 6.0, 192 6.5 / 6.8, 256 7.9 / 7.7, 512 13.3 / 11.0; 512 x 2048 in tiles of 64 x 64, K = 128 7.8 / 8.4,
+// 192 9.7 / 9.6, 512 20.0 / 15.9; 256 x 23040, K = 1024 77 / 57; 256 x 5760, K = 4096 91 / 70; 4096 x 256, sums of 5760 84 / 67.
+// Sums of up to 64 terms, which are more exact on three bf16 pieces, never get there.
 int run_xgemm(XGemmArgs a, hipStream_t s) {
   if (a.M < 1 || a.N < 1 || a.K < 1 || a.Z < 1 || a.nper < 1) return -2;
   if (a.reduce && a.scm == 1 && a.scn != 1 && a.nper < a.N) return -2;
   const long steps = (long)((a.K + 31) / 32) * a.Z;
+  const bool can_half = near(a);
   const bool sliced = a.reduce && !a.bias && !a.add && !a.act;
   auto tiles_of = [&](const Tile& t) { return (long)((a.M + rows_of(t) - 1) / rows_of(t)) * ((a.N + cols_of(t) - 1) / cols_of(t)); };
   Tile tile = a.N <= 32 ? COLS32 : a.N <= 64 ? COLS64 : NARROW;
   bool small = true;
   int slots = 512;
-  const Tile half = tiles_of(R64C32) < tiles_of(R32C64) ? R64C32 : R32C64;
+  const Tile pair = tiles_of(R64C32) < tiles_of(R32C64) ? R64C32 : R32C64;
   if (sliced) {
     if (a.M <= 32 && a.N <= 32) tile = T32;
-    else if ((a.M <= 32 || a.N <= 32) && tiles_of(half) * steps <= 4500) tile = half;
+    else if ((a.M <= 32 || a.N <= 32) && tiles_of(pair) * steps <= 4500) tile = pair;
     else if (a.M > 32 && a.N > 32 && tiles_of(T64) * steps <= (a.K % 4 ? 6000 : 18000)) {
       tile = T64;
       if (tiles_of(T64) * steps > 8000) slots = 1024;
@@ -77,38 +91,40 @@ int run_xgemm(XGemmArgs a, hipStream_t s) {
     else small = false;
   } else {
     if (tiles_of(T32) <= 256) tile = T32;
-    else if (tiles_of(half) <= 256) tile = half;
-    else if (a.M <= 32) tile = tiles_of(half) <= 512 ? half : ROWS32;
+    else if (tiles_of(pair) <= 256) tile = pair;
+    else if (a.M <= 32) tile = tiles_of(pair) <= 512 ? pair : ROWS32;
     else if (tiles_of(T64) <= 1024 || a.M <= 64) tile = T64;
     else small = false;
   }
-  if (!small && a.M > rows_of(NARROW) && a.N > 64) {
+  if (can_half && steps >= 6 && !small && a.M > rows_of(NARROW) && a.N > 64) {
     if (sliced) {
       const long t = tiles_of(WIDE128);
       if (steps >= 24 * (t < 256 ? 256 / t : 1)) tile = WIDE128;
     } else {
       auto rounds = [](long t, long slots) { return (double)((t + slots - 1) / slots); };
-      const double w4 = rounds(tiles_of(WIDE128), 256), w3 = 0.88 * rounds(tiles_of(WIDE96), 256);
+      const double w4 = rounds(tiles_of(WIDE128), 256), w3 = 0.9 * rounds(tiles_of(WIDE96), 256);
       const long t = tiles_of(NARROW);
       const double narrow = 1.2 * (double)(t / 512) + (t % 512 > 256 ? 1.2 : t % 512 ? 0.72 : 0.0);
       if (w3 < narrow || w4 < narrow) tile = w3 < w4 ? WIDE96 : WIDE128;
     }
   }
   const long tiles = tiles_of(tile);
-  long sl = 1;
+  long sl = 1, per = steps;
   if (sliced) {
-    sl = (tile.wm == 4 ? 256 : slots) / tiles;
+    sl = (tile.nw == 8 ? 256 : slots) / tiles;
     const long least = small && tiles * (steps / 4) < 200 ? 2 : 4;
     if (sl > steps / least) sl = steps / least;
     if (sl < 1) sl = 1;
-    const long per = (steps + sl - 1) / sl;
+    per = (steps + sl - 1) / sl;
     sl = (steps + per - 1) / per;
   }
+  const bool half = can_half && per >= (tile.em * tile.en <= 2 ? 8 : 6);
   if (steps > 0x7fffffffL || tiles * sl > 0x7fffffffL) return -2;
   a.slices = (int)sl;
   if (a.scm < 0 || a.scn < 0) return -2;
   const unsigned grid = (unsigned)(tiles * sl);
-  return a.K % 4 == 0 ? launch_xgemm<true>(tile, a, grid, s) : launch_xgemm<false>(tile, a, grid, s);
+  if (half) return a.K % 4 == 0 ? launch_xgemm<true, true>(tile, a, grid, s) : launch_xgemm<false, true>(tile, a, grid, s);
+  return a.K % 4 == 0 ? launch_xgemm<true, false>(tile, a, grid, s) : launch_xgemm<false, false>(tile, a, grid, s);
 }
 
 }  // namespace aussm

@@ -361,8 +361,8 @@ int aussm_operator_bwd(const aussm_operator_args* op, const float* grad_y, const
                        const float* nh_re, const float* nh_im, const aussm_operator_grads* grads, float* workspace, void* stream);
 
 /* ---------------------------------------------------------------------------------------
- * fp32-accurate matrix products of the blocks' linear layers (bf16 matrix cores on operands split into three exact
- * pieces, fp32 sums): nn.Linear of ai-modules/wavesAI/model/aussm.py:725-737, :813-828 and its gradients.
+ * fp32-accurate matrix products of the blocks' linear layers (16-bit matrix cores on operands split into three bf16 or
+ * two scaled f16 pieces, fp32 sums): nn.Linear of ai-modules/wavesAI/model/aussm.py:725-737, :813-828 and its gradients.
  *     C(m, n) = act( alpha sum_k A(m, k) B(k, n) + bias_scale bias[m] + add(m, n) )
  * Column n lies in batch n / nper, at position n % nper: B and C move by sbb / scb per batch and by sbn / scn per
  * position (one A for a batch of products).  With Z > 1 the product is also summed over z (A, B move by saz, sbz).
