@@ -38,9 +38,33 @@ __device__ __forceinline__ void oct_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // Orders LDS accesses of a wavefront for the compiler; the hardware executes them in order.
 __device__ __forceinline__ void oct_wave_fence() { asm volatile("" ::: "memory"); }
 
+// out[j]: a[j] + its partner's a[j] in the lanes of banks (four lanes) LOW, b[j] + its partner's b[j] in the others.  Two instructions
+// that write their banks only, where selecting both summands takes two more at twice the price of an addition (a DPP addition
+// and a select by a scalar mask take 5 cycles each); one wait for all sources.  S6, 32 x 512 x 16, 2048 steps: see below.
+#define OCT_PAIR(CTRL_, LOW_, HIGH_, o_, a_, b_)                                                      \
+  "v_add_f32_dpp " o_ ", " a_ ", " a_ " " CTRL_ " row_mask:0xf bank_mask:" LOW_ "\n\t"                  \
+  "v_add_f32_dpp " o_ ", " b_ ", " b_ " " CTRL_ " row_mask:0xf bank_mask:" HIGH_ "\n\t"
+__device__ __forceinline__ void bank_sums(const float (&v)[8], float (&q)[4]) {   // lane bit 2
+#define P_(o_, a_, b_) OCT_PAIR("row_half_mirror", "0x5", "0xa", o_, a_, b_)
+  asm("s_nop 1\n\t" P_("%0", "%4", "%8") P_("%1", "%5", "%9") P_("%2", "%6", "%10") P_("%3", "%7", "%11")
+      : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3])
+      : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
+}
+__device__ __forceinline__ void bank_sums(const float (&v)[4], float (&q)[2]) {
+  asm("s_nop 1\n\t" P_("%0", "%2", "%4") P_("%1", "%3", "%5")
+      : "=&v"(q[0]), "=&v"(q[1]) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]));
+#undef P_
+}
+__device__ __forceinline__ float bank_sum8(float a, float b) {                    // lane bit 3
+  float o;
+  asm("s_nop 1\n\t" OCT_PAIR("row_ror:8", "0x3", "0xc", "%0", "%1", "%2") : "=&v"(o) : "v"(a), "v"(b));
+  return o;
+}
+#undef OCT_PAIR
+
 // Sums over the eight channels of a wavefront (lane bits 3 .. 5) of eight values: lane 8 c + g returns the total of v[c]
-// over the lanes 8 * + g.  15 instructions: two rounds of row swaps, one rotation by half a row.
-__device__ __forceinline__ float channel_sums(const float (&v)[8], bool bit3) {
+// over the lanes 8 * + g.  14 instructions: two rounds of row swaps, one rotation by half a row.
+__device__ __forceinline__ float channel_sums(const float (&v)[8]) {
   float q[4], r[2];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -54,21 +78,20 @@ __device__ __forceinline__ float channel_sums(const float (&v)[8], bool bit3) {
     rows_swap16(a, b);
     r[j] = a + b;
   }
-  return (bit3 ? r[1] : r[0]) + dpp_perm<0x128>(bit3 ? r[0] : r[1]);      // row_ror:8
+  return bank_sum8(r[0], r[1]);
 }
 // Sums over the eight state groups of a channel (lane bits 0 .. 2): lane 8 c + g returns the total of v[g] over the lanes
 // 8 c + *.  The first step takes the mirrored lane of the half row, whose pairs the two steps inside the quads complete.
-__device__ __forceinline__ float state_sums(const float (&v)[8], bool bit2, bool bit1, bool bit0) {
+__device__ __forceinline__ float state_sums(const float (&v)[8], bool bit1, bool bit0) {
   float q[4], r[2];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) q[j] = (bit2 ? v[j + 4] : v[j]) + dpp_perm<0x141>(bit2 ? v[j] : v[j + 4]);   // row_half_mirror
+  bank_sums(v, q);
 #pragma unroll
   for (int j = 0; j < 2; ++j) r[j] = (bit1 ? q[j + 2] : q[j]) + dpp_perm<0x4E>(bit1 ? q[j] : q[j + 2]);    // quad_perm:[2,3,0,1]
   return (bit0 ? r[1] : r[0]) + dpp_perm<0xB1>(bit0 ? r[0] : r[1]);                                        // quad_perm:[1,0,3,2]
 }
-// The same sums of four values: lanes 8 c + g with bits 1 and 2 of c (of g) equal to j return the total of v[j] (7 and 10
+// The same sums of four values: lanes 8 c + g with bits 1 and 2 of c (of g) equal to j return the total of v[j] (7 and 8
 // instructions; where registers for eight steps at a time are not there).
-__device__ __forceinline__ float channel_sums(const float (&v)[4], bool) {
+__device__ __forceinline__ float channel_sums(const float (&v)[4]) {
   float q[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -80,10 +103,9 @@ __device__ __forceinline__ float channel_sums(const float (&v)[4], bool) {
   const float r = q[0] + q[1];
   return r + dpp_perm<0x128>(r);
 }
-__device__ __forceinline__ float state_sums(const float (&v)[4], bool bit2, bool bit1, bool) {
+__device__ __forceinline__ float state_sums(const float (&v)[4], bool bit1, bool) {
   float q[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) q[j] = (bit2 ? v[j + 2] : v[j]) + dpp_perm<0x141>(bit2 ? v[j] : v[j + 2]);
+  bank_sums(v, q);
   const float r = (bit1 ? q[1] : q[0]) + dpp_perm<0x4E>(bit1 ? q[0] : q[1]);
   return r + dpp_perm<0xB1>(r);
 }
@@ -251,7 +273,7 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int c = lane >> 3, g = lane & 7;
-  const bool bit2 = g & 4, bit1 = g & 2, bit0 = g & 1;
+  const bool bit1 = g & 2, bit0 = g & 1;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
   const int vb = wg / p.ncg, d0 = (wg % p.ncg) * CH;
   const int b = vb / p.ns, sg = vb - b * p.ns;
@@ -445,7 +467,7 @@ __global__ __launch_bounds__(512) void oct_fwd_kernel(const FwdArgs p) {
         for (int t = 0; t < G; ++t) ya[t] = 0.f;
       };
       auto sums = [&](int q) {                               // (over what the group has read)
-        if constexpr (!LEAN) in[q * G + (G == 8 ? g : g >> 1)] = state_sums(ya, bit2, bit1, bit0);
+        if constexpr (!LEAN) in[q * G + (G == 8 ? g : g >> 1)] = state_sums(ya, bit1, bit0);
         else {
 #pragma unroll
           for (int s = 0; s < S; ++s) pin(hr[s], hi[s]);
@@ -783,7 +805,7 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int c = lane >> 3, g = lane & 7;
-  const bool bit3 = lane & 8, bit2 = g & 4, bit1 = g & 2, bit0 = g & 1;
+  const bool bit1 = g & 2, bit0 = g & 1;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
   const int vb = wg / p.ncg, d0 = (wg % p.ncg) * CH;
   const int b = vb / p.ns, sg = vb - b * p.ns;
@@ -1128,9 +1150,9 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
         float* o = slab + (8 * s + g) * SR + (qq * G + cs_) * C;
         auto put = [&](float* o_) {
           if constexpr (C == 1) {
-            o_[0] = channel_sums(vb_r, bit3);
+            o_[0] = channel_sums(vb_r);
           } else {
-            const float re = channel_sums(vb_r, bit3), im = channel_sums(vb_i, bit3);
+            const float re = channel_sums(vb_r), im = channel_sums(vb_i);
             *reinterpret_cast<float2*>(o_) = make_float2(re, im);
           }
         };
@@ -1147,10 +1169,10 @@ __global__ __launch_bounds__(512) void oct_bwd_kernel(const RecBwdArgs p) {
       }
       // sums over the states, over what the group has read
       float* o = in + c * OP + t0 + qq * G + gs_;
-      o[PKA * PL] = state_sums(ka, bit2, bit1, bit0);
-      o[PXA * PL] = state_sums(xa, bit2, bit1, bit0);
-      if constexpr (VAR == VAR_COMPLEX) o[PZA * PL] = state_sums(za, bit2, bit1, bit0);
-      if constexpr (GATED) o[PYA * PL] = state_sums(ya, bit2, bit1, bit0);
+      o[PKA * PL] = state_sums(ka, bit1, bit0);
+      o[PXA * PL] = state_sums(xa, bit1, bit0);
+      if constexpr (VAR == VAR_COMPLEX) o[PZA * PL] = state_sums(za, bit1, bit0);
+      if constexpr (GATED) o[PYA * PL] = state_sums(ya, bit1, bit0);
     }
   };
 
