@@ -75,11 +75,17 @@ __device__ __forceinline__ const int* phase_rows(const u4* __restrict__ xp, int 
   return reinterpret_cast<const int*>(r + ks * NP * 64);
 }
 
-// sin and cos of any argument without a branch: reduction by 2 pi in two fused steps (the result is as exact
-// as the fp32 argument itself), then the hardware sine and cosine of the reduced argument (sincos_small_hw).  A
-// branch here would cut the four state groups of a lane into separate blocks that the scheduler cannot interleave.
+// sin and cos of any argument, in revolutions for the hardware's units: the turns drop out in the first fused step, the second one adds
+// what the constant 1 / 2 pi leaves (the result is as exact as the fp32 argument itself).  A branch here would cut the four state
+// groups of a lane into separate blocks that the scheduler cannot interleave.  (x and x_bias in revolutions from the start would save
+// two more instructions of four, but their rounding is the same at every step and adds up: y off by 1.2e-5 where it is 4.9e-6, 1 x 32 x
+// 64, 2048 steps of u in {0, 1}.)
 __device__ __forceinline__ void sincos_any(float x, float* sn, float* cs) {
-  sincos_small_hw(x, sn, cs);
+  constexpr float C = 0.15915493667125702f, C_REST = 6.4206383e-9f;
+  float t = fmaf(x, C, -rintf(x * C));
+  t = fmaf(x, C_REST, t);
+  *sn = __builtin_amdgcn_sinf(t);
+  *cs = __builtin_amdgcn_cosf(t);
 }
 
 // silu and its derivative with the hardware reciprocal (1 ulp) instead of an IEEE division (ten instructions)
@@ -93,19 +99,37 @@ __device__ __forceinline__ float op_radius(const DropinArgs& p, const float* r, 
   return p.raw ? softplusf_(v) : v;
 }
 __device__ __forceinline__ float op_phase(const DropinArgs& p, const float* th, int j) { return th[(size_t)j * p.bcs]; }
-// (Re Bt, Im Bt, Re Ct, Im Ct) of every state, 0 past n, and with UNIT (e^{i B_theta}, e^{i C_theta}), made by the first 128 threads of a
-// workgroup, one polar number each: a sine with its branches in every lane for its own four states, at either end of a kernel,
-// was half of the kernels' code and 3 to 4 us of every launch, mostly fetching it (5 x 48 pairs, 64 steps: 10.9 -> 9.0 us
+// The polar parameters of every state, 0 past n.  For the maps of the segments (Re Bt, Im Bt, Re Ct, Im Ct).  With TURNED, for the sweeps,
+// (B_r, 0, Re Ct', Im Ct') and the units (e^{i B_theta}, e^{i (B_theta + C_theta)}): a sweep works on states (and adjoints) turned by
+// e^{-i B_theta}, whose inputs are real, with Ct' = Ct e^{i B_theta} - three operations of six for p, one of two for hat w, three of
+// four for hat G (8 x 256 x 16, 720 steps: reverse sweep 131 -> 126 us, an instruction less per sine in it).
+// Made by the first 128 threads of a workgroup, one polar number each: a sine with its branches in every lane for its own four states,
+// at either end of a kernel, was half of the kernels' code and 3 to 4 us of every launch, mostly fetching it (5 x 48 pairs, 64 steps: 10.9 -> 9.0 us
 // forward, 21.5 -> 15.8 backward).
-template <bool UNIT>
+template <bool TURNED>
 __device__ __forceinline__ void polar_params(const DropinArgs& p, f4* s_par, f4* s_unit, int tid) {
   if (tid >= 2 * D_MAXN) return;
-  const int j = tid & (D_MAXN - 1), c = tid / D_MAXN, jc = j < p.n ? j : 0;
+  const int j = tid >> 1, c = tid & 1, jc = j < p.n ? j : 0;      // (neighbouring lanes: Bt, Ct of a state)
   float sn, cs;
   fast_sincosf(op_phase(p, c ? p.C_th : p.B_th, jc), &sn, &cs);
   const float r = j < p.n ? op_radius(p, c ? p.C_r : p.B_r, jc) : 0.0f;
-  reinterpret_cast<float2*>(s_par)[2 * j + c] = make_float2(r * cs, r * sn);
-  if (UNIT) reinterpret_cast<float2*>(s_unit)[2 * j + c] = make_float2(cs, sn);
+  if (TURNED) {
+    const float bc = __shfl_xor(cs, 1), bs = __shfl_xor(sn, 1);
+    const float2 unit = c ? make_float2(cs * bc - sn * bs, sn * bc + cs * bs) : make_float2(cs, sn);
+    reinterpret_cast<float2*>(s_par)[2 * j + c] = c ? make_float2(r * unit.x, r * unit.y) : make_float2(r, 0.0f);
+    reinterpret_cast<float2*>(s_unit)[2 * j + c] = unit;
+  } else {
+    reinterpret_cast<float2*>(s_par)[2 * j + c] = make_float2(r * cs, r * sn);
+  }
+}
+// A state or an adjoint into a sweep's frame and out of it
+__device__ __forceinline__ void turn_in(const f4& unit, float& re, float& im) {
+  const float r = re * unit[0] + im * unit[1];
+  im = im * unit[0] - re * unit[1];
+  re = r;
+}
+__device__ __forceinline__ float2 turn_out(const f4& unit, float re, float im) {
+  return make_float2(re * unit[0] - im * unit[1], re * unit[1] + im * unit[0]);
 }
 // Derivative of the softplus behind dt, from dt itself: 1 - e^-dt, below 1 by its Taylor series (the next term is below
 // 2^-28 of the value).  Measured through the gradient of dt's argument, the rounding of the product included: root mean
@@ -144,6 +168,20 @@ __device__ __forceinline__ float row_suffix(float v) {   // inclusive, towards l
   v += dpp_mov0<0x104>(v);
   v += dpp_mov0<0x108>(v);
   return v;
+}
+// Prefix sums of the first UP of N values and suffix sums of the others, a step of all before the next one of any: left to the compiler
+// they came one after the other, with two idle cycles and a full latency between two steps of one sum.  (The values are kept apart
+// from the sums they enter: a product fused into its first step takes three instructions instead of two.  Matrix instructions, LDS reads
+// and scalar work may cross the fences.)
+template <int UP, int N>
+__device__ __forceinline__ void rows_side_by_side(float (&v)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) asm("" : "+v"(v[k]));
+#define ROWS_STEP(C_)                                                                        \
+  _Pragma("unroll") for (int k = 0; k < N; ++k) v[k] += k < UP ? dpp_mov0<0x110 + C_>(v[k]) : dpp_mov0<0x100 + C_>(v[k]); \
+  __builtin_amdgcn_sched_barrier(0x10C);
+  ROWS_STEP(1) ROWS_STEP(2) ROWS_STEP(4) ROWS_STEP(8)      // row_shr, row_shl
+#undef ROWS_STEP
 }
 // value of the row's last / first lane in every lane of the row (DPP row broadcast: one vector instruction, where a
 // lane shuffle is an LDS round trip on the chain that hands the state from tile to tile)
@@ -442,7 +480,7 @@ template <int KS, int NW>
 __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 4 : 1) void dropin_fwd_kernel(const DropinArgs p) {
   typedef Phase<KS> P;
   __shared__ u4 s_u[2][P::REC];
-  __shared__ f4 s_par[D_MAXN];
+  __shared__ f4 s_par[D_MAXN], s_unit[D_MAXN];
   __shared__ float s_y[2][NW][DT];                     // shares of y of the tile, by tile parity (nb > 1)
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
   const int nb = p.nb, ncg = (p.d * nb + NW - 1) / NW;
@@ -460,17 +498,20 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 4 : 1) void dropin_fw
   // this wavefront's rows of x, split, for the whole launch
   u4 xa[KS][P::NP];
   const int* const xe = phase_rows<KS>(p.xp, p.ks, vc, lane, xa);
-  // per state j = j0 + 4 g + a: bias, Bt, Ct, carried state
-  float xb[4], hr[4], hi[4];
-  int at[4], ex[4];
+  // per state j = j0 + 4 g + a: bias and exponent of the phase (PAR_LDS: in LDS), carried state
+  constexpr bool PAR_LDS = NW == 4 && KS == 8;
+  __shared__ float2 s_row[PAR_LDS ? NW : 1][16];
+  float2 xrow[4];
+  float hr[4], hi[4];
+  int at[4];
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
     const int j = j0 + 4 * g + a;
     const bool ok = j < n;
     const int jc = ok ? j : 0;
     const size_t cell_ = ((size_t)(b - p.b0) * d + ic) * n + jc;
-    xb[a] = ok ? p.x_bias[(size_t)ic * p.xsi + (size_t)jc * p.xsj] : 0.0f;
-    ex[a] = P::HALF ? xe[4 * g + a] : 0;
+    xrow[a] = make_float2(ok ? p.x_bias[(size_t)ic * p.xsi + (size_t)jc * p.xsj] : 0.0f, __int_as_float(P::HALF ? xe[4 * g + a] : 0));
+    if (PAR_LDS && l_ == 0) s_row[wave][4 * g + a] = xrow[a];
     hr[a] = ok && p.h_re ? p.h_re[(size_t)p.b0 * d * n + cell_] : 0.0f;
     hi[a] = ok && p.h_im ? p.h_im[(size_t)p.b0 * d * n + cell_] : 0.0f;
     at[a] = (int)cell_;                                // (of use with segments, where there are few)
@@ -483,7 +524,6 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 4 : 1) void dropin_fw
   }
   const float Di = p.Dp[ic];
 
-  constexpr bool PAR_LDS = NW == 4 && KS == 8;
   constexpr bool DIRECT = KS <= 4 || (KS <= 8 && NW == 4);
   constexpr int NT = NW * 64, NREC = DIRECT ? 1 : (P::REC + NT - 1) / NT;
   u4 sv[NREC];
@@ -500,13 +540,14 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 4 : 1) void dropin_fw
     else tile_store<NT, NREC, P::REC>(sv, s_u[t & 1], tid);
   };
   fetch(tb);
-  polar_params<false>(p, s_par, nullptr, tid);
+  polar_params<true>(p, s_par, s_unit, tid);
   landed(tb);
   __syncthreads();
   f4 par[4];
-  if constexpr (!PAR_LDS) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) par[a] = s_par[j0 + 4 * g + a];
+  for (int a = 0; a < 4; ++a) {
+    if constexpr (!PAR_LDS) par[a] = s_par[j0 + 4 * g + a];
+    turn_in(s_unit[j0 + 4 * g + a], hr[a], hi[a]);
   }
   // the wavefront's own inputs, requested one tile ahead
   const int lf = tb * DT + l_;
@@ -535,20 +576,36 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 4 : 1) void dropin_fw
     const float ut = silu_fast(uv), w = dtv * ut;
     const float cnt = (float)(min(l_ + 1, L - l0));      // timesteps of the tile up to this one that exist
     float ysum = 0.0f;
+    // GS states side by side (rows_side_by_side; all four would spill registers where the parameters stay in LDS).  32 x 256 x 16, 720
+    // steps, in workgroups of four 243 -> 237 us; 8 x 180, 700 steps 70 -> 66
+    constexpr int GS = PAR_LDS ? 2 : 4;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const float G = fmaf(xb[a], cnt, th.value(a, ex[a] + eu));
-      float sn, cs;
-      sincos_any(G, &sn, &cs);
-      // p = conj(E) Bt w
-      const f4 pa = PAR_LDS ? s_par[j0 + 4 * g + a] : par[a];
-      const float pr = (cs * pa[0] + sn * pa[1]) * w, pi = (cs * pa[1] - sn * pa[0]) * w;
-      const float Rr = hr[a] + row_prefix(pr), Ri = hi[a] + row_prefix(pi);
-      // h = E R
-      const float her = cs * Rr - sn * Ri, hei = cs * Ri + sn * Rr;
-      ysum = fmaf(pa[2], her, fmaf(-pa[3], hei, ysum));
-      hr[a] = row_last(her, lane);
-      hi[a] = row_last(hei, lane);
+    for (int a0 = 0; a0 < 4; a0 += GS) {
+      float sn[GS], cs[GS], pq[2 * GS];
+      f4 pa[GS];
+#pragma unroll
+      for (int k = 0; k < GS; ++k) {
+        const int a = a0 + k;
+        const float2 xr = PAR_LDS ? s_row[wave][4 * g + a] : xrow[a];
+        pa[k] = PAR_LDS ? s_par[j0 + 4 * g + a] : par[a];
+        sincos_any(fmaf(xr.x, cnt, th.value(a, __float_as_int(xr.y) + eu)), &sn[k], &cs[k]);
+        // p = conj(E) B_r w = pr - i qi
+        const float rw = pa[k][0] * w;
+        pq[2 * k] = cs[k] * rw;
+        pq[2 * k + 1] = sn[k] * rw;
+      }
+      rows_side_by_side<2 * GS>(pq);
+#pragma unroll
+      for (int k = 0; k < GS; ++k) {
+        const int a = a0 + k;
+        const float Rr = hr[a] + pq[2 * k], Ri = hi[a] - pq[2 * k + 1];
+        // h = E R
+        const float her = cs[k] * Rr - sn[k] * Ri, hei = cs[k] * Ri + sn[k] * Rr;
+        ysum = fmaf(pa[k][2], her, fmaf(-pa[k][3], hei, ysum));
+        hr[a] = row_last(her, lane);
+        hi[a] = row_last(hei, lane);
+      }
+      if (PAR_LDS) __builtin_amdgcn_sched_barrier(0);
     }
     ysum = rows_sum(ysum);
     if (t + 1 < ntiles) landed(t + 1);                 // (in front of this tile's store, which the counter would wait for, too)
@@ -569,8 +626,9 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 4 : 1) void dropin_fw
     for (int a = 0; a < 4; ++a) {
       const int j = j0 + 4 * g + a;
       if (j < n) {
-        p.nh_re[((size_t)b * d + i) * n + j] = hr[a];
-        p.nh_im[((size_t)b * d + i) * n + j] = hi[a];
+        const float2 h = turn_out(s_unit[j], hr[a], hi[a]);
+        p.nh_re[((size_t)b * d + i) * n + j] = h.x;
+        p.nh_im[((size_t)b * d + i) * n + j] = h.y;
       }
     }
   }
@@ -641,7 +699,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
 
   u4 xa[KS][P::NP];
   const int* const xe = phase_rows<KS>(p.xp, p.ks, vc, lane, xa);
-  // per state: (Re Bt, Im Bt, Re Ct, Im Ct), shared by the workgroup, and the bias of this wavefront's channel.
+  // per state: (B_r, 0, Re Ct', Im Ct'), shared by the workgroup, and the bias of this wavefront's channel.
   // They are read from LDS where they are used: in registers they would push the kernel over 256.
   __shared__ f4 s_par[D_MAXN], s_unit[D_MAXN];
   __shared__ float s_xb[NW][16];
@@ -691,6 +749,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
   tile_load<NT, NREC, P::REC>(upb + (size_t)max(t_last - 1, t_first) * P::TILE, sv, tid);
   tile_store<NT, NREC, P::REC>(sv, s_u[(t_last + 1) & 1], tid);
   __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const f4 unit = s_unit[j0 + 4 * g + a];
+    turn_in(unit, hr[a], hi[a]);
+    turn_in(unit, ar[a], ai[a]);
+  }
   P th;
 #pragma unroll
   for (int a = 0; a < 4; ++a) phase_part<KS>(a, xa, s_u[t_last & 1], lane, th);
@@ -725,49 +789,70 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
     const float ut = silu_fast(uv), w = dtv * ut, sz = silu_fast(zv), av = gyv * sz;
     const float cnt = (float)(min(l_ + 1, L - l0));      // timesteps of the tile up to this one that exist
     float ysum = 0.0f, wsum = 0.0f, thv[4];
+    // GS states side by side, with their share of the next tile's phases.  us by one, two, four of them: 32 x 32 x 64 99, 97, 94; 8 x
+    // 180 x 16, 700 steps 111, 103, 101; 8 x 256, 720 steps 128, 118, 119 (there the long phase products stay between the pairs).
+    constexpr int GS = KS >= 8 ? 2 : 4;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      phase_part<KS>(a, xa, su, lane, nx);
-      const f4 par = s_par[j0 + 4 * g + a];
-      const float btr_ = par[0], bti_ = par[1], ctr_ = par[2], cti_ = par[3];
-      const float G = fmaf(s_xb[wave][4 * g + a], cnt, th.value(a, P::HALF ? s_ex[wave][4 * g + a] + eu : 0));
-      float sn, cs;
-      sincos_any(G, &sn, &cs);
-      const float csl = row_last(cs, lane), snl = row_last(sn, lane);
-      // forward quantities of the tile from the state at its end
-      const float pr = (cs * btr_ + sn * bti_) * w, pi = (cs * bti_ - sn * btr_) * w;
-      const float Ppr = row_prefix(pr), Ppi = row_prefix(pi);
-      const float Ptr = row_last(Ppr, lane), Pti = row_last(Ppi, lane);
-      const float Rer = csl * hr[a] + snl * hi[a], Rei = csl * hi[a] - snl * hr[a];   // conj(E_last) h_out
-      const float hinr = Rer - Ptr, hini = Rei - Pti;
-      const float Rr = hinr + Ppr, Ri = hini + Ppi;
-      const float her = cs * Rr - sn * Ri, hei = cs * Ri + sn * Rr;                  // h_l
-      ysum = fmaf(ctr_, her, fmaf(-cti_, hei, ysum));
-      // adjoints
-      const float hdr = av * ctr_, hdi = -av * cti_;                              // a conj(Ct)
-      const float Rhr = cs * hdr + sn * hdi, Rhi = cs * hdi - sn * hdr;               // conj(E_l) (a conj(Ct))
-      const float Kr = csl * ar[a] + snl * ai[a], Ki = csl * ai[a] - snl * ar[a];     // conj(E_last) hat h_out
-      const float phr = row_suffix(Rhr) + Kr, phi = row_suffix(Rhi) + Ki;             // hat p_s
-      // X = E hat p:  hat w = Re(conj(Bt) X),  hat Bt += w X
-      const float Xr = fmaf(cs, phr, -(sn * phi)), Xi = fmaf(cs, phi, sn * phr);
-      wsum = fmaf(btr_, Xr, fmaf(bti_, Xi, wsum));
-      gBr[a] = fmaf(w, Xr, gBr[a]);
-      gBi[a] = fmaf(w, Xi, gBi[a]);
-      // hat G
-      float Gh = fmaf(phr, pi, fmaf(-phi, pr, fmaf(hdi, her, -(hdr * hei))));
-      if (l_ == lend) Gh -= ar[a] * hi[a] - ai[a] * hr[a];                            // h at the last step is h_out
-      const float thh = row_suffix(Gh);
-      thv[a] = thh;
-      gxb[a] += thh;                                   // (zero past the end)
-      gCr[a] = fmaf(av, her, gCr[a]);                  // hat Ct += a conj(h)
-      gCi[a] = fmaf(-av, hei, gCi[a]);
-      // hand over to the previous tile
-      hr[a] = hinr;
-      hi[a] = hini;
-      ar[a] = row_first(phr, lane);
-      ai[a] = row_first(phi, lane);
-      // (Long phase products stay between the states: gathered by the scheduler, 32 x 256 x 16, 720 steps: 550 us, 540 so; 32 x
-      // 128, 220 gathered, 225.)
+    for (int a0 = 0; a0 < 4; a0 += GS) {
+      f4 par[GS];
+      float sn[GS], cs[GS], rw[GS], hdr[GS], hdi[GS], Gh[GS];
+      float sums[4 * GS];                              // of p, then of conj(E_l) (a conj(Ct))
+      float* const pq = sums;
+      float* const rh = sums + 2 * GS;
+#pragma unroll
+      for (int k = 0; k < GS; ++k) {
+        const int a = a0 + k;
+        phase_part<KS>(a, xa, su, lane, nx);
+        par[k] = s_par[j0 + 4 * g + a];
+        sincos_any(fmaf(s_xb[wave][4 * g + a], cnt, th.value(a, P::HALF ? s_ex[wave][4 * g + a] + eu : 0)), &sn[k], &cs[k]);
+        rw[k] = par[k][0] * w;                                                        // p = conj(E) B_r w = pr - i qi
+        pq[2 * k] = cs[k] * rw[k];
+        pq[2 * k + 1] = sn[k] * rw[k];
+        hdr[k] = av * par[k][2];                                                      // a conj(Ct)
+        hdi[k] = -av * par[k][3];
+        rh[2 * k] = cs[k] * hdr[k] + sn[k] * hdi[k];
+        rh[2 * k + 1] = cs[k] * hdi[k] - sn[k] * hdr[k];
+      }
+      rows_side_by_side<2 * GS>(sums);
+      float phr[GS], phi[GS], hinr[GS], hini[GS];
+#pragma unroll
+      for (int k = 0; k < GS; ++k) {
+        const int a = a0 + k;
+        const float csl = row_last(cs[k], lane), snl = row_last(sn[k], lane);
+        // forward quantities of the tile from the state at its end
+        const float Rer = csl * hr[a] + snl * hi[a], Rei = csl * hi[a] - snl * hr[a];   // conj(E_last) h_out
+        hinr[k] = Rer - row_last(pq[2 * k], lane);
+        hini[k] = Rei + row_last(pq[2 * k + 1], lane);
+        const float Rr = hinr[k] + pq[2 * k], Ri = hini[k] - pq[2 * k + 1];
+        const float her = cs[k] * Rr - sn[k] * Ri, hei = cs[k] * Ri + sn[k] * Rr;       // h_l
+        ysum = fmaf(par[k][2], her, fmaf(-par[k][3], hei, ysum));
+        // adjoints
+        const float Kr = csl * ar[a] + snl * ai[a], Ki = csl * ai[a] - snl * ar[a];     // conj(E_last) hat h_out
+        phr[k] = rh[2 * k] + Kr;                                                        // hat p_s
+        phi[k] = rh[2 * k + 1] + Ki;
+        // X = E hat p:  hat w = B_r Re(X),  hat Bt += w X,  Im(conj(hat p) p) = -B_r w Im(X)
+        const float Xr = fmaf(cs[k], phr[k], -(sn[k] * phi[k])), Xi = fmaf(cs[k], phi[k], sn[k] * phr[k]);
+        wsum = fmaf(par[k][0], Xr, wsum);
+        gBr[a] = fmaf(w, Xr, gBr[a]);
+        gBi[a] = fmaf(w, Xi, gBi[a]);
+        // hat G
+        Gh[k] = fmaf(-rw[k], Xi, fmaf(hdi[k], her, -(hdr[k] * hei)));
+        if (l_ == lend) Gh[k] -= ar[a] * hi[a] - ai[a] * hr[a];                         // h at the last step is h_out
+        gCr[a] = fmaf(av, her, gCr[a]);                                                 // hat Ct += a conj(h)
+        gCi[a] = fmaf(-av, hei, gCi[a]);
+      }
+      rows_side_by_side<0>(Gh);
+#pragma unroll
+      for (int k = 0; k < GS; ++k) {
+        const int a = a0 + k;
+        thv[a] = Gh[k];
+        gxb[a] += Gh[k];                                                                // (zero past the end)
+        // hand over to the previous tile
+        hr[a] = hinr[k];
+        hi[a] = hini[k];
+        ar[a] = row_first(phr[k], lane);
+        ai[a] = row_first(phi[k], lane);
+      }
       if (KS >= 8) __builtin_amdgcn_sched_barrier(0);
     }
     // Loads and stores share one in-order counter: the wait for the tile, requested in front of the states, comes before this
@@ -827,15 +912,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DROPIN_
       if (j < n) {
         const size_t sidx = ((size_t)b * d + i) * n + j;
         if (sg == 0) {
-          e->dh_re[sidx] = ar[a];
-          e->dh_im[sidx] = ai[a];
-          e->hc_re[sidx] = hr[a];
-          e->hc_im[sidx] = hi[a];
+          const float2 dh = turn_out(s_unit[j], ar[a], ai[a]), h = turn_out(s_unit[j], hr[a], hi[a]);
+          e->dh_re[sidx] = dh.x;
+          e->dh_im[sidx] = dh.y;
+          e->hc_re[sidx] = h.x;
+          e->hc_im[sidx] = h.y;
         }
         atomicAdd(e->dxb + (size_t)i * e->f.xsi + (size_t)j * e->f.xsj, gxb[a]);
-        const f4 par = s_par[j], un_ = s_unit[j];      // polar parameters: Bt = B_r e^{i B_theta}
-        atomicAdd(&s_red[0][j], gBr[a] * un_[0] + gBi[a] * un_[1]);
-        atomicAdd(&s_red[1][j], gBi[a] * par[0] - gBr[a] * par[1]);
+        const f4 par = s_par[j], un_ = s_unit[j];      // polar parameters, turned: B_r itself, Ct' = C_r e^{i (B_theta + C_theta)}
+        atomicAdd(&s_red[0][j], gBr[a]);
+        atomicAdd(&s_red[1][j], gBi[a] * par[0]);
         atomicAdd(&s_red[2][j], gCr[a] * un_[2] + gCi[a] * un_[3]);
         atomicAdd(&s_red[3][j], gCi[a] * par[2] - gCr[a] * par[3]);
       }

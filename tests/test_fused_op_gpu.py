@@ -218,6 +218,30 @@ def test_shapes_beyond_the_fused_kernels_take_the_composite_route():
         _close(g_.grad, w.grad, "gradient wrt " + name)
 
 
+# The sweeps turn states by the phase of B: radii of next to nothing, phases and biases of many turns, states and adjoints in and out,
+# part tiles, several blocks of states, segments.  (Tolerance: as in the tests above.  A running phase of up to 150 is rounded to 8e-6,
+# anew in every tile, below 4e-5 over 25 of them.)
+@pytest.mark.parametrize("b,d,n,l", [(2, 12, 16, 1), (1, 30, 40, 37), (2, 66, 5, 50), (1, 24, 16, 400), (3, 200, 7, 33)])
+def test_turned_states_and_phases_of_many_turns(b, d, n, l):
+    print(f"case turned states b={b} d={d} n={n} l={l}", flush=True)
+    g = torch.Generator().manual_seed(31)
+    args = list(_inputs(b, d, n, l, seed=30, xscale=d ** -0.5))
+    args[3] = (torch.rand(d, n, generator=g, dtype=torch.float64) * 2 - 1) * 9
+    args[4] = torch.where(torch.arange(n) % 3 > 0, args[4], 1e-30)      # (of a zero the oracle's derivative is one of torch's choice)
+    args[6] = torch.where(torch.arange(n) % 4 > 0, args[6], 1e-30)
+    args[5], args[7] = (torch.randn(n, generator=g, dtype=torch.float64) * 20 for _ in range(2))
+    args = [a.float().double() for a in args]
+    grads = [torch.randn(*s, generator=g, dtype=torch.float64).float().double() for s in ((b, d, l), (b, d, n), (b, d, n))]
+    leaves = [a.clone().requires_grad_(True) for a in args]
+    outs = O.adaptive_unitary_op_loop(*leaves)
+    want = [*outs, *torch.autograd.grad(outs, leaves, grads)]
+    dev, gdev = [a.float().cuda() for a in args], [a.float().cuda() for a in grads]
+    got = [*torch.ops.extension_cpp.ssm_adaptive_unitary(*dev), *torch.ops.extension_cpp.ssm_adaptive_backward_unitary(*gdev, *dev)]
+    for k, (a, w) in enumerate(zip(got, [t.detach() for t in want])):
+        scale = float(w.abs().max())
+        assert float((a.double().cpu() - w).abs().max()) <= 1e-4 * scale, (k, scale)
+
+
 def test_softplus_derivative_behind_dt():
     """dt_softplus: ddt is the gradient of the softplus' argument, sigmoid(argument) = 1 - e^-dt times the gradient of dt.  The
     quotient of the two calls' ddt against float64, from dt = 1e-6 to 30: rounding of the product 2^-24, of the series'
