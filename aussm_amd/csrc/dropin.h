@@ -189,17 +189,20 @@ __device__ __forceinline__ float row_last(float v, int) { return dpp_perm<0x15F>
 __device__ __forceinline__ float row_first(float v, int) { return dpp_perm<0x150>(v); }   // row_newbcast:0
 
 
-// Operand records of 16 rows (or columns) of ks steps of 32, by a workgroup of 256 threads: v(k, lane, out) gives the eight values of lane
-// (row = lane % 16, g = lane / 16) of step k, terms 32 k + 8 g .. + 7.  A row is scaled by one power of two, found from its largest
-// value first: a thread keeps its records of up to 512 terms between the two passes.
-template <typename Values>
-__device__ __forceinline__ void phase_records(Values&& values, int ks, bool half, u4* __restrict__ dst) {
+// Operand records of 16 rows (or columns) of ks steps of 32, by a workgroup of 256 threads: load(k, lane, v) reads what the eight values of
+// lane (row = lane % 16, g = lane / 16) of step k, terms 32 k + 8 g .. + 7, are made of, form(k, lane, v) makes them.  A row is scaled by one
+// power of two, found from its largest value first: a thread keeps its records of up to 512 terms between the two passes, and requests
+// them all before it works on the first - a launch lasts little longer than its loads (360 tiles of d = 256
+// 10.2 -> 5.4 us, 687 workgroups for d = 180 8.5 -> 5.8).
+template <typename Load, typename Form>
+__device__ __forceinline__ void phase_records(Load&& load, Form&& form, int ks, bool half, u4* __restrict__ dst) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (!half) {
     const SplitK sk = make_splitk();
     for (int k = wave; k < ks; k += 4) {
       float v[8];
-      values(k, lane, v);
+      load(k, lane, v);
+      form(k, lane, v);
       u4 pc[3];
       split8<3>(sk, v, pc);
 #pragma unroll
@@ -211,12 +214,12 @@ __device__ __forceinline__ void phase_records(Values&& values, int ks, bool half
   constexpr int R = D_MAXKS / 4;
   float v[R][8], most = 0.0f;
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (wave + 4 * r < ks) values(wave + 4 * r, lane, v[r]);
-    else {
+  for (int r = 0; r < R; ++r)
+    if (wave + 4 * r < ks) load(wave + 4 * r, lane, v[r]);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[r][q] = 0.0f;
-    }
+  for (int r = 0; r < R; ++r) {
+    if (wave + 4 * r >= ks) break;
+    form(wave + 4 * r, lane, v[r]);
 #pragma unroll
     for (int q = 0; q < 8; ++q) most = fmaxf(most, fabsf(v[r][q]));
   }
@@ -246,10 +249,15 @@ __device__ __forceinline__ void xprep_block(const DropinPrepArgs& a, unsigned vc
   const float* __restrict__ x = a.x;
   float* __restrict__ x_out = a.x_out;
   const int i = vc / nb, jb = 16 * (vc % nb);
-  auto values = [&](int k, int lane, float (&v)[8]) {
+  auto load = [&](int k, int lane, float (&v)[8]) {
     const int j = jb + (lane & 15), r0 = 32 * k + 8 * (lane >> 4);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = (j < n && r0 + q < d) ? x[((size_t)i * xsi + (size_t)j * xsj) * d + r0 + q] * scale : 0.0f;
+    for (int q = 0; q < 8; ++q) v[q] = x[((size_t)i * xsi + (size_t)min(j, n - 1) * xsj) * d + min(r0 + q, d - 1)];   // (no branch)
+  };
+  auto form = [&](int k, int lane, float (&v)[8]) {
+    const int j = jb + (lane & 15), r0 = 32 * k + 8 * (lane >> 4);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = (j < n && r0 + q < d) ? v[q] * scale : 0.0f;
     if (x_out && j < n) {
       float* const o = x_out + ((size_t)i * n + j) * d + r0;
       if (r0 + 8 <= d) {
@@ -264,7 +272,7 @@ __device__ __forceinline__ void xprep_block(const DropinPrepArgs& a, unsigned vc
     if (a.xb_out && j < n && r0 == 0) a.xb_out[(size_t)i * n + j] = a.x_bias[(size_t)i * xsi + (size_t)j * xsj];
   };
   const bool half = a.KS >= PHASE_HALF_KS;
-  phase_records(values, a.ks, half, a.xp + (size_t)vc * (a.ks * (half ? 2 : 3) * 64 + (half ? 4 : 0)));
+  phase_records(load, form, a.ks, half, a.xp + (size_t)vc * (a.ks * (half ? 2 : 3) * 64 + (half ? 4 : 0)));
 }
 
 // Tiles of u as the second operand of the phase product, one workgroup per (batch element, tile): column l holds U[r][l],
@@ -275,13 +283,19 @@ __device__ __forceinline__ void xprep_block(const DropinPrepArgs& a, unsigned vc
 __device__ __forceinline__ void uprep_block(const DropinPrepArgs& a, unsigned block) {
   const int d = a.d, L = a.L, t = a.t0 + block % a.nt;
   const float* __restrict__ ub = a.u + (size_t)(a.b0 + block / a.nt) * d * L;
-  auto values = [&](int k, int lane, float (&v)[8]) {
+  auto load = [&](int k, int lane, float (&v)[8]) {
     const int l = t * DT + (lane & 15), r0 = 32 * k + 8 * (lane >> 4);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = row_prefix((r0 + q < d && l < L) ? ub[(size_t)(r0 + q) * L + l] : 0.0f);
+    for (int q = 0; q < 8; ++q) v[q] = ub[(size_t)min(r0 + q, d - 1) * L + min(l, L - 1)];
+  };
+  auto form = [&](int k, int lane, float (&v)[8]) {
+    const int l = t * DT + (lane & 15), r0 = 32 * k + 8 * (lane >> 4);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = r0 + q < d && l < L ? v[q] : 0.0f;
+    rows_side_by_side<8>(v);
   };
   const bool half = a.KS >= PHASE_HALF_KS;
-  phase_records(values, a.KS, half, a.up + (size_t)block * (a.KS * (half ? 2 : 3) * 64 + (half ? 4 : 0)));
+  phase_records(load, form, a.KS, half, a.up + (size_t)block * (a.KS * (half ? 2 : 3) * 64 + (half ? 4 : 0)));
 }
 
 // A tile's records, global memory -> registers -> LDS, in two steps so that the loads of the next tile fly
@@ -577,7 +591,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && KS <= 8 ? 4 : 1) void dropin_fw
     const float cnt = (float)(min(l_ + 1, L - l0));      // timesteps of the tile up to this one that exist
     float ysum = 0.0f;
     // GS states side by side (rows_side_by_side; all four would spill registers where the parameters stay in LDS).  32 x 256 x 16, 720
-    // steps, in workgroups of four 243 -> 237 us; 8 x 180, 700 steps 70 -> 66
+    // steps, in workgroups of four 243 -> 237 us; 8 x 180, 700 steps 70 -> 57
     constexpr int GS = PAR_LDS ? 2 : 4;
 #pragma unroll
     for (int a0 = 0; a0 < 4; a0 += GS) {
