@@ -487,7 +487,7 @@ __global__ __launch_bounds__(NW * 64) void dropin_seg_kernel(const DropinBwdArgs
 // KS: 32-wide steps of the contraction over r (d <= 32 KS).
 // The kernel waits more than it works, so it takes the registers of four workgroups of four wavefronts to a compute unit at 128 < d:
 // the tiles of U go straight to LDS (there and up to d = 128, in workgroups of eight), and at d > 192 the polar parameters are read
-// from LDS where they are used.  Whole call of 32 x 256 x 16, 720 steps: 339 us with three bf16 pieces and three workgroups, now
+// from LDS where they are used.  Whole call of 32 x 256 x 16, 720 steps: 339 us with three bf16 pieces and three workgroups, then
 // 234 (249 with three workgroups, 307 in workgroups of eight); 32 x 180 198 -> 167, 32 x 128 107 -> 99.
 // One wavefront on a SIMD (d > 256) or two of wide x gain nothing from it: 8 x 300, 400 steps 109 -> 113, 8 x 250, 720 86 -> 90.
 template <int KS, int NW>
